@@ -176,6 +176,7 @@ EXPORTS = (
 )
 STATIC_WORKSPACE_BYTES = 64 << 20
 KMOE_FLAG_SIDE_STREAM = 1
+KMOE_FLAG_LOGITS_ACT_DTYPE = 2
 
 
 def check(rc: int) -> None:
@@ -190,9 +191,14 @@ def ptr(t: torch.Tensor | None):
     return None if t is None else C.c_void_p(t.data_ptr())
 
 
+def raw_stream(device_index: int | None = None) -> int:
+    """The current torch HIP stream of a device (default: the current one) as an integer handle."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if device_index is None else device_index)
+
+
 def stream():
     """The current torch HIP stream as a hipStream_t."""
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return C.c_void_p(raw_stream())
 
 
 def act_dtype(t: torch.Tensor, what: str = "kmoe") -> int:

@@ -21,7 +21,7 @@ from typing import Optional
 import torch
 
 from ... import _lib as L
-from ..._plan import is_tiled, tile_int8_weights_
+from ..._plan import WORKSPACE, tile_int8_weights_, weight_layout
 
 
 @dataclass
@@ -149,21 +149,18 @@ class KunlunScaledMMLinearKernel:
             raise RuntimeError("KunlunScaledMMLinearKernel: process_weights_after_loading has not run on this layer")
         from ...ops import _custom_ops as ops  # registers torch.ops._C.*
         lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1]).contiguous()
-        M, n, k = x2.shape[0], w.shape[1], w.shape[2]
+        x2 = x if x.dim() == 2 and x.is_contiguous() else x.reshape(-1, x.shape[-1]).contiguous()
+        (M, k), n = x2.shape, w.shape[1]
+        if k != w.shape[2]:
+            raise ValueError(f"KunlunScaledMMLinearKernel: rows of {k} values for weights of {w.shape[2]}")
         out = torch.empty((M, n), dtype=x.dtype, device=x.device)
-        if M == 0:
-            return out.reshape(*lead, n)
-        if x_s is not None:  # static: one scale for the tensor, so every row's max is scale x 127
+        if M and x_s is not None:  # static: one scale for the tensor, so every row's max is scale x 127
             x_q, x_s, _, _ = torch.ops._C.scaled_int8_quant(x2, x_s.data.to(torch.float32).reshape(1), None, True)
             x_max = (x_s * 127.0).expand(M).contiguous()
             ops._gemm_i8(x_q, x_max, w, w_s.data.reshape(-1), self._row_range(x.device, M), out, n, L.KMOE_ACT_NONE, M)
-        elif is_tiled(w) and M <= self.STREAM_MAX_ROWS:
-            self._stream_gemm(x2, w, w_s.data.reshape(-1), out)
-        else:
-            x_q, x_max, _, _ = torch.ops._C.scaled_int8_quant(x2, None, None, True)
-            ops._gemm_i8(x_q, x_max, w, w_s.data.reshape(-1), self._row_range(x.device, M), out, n, L.KMOE_ACT_NONE, M)
-        return out.reshape(*lead, n)
+        elif M:
+            self._dynamic_gemm(x2, w, w_s, out, dt)
+        return out if x.dim() == 2 else out.reshape(*lead, n)
 
     def _apply_asymmetric(self, layer, x, w_q, w_s, x_s, x_zp, azp_adj, bias):
         """Reference: scale_mm.py:60-82. Codes with a zero point (per token, or the layer's static one), the int8
@@ -194,22 +191,34 @@ class KunlunScaledMMLinearKernel:
             self._lod[key] = torch.tensor([0, rows], dtype=torch.int32).to(device)
         return self._lod[key]
 
-    def _stream_gemm(self, x2, w, w_max, out):
+    def _dynamic_gemm(self, x2, w, w_max, out, dt):
+        """Quantisation and GEMM of one call on a scratch buffer of the stream: codes, then row maxes. Two calls into
+        the library and one allocation (the output)."""
+        L.require_device(x2, w, w_max)
         M, k = x2.shape
         n = w.shape[1]
-        x_q = torch.empty((k // 64, M, 64), dtype=torch.int8, device=x2.device)  # chunk-major codes
-        x_max = torch.empty((M,), dtype=torch.float32, device=x2.device)
-        L.check(L.lib.kmoe_quant_i8_rows_chunked_dt(L.ptr(x2), k, M, k, L.ptr(x_q), L.ptr(x_max),
-                                                    L.act_dtype(x2), L.stream()))
+        codes = -(-M * k // 256) * 256
+        stream = L.raw_stream()
+        if torch._C._cuda_isCurrentStreamCapturing():
+            scratch = torch.empty(codes + 4 * M, dtype=torch.uint8, device=x2.device)  # the graph's own
+        else:
+            scratch = WORKSPACE.get(codes + 4 * M, x2.device, L.raw_stream(x2.device.index))
+        x_q = scratch.data_ptr()
+        x_max = x_q + codes
+        layout = weight_layout(w)
+        tail = layout == L.KMOE_W_TILED and M <= self.STREAM_MAX_ROWS
         g = L.GemmI8Args()
-        g.a, g.lda, g.a_max, g.src_div = x_q.data_ptr(), k, x_max.data_ptr(), 1
-        g.a_layout, g.a_rows = L.KMOE_A_CHUNKED, M
-        # one routed expert without rows (the launch needs an expert list), the matrix as the tail expert
-        g.w, g.w_max, g.lod = w.data_ptr(), w_max.data_ptr(), self._row_range(x2.device, 0).data_ptr()
-        g.E, g.n, g.k, g.rows = 1, n, k, 0
-        g.w_tail, g.w_max_tail = w.data_ptr(), w_max.data_ptr()
-        g.tail_row0, g.tail_rows, g.tail_src0 = 0, M, 0
-        g.y, g.ldy, g.act, g.w_layout = out.data_ptr(), n, L.KMOE_ACT_NONE, L.KMOE_W_TILED
-        g.act_dtype = L.act_dtype(out)
-        g.variant = 1 if M <= 128 else 2  # 16 or 32 rows per slice
-        L.check(L.lib.kmoe_grouped_gemm_i8(g, L.stream()))
+        g.a, g.lda, g.a_max, g.src_div = x_q, k, x_max, 1
+        g.w, g.w_max = w.data_ptr(), w_max.data_ptr()
+        g.E, g.n, g.k = 1, n, k
+        g.y, g.ldy, g.act, g.w_layout, g.act_dtype = out.data_ptr(), n, L.KMOE_ACT_NONE, layout, dt
+        if tail:
+            L.check(L.lib.kmoe_quant_i8_rows_chunked_dt(x2.data_ptr(), k, M, k, x_q, x_max, dt, stream))
+            # one routed expert without rows (the launch needs an expert list), the matrix as the tail expert
+            g.a_layout, g.a_rows, g.lod, g.rows = L.KMOE_A_CHUNKED, M, self._row_range(x2.device, 0).data_ptr(), 0
+            g.w_tail, g.w_max_tail, g.tail_rows = g.w, g.w_max, M
+            g.variant = 1 if M <= 128 else 2  # 16 or 32 rows per slice
+        else:
+            L.check(L.lib.kmoe_quant_i8_rows_dt(x2.data_ptr(), k, M, k, x_q, k, x_max, dt, stream))
+            g.lod, g.rows = self._row_range(x2.device, M).data_ptr(), M
+        L.check(L.lib.kmoe_grouped_gemm_i8(g, stream))
