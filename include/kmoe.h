@@ -577,7 +577,7 @@ typedef struct kmoe_moe_args {
   int32_t renormalize;   /* softmax only: divide the K weights by their sum     */
   int32_t n_group, topk_group; /* sigmoid only; n_group <= 1: no group stage    */
   float routed_scale;    /* sigmoid only: multiplies the routing weights        */
-  const float* logits;   /* [M,E] f32, or NULL with w_gate set: the layer then computes
+  const float* logits;   /* [M,E] f32 (16-bit with KMOE_FLAG_LOGITS_ACT_DTYPE), or NULL with w_gate set: the layer then computes
                             them itself (kmoe_router_gemm_bf16 without the reduction
                             pass: the routing kernel adds the partial planes)     */
   const float* bias;     /* [E] f32 correction bias or NULL                     */
@@ -643,6 +643,10 @@ typedef struct kmoe_moe_args {
  * process (0: never, 1: as if every call set it); it is read once. Ignored with stage_events and by
  * kmoe_moe_forward_static. */
 #define KMOE_FLAG_SIDE_STREAM 1
+/* KMOE_FLAG_LOGITS_ACT_DTYPE: `logits` points to 16-bit values of act_dtype (what a gate that is an ordinary 16-bit
+ * Linear leaves) instead of f32: the routing kernel widens them as it loads them, the same bits as after a
+ * conversion. */
+#define KMOE_FLAG_LOGITS_ACT_DTYPE 2
 
 /* Decode-sized int8 batches (at most 10 rows per expert, tiled weights): two of the layer's small launches are folded
  * into the GEMM launches. The gate_up launch sorts the routed pairs by expert itself (every workgroup scans the pairs'

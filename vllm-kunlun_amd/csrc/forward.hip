@@ -515,41 +515,20 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   const bool stream_mode = use_stream_path(a);
   bool quant_done = false;
   mark(KMOE_STAGE_ROUTING, 0);
-  const float* logits = a->logits;
-  int planes = 1;
-  size_t plane_stride = 0;
-  if (!logits) {
-    int mf = 0;
+  const bool f16 = a->act_dtype == KMOE_DT_F16;
+  LogitsView logits{a->logits, 1, 0, (a->flags & KMOE_FLAG_LOGITS_ACT_DTYPE) ? (f16 ? 2 : 1) : 0};
+  if (!a->logits) {
+    int mf = 0, planes = 1;
     router_plan(M, H, Eg, &planes, &mf);
     float* buf = static_cast<float*>(at(L.logit_planes));
-    plane_stride = static_cast<size_t>(M) * Eg;
-    rc = router_gemm_planes(a->x, H, a->w_gate, M, H, Eg, buf, plane_stride, Eg, planes, mf, as_stream(stream),
-                            a->act_dtype == KMOE_DT_F16);
-    if (rc) return rc;
-    logits = buf;
-  }
-  // 1. routing; on the int8 decode path together with step 3 (independent work, one launch)
-  if (a->format == KMOE_FMT_INT8) {
-    rc = fused_route_quant_i8(logits, planes, plane_stride, a->bias, M, Eg, K, a->scoring == KMOE_SCORE_SIGMOID, a->renormalize, a->n_group,
-                              a->topk_group, a->routed_scale, topk_w, topk_ids, a->x, H, static_cast<int8_t*>(at(L.xq)),
-                              static_cast<float*>(at(L.xmax)), stream_mode ? 1 : 0, a->act_dtype == KMOE_DT_F16,
-                              as_stream(stream));
-    if (rc < 0) return rc;
-    quant_done = rc == KMOE_OK;
-    rc = KMOE_OK;
-  }
-  if (!quant_done && planes > 1) {  // the stand-alone routing kernels take finished logits: add the planes into plane 0
-    rc = router_reduce(logits, plane_stride, planes, M, Eg, static_cast<float*>(at(L.logit_planes)), Eg, as_stream(stream));
+    logits = LogitsView{buf, planes, static_cast<size_t>(M) * Eg, 0};
+    rc = router_gemm_planes(a->x, H, a->w_gate, M, H, Eg, buf, logits.plane_stride, Eg, planes, mf, as_stream(stream), f16);
     if (rc) return rc;
   }
-  if (quant_done) {
-    // both done
-  } else if (a->scoring == KMOE_SCORE_SOFTMAX) {
-    rc = kmoe_softmax_topk(logits, M, Eg, K, a->renormalize, topk_w, topk_ids, stream);
-  } else {
-    rc = kmoe_sigmoid_group_topk_norm(logits, a->bias, M, Eg, K, a->n_group, a->topk_group, a->routed_scale, topk_w,
-                                      topk_ids, stream);
-  }
+  // 1. routing; for the quantised formats together with step 3 (independent work, one launch)
+  const RouteArgs route{logits, a->bias, M, Eg, K, a->renormalize, a->n_group, a->topk_group, a->routed_scale, topk_w, topk_ids};
+  rc = route_and_quantise(route, a->scoring == KMOE_SCORE_SIGMOID, a->format, a->x, H, at(L.xq),
+                          static_cast<float*>(at(L.xmax)), stream_mode, f16, &quant_done, as_stream(stream));
   if (rc) return rc;
   mark(KMOE_STAGE_ROUTING, 1);
   // 2. stable sort of the routed pairs by expert. On the weight-streaming path (a few rows per expert) the gate_up

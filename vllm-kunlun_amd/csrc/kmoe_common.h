@@ -61,11 +61,27 @@ bool w4_gate_up_streams(int rows, int rows_hint, int E, int k);
 int tiled_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream);
 int tiled_gemm_fp8(const kmoe_gemm_fp8_args* args, hipStream_t stream);
 int tiled_gemm_bf16(const kmoe_gemm_bf16_args* args, hipStream_t stream);
-// Routing + per-token int8 quantisation of x [M,H] in one launch. Returns 1 (nothing launched)
-// when the arguments are outside its instantiations: the caller then uses the two entry points.
-int fused_route_quant_i8(const float* logits, int planes, size_t plane_stride, const float* bias, int M, int E, int K, int sigmoid, int renorm,
-                         int n_group, int topk_group, float scale, float* topk_w, int32_t* topk_ids,
-                         const uint16_t* x, int H, int8_t* xq, float* xmax, int chunked, int f16, hipStream_t stream);
+// The router logits as a routing kernel finds them: f32, or 16-bit values (bf16 / half: what a gate that is an
+// ordinary 16-bit Linear leaves; widening them is exact, so reading them where they are used instead of after a
+// conversion launch changes no bit), or the partial planes of a split-K router GEMM, `plane_stride` floats apart.
+struct LogitsView {
+  const void* p;
+  int planes;  // > 1: f32 partial sums; the logit is their sum, plane 0 first
+  size_t plane_stride;
+  int type;  // 0: f32, 1: bf16, 2: half (planes == 1)
+};
+struct RouteArgs {
+  LogitsView logits;  // [M, E]
+  const float* bias;
+  int M, E, K, renorm, n_group, topk_group;
+  float scale;
+  float* topk_w;
+  int32_t* topk_ids;
+};
+// Routing of M tokens and, for KMOE_FMT_INT8 / _FP8_BLOCK where the kernel takes the row length, the quantisation of
+// x [M,H] in the same launch (*quantised says whether it was). M >= 1.
+int route_and_quantise(RouteArgs r, bool sigmoid, int format, const uint16_t* x, int H, void* xq, float* x_aux,
+                       bool chunked, bool f16, bool* quantised, hipStream_t stream);
 
 // Router GEMM pieces for the fused layer: the split (ks planes, mf*16 tokens per wave) chosen for
 // a shape, and the launch that leaves the partial planes [ks][M][E] (ks == 1: the logits).
@@ -205,54 +221,12 @@ __device__ inline int wave_sum_int(int v) {
   return v;
 }
 
-// (value, index) argmax with ties to the lower index; all lanes get the winner.
-__device__ inline void wave_argmax(float& v, int& idx) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const float ov = __shfl_xor(v, off, kWave);
-    const int oi = __shfl_xor(idx, off, kWave);
-    if (ov > v || (ov == v && oi < idx)) {
-      v = ov;
-      idx = oi;
-    }
-  }
-}
-
-// ---- wave-wide arg-max on packed keys, over DPP (no LDS crossbar) ------------
-// A float maps to an unsigned int with the same order (-0 counts as +0); the key
-// is (ordered value << 32) | ~index, so the largest key is the largest value
-// and, among equal values, the lowest index. Key 0 means "no candidate".
+// A float as an unsigned int with the same order (-0 counts as +0); no finite or infinite value maps to 0.
 __device__ inline uint32_t ordered_bits(float v) {
   union { float f; uint32_t u; } b;
   b.f = v + 0.0f;
   return (b.u & 0x80000000u) ? ~b.u : (b.u | 0x80000000u);
 }
-__device__ inline uint64_t arg_key(float v, int idx) {
-  return (static_cast<uint64_t>(ordered_bits(v)) << 32) | static_cast<uint32_t>(~static_cast<uint32_t>(idx));
-}
-__device__ inline int arg_key_index(uint64_t key) { return static_cast<int>(~static_cast<uint32_t>(key)); }
-
-template <int CTRL, int ROW_MASK>
-__device__ inline uint64_t dpp_max_step(uint64_t k) {
-  const uint32_t lo = static_cast<uint32_t>(k), hi = static_cast<uint32_t>(k >> 32);
-  const uint32_t olo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xf, false);
-  const uint32_t ohi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xf, false);
-  const uint64_t o = (static_cast<uint64_t>(ohi) << 32) | olo;
-  return o > k ? o : k;
-}
-// Max of a 64-bit key over the 64 lanes; every lane gets the result.
-__device__ inline uint64_t wave_max_u64(uint64_t k) {
-  k = dpp_max_step<0xB1, 0xf>(k);   // quad_perm [1,0,3,2]
-  k = dpp_max_step<0x4E, 0xf>(k);   // quad_perm [2,3,0,1]
-  k = dpp_max_step<0x141, 0xf>(k);  // row_half_mirror
-  k = dpp_max_step<0x140, 0xf>(k);  // row_mirror: every lane of a 16-lane row holds the row max
-  k = dpp_max_step<0x142, 0xa>(k);  // row_bcast15 into rows 1 and 3
-  k = dpp_max_step<0x143, 0xc>(k);  // row_bcast31 into rows 2 and 3: lane 63 holds the wave max
-  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(k), 63);
-  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(k >> 32), 63);
-  return (static_cast<uint64_t>(hi) << 32) | lo;
-}
-
 __device__ inline uint64_t lanemask_lt() {
   return (static_cast<uint64_t>(1) << lane_id()) - 1;
 }

@@ -1,5 +1,5 @@
-// Per-row dynamic int8 quantisation as a device function, shared by the stand-alone
-// kernel and the fused routing + quantisation launch.
+// Per-row dynamic int8 and per-group fp8 quantisation as device functions, shared by the stand-alone
+// kernels and the fused routing + quantisation launch.
 #pragma once
 #include "kmoe_common.h"
 
@@ -68,6 +68,49 @@ __device__ inline void quant_i8_rows_body(const uint16_t* __restrict__ x, int64_
     }
   }
   if (t == 0) row_max[r] = amax;
+}
+
+// ------------------------------------------------------------- fp8 group128
+// OCP e4m3fn encode of two floats, round-to-nearest-even, saturating at 448 (NaN -> the largest
+// code of its sign): the conversion instruction of gfx950 (v_cvt_pk_fp8_f32 encodes the OCP format
+// there) after an explicit clamp, so that its own overflow handling never comes into play.
+__device__ inline uint32_t pack2_e4m3fn(float a, float b) {
+  auto clamp = [](float f) {
+    f = f != f ? __builtin_copysignf(448.0f, f) : f;
+    return __builtin_fminf(__builtin_fmaxf(f, -448.0f), 448.0f);
+  };
+  return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(clamp(a), clamp(b), 0, false)) & 0xffffu;
+}
+
+// 16 lanes x 8 values = one 128-column group; 4 groups per wave. (Several groups per team, all
+// requested up front, measured no faster: the eight IEEE divisions per lane set the pace.)
+__device__ inline void quant_fp8_group128_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
+                                               uint8_t* __restrict__ q, int64_t ld_q, float* __restrict__ scale,
+                                               int block, bool f16) {
+  const int groups_per_row = C / 128;
+  const long long total = static_cast<long long>(R) * groups_per_row;
+  const long long gid = static_cast<long long>(block) * 16 + (threadIdx.x >> 4);
+  const int t = threadIdx.x & 15;
+  const bool live = gid < total;
+  const int r = live ? static_cast<int>(gid / groups_per_row) : 0;
+  const int g = live ? static_cast<int>(gid % groups_per_row) : 0;
+  Pack8 val;
+  val.v = make_uint4(0, 0, 0, 0);
+  if (live) val.v = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(r) * ld_x + g * 128 + t * 8);
+  float amax = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(act_to_f32(val.h[j], f16)));
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
+  if (!live) return;
+  const float s = amax / 448.0f;
+  float f[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) f[j] = s > 0.0f ? act_to_f32(val.h[j], f16) / s : 0.0f;
+  const uint32_t w[2] = {pack2_e4m3fn(f[0], f[1]) | (pack2_e4m3fn(f[2], f[3]) << 16),
+                         pack2_e4m3fn(f[4], f[5]) | (pack2_e4m3fn(f[6], f[7]) << 16)};
+  *reinterpret_cast<uint2*>(q + static_cast<size_t>(r) * ld_q + g * 128 + t * 8) = make_uint2(w[0], w[1]);
+  if (t == 0) scale[static_cast<size_t>(r) * groups_per_row + g] = s;
 }
 
 }  // namespace kmoe
