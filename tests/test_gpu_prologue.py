@@ -1,0 +1,58 @@
+"""The launch in front of a layer's first GEMM (routing, with the quantisation of the activations where the format has
+one): router logits in the activations' own 16-bit type must give the bits of the same logits widened to float32, for
+every format and slot count of the routing kernel; a layer call whose argument block is kept from an earlier call must
+follow what changed in between."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# experts on both sides of a routing kernel's slot counts (128, 256, 512), groups that are a power of two and not
+@pytest.mark.parametrize("E,n_group", [(8, 2), (96, 3), (128, 8), (129, 1), (192, 4), (256, 8), (320, 5), (520, 4)])
+@pytest.mark.parametrize("quant", ["int8", "fp8", "none"])
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_sixteen_bit_logits_route_like_their_float32_values(E, n_group, quant, scoring, dtype):
+    from vllm_kunlun_amd import synth
+    base = "dsv3-decode" if scoring == "sigmoid" else "qwen3-decode"
+    topk_group = max(1, n_group // 2)
+    shape = synth.scaled(synth.SHAPES[base], M=37, H=256, E=E, K=4, I=128, I_shared=0, quant=quant,
+                         n_group=n_group if scoring == "sigmoid" else 1, topk_group=topk_group)
+    sl = synth.make_layer(shape, "cuda", seed=E, dtype=dtype)
+    logits = (sl.logits * 2).to(dtype)  # (16-bit values repeat: ties go to the lower expert either way)
+    a = sl.layer(sl.x, logits)
+    b = sl.layer(sl.x, logits.float())
+    assert torch.equal(a, b) and float(a.float().abs().max()) > 0
+
+
+def test_kept_argument_block_follows_the_call():
+    """The second call of a layer reuses the first one's argument block: another batch size, other inputs, other
+    options, another layer at the same sizes and weights that were swapped must all be seen."""
+    from vllm_kunlun_amd import synth
+    shape = synth.scaled(synth.SHAPES["qwen3-decode"], M=48, H=256, E=16, K=4, I=128)
+    sl, other = synth.make_layer(shape, "cuda", seed=1), synth.make_layer(shape, "cuda", seed=2)
+    m = sl.layer.quant_method
+    full = m.apply_monolithic(sl.layer, sl.x, sl.logits)
+    assert torch.equal(m.apply_monolithic(sl.layer, sl.x, sl.logits), full)
+    for n in (1, 17, 48):
+        assert torch.equal(m.apply_monolithic(sl.layer, sl.x[:n], sl.logits[:n]), full[:n])
+    doubled = m.apply_monolithic(sl.layer, sl.x, sl.logits, out_scale=2.0)
+    assert torch.equal(doubled.float(), 2 * full.float())
+    want = other.layer.quant_method.apply_monolithic(other.layer, sl.x, sl.logits)
+    assert not torch.equal(want, full)
+    for name in ("w13_weight", "w2_weight", "w13_weight_scale", "w2_weight_scale"):
+        getattr(sl.layer, name).data = getattr(other.layer, name).data
+    assert torch.equal(m.apply_monolithic(sl.layer, sl.x, sl.logits), want)
+    with pytest.raises(ValueError):
+        m.apply_monolithic(sl.layer, sl.x, sl.logits[:5])
+    with pytest.raises(ValueError):
+        m.apply_monolithic(sl.layer, sl.x[:, :128].contiguous(), sl.logits)
+    with pytest.raises(RuntimeError):
+        m.apply_monolithic(sl.layer, sl.x.cpu(), sl.logits.cpu())
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        on_side = m.apply_monolithic(sl.layer, sl.x, sl.logits)
+    torch.cuda.synchronize()
+    assert torch.equal(on_side, want)

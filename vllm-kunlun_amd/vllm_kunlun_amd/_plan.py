@@ -18,7 +18,7 @@ from . import _lib as L
 
 
 def _current_stream_id(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    return L.raw_stream(device.index)
 
 
 class _Workspace:
@@ -81,9 +81,12 @@ class MoEPlan:
 # torch's StorageImpl, dropped when the storage dies), not to a tensor object: views, `.data`, `.detach()`,
 # `.t()` and a Parameter wrapped around the same memory all see it.
 _TILED: dict[int, tuple[int, int]] = {}  # storage -> (n, bytes of k) of the tiles it holds
+_layout_epoch = 0  # counts re-arrangements of weights: what run_layer remembers about a layout holds within one
 
 
 def _mark_tiled(w: torch.Tensor, n: int, k_bytes: int) -> None:
+    global _layout_epoch
+    _layout_epoch += 1
     storage = w.untyped_storage()
     key = storage._cdata
     _TILED[key] = (n, k_bytes)
@@ -155,6 +158,8 @@ def tile_w4_scales_(scale: torch.Tensor) -> bool:
     for e in range(E):
         L.check(L.lib.kmoe_tile_scales_w4(L.ptr(data[e]), L.ptr(tmp), 1, n, groups, L.stream()))
         data[e].copy_(tmp)
+    global _layout_epoch
+    _layout_epoch += 1
     storage = data.untyped_storage()
     _SCALES_FRAG16[key] = (n, groups)
     weakref.finalize(storage, _SCALES_FRAG16.pop, key, None)
@@ -219,7 +224,7 @@ def make_moe_plan(fmt: int, x: torch.Tensor, logits: torch.Tensor, out: torch.Te
                   w2_bias: Optional[torch.Tensor] = None, activation: str = "silu", act_alpha: float = 1.702,
                   act_limit: float = 7.0, group_size: Optional[int] = None, tile_variant: int = 0,
                   shared_scale: float = 1.0, first_expert: int = 0, side_stream: bool = False) -> MoEPlan:
-    """x bf16 [M,H] (or float16 with int8 or unquantized weights, the latter then float16 too), logits f32 [M,E], out [M,H] like x; w13 [E,2I,H], w2 [E,H,I] in the
+    """x bf16 [M,H] (or float16 with int8 or unquantized weights, the latter then float16 too), logits [M,E] f32 or in x's dtype, out [M,H] like x; w13 [E,2I,H], w2 [E,H,I] in the
     format's dtype; w13_aux/w2_aux: per-channel maxes (int8) or block scales (fp8), None for bf16.
     shared_expert: (ws13 [2Is,H], ws13_aux, ws2 [H,Is], ws2_aux) in the same format.
     logits may be None when router_weight (bf16 [E,H], the gate projection) is given: the
@@ -250,8 +255,8 @@ def make_moe_plan(fmt: int, x: torch.Tensor, logits: torch.Tensor, out: torch.Te
     if fmt == L.KMOE_FMT_BF16 and dt == L.KMOE_DT_F16 and (w13_bias is not None or w2_bias is not None
                                                            or activation == "swigluoai"):
         raise NotImplementedError("moe plan: expert biases and swigluoai are built for bfloat16 only")
-    if out.dtype != x.dtype or (logits is not None and logits.dtype != torch.float32):
-        raise ValueError("moe plan: out must have x's dtype and logits must be float32")
+    if out.dtype != x.dtype or (logits is not None and logits.dtype not in (torch.float32, x.dtype)):
+        raise ValueError("moe plan: out must have x's dtype and logits must be float32 or have x's dtype")
     if w13.dtype not in _WEIGHT_DTYPE[fmt] or w2.dtype != w13.dtype:
         raise ValueError(f"moe plan: weight dtype {w13.dtype} does not fit the layer format")
     E, two_i, H = w13.shape
@@ -333,6 +338,8 @@ def make_moe_plan(fmt: int, x: torch.Tensor, logits: torch.Tensor, out: torch.Te
     a.act_dtype = dt
     a.shared_scale = float(shared_scale)
     a.flags = L.KMOE_FLAG_SIDE_STREAM if side_stream else 0
+    if logits is not None and logits.dtype != torch.float32:
+        a.flags |= L.KMOE_FLAG_LOGITS_ACT_DTYPE
     a.out = out.data_ptr()
     if w_layout is None:  # per group of weights: tiled if both of its tensors have been tiled
         w_layout = L.KMOE_W_TILED if is_tiled(w13) and is_tiled(w2) else L.KMOE_W_ROWMAJOR
@@ -359,3 +366,99 @@ def make_moe_plan(fmt: int, x: torch.Tensor, logits: torch.Tensor, out: torch.Te
     else:
         ws = WORKSPACE.get(lay.total_bytes, x.device, stream_id)
     return MoEPlan(a, lay, ws, keep, stream_id)
+
+
+class _LayerCall:
+    """What run_layer keeps of a layer call: the filled argument block (everything but the batch), the tensors it was
+    filled from, and the workspace layout per batch size."""
+
+    __slots__ = ("args", "tensors", "epoch", "hidden", "experts", "layouts")
+
+    def __init__(self, plan: MoEPlan, tensors, experts: int):
+        self.args = L.MoEArgs.from_buffer_copy(plan.args)
+        self.tensors = [(weakref.ref(t), t.data_ptr(), t.shape) for t in tensors]
+        self.epoch = _layout_epoch
+        self.hidden, self.experts, self.layouts = int(plan.args.H), experts, {}
+
+    def holds(self) -> bool:
+        """Whether the tensors are still the objects, at the addresses and of the shapes the block was filled for, and
+        no weight was re-arranged since."""
+        if self.epoch != _layout_epoch:
+            return False
+        for ref, at, shape in self.tensors:
+            t = ref()
+            if t is None or t.data_ptr() != at or t.shape != shape:
+                return False
+        return True
+
+    def layout(self, M: int) -> L.MoELayout:
+        lay = self.layouts.get(M)
+        if lay is None:
+            if len(self.layouts) >= 512:
+                self.layouts.clear()
+            lay = L.MoELayout()
+            args = L.MoEArgs.from_buffer_copy(self.args)
+            args.M = M
+            L.check(L.lib.kmoe_moe_workspace_layout(args, lay))
+            self.layouts[M] = lay
+        return lay
+
+
+# Argument blocks of recent layer calls, least recently used first out. They hold no tensor alive.
+_CALLS: collections.OrderedDict = collections.OrderedDict()
+MAX_CALLS = 1024
+
+
+def run_layer(fmt: int, x: torch.Tensor, logits: Optional[torch.Tensor], top_k: int, w13: torch.Tensor, w2: torch.Tensor,
+              w13_aux: Optional[torch.Tensor], w2_aux: Optional[torch.Tensor], scoring_func: str = "softmax",
+              renormalize: bool = True, num_expert_group: Optional[int] = None, topk_group: Optional[int] = None,
+              routed_scaling_factor: float = 1.0, e_score_correction_bias: Optional[torch.Tensor] = None,
+              shared_expert=None, out_scale: float = 1.0, router_weight: Optional[torch.Tensor] = None,
+              group_size: Optional[int] = None, shared_scale: float = 1.0, first_expert: int = 0,
+              side_stream: bool = False):
+    """One layer call on a fresh output tensor: make_moe_plan's arguments, its checks and its result, as (out, layout,
+    workspace). x and logits may come strided and logits in any float type. Filling and checking an argument block
+    costs more host time than a decode step takes on the GPU, and a model's step makes the same call per layer again
+    and again, so the block is kept: a later call with the same weights and options copies it and fills in the batch
+    (Qwen3 shape, one token: host time per call 55 -> 19 us). What may have changed is compared, not assumed: the
+    tensors' identity, address and shape, and the state of the weights' re-arrangement."""
+    x = x.contiguous()
+    if logits is not None:
+        if logits.dtype != torch.float32 and logits.dtype != x.dtype:
+            logits = logits.float()
+        logits = logits.contiguous()
+    out = torch.empty_like(x)
+    key = (fmt, x.dtype, x.device, None if logits is None else logits.dtype, top_k, id(w13), id(w2), id(w13_aux), id(w2_aux),
+           scoring_func, renormalize, num_expert_group, topk_group, routed_scaling_factor, id(e_score_correction_bias),
+           None if shared_expert is None else tuple(map(id, shared_expert)), out_scale, id(router_weight), group_size,
+           shared_scale, first_expert, side_stream)
+    call = _CALLS.get(key)
+    if call is None or not call.holds():
+        plan = make_moe_plan(fmt, x, logits, out, top_k, w13, w2, w13_aux, w2_aux, scoring_func, renormalize,
+                             num_expert_group, topk_group, routed_scaling_factor, e_score_correction_bias, shared_expert,
+                             out_scale, router_weight=router_weight, group_size=group_size, shared_scale=shared_scale,
+                             first_expert=first_expert, side_stream=side_stream)
+        tensors = [t for t in (w13, w2, w13_aux, w2_aux, e_score_correction_bias, router_weight, *(shared_expert or ()))
+                   if t is not None]
+        routed = logits.shape[-1] if logits is not None else router_weight.shape[0]
+        _CALLS[key] = _LayerCall(plan, tensors, routed)
+        while len(_CALLS) > MAX_CALLS:
+            _CALLS.popitem(last=False)
+        plan()
+        return out, plan.layout, plan.workspace
+    M = x.shape[0]
+    if x.shape != (M, call.hidden) or (logits is not None and logits.shape != (M, call.experts)):
+        raise ValueError("moe plan: x must be [M,H] and logits [M,E]")
+    if not x.is_cuda or (logits is not None and logits.device != x.device):
+        raise RuntimeError(f"kmoe ops run on the GPU only; got a tensor on {logits.device if x.is_cuda else x.device}")
+    args = L.MoEArgs.from_buffer_copy(call.args)  # a copy: threads may share the block
+    args.M, args.x, args.out = M, x.data_ptr(), out.data_ptr()
+    if logits is not None:
+        args.logits = logits.data_ptr()
+    layout = call.layout(M)
+    if torch._C._cuda_isCurrentStreamCapturing():
+        workspace = torch.empty(layout.total_bytes, dtype=torch.uint8, device=x.device)  # the graph's own (see make_moe_plan)
+    else:
+        workspace = WORKSPACE.get(layout.total_bytes, x.device, L.raw_stream(x.device.index))
+    L.check(L.lib.kmoe_moe_forward(args, workspace.data_ptr(), workspace.numel(), L.raw_stream()))
+    return out, layout, workspace

@@ -13,7 +13,7 @@ from typing import Optional
 import torch
 
 from .. import _lib as L
-from .._plan import make_moe_plan
+from .._plan import make_moe_plan, run_layer
 
 
 class KunlunOps:
@@ -40,17 +40,17 @@ class KunlunOps:
         `use_grouped_topk` and `inplace` are accepted and ignored, :385-389 vs :413-431);
         the sigmoid path uses scale 1.0 (:428)."""
         L.act_dtype(hidden_states, "fused_moe")  # bfloat16 or float16; the weights must match
+        if w1_bias is None and w2_bias is None:
+            return run_layer(L.KMOE_FMT_BF16, hidden_states, router_logits, moe_top_k, w1, w2, None, None, scoring_func, True,
+                             num_expert_group, topk_group, 1.0, e_score_correction_bias)[0]
+        # the gpt-oss branch (:433-468): per-expert biases, gate/up interleaved, swigluoai_and_mul
         x = hidden_states.contiguous()
         logits = router_logits.to(torch.float).contiguous()
         out = torch.empty_like(x)
-        extra = {}
-        if w1_bias is not None or w2_bias is not None:
-            # the gpt-oss branch (:433-468): per-expert biases, gate/up interleaved, swigluoai_and_mul
-            extra = dict(w13_bias=None if w1_bias is None else w1_bias.to(torch.bfloat16).contiguous(),
-                         w2_bias=None if w2_bias is None else w2_bias.to(torch.bfloat16).contiguous(),
-                         activation="swigluoai")
         plan = make_moe_plan(L.KMOE_FMT_BF16, x, logits, out, moe_top_k, w1, w2, None, None, scoring_func, True,
-                             num_expert_group, topk_group, 1.0, e_score_correction_bias, **extra)
+                             num_expert_group, topk_group, 1.0, e_score_correction_bias, activation="swigluoai",
+                             w13_bias=None if w1_bias is None else w1_bias.to(torch.bfloat16).contiguous(),
+                             w2_bias=None if w2_bias is None else w2_bias.to(torch.bfloat16).contiguous())
         plan()
         return out
 
@@ -75,10 +75,5 @@ class KunlunOps:
         ep_rank * num_local_experts on (:677-678), and the result is what the pairs routed to them contribute -
         the caller's all-reduce over the ranks makes the layer's output, as in the reference."""
         L.act_dtype(hidden_states, "fused_moe_ep")
-        x = hidden_states.contiguous()
-        logits = router_logits.to(torch.float).contiguous()
-        out = torch.empty_like(x)
-        plan = make_moe_plan(L.KMOE_FMT_BF16, x, logits, out, top_k, w13_weight, w2_weight, None, None, "softmax",
-                             bool(renormalize), first_expert=int(ep_rank) * w13_weight.shape[0])
-        plan()
-        return out
+        return run_layer(L.KMOE_FMT_BF16, hidden_states, router_logits, top_k, w13_weight, w2_weight, None, None, "softmax",
+                         bool(renormalize), first_expert=int(ep_rank) * w13_weight.shape[0])[0]

@@ -8,7 +8,7 @@ KunlunCompressedTensorsW8A8Int8MoEMethod :111-291): `is_monolithic`,
 `apply_monolithic(layer, x, router_logits, ...)`, same argument meaning, same
 exceptions. Where the reference launches nine closed kernels and allocates every
 intermediate per call, `apply_monolithic` here makes ONE call into libkmoe
-(kmoe_moe_forward) on a cached workspace.
+(kmoe_moe_forward) on a cached workspace with a kept argument block.
 """
 from __future__ import annotations
 
@@ -17,7 +17,7 @@ from typing import Optional, Union
 import torch
 
 from ... import _lib as L
-from ..._plan import MoEPlan, make_moe_plan, tile_pair_, tile_w4_scales_
+from ..._plan import MoEPlan, make_moe_plan, run_layer, tile_pair_, tile_w4_scales_
 from ...ops import _custom_ops  # noqa: F401  (torch.ops._C.* used by the staged path)
 
 WNA16_SUPPORTED_BITS = (4, 8)
@@ -153,15 +153,23 @@ class _MonolithicQuantMoE:
         models/deepseek_v2.py:178-184) the gate projection of :275 runs inside the call too."""
         if x.dtype not in (torch.bfloat16, torch.float16):
             raise NotImplementedError(f"apply_monolithic: activations must be bfloat16 or float16, got {x.dtype}")
-        x = x.contiguous()
-        logits = None if router_logits is None else router_logits.float().contiguous()
-        out = torch.empty((x.shape[0], layer.w2_weight.shape[1]), dtype=x.dtype, device=x.device)
-        plan = self.make_plan(layer, x, logits, out, topk_group, num_expert_group, scoring_func,
-                              routed_scaling_factor, e_score_correction_bias, shared_expert, out_scale,
-                              router_weight=router_weight, shared_scale=shared_scale)
-        plan()
-        self.last_layout, self.last_workspace = plan.layout, plan.workspace  # lets tests read the intermediates
+        topk_group, num_expert_group, scoring_func, routed_scaling_factor, bias = self._routing(
+            layer, topk_group, num_expert_group, scoring_func, routed_scaling_factor, e_score_correction_bias)
+        w13 = layer.w13_weight
+        out, self.last_layout, self.last_workspace = run_layer(  # (kept: lets tests read the intermediates)
+            self.FORMAT, x, router_logits, self.moe.experts_per_token, w13, layer.w2_weight, layer.w13_weight_scale,
+            layer.w2_weight_scale, scoring_func, True, num_expert_group, topk_group, routed_scaling_factor, bias,
+            shared_expert, out_scale, router_weight, None, shared_scale,
+            self._first_expert(w13, router_logits, router_weight), bool(self.side_stream))
         return out
+
+    # Under expert parallelism the layer holds the experts of one rank while the logits (or the router weight)
+    # run over all of them: the rank's share, as KunlunOps.fused_moe_ep computes it for the unquantized layer
+    # (ops/_kunlun_ops.py:677-689). The reference's own quantized path takes the local experts for all (:135).
+    def _first_expert(self, w13, logits, router_weight) -> int:
+        E = w13.shape[0]
+        routed = logits.shape[-1] if logits is not None else (E if router_weight is None else router_weight.shape[0])
+        return int(getattr(self.moe, "ep_rank", 0) or 0) * E if routed > E else 0
 
     def make_plan(self, layer, x, logits, out, topk_group=None, num_expert_group=None, scoring_func="softmax",
                   routed_scaling_factor=1.0, e_score_correction_bias=None, shared_expert=None, out_scale=1.0,
@@ -171,12 +179,7 @@ class _MonolithicQuantMoE:
         capture replays without touching Python-side allocation."""
         topk_group, num_expert_group, scoring_func, routed_scaling_factor, bias = self._routing(
             layer, topk_group, num_expert_group, scoring_func, routed_scaling_factor, e_score_correction_bias)
-        # Under expert parallelism the layer holds the experts of one rank while the logits (or the router weight)
-        # run over all of them: the rank's share, as KunlunOps.fused_moe_ep computes it for the unquantized layer
-        # (ops/_kunlun_ops.py:677-689). The reference's own quantized path takes the local experts for all (:135).
-        E = layer.w13_weight.shape[0]
-        routed = logits.shape[-1] if logits is not None else router_weight.shape[0]
-        first = int(getattr(self.moe, "ep_rank", 0) or 0) * E if routed > E else 0
+        first = self._first_expert(layer.w13_weight, logits, router_weight)
         return make_moe_plan(self.FORMAT, x, logits, out, self.moe.experts_per_token, layer.w13_weight,
                              layer.w2_weight, layer.w13_weight_scale, layer.w2_weight_scale, scoring_func,
                              True,  # the reference always routes with the *_norm kernels
@@ -474,15 +477,11 @@ class KunlunCompressedTensorsWNA16MoEMethod:
             if x.dtype != layer.w13_weight_scale.dtype:
                 raise ValueError(f"4-bit MoE: activations ({x.dtype}) must have the dtype of the scales "
                                  f"({layer.w13_weight_scale.dtype})")
-            xc = x.contiguous()
-            out = torch.empty_like(xc)
-            gs = self.group_size or 2 * layer.w13_weight_packed.shape[-1]
-            plan = make_moe_plan(L.KMOE_FMT_W4A16, xc, router_logits.to(torch.float).contiguous(), out, top_k,
-                                 layer.w13_weight_packed, layer.w2_weight_packed, layer.w13_weight_scale,
-                                 layer.w2_weight_scale, scoring_func, renormalize, num_expert_group, topk_group, 1.0,
-                                 e_score_correction_bias, group_size=gs, first_expert=(ep_rank or 0) * E)
-            plan()
-            return out
+            packed = layer.w13_weight_packed
+            return run_layer(L.KMOE_FMT_W4A16, x, router_logits, top_k, packed, layer.w2_weight_packed,
+                             layer.w13_weight_scale, layer.w2_weight_scale, scoring_func, renormalize, num_expert_group,
+                             topk_group, 1.0, e_score_correction_bias, group_size=self.group_size or 2 * packed.shape[-1],
+                             first_expert=(ep_rank or 0) * E)[0]
         if not hasattr(layer, "w13_weight"):
             raise NotImplementedError("4-bit MoE: expert biases need the unpacked copy (native='both' or False)")
         from ...ops._kunlun_ops import KunlunOps as ops
