@@ -436,8 +436,8 @@ def main():
                          "14: one 8-wave tile of 192 rows per workgroup)")
     ap.add_argument("--one-stream", action="store_true",
                     help="keep every launch on the one stream (the C ABI's default). Without it the layer is called with "
-                         "KMOE_FLAG_SIDE_STREAM: a shared expert that cannot ride in the routed launches (the fp8 layers at "
-                         "decode sizes) runs on the library's second stream beside them; config.side_stream says which")
+                         "KMOE_FLAG_SIDE_STREAM: a shared expert that cannot ride in the routed launches (another "
+                         "width) runs on the library's second stream beside them; config.side_stream says which")
     ap.add_argument("--yardstick", action="store_true",
                     help="also time the vendor library's dense GEMM (torch._int_mm / bf16 matmul) with the gate_up "
                          "GEMM's operation count: [P,H] x [H,2I], one weight matrix, no gather, no epilogue")

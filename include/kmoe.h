@@ -635,7 +635,7 @@ typedef struct kmoe_moe_args {
 
 /* kmoe_moe_args.flags.
  * KMOE_FLAG_SIDE_STREAM: a shared expert that cannot ride in the routed launches (a width other than the routed
- * experts'; the fp8 layer at decode sizes) may run on a second stream of the library's own (one per GPU, default
+ * experts') may run on a second stream of the library's own (one per GPU, default
  * priority, non-blocking, created by the first such call that is not being captured), forked from `stream` by an
  * event after the first quantisation and joined back by an event before the combine: the caller still sees one
  * stream's worth of ordering, and under capture the fork and join become graph edges. Without the flag (the default)
@@ -648,13 +648,12 @@ typedef struct kmoe_moe_args {
  * conversion. */
 #define KMOE_FLAG_LOGITS_ACT_DTYPE 2
 
-/* Decode-sized int8 batches (at most 10 rows per expert, tiled weights): two of the layer's small launches are folded
- * into the GEMM launches. The gate_up launch sorts the routed pairs by expert itself (every workgroup scans the pairs'
- * expert ids; up to 4096 pairs and 512 tokens, one GPU holding every expert) and writes moe_index, sorted_src,
- * expert_m and lod as the sort's launch would (so does the gate_up launch of KMOE_FMT_W4A16 where it runs on that
- * format's streaming kernel); the down launch quantises its rows itself (rows up to 1024 values)
- * and writes actq and actmax as the quantiser's launch would. Same bits, same workspace contents, two launches
- * fewer; KMOE_STAGE_ALIGN / KMOE_STAGE_QUANT2 then bracket nothing. The environment variables KMOE_SORT_IN_GEMM=0
+/* Decode-sized batches (at most 10 rows per expert, tiled weights) run both GEMMs on the weight-streaming kernel, and
+ * small launches of the layer are folded into them. The gate_up launch sorts the routed pairs by expert itself (every
+ * workgroup scans the pairs' expert ids; up to 4096 pairs and 512 tokens, one GPU holding every expert) and writes
+ * moe_index, sorted_src, expert_m and lod as the sort's launch would; the down launch of int8 layers quantises its rows
+ * itself (rows up to 1024 values) and writes actq and actmax as the quantiser's launch would. Same bits, same workspace
+ * contents, two launches fewer; KMOE_STAGE_ALIGN / KMOE_STAGE_QUANT2 then bracket nothing. The environment variables KMOE_SORT_IN_GEMM=0
  * and KMOE_QUANT_IN_GEMM=0 (read once per process) keep the launches apart: for measurements. */
 
 #define KMOE_STAGE_ROUTING 0

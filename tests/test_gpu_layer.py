@@ -419,3 +419,33 @@ def test_int8_layer_as_an_expert_parallel_share(M, scoring):
         out2 = method.apply_monolithic(layer, x.cuda(), logits.cuda(), **kw)
         torch.cuda.synchronize()
         assert torch.equal(out2, out)
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8", "none"])
+@pytest.mark.parametrize("M,E,K", [(1, 16, 8), (1, 9, 8), (3, 64, 8), (7, 64, 8), (8, 64, 8), (31, 256, 8), (32, 257, 8),
+                                   (33, 300, 8), (63, 512, 4), (5, 1000, 16)])
+def test_decode_launches_with_a_column_per_pair(fmt, M, E, K):
+    """Batches with fewer routed pairs than experts give the streaming launches a column of workgroups per pair (up to
+    256 pairs): the layer's results, and the sort it leaves, around that switch - a token's result does not depend on
+    the batch it travels in, so each batch is compared with the same tokens inside one that has a column per expert."""
+    from vllm_kunlun_amd import synth
+    big = M + E // K + 2
+    shape = synth.scaled(synth.SHAPES["qwen3-decode"], M=big, H=256, E=E, K=K, I=128, quant=fmt)
+    sl = synth.make_layer(shape, "cuda", seed=M + E)
+    sl.logits[:, 3] += 1.5  # an expert that several tokens share
+    whole = sl.layer(sl.x, sl.logits)
+    part = sl.layer(sl.x[:M], sl.logits[:M])
+    if fmt == "int8":
+        m = sl.layer.quant_method
+        P = M * K
+        ids = _view(m.last_workspace, m.last_layout.topk_ids, P, torch.int32).cpu().numpy()
+        order = np.argsort(ids, kind="stable")
+        counts = np.bincount(ids, minlength=E)
+        for name, want in (("sorted_src", order), ("moe_index", np.argsort(order)), ("expert_m", counts),
+                           ("lod", np.concatenate([[0], np.cumsum(counts)]))):
+            got = _view(m.last_workspace, getattr(m.last_layout, name), len(want), torch.int32).cpu().numpy()
+            assert np.array_equal(got, want), name
+    if fmt == "none" or fmt == "fp8":  # (the same products; fp8 and bf16 sums may be split over K differently)
+        assert rel_l2(part, whole[:M]) <= 2e-3
+    else:
+        assert torch.equal(part, whole[:M])

@@ -1,5 +1,6 @@
 // Host side of libkmoe: error state, and the fused layer call that strings the
 // stage kernels together on one stream out of one caller-owned workspace.
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -146,15 +147,24 @@ bool use_stream_path(const kmoe_moe_args* a) {
 // A shared expert of the routed experts' width runs inside the routed GEMM launches
 // as one more ("tail") expert over rows [P, P+M): no extra launches, and its few
 // workgroups overlap the routed experts' instead of leaving most CUs idle.
-// fp8: only where the routed experts run on the tile kernel (more than 10 rows per expert). With fewer
-// rows the routed launch uses the 16-row LDS-staged kernel, which would stream the tail expert's weights once
-// per 16 token rows (measured at 128 tokens: gate_up +260 us against 57 us for a launch of its own).
 bool fold_shared(const kmoe_moe_args* a) {
   if (a->I_shared <= 0 || a->I_shared != a->I || a->ws_layout != a->w_layout) return false;
   if (a->format == KMOE_FMT_INT8) return true;
-  const long long P = local_pairs(a);
-  return a->format == KMOE_FMT_FP8_BLOCK && a->w_layout == KMOE_W_TILED && a->H <= 8192 && a->I <= 8192 &&
-         (P + a->E - 1) / a->E > 10;
+  return a->format == KMOE_FMT_FP8_BLOCK && a->w_layout == KMOE_W_TILED && a->H <= 8192 && a->I <= 8192;
+}
+
+// Whether both routed GEMMs run on the weight-streaming kernel (the packed 4-bit format has one of its own).
+bool routed_streams(const kmoe_moe_args* a) {
+  if (a->w_layout != KMOE_W_TILED) return false;
+  const long long rows = local_pairs(a);
+  switch (a->format) {
+    case KMOE_FMT_INT8: return use_stream_path(a);
+    case KMOE_FMT_FP8_BLOCK: return streams_fp8(static_cast<int>(rows), a->E, a->H) && streams_fp8(static_cast<int>(rows), a->E, a->I);
+    case KMOE_FMT_BF16:
+      return streams_bf16(static_cast<int>(rows), a->E, a->H) && streams_bf16(static_cast<int>(rows), a->E, a->I) &&
+             !a->w13_bias && !a->w2_bias && a->activation != KMOE_ACT_SWIGLUOAI;
+    default: return w4_gate_up_streams(a->M * a->K, 0, a->E, a->H);
+  }
 }
 
 // One expert-MLP pass (gate_up + SiLU-mul, requantise, down) over `rows` rows in
@@ -191,9 +201,10 @@ struct MlpPass {
   int group_size, scale_layout;
   int variant;  // INT8: kernel variant of the two GEMMs (0: from the shape)
   int act_dtype;  // INT8, BF16: KMOE_DT_* of x_rows' source, act and out (BF16: of the weights too)
-  // INT8 weight-streaming path: the gate_up launch sorts the routed pairs itself (row_src is then NULL and lod is
-  // what that launch writes)
+  // weight-streaming path: the gate_up launch sorts the routed pairs itself (row_src is then NULL and lod is
+  // what that launch writes); slots: the down launch has a column of workgroups per pair, as the gate_up launch had
   const StreamScan* scan;
+  const StreamSlots* slots;
   bool quant_in_gemm;  // the down launch quantises its rows itself: no launch between the two GEMMs
 };
 
@@ -242,7 +253,8 @@ int run_gemm(const MlpPass& m, bool first, kmoe_stream_t stream) {
       g.tail_src0 = first ? 0 : m.rows;  // gate_up reads token rows, down reads its own act rows
     }
     const StreamQuant quant{m.act, m.I, static_cast<int8_t*>(m.actq), m.act_aux};
-    return grouped_gemm_i8_checked(&g, stream, first ? m.scan : nullptr, !first && m.quant_in_gemm ? &quant : nullptr);
+    return grouped_gemm_i8_checked(&g, stream, first ? m.scan : nullptr, !first && m.quant_in_gemm ? &quant : nullptr,
+                                   first ? nullptr : m.slots);
   }
   if (m.format == KMOE_FMT_FP8_BLOCK) {
     kmoe_gemm_fp8_args g = {};
@@ -272,7 +284,7 @@ int run_gemm(const MlpPass& m, bool first, kmoe_stream_t stream) {
       g.tail_rows = m.tail_rows;
       g.tail_src0 = first ? 0 : m.rows;  // gate_up reads token rows, down reads its own act rows
     }
-    return kmoe_grouped_gemm_fp8_block(&g, stream);
+    return grouped_gemm_fp8_checked(&g, stream, first ? m.scan : nullptr, first ? nullptr : m.slots);
   }
   if (m.format == KMOE_FMT_W4A16) {
     kmoe_gemm_w4_args g = {};
@@ -317,7 +329,7 @@ int run_gemm(const MlpPass& m, bool first, kmoe_stream_t stream) {
   g.act_alpha = m.act_alpha;
   g.act_limit = m.act_limit;
   g.act_dtype = m.act_dtype;
-  return kmoe_grouped_gemm_bf16(&g, stream);
+  return grouped_gemm_bf16_checked(&g, stream, first ? m.scan : nullptr, first ? nullptr : m.slots);
 }
 
 template <class Mark>
@@ -375,7 +387,8 @@ extern "C" int kmoe_moe_workspace_layout(const kmoe_moe_args* a, kmoe_moe_layout
   L->sorted_src = take(P * 4);
   L->expert_m = take(E * 4);
   L->lod = take((E + 1) * 4);
-  L->align_ws = take(kmoe_align_workspace_bytes(static_cast<int>(P), a->E));
+  // (launches with a column of workgroups per pair keep their row ranges where the sort's launch would have its own)
+  L->align_ws = take(std::max(kmoe_align_workspace_bytes(static_cast<int>(P), a->E), P <= kStreamSlotMaxPairs ? P * sizeof(int2) : 0));
   L->xq = take(quant ? M * H : 0);
   L->xmax = take(quant ? M * 4 * (fp8 ? H / 128 : 1) : 0);
   L->act = take(R * I * 2);
@@ -535,11 +548,13 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   // launch does it in its prologue and writes the same four arrays: one launch and its round trips less
   // (Qwen3 decode: 4.8 us of 125). Not for an expert-parallel share (pairs of other ranks' experts get no row).
   mark(KMOE_STAGE_ALIGN, 0);
-  const StreamScan scan{topk_ids, P, lod, static_cast<int32_t*>(at(L.expert_m)), moe_index, sorted_src};
-  const bool streams = stream_mode || (a->format == KMOE_FMT_W4A16 && a->w_layout == KMOE_W_TILED &&
-                                       w4_gate_up_streams(P, 0, E, H));
-  const bool scan_in_gemm = streams && Eg == E && a->first_expert == 0 && P <= kStreamScanMaxPairs &&
+  const bool scan_in_gemm = routed_streams(a) && Eg == E && a->first_expert == 0 && P <= kStreamScanMaxPairs &&
                             M <= kStreamScanMaxRows && scan_allowed();
+  // Fewer pairs than experts: a column of workgroups per pair instead of per expert.
+  const bool per_pair = scan_in_gemm && a->format != KMOE_FMT_W4A16 && P < E && P <= kStreamSlotMaxPairs;
+  int2* slot_rows = per_pair ? static_cast<int2*>(at(L.align_ws)) : nullptr;
+  const StreamScan scan{topk_ids, P, lod, static_cast<int32_t*>(at(L.expert_m)), moe_index, sorted_src, slot_rows};
+  const StreamSlots slots{topk_ids, slot_rows, P};
   if (!scan_in_gemm) {
     rc = kmoe_align_local(topk_ids, P, E, a->first_expert, moe_index, sorted_src, static_cast<int32_t*>(at(L.expert_m)), lod,
                           at(L.align_ws), kmoe_align_workspace_bytes(P, E), stream);
@@ -572,6 +587,7 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   routed.x_aux = quant ? static_cast<const float*>(at(L.xmax)) : nullptr;
   routed.row_src = scan_in_gemm ? nullptr : sorted_src;
   routed.scan = scan_in_gemm ? &scan : nullptr;
+  routed.slots = per_pair ? &slots : nullptr;
   routed.src_div = K;
   routed.w13 = a->w13;
   routed.w2 = a->w2;
@@ -639,6 +655,7 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
     sh.tail_rows = 0;
     sh.row_src = nullptr;
     sh.scan = nullptr;
+    sh.slots = nullptr;
     sh.quant_in_gemm = false;
     sh.src_div = 1;
     sh.w13 = a->ws13;

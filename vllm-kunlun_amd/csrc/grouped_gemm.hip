@@ -416,7 +416,7 @@ int launch(const GemmParams& p, int rows, hipStream_t s, const char* what) {
 // Tiled weights: from this many rows per expert (on average) the persistent 128-row-tile kernel wins over
 // the 16/32/64-row kernels of this file although most of its tile is padding: its weight stream is asynchronous
 // and it is bound by the weight bytes either way (measured cross-over: 8 to 16 rows, all three formats).
-constexpr int kTiledMinRows = 10;
+constexpr int kTiledMinRows = kStreamMaxRows;
 // variants of the bf16 and fp8 launchers that force the tile kernel: 5 (tile height from the rows per expert),
 // 6 (128-row tiles), 11 (64-row tiles)
 inline bool tile_variant(int v) { return v == 5 || v == 6 || (v >= 11 && v <= 13); }
@@ -448,7 +448,7 @@ bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p
 }  // namespace
 
 int grouped_gemm_i8_checked(const kmoe_gemm_i8_args* a, kmoe_stream_t stream, const StreamScan* scan,
-                            const StreamQuant* quant) {
+                            const StreamQuant* quant, const StreamSlots* slots) {
   KMOE_REQUIRE(a, KMOE_ERR_NULL, "grouped_gemm_i8: args is NULL");
   KMOE_REQUIRE(a->a && a->a_max && a->w && a->w_max && (a->lod || scan) && a->y, KMOE_ERR_NULL,
                "grouped_gemm_i8: NULL tensor pointer");
@@ -481,7 +481,7 @@ int grouped_gemm_i8_checked(const kmoe_gemm_i8_args* a, kmoe_stream_t stream, co
                  "grouped_gemm_i8: chunked activations need tiled weights");
     KMOE_REQUIRE(a->a_rows >= 1, KMOE_ERR_SHAPE, "grouped_gemm_i8: a_rows=%d < 1", a->a_rows);
     if (a->rows == 0 && !(a->w_tail && a->tail_rows > 0) && !scan) return KMOE_OK;
-    return stream_gemm_i8(a, as_stream(stream), scan, quant);
+    return stream_gemm_i8(a, as_stream(stream), scan, quant, slots);
   }
   KMOE_REQUIRE(!scan && !quant, KMOE_ERR_UNSUPPORTED,
                "grouped_gemm_i8: only the weight-streaming kernel sorts the pairs or quantises its rows itself");
@@ -501,17 +501,10 @@ int grouped_gemm_i8_checked(const kmoe_gemm_i8_args* a, kmoe_stream_t stream, co
   return dispatch<Kind::I8>(p, a->rows, expected_rows(a->rows, a->rows_hint), swiglu, a->variant, as_stream(stream), "kmoe_grouped_gemm_i8");
 }
 
-}  // namespace kmoe
-
-using namespace kmoe;
-
-extern "C" int kmoe_grouped_gemm_i8(const kmoe_gemm_i8_args* a, kmoe_stream_t stream) {
-  return grouped_gemm_i8_checked(a, stream, nullptr);
-}
-
-extern "C" int kmoe_grouped_gemm_bf16(const kmoe_gemm_bf16_args* a, kmoe_stream_t stream) {
+int grouped_gemm_bf16_checked(const kmoe_gemm_bf16_args* a, kmoe_stream_t stream, const StreamScan* scan,
+                              const StreamSlots* slots) {
   KMOE_REQUIRE(a, KMOE_ERR_NULL, "grouped_gemm_bf16: args is NULL");
-  KMOE_REQUIRE(a->a && a->w && a->lod && a->y, KMOE_ERR_NULL, "grouped_gemm_bf16: NULL tensor pointer");
+  KMOE_REQUIRE(a->a && a->w && (a->lod || scan) && a->y, KMOE_ERR_NULL, "grouped_gemm_bf16: NULL tensor pointer");
   KMOE_REQUIRE(a->E >= 1 && a->n >= 16 && a->k >= 8 && a->rows >= 0, KMOE_ERR_SHAPE,
                "grouped_gemm_bf16: E=%d n=%d k=%d rows=%d", a->E, a->n, a->k, a->rows);
   KMOE_REQUIRE(a->k % 8 == 0, KMOE_ERR_SHAPE, "grouped_gemm_bf16: k=%d must be a multiple of 8", a->k);
@@ -539,23 +532,28 @@ extern "C" int kmoe_grouped_gemm_bf16(const kmoe_gemm_bf16_args* a, kmoe_stream_
   if (a->rows == 0) return KMOE_OK;
   KMOE_REQUIRE(a->w_layout == KMOE_W_ROWMAJOR || (a->w_layout == KMOE_W_TILED && a->k % 32 == 0), KMOE_ERR_SHAPE,
                "grouped_gemm_bf16: w_layout=%d (tiled weights need k %% 32 == 0, k=%d)", a->w_layout, a->k);
-  // tiled weights and more than a few rows per expert: the persistent tile kernel (variants 5, 6, 11 force it)
+  const int live = expected_rows(a->rows, a->rows_hint);
+  // tiled weights and a few rows per expert: the weight-streaming kernel
+  if (a->w_layout == KMOE_W_TILED && a->variant == 0 && !a->bias && !oai && streams_bf16(live, a->E, a->k))
+    return stream_gemm_bf16(a, as_stream(stream), scan, slots);
+  KMOE_REQUIRE(!scan && !slots, KMOE_ERR_UNSUPPORTED, "grouped_gemm_bf16: only the weight-streaming kernel sorts the pairs itself");
+  // tiled weights and more rows: the persistent tile kernel (variants 5, 6, 11 force it)
   if (a->w_layout == KMOE_W_TILED && a->k >= 64 && a->ldy % 8 == 0 &&
-      (tile_variant(a->variant) || (a->variant == 0 && ceil_div(expected_rows(a->rows, a->rows_hint), a->E) > kTiledMinRows)))
+      (tile_variant(a->variant) || (a->variant == 0 && ceil_div(live, a->E) > kTiledMinRows)))
     return tiled_gemm_bf16(a, as_stream(stream));
   KMOE_REQUIRE(!tile_variant(a->variant), KMOE_ERR_UNSUPPORTED, "grouped_gemm_bf16: variants 5, 6, 11-13 need tiled weights, k >= 64 and ldy %% 8 == 0");
   GemmParams p{reinterpret_cast<const int8_t*>(a->a), a->lda * 2, nullptr, a->row_src, a->src_div,
                reinterpret_cast<const int8_t*>(a->w), nullptr,    a->lod,  a->E,       a->n,
                a->k * 2,                              a->y,       a->ldy,  nullptr, a->w_layout == KMOE_W_TILED,
                nullptr, nullptr, 0, 0, 0, a->bias, oai ? 1 : 0, a->act_alpha, a->act_limit};
-  const int live = expected_rows(a->rows, a->rows_hint);
   if (half) return dispatch<Kind::F16>(p, a->rows, live, swiglu, a->variant, as_stream(stream), "kmoe_grouped_gemm_bf16 (half)");
   return dispatch<Kind::BF16>(p, a->rows, live, swiglu, a->variant, as_stream(stream), "kmoe_grouped_gemm_bf16");
 }
 
-extern "C" int kmoe_grouped_gemm_fp8_block(const kmoe_gemm_fp8_args* a, kmoe_stream_t stream) {
+int grouped_gemm_fp8_checked(const kmoe_gemm_fp8_args* a, kmoe_stream_t stream, const StreamScan* scan,
+                             const StreamSlots* slots) {
   KMOE_REQUIRE(a, KMOE_ERR_NULL, "grouped_gemm_fp8_block: args is NULL");
-  KMOE_REQUIRE(a->a && a->a_scale && a->w && a->w_scale && a->lod && a->y, KMOE_ERR_NULL,
+  KMOE_REQUIRE(a->a && a->a_scale && a->w && a->w_scale && (a->lod || scan) && a->y, KMOE_ERR_NULL,
                "grouped_gemm_fp8_block: NULL tensor pointer");
   KMOE_REQUIRE(a->E >= 1 && a->n >= 128 && a->k >= 128 && a->rows >= 0, KMOE_ERR_SHAPE,
                "grouped_gemm_fp8_block: E=%d n=%d k=%d rows=%d", a->E, a->n, a->k, a->rows);
@@ -582,10 +580,15 @@ extern "C" int kmoe_grouped_gemm_fp8_block(const kmoe_gemm_fp8_args* a, kmoe_str
   if (a->rows == 0 && tail_rows == 0) return KMOE_OK;
   KMOE_REQUIRE(a->w_layout == KMOE_W_ROWMAJOR || a->w_layout == KMOE_W_TILED, KMOE_ERR_UNSUPPORTED,
                "grouped_gemm_fp8_block: w_layout=%d unknown", a->w_layout);
-  // tiled weights and more than a few rows per expert: the persistent tile kernel (variants 5, 6, 11 force it)
+  const int live = expected_rows(a->rows, a->rows_hint);
+  // tiled weights and a few rows per expert: the weight-streaming kernel
+  if (a->w_layout == KMOE_W_TILED && a->variant == 0 && streams_fp8(live, a->E, a->k))
+    return stream_gemm_fp8(a, as_stream(stream), scan, slots);
+  KMOE_REQUIRE(!scan && !slots, KMOE_ERR_UNSUPPORTED, "grouped_gemm_fp8_block: only the weight-streaming kernel sorts the pairs itself");
+  // tiled weights and more rows: the persistent tile kernel (variants 5, 6, 11 force it)
   const bool tall_variant = a->variant == 8 || a->variant == 14 || (a->variant >= 17 && a->variant <= 19);  // 8-wave tiles of 256 / 192 rows; 17: chosen on the device; 18, 19: wide 192- / 128-row tiles
   if (a->w_layout == KMOE_W_TILED && a->k <= 8192 && a->ldy % 8 == 0 &&
-      (tile_variant(a->variant) || tall_variant || (a->variant == 0 && ceil_div(expected_rows(a->rows, a->rows_hint), a->E) > kTiledMinRows)))
+      (tile_variant(a->variant) || tall_variant || (a->variant == 0 && ceil_div(live, a->E) > kTiledMinRows)))
     return tiled_gemm_fp8(a, as_stream(stream));
   KMOE_REQUIRE(!tile_variant(a->variant) && !tall_variant, KMOE_ERR_UNSUPPORTED,
                "grouped_gemm_fp8_block: variants 5, 6, 8, 11-14 need tiled weights, k <= 8192");
@@ -594,5 +597,21 @@ extern "C" int kmoe_grouped_gemm_fp8_block(const kmoe_gemm_fp8_args* a, kmoe_str
                a->k,                                  a->y,       a->ldy,  nullptr, a->w_layout == KMOE_W_TILED,
                reinterpret_cast<const int8_t*>(a->w_tail), a->w_scale_tail, a->tail_row0, tail_rows, a->tail_src0,
                nullptr, 0, 0.f, 0.f, a->act_dtype == KMOE_DT_F16};
-  return dispatch<Kind::FP8>(p, a->rows, expected_rows(a->rows, a->rows_hint), swiglu, a->variant, as_stream(stream), "kmoe_grouped_gemm_fp8_block");
+  return dispatch<Kind::FP8>(p, a->rows, live, swiglu, a->variant, as_stream(stream), "kmoe_grouped_gemm_fp8_block");
+}
+
+}  // namespace kmoe
+
+using namespace kmoe;
+
+extern "C" int kmoe_grouped_gemm_i8(const kmoe_gemm_i8_args* a, kmoe_stream_t stream) {
+  return grouped_gemm_i8_checked(a, stream, nullptr, nullptr, nullptr);
+}
+
+extern "C" int kmoe_grouped_gemm_bf16(const kmoe_gemm_bf16_args* a, kmoe_stream_t stream) {
+  return grouped_gemm_bf16_checked(a, stream, nullptr, nullptr);
+}
+
+extern "C" int kmoe_grouped_gemm_fp8_block(const kmoe_gemm_fp8_args* a, kmoe_stream_t stream) {
+  return grouped_gemm_fp8_checked(a, stream, nullptr, nullptr);
 }

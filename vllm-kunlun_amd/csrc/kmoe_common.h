@@ -13,6 +13,7 @@ namespace kmoe {
 inline int expected_rows(int rows, int hint) { return hint > 0 && hint < rows ? hint : rows; }
 
 constexpr int kWave = 64;
+inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // ---- error plumbing (host) -------------------------------------------------
 int fail(int code, const char* fmt, ...);
@@ -34,7 +35,15 @@ struct StreamScan {
   int32_t* expert_m;
   int32_t* moe_index;
   int32_t* sorted_src;
+  int2* slot_rows;  // NULL, or [n_pairs]: a launch with a column of workgroups per pair (pair_scan.h, slots)
 };
+// The layer's down launch of a batch of few tokens, where the gate_up launch filled slot_rows: columns as there.
+struct StreamSlots {
+  const int32_t* ids;
+  const int2* rows;
+  int32_t n;  // 0: a column per expert
+};
+constexpr int kStreamSlotMaxPairs = 256;
 constexpr int kStreamScanMaxPairs = 4096;
 constexpr int kStreamScanMaxRows = 512;  // tokens: no expert gets more rows than that
 // With `quant` (the layer's down launch at decode sizes, k <= kStreamQuantMaxK) the launch quantises its rows
@@ -47,11 +56,23 @@ struct StreamQuant {
   float* amax;
 };
 constexpr int kStreamQuantMaxK = 1024;
-int stream_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream, const StreamScan* scan = nullptr,
-                   const StreamQuant* quant = nullptr);
-// kmoe_grouped_gemm_i8 with the options above for the layer's own launches.
+int stream_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream, const StreamScan* scan, const StreamQuant* quant,
+                   const StreamSlots* slots);
+// The same kernel on fp8 block-scaled and on 16-bit weights (tiled; row-major activations).
+int stream_gemm_fp8(const kmoe_gemm_fp8_args* args, hipStream_t stream, const StreamScan* scan, const StreamSlots* slots);
+int stream_gemm_bf16(const kmoe_gemm_bf16_args* args, hipStream_t stream, const StreamScan* scan, const StreamSlots* slots);
+// kmoe_grouped_gemm_* with the options above for the layer's own launches.
 int grouped_gemm_i8_checked(const kmoe_gemm_i8_args* args, kmoe_stream_t stream, const StreamScan* scan,
-                            const StreamQuant* quant = nullptr);
+                            const StreamQuant* quant, const StreamSlots* slots);
+int grouped_gemm_fp8_checked(const kmoe_gemm_fp8_args* args, kmoe_stream_t stream, const StreamScan* scan,
+                             const StreamSlots* slots);
+int grouped_gemm_bf16_checked(const kmoe_gemm_bf16_args* args, kmoe_stream_t stream, const StreamScan* scan,
+                              const StreamSlots* slots);
+// Whether a launch of these dimensions on tiled weights and without a variant runs on the weight-streaming kernel:
+// up to 10 rows per expert (the tile kernel's cross-over, measured for all formats), rows of the lengths it takes.
+constexpr int kStreamMaxRows = 10;
+inline bool streams_fp8(int live_rows, int E, int k) { return ceil_div(live_rows, E) <= kStreamMaxRows && k <= 8192; }
+inline bool streams_bf16(int live_rows, int E, int k) { return ceil_div(live_rows, E) <= kStreamMaxRows && k % 32 == 0; }
 // kmoe_grouped_gemm_w4a16 with `scan` for the layer's routed gate_up launch where it runs on the streaming kernel
 // (w4_gate_up_streams says whether a launch of these dimensions does).
 int grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* args, kmoe_stream_t stream, const StreamScan* scan);
@@ -233,7 +254,6 @@ __device__ inline uint64_t lanemask_lt() {
 
 inline hipStream_t as_stream(kmoe_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
-inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 }  // namespace kmoe

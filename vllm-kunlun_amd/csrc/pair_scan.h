@@ -14,7 +14,7 @@ constexpr int kScanWaves = 4;  // waves of the workgroups that scan
 constexpr int kScanBatch = 4;  // expert ids a lane asks for before it waits (a workgroup: one round trip per 1024 pairs)
 
 struct PairScanLds {
-  int list[kScanWaves][kStreamScanMaxRows];  // per quarter of the ids: the pairs of the expert, ascending
+  __attribute__((aligned(16))) int list[kScanWaves][kStreamScanMaxRows];  // per quarter of the ids: the pairs of the expert, ascending
   int cnt[kScanWaves], below[kScanWaves];
 };
 
@@ -40,8 +40,14 @@ struct ListedRows {
   }
 };
 
-// Called by all kScanWaves waves of the workgroup (one barrier inside). `publish`: this workgroup writes lod[e],
-// expert_m[e], (for the last expert) lod[E], and moe_index / sorted_src of the expert's pairs.
+// Called by all kScanWaves waves of the workgroup (one barrier inside). `publish`: this workgroup writes moe_index /
+// sorted_src of the expert's pairs and, where the launch has a workgroup column per expert (no slots), lod[e],
+// expert_m[e] and (for the last expert) lod[E].
+//
+// Slots (StreamScan::slot_rows): a batch of a few tokens hits few experts, and a launch with a column of workgroups
+// per expert is mostly columns that find nothing to do. Such a launch has a column per PAIR instead: column j serves
+// the expert of pair j if j is the first pair that chose it, and leaves the expert's rows in slot_rows[j] (no rows
+// otherwise) for the down launch, whose columns are the same. publish_lod writes lod and expert_m there.
 __device__ inline ListedRows scan_pairs(const StreamScan& sc, int e, int E, PairScanLds& s, bool publish) {
   const int lane = lane_id();
   const int wave_id = threadIdx.x >> 6;
@@ -84,7 +90,7 @@ __device__ inline ListedRows scan_pairs(const StreamScan& sc, int e, int E, Pair
   r.begin = s.below[0] + s.below[1] + s.below[2] + s.below[3];
   r.end = r.begin + cnt;
   if (publish && wave_id == 0) {
-    if (lane == 0) {
+    if (lane == 0 && !sc.slot_rows) {
       sc.lod[e] = r.begin;
       sc.expert_m[e] = cnt;
       if (e == E - 1) sc.lod[E] = r.end;
@@ -96,6 +102,26 @@ __device__ inline ListedRows scan_pairs(const StreamScan& sc, int e, int E, Pair
     }
   }
   return r;
+}
+
+// lod and expert_m of every expert, by one workgroup of kScanWaves waves (launches with slots: at most
+// kStreamSlotMaxPairs pairs, one per thread).
+__device__ inline void publish_lod(const StreamScan& sc, int E, PairScanLds& s) {
+  static_assert(kStreamSlotMaxPairs == kScanWaves * kWave && kStreamSlotMaxPairs <= kStreamScanMaxRows, "one id per thread");
+  int* ids = s.list[0];
+  ids[threadIdx.x] = static_cast<int>(threadIdx.x) < sc.n_pairs ? sc.ids[threadIdx.x] : 0x7fffffff;
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += kScanWaves * kWave) {
+    int below = 0, cnt = 0;
+    for (int j = 0; j < sc.n_pairs; j += 4) {  // (the ids past the last pair count for no expert)
+      const int4 id = *reinterpret_cast<const int4*>(ids + j);
+      below += (id.x < e) + (id.y < e) + (id.z < e) + (id.w < e);
+      cnt += (id.x == e) + (id.y == e) + (id.z == e) + (id.w == e);
+    }
+    sc.lod[e] = below;
+    sc.expert_m[e] = cnt;
+    if (e == E - 1) sc.lod[E] = below + cnt;
+  }
 }
 
 }  // namespace kmoe

@@ -1,20 +1,22 @@
-// Weight-streaming W8A8 grouped GEMM for the decode regime (a handful of rows
-// per expert): HBM-bound, every weight byte is read once, MFMA is ~5% busy.
+// Weight-streaming grouped GEMM for the decode regime (a handful of rows per expert), on int8 (W8A8), fp8-e4m3
+// (128x128 / 1x128 block scales), bf16 and half weights: HBM-bound, every weight byte is read once, MFMA is ~5% busy.
 //
-// Both operands arrive already arranged for v_mfma_i32_16x16x64_i8, so a wave
-// needs no LDS, no barrier and no address arithmetic beyond a stride:
-//   weights  "tiled": [E][n/16][k/64] blocks of 1 KB; inside a block byte
-//            256*g + 16*c + t is channel c (of 16), k = 16*g + t (g = 0..3) —
+// A wave needs no LDS, no barrier and no address arithmetic beyond a stride in its main loop:
+//   weights  "tiled": [E][n/16][k bytes/64] blocks of 1 KB; inside a block byte
+//            256*g + 16*c + t is channel c (of 16), byte 16*g + t of the block's 64 bytes of K (g = 0..3) —
 //            i.e. exactly what lane 16*g + c feeds the MFMA. A wave reads 1 KB
-//            of consecutive bytes per MFMA step and the next step's block follows
-//            directly: one long sequential stream per 16 output channels.
-//   activations "chunk-major": [k/64][rows][64 B], one chunk per MFMA step; lane
-//            (g, r) reads bytes [16 g, 16 g + 16) of row r's chunk. Rows of an expert
-//            are consecutive (down GEMM: 1 KB of consecutive bytes per step) or a
+//            of consecutive bytes per block and the next block follows
+//            directly: one long sequential stream per 16 output channels. int8, bf16 and half: a block is an MFMA
+//            step; fp8: a step is two blocks, one 128-value scale block, whose partial sums are scaled and added in f32.
+//   activations: lane (g, r) reads the same bytes of K of its row r. int8: "chunk-major" [k/64][rows][64 B], one
+//            chunk per step: the rows of an expert are consecutive (down GEMM: 1 KB of consecutive bytes per step) or a
 //            gather of 64-byte pieces (gate_up GEMM: one half cache line per row and
 //            step; with 16-byte chunks a gathered load touched four times as many
-//            lines, which cost the DeepSeek-V3 gate_up launch 9 %).
+//            lines, which cost the DeepSeek-V3 gate_up launch 9 %). The other formats: row-major, 64 or 128
+//            consecutive bytes of a row per step.
 // Each wave owns NF channel fragments and keeps D MFMA steps of loads in flight.
+#include <type_traits>
+
 #include "kmoe_common.h"
 #include "pair_scan.h"
 #include "quant_body.h"
@@ -23,35 +25,44 @@ namespace kmoe {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+enum class Fmt { I8, F8, BF16, F16 };
+constexpr const char* fmt_name(Fmt f) { return f == Fmt::I8 ? "i8" : (f == Fmt::F8 ? "fp8" : (f == Fmt::BF16 ? "bf16" : "f16")); }
 
 struct StreamParams {
-  const int8_t* a;  // chunk-major [k/64][a_rows][64]
-  int32_t a_rows;
-  const float* a_max;
+  const int8_t* a;
+  int64_t a_row, a_step;  // bytes between rows; between the MFMA steps of a row
+  int32_t a_rows;         // chunk-major activations: their rows
+  const float* a_aux;     // I8: row maxes; F8: [row][k/128] scales
   const int32_t* row_src;
   int32_t src_div;
-  const int8_t* w;  // tiled
-  const float* w_max;
+  const int8_t* w;        // tiled
+  const float* w_aux;     // I8: [E][n] maxes; F8: [E][n/128][k/128] scales
   const int32_t* lod;
-  int32_t E, n, k;
+  int32_t E, n, kbytes;
   uint16_t* y;
   int64_t ldy;
   int32_t* acc_out;
   const int8_t* w_tail;
-  const float* w_max_tail;
+  const float* w_aux_tail;
   int32_t tail_row0, tail_rows, tail_src0;
   int32_t f16;  // outputs (and the rounding of gate and up before SiLU-mul) in IEEE half instead of bf16
-  int32_t rotate;  // every wave starts its K range at a step of its own (see stream_gemm_i8)
-  StreamScan scan;  // SCAN instantiations: the routed pairs' expert ids instead of lod / row_src
+  int32_t rotate;  // every wave starts its K range at a step of its own (see run_i8)
+  StreamScan scan;    // SCAN instantiations: the routed pairs' expert ids instead of lod / row_src
   StreamQuant quant;  // QUANT instantiations: the rows as bf16 / half values instead of codes and row maxes
+  StreamSlots slots;  // n > 0: a column of workgroups per pair instead of per expert (pair_scan.h)
 };
 
 constexpr int kWaves = 4;
 constexpr int kQuantStride = kStreamQuantMaxK + 16;  // bytes between the rows of the LDS copy: row li starts 16 li B into the banks
 
 // KS: the workgroup's 4 waves split K KS ways (KS = 1, 2, 4): 4/KS waves own
-// different channels, KS waves share channels and add their exact int32 partial
-// sums through LDS. More, shorter streams: a finer-grained tail on small layers.
+// different channels, KS waves share channels and add their partial
+// sums through LDS in a fixed order (int8: exact). More, shorter streams: a finer-grained tail on small layers.
 //
 // SCAN: the launch does the stable sort by expert itself. Every workgroup reads all the routed pairs' expert ids
 // (p.scan.ids, a few KB from L2, a quarter per wave, kScanBatch loads in flight), counts the ids below its expert
@@ -60,20 +71,22 @@ constexpr int kQuantStride = kStreamQuantMaxK + 16;  // bytes between the rows o
 // The workgroups of channel block 0 also write the sort's outputs (lod, expert_m, moe_index, sorted_src) for the
 // launches that follow.
 //
-// QUANT: the launch quantises its rows itself (the down projection of a decode-sized layer with k <= 1024). Per
+// QUANT: the launch quantises its rows itself (the int8 down projection of a decode-sized layer with k <= 1024). Per
 // 16-row pass the workgroup's four waves read the pass's live rows as bf16 / half values (p.quant.act), one row
 // per wave at a time, and leave absmax and codes - the arithmetic of quant_i8_rows_body, hence its bits - in LDS,
-// where the K loop reads its row fragments; a and a_max are not read. The workgroups of channel block 0 also write
+// where the K loop reads its row fragments; a and a_aux are not read. The workgroups of channel block 0 also write
 // codes (chunk-major) and row maxes where the quantiser's launch would have left them. Built for four waves per
-// SIMD (see stream_gemm_i8).
-template <int MF, int NF, bool SWIGLU, int D, int KS, bool SCAN = false, bool QUANT = false>
-__global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_kernel(const StreamParams p) {
+// SIMD (see run_i8).
+template <Fmt FMT, int MF, int NF, bool SWIGLU, int D, int KS, bool SCAN = false, bool QUANT = false>
+__global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kernel(const StreamParams p) {
   static_assert(!SCAN || kWaves == kScanWaves, "scan_pairs is written for four waves");
-  static_assert(!QUANT || (MF == 1 && KS == 1 && !SWIGLU && !SCAN), "QUANT: the 16-row down-projection shape only");
+  static_assert(!QUANT || (FMT == Fmt::I8 && MF == 1 && KS == 1 && !SWIGLU && !SCAN), "QUANT: the 16-row int8 down-projection shape only");
+  using acc_t = typename std::conditional<FMT == Fmt::I8, v4i, v4f>::type;
+  constexpr int V = FMT == Fmt::F8 ? 2 : 1;  // 1 KB blocks per MFMA step
   constexpr int NFH = SWIGLU ? NF / 2 : NF;
   constexpr int TM = 16 * MF;
   constexpr int WN = kWaves / KS;  // waves along the channel dimension
-  __shared__ v4i red[KS > 1 ? (KS - 1) * WN * MF * NF * kWave : 1];
+  __shared__ acc_t red[KS > 1 ? (KS - 1) * WN * MF * NF * kWave : 1];
   __shared__ typename std::conditional<SCAN, PairScanLds, int>::type scan_lds;
   __shared__ __attribute__((aligned(16))) int8_t qrows[QUANT ? 16 * kQuantStride : 16];
   __shared__ float qmax[16];
@@ -83,16 +96,29 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
   const int wk = wave_id % KS;     // K part of this wave
   const int li = lane & 15;
   const int lg = lane >> 4;
-  const bool f16 = p.f16 != 0;
+  const bool f16 = FMT == Fmt::F16 || (FMT != Fmt::BF16 && p.f16 != 0);
 
-  // blockIdx.y < E: routed expert, all its rows. Beyond: one 16*MF-row slice of the tail expert.
-  const bool tail = static_cast<int>(blockIdx.y) >= p.E;
-  const int e = tail ? p.E : blockIdx.y;
-  const int8_t* w_base = tail ? p.w_tail : p.w + static_cast<size_t>(e) * p.n * p.k;
-  const float* w_max = tail ? p.w_max_tail : p.w_max + static_cast<size_t>(e) * p.n;
+  // Columns: one per expert (or, with slots, one per pair and - in the launch that sorts - one that writes lod), all of
+  // the expert's rows; beyond: one 16*MF-row slice of the tail expert each.
+  const int column = blockIdx.y;
+  const int n_cols = p.slots.n > 0 ? p.slots.n + (SCAN ? 1 : 0) : p.E;
+  const bool tail = column >= n_cols;
+  int e = tail ? p.E : column;
+  if (p.slots.n > 0 && !tail) {
+    if constexpr (SCAN) {
+      if (column == p.slots.n) {
+        if (blockIdx.x == 0) publish_lod(p.scan, p.E, scan_lds);
+        return;
+      }
+    }
+    e = p.slots.ids[column];
+  }
+  const int8_t* w_base = tail ? p.w_tail : p.w + static_cast<size_t>(e) * p.n * p.kbytes;
+  const size_t n_aux = FMT == Fmt::F8 ? static_cast<size_t>(p.n / 128) * (p.kbytes / 128) : p.n;
+  const float* w_aux = tail ? p.w_aux_tail : p.w_aux + static_cast<size_t>(e) * n_aux;
 
   const int n_half = SWIGLU ? p.n / 2 : p.n;
-  const int ksteps = p.k / 64;
+  const int ksteps = p.kbytes / (64 * V);
   const int col_base = (blockIdx.x * WN + wave) * NFH * 16;
   // whole wave has nothing to do (no barriers when KS == 1; with QUANT it stays for the quantisation and its barriers)
   const bool idle = KS == 1 && col_base >= n_half;
@@ -104,7 +130,8 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
   // multiple of the fragment stride.
   const int klen = kb_end - kb_begin;
   const unsigned wave_key = (static_cast<unsigned>(blockIdx.y) * gridDim.x + blockIdx.x) * kWaves + wave_id;
-  const int rot = p.rotate && klen > 1 ? static_cast<int>(((wave_key * 2654435761u) >> 12) % static_cast<unsigned>(klen)) : 0;
+  const int rot = FMT == Fmt::I8 && p.rotate && klen > 1
+                      ? static_cast<int>(((wave_key * 2654435761u) >> 12) % static_cast<unsigned>(klen)) : 0;
   auto kb_of = [&](int i) {
     const int s = i + rot;
     return kb_begin + (s >= klen ? s - klen : s);
@@ -120,9 +147,8 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
     wok[f] = c < n_half;
     col[f] = (SWIGLU && f >= NFH) ? n_half + c : c;
     const size_t frag = wok[f] ? col[f] / 16 : 0;
-    wp[f] = w_base + frag * ksteps * 1024 + lane * 16;
+    wp[f] = w_base + frag * ksteps * (V * 1024) + lane * 16;
   }
-  const size_t a_step = static_cast<size_t>(p.a_rows) * 64;  // bytes between MFMA steps
 
   // The first weight steps are requested before anything else: their addresses depend on the block's coordinates
   // only, while the rows do on two dependent loads (the expert's row range, then the gather indices). All
@@ -130,32 +156,50 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
   // loads leaves the memory queue idle for their latency. Done where a wave's K range is short (a workgroup lives
   // a few microseconds: Qwen3 decode down projection 42.8 -> 40.4 us); with long ranges it changes nothing for the
   // better (DeepSeek-V3 decode: +0.4 %), so those keep the plain order.
-  const bool w_first = QUANT || klen < 16;
-  v4i wreg[D][NF];
-  v4i areg[D][MF];
+  const bool w_first = QUANT || klen * V < 16;
+  v4i wreg[D][NF][V];
+  v4i areg[D][MF][V];
+  float asc[D][MF];  // F8: the rows' scales of the step
   auto load_w_step = [&](int slot, int kb) {
 #pragma unroll
     for (int f = 0; f < NF; ++f)
-      wreg[slot][f] = wok[f] ? *reinterpret_cast<const v4i*>(wp[f] + static_cast<size_t>(kb) * 1024)
-                             : (v4i){0, 0, 0, 0};
+#pragma unroll
+      for (int v = 0; v < V; ++v)
+        wreg[slot][f][v] = wok[f] ? *reinterpret_cast<const v4i*>(wp[f] + static_cast<size_t>(kb) * (V * 1024) + v * 1024)
+                                  : (v4i){0, 0, 0, 0};
   };
   if (w_first) {
 #pragma unroll
     for (int d = 0; d < D; ++d)
       if (d < klen) load_w_step(d, kb_of(d));
   }
+  // F8: lane l holds the block scale of step kb_begin + l for each fragment (the host keeps klen <= 64)
+  float wsc[NF];
+  if constexpr (FMT == Fmt::F8) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      wsc[f] = wok[f] ? w_aux[static_cast<size_t>(col[f] / 128) * ksteps + min(kb_begin + lane, ksteps - 1)] : 0.0f;
+  }
   __builtin_amdgcn_sched_barrier(0);
 
   int row_begin, row_end;
   ListedRows listed = {};  // SCAN: the expert's rows
   if (tail) {
-    row_begin = p.tail_row0 + (static_cast<int>(blockIdx.y) - p.E) * TM;
+    row_begin = p.tail_row0 + (column - n_cols) * TM;
     row_end = min(p.tail_row0 + p.tail_rows, row_begin + TM);
   } else if constexpr (SCAN) {
     listed = scan_pairs(p.scan, e, p.E, scan_lds, blockIdx.x == 0);
-    if (idle) return;  // (KS == 1: no barrier after the scan's)
     row_begin = listed.begin;
     row_end = listed.end;
+    if (p.slots.n > 0) {
+      if (listed.pair(scan_lds, 0) != column) row_end = row_begin;  // an earlier pair's column serves this expert
+      if (blockIdx.x == 0 && threadIdx.x == 0) p.scan.slot_rows[column] = make_int2(row_begin, row_end);
+    }
+    if (idle) return;  // (KS == 1: no barrier after the scan's)
+  } else if (p.slots.n > 0) {
+    const int2 range = p.slots.rows[column];
+    row_begin = range.x;
+    row_end = range.y;
   } else {
     row_begin = p.lod[e];
     row_end = p.lod[e + 1];
@@ -166,7 +210,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
   for (int row0 = row_begin; row0 < row_end; row0 += TM) {
     if (QUANT) {
       if (row0 != row_begin) __syncthreads();  // the pass before has read its fragments
-      const int nvec = p.k / 8;  // vectors of 8 values per row: at most 2 per lane
+      const int nvec = p.kbytes / 8;  // vectors of 8 values per row: at most 2 per lane
 #pragma unroll 1
       for (int q = 0; q < 4; ++q) {
         const int qi = wave_id + 4 * q;
@@ -212,6 +256,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
       if (idle) continue;
     }
     const int8_t* ap[MF];
+    const float* asp[MF];
     int srow[MF];
 #pragma unroll
     for (int mf = 0; mf < MF; ++mf) {
@@ -221,19 +266,24 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
       else
         srow[mf] = r < row_end ? (tail ? p.tail_src0 + r - p.tail_row0 : (p.row_src ? p.row_src[r] / p.src_div : r)) : -1;
       // rows past the end read row 0: valid memory, results never stored
-      ap[mf] = p.a + static_cast<size_t>(srow[mf] >= 0 ? srow[mf] : 0) * 64 + lg * 16;
+      const size_t at = srow[mf] >= 0 ? srow[mf] : 0;
+      ap[mf] = p.a + at * p.a_row + lg * 16;
+      if constexpr (FMT == Fmt::F8) asp[mf] = p.a_aux + at * ksteps;
     }
-
-    v4i acc[MF][NF];
+    acc_t acc[MF][NF];
 #pragma unroll
     for (int mf = 0; mf < MF; ++mf)
 #pragma unroll
-      for (int f = 0; f < NF; ++f) acc[mf][f] = (v4i){0, 0, 0, 0};
+      for (int f = 0; f < NF; ++f) acc[mf][f] = acc_t{0, 0, 0, 0};
 
     auto load_a_step = [&](int slot, int kb) {
       if (QUANT) return;  // (read from LDS where it is used)
 #pragma unroll
-      for (int mf = 0; mf < MF; ++mf) areg[slot][mf] = *reinterpret_cast<const v4i*>(ap[mf] + kb * a_step);
+      for (int mf = 0; mf < MF; ++mf) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) areg[slot][mf][v] = *reinterpret_cast<const v4i*>(ap[mf] + kb * p.a_step + v * 64);
+        if constexpr (FMT == Fmt::F8) asc[slot][mf] = asp[mf][kb];
+      }
     };
     auto load_step = [&](int slot, int kb) {
       load_w_step(slot, kb);
@@ -252,14 +302,39 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
       for (int d = 0; d < D; ++d) {
         const int kb = i0 + d;
         if (kb < klen) {
+          if constexpr (FMT == Fmt::F8) {
 #pragma unroll
-          for (int mf = 0; mf < MF; ++mf)
+            for (int f = 0; f < NF; ++f) {
+              const float sw = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsc[f]), kb));
+              const v8i wv = __builtin_shufflevector(wreg[d][f][0], wreg[d][f][V - 1], 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
-            for (int f = 0; f < NF; ++f)
-              acc[mf][f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                  wreg[d][f],
-                  QUANT ? *reinterpret_cast<const v4i*>(&qrows[li * kQuantStride + kb_of(kb) * 64 + lg * 16]) : areg[d][mf],
-                  acc[mf][f], 0, 0, 0);
+              for (int mf = 0; mf < MF; ++mf) {
+                const v8i av = __builtin_shufflevector(areg[d][mf][0], areg[d][mf][V - 1], 0, 1, 2, 3, 4, 5, 6, 7);
+                const v4f blk = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wv, av, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0,
+                                                                               0x7f7f7f7f, 0, 0x7f7f7f7f);
+                const float s = asc[d][mf] * sw;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[mf][f][q] = __builtin_fmaf(blk[q], s, acc[mf][f][q]);
+              }
+            }
+          } else {
+#pragma unroll
+            for (int mf = 0; mf < MF; ++mf)
+#pragma unroll
+              for (int f = 0; f < NF; ++f) {
+                if constexpr (FMT == Fmt::I8)
+                  acc[mf][f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                      wreg[d][f][0],
+                      QUANT ? *reinterpret_cast<const v4i*>(&qrows[li * kQuantStride + kb_of(kb) * 64 + lg * 16]) : areg[d][mf][0],
+                      acc[mf][f], 0, 0, 0);
+                else if constexpr (FMT == Fmt::BF16)
+                  acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wreg[d][f][0]),
+                                                                       __builtin_bit_cast(v8bf, areg[d][mf][0]), acc[mf][f], 0, 0, 0);
+                else
+                  acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wreg[d][f][0]),
+                                                                      __builtin_bit_cast(v8h, areg[d][mf][0]), acc[mf][f], 0, 0, 0);
+              }
+          }
           if (kb + D < klen) load_step(d, kb_of(kb + D));
         }
       }
@@ -283,7 +358,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
             for (int f = 0; f < NF; ++f)
               acc[mf][f] += red[(((part - 1) * WN + wave) * MF * NF + mf * NF + f) * kWave + lane];
       }
-      __syncthreads();  // red is reused by the next m-tile
+      if (row0 + TM < row_end) __syncthreads();  // red is reused by the next m-tile
       if (wk > 0) continue;
     }
 
@@ -291,23 +366,30 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
     for (int mf = 0; mf < MF; ++mf) {
       const int r = row0 + mf * 16 + li;
       if (r >= row_end) continue;
-      const float sa = (QUANT ? qmax[li] : p.a_max[srow[mf]]) / 127.0f;
+      float sa = 1.0f;
+      if constexpr (FMT == Fmt::I8) sa = (QUANT ? qmax[li] : p.a_aux[srow[mf]]) / 127.0f;
 #pragma unroll
       for (int f = 0; f < NFH; ++f) {
         if (!wok[f]) continue;
         const int c0 = col[f] + lg * 4;
         uint16_t yv[4];
-        auto finish = [&](const v4i& a, int cc, uint16_t(&out)[4]) {
-          const float4 wm = *reinterpret_cast<const float4*>(w_max + cc);
-          const float sw[4] = {wm.x / 127.0f, wm.y / 127.0f, wm.z / 127.0f, wm.w / 127.0f};
+        auto finish = [&](const acc_t& a, int ff, uint16_t(&out)[4]) {
+          if constexpr (FMT == Fmt::I8) {
+            const int cc = col[ff] + lg * 4;
+            const float4 wm = *reinterpret_cast<const float4*>(w_aux + cc);
+            const float sw[4] = {wm.x / 127.0f, wm.y / 127.0f, wm.z / 127.0f, wm.w / 127.0f};
 #pragma unroll
-          for (int q = 0; q < 4; ++q) out[q] = f32_to_act((static_cast<float>(a[q]) * sa) * sw[q], f16);
-          if (p.acc_out) *reinterpret_cast<v4i*>(p.acc_out + static_cast<size_t>(r) * p.n + cc) = a;
+            for (int q = 0; q < 4; ++q) out[q] = f32_to_act((static_cast<float>(a[q]) * sa) * sw[q], f16);
+            if (p.acc_out) *reinterpret_cast<v4i*>(p.acc_out + static_cast<size_t>(r) * p.n + cc) = a;
+          } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) out[q] = f32_to_act(a[q], f16);
+          }
         };
-        finish(acc[mf][f], c0, yv);
-        if (SWIGLU) {
+        finish(acc[mf][f], f, yv);
+        if constexpr (SWIGLU) {
           uint16_t uv[4];
-          finish(acc[mf][f + NFH], col[f + NFH] + lg * 4, uv);
+          finish(acc[mf][f + NFH], f + NFH, uv);
 #pragma unroll
           for (int q = 0; q < 4; ++q) yv[q] = f32_to_act(silu_hw(act_to_f32(yv[q], f16)) * act_to_f32(uv[q], f16), f16);
         }
@@ -319,17 +401,34 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_i8_k
   }
 }
 
-template <int MF, int NF, bool SWIGLU, int D, int KS = 1, bool SCAN = false, bool QUANT = false>
+template <Fmt FMT, int MF, int NF, bool SWIGLU, int D, int KS = 1, bool SCAN = false, bool QUANT = false>
 int launch_stream(const StreamParams& p, hipStream_t s) {
   constexpr int NFH = SWIGLU ? NF / 2 : NF;
   const int n_half = SWIGLU ? p.n / 2 : p.n;
-  const dim3 grid(ceil_div(n_half, (kWaves / KS) * NFH * 16), p.E + (p.w_tail ? ceil_div(p.tail_rows, 16 * MF) : 0));
+  const int cols = p.slots.n > 0 ? p.slots.n + (SCAN ? 1 : 0) : p.E;
+  const dim3 grid(ceil_div(n_half, (kWaves / KS) * NFH * 16), cols + (p.w_tail ? ceil_div(p.tail_rows, 16 * MF) : 0));
   if (tracing_kernels())
-    note_kernel("stream_gemm_i8_kernel<%d rows per pass, %d channel fragments per wave, %s, %d steps in flight, K split %d%s%s>",
-                16 * MF, NF, SWIGLU ? "SiLU-mul" : "plain", D, KS, SCAN ? ", sorts the pairs itself" : "",
-                QUANT ? ", quantises its rows itself" : "");
-  hipLaunchKernelGGL((stream_gemm_i8_kernel<MF, NF, SWIGLU, D, KS, SCAN, QUANT>), grid, dim3(kWaves * kWave), 0, s, p);
-  return check_launch("kmoe_grouped_gemm_i8 (stream)");
+    note_kernel("stream_gemm_kernel<%s, %d rows per pass, %d channel fragments per wave, %s, %d steps in flight, K split %d%s%s%s>",
+                fmt_name(FMT), 16 * MF, NF, SWIGLU ? "SiLU-mul" : "plain", D, KS, SCAN ? ", sorts the pairs itself" : "",
+                QUANT ? ", quantises its rows itself" : "", p.slots.n > 0 ? ", a column per pair" : "");
+  hipLaunchKernelGGL((stream_gemm_kernel<FMT, MF, NF, SWIGLU, D, KS, SCAN, QUANT>), grid, dim3(kWaves * kWave), 0, s, p);
+  return check_launch("kmoe_grouped_gemm (stream)");
+}
+
+// The shapes of a 16-row launch, from its dimensions alone (`blocks`: workgroups of four waves side by side):
+// K is split across the waves of a workgroup when its streams are long enough to share: more, shorter streams balance
+// the tail (measured: +6..12% at k = 2048). Batches of a few tokens take the same shapes: with a column of workgroups per
+// pair (Qwen3, one token: layer 53 -> 24 us, its launches no longer mostly workgroups of experts without rows) keeping
+// a wave's whole K range in flight (8 steps) gains nothing at one token and loses 10 to 25 % from four tokens on.
+template <Fmt FMT, bool SWIGLU, bool SCAN>
+int launch_rows16(const StreamParams& p, hipStream_t s) {
+  constexpr int V = FMT == Fmt::F8 ? 2 : 1;
+  const int ksteps = p.kbytes / 64;
+  const int n_half = SWIGLU ? p.n / 2 : p.n;
+  const int blocks = p.E * ceil_div(n_half, kWaves * (SWIGLU ? 1 : 2) * 16);
+  if (ksteps >= 24 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, 2, 4, SCAN>(p, s);
+  if (ksteps >= 24) return launch_stream<FMT, 1, 2, SWIGLU, 4 / V, 2, SCAN>(p, s);
+  return launch_stream<FMT, 1, 2, SWIGLU, 4 / V, 1, SCAN>(p, s);
 }
 
 // [E][n][k] row-major -> tiled blocks; one thread moves 16 bytes.
@@ -347,10 +446,25 @@ __global__ void tile_weights_kernel(const int8_t* __restrict__ src, int8_t* __re
   *reinterpret_cast<uint4*>(dst + v * 16) = *reinterpret_cast<const uint4*>(src + row * k + kk);
 }
 
+int check_scan(const StreamScan* scan, bool swiglu, int variant, const int32_t* row_src, int rows) {
+  KMOE_REQUIRE(swiglu && variant == 0 && row_src == nullptr && scan->ids && scan->lod && scan->expert_m &&
+                   scan->moe_index && scan->sorted_src && scan->n_pairs == rows && rows <= kStreamScanMaxPairs,
+               KMOE_ERR_UNSUPPORTED, "grouped_gemm (stream): not a launch that can sort the pairs itself");
+  KMOE_REQUIRE(!scan->slot_rows || rows <= kStreamSlotMaxPairs, KMOE_ERR_UNSUPPORTED,
+               "grouped_gemm (stream): %d pairs are too many for a column each", rows);
+  return KMOE_OK;
+}
+
+StreamSlots slots_of(const StreamScan* scan, const StreamSlots* slots) {
+  if (scan) return scan->slot_rows ? StreamSlots{scan->ids, scan->slot_rows, scan->n_pairs} : StreamSlots{};
+  return slots ? *slots : StreamSlots{};
+}
+
 }  // namespace
 
-int stream_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s, const StreamScan* scan, const StreamQuant* quant) {
-  StreamParams p{a->a, a->a_rows, a->a_max, a->row_src, a->src_div, a->w, a->w_max,
+int stream_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s, const StreamScan* scan, const StreamQuant* quant,
+                   const StreamSlots* slots) {
+  StreamParams p{a->a, 64, static_cast<int64_t>(a->a_rows) * 64, a->a_rows, a->a_max, a->row_src, a->src_div, a->w, a->w_max,
                  a->lod, a->E,     a->n,     a->k,       a->y,       a->ldy, a->acc_out,
                  a->w_tail, a->w_max_tail, a->tail_row0, a->tail_rows, a->tail_src0, a->act_dtype == KMOE_DT_F16,
                  // A fragment's blocks are k / 64 KB apart. When that stride is a multiple of 64 KB (k = 4096, 8192:
@@ -358,72 +472,77 @@ int stream_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s, const StreamScan* 
                  // and 6.0 at 4096 against 6.5 at 2048; with the rotated start 6.0 and 6.6. Other strides gain
                  // nothing from it (k = 7168: 6.2 either way).
                  a->k % 4096 == 0,
-                 scan ? *scan : StreamScan{}, quant ? *quant : StreamQuant{}};
+                 scan ? *scan : StreamScan{}, quant ? *quant : StreamQuant{}, slots_of(scan, slots)};
   const bool swiglu = a->act == KMOE_ACT_SWIGLU;
+  const int live = expected_rows(a->rows, a->rows_hint);
   if (quant) {
     // the down launch of a decode-sized layer: 16 rows per pass, one wave per K range
     KMOE_REQUIRE(!scan && !swiglu && a->variant == 0 && a->row_src == nullptr && !a->acc_out && quant->act &&
                      quant->codes && quant->amax && quant->ld >= a->k && quant->ld % 8 == 0 &&
-                     a->k <= kStreamQuantMaxK && a->k / 64 < 24 &&
-                     ceil_div(expected_rows(a->rows, a->rows_hint), a->E) <= 10,
+                     a->k <= kStreamQuantMaxK && a->k / 64 < 24 && ceil_div(live, a->E) <= 10,
                  KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8 (stream): not a launch that can quantise its rows itself");
     // (Four steps of weights in flight and two channel fragments per wave as in the plain launch. Two steps, or one
     // fragment per wave with 2 / 4 / 8 steps - 5 to 6 waves per SIMD - are 1.6 to 3.3 us slower; 6 and 8 steps with
     // two fragments need more registers than four waves per SIMD leave, and this launch needs the four: built for
     // three it took as long as the quantiser's launch and this one together had. Qwen3 decode, layer: 117.5 us with
     // the quantiser's launch, 117.0 built for three waves, 115.1 for four.)
-    return launch_stream<1, 2, false, 4, 1, false, true>(p, s);
+    return launch_stream<Fmt::I8, 1, 2, false, 4, 1, false, true>(p, s);
   }
   if (scan) {
-    // the routed gate_up launch of a decode-sized layer: 16 rows per pass, the three shapes of `case 1` below
-    KMOE_REQUIRE(swiglu && a->variant == 0 && a->row_src == nullptr && scan->ids && scan->lod && scan->expert_m &&
-                     scan->moe_index && scan->sorted_src && scan->n_pairs == a->rows &&
-                     a->rows <= kStreamScanMaxPairs && a->a_rows <= kStreamScanMaxRows,
-                 KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8 (stream): not a launch that can sort the pairs itself");
-    const int ksteps = p.k / 64;
-    const int blocks = p.E * ceil_div(p.n / 2, kWaves * 16);
-    if (ksteps >= 24 && blocks < 2048) return launch_stream<1, 2, true, 2, 4, true>(p, s);
-    if (ksteps >= 24) return launch_stream<1, 2, true, 4, 2, true>(p, s);
-    return launch_stream<1, 2, true, 4, 1, true>(p, s);
+    if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
+    KMOE_REQUIRE(a->a_rows <= kStreamScanMaxRows, KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8 (stream): %d tokens", a->a_rows);
+    return launch_rows16<Fmt::I8, true, true>(p, s);
   }
   // m-fragments per pass from the rows an expert gets under uniform routing
   int mf = a->variant;
   if (mf == 0) {
     // An expert with more rows than one pass holds streams its weights again: leave headroom
     // over the mean for the spread of a random routing (about +-2 sigma at these sizes).
-    const int avg = ceil_div(expected_rows(a->rows, a->rows_hint), a->E);
+    const int avg = ceil_div(live, a->E);
     mf = avg <= 10 ? 1 : (avg <= 22 ? 2 : (avg <= 48 ? 4 : 8));
   }
   switch (mf) {
-    // tuning variants of the 16-row kernel: 1xy = prefetch depth x, K split y
-    case 121: return swiglu ? launch_stream<1, 2, true, 2, 1>(p, s) : launch_stream<1, 2, false, 2, 1>(p, s);
-    case 181: return swiglu ? launch_stream<1, 2, true, 8, 1>(p, s) : launch_stream<1, 2, false, 8, 1>(p, s);
-    case 142: return swiglu ? launch_stream<1, 2, true, 4, 2>(p, s) : launch_stream<1, 2, false, 4, 2>(p, s);
-    case 144: return swiglu ? launch_stream<1, 2, true, 4, 4>(p, s) : launch_stream<1, 2, false, 4, 4>(p, s);
-    case 122: return swiglu ? launch_stream<1, 2, true, 2, 2>(p, s) : launch_stream<1, 2, false, 2, 2>(p, s);
-    case 124: return swiglu ? launch_stream<1, 2, true, 2, 4>(p, s) : launch_stream<1, 2, false, 2, 4>(p, s);
-    case 182: return swiglu ? launch_stream<1, 2, true, 8, 2>(p, s) : launch_stream<1, 2, false, 8, 2>(p, s);
-    case 1: {
-      // Split K across the waves of a workgroup when streams are long enough to share:
-      // more, shorter streams balance the tail (measured: +6..12% at k = 2048).
-      const int ksteps = p.k / 64;
-      const int n_half = swiglu ? p.n / 2 : p.n;
-      const int blocks = p.E * ceil_div(n_half, kWaves * (swiglu ? 1 : 2) * 16);
-      if (ksteps >= 24 && blocks < 2048)
-        return swiglu ? launch_stream<1, 2, true, 2, 4>(p, s) : launch_stream<1, 2, false, 2, 4>(p, s);
-      if (ksteps >= 24)
-        return swiglu ? launch_stream<1, 2, true, 4, 2>(p, s) : launch_stream<1, 2, false, 4, 2>(p, s);
-      return swiglu ? launch_stream<1, 2, true, 4>(p, s) : launch_stream<1, 2, false, 4>(p, s);
-    }
+    case 1:
+      return swiglu ? launch_rows16<Fmt::I8, true, false>(p, s)
+                    : launch_rows16<Fmt::I8, false, false>(p, s);
     case 2:
-      return swiglu ? launch_stream<2, 2, true, 4>(p, s) : launch_stream<2, 2, false, 4>(p, s);
+      return swiglu ? launch_stream<Fmt::I8, 2, 2, true, 4>(p, s) : launch_stream<Fmt::I8, 2, 2, false, 4>(p, s);
     case 4:
-      return swiglu ? launch_stream<4, 2, true, 4>(p, s) : launch_stream<4, 2, false, 4>(p, s);
+      return swiglu ? launch_stream<Fmt::I8, 4, 2, true, 4>(p, s) : launch_stream<Fmt::I8, 4, 2, false, 4>(p, s);
     case 8:
-      return swiglu ? launch_stream<8, 2, true, 2>(p, s) : launch_stream<8, 2, false, 2>(p, s);
+      return swiglu ? launch_stream<Fmt::I8, 8, 2, true, 2>(p, s) : launch_stream<Fmt::I8, 8, 2, false, 2>(p, s);
     default:
       return fail(KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8 (stream): variant=%d must be 0, 1, 2, 4 or 8", a->variant);
   }
+}
+
+int stream_gemm_fp8(const kmoe_gemm_fp8_args* a, hipStream_t s, const StreamScan* scan, const StreamSlots* slots) {
+  const StreamParams p{reinterpret_cast<const int8_t*>(a->a), a->lda, 128, 0, a->a_scale, a->row_src, a->src_div,
+                       reinterpret_cast<const int8_t*>(a->w), a->w_scale, a->lod, a->E, a->n, a->k, a->y, a->ldy, nullptr,
+                       reinterpret_cast<const int8_t*>(a->w_tail), a->w_scale_tail, a->tail_row0, a->w_tail ? a->tail_rows : 0,
+                       a->tail_src0, a->act_dtype == KMOE_DT_F16, 0, scan ? *scan : StreamScan{}, StreamQuant{},
+                       slots_of(scan, slots)};
+  const bool swiglu = a->act == KMOE_ACT_SWIGLU;
+  if (scan) {
+    if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
+    return launch_rows16<Fmt::F8, true, true>(p, s);
+  }
+  return swiglu ? launch_rows16<Fmt::F8, true, false>(p, s) : launch_rows16<Fmt::F8, false, false>(p, s);
+}
+
+int stream_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s, const StreamScan* scan, const StreamSlots* slots) {
+  const bool half = a->act_dtype == KMOE_DT_F16;
+  const StreamParams p{reinterpret_cast<const int8_t*>(a->a), a->lda * 2, 64, 0, nullptr, a->row_src, a->src_div,
+                       reinterpret_cast<const int8_t*>(a->w), nullptr, a->lod, a->E, a->n, a->k * 2, a->y, a->ldy, nullptr,
+                       nullptr, nullptr, 0, 0, 0, half, 0, scan ? *scan : StreamScan{}, StreamQuant{},
+                       slots_of(scan, slots)};
+  const bool swiglu = a->act == KMOE_ACT_SWIGLU;
+  if (scan) {
+    if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
+    return half ? launch_rows16<Fmt::F16, true, true>(p, s) : launch_rows16<Fmt::BF16, true, true>(p, s);
+  }
+  if (half) return swiglu ? launch_rows16<Fmt::F16, true, false>(p, s) : launch_rows16<Fmt::F16, false, false>(p, s);
+  return swiglu ? launch_rows16<Fmt::BF16, true, false>(p, s) : launch_rows16<Fmt::BF16, false, false>(p, s);
 }
 
 }  // namespace kmoe
