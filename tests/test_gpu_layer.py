@@ -421,7 +421,7 @@ def test_int8_layer_as_an_expert_parallel_share(M, scoring):
         assert torch.equal(out2, out)
 
 
-@pytest.mark.parametrize("fmt", ["int8", "fp8", "none"])
+@pytest.mark.parametrize("fmt", ["int8", "fp8", "none", "w4"])
 @pytest.mark.parametrize("M,E,K", [(1, 16, 8), (1, 9, 8), (3, 64, 8), (7, 64, 8), (8, 64, 8), (31, 256, 8), (32, 257, 8),
                                    (33, 300, 8), (63, 512, 4), (5, 1000, 16)])
 def test_decode_launches_with_a_column_per_pair(fmt, M, E, K):
@@ -445,7 +445,7 @@ def test_decode_launches_with_a_column_per_pair(fmt, M, E, K):
                            ("lod", np.concatenate([[0], np.cumsum(counts)]))):
             got = _view(m.last_workspace, getattr(m.last_layout, name), len(want), torch.int32).cpu().numpy()
             assert np.array_equal(got, want), name
-    if fmt == "none" or fmt == "fp8":  # (the same products; fp8 and bf16 sums may be split over K differently)
-        assert rel_l2(part, whole[:M]) <= 2e-3
-    else:
+    if fmt == "int8":
         assert torch.equal(part, whole[:M])
+    else:  # (the same products; these sums may be split over K differently)
+        assert rel_l2(part, whole[:M]) <= 4e-3

@@ -153,7 +153,8 @@ bool fold_shared(const kmoe_moe_args* a) {
   return a->format == KMOE_FMT_FP8_BLOCK && a->w_layout == KMOE_W_TILED && a->H <= 8192 && a->I <= 8192;
 }
 
-// Whether both routed GEMMs run on the weight-streaming kernel (the packed 4-bit format has one of its own).
+// Whether the routed gate_up GEMM runs on the weight-streaming kernel (and, 4-bit weights with long rows aside, the
+// down GEMM as well).
 bool routed_streams(const kmoe_moe_args* a) {
   if (a->w_layout != KMOE_W_TILED) return false;
   const long long rows = local_pairs(a);
@@ -163,7 +164,7 @@ bool routed_streams(const kmoe_moe_args* a) {
     case KMOE_FMT_BF16:
       return streams_bf16(static_cast<int>(rows), a->E, a->H) && streams_bf16(static_cast<int>(rows), a->E, a->I) &&
              !a->w13_bias && !a->w2_bias && a->activation != KMOE_ACT_SWIGLUOAI;
-    default: return w4_gate_up_streams(a->M * a->K, 0, a->E, a->H);
+    default: return w4_gate_up_streams(a->M * a->K, a->E_global > a->E ? static_cast<int>(rows) : 0, a->E, a->H);
   }
 }
 
@@ -307,7 +308,7 @@ int run_gemm(const MlpPass& m, bool first, kmoe_stream_t stream) {
     g.act = act;
     g.w_layout = m.w_layout;
     g.act_dtype = m.act_dtype;
-    return grouped_gemm_w4a16_checked(&g, stream, first ? m.scan : nullptr);
+    return grouped_gemm_w4a16_checked(&g, stream, first ? m.scan : nullptr, first ? nullptr : m.slots);
   }
   kmoe_gemm_bf16_args g = {};
   g.a = static_cast<const uint16_t*>(a);
@@ -551,7 +552,7 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   const bool scan_in_gemm = routed_streams(a) && Eg == E && a->first_expert == 0 && P <= kStreamScanMaxPairs &&
                             M <= kStreamScanMaxRows && scan_allowed();
   // Fewer pairs than experts: a column of workgroups per pair instead of per expert.
-  const bool per_pair = scan_in_gemm && a->format != KMOE_FMT_W4A16 && P < E && P <= kStreamSlotMaxPairs;
+  const bool per_pair = scan_in_gemm && P < E && P <= kStreamSlotMaxPairs;
   int2* slot_rows = per_pair ? static_cast<int2*>(at(L.align_ws)) : nullptr;
   const StreamScan scan{topk_ids, P, lod, static_cast<int32_t*>(at(L.expert_m)), moe_index, sorted_src, slot_rows};
   const StreamSlots slots{topk_ids, slot_rows, P};

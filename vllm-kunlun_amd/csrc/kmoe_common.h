@@ -75,7 +75,11 @@ inline bool streams_fp8(int live_rows, int E, int k) { return ceil_div(live_rows
 inline bool streams_bf16(int live_rows, int E, int k) { return ceil_div(live_rows, E) <= kStreamMaxRows && k % 32 == 0; }
 // kmoe_grouped_gemm_w4a16 with `scan` for the layer's routed gate_up launch where it runs on the streaming kernel
 // (w4_gate_up_streams says whether a launch of these dimensions does).
-int grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* args, kmoe_stream_t stream, const StreamScan* scan);
+int grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* args, kmoe_stream_t stream, const StreamScan* scan,
+                               const StreamSlots* slots);
+// The streaming kernel on packed 4-bit weights; passes: 1, 2, 4 for 16, 32, 64 rows per pass.
+int stream_gemm_w4(const kmoe_gemm_w4_args* args, hipStream_t stream, int passes, const StreamScan* scan,
+                   const StreamSlots* slots);
 bool w4_gate_up_streams(int rows, int rows_hint, int E, int k);
 // Persistent 128-row-tile GEMMs for many rows per expert (tiled weights, row-major activations);
 // arguments already validated.

@@ -1,5 +1,6 @@
 // Weight-streaming grouped GEMM for the decode regime (a handful of rows per expert), on int8 (W8A8), fp8-e4m3
-// (128x128 / 1x128 block scales), bf16 and half weights: HBM-bound, every weight byte is read once, MFMA is ~5% busy.
+// (128x128 / 1x128 block scales), bf16, half and packed 4-bit weights: HBM-bound, every weight byte is read once, MFMA is
+// ~5% busy.
 //
 // A wave needs no LDS, no barrier and no address arithmetic beyond a stride in its main loop:
 //   weights  "tiled": [E][n/16][k bytes/64] blocks of 1 KB; inside a block byte
@@ -7,19 +8,23 @@
 //            i.e. exactly what lane 16*g + c feeds the MFMA. A wave reads 1 KB
 //            of consecutive bytes per block and the next block follows
 //            directly: one long sequential stream per 16 output channels. int8, bf16 and half: a block is an MFMA
-//            step; fp8: a step is two blocks, one 128-value scale block, whose partial sums are scaled and added in f32.
+//            step; fp8: a step is two blocks, one 128-value scale block, whose partial sums are scaled and added in f32;
+//            4-bit: a step is one block of 128 values: a lane's 16 bytes are values 32 g + [0, 32) of its channel, its
+//            t-th word unpacked (w4_unpack.h) its operand of the t-th of four MFMAs, one group scale for all of them.
 //   activations: lane (g, r) reads the same bytes of K of its row r. int8: "chunk-major" [k/64][rows][64 B], one
 //            chunk per step: the rows of an expert are consecutive (down GEMM: 1 KB of consecutive bytes per step) or a
 //            gather of 64-byte pieces (gate_up GEMM: one half cache line per row and
 //            step; with 16-byte chunks a gathered load touched four times as many
-//            lines, which cost the DeepSeek-V3 gate_up launch 9 %). The other formats: row-major, 64 or 128
+//            lines, which cost the DeepSeek-V3 gate_up launch 9 %). The other formats: row-major, 64 to 256
 //            consecutive bytes of a row per step.
 // Each wave owns NF channel fragments and keeps D MFMA steps of loads in flight.
 #include <type_traits>
 
+#include "buffer_ops.h"
 #include "kmoe_common.h"
 #include "pair_scan.h"
 #include "quant_body.h"
+#include "w4_unpack.h"
 
 namespace kmoe {
 namespace {
@@ -30,8 +35,11 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-enum class Fmt { I8, F8, BF16, F16 };
-constexpr const char* fmt_name(Fmt f) { return f == Fmt::I8 ? "i8" : (f == Fmt::F8 ? "fp8" : (f == Fmt::BF16 ? "bf16" : "f16")); }
+enum class Fmt { I8, F8, BF16, F16, W4, W4H };  // W4H: half activations, scales and results
+constexpr const char* fmt_name(Fmt f) {
+  constexpr const char* names[] = {"i8", "fp8", "bf16", "f16", "4-bit", "4-bit, f16"};
+  return names[static_cast<int>(f)];
+}
 
 struct StreamParams {
   const int8_t* a;
@@ -54,6 +62,13 @@ struct StreamParams {
   int32_t rotate;  // every wave starts its K range at a step of its own (see run_i8)
   StreamScan scan;    // SCAN instantiations: the routed pairs' expert ids instead of lod / row_src
   StreamQuant quant;  // QUANT instantiations: the rows as bf16 / half values instead of codes and row maxes
+  // W4: group scales. Element strides inside the 16 x (k / group) scales of a fragment (16 channels), which start at
+  // channel * (k / group) in both layouts. KMOE_S_ROWMAJOR: channel k / group, group 1. KMOE_S_FRAG16
+  // (kmoe_tile_scales_w4): channel 1, group 16 - what a step needs is then 32 to 128 consecutive bytes: one cache line
+  // per load instruction where the row-major layout touches 16 (one per channel).
+  const uint16_t* w_scale;
+  int32_t groups, s_ch, s_g;
+  int32_t gs32, gs_shift;  // values per group / 32, and its log2 if it is a power of two, else -1
   StreamSlots slots;  // n > 0: a column of workgroups per pair instead of per expert (pair_scan.h)
 };
 
@@ -82,7 +97,10 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
   static_assert(!SCAN || kWaves == kScanWaves, "scan_pairs is written for four waves");
   static_assert(!QUANT || (FMT == Fmt::I8 && MF == 1 && KS == 1 && !SWIGLU && !SCAN), "QUANT: the 16-row int8 down-projection shape only");
   using acc_t = typename std::conditional<FMT == Fmt::I8, v4i, v4f>::type;
-  constexpr int V = FMT == Fmt::F8 ? 2 : 1;  // 1 KB blocks per MFMA step
+  constexpr bool W4 = FMT == Fmt::W4 || FMT == Fmt::W4H;
+  constexpr int V = FMT == Fmt::F8 ? 2 : 1;  // 1 KB blocks of weights per step
+  constexpr int AV = W4 ? 4 : V;             // 16-byte vectors of activations per lane and step ...
+  constexpr int kAVStride = W4 ? 16 : 64, kALane = W4 ? 64 : 16;  // ... bytes between them, between the lane groups
   constexpr int NFH = SWIGLU ? NF / 2 : NF;
   constexpr int TM = 16 * MF;
   constexpr int WN = kWaves / KS;  // waves along the channel dimension
@@ -91,12 +109,12 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
   __shared__ __attribute__((aligned(16))) int8_t qrows[QUANT ? 16 * kQuantStride : 16];
   __shared__ float qmax[16];
   const int lane = lane_id();
-  const int wave_id = threadIdx.x >> 6;
+  const int wave_id = W4 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
   const int wave = wave_id / KS;   // channel group of this wave
   const int wk = wave_id % KS;     // K part of this wave
   const int li = lane & 15;
   const int lg = lane >> 4;
-  const bool f16 = FMT == Fmt::F16 || (FMT != Fmt::BF16 && p.f16 != 0);
+  const bool f16 = FMT == Fmt::F16 || FMT == Fmt::W4H || ((FMT == Fmt::I8 || FMT == Fmt::F8) && p.f16 != 0);
 
   // Columns: one per expert (or, with slots, one per pair and - in the launch that sorts - one that writes lod), all of
   // the expert's rows; beyond: one 16*MF-row slice of the tail expert each.
@@ -137,6 +155,12 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
     return kb_begin + (s >= klen ? s - klen : s);
   };
 
+  // 4-bit weights: the loads of the K loop are raw buffer loads, a lane offset that stays and a scalar offset per step -
+  // no address arithmetic on the vector unit, which the unpacking keeps busy - and rows past the end lie past the
+  // descriptor's end: they read zero and fetch nothing (Kimi-K2 dimensions, 128 tokens: layer 1674 -> 1577 us, Qwen3
+  // 93 -> 90). The other formats leave the vector unit idle; there the same loads gain nothing (int8, bf16) or lose
+  // (fp8, DeepSeek-V3 at 128 tokens: 1800 -> 1854 us).
+  __amdgpu_buffer_rsrc_t wr[NF];
   const int8_t* wp[NF];
   bool wok[NF];
   int col[NF];
@@ -147,7 +171,11 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
     wok[f] = c < n_half;
     col[f] = (SWIGLU && f >= NFH) ? n_half + c : c;
     const size_t frag = wok[f] ? col[f] / 16 : 0;
-    wp[f] = w_base + frag * ksteps * (V * 1024) + lane * 16;
+    const int frag_bytes = ksteps * (V * 1024);
+    if constexpr (W4)
+      wr[f] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w_base + frag * frag_bytes), 0, wok[f] ? frag_bytes : 0, 0x00020000);
+    else
+      wp[f] = w_base + frag * frag_bytes + lane * 16;
   }
 
   // The first weight steps are requested before anything else: their addresses depend on the block's coordinates
@@ -156,17 +184,34 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
   // loads leaves the memory queue idle for their latency. Done where a wave's K range is short (a workgroup lives
   // a few microseconds: Qwen3 decode down projection 42.8 -> 40.4 us); with long ranges it changes nothing for the
   // better (DeepSeek-V3 decode: +0.4 %), so those keep the plain order.
-  const bool w_first = QUANT || klen * V < 16;
+  const bool w_first = QUANT || W4 || klen * V < 16;
+  const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.a), 0, 0xfffffff0, 0x00020000);
   v4i wreg[D][NF][V];
-  v4i areg[D][MF][V];
+  v4i areg[D][MF][AV];
   float asc[D][MF];  // F8: the rows' scales of the step
+  uint16_t gsc[D][NF];  // W4: the channels' group scales of the step
+  const uint16_t* sp[NF];
+  if constexpr (W4) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      sp[f] = p.w_scale + (static_cast<size_t>(e) * p.n + (wok[f] ? col[f] : 0)) * p.groups + li * p.s_ch;
+  }
   auto load_w_step = [&](int slot, int kb) {
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
       for (int v = 0; v < V; ++v)
-        wreg[slot][f][v] = wok[f] ? *reinterpret_cast<const v4i*>(wp[f] + static_cast<size_t>(kb) * (V * 1024) + v * 1024)
-                                  : (v4i){0, 0, 0, 0};
+        if constexpr (W4)
+          wreg[slot][f][v] = buffer_load16(wr[f], lane * 16, static_cast<uint32_t>(kb) * (V * 1024) + v * 1024);
+        else
+          wreg[slot][f][v] = wok[f] ? *reinterpret_cast<const v4i*>(wp[f] + static_cast<size_t>(kb) * (V * 1024) + v * 1024)
+                                    : (v4i){0, 0, 0, 0};
+    if constexpr (W4) {
+      const int g32 = 4 * kb + lg;  // this lane's 32 values of the step
+      const int g = p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / p.gs32;
+#pragma unroll
+      for (int f = 0; f < NF; ++f) gsc[slot][f] = sp[f][g * p.s_g];
+    }
   };
   if (w_first) {
 #pragma unroll
@@ -255,6 +300,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
       __syncthreads();
       if (idle) continue;
     }
+    uint32_t aoff[MF];
     const int8_t* ap[MF];
     const float* asp[MF];
     int srow[MF];
@@ -265,9 +311,10 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
         srow[mf] = r < row_end ? (tail ? p.tail_src0 + r - p.tail_row0 : listed.pair(scan_lds, r - row_begin) / p.src_div) : -1;
       else
         srow[mf] = r < row_end ? (tail ? p.tail_src0 + r - p.tail_row0 : (p.row_src ? p.row_src[r] / p.src_div : r)) : -1;
-      // rows past the end read row 0: valid memory, results never stored
       const size_t at = srow[mf] >= 0 ? srow[mf] : 0;
-      ap[mf] = p.a + at * p.a_row + lg * 16;
+      // rows past the end read row 0 (valid memory, results never stored) or nothing
+      ap[mf] = p.a + at * p.a_row + lg * kALane;
+      aoff[mf] = srow[mf] >= 0 ? static_cast<uint32_t>(srow[mf]) * static_cast<uint32_t>(p.a_row) + lg * kALane : 0xfffffff0u;
       if constexpr (FMT == Fmt::F8) asp[mf] = p.a_aux + at * ksteps;
     }
     acc_t acc[MF][NF];
@@ -281,7 +328,12 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
 #pragma unroll
       for (int mf = 0; mf < MF; ++mf) {
 #pragma unroll
-        for (int v = 0; v < V; ++v) areg[slot][mf][v] = *reinterpret_cast<const v4i*>(ap[mf] + kb * p.a_step + v * 64);
+        for (int v = 0; v < AV; ++v) {
+          if constexpr (W4)
+            areg[slot][mf][v] = buffer_load16(ar, aoff[mf], static_cast<uint32_t>(kb) * static_cast<uint32_t>(p.a_step) + v * kAVStride);
+          else
+            areg[slot][mf][v] = *reinterpret_cast<const v4i*>(ap[mf] + kb * p.a_step + v * kAVStride);
+        }
         if constexpr (FMT == Fmt::F8) asc[slot][mf] = asp[mf][kb];
       }
     };
@@ -315,6 +367,24 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
                 const float s = asc[d][mf] * sw;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) acc[mf][f][q] = __builtin_fmaf(blk[q], s, acc[mf][f][q]);
+              }
+            }
+          } else if constexpr (W4) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+              const W4Scale<FMT == Fmt::W4H> s(gsc[d][f]);
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                const v4i wv = unpack8(static_cast<uint32_t>(wreg[d][f][0][t]), s);
+#pragma unroll
+                for (int mf = 0; mf < MF; ++mf) {
+                  if constexpr (FMT == Fmt::W4)
+                    acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wv),
+                                                                         __builtin_bit_cast(v8bf, areg[d][mf][t]), acc[mf][f], 0, 0, 0);
+                  else
+                    acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wv),
+                                                                        __builtin_bit_cast(v8h, areg[d][mf][t]), acc[mf][f], 0, 0, 0);
+                }
               }
             }
           } else {
@@ -472,7 +542,7 @@ int stream_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s, const StreamScan* 
                  // and 6.0 at 4096 against 6.5 at 2048; with the rotated start 6.0 and 6.6. Other strides gain
                  // nothing from it (k = 7168: 6.2 either way).
                  a->k % 4096 == 0,
-                 scan ? *scan : StreamScan{}, quant ? *quant : StreamQuant{}, slots_of(scan, slots)};
+                 scan ? *scan : StreamScan{}, quant ? *quant : StreamQuant{}, nullptr, 0, 0, 0, 0, 0, slots_of(scan, slots)};
   const bool swiglu = a->act == KMOE_ACT_SWIGLU;
   const int live = expected_rows(a->rows, a->rows_hint);
   if (quant) {
@@ -521,7 +591,7 @@ int stream_gemm_fp8(const kmoe_gemm_fp8_args* a, hipStream_t s, const StreamScan
                        reinterpret_cast<const int8_t*>(a->w), a->w_scale, a->lod, a->E, a->n, a->k, a->y, a->ldy, nullptr,
                        reinterpret_cast<const int8_t*>(a->w_tail), a->w_scale_tail, a->tail_row0, a->w_tail ? a->tail_rows : 0,
                        a->tail_src0, a->act_dtype == KMOE_DT_F16, 0, scan ? *scan : StreamScan{}, StreamQuant{},
-                       slots_of(scan, slots)};
+                       nullptr, 0, 0, 0, 0, 0, slots_of(scan, slots)};
   const bool swiglu = a->act == KMOE_ACT_SWIGLU;
   if (scan) {
     if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
@@ -535,7 +605,7 @@ int stream_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s, const StreamSc
   const StreamParams p{reinterpret_cast<const int8_t*>(a->a), a->lda * 2, 64, 0, nullptr, a->row_src, a->src_div,
                        reinterpret_cast<const int8_t*>(a->w), nullptr, a->lod, a->E, a->n, a->k * 2, a->y, a->ldy, nullptr,
                        nullptr, nullptr, 0, 0, 0, half, 0, scan ? *scan : StreamScan{}, StreamQuant{},
-                       slots_of(scan, slots)};
+                       nullptr, 0, 0, 0, 0, 0, slots_of(scan, slots)};
   const bool swiglu = a->act == KMOE_ACT_SWIGLU;
   if (scan) {
     if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
@@ -543,6 +613,45 @@ int stream_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s, const StreamSc
   }
   if (half) return swiglu ? launch_rows16<Fmt::F16, true, false>(p, s) : launch_rows16<Fmt::F16, false, false>(p, s);
   return swiglu ? launch_rows16<Fmt::BF16, true, false>(p, s) : launch_rows16<Fmt::BF16, false, false>(p, s);
+}
+
+// 16-row launches split K two ways and keep one step (128 values) of loads in flight per wave: fewer registers and more
+// waves hide the unpacking and the loads of each other better than a deeper queue does (Qwen3, 64 tokens, layer, steps
+// in flight x split: 1x1 81.7 us, 2x1 81.9, 3x1 83.3, 1x2 78.8, 2x2 81.5; Kimi-K2 dimensions, 128 tokens: 1584 / 1577 /
+// 1606 / 1568 / 1598). Up to 32 columns of a launch with a column per pair do not fill the chip: two steps there (one
+// token 22.5 -> 21.1 and 62 -> 59 us). A caller's variant keeps one wave per K range: the tile kernel's order of sums.
+template <Fmt FMT>
+int stream_w4_shape(const StreamParams& p, bool swiglu, bool scan, int passes, bool split, hipStream_t s) {
+  if (passes == 1 && split && p.slots.n > 0 && p.slots.n <= 32)
+    return scan ? launch_stream<FMT, 1, 2, true, 2, 2, true>(p, s)
+                : (swiglu ? launch_stream<FMT, 1, 2, true, 2, 2>(p, s) : launch_stream<FMT, 1, 2, false, 2, 2>(p, s));
+  if (passes == 1 && split)
+    return scan ? launch_stream<FMT, 1, 2, true, 1, 2, true>(p, s)
+                : (swiglu ? launch_stream<FMT, 1, 2, true, 1, 2>(p, s) : launch_stream<FMT, 1, 2, false, 1, 2>(p, s));
+  if (passes == 1) return swiglu ? launch_stream<FMT, 1, 2, true, 1>(p, s) : launch_stream<FMT, 1, 2, false, 1>(p, s);
+  if (passes == 2)
+    return scan ? launch_stream<FMT, 2, 2, true, 2, 1, true>(p, s)
+                : (swiglu ? launch_stream<FMT, 2, 2, true, 2>(p, s) : launch_stream<FMT, 2, 2, false, 2>(p, s));
+  return swiglu ? launch_stream<FMT, 4, 2, true, 2>(p, s) : launch_stream<FMT, 4, 2, false, 2>(p, s);
+}
+
+int stream_gemm_w4(const kmoe_gemm_w4_args* a, hipStream_t s, int passes, const StreamScan* scan, const StreamSlots* slots) {
+  const int q = a->group_size / 32;
+  int shift = -1;
+  if ((q & (q - 1)) == 0)
+    for (shift = 0; (1 << shift) < q; ++shift) {}
+  const int groups = a->k / a->group_size;
+  const bool frag16 = a->scale_layout == KMOE_S_FRAG16;
+  const bool half = a->act_dtype == KMOE_DT_F16;
+  const StreamParams p{reinterpret_cast<const int8_t*>(a->a), a->lda * 2, 256, 0, nullptr, a->row_src, a->src_div,
+                       reinterpret_cast<const int8_t*>(a->w), nullptr, a->lod, a->E, a->n, a->k / 2, a->y, a->ldy, nullptr,
+                       nullptr, nullptr, 0, 0, 0, half, 0, scan ? *scan : StreamScan{}, StreamQuant{},
+                       a->w_scale, groups, frag16 ? 1 : groups, frag16 ? 16 : 1, q, shift, slots_of(scan, slots)};
+  const bool swiglu = a->act == KMOE_ACT_SWIGLU;
+  if (scan)
+    if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
+  return half ? stream_w4_shape<Fmt::W4H>(p, swiglu, scan != nullptr, passes, a->variant == 0, s)
+              : stream_w4_shape<Fmt::W4>(p, swiglu, scan != nullptr, passes, a->variant == 0, s);
 }
 
 }  // namespace kmoe

@@ -1,8 +1,8 @@
 // Grouped GEMM on 4-bit weights and bf16 activations (W4A16): a weight-streaming kernel for the
 // decode regime and a kernel on 128-row tiles for the prefill regime (further down). In both the
 // packed weights are unpacked in registers and fed to v_mfma_f32_16x16x32_bf16: a quarter of the
-// bytes of the bf16 path; the unpacking (23 VALU instructions per 8 weights) is what bounds the
-// streaming kernel once the bytes are that few, and what the tile kernel shares among 128 rows.
+// bytes of the bf16 path; the unpacking (17 VALU instructions per 8 weights, 13 for half) is what bounds the
+// streaming kernel once the bytes are that few, and what the tile kernel shares among its rows.
 //
 //   weights  [E][n][k/2] bytes, two codes per byte, low nibble first, code c means c - 8
 //            (dequant_int4_native, quantization/kernels/quant_ops.py:71-86), re-arranged by
@@ -14,19 +14,14 @@
 //            g = 0..3 - not a contiguous range, which the sum does not care about.
 //   scales   [E][n][k/group] bf16; a group is a multiple of 32 values, so a lane needs ONE
 //            scale per block: group (128 kb + 32 g) / group_size of its channel.
-//   value    bf16(float(c - 8) * scale), computed as fma(128 + c, scale, -136 scale): both
-//            products and their sum are exact in f32 (8-bit x 8-bit mantissas), so the one
-//            rounding is the bf16 one - the same bits as unpacking first (kmoe_dequant_w4_bf16).
-//   half     (F16 instantiations: activations, scales and results are IEEE half, the dtype
-//            dequant_int4_native itself produces) value = half(c - 8) * scale in half
-//            arithmetic: the code is OR-ed into the mantissa of 1024.0h (whose last place
-//            counts ones), 1032 is subtracted exactly and one packed multiply rounds the
-//            product - the reference's own two steps, two values per instruction.
+//   value    bf16(float(c - 8) * scale) (F16 instantiations: activations, scales and results are IEEE half, the
+//            dtype dequant_int4_native itself produces; value = half(c - 8) * scale in half arithmetic): one
+//            exact fused multiply-add and one rounding, the same bits as unpacking first (kmoe_dequant_w4).
 #include <type_traits>
 
 #include "buffer_ops.h"
 #include "kmoe_common.h"
-#include "pair_scan.h"
+#include "w4_unpack.h"
 
 namespace kmoe {
 namespace {
@@ -35,7 +30,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
 struct W4Params {
   const uint16_t* a;  // [a_rows, k] bf16
@@ -55,221 +49,9 @@ struct W4Params {
   int32_t E, n, k;
   uint16_t* y;
   int64_t ldy;
-  StreamScan scan;  // SCAN instantiations of the streaming kernel: the routed pairs' expert ids instead of lod / row_src
 };
 
 constexpr int kWaves = 4;
-
-// 128 + (byte J of v) as a float, in one full-rate instruction: v_perm_b32 puts the byte into
-// mantissa bits 16-23 of 0x43000000 = 128.0f (whose unit in the last place is 2^-16, so
-// bit 16 counts ones). The integer-to-float conversions run at a fraction of that rate.
-template <int J>
-__device__ inline float byte_plus_128(uint32_t v) {
-  // selector bytes, most significant first: byte 3 of the first source, byte J of the second, zero, zero
-  return __builtin_bit_cast(float, __builtin_amdgcn_perm(0x43000000u, v, 0x07000c0cu | (static_cast<uint32_t>(J) << 16)));
-}
-
-// 8 codes of one 4-byte word -> 8 bf16 values, value 2 j in the low half of register j:
-// 3 instructions split the nibbles into bytes, then per value 1 v_perm and 1 fma
-// ((128 + c) s - 136 s: both products have at most 16 significant bits and their sum is
-// (c - 8) s, so nothing rounds before the bf16 rounding), and 1 rounding per pair
-__device__ inline v4i unpack8(uint32_t word, float s, float m136s) {
-  const uint32_t lo = word & 0x0f0f0f0fu;         // codes 0, 2, 4, 6 in bytes 0..3
-  const uint32_t hi = (word >> 4) & 0x0f0f0f0fu;  // codes 1, 3, 5, 7
-  v4i out;
-  out[0] = static_cast<int>(pack2_bf16(__builtin_fmaf(byte_plus_128<0>(lo), s, m136s), __builtin_fmaf(byte_plus_128<0>(hi), s, m136s)));
-  out[1] = static_cast<int>(pack2_bf16(__builtin_fmaf(byte_plus_128<1>(lo), s, m136s), __builtin_fmaf(byte_plus_128<1>(hi), s, m136s)));
-  out[2] = static_cast<int>(pack2_bf16(__builtin_fmaf(byte_plus_128<2>(lo), s, m136s), __builtin_fmaf(byte_plus_128<2>(hi), s, m136s)));
-  out[3] = static_cast<int>(pack2_bf16(__builtin_fmaf(byte_plus_128<3>(lo), s, m136s), __builtin_fmaf(byte_plus_128<3>(hi), s, m136s)));
-  return out;
-}
-
-// The same 8 codes -> 8 half values (c - 8) * s: pair j is (code 2 j, code 2 j + 1) = byte j of lo and of hi.
-template <int J>
-__device__ inline int unpack2_half(uint32_t lo, uint32_t hi, v2h s2) {
-  // bytes, most significant first: zero, byte J of hi, zero, byte J of lo; then the exponent of 1024.0h on both
-  const uint32_t bits =
-      __builtin_amdgcn_perm(hi, lo, 0x0c000c00u | (static_cast<uint32_t>(4 + J) << 16) | static_cast<uint32_t>(J)) | 0x64006400u;
-  const v2h v = (__builtin_bit_cast(v2h, bits) - (v2h){(_Float16)1032.0f, (_Float16)1032.0f}) * s2;
-  return __builtin_bit_cast(int, v);
-}
-__device__ inline v4i unpack8_half(uint32_t word, v2h s2) {
-  const uint32_t lo = word & 0x0f0f0f0fu;
-  const uint32_t hi = (word >> 4) & 0x0f0f0f0fu;
-  v4i out;
-  out[0] = unpack2_half<0>(lo, hi, s2);
-  out[1] = unpack2_half<1>(lo, hi, s2);
-  out[2] = unpack2_half<2>(lo, hi, s2);
-  out[3] = unpack2_half<3>(lo, hi, s2);
-  return out;
-}
-
-// MF: 16-row fragments per pass over the weights; NF: 16-channel fragments per wave;
-// D: 128-value blocks of loads in flight per wave; F16: half activations, scales and results.
-// SLDS: every wave first copies the scales of its fragments (16 channels x k / group values each, one
-// contiguous piece of the scale tensor) into its own part of LDS and reads a block's scale from there.
-// Read from global memory per block, a lane's 2-byte scale load touches 16 cache lines per instruction
-// (16 channels, rows apart), as many as the weight load next to it moves bytes for: 20 % of the launch.
-// SCAN: the launch sorts the routed pairs by expert itself (pair_scan.h): rows and gather indices come from the
-// pairs' expert ids, and the workgroups of channel block 0 write what the sort's launch would have.
-template <int MF, int NF, bool SWIGLU, int D, bool F16, bool SLDS, bool SCAN = false>
-__global__ __launch_bounds__(kWaves* kWave) void w4_stream_kernel(const W4Params p) {
-  static_assert(!SCAN || kWaves == kScanWaves, "scan_pairs is written for four waves");
-  extern __shared__ uint16_t scale_lds[];  // SLDS: [kWaves][NF][16][groups]
-  __shared__ typename std::conditional<SCAN, PairScanLds, int>::type scan_lds;
-  constexpr int NFH = SWIGLU ? NF / 2 : NF;
-  constexpr int TM = 16 * MF;
-  const int lane = lane_id();
-  const int wave = threadIdx.x >> 6;
-  const int li = lane & 15;
-  const int lg = lane >> 4;
-  const int e = blockIdx.y;
-  int row_begin, row_end;
-  ListedRows listed = {};
-  if constexpr (SCAN) {
-    listed = scan_pairs(p.scan, e, p.E, scan_lds, blockIdx.x == 0);  // (all four waves: a barrier inside)
-    row_begin = listed.begin;
-    row_end = listed.end;
-  } else {
-    row_begin = p.lod[e];
-    row_end = p.lod[e + 1];
-  }
-  if (row_begin >= row_end) return;
-  const int n_half = SWIGLU ? p.n / 2 : p.n;
-  const int col_base = (blockIdx.x * kWaves + wave) * NFH * 16;
-  if (col_base >= n_half) return;
-  const int kblocks = p.k / 128;
-  const int groups = p.k / p.gs;
-  const uint8_t* w_base = p.w + static_cast<size_t>(e) * p.n * (p.k / 2);
-  const uint16_t* s_base = p.scale + static_cast<size_t>(e) * p.n * groups;
-
-  // group of this lane's 32 values of block kb: (128 kb + 32 lg) / gs
-  auto group_of = [&](int kb) { return p.gs_shift >= 0 ? (4 * kb + lg) >> p.gs_shift : (4 * kb + lg) / (p.gs / 32); };
-  const uint8_t* wp[NF];
-  const uint16_t* sp[NF];
-  int soff[NF];  // SLDS: this lane's channel row in the wave's LDS copy
-  bool wok[NF];
-  int col[NF];
-#pragma unroll
-  for (int f = 0; f < NF; ++f) {
-    const int fh = SWIGLU ? f % NFH : f;
-    const int c = col_base + fh * 16;
-    wok[f] = c < n_half;
-    col[f] = (SWIGLU && f >= NFH) ? n_half + c : c;
-    const int ch0 = wok[f] ? col[f] : 0;  // fragments past the last channel read fragment 0: never stored
-    wp[f] = w_base + static_cast<size_t>(ch0 / 16) * kblocks * 1024 + lane * 16;
-    sp[f] = s_base + static_cast<size_t>(ch0) * groups + li * p.s_ch;
-    if constexpr (SLDS) {
-      // the wave's own copy; it alone reads it, so no barrier: a wave's LDS accesses complete in order
-      uint32_t* dst = reinterpret_cast<uint32_t*>(scale_lds + (wave * NF + f) * 16 * groups);
-      const uint32_t* src = reinterpret_cast<const uint32_t*>(s_base + static_cast<size_t>(ch0) * groups);
-      for (int i = lane; i < 8 * groups; i += kWave) dst[i] = src[i];
-      soff[f] = (wave * NF + f) * 16 * groups + li * p.s_ch;
-    }
-  }
-  if constexpr (SLDS) __builtin_amdgcn_wave_barrier();  // the copies above stay above the reads below
-
-  for (int row0 = row_begin; row0 < row_end; row0 += TM) {
-    const uint16_t* ap[MF];
-#pragma unroll
-    for (int mf = 0; mf < MF; ++mf) {
-      const int r = row0 + mf * 16 + li;
-      const int rr = r < row_end ? r : row_begin;  // rows past the end read a valid row: never stored
-      int src;
-      if constexpr (SCAN)
-        src = listed.pair(scan_lds, rr - row_begin) / p.src_div;
-      else
-        src = p.row_src ? p.row_src[rr] / p.src_div : rr;
-      ap[mf] = p.a + static_cast<size_t>(src) * p.lda + 32 * lg;
-    }
-    v4f acc[MF][NF];
-#pragma unroll
-    for (int mf = 0; mf < MF; ++mf)
-#pragma unroll
-      for (int f = 0; f < NF; ++f) acc[mf][f] = (v4f){0.f, 0.f, 0.f, 0.f};
-
-    v4i wreg[D][NF];
-    uint16_t sreg[D][NF];
-    v4i areg[D][MF][4];
-    auto load_block = [&](int slot, int kb) {
-      const int g = group_of(kb);
-#pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        wreg[slot][f] = *reinterpret_cast<const v4i*>(wp[f] + static_cast<size_t>(kb) * 1024);
-        if constexpr (!SLDS) sreg[slot][f] = sp[f][g * p.s_g];
-      }
-#pragma unroll
-      for (int mf = 0; mf < MF; ++mf)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) areg[slot][mf][t] = *reinterpret_cast<const v4i*>(ap[mf] + 128 * kb + 8 * t);
-    };
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-      if (d < kblocks) load_block(d, d);
-
-    for (int kb0 = 0; kb0 < kblocks; kb0 += D) {
-#pragma unroll
-      for (int d = 0; d < D; ++d) {
-        const int kb = kb0 + d;
-        if (kb < kblocks) {
-#pragma unroll
-          for (int f = 0; f < NF; ++f) {
-            if constexpr (SLDS) sreg[d][f] = scale_lds[soff[f] + group_of(kb) * p.s_g];
-            if constexpr (F16) {
-              const _Float16 sh = __builtin_bit_cast(_Float16, sreg[d][f]);
-              const v2h s2 = {sh, sh};
-#pragma unroll
-              for (int t = 0; t < 4; ++t) {
-                const v4i wv = unpack8_half(static_cast<uint32_t>(wreg[d][f][t]), s2);
-#pragma unroll
-                for (int mf = 0; mf < MF; ++mf)
-                  acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wv),
-                                                                      __builtin_bit_cast(v8h, areg[d][mf][t]),
-                                                                      acc[mf][f], 0, 0, 0);
-              }
-            } else {
-              const float s = bf16_to_f32(sreg[d][f]);
-              const float m136s = -136.0f * s;
-#pragma unroll
-              for (int t = 0; t < 4; ++t) {
-                const v4i wv = unpack8(static_cast<uint32_t>(wreg[d][f][t]), s, m136s);
-#pragma unroll
-                for (int mf = 0; mf < MF; ++mf)
-                  acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wv),
-                                                                       __builtin_bit_cast(v8bf, areg[d][mf][t]),
-                                                                       acc[mf][f], 0, 0, 0);
-              }
-            }
-          }
-          if (kb + D < kblocks) load_block(d, kb + D);
-        }
-      }
-    }
-
-    // epilogue: as the bf16 grouped GEMM - round to bf16, optional SiLU-mul on the bf16 values
-#pragma unroll
-    for (int mf = 0; mf < MF; ++mf) {
-      const int r = row0 + mf * 16 + li;
-      if (r >= row_end) continue;
-#pragma unroll
-      for (int f = 0; f < NFH; ++f) {
-        if (!wok[f]) continue;
-        const int c0 = col[f] + lg * 4;
-        uint16_t yv[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) yv[q] = f32_to_act(acc[mf][f][q], F16);
-        if (SWIGLU) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            yv[q] = f32_to_act(silu_hw(act_to_f32(yv[q], F16)) * act_to_f32(f32_to_act(acc[mf][f + NFH][q], F16), F16), F16);
-        }
-        const uint2 packed = make_uint2(yv[0] | (static_cast<uint32_t>(yv[1]) << 16),
-                                        yv[2] | (static_cast<uint32_t>(yv[3]) << 16));
-        *reinterpret_cast<uint2*>(p.y + static_cast<size_t>(r) * p.ldy + c0) = packed;
-      }
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------------------------------
 // Prefill regime: tiles of 64, 96 or 128 rows. The unpacking of a weight word is shared by the row fragments of
@@ -446,13 +228,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
       v4i wv[NF];
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        if constexpr (F16) {
-          const _Float16 sh = __builtin_bit_cast(_Float16, sc[f]);
-          wv[f] = unpack8_half(static_cast<uint32_t>(w[f][t]), (v2h){sh, sh});
-        } else {
-          const float s = bf16_to_f32(sc[f]);
-          wv[f] = unpack8(static_cast<uint32_t>(w[f][t]), s, -136.0f * s);
-        }
+        wv[f] = unpack8(static_cast<uint32_t>(w[f][t]), W4Scale<F16>(sc[f]));
       }
       // two fragments in flight: the read of fragment mf + 1 leaves before the MFMAs of fragment mf
       v4i af[2];
@@ -554,29 +330,6 @@ int launch_w4_tile(const W4Params& p, int rows, bool f16, hipStream_t s) {
   return check_launch("kmoe_grouped_gemm_w4a16");
 }
 
-template <int MF, int NF, bool SWIGLU, int D, bool SCAN = false>
-int launch_w4(const W4Params& p, bool f16, hipStream_t s) {
-  constexpr int NFH = SWIGLU ? NF / 2 : NF;
-  const int n_half = SWIGLU ? p.n / 2 : p.n;
-  const dim3 grid(ceil_div(n_half, kWaves * NFH * 16), p.E);
-  const size_t lds = static_cast<size_t>(kWaves) * NF * 16 * (p.k / p.gs) * sizeof(uint16_t);
-  if (tracing_kernels())
-    note_kernel("w4_stream_kernel<%d rows per pass, %d channel fragments per wave, %s, %d blocks in flight, %s, group scales in %s%s>",
-                16 * MF, NF, SWIGLU ? "SiLU-mul" : "plain", D, f16 ? "f16" : "bf16", lds <= 32 * 1024 ? "LDS" : "global memory",
-                SCAN ? ", sorts the pairs itself" : "");
-  if (lds <= 32 * 1024) {  // beyond: many small groups on a long K; the scales stay in global memory
-    if (f16)
-      hipLaunchKernelGGL((w4_stream_kernel<MF, NF, SWIGLU, D, true, true, SCAN>), grid, dim3(kWaves * kWave), lds, s, p);
-    else
-      hipLaunchKernelGGL((w4_stream_kernel<MF, NF, SWIGLU, D, false, true, SCAN>), grid, dim3(kWaves * kWave), lds, s, p);
-  } else if (f16) {
-    hipLaunchKernelGGL((w4_stream_kernel<MF, NF, SWIGLU, D, true, false, SCAN>), grid, dim3(kWaves * kWave), 0, s, p);
-  } else {
-    hipLaunchKernelGGL((w4_stream_kernel<MF, NF, SWIGLU, D, false, false, SCAN>), grid, dim3(kWaves * kWave), 0, s, p);
-  }
-  return check_launch("kmoe_grouped_gemm_w4a16");
-}
-
 // scales [rows = E * n][groups] -> per 16 rows [groups][16]
 __global__ __launch_bounds__(256) void tile_scales_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
                                                          long long total, int groups) {
@@ -616,10 +369,11 @@ extern "C" int kmoe_tile_scales_w4(const uint16_t* src, uint16_t* dst, int E, in
 }
 
 extern "C" int kmoe_grouped_gemm_w4a16(const kmoe_gemm_w4_args* a, kmoe_stream_t stream) {
-  return grouped_gemm_w4a16_checked(a, stream, nullptr);
+  return grouped_gemm_w4a16_checked(a, stream, nullptr, nullptr);
 }
 
-int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t stream, const StreamScan* scan) {
+int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t stream, const StreamScan* scan,
+                                     const StreamSlots* slots) {
   KMOE_REQUIRE(a, KMOE_ERR_NULL, "grouped_gemm_w4a16: NULL args");
   KMOE_REQUIRE(a->a && a->w && a->w_scale && (a->lod || scan) && a->y, KMOE_ERR_NULL, "grouped_gemm_w4a16: NULL pointer");
   KMOE_REQUIRE(a->E >= 1 && a->rows >= 0, KMOE_ERR_SHAPE, "grouped_gemm_w4a16: E=%d rows=%d", a->E, a->rows);
@@ -650,18 +404,8 @@ int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t s
   const int groups = a->k / a->group_size;
   const bool frag16 = a->scale_layout == KMOE_S_FRAG16;
   const W4Params p{a->a, a->lda, a->row_src, a->src_div, a->w, a->w_scale, a->group_size, shift,
-                   frag16 ? 1 : groups, frag16 ? 16 : 1, a->lod, a->E, a->n, a->k, a->y, a->ldy,
-                   scan ? *scan : StreamScan{}};
+                   frag16 ? 1 : groups, frag16 ? 16 : 1, a->lod, a->E, a->n, a->k, a->y, a->ldy};
   hipStream_t s = as_stream(stream);
-  if (scan) {
-    // the routed gate_up launch of a decode-sized layer, on the streaming kernel
-    const int passes = w4_stream_passes(a->rows, a->rows_hint, a->E, a->k);
-    KMOE_REQUIRE(swiglu && a->variant == 0 && a->row_src == nullptr && passes != 0 && scan->ids && scan->lod &&
-                     scan->expert_m && scan->moe_index && scan->sorted_src && scan->n_pairs == a->rows &&
-                     a->rows <= kStreamScanMaxPairs,
-                 KMOE_ERR_UNSUPPORTED, "grouped_gemm_w4a16: not a launch that can sort the pairs itself");
-    return passes == 1 ? launch_w4<1, 2, true, 1, true>(p, f16, s) : launch_w4<2, 2, true, 2, true>(p, f16, s);
-  }
   int mf = a->variant;
   // the tile kernel reaches a source row (gathered or not: below `rows`) through a 32-bit byte offset
   const bool tile_ok = static_cast<uint64_t>(a->rows) * static_cast<uint64_t>(a->lda) * 2u + static_cast<uint64_t>(a->k) * 2u < (1ull << 32);
@@ -680,22 +424,14 @@ int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t s
     mf = passes ? passes : (!tile_ok ? 4 : (avg <= 48 ? 64 : (avg <= 76 ? 96 : 128)));
   }
   if (mf == 8) mf = 128;
+  KMOE_REQUIRE((!scan && !slots) || mf == 1 || mf == 2, KMOE_ERR_UNSUPPORTED, "grouped_gemm_w4a16: only the weight-streaming kernel sorts the pairs itself");
   if (mf == 64 || mf == 96 || mf == 128)
     KMOE_REQUIRE(tile_ok, KMOE_ERR_SHAPE, "grouped_gemm_w4a16: the tile kernel addresses the activations with 32 bits (rows=%d lda=%lld)",
                  a->rows, static_cast<long long>(a->lda));
   switch (mf) {
-    // One block in flight per wave: the registers that saves put more waves on a SIMD (5-6 instead of 3-4), and
-    // the unpacking work of one wave hides the loads of the others better than a deeper queue of its own does
-    // (Qwen3 decode GEMMs: 52.9 / 31.2 us against 54.2 / 33.1 with two blocks and 55.8 / 34.8 with three).
-    case 1: return swiglu ? launch_w4<1, 2, true, 1>(p, f16, s) : launch_w4<1, 2, false, 1>(p, f16, s);
-    // tuning variants of the 16-row kernel: 1xy = x fragments per wave, y blocks in flight
-    case 123: return swiglu ? launch_w4<1, 2, true, 3>(p, f16, s) : launch_w4<1, 2, false, 3>(p, f16, s);
-    case 141: return swiglu ? launch_w4<1, 4, true, 1>(p, f16, s) : launch_w4<1, 4, false, 1>(p, f16, s);
-    case 124: return swiglu ? launch_w4<1, 2, true, 4>(p, f16, s) : launch_w4<1, 2, false, 4>(p, f16, s);
-    case 142: return swiglu ? launch_w4<1, 4, true, 2>(p, f16, s) : launch_w4<1, 4, false, 2>(p, f16, s);
-    case 143: return swiglu ? launch_w4<1, 4, true, 3>(p, f16, s) : launch_w4<1, 4, false, 3>(p, f16, s);
-    case 2: return swiglu ? launch_w4<2, 2, true, 2>(p, f16, s) : launch_w4<2, 2, false, 2>(p, f16, s);
-    case 4: return swiglu ? launch_w4<4, 2, true, 2>(p, f16, s) : launch_w4<4, 2, false, 2>(p, f16, s);
+    case 1:
+    case 2:
+    case 4: return stream_gemm_w4(a, s, mf, scan, slots);
     case 64: return swiglu ? launch_w4_tile<4, true>(p, a->rows, f16, s) : launch_w4_tile<4, false>(p, a->rows, f16, s);
     case 96: return swiglu ? launch_w4_tile<6, true>(p, a->rows, f16, s) : launch_w4_tile<6, false>(p, a->rows, f16, s);
     case 128: return swiglu ? launch_w4_tile<8, true>(p, a->rows, f16, s) : launch_w4_tile<8, false>(p, a->rows, f16, s);
