@@ -18,6 +18,7 @@
 //            dtype dequant_int4_native itself produces; value = half(c - 8) * scale in half arithmetic): one
 //            exact fused multiply-add and one rounding, the same bits as unpacking first (kmoe_dequant_w4).
 #include <type_traits>
+#include <utility>
 
 #include "buffer_ops.h"
 #include "kmoe_common.h"
@@ -113,13 +114,29 @@ __device__ inline bool locate_w4_item(const W4Params& p, int n_blocks, int& e_ou
   return true;
 }
 
+template <class F, int... I>
+__device__ inline void static_for_each(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ inline void static_for(F&& f) {
+  static_for_each(f, std::make_integer_sequence<int, N>{});
+}
+
 // MF: 16-row fragments of a tile (4, 6, 8: 64-, 96- and 128-row tiles). Two workgroups per CU for every height:
 // with three, the 64-row instance had 170 registers to live in and lost to the 128-row one (121 against 111 us
 // over 4 to 64 rows per expert on the Qwen3 shape); with two it is a quarter ahead where experts fit its tile.
-template <int MF, int NF, bool SWIGLU, bool F16, bool SLDS>
+//
+// RW, RA: blocks of weights (registers) and of activations (LDS) in the rings. A stage waits for its own block, passes a
+// barrier, requests block kb + RA - 1 of the activations and kb + RW - 1 of the weights and multiplies: loads have two
+// to three stages to arrive. With one block in flight (as registers and 64 KB of LDS allow for 128-row tiles) the short
+// tiles, whose stage is half as long, waited for the memory in every stage.
+// No branch sits between a load and its use - the waits count loads - so blocks past the end are requested as well,
+// out of the descriptors' range: they fetch nothing.
+template <int MF, int NF, bool SWIGLU, bool F16, int RW, int RA>
 __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Params p) {
+  static_assert(RW >= RA && RA >= 2, "the weights are requested with the activations of the same block or before");
   constexpr int kTileRows = 16 * MF;
-  extern __shared__ uint16_t scale_lds[];  // SLDS: [kWaves][NF][16][groups], every wave its own part (as in the streaming kernel)
   constexpr int NFH = SWIGLU ? NF / 2 : NF;
   constexpr int NA = kTileRows / 4 / kWaves;  // asynchronous copies per wave and block: 4 rows (1 KB) each
   constexpr int kWaveRows = 4 * NA;           // tile rows a wave copies
@@ -127,24 +144,29 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
   // Row r of a block sits at r * 256; its 16-byte vector v at position v ^ (r % 16): the 16 rows of a
   // fragment read (same vector, rows r, r + 1, ...) fall on 16 different bank groups without padding, which
   // the asynchronous copies (1 KB of consecutive LDS bytes per instruction) could not write.
-  __shared__ __attribute__((aligned(1024))) int8_t lds_a[2][kBufBytes];
+  __shared__ __attribute__((aligned(1024))) int8_t lds_a[RA][kBufBytes];
   const int lane = lane_id();
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15;
   const int lg = lane >> 4;
   const int n_half = SWIGLU ? p.n / 2 : p.n;
   int e, row0, nb;
   if (!locate_w4_item<kTileRows>(p, (n_half + kWaves * NFH * 16 - 1) / (kWaves * NFH * 16), e, row0, nb)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  row0 = __builtin_amdgcn_readfirstlane(row0);
+  nb = __builtin_amdgcn_readfirstlane(nb);
   const int row_end = min(p.lod[e + 1], row0 + kTileRows);
   const int col_base = (nb * kWaves + wave) * NFH * 16;
   const int kblocks = p.k / 128;
   const int groups = p.k / p.gs;
-  const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(p.a);
-  const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(p.w + static_cast<size_t>(e) * p.n * (p.k / 2));
-  const __amdgpu_buffer_rsrc_t s_rsrc = make_rsrc(p.scale + static_cast<size_t>(e) * p.n * groups);
-  auto group_of = [&](int kb) { return p.gs_shift >= 0 ? (4 * kb + lg) >> p.gs_shift : (4 * kb + lg) / (p.gs / 32); };
+  constexpr uint32_t kRange = 0xfffffff0u;
+  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a), 0, kRange, 0x00020000);
+  const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(p.w + static_cast<size_t>(e) * p.n * (p.k / 2)), 0, kRange, 0x00020000);
+  const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(p.scale + static_cast<size_t>(e) * p.n * groups), 0, kRange, 0x00020000);
 
-  uint32_t woff[NF], soff[NF];
+  uint32_t woff[NF], soff[NF];  // scalar: the fragment's first block; vector: the lane's channel in the fragment's scales
   bool wok[NF];
   int col[NF];
 #pragma unroll
@@ -154,17 +176,9 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
     wok[f] = c < n_half;
     col[f] = (SWIGLU && f >= NFH) ? n_half + c : c;
     const int ch0 = wok[f] ? col[f] : 0;  // fragments past the last channel read fragment 0: never stored
-    woff[f] = static_cast<uint32_t>(ch0 / 16) * kblocks * 1024u + lane * 16u;
-    soff[f] = (static_cast<uint32_t>(ch0) * groups + li * p.s_ch) * 2u;
-    if constexpr (SLDS) {
-      uint16_t* mine = scale_lds + (wave * NF + f) * 16 * groups;
-      uint32_t* dst = reinterpret_cast<uint32_t*>(mine);
-      const uint32_t* src = reinterpret_cast<const uint32_t*>(p.scale + (static_cast<size_t>(e) * p.n + ch0) * groups);
-      for (int i = lane; i < 8 * groups; i += kWave) dst[i] = src[i];
-      soff[f] = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)(mine + li * p.s_ch)));  // LDS byte address of the lane's channel
-    }
+    woff[f] = static_cast<uint32_t>(ch0 / 16) * kblocks * 1024u;
+    soff[f] = static_cast<uint32_t>(ch0) * groups * 2u;
   }
-  if constexpr (SLDS) __builtin_amdgcn_wave_barrier();  // the copies above stay above the reads below (a wave's LDS accesses complete in order)
   // copy i of this wave fills tile rows kWaveRows wave + 4 i + lane / 16; the lane fetches the vector that belongs at its position
   uint32_t aoff[NA];
 #pragma unroll
@@ -185,97 +199,107 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
   for (int mf = 0; mf < MF; ++mf)
 #pragma unroll
     for (int f = 0; f < NF; ++f) acc[mf][f] = (v4f){0.f, 0.f, 0.f, 0.f};
-  v4i wbuf[2][NF];
-  uint16_t sbuf[2][NF];
-  auto load_w = [&](v4i(&w)[NF], uint16_t(&sc)[NF], int kb) {
-    const uint32_t g2 = static_cast<uint32_t>(group_of(kb) * p.s_g) * 2u;
+  v4i wbuf[RW][NF];
+  uint16_t sbuf[RW][NF];
+  const uint32_t lane16 = lane * 16u;
+  const uint32_t lane_s = li * p.s_ch * 2u;
+  auto load_w = [&](int slot, int kb) {
+    const bool live = kb < kblocks;
+    const int g32 = 4 * kb + lg;  // this lane's 32 values of the block
+    const uint32_t s_at = lane_s + static_cast<uint32_t>((p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / (p.gs / 32)) * p.s_g) * 2u;
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
-      w[f] = buffer_load16(w_rsrc, woff[f], static_cast<uint32_t>(kb) * 1024u);
-      if constexpr (!SLDS) sc[f] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(s_rsrc, soff[f] + g2, 0, 0));
-    }
-    if constexpr (SLDS) {
-      // reads the compiler does not see (it would drain the asynchronous copies in flight before them); the wait is
-      // part of the statement, so the values are there when it ends
-      static_assert(NF == 4, "four scale reads per block");
-      uint32_t s0, s1, s2, s3;
-      asm volatile(
-          "ds_read_u16 %0, %4\n\t"
-          "ds_read_u16 %1, %5\n\t"
-          "ds_read_u16 %2, %6\n\t"
-          "ds_read_u16 %3, %7\n\t"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(s0), "=&v"(s1), "=&v"(s2), "=&v"(s3)
-          : "v"(soff[0] + g2), "v"(soff[1] + g2), "v"(soff[2] + g2), "v"(soff[3] + g2)
-          : "memory");
-      sc[0] = static_cast<uint16_t>(s0);
-      sc[1] = static_cast<uint16_t>(s1);
-      sc[2] = static_cast<uint16_t>(s2);
-      sc[3] = static_cast<uint16_t>(s3);
+      wbuf[slot][f] = buffer_load16(w_rsrc, lane16, live ? woff[f] + static_cast<uint32_t>(kb) * 1024u : kRange);
+      sbuf[slot][f] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(s_rsrc, s_at, live ? soff[f] : kRange, 0));
     }
   };
-  auto dma_a = [&](int kb, int buf) {
+  auto dma_a = [&](int buf, int kb) {
+    const uint32_t at = kb < kblocks ? static_cast<uint32_t>(kb) * 256u : kRange;
 #pragma unroll
     for (int i = 0; i < NA; ++i)
-      buffer_load16_to_lds(a_rsrc, (lds_ptr_t)&lds_a[buf][(kWaveRows * wave + 4 * i) * 256], aoff[i], static_cast<uint32_t>(kb) * 256u);
+      buffer_load16_to_lds(a_rsrc, (lds_ptr_t)&lds_a[buf][(kWaveRows * wave + 4 * i) * 256], aoff[i], at);
   };
-  // one block: word t of a lane's 16 packed bytes is its operand of MFMA step t; the activation lane (lg, row)
-  // supplies values 32 lg + 8 t + [0, 8) of the block, i.e. vector 4 lg + t of the row's 16
-  auto compute = [&](const v4i(&w)[NF], const uint16_t(&sc)[NF], auto buf_tag) {
+  constexpr int kLoadsW = 2 * NF;
+  // loads of a wave younger than those a stage needs
+  constexpr int kYounger = RW == RA ? (RA - 2) * (NA + kLoadsW) : (RA - 1) * kLoadsW + (RA - 2) * NA;
+  // One block: word t of a lane's 16 packed bytes is its operand of MFMA step t; the activation lane (lg, row)
+  // supplies values 32 lg + 8 t + [0, 8) of the block, i.e. vector 4 lg + t of the row's 16. The words of step t + 1
+  // are unpacked between the row fragments of step t: the matrix and the vector unit both have work from one wave.
+  auto compute = [&](auto slot_tag, auto buf_tag) {
+    constexpr int slot = decltype(slot_tag)::value;
     constexpr int buf = decltype(buf_tag)::value;
+    const W4Scale<F16> sc[NF] = {W4Scale<F16>(sbuf[slot][0]), W4Scale<F16>(sbuf[slot][1]), W4Scale<F16>(sbuf[slot][2]),
+                                 W4Scale<F16>(sbuf[slot][3])};
+    // Row fragments are read two ahead, across the steps: fragment i = t MF + mf of the block's 4 MF.
+    v4i af[3];
+    auto request = [&](auto i_tag) {
+      constexpr int i = decltype(i_tag)::value;
+      // (the offset field of an LDS read reaches 64 KB)
+      constexpr int off = buf * kBufBytes + (i % MF) * 16 * 256;
+      af[i % 3] = off < 65536 ? lds_read16_raw<(off < 65536 ? off : 0)>(fa[i / MF])
+                              : lds_read16_raw<(off < 65536 ? 0 : off - 65536)>(fa[i / MF] + 65536u);
+    };
+    request(std::integral_constant<int, 0>{});
+    request(std::integral_constant<int, 1>{});
+    v4i wv[2][NF];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      v4i wv[NF];
+    for (int f = 0; f < NF; ++f) wv[0][f] = unpack8(static_cast<uint32_t>(wbuf[slot][f][0]), sc[f]);
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<4 * MF>([&](auto i_tag) {
+      constexpr int i = decltype(i_tag)::value;
+      constexpr int t = i / MF, mf = i % MF;
+      if constexpr (i + 2 < 4 * MF) {
+        request(std::integral_constant<int, i + 2>{});
+        lds_wait<2>(af[i % 3]);
+      } else if constexpr (i + 1 < 4 * MF) {
+        lds_wait<1>(af[i % 3]);
+      } else {
+        lds_wait<0>(af[i % 3]);
+      }
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        wv[f] = unpack8(static_cast<uint32_t>(w[f][t]), W4Scale<F16>(sc[f]));
+        if constexpr (F16)
+          acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wv[t & 1][f]),
+                                                              __builtin_bit_cast(v8h, af[i % 3]), acc[mf][f], 0, 0, 0);
+        else
+          acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wv[t & 1][f]),
+                                                               __builtin_bit_cast(v8bf, af[i % 3]), acc[mf][f], 0, 0, 0);
       }
-      // two fragments in flight: the read of fragment mf + 1 leaves before the MFMAs of fragment mf
-      v4i af[2];
-      af[0] = lds_read16_raw<buf * kBufBytes>(fa[t]);
+      if constexpr (t < 3) {
 #pragma unroll
-      for (int mf = 0; mf < MF; ++mf) {
-        if (mf + 1 < MF) {
-          asm volatile("ds_read_b128 %0, %1 offset:%2"
-                       : "=v"(af[(mf + 1) & 1])
-                       : "v"(fa[t]), "n"(buf * kBufBytes + (mf + 1) * 16 * 256)
-                       : "memory");
-          lds_wait<1>(af[mf & 1]);
-        } else {
-          lds_wait<0>(af[mf & 1]);
-        }
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          if constexpr (F16)
-            acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wv[f]),
-                                                                __builtin_bit_cast(v8h, af[mf & 1]), acc[mf][f], 0, 0, 0);
-          else
-            acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wv[f]),
-                                                                 __builtin_bit_cast(v8bf, af[mf & 1]), acc[mf][f], 0, 0, 0);
-        }
+        for (int f = 0; f < NF; ++f)
+          if (f * MF / NF == mf) wv[(t + 1) & 1][f] = unpack8(static_cast<uint32_t>(wbuf[slot][f][t + 1]), sc[f]);
       }
-    }
+      __builtin_amdgcn_sched_barrier(0);  // (all the unpacking of a block at once would not fit the registers)
+    });
   };
-  // The block after the current one is requested (weights and scales into registers, activations into the other
-  // LDS buffer, which every wave finished reading before the barrier that ended the previous stage) before the
-  // MFMAs of the current one; the wait at the end covers all of it, the barrier publishes the copies.
-  auto stage = [&](int kb, const v4i(&w)[NF], const uint16_t(&sc)[NF], v4i(&w_next)[NF], uint16_t(&sc_next)[NF], auto buf_tag) {
-    constexpr int buf = decltype(buf_tag)::value;
-    if (kb + 1 < kblocks) {
-      dma_a(kb + 1, buf ^ 1);
-      load_w(w_next, sc_next, kb + 1);
-    }
-    compute(w, sc, buf_tag);
-    vmem_wait<0>();
-    __syncthreads();
+  auto stage = [&](int kb, auto u_tag) {
+    constexpr int u = decltype(u_tag)::value;
+    vmem_wait<kYounger>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    dma_a((u + RA - 1) % RA, kb + RA - 1);
+    load_w((u + RW - 1) % RW, kb + RW - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(std::integral_constant<int, u % RW>{}, std::integral_constant<int, u % RA>{});
   };
-  dma_a(0, 0);
-  load_w(wbuf[0], sbuf[0], 0);
-  vmem_wait<0>();
-  __syncthreads();
-  for (int kb = 0; kb < kblocks; kb += 2) {
-    stage(kb, wbuf[0], sbuf[0], wbuf[1], sbuf[1], std::integral_constant<int, 0>{});
-    if (kb + 1 < kblocks) stage(kb + 1, wbuf[1], sbuf[1], wbuf[0], sbuf[0], std::integral_constant<int, 1>{});
+#pragma unroll
+  for (int i = 1 - RW; i < 0; ++i) {
+    if (i + RA - 1 >= 0) dma_a(i + RA - 1, i + RA - 1);
+    load_w(i + RW - 1, i + RW - 1);
+  }
+  constexpr int U = RW % RA == 0 ? RW : RW * RA;  // stages until both rings are back where they were
+  // (no exit inside the body: as one basic block it fits the registers. Stages past the last block multiply what the
+  // descriptors' ends returned, zeros by zeros.)
+  for (int kb0 = 0; kb0 < kblocks; kb0 += U) {
+    stage(kb0, std::integral_constant<int, 0>{});
+    stage(kb0 + 1, std::integral_constant<int, 1 % U>{});
+    if constexpr (U > 2) stage(kb0 + 2, std::integral_constant<int, 2 % U>{});
+    if constexpr (U > 3) stage(kb0 + 3, std::integral_constant<int, 3 % U>{});
+    if constexpr (U > 4) {
+      stage(kb0 + 4, std::integral_constant<int, 4 % U>{});
+      stage(kb0 + 5, std::integral_constant<int, 5 % U>{});
+    }
   }
 
   // epilogue: as the streaming kernel - round to the activation type, optional SiLU-mul on the rounded values
@@ -312,20 +336,24 @@ int launch_w4_tile(const W4Params& p, int rows, bool f16, hipStream_t s) {
   const int n_blocks = ceil_div(n_half, kWaves * NFH * 16);
   const int items = (rows / kTileRows + min(p.E, rows)) * n_blocks;
   const dim3 grid(ceil_div(items, 8) * 8);
-  // the scales of a wave's fragments in LDS, while two workgroups still fit a CU next to their activation buffers
-  const size_t lds = static_cast<size_t>(kWaves) * NF * 16 * (p.k / p.gs) * sizeof(uint16_t);
-  if (tracing_kernels())
-    note_kernel("w4_tile_kernel<%d-row tiles, %s, %s, group scales in %s>", kTileRows, SWIGLU ? "SiLU-mul" : "plain",
-                f16 ? "f16" : "bf16", lds <= 16 * 1024 ? "LDS" : "global memory");
-  if (lds <= 16 * 1024) {
+  // Blocks in flight: what the registers (weights) and 80 KB of LDS (activations) hold. A launch runs whole turns of
+  // its rings, so a 64-row tile takes three blocks where four would leave more stages without a block (k = 768: 6 blocks).
+  auto go = [&](auto ring_tag) {
+    constexpr int R = decltype(ring_tag)::value;
+    if (tracing_kernels())
+      note_kernel("w4_tile_kernel<%d-row tiles, %s, %s, %d blocks in flight>", kTileRows, SWIGLU ? "SiLU-mul" : "plain",
+                  f16 ? "f16" : "bf16", R);
     if (f16)
-      hipLaunchKernelGGL((w4_tile_kernel<MF, NF, SWIGLU, true, true>), grid, dim3(kWaves * kWave), lds, s, p);
+      hipLaunchKernelGGL((w4_tile_kernel<MF, NF, SWIGLU, true, R, R>), grid, dim3(kWaves * kWave), 0, s, p);
     else
-      hipLaunchKernelGGL((w4_tile_kernel<MF, NF, SWIGLU, false, true>), grid, dim3(kWaves * kWave), lds, s, p);
-  } else if (f16) {
-    hipLaunchKernelGGL((w4_tile_kernel<MF, NF, SWIGLU, true, false>), grid, dim3(kWaves * kWave), 0, s, p);
+      hipLaunchKernelGGL((w4_tile_kernel<MF, NF, SWIGLU, false, R, R>), grid, dim3(kWaves * kWave), 0, s, p);
+  };
+  const int kblocks = p.k / 128;
+  if constexpr (MF == 4) {
+    if (ceil_div(kblocks, 4) * 4 <= ceil_div(kblocks, 3) * 3) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, 3>{});
   } else {
-    hipLaunchKernelGGL((w4_tile_kernel<MF, NF, SWIGLU, false, false>), grid, dim3(kWaves * kWave), 0, s, p);
+    go(std::integral_constant<int, MF == 6 ? 3 : 2>{});
   }
   return check_launch("kmoe_grouped_gemm_w4a16");
 }

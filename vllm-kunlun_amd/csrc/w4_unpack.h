@@ -21,6 +21,7 @@ struct W4Scale;
 template <>
 struct W4Scale<false> {
   float lo, hi, m8;  // s 2^24, s 2^20, -8 s
+  W4Scale() = default;
   __device__ explicit W4Scale(uint16_t bits) {
     const float s = bf16_to_f32(bits);
     lo = s * 0x1p24f;
@@ -31,6 +32,7 @@ struct W4Scale<false> {
 template <>
 struct W4Scale<true> {
   w4_v2h s2;
+  W4Scale() = default;
   __device__ explicit W4Scale(uint16_t bits) {
     const _Float16 s = __builtin_bit_cast(_Float16, bits);
     s2 = w4_v2h{s, s};
