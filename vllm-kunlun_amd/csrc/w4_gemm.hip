@@ -114,6 +114,27 @@ __device__ inline bool locate_w4_item(const W4Params& p, int n_blocks, int& e_ou
   return true;
 }
 
+// The four MFMAs of row fragment `mf`, left out if the tile has no rows there: a branch the compiler does not see, so the
+// K loop stays one basic block (with a visible one the accumulators spill). The compare and the branch are the two
+// wait states between the unpacking's last write and the first MFMA that reads it.
+template <bool F16, int MF_INDEX>
+__device__ __forceinline__ void mfma4_if_live(v4f (&c)[4], const v4i (&w)[4], const v4i& a, int live_frags) {
+#define KMOE_W4_MFMA4(OP)                                                                                              \
+  asm volatile("s_cmp_le_i32 %[live], %[mf]\n\t"                                                                       \
+               "s_cbranch_scc1 1f\n\t" OP " %[c0], %[w0], %[a], %[c0]\n\t" OP " %[c1], %[w1], %[a], %[c1]\n\t" OP         \
+               " %[c2], %[w2], %[a], %[c2]\n\t" OP " %[c3], %[w3], %[a], %[c3]\n"                                        \
+               "1:"                                                                                                    \
+               : [c0] "+v"(c[0]), [c1] "+v"(c[1]), [c2] "+v"(c[2]), [c3] "+v"(c[3])                                     \
+               : [w0] "v"(w[0]), [w1] "v"(w[1]), [w2] "v"(w[2]), [w3] "v"(w[3]), [a] "v"(a), [live] "s"(live_frags),     \
+                 [mf] "n"(MF_INDEX)                                                                                    \
+               : "scc")
+  if constexpr (F16)
+    KMOE_W4_MFMA4("v_mfma_f32_16x16x32_f16");
+  else
+    KMOE_W4_MFMA4("v_mfma_f32_16x16x32_bf16");
+#undef KMOE_W4_MFMA4
+}
+
 template <class F, int... I>
 __device__ inline void static_for_each(F&& f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, I>{}), ...);
@@ -135,7 +156,7 @@ __device__ inline void static_for(F&& f) {
 // out of the descriptors' range: they fetch nothing.
 template <int MF, int NF, bool SWIGLU, bool F16, int RW, int RA>
 __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Params p) {
-  static_assert(RW >= RA && RA >= 2, "the weights are requested with the activations of the same block or before");
+  static_assert(NF == 4 && RW >= RA && RA >= 2, "the weights are requested with the activations of the same block or before");
   constexpr int kTileRows = 16 * MF;
   constexpr int NFH = SWIGLU ? NF / 2 : NF;
   constexpr int NA = kTileRows / 4 / kWaves;  // asynchronous copies per wave and block: 4 rows (1 KB) each
@@ -156,6 +177,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
   row0 = __builtin_amdgcn_readfirstlane(row0);
   nb = __builtin_amdgcn_readfirstlane(nb);
   const int row_end = min(p.lod[e + 1], row0 + kTileRows);
+  const int live_frags = __builtin_amdgcn_readfirstlane((row_end - row0 + 15) / 16);  // row fragments that hold rows
   const int col_base = (nb * kWaves + wave) * NFH * 16;
   const int kblocks = p.k / 128;
   const int groups = p.k / p.gs;
@@ -256,15 +278,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
       } else {
         lds_wait<0>(af[i % 3]);
       }
-#pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        if constexpr (F16)
-          acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wv[t & 1][f]),
-                                                              __builtin_bit_cast(v8h, af[i % 3]), acc[mf][f], 0, 0, 0);
-        else
-          acc[mf][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wv[t & 1][f]),
-                                                               __builtin_bit_cast(v8bf, af[i % 3]), acc[mf][f], 0, 0, 0);
-      }
+      mfma4_if_live<F16, mf>(acc[mf], wv[t & 1], af[i % 3], live_frags);
       if constexpr (t < 3) {
 #pragma unroll
         for (int f = 0; f < NF; ++f)
@@ -302,6 +316,8 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
     }
   }
 
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs' results, which the compiler does not know to wait for
+  __builtin_amdgcn_sched_barrier(0);
   // epilogue: as the streaming kernel - round to the activation type, optional SiLU-mul on the rounded values
 #pragma unroll
   for (int mf = 0; mf < MF; ++mf) {
