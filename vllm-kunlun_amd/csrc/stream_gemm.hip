@@ -59,7 +59,7 @@ struct StreamParams {
   const float* w_aux_tail;
   int32_t tail_row0, tail_rows, tail_src0;
   int32_t f16;  // outputs (and the rounding of gate and up before SiLU-mul) in IEEE half instead of bf16
-  int32_t rotate;  // every wave starts its K range at a step of its own (see run_i8)
+  int32_t rotate;  // every wave starts its K range at a step of its own (see stream_gemm_i8)
   StreamScan scan;    // SCAN instantiations: the routed pairs' expert ids instead of lod / row_src
   StreamQuant quant;  // QUANT instantiations: the rows as bf16 / half values instead of codes and row maxes
   // W4: group scales. Element strides inside the 16 x (k / group) scales of a fragment (16 channels), which start at
@@ -91,7 +91,7 @@ constexpr int kQuantStride = kStreamQuantMaxK + 16;  // bytes between the rows o
 // per wave at a time, and leave absmax and codes - the arithmetic of quant_i8_rows_body, hence its bits - in LDS,
 // where the K loop reads its row fragments; a and a_aux are not read. The workgroups of channel block 0 also write
 // codes (chunk-major) and row maxes where the quantiser's launch would have left them. Built for four waves per
-// SIMD (see run_i8).
+// SIMD (see stream_gemm_i8).
 template <Fmt FMT, int MF, int NF, bool SWIGLU, int D, int KS, bool SCAN = false, bool QUANT = false>
 __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kernel(const StreamParams p) {
   static_assert(!SCAN || kWaves == kScanWaves, "scan_pairs is written for four waves");
@@ -562,6 +562,17 @@ int stream_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s, const StreamScan* 
     if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
     KMOE_REQUIRE(a->a_rows <= kStreamScanMaxRows, KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8 (stream): %d tokens", a->a_rows);
     return launch_rows16<Fmt::I8, true, true>(p, s);
+  }
+  if (a->variant == 0 && a->rows == 0 && !swiglu) {
+    // A dense matrix (a tail expert alone) has n channels of workgroups and no experts to fill the chip with, so every
+    // launch has its four waves share K. Slices of 16 rows up to 64 of them, of 32 beyond (every slice reads the weights
+    // from the caches again); one channel fragment per wave where two would leave half of the 256 CUs without a
+    // workgroup. With the quantiser, [4096 x 7168] / [7168 x 2048], and 16 or 32 rows per slice by two fragments and two
+    // steps in flight at every size before: 1 row 15.2 -> 12.5 / 9.4 -> 9.0 us, 32 rows 15.7 -> 13.9 / 10.3, 100 rows
+    // 21.4 -> 20.2 / 15.2 -> 14.4, 256 rows 36.1 -> 29.8 / 23.7 -> 21.3. Slices of 64 rows and four fragments per wave
+    // are level at 192 to 256 rows and 10 to 40 % slower below.
+    if (a->tail_rows <= 32 && a->n <= 4096) return launch_stream<Fmt::I8, 1, 1, false, 4, 4>(p, s);
+    return a->tail_rows <= 64 ? launch_stream<Fmt::I8, 1, 2, false, 4, 4>(p, s) : launch_stream<Fmt::I8, 2, 2, false, 2, 4>(p, s);
   }
   // m-fragments per pass from the rows an expert gets under uniform routing
   int mf = a->variant;

@@ -13,8 +13,8 @@ typedef _Float16 w4_v2h __attribute__((ext_vector_type(2)));
 // bf16: value (c - 8) s is ONE fused multiply-add on the code's bits read as a half. A nibble alone in the low 8 bits
 // of a half is the subnormal c 2^-24 (in the upper half of a byte: c 2^-20), which v_fma_mix_f32 widens for free:
 // c 2^-24 * s 2^24 - 8 s, whose product and sum are exact in f32 (a code has 4 significant bits, a scale 8), so the one
-// rounding is the one to bf16. half: v_fma_mixlo_f16 would do the whole of it, but issues at half the rate (4.5 against
-// 2.5 clocks per instruction and SIMD), so the code is OR-ed into the mantissa of 1024.0h (whose last place counts
+// rounding is the one to bf16. half: v_fma_mixlo_f16 would do the whole of it, but issues at half the rate (8.45 against
+// 4.75 clocks per instruction and SIMD), so the code is OR-ed into the mantissa of 1024.0h (whose last place counts
 // ones), 1032 subtracted exactly and one packed multiply rounds the product.
 template <bool F16>
 struct W4Scale;

@@ -490,14 +490,15 @@ def _ones(device: torch.device, count: int) -> torch.Tensor:
 @operator("_C::silu_and_mul", mutates_args=("out",))
 def silu_and_mul(out: torch.Tensor, x: torch.Tensor, axis: int = -1, turn: bool = True) -> None:
     """out = silu(x[..., :d]) * x[..., d:] (reference: ops/_custom_ops.py:699-706)."""
-    L.require_device(out, x)
-    L.require_contig(out, x)
-    dt = _dt(x, "silu_and_mul")
+    if not (out.is_cuda and x.is_cuda and out.is_contiguous() and x.is_contiguous()):
+        L.require_device(out, x)
+        L.require_contig(out, x)
+    dt = L.act_dtype(x, "silu_and_mul")
     _need(out.dtype == x.dtype, "silu_and_mul: out and x must share a dtype")
     two_i = x.shape[-1]
-    R = x.numel() // two_i
-    _need(two_i % 2 == 0 and out.numel() == R * (two_i // 2), "silu_and_mul: out must be [..., d] for x [..., 2d]")
-    L.check(L.lib.kmoe_silu_and_mul_dt(L.ptr(x), two_i, R, two_i // 2, L.ptr(out), two_i // 2, dt, L.stream()))
+    R, d = x.numel() // two_i, two_i // 2
+    _need(two_i % 2 == 0 and out.numel() == R * d, "silu_and_mul: out must be [..., d] for x [..., 2d]")
+    L.check(L.lib.kmoe_silu_and_mul_dt(x.data_ptr(), two_i, R, d, out.data_ptr(), d, dt, L.raw_stream()))
 
 
 @operator("_C::moe_post", mutates_args=("y",))

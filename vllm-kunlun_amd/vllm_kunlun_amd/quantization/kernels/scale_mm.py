@@ -21,7 +21,8 @@ from typing import Optional
 import torch
 
 from ... import _lib as L
-from ..._plan import WORKSPACE, tile_int8_weights_, weight_layout
+from ... import _plan
+from ..._plan import tile_int8_weights_, weight_layout
 
 
 @dataclass
@@ -32,6 +33,101 @@ class Int8ScaledMMLinearLayerConfig:
     input_symmetric: bool = True
 
 
+_ROW_RANGES: dict = {}  # (device, rows) -> the {0, rows} row range of a dense GEMM's single expert, made once
+
+
+def _row_range(device, rows):
+    key = (device, rows)
+    if key not in _ROW_RANGES:
+        _ROW_RANGES[key] = torch.tensor([0, rows], dtype=torch.int32).to(device)
+    return _ROW_RANGES[key]
+
+
+class _DynamicCall:
+    """Quantisation and GEMM of one Linear with dynamic symmetric activations: the GEMM's argument block with everything
+    but the batch filled in, kept on the layer. A call is two launches on a scratch buffer of the stream (codes, then row
+    maxes) and one allocation, the output: 11 us of host time where building the block and looking the parameters up on
+    every call took 21."""
+
+    __slots__ = ("args", "n", "k", "device", "scale", "weight", "at", "epoch", "tiled")
+
+    # Up to this many rows the GEMM runs on the weight-streaming kernel (the one the fused MoE layer
+    # runs decode batches and its folded shared expert on): the dense matrix is handed over as the
+    # launch's "tail expert", whose rows the kernel cuts into slices of 16 or 32 for as many
+    # workgroups - a tile kernel has too few tiles to fill the chip here. Measured on
+    # [M,7168] x [4096,7168]: 13 us against 36 us at 16 rows, 20 against 38 at 128, 30 against 38 at 256;
+    # at 512 rows the tile kernel is ahead (39 against 46 us).
+    STREAM_MAX_ROWS = 256
+
+    def __init__(self, layer, names, w, w_max):
+        L.require_device(w, w_max)
+        L.require_contig(w, w_max)
+        _, self.n, self.k = w.shape
+        self.device = w.device
+        params = self._params(layer)
+        self.weight, self.scale = params.get(names[0]), params.get(names[1])
+        self.at = (w.data_ptr(), w_max.data_ptr())
+        self.epoch = _plan._layout_epoch
+        layout = weight_layout(w)
+        self.tiled = layout == L.KMOE_W_TILED
+        g = L.GemmI8Args()
+        g.w, g.w_max = self.at
+        g.E, g.n, g.k, g.lda, g.ldy, g.src_div = 1, self.n, self.k, self.k, self.n, 1
+        g.act, g.w_layout = L.KMOE_ACT_NONE, layout
+        self.args = g
+
+    @staticmethod
+    def _params(layer) -> dict:
+        return layer.__dict__.get("_parameters", layer.__dict__)  # (a plain object holds them as attributes)
+
+    def holds(self, layer, names) -> bool:
+        """Whether the layer's parameters are still the ones the block was filled from."""
+        params = self._params(layer)
+        w, scale = layer.__dict__.get("_kmoe_w_1nk"), params.get(names[1])
+        return (scale is self.scale and params.get(names[0]) is self.weight and w is not None
+                and w.data_ptr() == self.at[0] and scale.data_ptr() == self.at[1] and params.get(names[2]) is None
+                and params.get(names[4]) is None and self.epoch == _plan._layout_epoch)
+
+    def __deepcopy__(self, memo):
+        return None  # (a copied layer fills a block of its own)
+
+    def __reduce__(self):
+        return type(None), ()
+
+    def __call__(self, x: torch.Tensor) -> torch.Tensor:
+        dt = L.act_dtype(x, "KunlunScaledMMLinearKernel")
+        flat = x.dim() == 2 and x.is_contiguous()
+        x2 = x if flat else x.reshape(-1, x.shape[-1]).contiguous()
+        M, k = x2.shape
+        n = self.n
+        if k != self.k:
+            raise ValueError(f"KunlunScaledMMLinearKernel: rows of {k} values for weights of {self.k}")
+        if x2.device != self.device:
+            raise RuntimeError(f"kmoe ops run on the GPU only; got a tensor on {x2.device}")
+        out = x2.new_empty((M, n))
+        if M:
+            codes = -(-M * k // 256) * 256
+            stream = L.raw_stream()
+            if torch._C._cuda_isCurrentStreamCapturing():
+                scratch = torch.empty(codes + 4 * M, dtype=torch.uint8, device=self.device)  # the graph's own
+            else:
+                scratch = _plan.WORKSPACE.get(codes + 4 * M, self.device, L.raw_stream(self.device.index))
+            g = L.GemmI8Args.from_buffer_copy(self.args)  # a copy: threads may share the block
+            g.a = x_q = scratch.data_ptr()
+            g.a_max = x_max = x_q + codes
+            g.y, g.act_dtype = out.data_ptr(), dt
+            if self.tiled and M <= self.STREAM_MAX_ROWS:
+                L.check(L.lib.kmoe_quant_i8_rows_chunked_dt(x2.data_ptr(), k, M, k, x_q, x_max, dt, stream))
+                # one routed expert without rows (the launch needs an expert list), the matrix as the tail expert
+                g.a_layout, g.a_rows, g.lod = L.KMOE_A_CHUNKED, M, _row_range(self.device, 0).data_ptr()
+                g.w_tail, g.w_max_tail, g.tail_rows = self.at[0], self.at[1], M
+            else:
+                L.check(L.lib.kmoe_quant_i8_rows_dt(x2.data_ptr(), k, M, k, x_q, k, x_max, dt, stream))
+                g.lod, g.rows = _row_range(self.device, M).data_ptr(), M
+            L.check(L.lib.kmoe_grouped_gemm_i8(g, stream))
+        return out if flat else out.reshape(*x.shape[:-1], n)
+
+
 class KunlunScaledMMLinearKernel:
     def __init__(self, c: Optional[Int8ScaledMMLinearLayerConfig] = None, w_q_param_name: str = "weight",
                  w_s_param_name: str = "weight_scale", i_s_param_name: str = "input_scale",
@@ -39,7 +135,6 @@ class KunlunScaledMMLinearKernel:
         self.config = c or Int8ScaledMMLinearLayerConfig()
         self.layer_param_names = (w_q_param_name, w_s_param_name, i_s_param_name, i_zp_param_name,
                                   azp_adj_param_name)
-        self._lod = {}  # (device, rows) -> the {0, rows} row range of the single expert, made once
 
     @classmethod
     def is_supported(cls, compute_capability: Optional[int] = None) -> tuple[bool, Optional[str]]:
@@ -132,6 +227,9 @@ class KunlunScaledMMLinearKernel:
         """Reference: scale_mm.py:52-90. The symmetric branch: quantise per token (dynamic) or with the
         layer's one input scale (static), multiply, rescale by x_max * w_max / 127^2, in x's dtype.
         Output [..., n]."""
+        call = layer.__dict__.get("_kmoe_dynamic")
+        if call is not None and bias is None and call.holds(layer, self.layer_param_names):
+            return call(x)
         w_q, w_s, x_s, x_zp, azp_adj = self._get_layer_params(layer)
         if azp_adj is not None:
             return self._apply_asymmetric(layer, x, w_q, w_s, x_s, x_zp, azp_adj, bias)
@@ -143,24 +241,23 @@ class KunlunScaledMMLinearKernel:
             out = torch.ops._C.matmul(x_q, w_q.transpose(0, 1), x.dtype, x_pc_max=x_s2 * 127.0 if static else x_s2,
                                       w_pc_max=w_s.data, bias=bias.to(torch.float32).contiguous())
             return out.reshape(*x.shape[:-1], out.shape[-1])
-        dt = L.act_dtype(x, "KunlunScaledMMLinearKernel")
+        L.act_dtype(x, "KunlunScaledMMLinearKernel")
         w = getattr(layer, "_kmoe_w_1nk", None)
         if w is None:
             raise RuntimeError("KunlunScaledMMLinearKernel: process_weights_after_loading has not run on this layer")
         from ...ops import _custom_ops as ops  # registers torch.ops._C.*
         lead = x.shape[:-1]
-        x2 = x if x.dim() == 2 and x.is_contiguous() else x.reshape(-1, x.shape[-1]).contiguous()
-        (M, k), n = x2.shape, w.shape[1]
-        if k != w.shape[2]:
-            raise ValueError(f"KunlunScaledMMLinearKernel: rows of {k} values for weights of {w.shape[2]}")
+        if x_s is None:
+            layer.__dict__["_kmoe_dynamic"] = call = _DynamicCall(layer, self.layer_param_names, w, w_s)
+            return call(x)
+        x2 = x.reshape(-1, x.shape[-1]).contiguous()
+        M, n = x2.shape[0], w.shape[1]
         out = torch.empty((M, n), dtype=x.dtype, device=x.device)
-        if M and x_s is not None:  # static: one scale for the tensor, so every row's max is scale x 127
+        if M:  # static: one scale for the tensor, so every row's max is scale x 127
             x_q, x_s, _, _ = torch.ops._C.scaled_int8_quant(x2, x_s.data.to(torch.float32).reshape(1), None, True)
             x_max = (x_s * 127.0).expand(M).contiguous()
             ops._gemm_i8(x_q, x_max, w, w_s.data.reshape(-1), self._row_range(x.device, M), out, n, L.KMOE_ACT_NONE, M)
-        elif M:
-            self._dynamic_gemm(x2, w, w_s, out, dt)
-        return out if x.dim() == 2 else out.reshape(*lead, n)
+        return out.reshape(*lead, n)
 
     def _apply_asymmetric(self, layer, x, w_q, w_s, x_s, x_zp, azp_adj, bias):
         """Reference: scale_mm.py:60-82. Codes with a zero point (per token, or the layer's static one), the int8
@@ -177,48 +274,5 @@ class KunlunScaledMMLinearKernel:
             None if bias is None else bias.to(torch.float32).contiguous())
         return out.reshape(*lead, out.shape[-1])
 
-    # Up to this many rows the GEMM runs on the weight-streaming kernel (the one the fused MoE layer
-    # runs decode batches and its folded shared expert on): the dense matrix is handed over as the
-    # launch's "tail expert", whose rows the kernel cuts into slices of 16 or 32 for as many
-    # workgroups - a tile kernel has too few tiles to fill the chip here. Measured on
-    # [M,7168] x [4096,7168]: 16 us against 36 us at 16 rows, 25 against 38 at 128, 31 against 38 at 256;
-    # at 512 rows the tile kernel is ahead (39 against 46 us).
-    STREAM_MAX_ROWS = 256
-
     def _row_range(self, device, rows):
-        key = (device, rows)
-        if key not in self._lod:
-            self._lod[key] = torch.tensor([0, rows], dtype=torch.int32).to(device)
-        return self._lod[key]
-
-    def _dynamic_gemm(self, x2, w, w_max, out, dt):
-        """Quantisation and GEMM of one call on a scratch buffer of the stream: codes, then row maxes. Two calls into
-        the library and one allocation (the output)."""
-        L.require_device(x2, w, w_max)
-        M, k = x2.shape
-        n = w.shape[1]
-        codes = -(-M * k // 256) * 256
-        stream = L.raw_stream()
-        if torch._C._cuda_isCurrentStreamCapturing():
-            scratch = torch.empty(codes + 4 * M, dtype=torch.uint8, device=x2.device)  # the graph's own
-        else:
-            scratch = WORKSPACE.get(codes + 4 * M, x2.device, L.raw_stream(x2.device.index))
-        x_q = scratch.data_ptr()
-        x_max = x_q + codes
-        layout = weight_layout(w)
-        tail = layout == L.KMOE_W_TILED and M <= self.STREAM_MAX_ROWS
-        g = L.GemmI8Args()
-        g.a, g.lda, g.a_max, g.src_div = x_q, k, x_max, 1
-        g.w, g.w_max = w.data_ptr(), w_max.data_ptr()
-        g.E, g.n, g.k = 1, n, k
-        g.y, g.ldy, g.act, g.w_layout, g.act_dtype = out.data_ptr(), n, L.KMOE_ACT_NONE, layout, dt
-        if tail:
-            L.check(L.lib.kmoe_quant_i8_rows_chunked_dt(x2.data_ptr(), k, M, k, x_q, x_max, dt, stream))
-            # one routed expert without rows (the launch needs an expert list), the matrix as the tail expert
-            g.a_layout, g.a_rows, g.lod, g.rows = L.KMOE_A_CHUNKED, M, self._row_range(x2.device, 0).data_ptr(), 0
-            g.w_tail, g.w_max_tail, g.tail_rows = g.w, g.w_max, M
-            g.variant = 1 if M <= 128 else 2  # 16 or 32 rows per slice
-        else:
-            L.check(L.lib.kmoe_quant_i8_rows_dt(x2.data_ptr(), k, M, k, x_q, k, x_max, dt, stream))
-            g.lod, g.rows = self._row_range(x2.device, M).data_ptr(), M
-        L.check(L.lib.kmoe_grouped_gemm_i8(g, stream))
+        return _row_range(device, rows)
