@@ -56,3 +56,26 @@ def test_kept_argument_block_follows_the_call():
         on_side = m.apply_monolithic(sl.layer, sl.x, sl.logits)
     torch.cuda.synchronize()
     assert torch.equal(on_side, want)
+
+
+# pairs and experts on both sides of every choice of launches, the last chunk full and not, ids of other ranks' experts
+@pytest.mark.parametrize("P", [0, 255, 256, 257, 1024, 1025, 8192, 8193, 24576, 24577, 131073, 300000])
+@pytest.mark.parametrize("E,first", [(1, 0), (256, 0), (257, 3), (1000, 0)])
+def test_stable_sort_by_expert(P, E, first):
+    from vllm_kunlun_amd import _lib as L
+    ids = torch.randint(first - 2, first + E + 2, (P,), generator=torch.Generator().manual_seed(P + E)).clamp(min=0)
+    ids[: P // 3] = first + E // 2
+    local = torch.where((ids >= first) & (ids < first + E), ids - first, torch.full_like(ids, E))
+    order = torch.argsort(local, stable=True)
+    counts = torch.bincount(local, minlength=E + 1)[:E]
+    kept = int(counts.sum())
+    index = torch.full((P,), -1)
+    index[order[:kept]] = torch.arange(kept)
+    nbytes = L.lib.kmoe_align_workspace_bytes(P, E)
+    dev = ids.int().cuda()
+    out = [torch.full((n,), -7, dtype=torch.int32, device="cuda") for n in (max(P, 1), max(P, 1), E, E + 1)]
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    L.check(L.lib.kmoe_align_local(L.ptr(dev), P, E, first, *(L.ptr(t) for t in out), L.ptr(ws), nbytes, L.stream()))
+    moe_index, sorted_src, expert_m, lod = (t.cpu().long() for t in out)
+    assert torch.equal(moe_index[:P], index) and torch.equal(sorted_src[:kept], order[:kept])
+    assert torch.equal(expert_m, counts) and torch.equal(lod, torch.cat([torch.zeros(1), counts.cumsum(0)]).long())

@@ -1,7 +1,7 @@
 // moe_align: stable counting sort of routed pairs by expert id, built from LDS
 // histograms, a per-expert scan and wavefront ballot ranks.
 //
-// Decomposition: the P pairs are cut into chunks of kChunk consecutive pairs,
+// Decomposition: the P pairs are cut into chunks of kThreads*steps consecutive pairs,
 // one workgroup each; inside a chunk wave w owns the next kWave*steps pairs.
 // The sorted row of pair j with expert e is
 //   lod[e] + (#pairs of e in earlier chunks) + (#pairs of e in earlier waves /
@@ -15,8 +15,18 @@ namespace {
 constexpr int kThreads = 1024;            // workgroup size of the multi-workgroup kernels
 constexpr int kWaves = kThreads / kWave;  // 16
 constexpr int kMaxE = 1024;
-constexpr int kSingleMaxP = 4096;         // one workgroup handles up to this many pairs
-constexpr int kChunk = 2048;              // pairs per workgroup in the multi-workgroup path
+// Launches by the number of pairs. One workgroup of 256 threads and cheap barriers up to 256 pairs and experts (3.3 us a
+// call in a row of calls; 4.1 by the next). One launch of P / 1024 workgroups that each count every pair: 4.2 us at 512
+// pairs, 5.3 at 4096, 5.7 at 6216, 7.5 at 16384, 10.6 at 32768 (one workgroup for all took 4.5 us at 512 and 9.1 at 4096,
+// launches for the histograms, their scan and the scatter 10.0 at 6216, 10.3 at 16384, 11.2 at 32768). Two launches beyond,
+// where reading all the ids in every workgroup costs more than the second launch: 9.3 us at 32768 pairs, 9.4 at 65536
+// (three: 13.2), 22 at 2^20 (76). With other kernels around, a second launch costs some 2 us more than in such a row.
+constexpr int kSingleMaxP = 256, kSingleMaxE = 256;
+constexpr int kOneLaunchMaxP = 24576;
+constexpr int kMaxChunks = 128;           // workgroups of the two-launch path at most
+
+// two-launch path: pairs per thread
+inline int chunk_steps(int P) { return max(2, ceil_div(P, kMaxChunks * kThreads)); }
 
 __device__ inline int key_bits(int E) { return 32 - __builtin_clz(max(E - 1, 1)); }
 
@@ -110,7 +120,7 @@ __device__ inline void scatter_chunk(const IdView ids, int begin, int end, int E
 
 // Exclusive scan of cnt[0..E) by one workgroup (blockDim.x >= E): a shuffle scan
 // inside each wave, then the wave totals through LDS. Writes lod[0..E] and
-// expert_m, and leaves lod[e] also in out_base[e]. `wtot` is LDS scratch of 16 ints.
+// expert_m (where they are given), and leaves lod[e] also in out_base[e]. `wtot` is LDS scratch of 16 ints.
 __device__ inline void scan_experts(int my_count /* thread e < E */, int E, int* wtot, int* out_base,
                                     int32_t* __restrict__ lod, int32_t* __restrict__ expert_m) {
   const int t = threadIdx.x;
@@ -128,92 +138,141 @@ __device__ inline void scan_experts(int my_count /* thread e < E */, int E, int*
   if (t < E) {
     const int excl = before + incl - my_count;
     out_base[t] = excl;
-    lod[t] = excl;
+    if (lod) lod[t] = excl;
     if (expert_m) expert_m[t] = my_count;
-    if (t == E - 1) lod[E] = before + incl;
+    if (lod && t == E - 1) lod[E] = before + incl;
   }
   __syncthreads();
 }
 
-// Single-workgroup path (P <= kSingleMaxP); blockDim.x is 256 or 1024, >= E.
-__global__ __launch_bounds__(kThreads) void align_single_kernel(
-    const IdView ids, int P, int E, int steps, int32_t* __restrict__ moe_index,
+// One workgroup of 256 threads, one pair each (P <= kSingleMaxP, E <= kSingleMaxE).
+__global__ __launch_bounds__(kSingleMaxP) void align_single_kernel(
+    const IdView ids, int P, int E, int32_t* __restrict__ moe_index,
     int32_t* __restrict__ sorted_src, int32_t* __restrict__ expert_m, int32_t* __restrict__ lod) {
   extern __shared__ int lds[];
   int* wtot = lds;          // [16]
   int* base = wtot + 16;    // [E]
   int* wcnt = base + E;     // [waves][E]
-  const int mine = count_chunk(ids, 0, P, E, steps, wcnt);
+  const int mine = count_chunk(ids, 0, P, E, 1, wcnt);
   scan_experts(mine, E, wtot, base, lod, expert_m);
-  scatter_chunk(ids, 0, P, E, steps, base, wcnt, moe_index, sorted_src);
+  scatter_chunk(ids, 0, P, E, 1, base, wcnt, moe_index, sorted_src);
 }
 
-// Multi-workgroup path, kernel 1: chunk histograms -> hist[chunk][E].
-__global__ __launch_bounds__(kThreads) void align_hist_kernel(const IdView ids, int P, int E,
+// One launch for several workgroups (P <= kOneLaunchMaxP): workgroup b owns the kThreads pairs of chunk b, one per
+// thread, and counts ALL the pairs itself - those of earlier chunks apart from the rest - so that it knows where its
+// chunk begins in every expert without waiting for another workgroup. Bound by latencies: a launch, the round trip of
+// the ids (eight loads in flight per thread), the barriers and the scan.
+__global__ __launch_bounds__(kThreads) void align_one_launch_kernel(
+    const IdView ids, int P, int E, int32_t* __restrict__ moe_index, int32_t* __restrict__ sorted_src,
+    int32_t* __restrict__ expert_m, int32_t* __restrict__ lod) {
+  extern __shared__ int lds[];
+  int* wtot = lds;           // [16]
+  int* base = wtot + 16;     // [E]
+  int* before = base + E;    // [E]: pairs of earlier chunks
+  int* rest = before + E;    // [E]: the others
+  int* wcnt = rest + E;      // [kWaves][E]
+  const int t = threadIdx.x, wave = t >> 6;
+  const int begin = blockIdx.x * kThreads;
+  const int key = load_key(ids, begin + t, P, E);
+  constexpr int kBatch = 8;
+  int v[kBatch];
+  auto load = [&](int j0) {
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) v[i] = load_key(ids, j0 + i * kThreads + t, P, E);
+  };
+  load(0);
+  for (int i = t; i < (2 + kWaves) * E; i += kThreads) before[i] = 0;
+  __syncthreads();
+  int rank, count;
+  wave_match_rank(key, key_bits(E), rank, count);
+  if (key >= 0 && rank == 0) wcnt[wave * E + key] = count;
+  for (int j0 = 0; j0 < P; j0 += kBatch * kThreads) {
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i)
+      if (v[i] >= 0) atomicAdd((j0 + i * kThreads < begin ? before : rest) + v[i], 1);  // (chunks are whole: uniform)
+    load(j0 + kBatch * kThreads);
+  }
+  __syncthreads();
+  int earlier = 0, total = 0;
+  if (t < E) {
+    earlier = before[t];
+    total = earlier + rest[t];
+    int mine = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const int c = wcnt[w * E + t];
+      wcnt[w * E + t] = mine;
+      mine += c;
+    }
+  }
+  scan_experts(total, E, wtot, base, blockIdx.x == 0 ? lod : nullptr, blockIdx.x == 0 ? expert_m : nullptr);
+  if (begin + t >= P) return;
+  if (key < 0) {
+    moe_index[begin + t] = -1;
+    return;
+  }
+  const int pos = base[key] + before[key] + wcnt[wave * E + key] + rank;
+  moe_index[begin + t] = pos;
+  if (sorted_src) sorted_src[pos] = begin + t;
+}
+
+// Two launches for more pairs than that, chunks of `steps` x kThreads pairs. Kernel 1: chunk histograms ->
+// hist[chunk][E].
+__global__ __launch_bounds__(kThreads) void align_hist_kernel(const IdView ids, int P, int E, int steps,
                                                              int32_t* __restrict__ hist) {
   extern __shared__ int lds[];
   for (int e = threadIdx.x; e < E; e += kThreads) lds[e] = 0;
   __syncthreads();
-  const int begin = blockIdx.x * kChunk;
-  const int end = min(P, begin + kChunk);
+  const int begin = blockIdx.x * steps * kThreads;
+  const int end = min(P, begin + steps * kThreads);
   for (int j = begin + threadIdx.x; j < end; j += kThreads) {
-    const int e = ids[j];
-    if (static_cast<unsigned>(e) < static_cast<unsigned>(E)) atomicAdd(&lds[e], 1);
+    const int e = load_key(ids, j, end, E);
+    if (e >= 0) atomicAdd(&lds[e], 1);
   }
   __syncthreads();
   for (int e = threadIdx.x; e < E; e += kThreads) hist[static_cast<size_t>(blockIdx.x) * E + e] = lds[e];
 }
 
-// Kernel 2 (one workgroup): per-expert prefix over chunks, then lod; hist is
-// rewritten in place to the sorted row where each chunk's expert-e pairs begin.
-__global__ __launch_bounds__(kThreads) void align_scan_kernel(int E, int n_chunks, int32_t* __restrict__ hist,
-                                                             int32_t* __restrict__ expert_m,
-                                                             int32_t* __restrict__ lod) {
-  __shared__ int scan[16];
-  __shared__ int base[kMaxE];
-  const int e = threadIdx.x;
-  int total = 0;
-  constexpr int kBatch = 8;  // loads of a batch are independent: one memory round trip per 8 chunks, not per chunk
-  if (e < E) {
-    for (int c0 = 0; c0 < n_chunks; c0 += kBatch) {
-      int v[kBatch];
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) v[i] = c0 + i < n_chunks ? hist[static_cast<size_t>(c0 + i) * E + e] : 0;
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        if (c0 + i < n_chunks) hist[static_cast<size_t>(c0 + i) * E + e] = total;
-        total += v[i];
-      }
-    }
-  }
-  scan_experts(total, E, scan, base, lod, expert_m);
-  if (e < E) {
-    const int b = base[e];
-    for (int c0 = 0; c0 < n_chunks; c0 += kBatch) {
-      int v[kBatch];
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) v[i] = c0 + i < n_chunks ? hist[static_cast<size_t>(c0 + i) * E + e] : 0;
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i)
-        if (c0 + i < n_chunks) hist[static_cast<size_t>(c0 + i) * E + e] = v[i] + b;
-    }
-  }
-}
-
-// Kernel 3: stable scatter of each chunk.
-__global__ __launch_bounds__(kThreads) void align_scatter_kernel(const IdView ids, int P, int E,
+// Kernel 2: stable scatter of each chunk. Every workgroup sums the (at most kMaxChunks) histograms itself, the earlier
+// chunks' apart: kThreads / E threads per expert, eight loads in flight each.
+__global__ __launch_bounds__(kThreads) void align_scatter_kernel(const IdView ids, int P, int E, int steps, int n_chunks,
                                                                 const int32_t* __restrict__ hist,
                                                                 int32_t* __restrict__ moe_index,
-                                                                int32_t* __restrict__ sorted_src) {
+                                                                int32_t* __restrict__ sorted_src,
+                                                                int32_t* __restrict__ expert_m, int32_t* __restrict__ lod) {
   extern __shared__ int lds[];
-  int* base = lds;       // [E]
-  int* wcnt = base + E;  // [kWaves][E]
-  for (int e = threadIdx.x; e < E; e += kThreads) base[e] = hist[static_cast<size_t>(blockIdx.x) * E + e];
-  const int begin = blockIdx.x * kChunk;
-  const int end = min(P, begin + kChunk);
-  count_chunk(ids, begin, end, E, kChunk / kThreads, wcnt);
+  int* wtot = lds;         // [16]
+  int* base = wtot + 16;   // [E]
+  int* before = base + E;  // [E]: pairs of earlier chunks
+  int* rest = before + E;  // [E]: the others
+  int* wcnt = rest + E;    // [kWaves][E]
+  const int t = threadIdx.x, me = blockIdx.x;
+  for (int i = t; i < 2 * E; i += kThreads) before[i] = 0;
+  const int begin = me * steps * kThreads;
+  const int end = min(P, begin + steps * kThreads);
+  count_chunk(ids, begin, end, E, steps, wcnt);  // (its barriers publish the zeros)
+  const int parts = kThreads / E, part = t / E, e = t - part * E;
+  if (part < parts) {
+    constexpr int kBatch = 8;
+    int lo = 0, hi = 0;
+    for (int c0 = part; c0 < n_chunks; c0 += kBatch * parts) {
+      int v[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int c = c0 + i * parts;
+        v[i] = c < n_chunks ? hist[static_cast<size_t>(c) * E + e] : 0;
+      }
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) (c0 + i * parts < me ? lo : hi) += v[i];
+    }
+    if (lo) atomicAdd(&before[e], lo);
+    if (hi) atomicAdd(&rest[e], hi);
+  }
   __syncthreads();
-  scatter_chunk(ids, begin, end, E, kChunk / kThreads, base, wcnt, moe_index, sorted_src);
+  scan_experts(t < E ? before[t] + rest[t] : 0, E, wtot, base, me == 0 ? lod : nullptr, me == 0 ? expert_m : nullptr);
+  if (t < E) base[t] += before[t];
+  __syncthreads();
+  scatter_chunk(ids, begin, end, E, steps, base, wcnt, moe_index, sorted_src);
 }
 
 __global__ void block_statistic_kernel(const int32_t* __restrict__ ids, int P, int E, int per_block,
@@ -247,8 +306,8 @@ __global__ void gather_rows_kernel(const uint16_t* __restrict__ src, int64_t ld_
 using namespace kmoe;
 
 extern "C" size_t kmoe_align_workspace_bytes(int P, int E) {
-  if (P <= kSingleMaxP || E <= 0) return 256;  // unused, but never report zero
-  return align_up(static_cast<size_t>(ceil_div(P, kChunk)) * E * sizeof(int32_t), 256);
+  if (P <= kOneLaunchMaxP || E <= 0) return 256;  // unused, but never report zero
+  return align_up(static_cast<size_t>(ceil_div(P, chunk_steps(P) * kThreads)) * E * sizeof(int32_t), 256);
 }
 
 extern "C" int kmoe_align(const int32_t* topk_ids, int P, int E, int32_t* moe_index, int32_t* sorted_src,
@@ -266,25 +325,28 @@ extern "C" int kmoe_align_local(const int32_t* ids_global, int P, int E, int fir
   KMOE_REQUIRE(E >= 1 && E <= kMaxE, KMOE_ERR_SHAPE, "align: E=%d outside [1,%d]", E, kMaxE);
   KMOE_REQUIRE(P >= 0 && P <= (1 << 24), KMOE_ERR_SHAPE, "align: P=%d outside [0,2^24]", P);
   hipStream_t s = as_stream(stream);
-  if (P <= kSingleMaxP) {
-    const int threads = (E <= 256 && P <= 512) ? 256 : kThreads;  // few waves: cheap barriers for decode sizes
-    const int steps = max(1, ceil_div(P, threads));
-    const size_t lds = sizeof(int) * (16 + E + static_cast<size_t>(threads / kWave) * E);
-    hipLaunchKernelGGL(align_single_kernel, dim3(1), dim3(threads), lds, s, topk_ids, P, E, steps, moe_index,
-                       sorted_src, expert_m, lod);
+  if (P <= kSingleMaxP && E <= kSingleMaxE) {
+    const size_t lds = sizeof(int) * (16 + E + static_cast<size_t>(kSingleMaxP / kWave) * E);
+    hipLaunchKernelGGL(align_single_kernel, dim3(1), dim3(kSingleMaxP), lds, s, topk_ids, P, E, moe_index, sorted_src,
+                       expert_m, lod);
     return check_launch("kmoe_align");
   }
-  const int n_chunks = ceil_div(P, kChunk);
+  if (P <= kOneLaunchMaxP) {
+    hipLaunchKernelGGL(align_one_launch_kernel, dim3(max(1, ceil_div(P, kThreads))), dim3(kThreads),
+                       sizeof(int) * (16 + (3 + static_cast<size_t>(kWaves)) * E), s, topk_ids, P, E, moe_index, sorted_src,
+                       expert_m, lod);
+    return check_launch("kmoe_align");
+  }
+  const int steps = chunk_steps(P), n_chunks = ceil_div(P, steps * kThreads);
   const size_t need = static_cast<size_t>(n_chunks) * E * sizeof(int32_t);
   KMOE_REQUIRE(workspace, KMOE_ERR_WORKSPACE, "align: workspace is NULL (need %zu bytes)", need);
   KMOE_REQUIRE(workspace_bytes >= need, KMOE_ERR_WORKSPACE, "align: workspace %zu < %zu bytes", workspace_bytes,
                need);
   int32_t* hist = static_cast<int32_t*>(workspace);
-  hipLaunchKernelGGL(align_hist_kernel, dim3(n_chunks), dim3(kThreads), sizeof(int) * E, s, topk_ids, P, E, hist);
-  hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(kThreads), 0, s, E, n_chunks, hist, expert_m, lod);
+  hipLaunchKernelGGL(align_hist_kernel, dim3(n_chunks), dim3(kThreads), sizeof(int) * E, s, topk_ids, P, E, steps, hist);
   hipLaunchKernelGGL(align_scatter_kernel, dim3(n_chunks), dim3(kThreads),
-                     sizeof(int) * (E + static_cast<size_t>(kWaves) * E), s, topk_ids, P, E, hist, moe_index,
-                     sorted_src);
+                     sizeof(int) * (16 + (3 + static_cast<size_t>(kWaves)) * E), s, topk_ids, P, E, steps, n_chunks, hist,
+                     moe_index, sorted_src, expert_m, lod);
   return check_launch("kmoe_align");
 }
 
