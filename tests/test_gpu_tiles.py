@@ -1,0 +1,43 @@
+"""The tile kernel on 16-bit operands: every tile height at the edges of its row fragments (which are skipped past an
+expert's rows) and of the tile, against a float32 product of the same values."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 15, 16, 17, 0, 95, 96, 97, 33, 127, 128, 129, 191, 192, 193, 400]
+
+
+@pytest.mark.parametrize("variant", [6, 11, 13, 18])  # 128, 64, 96 and 192 rows
+@pytest.mark.parametrize("n,k", [(64, 128), (320, 96), (256, 608)])  # an odd number of 64-byte steps; several periods
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_row_fragments(variant, n, k, act, dtype):
+    from vllm_kunlun_amd import _lib as L
+    gen = torch.Generator().manual_seed(n + k)
+    E, rows, n_out = len(ROWS), sum(ROWS), n // 2 if act else n
+    # (a source row per sorted row, not its own: the rows are gathered)
+    src = torch.randperm(rows, generator=gen)
+    a = torch.randn(rows, k, generator=gen).to(dtype).cuda()
+    w = (torch.randn(E, n, k, generator=gen) * 0.05).to(dtype).cuda()
+    tiled = torch.empty_like(w)
+    L.check(L.lib.kmoe_tile_weights_i8(w.data_ptr(), tiled.data_ptr(), E, n, 2 * k, L.stream()))
+    lod = torch.tensor([0] + ROWS).cumsum(0).int().cuda()
+    dsrc = src.int().cuda()
+    y = torch.full((rows, n_out), float("nan"), dtype=dtype, device="cuda")
+    g = L.GemmBf16Args()
+    g.a, g.lda, g.row_src, g.src_div = a.data_ptr(), k, dsrc.data_ptr(), 1
+    g.w, g.w_layout, g.lod = tiled.data_ptr(), L.KMOE_W_TILED, lod.data_ptr()
+    g.E, g.n, g.k, g.rows = E, n, k, rows
+    g.y, g.ldy, g.act, g.variant = y.data_ptr(), n_out, act, variant
+    g.act_dtype = L.act_dtype(a, "test")
+    L.check(L.lib.kmoe_grouped_gemm_bf16(g, L.stream()))
+    ref = torch.cat([a[src[lo:lo + c]].float() @ w[e].float().T
+                     for e, (c, lo) in enumerate(zip(ROWS, lod.tolist()))])
+    if act:
+        gate, up = (t.to(dtype).float() for t in ref.split(n_out, 1))
+        ref = torch.nn.functional.silu(gate) * up
+    got = y.float()
+    assert not got.isnan().any()
+    per_row = (got - ref).norm(dim=1) / ref.norm(dim=1).clamp(min=1e-6)
+    assert float((got - ref).norm() / ref.norm()) <= 4e-3 and float(per_row.max()) <= 2e-2

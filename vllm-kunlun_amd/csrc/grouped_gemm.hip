@@ -418,7 +418,7 @@ int launch(const GemmParams& p, int rows, hipStream_t s, const char* what) {
 // and it is bound by the weight bytes either way (measured cross-over: 8 to 16 rows, all three formats).
 constexpr int kTiledMinRows = kStreamMaxRows;
 // variants of the bf16 and fp8 launchers that force the tile kernel: 5 (tile height from the rows per expert),
-// 6 (128-row tiles), 11 (64-row tiles)
+// 6 (128-row tiles), 11 (64-row tiles), 13 (96-row tiles); bf16 also 18 (192-row wide tiles)
 inline bool tile_variant(int v) { return v == 5 || v == 6 || (v >= 11 && v <= 13); }
 
 template <Kind KIND>
@@ -537,11 +537,12 @@ int grouped_gemm_bf16_checked(const kmoe_gemm_bf16_args* a, kmoe_stream_t stream
   if (a->w_layout == KMOE_W_TILED && a->variant == 0 && !a->bias && !oai && streams_bf16(live, a->E, a->k))
     return stream_gemm_bf16(a, as_stream(stream), scan, slots);
   KMOE_REQUIRE(!scan && !slots, KMOE_ERR_UNSUPPORTED, "grouped_gemm_bf16: only the weight-streaming kernel sorts the pairs itself");
-  // tiled weights and more rows: the persistent tile kernel (variants 5, 6, 11 force it)
+  // tiled weights and more rows: the persistent tile kernel (variants 5, 6, 11-13, 18 force it)
+  const bool forced = tile_variant(a->variant) || a->variant == 18;
   if (a->w_layout == KMOE_W_TILED && a->k >= 64 && a->ldy % 8 == 0 &&
-      (tile_variant(a->variant) || (a->variant == 0 && ceil_div(live, a->E) > kTiledMinRows)))
+      (forced || (a->variant == 0 && ceil_div(live, a->E) > kTiledMinRows)))
     return tiled_gemm_bf16(a, as_stream(stream));
-  KMOE_REQUIRE(!tile_variant(a->variant), KMOE_ERR_UNSUPPORTED, "grouped_gemm_bf16: variants 5, 6, 11-13 need tiled weights, k >= 64 and ldy %% 8 == 0");
+  KMOE_REQUIRE(!forced, KMOE_ERR_UNSUPPORTED, "grouped_gemm_bf16: variants 5, 6, 11-13 and 18 need tiled weights, k >= 64 and ldy %% 8 == 0");
   GemmParams p{reinterpret_cast<const int8_t*>(a->a), a->lda * 2, nullptr, a->row_src, a->src_div,
                reinterpret_cast<const int8_t*>(a->w), nullptr,    a->lod,  a->E,       a->n,
                a->k * 2,                              a->y,       a->ldy,  nullptr, a->w_layout == KMOE_W_TILED,

@@ -528,15 +528,16 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
   };
   // fragment n of a step: (row fragment, K part); 16x16: 8 row fragments; 32x32: 2 K parts x 4
   constexpr int kFragReads = M32 ? 2 * AM : kMF;
-  // Row fragments of this wave that hold rows of the current tile (wave-uniform, set per tile): the K loop of the
-  // int8 path neither reads nor multiplies the others (the padding of an expert's last tile).
+  // Row fragments of this wave that hold rows of the current tile (wave-uniform, set per tile): the K loop neither
+  // reads nor multiplies the others (the padding of an expert's last tile).
+  constexpr bool kSkips = ADMA && !F8 && !M32;
   int live_frags = kMF;
-  // One row fragment of one MFMA step, int8: LDS read of the NEXT live fragment, wait for this one's, NF MFMAs -
+  // One row fragment of one MFMA step: LDS read of the NEXT live fragment, wait for this one's, NF MFMAs -
   // all inside one assembly statement, because the skip is a branch: a branch the compiler can see splits the
   // loop body into basic blocks, after which its register allocator spills hundreds of registers. `live` is
   // wave-uniform (an SGPR); a live fragment falls through its test, a dead one costs a compare and a taken branch.
   // LDS operations of a wave complete in order, so "at most one in flight" means this fragment's read has landed.
-  auto frag_i8 = [&](const v4i(&w)[kNF], v4i& af_cur, v4i& af_next, uint32_t addr, auto n_tag, auto off_own, auto off_next,
+  auto frag_step = [&](const v4i(&w)[kNF], v4i& af_cur, v4i& af_next, uint32_t addr, auto n_tag, auto off_own, auto off_next,
                      int mf) {
     constexpr int n = decltype(n_tag)::value;
     constexpr bool kFirst = n == 0, kLast = n + 1 == kMF;
@@ -550,54 +551,41 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
 // If the next fragment is dead its bytes arrive unused, and the wait at the end of the step retires the request.
 #define KMOE_FRAG_NEXT "ds_read_b128 %[nxt], %[addr] offset:%[onext]\n\ts_waitcnt lgkmcnt(1)\n\t"
 #define KMOE_FRAG_WAIT "s_waitcnt lgkmcnt(0)\n\t"
-#define KMOE_FRAG_MFMA2                                          \
-  "v_mfma_i32_16x16x64_i8 %[c0], %[w0], %[cur], %[c0]\n\t"       \
-  "v_mfma_i32_16x16x64_i8 %[c1], %[w1], %[cur], %[c1]\n\t"
-#define KMOE_FRAG_MFMA4                                          \
-  KMOE_FRAG_MFMA2                                                \
-  "v_mfma_i32_16x16x64_i8 %[c2], %[w2], %[cur], %[c2]\n\t"       \
-  "v_mfma_i32_16x16x64_i8 %[c3], %[w3], %[cur], %[c3]\n\t"
+#define KMOE_FRAG_MFMA2(OP) OP " %[c0], %[w0], %[cur], %[c0]\n\t" OP " %[c1], %[w1], %[cur], %[c1]\n\t"
+#define KMOE_FRAG_MFMA4(OP) \
+  KMOE_FRAG_MFMA2(OP) OP " %[c2], %[w2], %[cur], %[c2]\n\t" OP " %[c3], %[w3], %[cur], %[c3]\n\t"
 #define KMOE_FRAG_IMMS                                                                                       \
   [addr] "v"(addr), [live] "s"(live_frags), [n1] "n"(n + 1), [own] "n"(decltype(off_own)::value), \
       [onext] "n"(decltype(off_next)::value)
-    if constexpr (kNF == 4) {
-#define KMOE_FRAG_ACC [c0] "+v"(acc[mf][0]), [c1] "+v"(acc[mf][1]), [c2] "+v"(acc[mf][2]), [c3] "+v"(acc[mf][3])
-#define KMOE_FRAG_W [w0] "v"(w[0]), [w1] "v"(w[1]), [w2] "v"(w[2]), [w3] "v"(w[3])
-      if constexpr (kFirst && kLast)
-        asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_OWN KMOE_FRAG_WAIT KMOE_FRAG_MFMA4 "3:\n\t"
-                     : KMOE_FRAG_ACC, [cur] "=&v"(af_cur) : KMOE_FRAG_W, KMOE_FRAG_IMMS : "scc", "memory");
-      else if constexpr (kFirst)
-        asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_OWN KMOE_FRAG_NEXT KMOE_FRAG_MFMA4 "3:\n\t"
-                     : KMOE_FRAG_ACC, [cur] "=&v"(af_cur), [nxt] "=&v"(af_next) : KMOE_FRAG_W, KMOE_FRAG_IMMS
-                     : "scc", "memory");
-      else if constexpr (kLast)
-        asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_WAIT KMOE_FRAG_MFMA4 "3:\n\t"
-                     : KMOE_FRAG_ACC : KMOE_FRAG_W, [cur] "v"(af_cur), KMOE_FRAG_IMMS : "scc", "memory");
-      else
-        asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_NEXT KMOE_FRAG_MFMA4 "3:\n\t"
-                     : KMOE_FRAG_ACC, [nxt] "=&v"(af_next) : KMOE_FRAG_W, [cur] "v"(af_cur), KMOE_FRAG_IMMS
-                     : "scc", "memory");
-#undef KMOE_FRAG_ACC
-#undef KMOE_FRAG_W
+#define KMOE_FRAG_ACC2 [c0] "+v"(acc[mf][0]), [c1] "+v"(acc[mf][1])
+#define KMOE_FRAG_ACC4 KMOE_FRAG_ACC2, [c2] "+v"(acc[mf][2]), [c3] "+v"(acc[mf][3])
+#define KMOE_FRAG_W2 [w0] "v"(w[0]), [w1] "v"(w[1])
+#define KMOE_FRAG_W4 KMOE_FRAG_W2, [w2] "v"(w[2]), [w3] "v"(w[3])
+#define KMOE_FRAG_STEP(MFMA, ACC, W)                                                                         \
+  if constexpr (kFirst && kLast)                                                                             \
+    asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_OWN KMOE_FRAG_WAIT MFMA "3:\n\t"                                   \
+                 : ACC, [cur] "=&v"(af_cur) : W, KMOE_FRAG_IMMS : "scc", "memory");                          \
+  else if constexpr (kFirst)                                                                                 \
+    asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_OWN KMOE_FRAG_NEXT MFMA "3:\n\t"                                   \
+                 : ACC, [cur] "=&v"(af_cur), [nxt] "=&v"(af_next) : W, KMOE_FRAG_IMMS : "scc", "memory");    \
+  else if constexpr (kLast)                                                                                  \
+    asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_WAIT MFMA "3:\n\t"                                                 \
+                 : ACC : W, [cur] "v"(af_cur), KMOE_FRAG_IMMS : "scc", "memory");                            \
+  else                                                                                                       \
+    asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_NEXT MFMA "3:\n\t"                                                 \
+                 : ACC, [nxt] "=&v"(af_next) : W, [cur] "v"(af_cur), KMOE_FRAG_IMMS : "scc", "memory")
+#define KMOE_FRAG_STEP_OF(OP)                                                \
+  if constexpr (kNF == 4) {                                                  \
+    KMOE_FRAG_STEP(KMOE_FRAG_MFMA4(OP), KMOE_FRAG_ACC4, KMOE_FRAG_W4);       \
+  } else {                                                                   \
+    KMOE_FRAG_STEP(KMOE_FRAG_MFMA2(OP), KMOE_FRAG_ACC2, KMOE_FRAG_W2);       \
+  }
+    if constexpr (I8) {
+      KMOE_FRAG_STEP_OF("v_mfma_i32_16x16x64_i8")
+    } else if constexpr (F16) {
+      KMOE_FRAG_STEP_OF("v_mfma_f32_16x16x32_f16")
     } else {
-#define KMOE_FRAG_ACC [c0] "+v"(acc[mf][0]), [c1] "+v"(acc[mf][1])
-#define KMOE_FRAG_W [w0] "v"(w[0]), [w1] "v"(w[1])
-      if constexpr (kFirst && kLast)
-        asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_OWN KMOE_FRAG_WAIT KMOE_FRAG_MFMA2 "3:\n\t"
-                     : KMOE_FRAG_ACC, [cur] "=&v"(af_cur) : KMOE_FRAG_W, KMOE_FRAG_IMMS : "scc", "memory");
-      else if constexpr (kFirst)
-        asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_OWN KMOE_FRAG_NEXT KMOE_FRAG_MFMA2 "3:\n\t"
-                     : KMOE_FRAG_ACC, [cur] "=&v"(af_cur), [nxt] "=&v"(af_next) : KMOE_FRAG_W, KMOE_FRAG_IMMS
-                     : "scc", "memory");
-      else if constexpr (kLast)
-        asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_WAIT KMOE_FRAG_MFMA2 "3:\n\t"
-                     : KMOE_FRAG_ACC : KMOE_FRAG_W, [cur] "v"(af_cur), KMOE_FRAG_IMMS : "scc", "memory");
-      else
-        asm volatile(KMOE_FRAG_HEAD KMOE_FRAG_NEXT KMOE_FRAG_MFMA2 "3:\n\t"
-                     : KMOE_FRAG_ACC, [nxt] "=&v"(af_next) : KMOE_FRAG_W, [cur] "v"(af_cur), KMOE_FRAG_IMMS
-                     : "scc", "memory");
-#undef KMOE_FRAG_ACC
-#undef KMOE_FRAG_W
+      KMOE_FRAG_STEP_OF("v_mfma_f32_16x16x32_bf16")
     }
 #undef KMOE_FRAG_HEAD
 #undef KMOE_FRAG_OWN
@@ -606,11 +594,17 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
 #undef KMOE_FRAG_MFMA2
 #undef KMOE_FRAG_MFMA4
 #undef KMOE_FRAG_IMMS
+#undef KMOE_FRAG_ACC2
+#undef KMOE_FRAG_ACC4
+#undef KMOE_FRAG_W2
+#undef KMOE_FRAG_W4
+#undef KMOE_FRAG_STEP
+#undef KMOE_FRAG_STEP_OF
   };
   // The same for tiles whose waves own TWO channel fragments (eight waves along the channels): a statement handles
   // a pair of row fragments - four MFMAs again, so that the reads of the next pair have as many clocks to arrive -
   // and the skip works on pairs (a pair with one live fragment is computed whole).
-  auto frag_pair_i8 = [&](const v4i(&w)[kNF], v4i& c0, v4i& c1, v4i& n0, v4i& n1, uint32_t addr, auto p_tag, auto off_own,
+  auto frag_pair = [&](const v4i(&w)[kNF], v4i& c0, v4i& c1, v4i& n0, v4i& n1, uint32_t addr, auto p_tag, auto off_own,
                           int mf) {
     constexpr int pr = decltype(p_tag)::value;
     constexpr bool kFirst = pr == 0, kLast = 2 * pr + 2 == kMF;
@@ -620,30 +614,36 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
 #define KMOE_PAIR_NEXT \
   "ds_read_b128 %[b0], %[addr] offset:%[o2]\n\tds_read_b128 %[b1], %[addr] offset:%[o3]\n\ts_waitcnt lgkmcnt(2)\n\t"
 #define KMOE_PAIR_WAIT "s_waitcnt lgkmcnt(0)\n\t"
-#define KMOE_PAIR_MFMA                                          \
-  "v_mfma_i32_16x16x64_i8 %[c00], %[w0], %[a0], %[c00]\n\t"     \
-  "v_mfma_i32_16x16x64_i8 %[c01], %[w1], %[a0], %[c01]\n\t"     \
-  "v_mfma_i32_16x16x64_i8 %[c10], %[w0], %[a1], %[c10]\n\t"     \
-  "v_mfma_i32_16x16x64_i8 %[c11], %[w1], %[a1], %[c11]\n\t"
+#define KMOE_PAIR_MFMA(OP)                                                               \
+  OP " %[c00], %[w0], %[a0], %[c00]\n\t" OP " %[c01], %[w1], %[a0], %[c01]\n\t"          \
+  OP " %[c10], %[w0], %[a1], %[c10]\n\t" OP " %[c11], %[w1], %[a1], %[c11]\n\t"
 #define KMOE_PAIR_ACC \
   [c00] "+v"(acc[mf][0]), [c01] "+v"(acc[mf][1]), [c10] "+v"(acc[mf + 1][0]), [c11] "+v"(acc[mf + 1][1])
 #define KMOE_PAIR_INS                                                                                              \
   [w0] "v"(w[0]), [w1] "v"(w[1]), [addr] "v"(addr), [live] "s"(live_frags), [n1] "n"(2 * pr + 1), [o0] "n"(kOwn),    \
       [o1] "n"(kOwn + kStep), [o2] "n"(kOwn + 2 * kStep), [o3] "n"(kOwn + 3 * kStep)
-    if constexpr (kFirst && kLast)
-      asm volatile(KMOE_PAIR_HEAD KMOE_PAIR_OWN KMOE_PAIR_WAIT KMOE_PAIR_MFMA "3:\n\t"
-                   : KMOE_PAIR_ACC, [a0] "=&v"(c0), [a1] "=&v"(c1) : KMOE_PAIR_INS : "scc", "memory");
-    else if constexpr (kFirst)
-      asm volatile(KMOE_PAIR_HEAD KMOE_PAIR_OWN KMOE_PAIR_NEXT KMOE_PAIR_MFMA "3:\n\t"
-                   : KMOE_PAIR_ACC, [a0] "=&v"(c0), [a1] "=&v"(c1), [b0] "=&v"(n0), [b1] "=&v"(n1) : KMOE_PAIR_INS
-                   : "scc", "memory");
-    else if constexpr (kLast)
-      asm volatile(KMOE_PAIR_HEAD KMOE_PAIR_WAIT KMOE_PAIR_MFMA "3:\n\t"
-                   : KMOE_PAIR_ACC : [a0] "v"(c0), [a1] "v"(c1), KMOE_PAIR_INS : "scc", "memory");
-    else
-      asm volatile(KMOE_PAIR_HEAD KMOE_PAIR_NEXT KMOE_PAIR_MFMA "3:\n\t"
-                   : KMOE_PAIR_ACC, [b0] "=&v"(n0), [b1] "=&v"(n1) : [a0] "v"(c0), [a1] "v"(c1), KMOE_PAIR_INS
-                   : "scc", "memory");
+#define KMOE_PAIR_STEP_OF(OP)                                                                                      \
+  if constexpr (kFirst && kLast)                                                                                   \
+    asm volatile(KMOE_PAIR_HEAD KMOE_PAIR_OWN KMOE_PAIR_WAIT KMOE_PAIR_MFMA(OP) "3:\n\t"                           \
+                 : KMOE_PAIR_ACC, [a0] "=&v"(c0), [a1] "=&v"(c1) : KMOE_PAIR_INS : "scc", "memory");               \
+  else if constexpr (kFirst)                                                                                       \
+    asm volatile(KMOE_PAIR_HEAD KMOE_PAIR_OWN KMOE_PAIR_NEXT KMOE_PAIR_MFMA(OP) "3:\n\t"                           \
+                 : KMOE_PAIR_ACC, [a0] "=&v"(c0), [a1] "=&v"(c1), [b0] "=&v"(n0), [b1] "=&v"(n1) : KMOE_PAIR_INS   \
+                 : "scc", "memory");                                                                               \
+  else if constexpr (kLast)                                                                                        \
+    asm volatile(KMOE_PAIR_HEAD KMOE_PAIR_WAIT KMOE_PAIR_MFMA(OP) "3:\n\t"                                         \
+                 : KMOE_PAIR_ACC : [a0] "v"(c0), [a1] "v"(c1), KMOE_PAIR_INS : "scc", "memory");                   \
+  else                                                                                                             \
+    asm volatile(KMOE_PAIR_HEAD KMOE_PAIR_NEXT KMOE_PAIR_MFMA(OP) "3:\n\t"                                         \
+                 : KMOE_PAIR_ACC, [b0] "=&v"(n0), [b1] "=&v"(n1) : [a0] "v"(c0), [a1] "v"(c1), KMOE_PAIR_INS       \
+                 : "scc", "memory");
+    if constexpr (I8) {
+      KMOE_PAIR_STEP_OF("v_mfma_i32_16x16x64_i8")
+    } else if constexpr (F16) {
+      KMOE_PAIR_STEP_OF("v_mfma_f32_16x16x32_f16")
+    } else {
+      KMOE_PAIR_STEP_OF("v_mfma_f32_16x16x32_bf16")
+    }
 #undef KMOE_PAIR_HEAD
 #undef KMOE_PAIR_OWN
 #undef KMOE_PAIR_NEXT
@@ -651,11 +651,15 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
 #undef KMOE_PAIR_MFMA
 #undef KMOE_PAIR_ACC
 #undef KMOE_PAIR_INS
+#undef KMOE_PAIR_STEP_OF
   };
   // keep: std::false_type (every fragment as read), or an int mask (0: the fragments count as zeros)
   auto compute = [&](const v4i(&wcur)[kNF], auto buf_tag, auto j_tag, auto keep) {
     constexpr int buf = decltype(buf_tag)::value, j = decltype(j_tag)::value;
-    if constexpr (ADMA && I8 && !M32 && kNF == 2 && kMF % 2 == 0 && kWN == 8) {
+    // (a masked step of 16-bit operands must zero the activations between the read and the MFMA: it multiplies every
+    // fragment, on the compiler's own path)
+    constexpr bool kSkip = kSkips && (I8 || !std::is_same_v<decltype(keep), int>);
+    if constexpr (kSkip && kNF == 2 && kMF % 2 == 0 && kWN == 8) {
       constexpr bool kFarStages = kStagesA * kStageBytes > 65536;
       constexpr int kImm = kFarStages ? 0 : buf * kStageBytes;
       const uint32_t addr = fa[j] + (kFarStages ? buf * kStageBytes : 0);
@@ -669,14 +673,14 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       auto run = [&](auto self, auto p_tag) {
         constexpr int pr = decltype(p_tag)::value;
         if constexpr (2 * pr < kMF) {
-          frag_pair_i8(wm, af[(2 * pr) & 3], af[(2 * pr + 1) & 3], af[(2 * pr + 2) & 3], af[(2 * pr + 3) & 3], addr, p_tag,
+          frag_pair(wm, af[(2 * pr) & 3], af[(2 * pr + 1) & 3], af[(2 * pr + 2) & 3], af[(2 * pr + 3) & 3], addr, p_tag,
                        std::integral_constant<int, kImm + 2 * pr * 16 * kChunk>{}, 2 * pr);
           self(self, std::integral_constant<int, pr + 1>{});
         }
       };
       run(run, std::integral_constant<int, 0>{});
       asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(af[0]), "+v"(af[1]), "+v"(af[2]), "+v"(af[3]));
-    } else if constexpr (ADMA && I8 && !M32) {
+    } else if constexpr (kSkip) {
       constexpr bool kFarStages = kStagesA * kStageBytes > 65536;
       constexpr int kImm = kFarStages ? 0 : buf * kStageBytes;
       const uint32_t addr = fa[j] + (kFarStages ? buf * kStageBytes : 0);
@@ -691,8 +695,8 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       auto run = [&](auto self, auto n_tag) {
         constexpr int n = decltype(n_tag)::value;
         if constexpr (n < kMF) {
-          frag_i8(wm, af[n & 1], af[(n + 1) & 1], addr, n_tag, std::integral_constant<int, kImm + n * 16 * kChunk>{},
-                  std::integral_constant<int, kImm + (n + 1 < kMF ? n + 1 : n) * 16 * kChunk>{}, n);
+          frag_step(wm, af[n & 1], af[(n + 1) & 1], addr, n_tag, std::integral_constant<int, kImm + n * 16 * kChunk>{},
+                    std::integral_constant<int, kImm + (n + 1 < kMF ? n + 1 : n) * 16 * kChunk>{}, n);
           self(self, std::integral_constant<int, n + 1>{});
         }
       };
@@ -1011,7 +1015,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       seen_prev = seen_next = 0;  // nothing polled for this tile yet: its first chunk starts without waiting
       patience = kSyncPatience;
     }
-    if constexpr ((ADMA && I8 && !M32) || (F8 && ADMA)) {
+    if constexpr (kSkips || (F8 && ADMA)) {
       const int rows_here = min(cur.end, cur.row0 + kTM) - cur.row0 - wave_m * 16 * kMF;
       live_frags = __builtin_amdgcn_readfirstlane(max(0, min(kMF, (rows_here + 15) >> 4)));
     }
@@ -1154,9 +1158,9 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       }
     }
 
-    // (the int8 MFMAs are issued from assembly statements: the compiler does not know that the accumulators come
+    // (the MFMAs are issued from assembly statements: the compiler does not know that the accumulators come
     // out of the matrix pipe and inserts no wait states before the first VALU instruction that reads them)
-    if constexpr (ADMA && I8 && !M32) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+    if constexpr (kSkips) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
     // ---- switch: the finished tile's scales leave LDS first (LDS reads the compiler sees wait
     // for every asynchronous copy in flight, so none may follow start_tile), then the next
     // tile's first loads are requested, then this tile is finished ----
@@ -1672,16 +1676,35 @@ int tiled_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s) {
   if (a->act == KMOE_ACT_SWIGLUOAI)
     return shorter ? launch_tiled<K, false, 4, 4, 2, 1, false, 4, true>(p, a->rows, s, n_cu, what)
                    : launch_tiled<K, false, 4, 4, 2, 1, false, 8, true>(p, a->rows, s, n_cu, what);
-  if (a->act_dtype == KMOE_DT_F16) {  // half operands and results (no bias, no interleaved activation: checked by the caller)
-    if (shorter)
+  // One tile that holds nearly every expert (average + 3 sqrt(average) rows) where there is one, of 96, 128 or 192 rows;
+  // 128 rows beyond: row fragments past an expert's end are neither read nor multiplied, so a taller tile costs its
+  // registers only, a second tile of an expert the expert's weights once more. Layer, Qwen3 dims, tokens: us on 64- / 96-
+  // / 128- / 192-row (wide) / 256-row (wide) tiles; 512: 227.6 / 228 / 230 / 240 / 247, 1024: 269 / 245.7 / 247.5 / 258 /
+  // 265, 1536: 288 / 290 / 265.7 / 277 / 285, 2048: 340 / 308 / 316 / 296 / 304, 3072: 423 / 379 / 352 / 386 / 347, 4096:
+  // 514 / 451 / 427 / 443 / 458, 8192: 891 / 772 / 733 / 727 / 745. (128-row tiles that multiplied every fragment: 1024
+  // 251, 2048 319, 4096 440, 8192 747.)
+  const float avg = static_cast<float>(ceil_div(expected_rows(a->rows, a->rows_hint), a->E));
+  const float reach = avg + 3.0f * sqrtf(avg);
+  const bool half = a->act_dtype == KMOE_DT_F16;  // half operands and results (no bias, no interleaved activation: checked by the caller)
+  if (shorter) {
+    if (half)
       return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what)
                     : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what);
-    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 8, false, false, true>(p, a->rows, s, n_cu, what)
-                  : launch_tiled<K, false, 4, 4, 2, 1, false, 8, false, false, true>(p, a->rows, s, n_cu, what);
-  }
-  if (shorter)
     return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4>(p, a->rows, s, n_cu, what)
                   : launch_tiled<K, false, 4, 4, 2, 1, false, 4>(p, a->rows, s, n_cu, what);
+  }
+  if (a->variant == 13 || (a->variant == 0 && reach <= 96.0f)) {
+    if (half)
+      return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 6, false, false, true>(p, a->rows, s, n_cu, what)
+                    : launch_tiled<K, false, 4, 4, 2, 1, false, 6, false, false, true>(p, a->rows, s, n_cu, what);
+    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 6>(p, a->rows, s, n_cu, what)
+                  : launch_tiled<K, false, 4, 4, 2, 1, false, 6>(p, a->rows, s, n_cu, what);
+  }
+  if (!a->bias && (a->variant == 18 || (a->variant == 0 && reach > 128.0f && reach <= 192.0f)))
+    return launch_wide<K, 12>(p, a->rows, s, n_cu, what, swiglu, half);
+  if (half)
+    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 8, false, false, true>(p, a->rows, s, n_cu, what)
+                  : launch_tiled<K, false, 4, 4, 2, 1, false, 8, false, false, true>(p, a->rows, s, n_cu, what);
   return swiglu ? launch_tiled<K, true, 4, 4, 2, 1>(p, a->rows, s, n_cu, what)
                 : launch_tiled<K, false, 4, 4, 2, 1>(p, a->rows, s, n_cu, what);
 }
