@@ -1,4 +1,4 @@
-"""The tile kernel on 16-bit operands: every tile height at the edges of its row fragments (which are skipped past an
+"""The tile kernels on 16-bit and packed 4-bit weights: every tile height at the edges of its row fragments (which are skipped past an
 expert's rows) and of the tile, against a float32 product of the same values."""
 import pytest
 import torch
@@ -41,3 +41,34 @@ def test_row_fragments(variant, n, k, act, dtype):
     assert not got.isnan().any()
     per_row = (got - ref).norm(dim=1) / ref.norm(dim=1).clamp(min=1e-6)
     assert float((got - ref).norm() / ref.norm()) <= 4e-3 and float(per_row.max()) <= 2e-2
+
+
+@pytest.mark.parametrize("variant", [16, 32, 64, 96, 128])
+@pytest.mark.parametrize("blocks", [1, 2, 3, 5])  # 128-value blocks: fewer than a turn of the rings, a turn, turns and a rest
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_packed_tiles_give_the_streaming_kernels_bits(variant, blocks, act, dtype):
+    """4-bit weights: every tile height against the streaming kernel, which adds the same products in the same order."""
+    from vllm_kunlun_amd import _lib as L
+    gen = torch.Generator().manual_seed(blocks)
+    counts = ROWS + [31, 32, 63, 64, 65]
+    E, rows, n, k, group = len(counts), sum(counts), 160, 128 * blocks, 32
+    src = torch.randperm(rows, generator=gen).int().cuda()
+    a = torch.randn(rows, k, generator=gen).to(dtype).cuda()
+    packed = torch.randint(0, 256, (E, n, k // 2), generator=gen, dtype=torch.uint8).cuda()
+    scale = (torch.rand(E, n, k // group, generator=gen) * 0.02 + 0.002).to(dtype).cuda()
+    tiled = torch.empty_like(packed)
+    L.check(L.lib.kmoe_tile_weights_i8(packed.data_ptr(), tiled.data_ptr(), E, n, k // 2, L.stream()))
+    lod = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    n_out = n // 2 if act else n
+    out = []
+    for v in (1, variant):
+        y = torch.full((rows, n_out), float("nan"), dtype=dtype, device="cuda")
+        g = L.GemmW4Args()
+        g.a, g.lda, g.row_src, g.src_div = a.data_ptr(), k, src.data_ptr(), 1
+        g.w, g.w_scale, g.group_size, g.lod = tiled.data_ptr(), scale.data_ptr(), group, lod.data_ptr()
+        g.E, g.n, g.k, g.rows, g.w_layout = E, n, k, rows, L.KMOE_W_TILED
+        g.y, g.ldy, g.act, g.variant, g.act_dtype = y.data_ptr(), n_out, act, v, L.act_dtype(a, "test")
+        L.check(L.lib.kmoe_grouped_gemm_w4a16(g, L.stream()))
+        out.append(y)
+    assert not out[0].isnan().any() and torch.equal(out[0], out[1])

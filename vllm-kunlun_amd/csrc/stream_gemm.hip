@@ -641,8 +641,7 @@ int stream_w4_shape(const StreamParams& p, bool swiglu, bool scan, int passes, b
                 : (swiglu ? launch_stream<FMT, 1, 2, true, 1, 2>(p, s) : launch_stream<FMT, 1, 2, false, 1, 2>(p, s));
   if (passes == 1) return swiglu ? launch_stream<FMT, 1, 2, true, 1>(p, s) : launch_stream<FMT, 1, 2, false, 1>(p, s);
   if (passes == 2)
-    return scan ? launch_stream<FMT, 2, 2, true, 2, 1, true>(p, s)
-                : (swiglu ? launch_stream<FMT, 2, 2, true, 2>(p, s) : launch_stream<FMT, 2, 2, false, 2>(p, s));
+    return swiglu ? launch_stream<FMT, 2, 2, true, 2>(p, s) : launch_stream<FMT, 2, 2, false, 2>(p, s);
   return swiglu ? launch_stream<FMT, 4, 2, true, 2>(p, s) : launch_stream<FMT, 4, 2, false, 2>(p, s);
 }
 

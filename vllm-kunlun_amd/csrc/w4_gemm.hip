@@ -1,5 +1,5 @@
-// Grouped GEMM on 4-bit weights and bf16 activations (W4A16): a weight-streaming kernel for the
-// decode regime and a kernel on 128-row tiles for the prefill regime (further down). In both the
+// Grouped GEMM on 4-bit weights and bf16 activations (W4A16): the launch on tiles of 16 to 128 rows, and the choice
+// between it and the weight-streaming kernel (stream_gemm.hip). In both the
 // packed weights are unpacked in registers and fed to v_mfma_f32_16x16x32_bf16: a quarter of the
 // bytes of the bf16 path; the unpacking (17 VALU instructions per 8 weights, 13 for half) is what bounds the
 // streaming kernel once the bytes are that few, and what the tile kernel shares among its rows.
@@ -55,13 +55,11 @@ struct W4Params {
 constexpr int kWaves = 4;
 
 // ---------------------------------------------------------------------------------------------------
-// Prefill regime: tiles of 64, 96 or 128 rows. The unpacking of a weight word is shared by the row fragments of
-// the tile (23 VALU instructions against 8 MFMAs of 16 cycles on the tallest), so the kernel is bound by the matrix cores
-// like the 16-bit tile kernels while it reads a quarter of their weight bytes. One workgroup: up to 128 sorted
-// rows of one expert x 4 waves x NF fragments of 16 channels. Activations are copied global -> LDS
-// asynchronously, one 128-value block of K (256 bytes per row) ahead, two buffers; every wave reads its A
-// fragments from there. Weights and their scales go global -> registers, one block ahead; they never pass
-// through LDS.
+// Tiles of 16, 32, 64, 96 or 128 rows. The unpacking of a weight word (17 VALU instructions per 8 values) is shared by
+// the row fragments of the tile, one MFMA each; the kernel is bound by issuing both, at a quarter of the 16-bit weights'
+// bytes. One workgroup: one tile of sorted rows of one expert x 4 waves x 4 fragments of 16 channels. Activations are
+// copied global -> LDS asynchronously in 128-value blocks of K (256 bytes per row); every wave reads its A fragments
+// from there. Weights and their scales go global -> registers, one or two blocks ahead; they never pass through LDS.
 
 // Work item `item` = (m-tile, channel block) when every expert's rows are cut into tiles of kTileRows and the
 // items are numbered m-tile by m-tile: expert, first row and channel block (false: no such item). The hardware
@@ -136,36 +134,41 @@ __device__ __forceinline__ void mfma4_if_live(v4f (&c)[4], const v4i (&w)[4], co
 }
 
 template <class F, int... I>
-__device__ inline void static_for_each(F&& f, std::integer_sequence<int, I...>) {
+__device__ __forceinline__ void static_for_each(F&& f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, I>{}), ...);
 }
 template <int N, class F>
-__device__ inline void static_for(F&& f) {
+__device__ __forceinline__ void static_for(F&& f) {
   static_for_each(f, std::make_integer_sequence<int, N>{});
 }
 
-// MF: 16-row fragments of a tile (4, 6, 8: 64-, 96- and 128-row tiles). Two workgroups per CU for every height:
-// with three, the 64-row instance had 170 registers to live in and lost to the 128-row one (121 against 111 us
-// over 4 to 64 rows per expert on the Qwen3 shape); with two it is a quarter ahead where experts fit its tile.
-//
-// RW, RA: blocks of weights (registers) and of activations (LDS) in the rings. A stage waits for its own block, passes a
-// barrier, requests block kb + RA - 1 of the activations and kb + RW - 1 of the weights and multiplies: loads have two
-// to three stages to arrive. With one block in flight (as registers and 64 KB of LDS allow for 128-row tiles) the short
-// tiles, whose stage is half as long, waited for the memory in every stage.
-// No branch sits between a load and its use - the waits count loads - so blocks past the end are requested as well,
-// out of the descriptors' range: they fetch nothing.
-template <int MF, int NF, bool SWIGLU, bool F16, int RW, int RA>
-__global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Params p) {
-  static_assert(NF == 4 && RW >= RA && RA >= 2, "the weights are requested with the activations of the same block or before");
+// MF: 16-row fragments of a tile (1, 2, 4, 6, 8). The short tiles keep one block of weights and activations ahead and
+// run three or four workgroups per CU instead of more blocks and two: the unpacking of one wave then has three others'
+// waits and MFMAs to run beside. Layer, Kimi-K2 dims with groups of 32: 2048 tokens on 64-row tiles 2650 us with four
+// blocks and two workgroups, 2450 with two and three; 700 tokens on 32-row tiles 1786, where 16-row passes of the
+// streaming kernel took 2776 and 64-row tiles with two workgroups 2101; 128 tokens on 16-row tiles 1537 (streaming 1599).
+// The tall tiles' accumulators leave room for two.
+constexpr int w4_workgroups(int MF) { return MF <= 2 ? 4 : (MF == 4 ? 3 : 2); }
+// R: blocks of weights (registers) and of activations (LDS) in the rings. A stage waits for its own block, passes a
+// barrier, requests block kb + R - 1 of both and multiplies. No branch sits between a load and its use - the waits count
+// loads - so blocks past the end are requested as well, out of the descriptors' range: they fetch nothing.
+constexpr int w4_ring(int MF) { return MF == 6 ? 3 : 2; }
+template <int MF, bool SWIGLU, bool F16>
+__global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kernel(const W4Params p) {
+  constexpr int NF = 4, R = w4_ring(MF);
   constexpr int kTileRows = 16 * MF;
   constexpr int NFH = SWIGLU ? NF / 2 : NF;
   constexpr int NA = kTileRows / 4 / kWaves;  // asynchronous copies per wave and block: 4 rows (1 KB) each
   constexpr int kWaveRows = 4 * NA;           // tile rows a wave copies
   constexpr int kBufBytes = kTileRows * 256;
-  // Row r of a block sits at r * 256; its 16-byte vector v at position v ^ (r % 16): the 16 rows of a
-  // fragment read (same vector, rows r, r + 1, ...) fall on 16 different bank groups without padding, which
-  // the asynchronous copies (1 KB of consecutive LDS bytes per instruction) could not write.
-  __shared__ __attribute__((aligned(1024))) int8_t lds_a[RA][kBufBytes];
+  // Row r of a block sits at r * 256; its 16-byte vector v at position v ^ swizzle(r % 16): the rows of a fragment read
+  // fall on different bank groups without padding, which the asynchronous copies (1 KB of consecutive LDS bytes per
+  // instruction) could not write. A read serves lanes 0-3, 12-15 and 20-27 together, then 4-11, 16-19 and 28-31, and
+  // so on: rows 0-3 and 12-15 of one vector with rows 4-11 of the vector four further. The swizzle has to keep those
+  // apart: it sends the first eight rows to 0-7 and the others to 8-15 (r itself makes every pair of them collide:
+  // four clocks more per read).
+  auto swizzle = [](int r) { return r ^ ((r & 4) << 1); };
+  __shared__ __attribute__((aligned(1024))) int8_t lds_a[R][kBufBytes];
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15;
@@ -209,23 +212,23 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
     const int r = row0 + tr;
     const int rr = r < row_end ? r : row0;  // rows past the end read the tile's first row: never stored
     const int src = p.row_src ? p.row_src[rr] / p.src_div : rr;
-    aoff[i] = static_cast<uint32_t>(src) * static_cast<uint32_t>(p.lda * 2) + ((li ^ (tr & 15)) << 4);  // < 4 GiB: host-checked
+    aoff[i] = static_cast<uint32_t>(src) * static_cast<uint32_t>(p.lda * 2) + ((li ^ swizzle(tr & 15)) << 4);  // < 4 GiB: host-checked
   }
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)&lds_a[0][0]));
   // fragment reads of MFMA step t: row li (+ 16 per fragment: same row % 16), vector 4 lg + t
   uint32_t fa[4];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) fa[t] = lds_base + li * 256 + (((4 * lg + t) ^ li) << 4);
+  for (int t = 0; t < 4; ++t) fa[t] = lds_base + li * 256 + (((4 * lg + t) ^ swizzle(li)) << 4);
   v4f acc[MF][NF];
 #pragma unroll
   for (int mf = 0; mf < MF; ++mf)
 #pragma unroll
     for (int f = 0; f < NF; ++f) acc[mf][f] = (v4f){0.f, 0.f, 0.f, 0.f};
-  v4i wbuf[RW][NF];
-  uint16_t sbuf[RW][NF];
+  v4i wbuf[R][NF];
+  uint16_t sbuf[R][NF];
   const uint32_t lane16 = lane * 16u;
   const uint32_t lane_s = li * p.s_ch * 2u;
-  auto load_w = [&](int slot, int kb) {
+  auto load_w = [&](int slot, int kb) __attribute__((always_inline)) {
     const bool live = kb < kblocks;
     const int g32 = 4 * kb + lg;  // this lane's 32 values of the block
     const uint32_t s_at = lane_s + static_cast<uint32_t>((p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / (p.gs / 32)) * p.s_g) * 2u;
@@ -235,29 +238,25 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
       sbuf[slot][f] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(s_rsrc, s_at, live ? soff[f] : kRange, 0));
     }
   };
-  auto dma_a = [&](int buf, int kb) {
+  auto dma_a = [&](int buf, int kb) __attribute__((always_inline)) {
     const uint32_t at = kb < kblocks ? static_cast<uint32_t>(kb) * 256u : kRange;
 #pragma unroll
     for (int i = 0; i < NA; ++i)
       buffer_load16_to_lds(a_rsrc, (lds_ptr_t)&lds_a[buf][(kWaveRows * wave + 4 * i) * 256], aoff[i], at);
   };
-  constexpr int kLoadsW = 2 * NF;
-  // loads of a wave younger than those a stage needs
-  constexpr int kYounger = RW == RA ? (RA - 2) * (NA + kLoadsW) : (RA - 1) * kLoadsW + (RA - 2) * NA;
   // One block: word t of a lane's 16 packed bytes is its operand of MFMA step t; the activation lane (lg, row)
   // supplies values 32 lg + 8 t + [0, 8) of the block, i.e. vector 4 lg + t of the row's 16. The words of step t + 1
   // are unpacked between the row fragments of step t: the matrix and the vector unit both have work from one wave.
-  auto compute = [&](auto slot_tag, auto buf_tag) {
+  auto compute = [&](auto slot_tag) __attribute__((always_inline)) {
     constexpr int slot = decltype(slot_tag)::value;
-    constexpr int buf = decltype(buf_tag)::value;
     const W4Scale<F16> sc[NF] = {W4Scale<F16>(sbuf[slot][0]), W4Scale<F16>(sbuf[slot][1]), W4Scale<F16>(sbuf[slot][2]),
                                  W4Scale<F16>(sbuf[slot][3])};
     // Row fragments are read two ahead, across the steps: fragment i = t MF + mf of the block's 4 MF.
     v4i af[3];
-    auto request = [&](auto i_tag) {
+    auto request = [&](auto i_tag) __attribute__((always_inline)) {
       constexpr int i = decltype(i_tag)::value;
       // (the offset field of an LDS read reaches 64 KB)
-      constexpr int off = buf * kBufBytes + (i % MF) * 16 * 256;
+      constexpr int off = slot * kBufBytes + (i % MF) * 16 * 256;
       af[i % 3] = off < 65536 ? lds_read16_raw<(off < 65536 ? off : 0)>(fa[i / MF])
                               : lds_read16_raw<(off < 65536 ? 0 : off - 65536)>(fa[i / MF] + 65536u);
     };
@@ -267,7 +266,7 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
 #pragma unroll
     for (int f = 0; f < NF; ++f) wv[0][f] = unpack8(static_cast<uint32_t>(wbuf[slot][f][0]), sc[f]);
     __builtin_amdgcn_sched_barrier(0);
-    static_for<4 * MF>([&](auto i_tag) {
+    static_for<4 * MF>([&](auto i_tag) __attribute__((always_inline)) {
       constexpr int i = decltype(i_tag)::value;
       constexpr int t = i / MF, mf = i % MF;
       if constexpr (i + 2 < 4 * MF) {
@@ -287,90 +286,71 @@ __global__ __launch_bounds__(kWaves* kWave, 2) void w4_tile_kernel(const W4Param
       __builtin_amdgcn_sched_barrier(0);  // (all the unpacking of a block at once would not fit the registers)
     });
   };
-  auto stage = [&](int kb, auto u_tag) {
+  auto stage = [&](int kb, auto u_tag) __attribute__((always_inline)) {
     constexpr int u = decltype(u_tag)::value;
-    vmem_wait<kYounger>();
+    vmem_wait<(R - 2) * (NA + 2 * NF)>();  // the loads of a wave younger than those the stage needs
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    dma_a((u + RA - 1) % RA, kb + RA - 1);
-    load_w((u + RW - 1) % RW, kb + RW - 1);
+    dma_a((u + R - 1) % R, kb + R - 1);
+    load_w((u + R - 1) % R, kb + R - 1);
     __builtin_amdgcn_sched_barrier(0);
-    compute(std::integral_constant<int, u % RW>{}, std::integral_constant<int, u % RA>{});
+    compute(u_tag);
   };
 #pragma unroll
-  for (int i = 1 - RW; i < 0; ++i) {
-    if (i + RA - 1 >= 0) dma_a(i + RA - 1, i + RA - 1);
-    load_w(i + RW - 1, i + RW - 1);
+  for (int i = 0; i < R - 1; ++i) {
+    dma_a(i, i);
+    load_w(i, i);
   }
-  constexpr int U = RW % RA == 0 ? RW : RW * RA;  // stages until both rings are back where they were
-  // (no exit inside the body: as one basic block it fits the registers. Stages past the last block multiply what the
-  // descriptors' ends returned, zeros by zeros.)
-  for (int kb0 = 0; kb0 < kblocks; kb0 += U) {
-    stage(kb0, std::integral_constant<int, 0>{});
-    stage(kb0 + 1, std::integral_constant<int, 1 % U>{});
-    if constexpr (U > 2) stage(kb0 + 2, std::integral_constant<int, 2 % U>{});
-    if constexpr (U > 3) stage(kb0 + 3, std::integral_constant<int, 3 % U>{});
-    if constexpr (U > 4) {
-      stage(kb0 + 4, std::integral_constant<int, 4 % U>{});
-      stage(kb0 + 5, std::integral_constant<int, 5 % U>{});
-    }
-  }
+  // (no exit inside the body: as one basic block it fits the registers)
+  int kb = 0;
+  for (; kb + R <= kblocks; kb += R)
+    static_for<R>([&](auto u) __attribute__((always_inline)) { stage(kb + decltype(u)::value, u); });
+  static_for<R - 1>([&](auto u) __attribute__((always_inline)) {
+    if (kb + decltype(u)::value < kblocks) stage(kb + decltype(u)::value, u);
+  });
 
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs' results, which the compiler does not know to wait for
   __builtin_amdgcn_sched_barrier(0);
   // epilogue: as the streaming kernel - round to the activation type, optional SiLU-mul on the rounded values
+  auto pack2 = [](float lo, float hi) { return F16 ? pack2_half(lo, hi) : pack2_bf16(lo, hi); };
+  auto low = [](uint32_t v) { return act_to_f32(static_cast<uint16_t>(v), F16); };
+  auto high = [](uint32_t v) { return act_to_f32(static_cast<uint16_t>(v >> 16), F16); };
 #pragma unroll
   for (int mf = 0; mf < MF; ++mf) {
+    if (mf >= live_frags) continue;  // (wave-uniform)
     const int r = row0 + mf * 16 + li;
-    if (r >= row_end) continue;
 #pragma unroll
     for (int f = 0; f < NFH; ++f) {
-      if (!wok[f]) continue;
       const int c0 = col[f] + lg * 4;
-      uint16_t yv[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) yv[q] = f32_to_act(acc[mf][f][q], F16);
-      if (SWIGLU) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          yv[q] = f32_to_act(silu_hw(act_to_f32(yv[q], F16)) * act_to_f32(f32_to_act(acc[mf][f + NFH][q], F16), F16), F16);
+      const v4f g = acc[mf][f];
+      uint2 out = make_uint2(pack2(g[0], g[1]), pack2(g[2], g[3]));
+      if constexpr (SWIGLU) {
+        const v4f u = acc[mf][f + NFH];
+        const uint32_t u0 = pack2(u[0], u[1]), u1 = pack2(u[2], u[3]);
+        out.x = pack2(silu_hw(low(out.x)) * low(u0), silu_hw(high(out.x)) * high(u0));
+        out.y = pack2(silu_hw(low(out.y)) * low(u1), silu_hw(high(out.y)) * high(u1));
       }
-      const uint2 packed = make_uint2(yv[0] | (static_cast<uint32_t>(yv[1]) << 16),
-                                      yv[2] | (static_cast<uint32_t>(yv[3]) << 16));
-      *reinterpret_cast<uint2*>(p.y + static_cast<size_t>(r) * p.ldy + c0) = packed;
+      if (wok[f] && r < row_end) *reinterpret_cast<uint2*>(p.y + static_cast<size_t>(r) * p.ldy + c0) = out;
     }
   }
 }
 
 template <int MF, bool SWIGLU>
 int launch_w4_tile(const W4Params& p, int rows, bool f16, hipStream_t s) {
-  constexpr int NF = 4;
   constexpr int kTileRows = 16 * MF;
-  constexpr int NFH = SWIGLU ? NF / 2 : NF;
+  constexpr int NFH = SWIGLU ? 2 : 4;
   const int n_half = SWIGLU ? p.n / 2 : p.n;
   // an upper bound of the work items (m-tiles x channel blocks), a multiple of 8
   const int n_blocks = ceil_div(n_half, kWaves * NFH * 16);
   const int items = (rows / kTileRows + min(p.E, rows)) * n_blocks;
   const dim3 grid(ceil_div(items, 8) * 8);
-  // Blocks in flight: what the registers (weights) and 80 KB of LDS (activations) hold. A launch runs whole turns of
-  // its rings, so a 64-row tile takes three blocks where four would leave more stages without a block (k = 768: 6 blocks).
-  auto go = [&](auto ring_tag) {
-    constexpr int R = decltype(ring_tag)::value;
-    if (tracing_kernels())
-      note_kernel("w4_tile_kernel<%d-row tiles, %s, %s, %d blocks in flight>", kTileRows, SWIGLU ? "SiLU-mul" : "plain",
-                  f16 ? "f16" : "bf16", R);
-    if (f16)
-      hipLaunchKernelGGL((w4_tile_kernel<MF, NF, SWIGLU, true, R, R>), grid, dim3(kWaves * kWave), 0, s, p);
-    else
-      hipLaunchKernelGGL((w4_tile_kernel<MF, NF, SWIGLU, false, R, R>), grid, dim3(kWaves * kWave), 0, s, p);
-  };
-  const int kblocks = p.k / 128;
-  if constexpr (MF == 4) {
-    if (ceil_div(kblocks, 4) * 4 <= ceil_div(kblocks, 3) * 3) go(std::integral_constant<int, 4>{});
-    else go(std::integral_constant<int, 3>{});
-  } else {
-    go(std::integral_constant<int, MF == 6 ? 3 : 2>{});
-  }
+  if (tracing_kernels())
+    note_kernel("w4_tile_kernel<%d-row tiles, %s, %s, %d per CU>", kTileRows, SWIGLU ? "SiLU-mul" : "plain",
+                f16 ? "f16" : "bf16", w4_workgroups(MF));
+  if (f16)
+    hipLaunchKernelGGL((w4_tile_kernel<MF, SWIGLU, true>), grid, dim3(kWaves * kWave), 0, s, p);
+  else
+    hipLaunchKernelGGL((w4_tile_kernel<MF, SWIGLU, false>), grid, dim3(kWaves * kWave), 0, s, p);
   return check_launch("kmoe_grouped_gemm_w4a16");
 }
 
@@ -385,19 +365,14 @@ __global__ __launch_bounds__(256) void tile_scales_kernel(const uint16_t* __rest
   dst[i] = src[(frag * 16 + c) * groups + g];
 }
 
-// Rows per pass of the streaming kernel for a launch (1: 16, 2: 32), or 0 where the tile kernel takes over.
-int w4_stream_passes(int rows, int rows_hint, int E, int k) {
-  const int avg = ceil_div(expected_rows(rows, rows_hint), E);
-  // (with K = 2048 the 32-row streaming pass is never the best: 12 rows per expert 75 on 16-row passes, 84 on
-  // 32-row passes, 87 on 64-row tiles; 16 rows 99 / 96 / 87)
-  const int one_max = k > 4096 ? 10 : 13;
-  const int stream_max = k > 4096 ? 20 : 13;
-  return avg <= one_max ? 1 : (avg <= stream_max ? 2 : 0);
-}
-
 }  // namespace
 
-bool w4_gate_up_streams(int rows, int rows_hint, int E, int k) { return w4_stream_passes(rows, rows_hint, E, k) != 0; }
+// Layer, us, 16-row passes of the streaming kernel (which sorts the pairs on the way) against 16-row tiles (whose launch
+// needs the sort's): Qwen3 dims 16 tokens (1 row per expert) 62.9 / 64.6, 64 (4) 79.1 / 78.4, 96 (6) 83.5 / 79.7, 128 88.0 /
+// 79.7; Kimi-K2 dims 8 tokens 287 / 291, 32 (1) 832 / 813, 64 (2) 1236 / 1188, 128 (3) 1599 / 1537 - with a long K the sort's launch is nothing.
+bool w4_gate_up_streams(int rows, int rows_hint, int E, int k) {
+  return ceil_div(expected_rows(rows, rows_hint), E) <= (k > 4096 ? 1 : 4);
+}
 
 }  // namespace kmoe
 
@@ -454,32 +429,39 @@ int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t s
   // the tile kernel reaches a source row (gathered or not: below `rows`) through a 32-bit byte offset
   const bool tile_ok = static_cast<uint64_t>(a->rows) * static_cast<uint64_t>(a->lda) * 2u + static_cast<uint64_t>(a->k) * 2u < (1ull << 32);
   if (mf == 0) {
-    // rows an expert gets under uniform routing, with headroom for the spread: an expert with
-    // more rows than one pass holds streams (and unpacks) its weights again. From a dozen and a half rows per
-    // expert the tile kernel is ahead on its shortest tile, which is mostly padding there (later when K is long:
-    // the streaming kernel's waves then live longer per weight byte); the tile grows when too many experts would
-    // need a second one (gate_up, Qwen3 shape / Kimi-K2 shape with groups of 32, us: 12 rows per expert streaming
-    // 75 against 87 on 64-row tiles, 16 rows 96 / 1976 against 87 / 2196, 21 rows - / 2196 against - / 2225, 24 rows
-    // 109 against 82, 32 rows 3176 against 2250; 64-, 96-, 128-row tiles at 44 rows 84 / 99 / 109, at 48 rows
-    // 111 / 109 / 120 and 2440 / 2609 / 2918, at 56 rows 111 / 107 / 119 and 2634 / 2614 / 2993, at 64 rows
-    // 133 / 109 / 121, at 76 rows 156 / 109 / 122 and 4073 / 2708 / 3113, at 80 rows - / 136 / 127).
+    // The streaming kernel where it sorts the pairs itself or has a column of workgroups per pair, or for a gate_up of
+    // few rows; its plain down launch is 4 to 7 % behind 16-row tiles from one row per expert on (Qwen3 dims, 16 / 32 /
+    // 64 tokens: 19.7 / 24.2 / 26.7 us against 18.8 / 23.7 / 24.9). Tiles by the rows an expert gets under uniform routing, with
+    // headroom for the spread - an expert with more rows unpacks its weights again, one with fewer leaves its tile's
+    // accumulators unused and workgroups out of the CU. Layer, us, 16- / 32- / 64-row tiles, Qwen3 dims: 112 tokens (7 rows)
+    // 80.0 / 81.7 / 88.2, 144 (9) 87.2 / 82.5 / 89.8, 330 (21) 119 / 95.8 / 100, 360 (23) 123 / 105 / 101; Kimi-K2 dims:
+    // 350 (8) 1688 / 1703 / 1840, 1000 (21) 2681 / 2002 / 2064, 1200 (25) 2987 / 2155 / 2137. 64- / 96- / 128-row, Qwen3
+    // dims: 768 (48) 140.7 / 141.0 / 149.1, 832 (52) 146.2 / 144.5 / 152.0, 1152 (72) 183 / 168 / 170, 1300 (82) 192 / 189 /
+    // 176, 1800 (113) 225 / 251 / 224, 2048 (128) 252 / 263 / 262, 2300 (144) 275 / 270 / 290, 2560 (160) 291 / 285 / 305,
+    // 3072 (192) 333 / 335 / 324, 8192 (512) 776 / 756 / 716.
     const int avg = ceil_div(expected_rows(a->rows, a->rows_hint), a->E);
-    const int passes = w4_stream_passes(a->rows, a->rows_hint, a->E, a->k);
-    mf = passes ? passes : (!tile_ok ? 4 : (avg <= 48 ? 64 : (avg <= 76 ? 96 : 128)));
+    if (scan || slots || (swiglu && w4_gate_up_streams(a->rows, a->rows_hint, a->E, a->k))) mf = 1;
+    else if (!tile_ok) mf = avg <= 13 ? 1 : (avg <= 20 ? 2 : 4);
+    else if (avg <= 22) mf = avg <= 8 ? 16 : 32;
+    else if (avg <= 112) mf = avg <= 50 ? 64 : (avg <= 76 ? 96 : 128);
+    else mf = avg <= 136 ? 64 : (avg <= 176 ? 96 : 128);
   }
   if (mf == 8) mf = 128;
-  KMOE_REQUIRE((!scan && !slots) || mf == 1 || mf == 2, KMOE_ERR_UNSUPPORTED, "grouped_gemm_w4a16: only the weight-streaming kernel sorts the pairs itself");
-  if (mf == 64 || mf == 96 || mf == 128)
+  const bool tile = mf == 16 || mf == 32 || mf == 64 || mf == 96 || mf == 128;
+  KMOE_REQUIRE((!scan && !slots) || mf == 1, KMOE_ERR_UNSUPPORTED, "grouped_gemm_w4a16: only the weight-streaming kernel sorts the pairs itself");
+  if (tile)
     KMOE_REQUIRE(tile_ok, KMOE_ERR_SHAPE, "grouped_gemm_w4a16: the tile kernel addresses the activations with 32 bits (rows=%d lda=%lld)",
                  a->rows, static_cast<long long>(a->lda));
   switch (mf) {
     case 1:
     case 2:
     case 4: return stream_gemm_w4(a, s, mf, scan, slots);
+    case 16: return swiglu ? launch_w4_tile<1, true>(p, a->rows, f16, s) : launch_w4_tile<1, false>(p, a->rows, f16, s);
+    case 32: return swiglu ? launch_w4_tile<2, true>(p, a->rows, f16, s) : launch_w4_tile<2, false>(p, a->rows, f16, s);
     case 64: return swiglu ? launch_w4_tile<4, true>(p, a->rows, f16, s) : launch_w4_tile<4, false>(p, a->rows, f16, s);
     case 96: return swiglu ? launch_w4_tile<6, true>(p, a->rows, f16, s) : launch_w4_tile<6, false>(p, a->rows, f16, s);
     case 128: return swiglu ? launch_w4_tile<8, true>(p, a->rows, f16, s) : launch_w4_tile<8, false>(p, a->rows, f16, s);
     default:
-      return fail(KMOE_ERR_UNSUPPORTED, "grouped_gemm_w4a16: variant=%d must be 0, 1, 2, 4, 8, 64, 96 or 128 (or a tuning variant)", a->variant);
+      return fail(KMOE_ERR_UNSUPPORTED, "grouped_gemm_w4a16: variant=%d must be 0, 1, 2, 4, 8, 16, 32, 64, 96 or 128", a->variant);
   }
 }
