@@ -2,8 +2,16 @@
 one): router logits in the activations' own 16-bit type must give the bits of the same logits widened to float32, for
 every format and slot count of the routing kernel; a layer call whose argument block is kept from an earlier call must
 follow what changed in between."""
+import os
+import sys
+
+import numpy as np
 import pytest
 import torch
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), ".."))
+from conftest import bits  # noqa: E402
+from oracle import c_oracle as co  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -79,3 +87,34 @@ def test_stable_sort_by_expert(P, E, first):
     moe_index, sorted_src, expert_m, lod = (t.cpu().long() for t in out)
     assert torch.equal(moe_index[:P], index) and torch.equal(sorted_src[:kept], order[:kept])
     assert torch.equal(expert_m, counts) and torch.equal(lod, torch.cat([torch.zeros(1), counts.cumsum(0)]).long())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fp8_group_quantiser_on_every_mantissa(dtype):
+    """Groups whose maximum has every mantissa, over the exponents where the quotients come from the reciprocal and those
+    where they are divided; zeros of both signs, subnormals, infinities and NaNs among the values."""
+    from vllm_kunlun_amd import _lib as L
+    gen = torch.Generator().manual_seed(3)
+    half = dtype == torch.float16
+    mantissas = 1024 if half else 128
+    exponents = [0, 1, 14, 15, 16, 30] if half else [0, 1, 60, 70, 76, 77, 127, 195, 196, 250, 254]
+    top = torch.tensor([(e << (10 if half else 7)) | m for e in exponents for m in range(mantissas)], dtype=torch.int32)
+    groups = len(top)
+    x = torch.randint(0, 1 << 15, (groups, 128), generator=gen, dtype=torch.int32) % (top[:, None] + 1)
+    near = torch.randint(0, (4 << 10) if half else (10 << 7), (groups, 128), generator=gen, dtype=torch.int32)
+    x[:, :96] = (top[:, None] - near[:, :96]).clamp(min=0)  # most values within a few exponents of the maximum
+    x[:, 5] = top
+    x[:, 6] = 0
+    x[::7, 9] = 0x7c00 if half else 0x7f80  # infinity: an infinite scale
+    x[::5, 11] = 0x7e00 if half else 0x7fc0  # NaN: not part of the maximum
+    x[3] = 0
+    x |= torch.randint(0, 2, x.shape, generator=gen, dtype=torch.int32) << 15
+    x = torch.from_numpy(x.numpy().astype(np.uint16).view(np.int16)).view(dtype).reshape(groups // 2, 256)
+    R = x.shape[0]
+    q_ref, s_ref = co.quant_fp8_group128(bits(x), f16=half)
+    dx = x.cuda()
+    q = torch.zeros(R, 256, dtype=torch.uint8, device="cuda")
+    s = torch.zeros(R, 2, dtype=torch.float32, device="cuda")
+    L.check(L.lib.kmoe_quant_fp8_group128_dt(L.ptr(dx), 256, R, 256, L.ptr(q), 256, L.ptr(s), L.act_dtype(dx, "test"), L.stream()))
+    assert np.array_equal(s.cpu().numpy().view(np.uint32), s_ref.view(np.uint32))
+    assert np.array_equal(q.cpu().numpy(), q_ref)
