@@ -30,14 +30,28 @@ def _linear(n, k, seed):
 
 # rows on both sides of the slices' sizes and of their choice, one channel fragment per wave and two, few K steps (an
 # empty share for some of a workgroup's waves) and a remainder of the steps in flight
-@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65, 255, 256])
-@pytest.mark.parametrize("n,k", [(16, 64), (64, 448), (4112, 192), (144, 1728)])
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65, 128, 129, 255, 257])
+@pytest.mark.parametrize("n,k", [(16, 64), (64, 448), (4112, 192), (144, 1728), (48, 4160)])
 def test_dense_slices(rows, n, k):
     kern, layer, codes, w_max = _linear(n, k, n + k)
     x = (torch.randn(rows, k, generator=torch.Generator().manual_seed(rows)) * 1.5).bfloat16()
     out = kern.apply_weights(layer, x.cuda())
     xq, x_max = co.quant_i8_rows(bits(x))
     ref, _ = co.grouped_gemm_i8(xq, x_max, codes.numpy()[None], w_max.numpy()[None], np.array([0, rows], np.int32))
+    assert np.array_equal(bits(out), ref)
+
+
+# tiles of 32 x 128, 64 x 128 and beyond: rows and channels at their edges, an odd number of 64-byte steps, both types
+@pytest.mark.parametrize("rows,n", [(289, 4096), (384, 4112), (513, 4000), (449, 7168), (1100, 4096)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dense_tiles(rows, n, dtype):
+    k = 192
+    kern, layer, codes, w_max = _linear(n, k, n)
+    x = (torch.randn(rows, k, generator=torch.Generator().manual_seed(rows)) * 1.5).to(dtype)
+    out = kern.apply_weights(layer, x.cuda())
+    f16 = dtype == torch.float16
+    xq, x_max = co.quant_i8_rows(bits(x), f16=f16)
+    ref, _ = co.grouped_gemm_i8(xq, x_max, codes.numpy()[None], w_max.numpy()[None], np.array([0, rows], np.int32), f16=f16)
     assert np.array_equal(bits(out), ref)
 
 

@@ -1472,7 +1472,8 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   if (int rc = tiled_common(p, a->rows, &n_cu, what)) return rc;
   constexpr TKind K = TKind::I8;
   const int live = expected_rows(a->rows, a->rows_hint);  // (chooses the tile shape; grids and bounds keep a->rows)
-  const int avg_rows = ceil_div(live + (a->w_tail ? a->tail_rows : 0), a->E + (a->w_tail ? 1 : 0));
+  const int n_exp = a->E + (a->w_tail ? 1 : 0);
+  const int avg_rows = ceil_div(live + (a->w_tail ? a->tail_rows : 0), n_exp);
   const bool shorter = short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu);
   // 128-row 4-wave tiles whose sibling m-tiles are paced against each other (see g_board): variant 12, and the
   // second launch of the device-decided pair (variant 17). They were the default where experts have several m-tiles
@@ -1513,6 +1514,21 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   // the paced tiles as variant 12; 19 / 18 / 22 (and 15 / 14 / 8, 16): 128- / 192- / 256-row wide tiles forced.
   // (an expert of up to 3 MiB stays in an XCD's 4 MB L2 while its m-tiles run: their channel blocks go side by side)
   p.m_major = static_cast<long long>(a->n) * a->k <= (3ll << 20) ? 1 : 0;
+  // A plain GEMM of so few tiles that most CUs would stay without one (a dense linear of some hundred rows): 128 channels
+  // per tile instead of 256, of 32 rows while those fill the chip about once, of 64 while 64 x 256 tiles would not.
+  // With the quantiser, us, 64 x 256 / 64 x 128 / 32 x 128 tiles: [4096 x 7168] 257 rows 37.3 / 28.0 / 27.2, 384 38.1 / 29.8 /
+  // 31.4, 512 38.5 / 30.1 / 33.8, 768 40.0 / 39.5 / 48.7, 1024 42.6 / 44.0 / 60.3; [7168 x 2048] 128 rows - / 14.8 / 13.2, 257
+  // 18.4 / 17.0 / 16.0, 512 20.2 / 18.8 / 22.8, 1024 27.3 / 29.3 / 35.0.
+  if (a->variant == 0 && !swiglu) {
+    const bool f16 = a->act_dtype == KMOE_DT_F16;
+    auto items = [&](int rows, int channels) { return (ceil_div(live + p.tail_rows, rows) + n_exp - 1) * ceil_div(a->n, channels); };
+    if (items(32, 128) * 4 <= n_cu * 5)
+      return f16 ? launch_tiled<K, false, 2, 8, 3, 1, false, 2, false, false, true>(p, a->rows, s, n_cu, what)
+                 : launch_tiled<K, false, 2, 8, 3, 1, false, 2>(p, a->rows, s, n_cu, what);
+    if (items(64, 256) < n_cu)
+      return f16 ? launch_tiled<K, false, 2, 4, 3, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what)
+                 : launch_tiled<K, false, 2, 4, 3, 1, false, 4>(p, a->rows, s, n_cu, what);
+  }
   const float avg_routed = static_cast<float>(ceil_div(live, a->E));
   const float reach = avg_routed + 3.0f * sqrtf(avg_routed);
   const bool big = weight_bytes > (1ll << 30);

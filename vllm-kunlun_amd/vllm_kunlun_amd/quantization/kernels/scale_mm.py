@@ -49,15 +49,15 @@ class _DynamicCall:
     maxes) and one allocation, the output: 11 us of host time where building the block and looking the parameters up on
     every call took 21."""
 
-    __slots__ = ("args", "n", "k", "device", "scale", "weight", "at", "epoch", "tiled")
+    __slots__ = ("args", "n", "k", "device", "scale", "weight", "at", "epoch", "stream_max")
 
-    # Up to this many rows the GEMM runs on the weight-streaming kernel (the one the fused MoE layer
+    # Up to this many rows (by K) the GEMM runs on the weight-streaming kernel (the one the fused MoE layer
     # runs decode batches and its folded shared expert on): the dense matrix is handed over as the
     # launch's "tail expert", whose rows the kernel cuts into slices of 16 or 32 for as many
-    # workgroups - a tile kernel has too few tiles to fill the chip here. Measured on
-    # [M,7168] x [4096,7168]: 13 us against 36 us at 16 rows, 20 against 38 at 128, 30 against 38 at 256;
-    # at 512 rows the tile kernel is ahead (39 against 46 us).
-    STREAM_MAX_ROWS = 256
+    # workgroups, each reading its weights again. Beyond, the tile kernel on its small tiles. With the quantiser, us:
+    # [M, 7168] x [4096, 7168] 100 rows 19.5 against 22.8, 128 20.1 / 23.2, 160 24.5 / 23.4, 256 29.9 / 24.1;
+    # [M, 2048] x [7168, 2048] 40 rows 11.6 / 12.9, 65 13.2 / 13.0, 100 14.6 / 13.1, 256 21.5 / 15.7.
+    STREAM_MAX_ROWS, STREAM_MAX_ROWS_SHORT_K = 128, 64
 
     def __init__(self, layer, names, w, w_max):
         L.require_device(w, w_max)
@@ -69,7 +69,7 @@ class _DynamicCall:
         self.at = (w.data_ptr(), w_max.data_ptr())
         self.epoch = _plan._layout_epoch
         layout = weight_layout(w)
-        self.tiled = layout == L.KMOE_W_TILED
+        self.stream_max = (self.STREAM_MAX_ROWS if self.k > 4096 else self.STREAM_MAX_ROWS_SHORT_K) if layout == L.KMOE_W_TILED else 0
         g = L.GemmI8Args()
         g.w, g.w_max = self.at
         g.E, g.n, g.k, g.lda, g.ldy, g.src_div = 1, self.n, self.k, self.k, self.n, 1
@@ -116,7 +116,7 @@ class _DynamicCall:
             g.a = x_q = scratch.data_ptr()
             g.a_max = x_max = x_q + codes
             g.y, g.act_dtype = out.data_ptr(), dt
-            if self.tiled and M <= self.STREAM_MAX_ROWS:
+            if M <= self.stream_max:
                 L.check(L.lib.kmoe_quant_i8_rows_chunked_dt(x2.data_ptr(), k, M, k, x_q, x_max, dt, stream))
                 # one routed expert without rows (the launch needs an expert list), the matrix as the tail expert
                 g.a_layout, g.a_rows, g.lod = L.KMOE_A_CHUNKED, M, _row_range(self.device, 0).data_ptr()
