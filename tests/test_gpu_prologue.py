@@ -118,3 +118,44 @@ def test_fp8_group_quantiser_on_every_mantissa(dtype):
     L.check(L.lib.kmoe_quant_fp8_group128_dt(L.ptr(dx), 256, R, 256, L.ptr(q), 256, L.ptr(s), L.act_dtype(dx, "test"), L.stream()))
     assert np.array_equal(s.cpu().numpy().view(np.uint32), s_ref.view(np.uint32))
     assert np.array_equal(q.cpu().numpy(), q_ref)
+
+
+@pytest.mark.parametrize("E,K,n_group", [(8, 4, 2), (64, 8, 1), (129, 8, 1), (256, 8, 8), (520, 8, 4)])
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
+def test_nan_scores_still_give_every_pair_an_expert(E, K, n_group, scoring):
+    """Rows whose scores are NaN with every bit set (memory filled with -1), all of them or all but two: K different
+    experts of the layer, numbers before NaNs."""
+    from vllm_kunlun_amd import _lib as L
+    logits = torch.randn(6, E, generator=torch.Generator().manual_seed(E))
+    nan = torch.full((1,), -1, dtype=torch.int32).view(torch.float32)
+    bias = torch.zeros(E)
+    if scoring == "softmax":
+        logits[1], logits[3, 2:] = nan, nan
+        logits[5, : E - 2] = nan
+    else:  # (the sigmoid of a NaN is a number; a NaN in the correction bias reaches the comparison)
+        bias[2:] = nan
+    logits, bias = logits.cuda(), bias.cuda()
+    w = torch.empty(6, K, device="cuda")
+    ids = torch.full((6, K), -7, dtype=torch.int32, device="cuda")
+    if scoring == "softmax":
+        L.check(L.lib.kmoe_softmax_topk(L.ptr(logits), 6, E, K, 1, L.ptr(w), L.ptr(ids), L.stream()))
+    else:
+        L.check(L.lib.kmoe_sigmoid_group_topk_norm(L.ptr(logits), L.ptr(bias), 6, E, K, n_group, max(1, n_group // 2), 1.0,
+                                                   L.ptr(w), L.ptr(ids), L.stream()))
+    ids = ids.cpu().long()
+    assert int(ids.min()) >= 0 and int(ids.max()) < E
+    assert all(len(set(row.tolist())) == K for row in ids)
+    if scoring == "softmax":
+        assert set(ids[3, :2].tolist()) == {0, 1} and set(ids[5, :2].tolist()) == {E - 2, E - 1}
+
+
+@pytest.mark.parametrize("M", [1, 40])  # a column of workgroups per pair, and one per expert
+def test_nan_logits_of_a_token_leave_the_others_alone(M):
+    from vllm_kunlun_amd import synth
+    shape = synth.scaled(synth.SHAPES["qwen3-decode"], M=M + 1, H=256, E=64, K=8, I=128)
+    sl = synth.make_layer(shape, "cuda", seed=M)
+    want = sl.layer(sl.x, sl.logits)
+    logits = sl.logits.clone()
+    logits[0] = torch.full((1,), -1, dtype=torch.int32).view(torch.float32).cuda()
+    got = sl.layer(sl.x, logits)
+    assert torch.equal(got[1:], want[1:])

@@ -246,11 +246,14 @@ __device__ inline int wave_sum_int(int v) {
   return v;
 }
 
-// A float as an unsigned int with the same order (-0 counts as +0); no finite or infinite value maps to 0.
-__device__ inline uint32_t ordered_bits(float v) {
+// A float as an unsigned int with the same order (-0 counts as +0). Never 0, which stands for "not a candidate" where
+// the largest is picked: one NaN pattern (all bits set, what memory filled with -1 holds) would map there and counts as
+// its neighbour instead; no number does.
+__host__ __device__ inline uint32_t ordered_bits(float v) {
   union { float f; uint32_t u; } b;
   b.f = v + 0.0f;
-  return (b.u & 0x80000000u) ? ~b.u : (b.u | 0x80000000u);
+  const uint32_t key = (b.u & 0x80000000u) ? ~b.u : (b.u | 0x80000000u);
+  return key != 0 ? key : 1;
 }
 __device__ inline uint64_t lanemask_lt() {
   return (static_cast<uint64_t>(1) << lane_id()) - 1;
