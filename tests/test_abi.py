@@ -6,6 +6,7 @@ import os
 import re
 
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -196,3 +197,39 @@ def test_kernel_trace_record_is_per_thread_and_empty_without_launches(L):
     assert lib.kmoe_traced_kernels() == b""
     lib.kmoe_trace_kernels(0)
     assert lib.kmoe_traced_kernels() == b""
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="names the kernel a launch would take, on addresses that are not memory")
+def test_packed_launches_on_rows_beyond_4_gib_do_not_take_32_bit_offsets(L):
+    """Which kernel kmoe_grouped_gemm_w4a16 launches (the record is written before the launch, which fails without a
+    GPU): 32-bit row offsets only where rows * lda * 2 bytes, and a row beyond, stay below 4 GiB and the rows are the
+    launch's own."""
+    def kernel(rows, lda, E=384, k=2048, act=0, variant=0, gather=False):
+        g = L.GemmW4Args()
+        for f in ("a", "w", "w_scale", "lod", "y"):
+            setattr(g, f, 0x10000)
+        g.row_src = 0x10000 if gather else None
+        g.E, g.n, g.k, g.rows, g.lda, g.ldy, g.src_div = E, 7168, k, rows, lda, 7168, 1
+        g.group_size, g.act, g.variant, g.w_layout = 32, act, variant, L.KMOE_W_TILED
+        L.lib.kmoe_trace_kernels(1)
+        assert L.lib.kmoe_grouped_gemm_w4a16(g, None) == -5
+        L.lib.kmoe_trace_kernels(0)
+        return L.lib.kmoe_traced_kernels().decode()
+
+    most = (1 << 32) // (2 * 2048) - 2  # the most rows of 2048 values
+    for rows in (384, most):
+        assert "w4_tile_kernel" in kernel(rows, 2048)
+    for rows in (most + 1, 131072 * 8):
+        assert "stream_gemm_kernel" in kernel(rows, 2048) and "32-bit" not in kernel(rows, 2048)
+    assert "32-bit" in kernel(384, 2048, act=1)                      # few rows per expert: the split launch
+    assert "32-bit" not in kernel(384, 1 << 23, act=1)               # ... far apart
+    assert "32-bit" not in kernel(2, 1 << 32, act=1)                 # (a stride whose product leaves 32 bits itself)
+    assert "32-bit" not in kernel(384, 2048, act=1, gather=True)     # ... or gathered from who knows where
+    for variant in (1, 2, 4):
+        assert "32-bit" not in kernel(384, 2048, variant=variant) and "stream_gemm_kernel" in kernel(most + 1, 2048, variant=variant)
+    g_tile = L.GemmW4Args()
+    for f in ("a", "w", "w_scale", "lod", "y"):
+        setattr(g_tile, f, 0x10000)
+    g_tile.E, g_tile.n, g_tile.k, g_tile.rows, g_tile.lda, g_tile.ldy, g_tile.src_div = 4, 64, 128, 1 << 20, 4096, 64, 1
+    g_tile.group_size, g_tile.variant, g_tile.w_layout = 32, 64, L.KMOE_W_TILED
+    assert L.lib.kmoe_grouped_gemm_w4a16(g_tile, None) == -2 and b"32 bits" in L.lib.kmoe_last_error()

@@ -72,3 +72,44 @@ def test_packed_tiles_give_the_streaming_kernels_bits(variant, blocks, act, dtyp
         L.check(L.lib.kmoe_grouped_gemm_w4a16(g, L.stream()))
         out.append(y)
     assert not out[0].isnan().any() and torch.equal(out[0], out[1])
+
+
+def _dequantised(packed, scale, dtype):
+    """[n, k/2] codes and [n, k/32] scales -> the values the kernels multiply, in float32."""
+    codes = torch.stack([packed & 15, packed >> 4], -1).reshape(packed.shape[0], -1).float() - 8
+    return (codes * scale.float().repeat_interleave(32, 1)).to(dtype).float()
+
+
+@pytest.mark.parametrize("variant", [0, 1, 2, 4])
+@pytest.mark.parametrize("act,gather", [(0, False), (1, False), (1, True)])
+def test_packed_weights_on_rows_far_apart(variant, act, gather):
+    """4-bit weights and activation rows 128 MiB apart: the last ones lie beyond 4 GiB, the reach of a 32-bit offset."""
+    from vllm_kunlun_amd import _lib as L
+    gen = torch.Generator().manual_seed(variant + act)
+    counts, n, k, lda = [9, 0, 20, 11], 64, 256, 1 << 26
+    E, rows, n_out = len(counts), sum(counts), n // 2 if act else n
+    a = torch.randn(rows, k, generator=gen).bfloat16().cuda()
+    far = torch.empty(rows * lda, dtype=torch.bfloat16, device="cuda").view(rows, lda)
+    far[:, :k] = a
+    src = torch.randperm(rows, generator=gen) if gather else torch.arange(rows)
+    dsrc = src.int().cuda()
+    packed = torch.randint(0, 256, (E, n, k // 2), generator=gen, dtype=torch.uint8).cuda()
+    scale = (torch.rand(E, n, k // 32, generator=gen) * 0.02 + 0.002).bfloat16().cuda()
+    tiled = torch.empty_like(packed)
+    L.check(L.lib.kmoe_tile_weights_i8(packed.data_ptr(), tiled.data_ptr(), E, n, k // 2, L.stream()))
+    lod = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    y = torch.full((rows, n_out), float("nan"), dtype=torch.bfloat16, device="cuda")
+    g = L.GemmW4Args()
+    g.a, g.lda, g.row_src, g.src_div = far.data_ptr(), lda, dsrc.data_ptr() if gather else None, 1
+    g.w, g.w_scale, g.group_size, g.lod = tiled.data_ptr(), scale.data_ptr(), 32, lod.data_ptr()
+    g.E, g.n, g.k, g.rows, g.w_layout = E, n, k, rows, L.KMOE_W_TILED
+    g.y, g.ldy, g.act, g.variant, g.act_dtype = y.data_ptr(), n_out, act, variant, L.KMOE_DT_BF16
+    L.check(L.lib.kmoe_grouped_gemm_w4a16(g, L.stream()))
+    ref = torch.cat([a[src[lo:lo + c]].float() @ _dequantised(packed[e], scale[e], torch.bfloat16).T
+                     for e, (c, lo) in enumerate(zip(counts, lod.tolist()))])
+    if act:
+        gate, up = (t.bfloat16().float() for t in ref.split(n_out, 1))
+        ref = torch.nn.functional.silu(gate) * up
+    got = y.float()
+    per_row = (got - ref).norm(dim=1) / ref.norm(dim=1).clamp(min=1e-6)
+    assert not got.isnan().any() and float(per_row.max()) <= 2e-2

@@ -164,7 +164,9 @@ bool routed_streams(const kmoe_moe_args* a) {
     case KMOE_FMT_BF16:
       return streams_bf16(static_cast<int>(rows), a->E, a->H) && streams_bf16(static_cast<int>(rows), a->E, a->I) &&
              !a->w13_bias && !a->w2_bias && a->activation != KMOE_ACT_SWIGLUOAI;
-    default: return w4_gate_up_streams(a->M * a->K, a->E_global > a->E ? static_cast<int>(rows) : 0, a->E, a->H);
+    default:
+      return w4_gate_up_streams(a->M * a->K, a->E_global > a->E ? static_cast<int>(rows) : 0, a->E, a->H) &&
+             w4_rows_fit_32(a->M, a->H, a->H) && w4_rows_fit_32(static_cast<long long>(a->M) * a->K, a->I, a->I);
   }
 }
 
@@ -308,7 +310,8 @@ int run_gemm(const MlpPass& m, bool first, kmoe_stream_t stream) {
     g.act = act;
     g.w_layout = m.w_layout;
     g.act_dtype = m.act_dtype;
-    return grouped_gemm_w4a16_checked(&g, stream, first ? m.scan : nullptr, first ? nullptr : m.slots);
+    return grouped_gemm_w4a16_checked(&g, stream, first ? m.scan : nullptr, first ? nullptr : m.slots,
+                                      first ? m.x_count : m.rows);
   }
   kmoe_gemm_bf16_args g = {};
   g.a = static_cast<const uint16_t*>(a);

@@ -74,13 +74,20 @@ constexpr int kStreamMaxRows = 10;
 inline bool streams_fp8(int live_rows, int E, int k) { return ceil_div(live_rows, E) <= kStreamMaxRows && k <= 8192; }
 inline bool streams_bf16(int live_rows, int E, int k) { return ceil_div(live_rows, E) <= kStreamMaxRows && k % 32 == 0; }
 // kmoe_grouped_gemm_w4a16 with `scan` for the layer's routed gate_up launch where it runs on the streaming kernel
-// (w4_gate_up_streams says whether a launch of these dimensions does).
+// (w4_gate_up_streams says whether a launch of these dimensions does). a_rows: rows of the activations, every source row
+// lies below (-1: not known).
 int grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* args, kmoe_stream_t stream, const StreamScan* scan,
-                               const StreamSlots* slots);
-// The streaming kernel on packed 4-bit weights; passes: 1, 2, 4 for 16, 32, 64 rows per pass.
+                               const StreamSlots* slots, long long a_rows);
+// The streaming kernel on packed 4-bit weights; passes: 1, 2, 4 for 16, 32, 64 rows per pass; rows_fit_32: 32-bit
+// offsets reach every source row.
 int stream_gemm_w4(const kmoe_gemm_w4_args* args, hipStream_t stream, int passes, const StreamScan* scan,
-                   const StreamSlots* slots);
+                   const StreamSlots* slots, bool rows_fit_32);
 bool w4_gate_up_streams(int rows, int rows_hint, int E, int k);
+// Whether a 32-bit byte offset reaches every value of `rows` 16-bit activation rows (and a row's worth beyond, what the
+// kernels' K steps add to the offset of a row).
+inline bool w4_rows_fit_32(long long rows, int64_t lda, int k) {
+  return lda < (1ll << 31) && static_cast<uint64_t>(rows) * static_cast<uint64_t>(lda) * 2u + static_cast<uint64_t>(k) * 2u < (1ull << 32);
+}
 // Persistent 128-row-tile GEMMs for many rows per expert (tiled weights, row-major activations);
 // arguments already validated.
 int tiled_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream);

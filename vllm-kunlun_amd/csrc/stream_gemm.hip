@@ -98,6 +98,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
   static_assert(!QUANT || (FMT == Fmt::I8 && MF == 1 && KS == 1 && !SWIGLU && !SCAN), "QUANT: the 16-row int8 down-projection shape only");
   using acc_t = typename std::conditional<FMT == Fmt::I8, v4i, v4f>::type;
   constexpr bool W4 = FMT == Fmt::W4 || FMT == Fmt::W4H;
+  constexpr bool kRows32 = W4 && KS > 1;  // activation rows through 32-bit offsets (stream_gemm_w4 sees to it that they fit)
   constexpr int V = FMT == Fmt::F8 ? 2 : 1;  // 1 KB blocks of weights per step
   constexpr int AV = W4 ? 4 : V;             // 16-byte vectors of activations per lane and step ...
   constexpr int kAVStride = W4 ? 16 : 64, kALane = W4 ? 64 : 16;  // ... bytes between them, between the lane groups
@@ -159,7 +160,8 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
   // no address arithmetic on the vector unit, which the unpacking keeps busy - and rows past the end lie past the
   // descriptor's end: they read zero and fetch nothing (Kimi-K2 dimensions, 128 tokens: layer 1674 -> 1577 us, Qwen3
   // 93 -> 90). The other formats leave the vector unit idle; there the same loads gain nothing (int8, bf16) or lose
-  // (fp8, DeepSeek-V3 at 128 tokens: 1800 -> 1854 us).
+  // (fp8, DeepSeek-V3 at 128 tokens: 1800 -> 1854 us). A descriptor spans 4 GiB: the weights have one per fragment, the
+  // activations one in all, so launches whose rows may lie further apart (kRows32 false) read them through pointers.
   __amdgpu_buffer_rsrc_t wr[NF];
   const int8_t* wp[NF];
   bool wok[NF];
@@ -314,7 +316,8 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
       const size_t at = srow[mf] >= 0 ? srow[mf] : 0;
       // rows past the end read row 0 (valid memory, results never stored) or nothing
       ap[mf] = p.a + at * p.a_row + lg * kALane;
-      aoff[mf] = srow[mf] >= 0 ? static_cast<uint32_t>(srow[mf]) * static_cast<uint32_t>(p.a_row) + lg * kALane : 0xfffffff0u;
+      if constexpr (kRows32)
+        aoff[mf] = srow[mf] >= 0 ? static_cast<uint32_t>(srow[mf]) * static_cast<uint32_t>(p.a_row) + lg * kALane : 0xfffffff0u;
       if constexpr (FMT == Fmt::F8) asp[mf] = p.a_aux + at * ksteps;
     }
     acc_t acc[MF][NF];
@@ -329,7 +332,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
       for (int mf = 0; mf < MF; ++mf) {
 #pragma unroll
         for (int v = 0; v < AV; ++v) {
-          if constexpr (W4)
+          if constexpr (kRows32)
             areg[slot][mf][v] = buffer_load16(ar, aoff[mf], static_cast<uint32_t>(kb) * static_cast<uint32_t>(p.a_step) + v * kAVStride);
           else
             areg[slot][mf][v] = *reinterpret_cast<const v4i*>(ap[mf] + kb * p.a_step + v * kAVStride);
@@ -478,9 +481,10 @@ int launch_stream(const StreamParams& p, hipStream_t s) {
   const int cols = p.slots.n > 0 ? p.slots.n + (SCAN ? 1 : 0) : p.E;
   const dim3 grid(ceil_div(n_half, (kWaves / KS) * NFH * 16), cols + (p.w_tail ? ceil_div(p.tail_rows, 16 * MF) : 0));
   if (tracing_kernels())
-    note_kernel("stream_gemm_kernel<%s, %d rows per pass, %d channel fragments per wave, %s, %d steps in flight, K split %d%s%s%s>",
+    note_kernel("stream_gemm_kernel<%s, %d rows per pass, %d channel fragments per wave, %s, %d steps in flight, K split %d%s%s%s%s>",
                 fmt_name(FMT), 16 * MF, NF, SWIGLU ? "SiLU-mul" : "plain", D, KS, SCAN ? ", sorts the pairs itself" : "",
-                QUANT ? ", quantises its rows itself" : "", p.slots.n > 0 ? ", a column per pair" : "");
+                QUANT ? ", quantises its rows itself" : "", p.slots.n > 0 ? ", a column per pair" : "",
+                (FMT == Fmt::W4 || FMT == Fmt::W4H) && KS > 1 ? ", 32-bit row offsets" : "");
   hipLaunchKernelGGL((stream_gemm_kernel<FMT, MF, NF, SWIGLU, D, KS, SCAN, QUANT>), grid, dim3(kWaves * kWave), 0, s, p);
   return check_launch("kmoe_grouped_gemm (stream)");
 }
@@ -630,7 +634,8 @@ int stream_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s, const StreamSc
 // waves hide the unpacking and the loads of each other better than a deeper queue does (Qwen3, 64 tokens, layer, steps
 // in flight x split: 1x1 81.7 us, 2x1 81.9, 3x1 83.3, 1x2 78.8, 2x2 81.5; Kimi-K2 dimensions, 128 tokens: 1584 / 1577 /
 // 1606 / 1568 / 1598). Up to 32 columns of a launch with a column per pair do not fill the chip: two steps there (one
-// token 22.5 -> 21.1 and 62 -> 59 us). A caller's variant keeps one wave per K range: the tile kernel's order of sums.
+// token 22.5 -> 21.1 and 62 -> 59 us). A caller's variant, and rows beyond the reach of the split launches' 32-bit
+// offsets, keep one wave per K range: the tile kernel's order of sums, and rows anywhere in memory.
 template <Fmt FMT>
 int stream_w4_shape(const StreamParams& p, bool swiglu, bool scan, int passes, bool split, hipStream_t s) {
   if (passes == 1 && split && p.slots.n > 0 && p.slots.n <= 32)
@@ -645,7 +650,8 @@ int stream_w4_shape(const StreamParams& p, bool swiglu, bool scan, int passes, b
   return swiglu ? launch_stream<FMT, 4, 2, true, 2>(p, s) : launch_stream<FMT, 4, 2, false, 2>(p, s);
 }
 
-int stream_gemm_w4(const kmoe_gemm_w4_args* a, hipStream_t s, int passes, const StreamScan* scan, const StreamSlots* slots) {
+int stream_gemm_w4(const kmoe_gemm_w4_args* a, hipStream_t s, int passes, const StreamScan* scan, const StreamSlots* slots,
+                   bool rows_fit_32) {
   const int q = a->group_size / 32;
   int shift = -1;
   if ((q & (q - 1)) == 0)
@@ -660,8 +666,12 @@ int stream_gemm_w4(const kmoe_gemm_w4_args* a, hipStream_t s, int passes, const 
   const bool swiglu = a->act == KMOE_ACT_SWIGLU;
   if (scan)
     if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
-  return half ? stream_w4_shape<Fmt::W4H>(p, swiglu, scan != nullptr, passes, a->variant == 0, s)
-              : stream_w4_shape<Fmt::W4>(p, swiglu, scan != nullptr, passes, a->variant == 0, s);
+  KMOE_REQUIRE(rows_fit_32 || (!scan && !slots), KMOE_ERR_UNSUPPORTED,
+               "grouped_gemm_w4a16 (stream): a launch that sorts the pairs itself reaches the activations with 32 bits (rows=%d lda=%lld)",
+               a->rows, static_cast<long long>(a->lda));
+  const bool split = a->variant == 0 && rows_fit_32;
+  return half ? stream_w4_shape<Fmt::W4H>(p, swiglu, scan != nullptr, passes, split, s)
+              : stream_w4_shape<Fmt::W4>(p, swiglu, scan != nullptr, passes, split, s);
 }
 
 }  // namespace kmoe

@@ -388,11 +388,11 @@ extern "C" int kmoe_tile_scales_w4(const uint16_t* src, uint16_t* dst, int E, in
 }
 
 extern "C" int kmoe_grouped_gemm_w4a16(const kmoe_gemm_w4_args* a, kmoe_stream_t stream) {
-  return grouped_gemm_w4a16_checked(a, stream, nullptr, nullptr);
+  return grouped_gemm_w4a16_checked(a, stream, nullptr, nullptr, a && !a->row_src ? a->rows : -1);
 }
 
 int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t stream, const StreamScan* scan,
-                                     const StreamSlots* slots) {
+                                     const StreamSlots* slots, long long a_rows) {
   KMOE_REQUIRE(a, KMOE_ERR_NULL, "grouped_gemm_w4a16: NULL args");
   KMOE_REQUIRE(a->a && a->w && a->w_scale && (a->lod || scan) && a->y, KMOE_ERR_NULL, "grouped_gemm_w4a16: NULL pointer");
   KMOE_REQUIRE(a->E >= 1 && a->rows >= 0, KMOE_ERR_SHAPE, "grouped_gemm_w4a16: E=%d rows=%d", a->E, a->rows);
@@ -426,8 +426,10 @@ int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t s
                    frag16 ? 1 : groups, frag16 ? 16 : 1, a->lod, a->E, a->n, a->k, a->y, a->ldy};
   hipStream_t s = as_stream(stream);
   int mf = a->variant;
-  // the tile kernel reaches a source row (gathered or not: below `rows`) through a 32-bit byte offset
-  const bool tile_ok = static_cast<uint64_t>(a->rows) * static_cast<uint64_t>(a->lda) * 2u + static_cast<uint64_t>(a->k) * 2u < (1ull << 32);
+  // the tile kernel reaches a source row (gathered or not: below `rows`) through a 32-bit byte offset, the streaming
+  // kernel's split launches too (gathered rows of a caller may lie anywhere: those take its other launches)
+  const bool tile_ok = w4_rows_fit_32(a->rows, a->lda, a->k);
+  const bool stream_fits_32 = a_rows >= 0 && w4_rows_fit_32(a_rows, a->lda, a->k);
   if (mf == 0) {
     // The streaming kernel where it sorts the pairs itself or has a column of workgroups per pair, or for a gate_up of
     // few rows; its plain down launch is 4 to 7 % behind 16-row tiles from one row per expert on (Qwen3 dims, 16 / 32 /
@@ -455,7 +457,7 @@ int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t s
   switch (mf) {
     case 1:
     case 2:
-    case 4: return stream_gemm_w4(a, s, mf, scan, slots);
+    case 4: return stream_gemm_w4(a, s, mf, scan, slots, stream_fits_32);
     case 16: return swiglu ? launch_w4_tile<1, true>(p, a->rows, f16, s) : launch_w4_tile<1, false>(p, a->rows, f16, s);
     case 32: return swiglu ? launch_w4_tile<2, true>(p, a->rows, f16, s) : launch_w4_tile<2, false>(p, a->rows, f16, s);
     case 64: return swiglu ? launch_w4_tile<4, true>(p, a->rows, f16, s) : launch_w4_tile<4, false>(p, a->rows, f16, s);
