@@ -86,6 +86,14 @@ def test_process_weights_after_loading_on_the_host():
         kern.process_weights_after_loading(bad)
 
 
+def test_rows_the_streaming_kernel_takes_depend_on_the_channels():
+    """Narrow matrices stay on the weight-streaming kernel up to 256 rows, wide ones leave it as soon as its slices fill
+    the chip; every matrix has its first 16 rows there."""
+    from vllm_kunlun_amd.quantization.kernels.scale_mm import _DynamicCall
+    rows = [_DynamicCall._stream_max_rows(n) for n in (16, 576, 1536, 2560, 4096, 7168, 12288, 24576, 1 << 20)]
+    assert rows == [256, 256, 256, 256, 160, 64, 32, 16, 16]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,n,k", [(1, 64, 128), (37, 256, 512), (128, 512, 1024), (700, 256, 256),
                                    (5, 48, 80)])  # the last one does not tile: row-major weights

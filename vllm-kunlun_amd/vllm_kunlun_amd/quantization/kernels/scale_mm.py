@@ -51,13 +51,18 @@ class _DynamicCall:
 
     __slots__ = ("args", "n", "k", "device", "scale", "weight", "at", "epoch", "stream_max")
 
-    # Up to this many rows (by K) the GEMM runs on the weight-streaming kernel (the one the fused MoE layer
-    # runs decode batches and its folded shared expert on): the dense matrix is handed over as the
-    # launch's "tail expert", whose rows the kernel cuts into slices of 16 or 32 for as many
-    # workgroups, each reading its weights again. Beyond, the tile kernel on its small tiles. With the quantiser, us:
-    # [M, 7168] x [4096, 7168] 100 rows 19.5 against 22.8, 128 20.1 / 23.2, 160 24.5 / 23.4, 256 29.9 / 24.1;
-    # [M, 2048] x [7168, 2048] 40 rows 11.6 / 12.9, 65 13.2 / 13.0, 100 14.6 / 13.1, 256 21.5 / 15.7.
-    STREAM_MAX_ROWS, STREAM_MAX_ROWS_SHORT_K = 128, 64
+    # The weight-streaming kernel (the one the fused MoE layer runs decode batches and its folded shared expert on) gets
+    # the dense matrix as the launch's "tail expert", whose rows it cuts into slices of 16 or 32, each reading the
+    # weights again. It is ahead of the tile kernel while its launch has few workgroups - slices of 32 rows times groups
+    # of 32 channels - and the tile kernel fewer still; both grow with K alike. With the quantiser, weights cold, us:
+    # [4096 x 7168] 128 rows 24.5 against 31.0, 160 27.7 / 31.4, 256 35.6 / 32.0; [1536 x 7168] 256 rows 22.4 / 31.4;
+    # [7168 x 2048] 64 rows 13.8 / 14.3, 65 14.7 / 14.1, 128 17.2 / 14.4; [2048 x 2048] 256 rows 11.8 / 12.6;
+    # [8192 x 8192] 64 rows 31.6 / 36.4, 65 39.0 / 36.0; [24576 x 1536] 32 rows 18.1 / 15.3.
+    STREAM_MAX_GROUPS, STREAM_MAX_ROWS = 640, 256
+
+    @classmethod
+    def _stream_max_rows(cls, n: int) -> int:
+        return max(16, min(cls.STREAM_MAX_ROWS, 32 * (cls.STREAM_MAX_GROUPS // -(-n // 32))))
 
     def __init__(self, layer, names, w, w_max):
         L.require_device(w, w_max)
@@ -69,7 +74,7 @@ class _DynamicCall:
         self.at = (w.data_ptr(), w_max.data_ptr())
         self.epoch = _plan._layout_epoch
         layout = weight_layout(w)
-        self.stream_max = (self.STREAM_MAX_ROWS if self.k > 4096 else self.STREAM_MAX_ROWS_SHORT_K) if layout == L.KMOE_W_TILED else 0
+        self.stream_max = self._stream_max_rows(self.n) if layout == L.KMOE_W_TILED else 0
         g = L.GemmI8Args()
         g.w, g.w_max = self.at
         g.E, g.n, g.k, g.lda, g.ldy, g.src_div = 1, self.n, self.k, self.k, self.n, 1
