@@ -55,6 +55,34 @@ def test_dense_tiles(rows, n, dtype):
     assert np.array_equal(bits(out), ref)
 
 
+# several experts on the small tiles: 32 rows, 64 rows (more channel blocks than CUs for the former) and neither, uneven
+# and empty experts, with and without a tail expert
+@pytest.mark.parametrize("counts", [[70, 0, 33], [1, 64, 65, 0, 20, 31, 90, 17], [300, 40]])
+@pytest.mark.parametrize("n", [272, 3088, 6160])
+@pytest.mark.parametrize("tail", [0, 45])
+def test_small_tiles_of_several_experts(counts, n, tail):
+    from vllm_kunlun_amd import _lib as L
+    from vllm_kunlun_amd import _plan
+    k, rows, E = 192, sum(counts), len(counts)
+    gen = torch.Generator().manual_seed(n + tail)
+    a = torch.randint(-127, 128, (rows + tail, k), generator=gen, dtype=torch.int8)
+    a_max, w_max = torch.rand(rows + tail, generator=gen) + 0.5, torch.rand(E + 1, n, generator=gen) + 0.5
+    w = torch.randint(-127, 128, (E + 1, n, k), generator=gen, dtype=torch.int8)
+    lod = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    ref, _ = co.grouped_gemm_i8(a.numpy(), a_max.numpy(), w.numpy(), w_max.numpy(), np.append(lod, rows + tail).astype(np.int32))
+    da, dmax, dw, dw_max, dlod = a.cuda(), a_max.cuda(), w.cuda(), w_max.cuda(), torch.from_numpy(lod).cuda()
+    assert _plan.tile_int8_weights_(dw)
+    y = torch.full((rows + tail, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    g = L.GemmI8Args()
+    g.a, g.lda, g.a_max, g.src_div, g.w, g.w_max, g.lod = da.data_ptr(), k, dmax.data_ptr(), 1, dw.data_ptr(), dw_max.data_ptr(), dlod.data_ptr()
+    g.E, g.n, g.k, g.rows, g.y, g.ldy, g.w_layout = E, n, k, rows, y.data_ptr(), n, L.KMOE_W_TILED
+    if tail:
+        g.w_tail, g.w_max_tail = dw[E].data_ptr(), dw_max[E].data_ptr()
+        g.tail_row0, g.tail_rows, g.tail_src0 = rows, tail, rows
+    L.check(L.lib.kmoe_grouped_gemm_i8(g, L.stream()))
+    assert np.array_equal(bits(y), ref)
+
+
 def test_kept_call_follows_the_layer():
     kern, layer, *_ = _linear(256, 512, 1)
     _, other, *_ = _linear(256, 512, 2)

@@ -1514,18 +1514,30 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   // the paced tiles as variant 12; 19 / 18 / 22 (and 15 / 14 / 8, 16): 128- / 192- / 256-row wide tiles forced.
   // (an expert of up to 3 MiB stays in an XCD's 4 MB L2 while its m-tiles run: their channel blocks go side by side)
   p.m_major = static_cast<long long>(a->n) * a->k <= (3ll << 20) ? 1 : 0;
-  // A plain GEMM of so few tiles that most CUs would stay without one (a dense linear of some hundred rows): 128 channels
-  // per tile instead of 256, of 32 rows while those fill the chip about once, of 64 while 64 x 256 tiles would not.
-  // With the quantiser, us, 64 x 256 / 64 x 128 / 32 x 128 tiles: [4096 x 7168] 257 rows 37.3 / 28.0 / 27.2, 384 38.1 / 29.8 /
-  // 31.4, 512 38.5 / 30.1 / 33.8, 768 40.0 / 39.5 / 48.7, 1024 42.6 / 44.0 / 60.3; [7168 x 2048] 128 rows - / 14.8 / 13.2, 257
-  // 18.4 / 17.0 / 16.0, 512 20.2 / 18.8 / 22.8, 1024 27.3 / 29.3 / 35.0.
+  // A plain GEMM of so few tiles that most CUs would stay without one (a dense linear of some hundred rows, a layer of few
+  // experts): 128 channels per tile instead of 256, of 32 rows while every CU gets at most one, else of 64 on the same
+  // condition. One tile more than CUs and a CU has two to do while the others wait: the taller tiles below are then level
+  // or ahead, unless the weights are so few (16 MB) that reading them per tile costs nothing. With the quantiser, weights
+  // cold, us, 32 x 128 / 64 x 128 / the tiles below: [4096 x 7168] 256 rows 32.0 / 35.9 / 47.5, 512 - / 37.5 / 48.3;
+  // [8192 x 8192] 128 rows 36.9 / 41.2 / 54.1, 129 47.1 / 39.9 / 51.3, 257 - / 53.0 / 51.2; [12288 x 5120] 65 rows 34.0 /
+  // 28.6 / 36.6, 256 48.8 / 42.5 / 39.3; [7168 x 2048] 257 rows - / 17.1 / 19.9, 512 - / 21.5 / 21.6.
+  // Several experts: the tiles are counted for rows spread evenly with two standard deviations of headroom, and a quarter of
+  // the CUs is left for an uneven load where 64-row tiles would be as good. [4096 x 14336] of 8 experts, us, the tiles below
+  // / 64 x 128: 24 rows each 100 / 85, 48 108 / 88, 64 (two tiles each, not taken) 110 / 125; with a third of the rows on one
+  // expert 16 rows each 104 / 87 (32 x 128: 110), but 32 rows each 103 / 114: two tiles for that expert, one too many for the
+  // CUs. [4096 x 4096] of 2 experts 25 / 18, [7168 x 2048] of 4 experts at 16 rows each 17.4 / 15.2.
   if (a->variant == 0 && !swiglu) {
     const bool f16 = a->act_dtype == KMOE_DT_F16;
-    auto items = [&](int rows, int channels) { return (ceil_div(live + p.tail_rows, rows) + n_exp - 1) * ceil_div(a->n, channels); };
-    if (items(32, 128) * 4 <= n_cu * 5)
+    const float mean = static_cast<float>(live) / a->E;
+    const int most = a->E == 1 ? live : static_cast<int>(ceilf(mean + 2.0f * sqrtf(mean)));  // rows of an expert
+    auto items = [&](int rows, int channels) {
+      return (static_cast<long long>(a->E) * ceil_div(most, rows) + ceil_div(p.tail_rows, rows)) * ceil_div(a->n, channels);
+    };
+    const bool few_weights = weight_bytes <= (16ll << 20);
+    if (items(32, 128) <= (n_exp <= 2 ? n_cu : n_cu * 3 / 4))
       return f16 ? launch_tiled<K, false, 2, 8, 3, 1, false, 2, false, false, true>(p, a->rows, s, n_cu, what)
                  : launch_tiled<K, false, 2, 8, 3, 1, false, 2>(p, a->rows, s, n_cu, what);
-    if (items(64, 256) < n_cu)
+    if (items(64, 128) <= n_cu || (few_weights && items(64, 256) < n_cu))
       return f16 ? launch_tiled<K, false, 2, 4, 3, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what)
                  : launch_tiled<K, false, 2, 4, 3, 1, false, 4>(p, a->rows, s, n_cu, what);
   }
