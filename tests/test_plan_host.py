@@ -61,3 +61,28 @@ def test_plan_refuses_another_stream(monkeypatch):
     monkeypatch.setattr(_plan, "_current_stream_id", lambda device: 0x20)
     with pytest.raises(RuntimeError, match="built on stream 0x10"):
         plan()
+
+
+def _kept_call(*tensors):
+    plan = _plan.MoEPlan(L.MoEArgs(), None, None, [])
+    return _plan._LayerCall(plan, tensors, experts=4)
+
+
+@pytest.mark.parametrize("change", [lambda d: d.transpose(1, 2), lambda d: d.view(torch.float16), lambda d: d.view(2, 32, 16),
+                                    lambda d: d.clone(), lambda d: d[:, :, :8]])
+def test_kept_block_is_dropped_when_a_weight_becomes_another_view(change):
+    """The same Parameter over the same memory with other strides, another type or another shape (which filling a block
+    refuses) must not be served from the block kept for it."""
+    w = torch.nn.Parameter(torch.zeros(4, 16, 16, dtype=torch.bfloat16), requires_grad=False)
+    call = _kept_call(w, torch.zeros(4))
+    assert not call.holds()  # (the second tensor is gone)
+    scale = torch.zeros(4)
+    call = _kept_call(w, scale)
+    assert call.holds()
+    w.data = w.data[:]
+    assert call.holds()
+    kept = w.data  # (the memory stays alive: another tensor cannot take its place)
+    w.data = change(w.data)
+    assert not call.holds()
+    w.data = kept
+    assert call.holds()

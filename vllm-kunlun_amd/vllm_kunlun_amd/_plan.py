@@ -376,18 +376,19 @@ class _LayerCall:
 
     def __init__(self, plan: MoEPlan, tensors, experts: int):
         self.args = L.MoEArgs.from_buffer_copy(plan.args)
-        self.tensors = [(weakref.ref(t), t.data_ptr(), t.shape) for t in tensors]
+        self.tensors = [(weakref.ref(t), t.data_ptr(), t.shape, t.dtype) for t in tensors]
         self.epoch = _layout_epoch
         self.hidden, self.experts, self.layouts = int(plan.args.H), experts, {}
 
     def holds(self) -> bool:
-        """Whether the tensors are still the objects, at the addresses and of the shapes the block was filled for, and
-        no weight was re-arranged since."""
+        """Whether the tensors are still the objects, at the addresses, of the shapes and types and contiguous as the
+        block was filled for (a tensor's `.data` may have become another view of its memory), and no weight was
+        re-arranged since."""
         if self.epoch != _layout_epoch:
             return False
-        for ref, at, shape in self.tensors:
+        for ref, at, shape, dtype in self.tensors:
             t = ref()
-            if t is None or t.data_ptr() != at or t.shape != shape:
+            if t is None or t.data_ptr() != at or t.shape != shape or t.dtype != dtype or not t.is_contiguous():
                 return False
         return True
 
@@ -421,7 +422,7 @@ def run_layer(fmt: int, x: torch.Tensor, logits: Optional[torch.Tensor], top_k: 
     costs more host time than a decode step takes on the GPU, and a model's step makes the same call per layer again
     and again, so the block is kept: a later call with the same weights and options copies it and fills in the batch
     (Qwen3 shape, one token: host time per call 55 -> 19 us). What may have changed is compared, not assumed: the
-    tensors' identity, address and shape, and the state of the weights' re-arrangement."""
+    tensors' identity, address, shape, type and contiguity, and the state of the weights' re-arrangement."""
     x = x.contiguous()
     if logits is not None:
         if logits.dtype != torch.float32 and logits.dtype != x.dtype:
