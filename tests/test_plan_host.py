@@ -86,3 +86,20 @@ def test_kept_block_is_dropped_when_a_weight_becomes_another_view(change):
     assert not call.holds()
     w.data = kept
     assert call.holds()
+
+
+def test_kept_block_is_dropped_when_re_arranged_memory_is_freed():
+    """Weights that were re-tiled, freed, and loaded again row-major: the allocator may hand out the same address, so
+    the block that says "tiled" must not outlive the mark."""
+    memory = torch.zeros(4096, dtype=torch.int8)  # two storages over one piece of memory stand for a reused address
+    first, second = (torch.from_numpy(memory.numpy()).view(4, 16, 64) for _ in range(2))
+    assert first.untyped_storage()._cdata != second.untyped_storage()._cdata
+    _plan._mark_tiled(first, 16, 64)
+    w = torch.nn.Parameter(first, requires_grad=False)
+    call = _kept_call(w)
+    assert call.holds() and _plan.is_tiled(w)
+    del first
+    w.data = second
+    gc.collect()
+    assert not _plan.is_tiled(w) and not call.holds()
+    assert _kept_call(w).holds()

@@ -9,6 +9,7 @@ refuses to launch on another.
 from __future__ import annotations
 
 import collections
+import itertools
 import weakref
 from typing import Optional
 
@@ -81,16 +82,27 @@ class MoEPlan:
 # torch's StorageImpl, dropped when the storage dies), not to a tensor object: views, `.data`, `.detach()`,
 # `.t()` and a Parameter wrapped around the same memory all see it.
 _TILED: dict[int, tuple[int, int]] = {}  # storage -> (n, bytes of k) of the tiles it holds
-_layout_epoch = 0  # counts re-arrangements of weights: what run_layer remembers about a layout holds within one
+_EPOCHS = itertools.count(1)
+_layout_epoch = 0  # another number whenever memory begins or ceases to be re-arranged: a kept block holds within one
+
+
+def _mark(marks: dict, storage, dims: tuple) -> None:
+    """Enters re-arranged memory into `marks` for as long as its storage lives. A later storage may lie at the same
+    address and not be re-arranged, so what was kept about a layout ends with a mark as it does with a new one."""
+    def drop():
+        global _layout_epoch
+        marks.pop(key, None)
+        _layout_epoch = next(_EPOCHS)
+
+    global _layout_epoch
+    _layout_epoch = next(_EPOCHS)
+    key = storage._cdata
+    marks[key] = dims
+    weakref.finalize(storage, drop)
 
 
 def _mark_tiled(w: torch.Tensor, n: int, k_bytes: int) -> None:
-    global _layout_epoch
-    _layout_epoch += 1
-    storage = w.untyped_storage()
-    key = storage._cdata
-    _TILED[key] = (n, k_bytes)
-    weakref.finalize(storage, _TILED.pop, key, None)
+    _mark(_TILED, w.untyped_storage(), (n, k_bytes))
 
 
 def is_tiled(w: torch.Tensor) -> bool:
@@ -158,11 +170,7 @@ def tile_w4_scales_(scale: torch.Tensor) -> bool:
     for e in range(E):
         L.check(L.lib.kmoe_tile_scales_w4(L.ptr(data[e]), L.ptr(tmp), 1, n, groups, L.stream()))
         data[e].copy_(tmp)
-    global _layout_epoch
-    _layout_epoch += 1
-    storage = data.untyped_storage()
-    _SCALES_FRAG16[key] = (n, groups)
-    weakref.finalize(storage, _SCALES_FRAG16.pop, key, None)
+    _mark(_SCALES_FRAG16, data.untyped_storage(), (n, groups))
     return True
 
 
