@@ -83,6 +83,21 @@ def test_small_tiles_of_several_experts(counts, n, tail):
     assert np.array_equal(bits(y), ref)
 
 
+@pytest.mark.parametrize("kind", ["buffer", "attribute"])
+def test_scale_that_is_no_parameter(kind):
+    kern, layer, codes, w_max = _linear(64, 128, 5)
+    x = torch.randn(9, 128, generator=torch.Generator().manual_seed(1)).bfloat16()
+    want = kern.apply_weights(layer, x.cuda())
+    scale = layer.weight_scale.data
+    del layer.weight_scale
+    if kind == "buffer":
+        layer.register_buffer("weight_scale", scale)
+    else:
+        layer.weight_scale = scale
+    for _ in range(2):
+        assert torch.equal(kern.apply_weights(layer, x.cuda()), want)
+
+
 def test_kept_call_follows_the_layer():
     kern, layer, *_ = _linear(256, 512, 1)
     _, other, *_ = _linear(256, 512, 2)

@@ -86,6 +86,43 @@ def test_process_weights_after_loading_on_the_host():
         kern.process_weights_after_loading(bad)
 
 
+@pytest.mark.parametrize("kind", ["parameter", "buffer", "attribute", "plain object"])
+def test_kept_dynamic_call_finds_the_tensors_where_the_layer_has_them(kind, monkeypatch):
+    """The block kept on a layer asks for the scale where getattr would: a Parameter, a buffer or a plain tensor an engine
+    put in its place; an input scale or zero-point sums that appear in any of these forms end the dynamic call."""
+    from vllm_kunlun_amd import _lib as L
+    from vllm_kunlun_amd.quantization.kernels.scale_mm import KunlunScaledMMLinearKernel, _DynamicCall
+    monkeypatch.setattr(L, "require_device", lambda *tensors: None)
+    names = KunlunScaledMMLinearKernel().layer_param_names
+    scale = torch.ones(16, 1)
+    layer = SimpleNamespace() if kind == "plain object" else torch.nn.Module()
+    if kind == "parameter":
+        scale = layer.weight_scale = torch.nn.Parameter(scale, requires_grad=False)
+    elif kind == "buffer":
+        layer.register_buffer("weight_scale", scale)
+    else:
+        layer.weight_scale = scale
+    layer._kmoe_w_1nk = torch.zeros(1, 16, 64, dtype=torch.int8)
+    call = _DynamicCall(layer, names, layer._kmoe_w_1nk, scale)
+    assert call.holds(layer, names)
+    for name in (names[2], names[4]):
+        for value in (torch.ones(1), torch.nn.Parameter(torch.ones(1), requires_grad=False)):
+            setattr(layer, name, value)
+            assert not call.holds(layer, names)
+            delattr(layer, name)
+            setattr(layer, name, None)
+            assert call.holds(layer, names)
+            delattr(layer, name)
+    kept = layer._kmoe_w_1nk
+    layer._kmoe_w_1nk = kept.view(1, 64, 16)
+    assert not call.holds(layer, names)
+    layer._kmoe_w_1nk = kept
+    del layer.weight_scale
+    assert not call.holds(layer, names)
+    layer.weight_scale = torch.nn.Parameter(scale.detach().clone(), requires_grad=False)
+    assert not call.holds(layer, names)
+
+
 def test_rows_the_streaming_kernel_takes_depend_on_the_channels():
     """Narrow matrices stay on the weight-streaming kernel up to 256 rows, wide ones leave it as soon as its slices fill
     the chip; every matrix has its first 16 rows there."""

@@ -43,13 +43,16 @@ def _row_range(device, rows):
     return _ROW_RANGES[key]
 
 
+_NOTHING: dict = {}
+
+
 class _DynamicCall:
     """Quantisation and GEMM of one Linear with dynamic symmetric activations: the GEMM's argument block with everything
     but the batch filled in, kept on the layer. A call is two launches on a scratch buffer of the stream (codes, then row
     maxes) and one allocation, the output: 11 us of host time where building the block and looking the parameters up on
     every call took 21."""
 
-    __slots__ = ("args", "n", "k", "device", "scale", "weight", "at", "epoch", "stream_max")
+    __slots__ = ("args", "n", "k", "device", "scale", "at", "epoch", "stream_max")
 
     # The weight-streaming kernel (the one the fused MoE layer runs decode batches and its folded shared expert on) gets
     # the dense matrix as the launch's "tail expert", whose rows it cuts into slices of 16 or 32, each reading the
@@ -69,8 +72,7 @@ class _DynamicCall:
         L.require_contig(w, w_max)
         _, self.n, self.k = w.shape
         self.device = w.device
-        params = self._params(layer)
-        self.weight, self.scale = params.get(names[0]), params.get(names[1])
+        self.scale = self._value(layer, names[1])
         self.at = (w.data_ptr(), w_max.data_ptr())
         self.epoch = _plan._layout_epoch
         layout = weight_layout(w)
@@ -82,16 +84,19 @@ class _DynamicCall:
         self.args = g
 
     @staticmethod
-    def _params(layer) -> dict:
-        return layer.__dict__.get("_parameters", layer.__dict__)  # (a plain object holds them as attributes)
+    def _value(layer, name):
+        """getattr(layer, name, None), sooner for a Module's parameters (an engine may also put a buffer or a plain tensor
+        in a parameter's place)."""
+        value = layer.__dict__.get("_parameters", _NOTHING).get(name)
+        return getattr(layer, name, None) if value is None else value
 
     def holds(self, layer, names) -> bool:
-        """Whether the layer's parameters are still the ones the block was filled from."""
-        params = self._params(layer)
-        w, scale = layer.__dict__.get("_kmoe_w_1nk"), params.get(names[1])
-        return (scale is self.scale and params.get(names[0]) is self.weight and w is not None
-                and w.data_ptr() == self.at[0] and scale.data_ptr() == self.at[1] and params.get(names[2]) is None
-                and params.get(names[4]) is None and self.epoch == _plan._layout_epoch)
+        """Whether the layer's tensors are still the ones the block was filled from, and a call of it still dynamic and
+        symmetric (no input scale, no zero-point sums)."""
+        w, scale = getattr(layer, "_kmoe_w_1nk", None), self._value(layer, names[1])
+        return (scale is not None and scale is self.scale and w is not None and w.data_ptr() == self.at[0]
+                and w.shape == (1, self.n, self.k) and scale.data_ptr() == self.at[1] and self._value(layer, names[2]) is None
+                and self._value(layer, names[4]) is None and self.epoch == _plan._layout_epoch)
 
     def __deepcopy__(self, memo):
         return None  # (a copied layer fills a block of its own)
@@ -223,7 +228,7 @@ class KunlunScaledMMLinearKernel:
         setattr(layer, w_s_name, torch.nn.Parameter(scale, requires_grad=False))
         if getattr(layer, i_s_name, None) is not None and not self.config.is_static_input_scheme:
             setattr(layer, i_s_name, None)
-        for name in (i_zp_name, azp_adj_name):
+        for name in (i_s_name, i_zp_name, azp_adj_name):
             if not hasattr(layer, name):
                 setattr(layer, name, None)
 
