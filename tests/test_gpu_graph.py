@@ -127,6 +127,30 @@ def test_dense_matmul_op_under_graph_capture():
     _replays(graph, (x, x_max), fresh, out, eager)
 
 
+@pytest.mark.parametrize("M", [7, 203, 300])  # the weight-streaming kernel (twice) and the tiles
+def test_dense_linear_of_a_new_size_under_graph_capture(M, monkeypatch):
+    """A capture may be the first to see a batch size: nothing the linear needs is uploaded per size."""
+    from vllm_kunlun_amd.quantization.kernels import scale_mm
+    n, k = 256, 512
+    g = torch.Generator(device="cuda").manual_seed(M)
+    layer = torch.nn.Module()
+    layer.weight = torch.nn.Parameter(torch.randint(-127, 128, (n, k), generator=g, device="cuda", dtype=torch.int8), requires_grad=False)
+    layer.weight_scale = torch.nn.Parameter(torch.rand(n, 1, generator=g, device="cuda") * 0.01 + 0.001, requires_grad=False)
+    kern = scale_mm.KunlunScaledMMLinearKernel()
+    kern.process_weights_after_loading(layer)
+    kern.apply_weights(layer, torch.randn(1, k, generator=g, device="cuda").bfloat16())
+    monkeypatch.setattr(scale_mm, "_ROW_RANGES", {})
+    x = torch.randn(M, k, generator=g, device="cuda").bfloat16()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = kern.apply_weights(layer, x)
+        other = kern.apply_weights(layer, x)  # (reuses what the first call's scratch left in the graph's memory)
+    fresh = [(torch.randn(M, k, generator=g, device="cuda").bfloat16(),) for _ in range(4)]
+    _replays(graph, (x,), fresh, out, lambda xx: kern.apply_weights(layer, xx))
+    assert torch.equal(out, other)
+
+
 def test_two_threads_share_the_side_stream():
     """Two host threads, each with a stream and a layer of its own whose shared expert runs on the library's second
     stream (one per GPU: both threads fork to it and join from it), calling at the same time: every call gives the

@@ -123,6 +123,21 @@ def test_kept_dynamic_call_finds_the_tensors_where_the_layer_has_them(kind, monk
     assert not call.holds(layer, names)
 
 
+def test_row_ranges_made_in_a_capture_are_the_graphs_own(monkeypatch):
+    from vllm_kunlun_amd.quantization.kernels import scale_mm
+    monkeypatch.setattr(scale_mm, "_ROW_RANGES", {})
+    cpu = torch.device("cpu")
+    with monkeypatch.context() as m:
+        m.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        for rows in (0, 1, 2, 203, 1 << 20):
+            made = scale_mm._row_range(cpu, rows)
+            assert made.dtype == torch.int32 and made.tolist() == [0, rows]
+        assert not scale_mm._ROW_RANGES
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    kept = scale_mm._row_range(cpu, 203)
+    assert kept.tolist() == [0, 203] and scale_mm._row_range(cpu, 203) is kept
+
+
 def test_rows_the_streaming_kernel_takes_depend_on_the_channels():
     """Narrow matrices stay on the weight-streaming kernel up to 256 rows, wide ones leave it as soon as its slices fill
     the chip; every matrix has its first 16 rows there."""

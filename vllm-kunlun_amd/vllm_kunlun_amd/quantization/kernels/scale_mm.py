@@ -38,9 +38,15 @@ _ROW_RANGES: dict = {}  # (device, rows) -> the {0, rows} row range of a dense G
 
 def _row_range(device, rows):
     key = (device, rows)
-    if key not in _ROW_RANGES:
-        _ROW_RANGES[key] = torch.tensor([0, rows], dtype=torch.int32).to(device)
-    return _ROW_RANGES[key]
+    found = _ROW_RANGES.get(key)
+    if found is None:
+        if torch.cuda.is_current_stream_capturing():
+            # (an upload cannot be captured; a launch of the graph's own writes the two numbers on every replay, into
+            # the graph's memory, so the tensor is of no use to other calls)
+            return torch.arange(0, rows + 1, rows, dtype=torch.int32, device=device) if rows else \
+                torch.zeros(2, dtype=torch.int32, device=device)
+        found = _ROW_RANGES[key] = torch.tensor([0, rows], dtype=torch.int32).to(device)
+    return found
 
 
 _NOTHING: dict = {}
@@ -129,11 +135,14 @@ class _DynamicCall:
             if M <= self.stream_max:
                 L.check(L.lib.kmoe_quant_i8_rows_chunked_dt(x2.data_ptr(), k, M, k, x_q, x_max, dt, stream))
                 # one routed expert without rows (the launch needs an expert list), the matrix as the tail expert
-                g.a_layout, g.a_rows, g.lod = L.KMOE_A_CHUNKED, M, _row_range(self.device, 0).data_ptr()
+                lod = _row_range(self.device, 0)
+                g.a_layout, g.a_rows = L.KMOE_A_CHUNKED, M
                 g.w_tail, g.w_max_tail, g.tail_rows = self.at[0], self.at[1], M
             else:
                 L.check(L.lib.kmoe_quant_i8_rows_dt(x2.data_ptr(), k, M, k, x_q, k, x_max, dt, stream))
-                g.lod, g.rows = _row_range(self.device, M).data_ptr(), M
+                lod = _row_range(self.device, M)
+                g.rows = M
+            g.lod = lod.data_ptr()
             L.check(L.lib.kmoe_grouped_gemm_i8(g, stream))
         return out if flat else out.reshape(*x.shape[:-1], n)
 
