@@ -103,3 +103,20 @@ def test_kept_block_is_dropped_when_re_arranged_memory_is_freed():
     gc.collect()
     assert not _plan.is_tiled(w) and not call.holds()
     assert _kept_call(w).holds()
+
+
+def test_layers_that_hit_outlive_calls_that_always_miss(monkeypatch):
+    """Least recently USED first out: a layer called in every step keeps its block although another one's calls (fresh
+    tensors each time) fill the table over and over."""
+    monkeypatch.setattr(_plan, "_CALLS", type(_plan._CALLS)())
+    monkeypatch.setattr(_plan, "MAX_CALLS", 4)
+    w = torch.zeros(4, 16, 64)
+    mine = _kept_call(w)
+    _plan._keep_call("layer", mine)
+    for step in range(20):
+        assert _plan._kept_call("layer") is mine
+        _plan._keep_call(("other", step), _kept_call(w))
+    assert len(_plan._CALLS) == 4
+    for step in range(4):
+        _plan._keep_call(("other", step), _kept_call(w))
+    assert _plan._kept_call("layer") is None

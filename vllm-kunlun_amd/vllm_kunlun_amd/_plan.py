@@ -418,6 +418,24 @@ _CALLS: collections.OrderedDict = collections.OrderedDict()
 MAX_CALLS = 1024
 
 
+def _kept_call(key) -> Optional[_LayerCall]:
+    call = _CALLS.get(key)
+    if call is None or not call.holds():
+        return None
+    try:
+        _CALLS.move_to_end(key)
+    except KeyError:  # (another thread has just dropped it)
+        pass
+    return call
+
+
+def _keep_call(key, call: _LayerCall) -> None:
+    _CALLS[key] = call
+    _CALLS.move_to_end(key)
+    while len(_CALLS) > MAX_CALLS:
+        _CALLS.popitem(last=False)
+
+
 def run_layer(fmt: int, x: torch.Tensor, logits: Optional[torch.Tensor], top_k: int, w13: torch.Tensor, w2: torch.Tensor,
               w13_aux: Optional[torch.Tensor], w2_aux: Optional[torch.Tensor], scoring_func: str = "softmax",
               renormalize: bool = True, num_expert_group: Optional[int] = None, topk_group: Optional[int] = None,
@@ -441,8 +459,8 @@ def run_layer(fmt: int, x: torch.Tensor, logits: Optional[torch.Tensor], top_k: 
            scoring_func, renormalize, num_expert_group, topk_group, routed_scaling_factor, id(e_score_correction_bias),
            None if shared_expert is None else tuple(map(id, shared_expert)), out_scale, id(router_weight), group_size,
            shared_scale, first_expert, side_stream)
-    call = _CALLS.get(key)
-    if call is None or not call.holds():
+    call = _kept_call(key)
+    if call is None:
         plan = make_moe_plan(fmt, x, logits, out, top_k, w13, w2, w13_aux, w2_aux, scoring_func, renormalize,
                              num_expert_group, topk_group, routed_scaling_factor, e_score_correction_bias, shared_expert,
                              out_scale, router_weight=router_weight, group_size=group_size, shared_scale=shared_scale,
@@ -450,9 +468,7 @@ def run_layer(fmt: int, x: torch.Tensor, logits: Optional[torch.Tensor], top_k: 
         tensors = [t for t in (w13, w2, w13_aux, w2_aux, e_score_correction_bias, router_weight, *(shared_expert or ()))
                    if t is not None]
         routed = logits.shape[-1] if logits is not None else router_weight.shape[0]
-        _CALLS[key] = _LayerCall(plan, tensors, routed)
-        while len(_CALLS) > MAX_CALLS:
-            _CALLS.popitem(last=False)
+        _keep_call(key, _LayerCall(plan, tensors, routed))
         plan()
         return out, plan.layout, plan.workspace
     M = x.shape[0]
