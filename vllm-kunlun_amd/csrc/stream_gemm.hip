@@ -70,6 +70,7 @@ struct StreamParams {
   int32_t groups, s_ch, s_g;
   int32_t gs32, gs_shift;  // values per group / 32, and its log2 if it is a power of two, else -1
   StreamSlots slots;  // n > 0: a column of workgroups per pair instead of per expert (pair_scan.h)
+  int32_t late_w;  // the first weight steps are requested when the column's rows are known
 };
 
 constexpr int kWaves = 4;
@@ -185,8 +186,11 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
   // workgroups of a launch do the same work, so they start and end in rounds, and a round that begins with those
   // loads leaves the memory queue idle for their latency. Done where a wave's K range is short (a workgroup lives
   // a few microseconds: Qwen3 decode down projection 42.8 -> 40.4 us); with long ranges it changes nothing for the
-  // better (DeepSeek-V3 decode: +0.4 %), so those keep the plain order.
-  const bool w_first = QUANT || W4 || klen * V < 16;
+  // better (DeepSeek-V3 decode: +0.4 %), so those keep the plain order. So do 16-bit launches
+  // with a column per expert and fewer than three rows per expert (p.late_w): a third of an expert's bytes is much to ask
+  // for where it may have no rows (Qwen3 dims, layer: 16 tokens 150 -> 143 us, with +2.0 on the logits of 8 experts 115
+  // -> 104; 48 tokens 204.5 / 205.6); the columns of pairs rarely have none (6 tokens 79 / 81).
+  const bool w_first = QUANT || W4 || (klen * V < 16 && !p.late_w);
   const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.a), 0, 0xfffffff0, 0x00020000);
   v4i wreg[D][NF][V];
   v4i areg[D][MF][AV];
@@ -625,10 +629,11 @@ int stream_gemm_fp8(const kmoe_gemm_fp8_args* a, hipStream_t s, const StreamScan
 
 int stream_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s, const StreamScan* scan, const StreamSlots* slots) {
   const bool half = a->act_dtype == KMOE_DT_F16;
+  const StreamSlots columns = slots_of(scan, slots);
   const StreamParams p{reinterpret_cast<const int8_t*>(a->a), a->lda * 2, 64, 0, nullptr, a->row_src, a->src_div,
                        reinterpret_cast<const int8_t*>(a->w), nullptr, a->lod, a->E, a->n, a->k * 2, a->y, a->ldy, nullptr,
                        nullptr, nullptr, 0, 0, 0, half, 0, scan ? *scan : StreamScan{}, StreamQuant{},
-                       nullptr, 0, 0, 0, 0, 0, slots_of(scan, slots)};
+                       nullptr, 0, 0, 0, 0, 0, columns, columns.n == 0 && expected_rows(a->rows, a->rows_hint) < 3ll * a->E};
   const bool swiglu = a->act == KMOE_ACT_SWIGLU;
   if (scan) {
     if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
