@@ -48,7 +48,9 @@ def test_row_fragments(variant, n, k, act, dtype):
 @pytest.mark.parametrize("act", [0, 1])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_packed_tiles_give_the_streaming_kernels_bits(variant, blocks, act, dtype):
-    """4-bit weights: every tile height against the streaming kernel, which adds the same products in the same order."""
+    """4-bit weights: every tile height against the streaming kernel's launches that do not split K (variant 1), which
+    add the same products in the same order, and both, with the launch the sizes choose (variant 0), against a float32
+    product of the unpacked values."""
     from vllm_kunlun_amd import _lib as L
     gen = torch.Generator().manual_seed(blocks)
     counts = ROWS + [31, 32, 63, 64, 65]
@@ -62,7 +64,7 @@ def test_packed_tiles_give_the_streaming_kernels_bits(variant, blocks, act, dtyp
     lod = torch.tensor([0] + counts).cumsum(0).int().cuda()
     n_out = n // 2 if act else n
     out = []
-    for v in (1, variant):
+    for v in (1, variant, 0):
         y = torch.full((rows, n_out), float("nan"), dtype=dtype, device="cuda")
         g = L.GemmW4Args()
         g.a, g.lda, g.row_src, g.src_div = a.data_ptr(), k, src.data_ptr(), 1
@@ -72,6 +74,14 @@ def test_packed_tiles_give_the_streaming_kernels_bits(variant, blocks, act, dtyp
         L.check(L.lib.kmoe_grouped_gemm_w4a16(g, L.stream()))
         out.append(y)
     assert not out[0].isnan().any() and torch.equal(out[0], out[1])
+    ref = torch.cat([a[src[lo:lo + c].long()].float() @ _dequantised(packed[e], scale[e], dtype).T
+                     for e, (c, lo) in enumerate(zip(counts, lod.tolist()))])
+    if act:
+        gate, up = (t.to(dtype).float() for t in ref.split(n_out, 1))
+        ref = torch.nn.functional.silu(gate) * up
+    for y in out[1:]:
+        per_row = (y.float() - ref).norm(dim=1) / ref.norm(dim=1).clamp(min=1e-6)
+        assert float((y.float() - ref).norm() / ref.norm()) <= 4e-3 and float(per_row.max()) <= 2e-2
 
 
 def _dequantised(packed, scale, dtype):
