@@ -82,6 +82,33 @@ def test_shared_expert_on_the_side_stream_under_graph_capture(quant, side):
     _replays(graph, (x, logits), fresh, out, eager)
 
 
+@pytest.mark.parametrize("M", [64, 65, 80])
+def test_fp8_shared_expert_in_the_routed_launches_and_beside_them(M):
+    """The fp8 layer's shared expert of the routed experts' width rides in the routed launches, or, from 65 tokens on for
+    a caller that allows the second stream, runs beside them: the same result up to the order of its sums, eager and
+    captured."""
+    from vllm_kunlun_amd import synth
+    shape = synth.scaled(synth.SHAPES["dsv3-fp8-decode"], M=M, H=512, E=32, K=4, I=256, n_group=4, topk_group=2, I_shared=256)
+    sl = synth.make_layer(shape, "cuda", seed=M)
+    method, kw = sl.layer.quant_method, sl.apply_kwargs()
+    call = lambda xx, ll: method.apply_monolithic(sl.layer, xx, ll, **kw)  # noqa: E731
+    folded = call(sl.x, sl.logits)
+    own_bytes = method.last_layout.sh_out - method.last_layout.sh_act
+    method.side_stream = True
+    beside = call(sl.x, sl.logits)
+    assert (method.last_layout.sh_out - method.last_layout.sh_act > own_bytes) == (M > 64)
+    torch.cuda.synchronize()
+    assert float((beside.float() - folded.float()).norm() / folded.float().norm()) <= 4e-3
+    x, logits = sl.x.clone(), sl.logits.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call(x, logits)
+    g = torch.Generator(device="cuda").manual_seed(12)
+    fresh = [(torch.randn(M, shape.H, generator=g, device="cuda").bfloat16(),
+              torch.randn(M, shape.E, generator=g, device="cuda")) for _ in range(4)]
+    _replays(graph, (x, logits), fresh, out, call)
+
+
 def test_static_workspace_forward_under_graph_capture():
     from vllm_kunlun_amd import _lib as L
     from vllm_kunlun_amd import synth

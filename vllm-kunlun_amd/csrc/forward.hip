@@ -144,15 +144,6 @@ bool use_stream_path(const kmoe_moe_args* a) {
          (a->I_shared == 0 || a->ws_layout == KMOE_W_TILED);
 }
 
-// A shared expert of the routed experts' width runs inside the routed GEMM launches
-// as one more ("tail") expert over rows [P, P+M): no extra launches, and its few
-// workgroups overlap the routed experts' instead of leaving most CUs idle.
-bool fold_shared(const kmoe_moe_args* a) {
-  if (a->I_shared <= 0 || a->I_shared != a->I || a->ws_layout != a->w_layout) return false;
-  if (a->format == KMOE_FMT_INT8) return true;
-  return a->format == KMOE_FMT_FP8_BLOCK && a->w_layout == KMOE_W_TILED && a->H <= 8192 && a->I <= 8192;
-}
-
 // Whether the routed gate_up GEMM runs on the weight-streaming kernel (and, 4-bit weights with long rows aside, the
 // down GEMM as well).
 bool routed_streams(const kmoe_moe_args* a) {
@@ -168,6 +159,30 @@ bool routed_streams(const kmoe_moe_args* a) {
       return w4_gate_up_streams(a->M * a->K, a->E_global > a->E ? static_cast<int>(rows) : 0, a->E, a->H) &&
              w4_rows_fit_32(a->M, a->H, a->H) && w4_rows_fit_32(static_cast<long long>(a->M) * a->K, a->I, a->I);
   }
+}
+
+// Whether this call may use the side stream: KMOE_FLAG_SIDE_STREAM of the call, unless the environment variable
+// KMOE_SIDE_STREAM (read once) says 0 (never) or 1 (always).
+bool wants_side_stream(const kmoe_moe_args* a) {
+  static const int forced = [] {
+    const char* v = getenv("KMOE_SIDE_STREAM");
+    return (v && v[0]) ? (v[0] != '0' ? 1 : 0) : -1;
+  }();
+  return forced >= 0 ? forced == 1 : (a->flags & KMOE_FLAG_SIDE_STREAM) != 0;
+}
+
+// A shared expert of the routed experts' width runs inside the routed GEMM launches
+// as one more ("tail") expert over rows [P, P+M): no extra launches, and its few
+// workgroups overlap the routed experts' instead of leaving most CUs idle.
+// fp8 on the weight-streaming kernel: the tail's 16-row slices read the shared weights once each, the pass of its own
+// reads them once and costs its launches, unless a side stream hides them. DeepSeek-V3 dims, layer, us, folded / own
+// pass: 23 tokens 949 / 1010, 128 1830 / 1873, 256 1942 / 1951, 288 1979 / 1974, 320 2035 / 2024; own pass on the side
+// stream: 23 tokens 959, 64 1559 (folded 1557), 96 1748 (1754), 128 1822, 256 1895, 320 1983.
+bool fold_shared(const kmoe_moe_args* a) {
+  if (a->I_shared <= 0 || a->I_shared != a->I || a->ws_layout != a->w_layout) return false;
+  if (a->format == KMOE_FMT_INT8) return true;
+  if (a->format != KMOE_FMT_FP8_BLOCK || a->w_layout != KMOE_W_TILED || a->H > 8192 || a->I > 8192) return false;
+  return !routed_streams(a) || a->M <= (wants_side_stream(a) ? 64 : 256);
 }
 
 // One expert-MLP pass (gate_up + SiLU-mul, requantise, down) over `rows` rows in
@@ -415,11 +430,11 @@ extern "C" int kmoe_moe_workspace_layout(const kmoe_moe_args* a, kmoe_moe_layout
 
 namespace {
 
-// A shared expert that cannot ride in the routed launches (another width; the fp8 decode kernels) is a chain of
+// A shared expert that does not ride in the routed launches (another width; larger fp8 decode batches) is a chain of
 // small launches that depends on the layer's input only. It runs on a stream of the library's own, forked from
 // the caller's stream after the first quantisation and joined back before the combine, so that it hides under
-// the routed GEMMs instead of adding its launches' latencies to the layer (DeepSeek-V3 fp8 decode: 85 us of
-// 1.86 ms). Only for calls that ask for it (KMOE_FLAG_SIDE_STREAM): by default every launch goes to the caller's
+// the routed GEMMs instead of adding its launches' latencies to the layer (DeepSeek-V3 fp8, 256 tokens: 56 us of
+// 1.95 ms). Only for calls that ask for it (KMOE_FLAG_SIDE_STREAM): by default every launch goes to the caller's
 // stream. One stream and two events per GPU, created on the first call that wants them and is not being
 // captured (default priority, non-blocking); work of consecutive calls is ordered on it like on any stream.
 struct SideStream {
@@ -430,16 +445,6 @@ struct SideStream {
 constexpr int kSideDevices = 64;
 SideStream g_side[kSideDevices];
 std::mutex g_side_mutex;
-
-// Whether this call may use the side stream: KMOE_FLAG_SIDE_STREAM of the call, unless the environment variable
-// KMOE_SIDE_STREAM (read once) says 0 (never) or 1 (always).
-bool wants_side_stream(const kmoe_moe_args* a) {
-  static const int forced = [] {
-    const char* v = getenv("KMOE_SIDE_STREAM");
-    return (v && v[0]) ? (v[0] != '0' ? 1 : 0) : -1;
-  }();
-  return forced >= 0 ? forced == 1 : (a->flags & KMOE_FLAG_SIDE_STREAM) != 0;
-}
 
 // The side stream of the current device, or NULL: not created yet while the caller's stream is being captured (a
 // capture must not be the first to ask), or the runtime refused.
