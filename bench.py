@@ -403,6 +403,15 @@ def measure(a, workload, shape, label, sl, with_cpu_baseline, exact_steps=True):
     return res
 
 
+def brief(r):
+    """A suite workload's figures for the result line."""
+    return {"tokens_per_s": round(r["value"], 1), "ms_per_step": round(r["ms_per_step"], 5), "dtype": r["dtype"],
+            "tokens": r["config"]["tokens"], "launch": r["config"]["launch"], "bound": r["roofline"]["bound"],
+            "gate_up_ms": round(r["roofline"]["kernel_ms"], 5), "gate_up_hbm_frac": round(r["roofline"]["hbm_frac"], 4),
+            "gate_up_mfma_frac": round(r["roofline"]["mfma_frac"], 4), "layer_hbm_frac": round(r["layer"]["hbm_frac"], 4),
+            "layer_mfma_frac": round(r["layer"]["mfma_frac"], 4)}
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -507,7 +516,9 @@ def main():
                     t.data.zero_()
         results[name] = measure(a, name, shape, label, sl, name == headline and not a.no_cpu_baseline,
                                 exact_steps=name == headline)
-        print(f"bench.py: {name}: {results[name]['ms_per_step']:.4f} ms/step", file=sys.stderr, flush=True)
+        r = results[name]
+        print(f"bench.py: {name}: {r['ms_per_step']:.4f} ms/step " + json.dumps({k: r[k] for k in ("config", "roofline", "layer")}),
+              file=sys.stderr, flush=True)
 
     head = results[headline]
     result = {
@@ -532,10 +543,9 @@ def main():
         if extra in head:
             result[extra] = head[extra]
     if len(results) > 1:
-        result["workloads"] = {
-            n: {"tokens_per_s": r["value"], "ms_per_step": r["ms_per_step"], "dtype": r["dtype"], "config": r["config"],
-                "roofline": r["roofline"], "layer": r["layer"]}
-            for n, r in results.items() if n != headline}
+        # (short: a line of every workload's configuration and stages is longer than what a log keeps of it; they are on
+        # stderr, a line each)
+        result["workloads"] = {n: brief(r) for n, r in results.items() if n != headline}
     print(json.dumps(result))
 
 
