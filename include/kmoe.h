@@ -429,12 +429,15 @@ typedef struct kmoe_gemm_w4_args {
  *   y[r,c] = bf16( sum_k float(a[src(r),k]) * float(bf16((code[e,c,k] - 8) * scale[e,c,k/group])) )
  * i.e. the bf16 grouped GEMM on the weights kmoe_dequant_w4_bf16 would produce, with
  * f32 accumulation on MFMA (compare within tolerance). Two kernels: a weight-streaming
- * one for the decode regime (an expert with more rows than one pass holds streams its
- * weights again) and, from two dozen rows per expert, one on 128-row tiles that shares
- * the unpacking of a weight among the tile's rows; both sum in the same order and give
- * the same bits.
+ * one for the smallest batches (an expert with more rows than one pass holds streams its
+ * weights again) and, from 1 to 5 rows per expert on, one on tiles of 16 to 128 rows that
+ * shares the unpacking of a weight among the tile's rows. The tile kernel and the streaming
+ * kernel's variants 1, 2, 4 sum in the same order and give the same bits; the streaming
+ * launches chosen for variant 0 split K two ways, so a row's last bit may depend on the
+ * batch it is in.
  * Limits: k % 128 == 0, n % 16 == 0 (SwiGLU: n % 32 == 0), tiled weights; the tile
- * kernel needs rows * lda * 2 < 4 GiB (else the streaming kernel serves every size).
+ * kernel needs rows * lda * 2 < 4 GiB and source rows below `rows` (row_src[r] / src_div;
+ * beyond 4 GiB the streaming kernel serves every size, and rows anywhere).
  */
 int kmoe_grouped_gemm_w4a16(const kmoe_gemm_w4_args* args, kmoe_stream_t stream);
 

@@ -49,8 +49,8 @@ def test_apply_monolithic_under_graph_capture():
 @pytest.mark.parametrize("side", [False, True], ids=["one-stream", "side-stream"])
 @pytest.mark.parametrize("quant", ["int8", "fp8"])
 def test_shared_expert_on_the_side_stream_under_graph_capture(quant, side):
-    """A shared expert of another width (int8) and the fp8 decode layer run their shared MLP in launches of its own:
-    on the caller's stream by default, and with KMOE_FLAG_SIDE_STREAM (the method's side_stream) on the library's
+    """A shared expert of another width (int8) runs its MLP in launches of its own, one of the same width (fp8, up to 64
+    tokens) rides in the routed ones: on the caller's stream by default, and with KMOE_FLAG_SIDE_STREAM (the method's side_stream) on the library's
     second stream, forked from and joined into the caller's. Both settings, eager and captured (the fork and join
     become graph edges): same bits every time (int8: the oracle's)."""
     from vllm_kunlun_amd import synth

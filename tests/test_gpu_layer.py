@@ -426,8 +426,10 @@ def test_int8_layer_as_an_expert_parallel_share(M, scoring):
                                    (33, 300, 8), (63, 512, 4), (5, 1000, 16)])
 def test_decode_launches_with_a_column_per_pair(fmt, M, E, K):
     """Batches with fewer routed pairs than experts give the streaming launches a column of workgroups per pair (up to
-    256 pairs): the layer's results, and the sort it leaves, around that switch - a token's result does not depend on
-    the batch it travels in, so each batch is compared with the same tokens inside one that has a column per expert."""
+    256 pairs): the layer's results, and the sort it leaves, around that switch. Each batch is compared with the same
+    tokens inside one that has a column per expert: the same bits in int8, whose sums are exact; in the other formats
+    the two launches may split K differently, which moves a 16-bit result by its rounding (2^-9 of it, and the same
+    again behind the second GEMM: 4e-3)."""
     from vllm_kunlun_amd import synth
     big = M + E // K + 2
     shape = synth.scaled(synth.SHAPES["qwen3-decode"], M=big, H=256, E=E, K=K, I=128, quant=fmt)

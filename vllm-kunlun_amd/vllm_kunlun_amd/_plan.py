@@ -447,7 +447,8 @@ def run_layer(fmt: int, x: torch.Tensor, logits: Optional[torch.Tensor], top_k: 
     workspace). x and logits may come strided and logits in any float type. Filling and checking an argument block
     costs more host time than a decode step takes on the GPU, and a model's step makes the same call per layer again
     and again, so the block is kept: a later call with the same weights and options copies it and fills in the batch
-    (Qwen3 shape, one token: host time per call 55 -> 19 us). What may have changed is compared, not assumed: the
+    (Qwen3 shape, one token: 19 us of host time with the kept block, 27 filling it: a layer's first call, and the first
+    one after any weights were re-arranged or such weights freed). What may have changed is compared, not assumed: the
     tensors' identity, address, shape, type and contiguity, and the state of the weights' re-arrangement."""
     x = x.contiguous()
     if logits is not None:

@@ -47,9 +47,10 @@ def _count_writes(args, at) -> None:
 
 def operator(name: str, mutates_args):
     """Registers a function as torch.ops.<namespace>.<op> with the schema its annotations give. The dispatcher calls it
-    directly, for every device (the bodies refuse what is not on the GPU): 3 us of host time per call where
-    torch.library.custom_op's own wrapping takes 13 to 23, several times what the launch itself costs. Autograd sees
-    what it sees of such an operator: there is no backward, and written arguments count as written."""
+    directly, for every device (the bodies refuse what is not on the GPU): a tenth of the host time of
+    torch.library.custom_op's own wrapping (2.2 us a call against 23 on a slow core, 1.0 on a fast one; counting the
+    writes adds 0.5), which is several times what the launch itself costs. Autograd sees of such an operator what it
+    sees of a wrapped one: there is no backward, and written arguments count as written."""
     namespace, op = name.split("::")
 
     def register(fn):
