@@ -238,6 +238,19 @@ __device__ inline float group_max(float v) {
   return v;
 }
 
+// the same of unsigned numbers: four DPP steps inside the rows of 16 lanes, then exchanges between them
+template <int G>
+__device__ inline uint32_t group_max_u32(uint32_t v) {
+  static_assert(G >= 16, "whole rows of 16 lanes");
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x128, 0xf, 0xf, true)));  // rotated by 8, 4, 2, 1
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x124, 0xf, 0xf, true)));
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x122, 0xf, 0xf, true)));
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x121, 0xf, 0xf, true)));
+#pragma unroll
+  for (int off = 16; off < G; off <<= 1) v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), off, kWave)));
+  return v;
+}
+
 // Butterfly sum: every lane ends with the same bits (each step adds the same
 // two numbers on both sides). Equivalent to the balanced binary tree
 // t[l] = t[l] + t[l + off], off = 32,16,...,1, over the 64 lane values.
