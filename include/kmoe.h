@@ -318,6 +318,33 @@ int kmoe_tile_weights_i8(const int8_t* src, int8_t* dst, int E, int n, int k,
  */
 int kmoe_grouped_gemm_i8(const kmoe_gemm_i8_args* args, kmoe_stream_t stream);
 
+/*
+ * A dense W8A8 Linear with dynamic symmetric activations in one call (quantization/kernels/scale_mm.py:52-90: quantise
+ * per token, then matmul): kmoe_quant_i8_rows_dt and the product above with one matrix, the same bits.
+ *   y[r,c] = round( float(acc) * (x_max[r]/127) * (w_max[c]/127) ),  acc over the codes of x's rows.
+ * lod == NULL: a kernel of tiles that split K over a workgroup's waves, ahead for up to kmoe_linear_i8_split_rows(n, k)
+ * rows (tiled weights; up to 4 rows are quantised in its own launch); any number of rows is computed. Else lod is the row range {0, rows} (device)
+ * and the rows go to kmoe_grouped_gemm_i8 as one expert's.
+ */
+typedef struct kmoe_linear_i8_args {
+  const uint16_t* x;      /* [rows, k] bf16 / half, row stride ld_x, multiple of 8   */
+  int64_t ld_x;
+  const int8_t* w;        /* [n, k]                                                  */
+  const float* w_max;     /* [n] absmax of each output channel                       */
+  const int32_t* lod;
+  uint16_t* y;            /* [rows, n]                                               */
+  int64_t ldy;
+  void* scratch;          /* kmoe_linear_i8_workspace_bytes(rows, k), 256-byte aligned */
+  size_t scratch_bytes;
+  int32_t rows, n, k;
+  int32_t w_layout;       /* KMOE_W_*                                                */
+  int32_t act_dtype;      /* KMOE_DT_* of x and y                                    */
+} kmoe_linear_i8_args;
+
+int kmoe_linear_i8(const kmoe_linear_i8_args* args, kmoe_stream_t stream);
+int kmoe_linear_i8_split_rows(int n, int k);
+size_t kmoe_linear_i8_workspace_bytes(int rows, int k);
+
 typedef struct kmoe_gemm_bf16_args {
   const uint16_t* a;      /* [a_rows, k] bf16 activations, row stride lda (elements) */
   int64_t lda;

@@ -1,4 +1,4 @@
-"""The dense W8A8 linear on the weight-streaming kernel: the launch's slices and channel fragments at their edges, and the
+"""The dense W8A8 linear: the split-K kernel's tiles and channel fragments at their edges, and the
 call kept on the layer following what changes in between."""
 import os
 import sys
@@ -36,6 +36,46 @@ def test_dense_slices(rows, n, k):
     kern, layer, codes, w_max = _linear(n, k, n + k)
     x = (torch.randn(rows, k, generator=torch.Generator().manual_seed(rows)) * 1.5).bfloat16()
     out = kern.apply_weights(layer, x.cuda())
+    xq, x_max = co.quant_i8_rows(bits(x))
+    ref, _ = co.grouped_gemm_i8(xq, x_max, codes.numpy()[None], w_max.numpy()[None], np.array([0, rows], np.int32))
+    assert np.array_equal(bits(out), ref)
+
+
+# up to four rows are quantised by the GEMM's own launch, five are not; one channel fragment per workgroup and two, K up to
+# the most it takes and beyond, rows of zeros and of one tiny value
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("n,k", [(16, 64), (4096, 576), (4112, 640), (80, 8192), (48, 8256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_quantised_in_the_launch(rows, n, k, dtype):
+    from vllm_kunlun_amd import _lib as L
+    kern, layer, codes, w_max = _linear(n, k, n + k)
+    x = (torch.randn(rows, k, generator=torch.Generator().manual_seed(rows)) * 1.5).to(dtype)
+    if rows > 1:
+        x[1] = 0
+        x[rows - 1, k - 1] = 1e-7 if rows != 2 else 0
+    f16 = dtype == torch.float16
+    L.lib.kmoe_trace_kernels(1)
+    out = kern.apply_weights(layer, x.cuda())
+    named = L.lib.kmoe_traced_kernels().decode()
+    L.lib.kmoe_trace_kernels(0)
+    assert ("quantises its rows itself" in named) == (rows <= 4 and k <= 8192), named
+    xq, x_max = co.quant_i8_rows(bits(x), f16=f16)
+    ref, _ = co.grouped_gemm_i8(xq, x_max, codes.numpy()[None], w_max.numpy()[None], np.array([0, rows], np.int32), f16=f16)
+    assert np.array_equal(bits(out), ref)
+
+
+# every tile of the split-K kernel at its remainders (rows split evenly over the tiles, channels past the last fragment)
+@pytest.mark.parametrize("rows,n", [(16, 4112), (23, 8176), (49, 4080), (65, 8176), (127, 8144), (250, 4080), (511, 1552), (512, 48)])
+def test_tiles_of_the_split_kernel(rows, n):
+    from vllm_kunlun_amd import _lib as L
+    k = 1216
+    kern, layer, codes, w_max = _linear(n, k, n)
+    x = (torch.randn(rows, k, generator=torch.Generator().manual_seed(rows)) * 1.5).bfloat16()
+    L.lib.kmoe_trace_kernels(1)
+    out = kern.apply_weights(layer, x.cuda())
+    named = L.lib.kmoe_traced_kernels().decode()
+    L.lib.kmoe_trace_kernels(0)
+    assert "dense_i8_kernel" in named, named
     xq, x_max = co.quant_i8_rows(bits(x))
     ref, _ = co.grouped_gemm_i8(xq, x_max, codes.numpy()[None], w_max.numpy()[None], np.array([0, rows], np.int32))
     assert np.array_equal(bits(out), ref)

@@ -39,6 +39,18 @@ void note_kernel(const char* fmt, ...) {
   g_trace[g_trace_len] = '\0';
 }
 
+int compute_units(int* n_cu) {
+  static int found = 0;
+  if (found == 0) {
+    int dev = 0, count = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || count < 1)
+      return fail(KMOE_ERR_LAUNCH, "cannot query the device");
+    found = count;
+  }
+  *n_cu = found;
+  return KMOE_OK;
+}
+
 int check_launch(const char* what) {
   const hipError_t err = hipGetLastError();
   if (err == hipSuccess) return KMOE_OK;

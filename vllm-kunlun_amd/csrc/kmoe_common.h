@@ -18,6 +18,8 @@ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // ---- error plumbing (host) -------------------------------------------------
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
+// Compute units of the current device (asked for once).
+int compute_units(int* n_cu);
 // The calling thread's record of launched GEMM kernels (kmoe_trace_kernels): a launcher notes the kernel it chose.
 bool tracing_kernels();
 void note_kernel(const char* fmt, ...);
@@ -56,6 +58,8 @@ struct StreamQuant {
   float* amax;
 };
 constexpr int kStreamQuantMaxK = 1024;
+// Dense int8 GEMM of a few rows (a tail expert alone, tiled weights, chunk-major activations); arguments already validated.
+int dense_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream);
 int stream_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream, const StreamScan* scan, const StreamQuant* quant,
                    const StreamSlots* slots);
 // The same kernel on fp8 block-scaled and on 16-bit weights (tiled; row-major activations).

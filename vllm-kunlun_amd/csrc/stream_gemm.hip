@@ -571,25 +571,8 @@ int stream_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s, const StreamScan* 
     KMOE_REQUIRE(a->a_rows <= kStreamScanMaxRows, KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8 (stream): %d tokens", a->a_rows);
     return launch_rows16<Fmt::I8, true, true>(p, s);
   }
-  if (a->variant == 0 && a->rows == 0 && !swiglu) {
-    // A dense matrix (a tail expert alone) has n channels of workgroups and no experts to fill the chip with, so every
-    // launch has its four waves share K. While a CU gets no more than two workgroups, the smallest pieces are ahead:
-    // slices of 16 rows, one channel fragment per wave if that stays within the two, else two fragments. Up to three,
-    // two steps in flight instead of four; beyond (and where the slices would read 160 MiB of weights and more again
-    // from the caches) slices of 32 rows. With the quantiser, weights cold, us, 16 rows x 1 fragment / x 2 / x 2 and two
-    // steps / 32 rows x 2:
-    //   [4096 x 7168]  32 rows 17.0 / 18.1 / 19.8 / 21.6, 64 22.3 / 20.2 / 20.2 / 21.8, 65 - / 22.4 / 20.7 / 21.9, 128 - / 33.1 / 27.4 / 24.5
-    //   [1536 x 7168]  64 rows 14.9 / 16.4 / 18.4 / 20.0, 128 - / 17.8 / 18.7 / 20.4, 256 - / 23.9 / 23.0 / 22.4
-    //   [7168 x 2048]  32 rows 11.9 / 11.5 / 11.7 / 12.8, 33 13.7 / 12.8 / 12.5 / 13.5, 64 15.4 / 14.8 / 13.9 / 13.8
-    //   [8192 x 8192]  33 rows 38.3 / 35.2 / 37.5 / 29.9;  [12288 x 5120] 32 rows 28.4 / 23.1 / 25.4 / 24.1
-    // K split two ways or not at all is slower everywhere, slices of 64 rows where the tile kernel takes over.
-    const int slices = ceil_div(a->tail_rows, 16), groups = slices * ceil_div(a->n, 32);
-    if (slices * ceil_div(a->n, 16) <= 512) return launch_stream<Fmt::I8, 1, 1, false, 4, 4>(p, s);
-    if (groups <= (slices <= 2 ? 768 : 512)) return launch_stream<Fmt::I8, 1, 2, false, 4, 4>(p, s);
-    if (groups <= 768 && static_cast<int64_t>(slices) * a->n * a->k <= (160ll << 20))
-      return launch_stream<Fmt::I8, 1, 2, false, 2, 4>(p, s);
-    return launch_stream<Fmt::I8, 2, 2, false, 2, 4>(p, s);
-  }
+  // a dense matrix: a tail expert alone
+  if (a->variant == 0 && a->rows == 0 && !swiglu) return dense_gemm_i8(a, s);
   // m-fragments per pass from the rows an expert gets under uniform routing
   int mf = a->variant;
   if (mf == 0) {

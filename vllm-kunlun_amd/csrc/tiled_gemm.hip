@@ -1401,11 +1401,7 @@ int tiled_common(const TiledParams& p, int rows, int* n_cu_out, const char* what
                "%s: y must be 16-byte aligned with ldy %% 8 == 0 (ldy=%lld)", what, static_cast<long long>(p.ldy));
   static int n_cu = 0;
   if (n_cu == 0) {
-    int dev = 0;
-    hipDeviceProp_t prop;
-    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess)
-      return fail(KMOE_ERR_LAUNCH, "%s: cannot query the device", what);
-    n_cu = prop.multiProcessorCount;
+    if (int rc = compute_units(&n_cu)) return rc;
     // KMOE_SPARE_CUS=n (read once): the persistent grids are cut for n fewer CUs, which stay free for a kernel that
     // runs beside these launches on another stream (a collective; the clock probe). Multiples of 8 keep the XCDs even.
     if (const char* spare = getenv("KMOE_SPARE_CUS")) {

@@ -45,6 +45,14 @@ class GemmI8Args(C.Structure):
     ]
 
 
+class LinearI8Args(C.Structure):
+    _fields_ = [
+        ("x", C.c_void_p), ("ld_x", C.c_int64), ("w", C.c_void_p), ("w_max", C.c_void_p), ("lod", C.c_void_p),
+        ("y", C.c_void_p), ("ldy", C.c_int64), ("scratch", C.c_void_p), ("scratch_bytes", C.c_size_t),
+        ("rows", C.c_int32), ("n", C.c_int32), ("k", C.c_int32), ("w_layout", C.c_int32), ("act_dtype", C.c_int32),
+    ]
+
+
 class GemmBf16Args(C.Structure):
     _fields_ = [
         ("a", C.c_void_p), ("lda", C.c_int64), ("row_src", C.c_void_p), ("src_div", C.c_int32),
@@ -142,6 +150,9 @@ def _load() -> C.CDLL:
         "kmoe_quant_fp8_group128": (i32, [vp, i64, i32, i32, vp, i64, vp, vp]),
         "kmoe_quant_fp8_group128_dt": (i32, [vp, i64, i32, i32, vp, i64, vp, i32, vp]),
         "kmoe_grouped_gemm_i8": (i32, [C.POINTER(GemmI8Args), vp]),
+        "kmoe_linear_i8": (i32, [C.POINTER(LinearI8Args), vp]),
+        "kmoe_linear_i8_split_rows": (i32, [i32, i32]),
+        "kmoe_linear_i8_workspace_bytes": (sz, [i32, i32]),
         "kmoe_silu_and_mul": (i32, [vp, i64, i32, i32, vp, i64, vp]),
         "kmoe_combine": (i32, [vp, i64, vp, vp, vp, i32, i32, i32, f32, vp, i64, vp, i64, vp]),
         "kmoe_grouped_gemm_bf16": (i32, [C.POINTER(GemmBf16Args), vp]),
@@ -172,6 +183,7 @@ EXPORTS = (
     "kmoe_swigluoai_and_mul", "kmoe_dequant_w4_bf16", "kmoe_dequant_w4", "kmoe_moe_forward_static",
     "kmoe_quant_i8_static", "kmoe_quant_i8_rows_azp", "kmoe_tile_scales_w4", "kmoe_scaled_mm_azp_epilogue", "kmoe_align_local",
     "kmoe_quant_i8_rows_dt", "kmoe_quant_i8_rows_chunked_dt", "kmoe_silu_and_mul_dt", "kmoe_combine_dt", "kmoe_router_gemm",
+    "kmoe_linear_i8", "kmoe_linear_i8_split_rows", "kmoe_linear_i8_workspace_bytes",
     "kmoe_trace_kernels", "kmoe_traced_kernels", "kmoe_silu_table", "kmoe_clock_probe",
 )
 STATIC_WORKSPACE_BYTES = 64 << 20

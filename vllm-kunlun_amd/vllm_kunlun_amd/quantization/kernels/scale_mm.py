@@ -8,10 +8,10 @@ few pieces of that base it relies on (the parameter names and what the base's
 `process_weights_after_loading` leaves behind: the weight as the [k, n] transpose view of its
 [n, k] storage, a per-channel weight scale, no input scale for dynamic quantisation).
 
-Path taken by `apply_weights`: per-token absmax int8 quantisation and the grouped int8 GEMM
-(`kmoe_grouped_gemm_i8`) on the weights re-arranged at load time into the MFMA tiles - for 16 to 256
-rows, by the channels (`_DynamicCall`), as the tail expert of the weight-streaming kernel, beyond as the
-one-expert case of the tile kernel: the same kernels the fused MoE layer runs its shared expert on.
+Path taken by `apply_weights`: per-token absmax int8 quantisation and the int8 GEMM in one library call
+(`kmoe_linear_i8`) on the weights re-arranged at load time into the MFMA tiles - up to a number of rows that
+depends on the matrix (`_DynamicCall`) on a kernel whose waves split K, which quantises up to four rows itself, beyond as the
+one-expert case of the tile kernel the fused MoE layer's prefill batches run on.
 """
 from __future__ import annotations
 
@@ -53,20 +53,15 @@ _NOTHING: dict = {}
 
 
 class _DynamicCall:
-    """Quantisation and GEMM of one Linear with dynamic symmetric activations: the GEMM's argument block with everything
-    but the batch filled in, kept on the layer. A call is two launches on a scratch buffer of the stream (codes, then row
-    maxes) and one allocation, the output (a dense MLP of two such calls and SiLU-mul: 31 us of host time where building
-    the block and looking the parameters up on every call took 65)."""
+    """Quantisation and GEMM of one Linear with dynamic symmetric activations: the argument block of kmoe_linear_i8 with
+    everything but the batch filled in, kept on the layer. A call is one or two launches on a scratch buffer of the stream
+    and one allocation, the output (a dense MLP of two such calls and SiLU-mul: 31 us of host time where building the block
+    and looking the parameters up on every call took 65)."""
 
-    __slots__ = ("args", "n", "k", "device", "scale", "at", "epoch", "stream_max")
+    __slots__ = ("args", "n", "k", "device", "scale", "at", "epoch", "split_max")
 
-    # The weight-streaming kernel (the one the fused MoE layer runs decode batches and its folded shared expert on) gets
-    # the dense matrix as the launch's "tail expert", whose rows it cuts into slices of 16 or 32, each reading the
-    # weights again. It is ahead of the tile kernel while its launch has few workgroups - slices of 32 rows times groups
-    # of 32 channels - and the tile kernel fewer still; both grow with K alike. With the quantiser, weights cold, us:
-    # [4096 x 7168] 128 rows 24.5 against 31.0, 160 27.7 / 31.4, 256 35.6 / 32.0; [1536 x 7168] 256 rows 22.4 / 31.4;
-    # [7168 x 2048] 64 rows 13.8 / 14.3, 65 14.7 / 14.1, 128 17.2 / 14.4; [2048 x 2048] 256 rows 11.8 / 12.6;
-    # [8192 x 8192] 64 rows 31.6 / 36.4, 65 39.0 / 36.0; [24576 x 1536] 32 rows 18.1 / 15.3.
+    # Rows that go to the kernel whose waves split K: kmoe_linear_i8_split_rows knows from the matrix up to where it is
+    # ahead of the tile kernel; at least the rows below, which leave the tile kernel too few workgroups.
     STREAM_MAX_GROUPS, STREAM_MAX_ROWS = 640, 256
 
     @classmethod
@@ -82,11 +77,12 @@ class _DynamicCall:
         self.at = (w.data_ptr(), w_max.data_ptr())
         self.epoch = _plan._layout_epoch
         layout = weight_layout(w)
-        self.stream_max = self._stream_max_rows(self.n) if layout == L.KMOE_W_TILED else 0
-        g = L.GemmI8Args()
+        self.split_max = 0
+        if layout == L.KMOE_W_TILED:
+            self.split_max = max(self._stream_max_rows(self.n), L.lib.kmoe_linear_i8_split_rows(self.n, self.k))
+        g = L.LinearI8Args()
         g.w, g.w_max = self.at
-        g.E, g.n, g.k, g.lda, g.ldy, g.src_div = 1, self.n, self.k, self.k, self.n, 1
-        g.act, g.w_layout = L.KMOE_ACT_NONE, layout
+        g.n, g.k, g.ld_x, g.ldy, g.w_layout = self.n, self.k, self.k, self.n, layout
         self.args = g
 
     @staticmethod
@@ -122,28 +118,18 @@ class _DynamicCall:
             raise RuntimeError(f"kmoe ops run on the GPU only; got a tensor on {x2.device}")
         out = x2.new_empty((M, n))
         if M:
-            codes = -(-M * k // 256) * 256
-            stream = L.raw_stream()
+            need = -(-M * k // 256) * 256 + 4 * M
             if torch._C._cuda_isCurrentStreamCapturing():
-                scratch = torch.empty(codes + 4 * M, dtype=torch.uint8, device=self.device)  # the graph's own
+                scratch = torch.empty(need, dtype=torch.uint8, device=self.device)  # the graph's own
             else:
-                scratch = _plan.WORKSPACE.get(codes + 4 * M, self.device, L.raw_stream(self.device.index))
-            g = L.GemmI8Args.from_buffer_copy(self.args)  # a copy: threads may share the block
-            g.a = x_q = scratch.data_ptr()
-            g.a_max = x_max = x_q + codes
-            g.y, g.act_dtype = out.data_ptr(), dt
-            if M <= self.stream_max:
-                L.check(L.lib.kmoe_quant_i8_rows_chunked_dt(x2.data_ptr(), k, M, k, x_q, x_max, dt, stream))
-                # one routed expert without rows (the launch needs an expert list), the matrix as the tail expert
-                lod = _row_range(self.device, 0)
-                g.a_layout, g.a_rows = L.KMOE_A_CHUNKED, M
-                g.w_tail, g.w_max_tail, g.tail_rows = self.at[0], self.at[1], M
-            else:
-                L.check(L.lib.kmoe_quant_i8_rows_dt(x2.data_ptr(), k, M, k, x_q, k, x_max, dt, stream))
+                scratch = _plan.WORKSPACE.get(need, self.device, L.raw_stream(self.device.index))
+            g = L.LinearI8Args.from_buffer_copy(self.args)  # a copy: threads may share the block
+            g.x, g.rows, g.y, g.act_dtype = x2.data_ptr(), M, out.data_ptr(), dt
+            g.scratch, g.scratch_bytes = scratch.data_ptr(), need
+            if M > self.split_max:
                 lod = _row_range(self.device, M)
-                g.rows = M
-            g.lod = lod.data_ptr()
-            L.check(L.lib.kmoe_grouped_gemm_i8(g, stream))
+                g.lod = lod.data_ptr()
+            L.check(L.lib.kmoe_linear_i8(g, L.raw_stream()))
         return out if flat else out.reshape(*x.shape[:-1], n)
 
 
