@@ -1,0 +1,78 @@
+"""Batches of a few tokens, whose second quantisation, down projection and combine are one launch: the launch's limits (row
+lengths on both sides of its two forms, waves, remainders of the steps in flight), and the calls that stay apart."""
+import os
+import sys
+
+import pytest
+import torch
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), ".."))
+from conftest import rel_l2  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+FUSED = "down projection and combine"
+
+
+def _named(call):
+    from vllm_kunlun_amd import _lib as L
+    L.lib.kmoe_trace_kernels(1)
+    out = call()
+    named = L.lib.kmoe_traced_kernels().decode()
+    L.lib.kmoe_trace_kernels(0)
+    return out, named
+
+
+@pytest.mark.parametrize("fmt,I", [("int8", 64), ("int8", 1024), ("int8", 1088), ("int8", 2048), ("int8", 2112), ("fp8", 128),
+                                   ("fp8", 1152), ("fp8", 2048), ("fp8", 2176), ("none", 96), ("none", 1056), ("none", 2048),
+                                   ("none", 2080), ("w4", 128), ("w4", 1152), ("w4", 2048), ("w4", 2176)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_of_every_length(fmt, I, dtype):
+    """Against the same tokens in a batch with a column per expert: the same bits in int8; elsewhere sums split otherwise
+    move a 16-bit result by its rounding (2^-9 of it, and the same again behind the second GEMM: 4e-3)."""
+    from vllm_kunlun_amd import synth
+    M, E, K = 3, 48, 6
+    big = E // K + 2
+    shape = synth.scaled(synth.SHAPES["qwen3-decode"], M=big, H=256, E=E, K=K, I=I, quant=fmt)
+    sl = synth.make_layer(shape, "cuda", seed=I, dtype=dtype)
+    whole = sl.layer(sl.x, sl.logits)
+    part, named = _named(lambda: sl.layer(sl.x[:M], sl.logits[:M]))
+    padded = -(-I // 64) * 64 if fmt == "int8" else I
+    assert (FUSED in named) == (padded <= 2048), named
+    if fmt == "int8":
+        assert torch.equal(part, whole[:M])
+    else:
+        assert rel_l2(part, whole[:M]) <= 4e-3
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+@pytest.mark.parametrize("K,fused", [(1, True), (15, True), (16, False)])
+@pytest.mark.parametrize("scales", [(1.0, 1.0), (0.5, 0.75)])
+def test_shared_expert_rides_along(fmt, K, fused, scales):
+    """A wave for the shared expert beside one per routed expert, up to 16; with the caller's epilogue (scale of the routed
+    sum, scale of the shared expert's rows)."""
+    from vllm_kunlun_amd import synth
+    M, E = 3, 64
+    big = E // K + 2
+    shape = synth.scaled(synth.SHAPES["dsv3-fp8-decode" if fmt == "fp8" else "dsv3-decode"], M=big, H=384, E=E, K=K, I=256, I_shared=256, n_group=1,
+                         topk_group=1)
+    sl = synth.make_layer(shape, "cuda", seed=K)
+    kw = dict(sl.apply_kwargs(), out_scale=scales[0], shared_scale=scales[1])
+    m = sl.layer.quant_method
+    whole = m.apply_monolithic(sl.layer, sl.x, sl.logits, **kw)
+    part, named = _named(lambda: m.apply_monolithic(sl.layer, sl.x[:M].contiguous(), sl.logits[:M].contiguous(), **kw))
+    assert (FUSED in named) == fused, named
+    if fmt == "int8":
+        assert torch.equal(part, whole[:M])
+    else:
+        assert rel_l2(part, whole[:M]) <= 4e-3
+
+
+def test_batches_that_read_too_much_twice_stay_apart():
+    from vllm_kunlun_amd import synth
+    shape = synth.scaled(synth.SHAPES["qwen3-decode"], M=14, H=2048, E=128, K=8, I=768)
+    sl = synth.make_layer(shape, "cuda", seed=1)
+    for M, fused in ((1, True), (10, True), (14, False)):
+        out, named = _named(lambda: sl.layer(sl.x[:M], sl.logits[:M]))
+        assert (FUSED in named) == fused, (M, named)
+        assert torch.equal(out, sl.layer(sl.x, sl.logits)[:M])

@@ -1,0 +1,232 @@
+// The end of a layer of a few tokens in one launch: second quantisation, down projection and weighted combine.
+//
+// A batch of a few tokens is a chain of launches that each read a few MB: what it costs is launches and dependent memory
+// round trips. In the down projection every routed pair is one row, so a workgroup can own 16 output channels of one TOKEN:
+// a wave per routed expert (and one for the shared expert that rides along) streams that expert's 16 channels over all of K
+// for the pair's row, the rows of the result meet in LDS, and the workgroup adds them up as the combine would - no down
+// rows to write and read back, no launch for them, none for the quantisation in front: each wave quantises its own row
+// while its weights are on their way. An expert that several tokens share is read once per token (from the caches), which
+// is why this stops at a few of them.
+#include "buffer_ops.h"
+#include "formats.h"
+#include "kmoe_common.h"
+#include "quant_body.h"
+#include "w4_unpack.h"
+
+namespace kmoe {
+namespace {
+
+constexpr bool few_wide_i8(Fmt f, int vecs) { return f == Fmt::I8 && vecs > 2; }
+
+// kVecs: vectors of 8 values a lane holds of its row (rows of up to 512 kVecs values)
+template <Fmt FMT, int kVecs>
+__global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 5) void few_down_kernel(const FewDown p) {
+  using acc_t = typename std::conditional<FMT == Fmt::I8, v4i, v4f>::type;
+  constexpr bool W4 = FMT == Fmt::W4 || FMT == Fmt::W4H;
+  constexpr bool QUANT = FMT == Fmt::I8 || FMT == Fmt::F8;
+  constexpr int V = FMT == Fmt::F8 ? 2 : 1;   // 1 KB blocks of weights per step
+  constexpr int AV = W4 ? 4 : V;              // 16-byte vectors of activations per lane and step ...
+  constexpr int kAVStride = W4 ? 16 : 64, kALane = W4 ? 64 : 16, kAStep = W4 ? 256 : 64 * V;
+  constexpr int D = FMT == Fmt::F8 ? 4 : (few_wide_i8(FMT, kVecs) ? 12 : 8);  // steps in flight (a multiple of the four chains)
+  extern __shared__ __attribute__((aligned(16))) int8_t rows_lds[];  // [wave][row bytes + 16]
+  __shared__ float y_lds[kFewMaxWaves][16];
+  __shared__ float w_lds[kFewMaxWaves];
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  const int m = blockIdx.y, col = blockIdx.x * 16;
+  const bool f16 = FMT == Fmt::F16 || FMT == Fmt::W4H || ((FMT == Fmt::I8 || FMT == Fmt::F8) && p.f16 != 0);
+  const bool tail = wave >= p.K;
+  const int pair = m * p.K + wave;
+  const int e = tail ? 0 : p.ids[pair];
+  const int row = tail ? p.M * p.K + m : p.moe_index[pair];
+  const float weight = tail ? 0.0f : p.topk_w[pair];
+
+  // ---- weights: as many steps of the 16 channels as the ring holds ----
+  const int ksteps = p.kbytes / (64 * V);
+  const size_t frag_bytes = static_cast<size_t>(ksteps) * (V * 1024);
+  const int8_t* w_base = (tail ? p.w_tail : p.w + static_cast<size_t>(e) * p.H * p.kbytes) + (col / 16) * frag_bytes;
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w_base), 0, static_cast<int>(frag_bytes), 0x00020000);
+  v4i wreg[D][V];
+  uint16_t gsc[W4 ? D : 1];
+  const uint16_t* sp = W4 ? p.w_scale + (static_cast<size_t>(e) * p.H + col) * p.groups + li * p.s_ch : nullptr;
+  auto load_w = [&](int slot, int s) {
+#pragma unroll
+    for (int v = 0; v < V; ++v) wreg[slot][v] = buffer_load16(wr, lane * 16, static_cast<uint32_t>(s) * (V * 1024) + v * 1024);
+    if constexpr (W4) {
+      const int g32 = 4 * s + lg;  // this lane's 32 values of the step
+      gsc[slot] = sp[(p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / p.gs32) * p.s_g];
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < ksteps) load_w(d, d);
+  float4 wmax = make_float4(0, 0, 0, 0);
+  float wsc = 0.0f;  // F8: lane l holds the block scale of step l
+  if constexpr (FMT == Fmt::I8) wmax = *reinterpret_cast<const float4*>((tail ? p.w_aux_tail : p.w_aux + static_cast<size_t>(e) * p.H) + col + lg * 4);
+  if constexpr (FMT == Fmt::F8)
+    wsc = (tail ? p.w_aux_tail : p.w_aux + static_cast<size_t>(e) * (p.H / 128) * ksteps)[static_cast<size_t>(col / 128) * ksteps + min(lane, ksteps - 1)];
+
+  __builtin_amdgcn_sched_barrier(0);
+  // ---- the row: quantised (the arithmetic of the quantisers' launches, hence their bits) or as it is, into LDS ----
+  const uint4* src = reinterpret_cast<const uint4*>(p.act + static_cast<size_t>(row) * p.I);
+  const int nvec = p.I / 8;
+  Pack8 val[kVecs];
+#pragma unroll
+  for (int i = 0; i < kVecs; ++i) {
+    val[i].v = make_uint4(0, 0, 0, 0);
+    if (lane + i * kWave < nvec) val[i].v = src[lane + i * kWave];
+  }
+  const int row_bytes = p.I * (QUANT ? 1 : 2) + (FMT == Fmt::F8 ? p.I / 32 : 0);  // (F8: and the scales of its groups)
+  int8_t* mine = rows_lds + wave * (row_bytes + 16);
+  [[maybe_unused]] float* scales = reinterpret_cast<float*>(mine + p.I);
+  float amax = 1.0f;
+  if constexpr (FMT == Fmt::I8) {
+    uint32_t mag = 0;
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) mag = max_magnitudes(mag, magnitudes8(val[i]));
+    RowScale s = row_scale_i8(group_max_u32<kWave>(max_of_pair(mag)), f16);
+    if (!s.numbers) {
+      float top = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kVecs; ++i) top = fmaxf(top, amax8(val[i], f16));
+      s.amax = __builtin_bit_cast(float, group_max_u32<kWave>(__builtin_bit_cast(uint32_t, top)));
+      s.inv = s.amax > 0.0f ? 127.0f / s.amax : 0.0f;
+    }
+    amax = s.amax;
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+      const int v = lane + i * kWave;
+      if (v < nvec) {
+        const uint2 codes = quant8_i8_of(val[i], s, f16);
+        *reinterpret_cast<uint2*>(mine + v * 8) = codes;
+        if (blockIdx.x == 0)  // what the quantiser's launch would have left
+          *reinterpret_cast<uint2*>(p.codes + (static_cast<size_t>(v >> 3) * p.rows + row) * 64 + (v & 7) * 8) = codes;
+      }
+    }
+    if (blockIdx.x == 0 && lane == 0) p.code_aux[row] = amax;
+  } else if constexpr (FMT == Fmt::F8) {
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+      const int v = lane + i * kWave;
+      if (v < nvec) {  // (a group's 16 lanes together: nvec is a multiple of 16)
+        float s;
+        const uint2 codes = quant8_fp8(val[i], f16, s);
+        *reinterpret_cast<uint2*>(mine + v * 8) = codes;
+        if (blockIdx.x == 0) *reinterpret_cast<uint2*>(p.codes + static_cast<size_t>(row) * p.I + v * 8) = codes;
+        if ((lane & 15) == 0) {
+          scales[v >> 4] = s;
+          if (blockIdx.x == 0) p.code_aux[static_cast<size_t>(row) * (p.I / 128) + (v >> 4)] = s;
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i)
+      if (lane + i * kWave < nvec) *reinterpret_cast<uint4*>(mine + (lane + i * kWave) * 16) = val[i].v;
+  }
+
+  // ---- product: all 16 rows of the MFMA are this row (its bytes are broadcast from LDS); four chains of sums ----
+  acc_t acc[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) acc[c] = acc_t{0, 0, 0, 0};
+  const int8_t* ap = mine + lg * kALane;
+  for (int i0 = 0; i0 < ksteps; i0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int s = i0 + d;
+      if (s < ksteps) {
+        v4i av[AV];
+#pragma unroll
+        for (int v = 0; v < AV; ++v) av[v] = *reinterpret_cast<const v4i*>(ap + s * kAStep + v * kAVStride);
+        acc_t& sum = acc[d & 3];
+        if constexpr (FMT == Fmt::I8) {
+          sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[d][0], av[0], sum, 0, 0, 0);
+        } else if constexpr (FMT == Fmt::F8) {
+          const float sw = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsc), s));
+          const v4f blk = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+              __builtin_shufflevector(wreg[d][0], wreg[d][V - 1], 0, 1, 2, 3, 4, 5, 6, 7),
+              __builtin_shufflevector(av[0], av[V - 1], 0, 1, 2, 3, 4, 5, 6, 7), (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+          const float sc = scales[s] * sw;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sum[q] = __builtin_fmaf(blk[q], sc, sum[q]);
+        } else if constexpr (W4) {
+          const W4Scale<FMT == Fmt::W4H> sc(gsc[W4 ? d : 0]);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const v4i wv = unpack8(static_cast<uint32_t>(wreg[d][0][t]), sc);
+            if constexpr (FMT == Fmt::W4)
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wv), __builtin_bit_cast(v8bf, av[AV > 1 ? t : 0]), acc[t], 0, 0, 0);
+            else
+              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wv), __builtin_bit_cast(v8h, av[AV > 1 ? t : 0]), acc[t], 0, 0, 0);
+          }
+        } else if constexpr (FMT == Fmt::BF16) {
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wreg[d][0]), __builtin_bit_cast(v8bf, av[0]), sum, 0, 0, 0);
+        } else {
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wreg[d][0]), __builtin_bit_cast(v8h, av[0]), sum, 0, 0, 0);
+        }
+        if (s + D < ksteps) load_w(d, s + D);
+      }
+    }
+  }
+  const acc_t total = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+
+  // ---- 16 channels of the pair's row, rounded as the down launch stores them; lanes 0, 16, 32, 48 hold four each ----
+  if (li == 0) {
+    uint16_t y[4];
+    const float wm[4] = {wmax.x, wmax.y, wmax.z, wmax.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if constexpr (FMT == Fmt::I8) y[q] = f32_to_act((static_cast<float>(total[q]) * (amax / 127.0f)) * (wm[q] / 127.0f), f16);
+      else y[q] = f32_to_act(total[q], f16);
+      y_lds[wave][lg * 4 + q] = act_to_f32(y[q], f16);
+    }
+    *reinterpret_cast<uint2*>(p.down + static_cast<size_t>(row) * p.H + col + lg * 4) =
+        make_uint2(y[0] | (static_cast<uint32_t>(y[1]) << 16), y[2] | (static_cast<uint32_t>(y[3]) << 16));
+    if (lane == 0) w_lds[wave] = weight;
+  }
+  __syncthreads();
+
+  // ---- combine: f32 sum over the token's experts in routing order, one rounding, the caller's epilogue ----
+  if (threadIdx.x < 16) {
+    const int c = threadIdx.x;
+    float sum = 0.0f;
+    for (int k = 0; k < p.K; ++k) sum = __builtin_fmaf(w_lds[k], y_lds[k][c], sum);
+    uint16_t o = f32_to_act(sum, f16);
+    if (p.out_scale != 1.0f) o = f32_to_act(act_to_f32(o, f16) * p.out_scale, f16);
+    if (p.w_tail) {
+      float add = y_lds[p.K][c];
+      if (p.shared_scale != 1.0f) add = act_to_f32(f32_to_act(add * p.shared_scale, f16), f16);
+      o = f32_to_act(act_to_f32(o, f16) + add, f16);
+    }
+    p.out[static_cast<size_t>(m) * p.H + col + c] = o;
+  }
+}
+
+template <Fmt FMT, int kVecs>
+int launch_few_down(const FewDown& p, hipStream_t s) {
+  const int waves = p.K + (p.w_tail ? 1 : 0);
+  const int row_bytes = p.I * (FMT == Fmt::I8 || FMT == Fmt::F8 ? 1 : 2) + (FMT == Fmt::F8 ? p.I / 32 : 0);
+  if (tracing_kernels())
+    note_kernel("few_down_kernel<%s>, %d waves: quantisation, down projection and combine of a token's 16 channels", fmt_name(FMT), waves);
+  hipLaunchKernelGGL((few_down_kernel<FMT, kVecs>), dim3(p.H / 16, p.M), dim3(waves * kWave), static_cast<size_t>(waves) * (row_bytes + 16), s, p);
+  return check_launch("kmoe_moe_forward (down + combine)");
+}
+
+template <Fmt FMT>
+int launch_few_down(const FewDown& p, hipStream_t s) {
+  return p.I <= 1024 ? launch_few_down<FMT, 2>(p, s) : launch_few_down<FMT, 4>(p, s);
+}
+
+}  // namespace
+
+int few_down(const FewDown& p, int format, hipStream_t s) {
+  switch (format) {
+    case KMOE_FMT_INT8: return launch_few_down<Fmt::I8>(p, s);
+    case KMOE_FMT_FP8_BLOCK: return launch_few_down<Fmt::F8>(p, s);
+    case KMOE_FMT_BF16: return p.f16 ? launch_few_down<Fmt::F16>(p, s) : launch_few_down<Fmt::BF16>(p, s);
+    default: return p.f16 ? launch_few_down<Fmt::W4H>(p, s) : launch_few_down<Fmt::W4>(p, s);
+  }
+}
+
+}  // namespace kmoe

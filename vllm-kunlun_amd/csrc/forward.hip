@@ -197,6 +197,24 @@ bool fold_shared(const kmoe_moe_args* a) {
   return !routed_streams(a) || a->M <= (wants_side_stream(a) ? 64 : 256);
 }
 
+// Whether the layer of a few tokens ends in one launch (few_down). It saves a launch or two, 4 to 8 us, and reads the down
+// projection of an expert once per TOKEN that chose it (and of a shared expert that rides along once per token): what is read
+// twice comes from the caches, at about 6 MB a microsecond, and in the formats that are unpacked or scaled in the
+// launch every reading is worked on again. Layer, launches apart / in one, us, and the MB that uniform routing reads again:
+//   Qwen3 dims int8 1 token 23.7 / 18.9 (0), 4 42.5 / 36.6 (4), 8 60.4 / 56.6 (20), 10 64.9 / 62.2 (30), 12 74.4 / 74.0 (43);
+//   bf16 1 token 26.3 / 22.3, 8 89.9 / 88.3 (39), 12 116 / 118 (85); 4-bit 1 token 21.4 / 18.6, 6 39.4 / 37.5 (6), 8 44.2 / 43.7 (10);
+//   DeepSeek-V3 dims int8 1 token 95.3 / 87.5, 2 149.0 / 147.3 (18), 3 193.7 / 198.3 (40); fp8 1 token 95.3 / 88.6, 2 149 / 153 (18);
+//   Kimi-K2 dims 4-bit 1 token 59.6 / 57.4, 2 93.3 / 92.8 (1), 4 160 / 161 (7).
+bool few_down_pays(const kmoe_moe_args* a, bool fold) {
+  if (a->I > kFewMaxI || a->K + (fold ? 1 : 0) > kFewMaxWaves) return false;
+  const double pairs = static_cast<double>(a->M) * a->K;
+  double hit = a->E;
+  for (int m = 0; m < a->M; ++m) hit *= 1.0 - static_cast<double>(a->K) / a->E;
+  const double again = pairs - (a->E - hit) + (fold ? a->M - 1 : 0);
+  const double bytes = static_cast<double>(a->H) * a->I * (a->format == KMOE_FMT_BF16 ? 2.0 : (a->format == KMOE_FMT_W4A16 ? 0.5 : 1.0));
+  return again * bytes <= (a->format == KMOE_FMT_FP8_BLOCK || a->format == KMOE_FMT_W4A16 ? 6e6 : 32e6);
+}
+
 // One expert-MLP pass (gate_up + SiLU-mul, requantise, down) over `rows` rows in
 // the layer's format. `x_rows` is what the first GEMM reads: quantised codes, or
 // the bf16 activations themselves for KMOE_FMT_BF16.
@@ -236,6 +254,7 @@ struct MlpPass {
   const StreamScan* scan;
   const StreamSlots* slots;
   bool quant_in_gemm;  // the down launch quantises its rows itself: no launch between the two GEMMs
+  bool few_down;       // a few tokens: one launch for quantisation, down projection and combine ends the layer
 };
 
 int run_gemm(const MlpPass& m, bool first, kmoe_stream_t stream) {
@@ -363,6 +382,44 @@ int run_gemm(const MlpPass& m, bool first, kmoe_stream_t stream) {
   return grouped_gemm_bf16_checked(&g, stream, first ? m.scan : nullptr, first ? nullptr : m.slots);
 }
 
+// The launch of a few tokens' down projection, combine included; gate_up has left its rows in m.act.
+int run_few_down(const MlpPass& m, const kmoe_moe_args* a, const int32_t* ids, const int32_t* moe_index, const float* topk_w, hipStream_t stream) {
+  FewDown p = {};
+  p.M = a->M;
+  p.K = a->K;
+  p.H = m.H;
+  p.I = m.I;
+  p.kbytes = m.format == KMOE_FMT_BF16 ? 2 * m.I : (m.format == KMOE_FMT_W4A16 ? m.I / 2 : m.I);
+  p.ids = ids;
+  p.moe_index = moe_index;
+  p.topk_w = topk_w;
+  p.act = m.act;
+  p.rows = m.rows + m.tail_rows;
+  p.codes = static_cast<int8_t*>(m.actq);
+  p.code_aux = m.act_aux;
+  p.w = static_cast<const int8_t*>(m.w2);
+  p.w_aux = m.w2_aux;
+  if (m.tail_rows > 0) {
+    p.w_tail = static_cast<const int8_t*>(m.w2_tail);
+    p.w_aux_tail = m.w2_aux_tail;
+  }
+  if (m.format == KMOE_FMT_W4A16) {
+    const bool frag16 = m.scale_layout == KMOE_S_FRAG16;
+    p.w_scale = m.w2_scale;
+    p.groups = m.I / m.group_size;
+    p.s_ch = frag16 ? 1 : p.groups;
+    p.s_g = frag16 ? 16 : 1;
+    p.gs32 = m.group_size / 32;
+    p.gs_shift = (p.gs32 & (p.gs32 - 1)) == 0 ? __builtin_ctz(p.gs32) : -1;
+  }
+  p.down = m.out;
+  p.out_scale = a->out_scale;
+  p.shared_scale = a->shared_scale == 0.0f ? 1.0f : a->shared_scale;
+  p.out = a->out;
+  p.f16 = m.act_dtype == KMOE_DT_F16;
+  return few_down(p, m.format, stream);
+}
+
 template <class Mark>
 int run_mlp(const MlpPass& m, kmoe_stream_t stream, Mark&& mark) {
   int rc;
@@ -373,6 +430,10 @@ int run_mlp(const MlpPass& m, kmoe_stream_t stream, Mark&& mark) {
   if (rc) return rc;
   mark(KMOE_STAGE_GEMM1, 1);
   mark(KMOE_STAGE_QUANT2, 0);
+  if (m.few_down) {  // (the rest is the caller's)
+    mark(KMOE_STAGE_QUANT2, 1);
+    return KMOE_OK;
+  }
   if (m.format == KMOE_FMT_INT8 && m.quant_in_gemm) {
     // (the down launch does it)
   } else if (m.format == KMOE_FMT_INT8) {
@@ -657,6 +718,7 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
     routed.w2_aux_tail = a->ws2_max;
     routed.tail_rows = M;
   }
+  routed.few_down = per_pair && (a->I_shared == 0 || fold) && few_down_pays(a, fold);
   // 7. dense shared expert on all M rows: the grouped GEMM with a single expert whose lod is {0, M}. With a side
   // stream it is enqueued there BEFORE the routed pass (it reads x / its codes only) and joined after it.
   const uint16_t* shared_out = fold ? routed.out + static_cast<size_t>(P) * H : nullptr;
@@ -678,6 +740,7 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
     sh.scan = nullptr;
     sh.slots = nullptr;
     sh.quant_in_gemm = false;
+    sh.few_down = false;
     sh.src_div = 1;
     sh.w13 = a->ws13;
     sh.w2 = a->ws2;
@@ -741,6 +804,17 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
     if (rc) return rc;
   }
   mark(KMOE_STAGE_SHARED, 1);
+  if (routed.few_down) {  // 8. with the down projection
+    mark(KMOE_STAGE_GEMM2, 0);
+    if (tracing_kernels()) note_kernel("[down, routed experts]");
+    rc = run_few_down(routed, a, topk_ids, moe_index, topk_w, as_stream(stream));
+    mark(KMOE_STAGE_GEMM2, 1);
+    mark(KMOE_STAGE_SHARED, 0);
+    mark(KMOE_STAGE_SHARED, 1);
+    mark(KMOE_STAGE_COMBINE, 0);
+    mark(KMOE_STAGE_COMBINE, 1);
+    return rc;
+  }
   // 8. weighted combine (+ caller epilogue)
   mark(KMOE_STAGE_COMBINE, 0);
   // shared_scale == 0 (a zeroed field) means 1

@@ -58,6 +58,30 @@ struct StreamQuant {
   float* amax;
 };
 constexpr int kStreamQuantMaxK = 1024;
+// Second quantisation, down projection and combine of a layer of a few tokens in one launch (few_tokens.hip). Rows of
+// act: routed pairs by moe_index, then (w_tail) the M rows of a shared expert of the same width. Tiled weights.
+struct FewDown {
+  int32_t M, K, H, I;
+  int32_t kbytes;  // bytes of a weight row
+  const int32_t *ids, *moe_index;
+  const float* topk_w;
+  const uint16_t* act;  // [rows, I]
+  int32_t rows;
+  int8_t* codes;  // what the quantiser's launch would leave: codes (int8: chunk-major) and row maxes / group scales
+  float* code_aux;
+  const int8_t* w;
+  const float* w_aux;
+  const int8_t* w_tail;
+  const float* w_aux_tail;
+  const uint16_t* w_scale;  // 4-bit: as in StreamParams
+  int32_t groups, s_ch, s_g, gs32, gs_shift;
+  uint16_t* down;  // [rows, H]
+  float out_scale, shared_scale;
+  uint16_t* out;  // [M, H]
+  int32_t f16;
+};
+constexpr int kFewMaxI = 2048, kFewMaxWaves = 16;  // K, and one for the shared expert
+int few_down(const FewDown& p, int format, hipStream_t stream);
 // Dense int8 GEMM of a few rows (a tail expert alone, tiled weights, chunk-major activations); arguments already validated.
 int dense_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream);
 int stream_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream, const StreamScan* scan, const StreamQuant* quant,

@@ -159,20 +159,10 @@ __device__ inline uint32_t pack2_e4m3fn(float a, float b) {
 // 448; all combinations were compared, down to x = 2^-24 of the maximum), as long as neither s nor 1 / s nor the remainder
 // leaves the normal range: other groups, and those with a NaN, divide. No value beyond 448 reaches the conversion by more
 // than the quotient's rounding, so the quick way needs no clamp.
-__device__ inline void quant_fp8_group128_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
-                                               uint8_t* __restrict__ q, int64_t ld_q, float* __restrict__ scale,
-                                               int block, bool f16) {
-  const int groups_per_row = C / 128;
-  const long long total = static_cast<long long>(R) * groups_per_row;
-  const long long gid = static_cast<long long>(block) * 16 + (threadIdx.x >> 4);
-  const int t = threadIdx.x & 15;
-  if (gid >= total) return;  // (a group's 16 lanes leave together)
-  const int r = static_cast<int>(gid / groups_per_row);
-  const int g = static_cast<int>(gid - static_cast<long long>(r) * groups_per_row);
-  Pack8 val;
-  val.v = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(r) * ld_x + g * 128 + t * 8);
+// quant8_fp8: the codes of this lane's 8 values of a group (the group's 16 lanes call together), its scale in `s`.
+__device__ inline uint2 quant8_fp8(const Pack8& val, bool f16, float& s) {
   const uint32_t m = group_max_u32<16>(max_of_pair(magnitudes8(val)));
-  float s = act_to_f32(static_cast<uint16_t>(m), f16) / 448.0f;
+  s = act_to_f32(static_cast<uint16_t>(m), f16) / 448.0f;
   uint32_t w[2] = {0, 0};
   if (s >= 0x1p-60f && s <= 0x1p60f) {  // (false for a NaN)
     const float y = 1.0f / s;
@@ -201,7 +191,23 @@ __device__ inline void quant_fp8_group128_body(const uint16_t* __restrict__ x, i
     w[0] = pack2_e4m3fn(f[0], f[1]) | (pack2_e4m3fn(f[2], f[3]) << 16);
     w[1] = pack2_e4m3fn(f[4], f[5]) | (pack2_e4m3fn(f[6], f[7]) << 16);
   }
-  *reinterpret_cast<uint2*>(q + static_cast<size_t>(r) * ld_q + g * 128 + t * 8) = make_uint2(w[0], w[1]);
+  return make_uint2(w[0], w[1]);
+}
+
+__device__ inline void quant_fp8_group128_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
+                                               uint8_t* __restrict__ q, int64_t ld_q, float* __restrict__ scale,
+                                               int block, bool f16) {
+  const int groups_per_row = C / 128;
+  const long long total = static_cast<long long>(R) * groups_per_row;
+  const long long gid = static_cast<long long>(block) * 16 + (threadIdx.x >> 4);
+  const int t = threadIdx.x & 15;
+  if (gid >= total) return;  // (a group's 16 lanes leave together)
+  const int r = static_cast<int>(gid / groups_per_row);
+  const int g = static_cast<int>(gid - static_cast<long long>(r) * groups_per_row);
+  Pack8 val;
+  val.v = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(r) * ld_x + g * 128 + t * 8);
+  float s;
+  *reinterpret_cast<uint2*>(q + static_cast<size_t>(r) * ld_q + g * 128 + t * 8) = quant8_fp8(val, f16, s);
   if (t == 0) scale[static_cast<size_t>(r) * groups_per_row + g] = s;
 }
 
