@@ -76,3 +76,69 @@ def test_batches_that_read_too_much_twice_stay_apart():
         out, named = _named(lambda: sl.layer(sl.x[:M], sl.logits[:M]))
         assert (FUSED in named) == fused, (M, named)
         assert torch.equal(out, sl.layer(sl.x, sl.logits)[:M])
+
+
+ROUTED = "routing, quantisation, sort and gate_up"
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8", "none", "w4"])
+@pytest.mark.parametrize("M,K,E", [(1, 1, 2), (1, 16, 17), (2, 8, 128), (3, 6, 129), (4, 16, 65), (4, 8, 256), (4, 3, 257), (3, 8, 512),
+                                   (4, 4, 513), (5, 4, 128)])
+@pytest.mark.parametrize("H", [128, 640])
+def test_routing_in_the_gate_up_launch(fmt, M, K, E, H):
+    """Up to four tokens are routed, quantised and sorted by the gate_up launch: experts on both sides of a wave's 64 slots,
+    tokens that share experts, parts of K that are empty for some waves. Against the same tokens in a batch with a
+    column per expert."""
+    from vllm_kunlun_amd import synth
+    shape = synth.scaled(synth.SHAPES["qwen3-decode"], M=max(M + 1, E // K + 2), H=H, E=E, K=K, I=128, quant=fmt)
+    sl = synth.make_layer(shape, "cuda", seed=M * E + K)
+    sl.logits[:M, :K // 2] += 4.0  # shared experts
+    whole = sl.layer(sl.x, sl.logits)
+    part, named = _named(lambda: sl.layer(sl.x[:M], sl.logits[:M]))
+    assert (ROUTED in named) == (M <= 4 and M * K < E and E <= 512), named
+    if fmt == "int8":
+        assert torch.equal(part, whole[:M])
+    else:
+        assert rel_l2(part, whole[:M]) <= 4e-3
+
+
+@pytest.mark.parametrize("fmt,M,fused", [("int8", 3, True), ("int8", 4, False), ("fp8", 3, True), ("fp8", 4, False), ("none", 1, True),
+                                         ("none", 2, False), ("w4", 1, True), ("w4", 2, False)])
+def test_long_rows_stay_apart(fmt, M, fused):
+    """The gate_up launch holds all its rows in LDS: where they are too long for five workgroups a CU, routing is a launch of
+    its own again; a shared expert's column has a row per token."""
+    from vllm_kunlun_amd import synth
+    E, K = 32, 4
+    shared = fmt in ("int8", "fp8")
+    base = "qwen3-decode" if not shared else ("dsv3-fp8-decode" if fmt == "fp8" else "dsv3-decode")
+    over = dict(I_shared=128, n_group=4, topk_group=2) if shared else {}
+    shape = synth.scaled(synth.SHAPES[base], M=E // K + 2, H=7168, E=E, K=K, I=128, quant=fmt, **over)
+    sl = synth.make_layer(shape, "cuda", seed=3)
+    sl.logits[:M, :K] += 6.0  # every token on the same experts
+    kw = sl.apply_kwargs()
+    m = sl.layer.quant_method
+    run = (lambda x, l: m.apply_monolithic(sl.layer, x, l, **kw)) if shared else (lambda x, l: sl.layer(x, l))  # noqa: E731
+    whole = run(sl.x, sl.logits)
+    part, named = _named(lambda: run(sl.x[:M].contiguous(), sl.logits[:M].contiguous()))
+    assert (ROUTED in named) == fused, named
+    if fmt == "int8":
+        assert torch.equal(part, whole[:M])
+    else:
+        assert rel_l2(part, whole[:M]) <= 4e-3
+
+
+@pytest.mark.parametrize("kind", ["nan", "inf", "zero", "tiny"])
+def test_rows_that_are_not_all_numbers(kind):
+    """int8: a token whose row has a NaN, an infinity or nothing to scale by gets the codes the quantiser gives it, and the
+    other tokens keep their results."""
+    from vllm_kunlun_amd import synth
+    sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], M=10, H=640, E=64, K=8, I=128), "cuda", seed=9)
+    value = {"nan": float("nan"), "inf": float("inf"), "zero": 0.0, "tiny": 1e-40}[kind]
+    if kind in ("zero", "tiny"):
+        sl.x[1] = 0
+    sl.x[1, 639] = value
+    whole = sl.layer(sl.x, sl.logits)
+    part, named = _named(lambda: sl.layer(sl.x[:3], sl.logits[:3]))
+    assert ROUTED in named
+    assert torch.equal(part.view(torch.int16)[[0, 2]], whole[:3].view(torch.int16)[[0, 2]])
+    assert torch.equal(torch.isnan(part[1]), torch.isnan(whole[1])) and torch.equal(part[1].nan_to_num(), whole[1].nan_to_num())

@@ -1,4 +1,6 @@
-// The end of a layer of a few tokens in one launch: second quantisation, down projection and weighted combine.
+// The layer of a few tokens in two launches.
+//
+// few_down_kernel: second quantisation, down projection and weighted combine.
 //
 // A batch of a few tokens is a chain of launches that each read a few MB: what it costs is launches and dependent memory
 // round trips. In the down projection every routed pair is one row, so a workgroup can own 16 output channels of one TOKEN:
@@ -7,10 +9,13 @@
 // rows to write and read back, no launch for them, none for the quantisation in front: each wave quantises its own row
 // while its weights are on their way. An expert that several tokens share is read once per token (from the caches), which
 // is why this stops at a few of them.
+#include <algorithm>
+
 #include "buffer_ops.h"
 #include "formats.h"
 #include "kmoe_common.h"
 #include "quant_body.h"
+#include "routing_body.h"
 #include "w4_unpack.h"
 
 namespace kmoe {
@@ -218,6 +223,295 @@ int launch_few_down(const FewDown& p, hipStream_t s) {
   return p.I <= 1024 ? launch_few_down<FMT, 2>(p, s) : launch_few_down<FMT, 4>(p, s);
 }
 
+
+// few_gate_up_kernel (up to kFewRouted tokens): routing, first quantisation, sort, gate_up projection and SiLU-mul.
+//
+// A workgroup serves 16 output channels of one routed PAIR's expert (columns of the grid: pairs, then the shared expert if
+// one rides along, then one that leaves the routing and the sort for whoever reads them). It routes every token itself, a
+// wave each, from the logits: a dozen cache lines and a microsecond against a launch of four before this one. The first
+// pair that chose an expert serves all its rows; the other columns leave. The four waves split K; each quantises its own
+// part of the rows while its weights are on their way (int8: one exchange of the maxima), and the codes wait in LDS.
+template <Fmt FMT, int SLOTS, bool SIGMOID>
+__global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up_kernel(const FewGateUp p) {
+  using acc_t = typename std::conditional<FMT == Fmt::I8, v4i, v4f>::type;
+  constexpr bool W4 = FMT == Fmt::W4 || FMT == Fmt::W4H;
+  constexpr bool QUANT = FMT == Fmt::I8 || FMT == Fmt::F8;
+  constexpr int V = FMT == Fmt::F8 ? 2 : 1;
+  constexpr int AV = W4 ? 4 : V;
+  constexpr int kAVStride = W4 ? 16 : 64, kALane = W4 ? 64 : 16, kAStep = W4 ? 256 : 64 * V;
+  constexpr int D = FMT == Fmt::F8 || W4 ? 2 : (FMT == Fmt::I8 ? 4 : 8);
+  constexpr int kStepValues = W4 ? 128 : (QUANT ? 64 * V : 32);
+  extern __shared__ __attribute__((aligned(16))) int8_t lds[];  // sigmoid routing: [4][E] floats; then [M][row bytes + 16]
+  __shared__ float tw_lds[kFewRouted * kFewMaxWaves];
+  __shared__ int32_t id_lds[kFewRouted * kFewMaxWaves];
+  __shared__ uint32_t max_lds[kFewRouted][4];
+  __shared__ acc_t red[3][2][kWave];
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  const bool f16 = FMT == Fmt::F16 || FMT == Fmt::W4H || (QUANT && p.f16 != 0);
+  const RouteArgs& r = p.route;
+  const int P = r.M * r.K;
+  const int column = blockIdx.y;
+  const bool tail = p.w_tail != nullptr && column == P;
+  const bool publish = column == P + (p.w_tail ? 1 : 0);
+  if (publish && blockIdx.x != 0) return;
+
+  // ---- which expert, which rows ----
+  int e = 0, rows = 0, begin = 0;
+  int my_pair = 0;  // lane l: the pair of row l % 16 of this column
+  if (!tail) {
+    if constexpr (SIGMOID)
+      sigmoid_group_topk_body<SLOTS>(r.logits, r.bias, r.M, r.E, r.K, r.n_group, r.topk_group, r.scale, tw_lds, id_lds, reinterpret_cast<float*>(lds), 0);
+    else
+      softmax_topk_body<SLOTS>(r.logits, r.M, r.E, r.K, r.renorm, tw_lds, id_lds, 0);
+    __syncthreads();
+    const int id = lane < P ? id_lds[lane] : 0x7fffffff;  // (P <= 64)
+    if (publish) {
+      if (threadIdx.x < P) {
+        r.topk_w[threadIdx.x] = tw_lds[threadIdx.x];
+        r.topk_ids[threadIdx.x] = id;
+        int below = 0, before = 0, equal = 0;  // pairs of lower experts; earlier pairs and all pairs of this one
+        for (int j = 0; j < P; ++j) {
+          below += id_lds[j] < id;
+          before += id_lds[j] == id && j < static_cast<int>(threadIdx.x);
+          equal += id_lds[j] == id;
+        }
+        p.sort.moe_index[threadIdx.x] = below + before;
+        p.sort.sorted_src[below + before] = threadIdx.x;
+        p.sort.slot_rows[threadIdx.x] = make_int2(below, before == 0 ? below + equal : below);  // (as scan_pairs leaves them)
+      }
+      for (int x = threadIdx.x; x < r.E; x += 4 * kWave) {
+        int below = 0, equal = 0;
+        for (int j = 0; j < P; ++j) {
+          below += id_lds[j] < x;
+          equal += id_lds[j] == x;
+        }
+        p.sort.lod[x] = below;
+        p.sort.expert_m[x] = equal;
+        if (x == r.E - 1) p.sort.lod[r.E] = below + equal;
+      }
+      return;
+    }
+    e = __builtin_amdgcn_readfirstlane(id_lds[column]);
+    const uint64_t mine = __ballot(id == e);
+    if (__builtin_ctzll(mine) != column) return;  // an earlier pair's column serves this expert
+    rows = __builtin_popcountll(mine);            // (a token picks an expert once: at most kFewRouted)
+    begin = __builtin_popcountll(__ballot(id < e));
+    uint64_t left = mine;
+#pragma unroll
+    for (int i = 0; i < kFewRouted; ++i) {
+      if (left != 0 && li == i) my_pair = __builtin_ctzll(left);
+      left &= left - 1;
+    }
+  } else {
+    rows = r.M;
+    begin = P;
+  }
+  const int my_token = tail ? min(li, rows - 1) : my_pair / r.K;  // of row li (rows past the last: any token)
+
+  // ---- weights of the gate and the up fragment: this wave's part of K, as many steps as the ring holds ----
+  const int col = blockIdx.x * 16;
+  const int ksteps = p.kbytes / (64 * V);
+  const int kb0 = ksteps * wave / 4, klen = ksteps * (wave + 1) / 4 - kb0;
+  const size_t frag_bytes = static_cast<size_t>(ksteps) * (V * 1024);
+  const int8_t* w_base = tail ? p.w_tail : p.w + static_cast<size_t>(e) * (2 * p.I) * p.kbytes;
+  __amdgpu_buffer_rsrc_t wr[2];
+  const uint16_t* sp[2];
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    const int c = f * p.I + col;
+    wr[f] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w_base + (c / 16) * frag_bytes), 0, static_cast<int>(frag_bytes), 0x00020000);
+    sp[f] = W4 ? p.w_scale + (static_cast<size_t>(e) * (2 * p.I) + c) * p.groups + li * p.s_ch : nullptr;
+  }
+  v4i wreg[D][2][V];
+  uint16_t gsc[W4 ? D : 1][2];
+  auto load_w = [&](int slot, int i) {
+    const uint32_t s = kb0 + i;
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+#pragma unroll
+      for (int v = 0; v < V; ++v) wreg[slot][f][v] = buffer_load16(wr[f], lane * 16, s * (V * 1024) + v * 1024);
+      if constexpr (W4) {
+        const int g32 = 4 * s + lg;
+        gsc[slot][f] = sp[f][(p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / p.gs32) * p.s_g];
+      }
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < klen) load_w(d, d);
+  float4 wmax[2];
+  float wsc[2];  // F8: lane l holds the block scale of step kb0 + l
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    const int c = f * p.I + col;
+    if constexpr (FMT == Fmt::I8)
+      wmax[f] = *reinterpret_cast<const float4*>((tail ? p.w_aux_tail : p.w_aux + static_cast<size_t>(e) * (2 * p.I)) + c + lg * 4);
+    if constexpr (FMT == Fmt::F8)
+      wsc[f] = (tail ? p.w_aux_tail : p.w_aux + static_cast<size_t>(e) * (2 * p.I / 128) * ksteps)[static_cast<size_t>(c / 128) * ksteps + min(kb0 + lane, ksteps - 1)];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- the rows: this wave's part of K, quantised (the quantisers' arithmetic) or as it is, into LDS ----
+  const int row_bytes = p.H * (QUANT ? 1 : 2) + (FMT == Fmt::F8 ? p.H / 32 : 0);
+  const int pitch = row_bytes + 16;
+  int8_t* rows_lds = lds;
+  const int v0 = kb0 * (kStepValues / 8), nvec = klen * (kStepValues / 8);  // vectors of 8 values
+  float amax = 1.0f;
+  for (int i = 0; i < rows; ++i) {
+    const int token = __builtin_amdgcn_readlane(my_token, i);
+    const uint4* src = reinterpret_cast<const uint4*>(p.x + static_cast<size_t>(token) * p.H) + v0;
+    int8_t* dst = rows_lds + i * pitch;
+    if constexpr (FMT == Fmt::I8) {
+      uint32_t mag = 0;
+      for (int v = lane; v < nvec; v += kWave) {
+        Pack8 val;
+        val.v = src[v];
+        mag = max_magnitudes(mag, magnitudes8(val));
+      }
+      mag = group_max_u32<kWave>(max_of_pair(mag));
+      if (lane == 0) max_lds[i][wave] = mag;
+    } else if constexpr (FMT == Fmt::F8) {
+      for (int v = lane; v < nvec; v += kWave) {
+        Pack8 val;
+        val.v = src[v];
+        float s;
+        *reinterpret_cast<uint2*>(dst + (v0 + v) * 8) = quant8_fp8(val, f16, s);
+        if ((lane & 15) == 0) reinterpret_cast<float*>(dst + p.H)[(v0 + v) >> 4] = s;
+      }
+    } else {
+      for (int v = lane; v < nvec; v += kWave) *reinterpret_cast<uint4*>(dst + (v0 + v) * 16) = src[v];
+    }
+  }
+  if constexpr (FMT == Fmt::I8) {
+    __syncthreads();
+    for (int i = 0; i < rows; ++i) {
+      const int token = __builtin_amdgcn_readlane(my_token, i);
+      const uint4* src = reinterpret_cast<const uint4*>(p.x + static_cast<size_t>(token) * p.H) + v0;
+      int8_t* dst = rows_lds + i * pitch;
+      RowScale s = row_scale_i8(max(max(max_lds[i][0], max_lds[i][1]), max(max_lds[i][2], max_lds[i][3])), f16);
+      if (!s.numbers) {  // (the same for the whole workgroup) every wave goes over the whole row: rare
+        float top = 0.0f;
+        for (int v = lane; v < p.H / 8; v += kWave) {
+          Pack8 val;
+          val.v = (src - v0)[v];
+          top = fmaxf(top, amax8(val, f16));
+        }
+        s.amax = __builtin_bit_cast(float, group_max_u32<kWave>(__builtin_bit_cast(uint32_t, top)));
+        s.inv = s.amax > 0.0f ? 127.0f / s.amax : 0.0f;
+      }
+      if (li == i) amax = s.amax;
+      for (int v = lane; v < nvec; v += kWave) {
+        Pack8 val;
+        val.v = src[v];
+        *reinterpret_cast<uint2*>(dst + (v0 + v) * 8) = quant8_i8_of(val, s, f16);
+      }
+    }
+  }
+
+  // ---- product ----
+  acc_t acc[2][2];
+#pragma unroll
+  for (int f = 0; f < 2; ++f)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[f][c] = acc_t{0, 0, 0, 0};
+  const int8_t* arow = rows_lds + min(li, rows - 1) * pitch;
+  const int8_t* ap = arow + lg * kALane + kb0 * kAStep;
+  for (int i0 = 0; i0 < klen; i0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int i = i0 + d;
+      if (i < klen) {
+        v4i av[AV];
+#pragma unroll
+        for (int v = 0; v < AV; ++v) av[v] = *reinterpret_cast<const v4i*>(ap + i * kAStep + v * kAVStride);
+        float sa = 1.0f;
+        if constexpr (FMT == Fmt::F8) sa = reinterpret_cast<const float*>(arow + p.H)[kb0 + i];
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+          acc_t& sum = acc[f][d & 1];
+          if constexpr (FMT == Fmt::I8) {
+            sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[d][f][0], av[0], sum, 0, 0, 0);
+          } else if constexpr (FMT == Fmt::F8) {
+            const float sw = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wsc[f]), i));
+            const v4f blk = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                __builtin_shufflevector(wreg[d][f][0], wreg[d][f][V - 1], 0, 1, 2, 3, 4, 5, 6, 7),
+                __builtin_shufflevector(av[0], av[V - 1], 0, 1, 2, 3, 4, 5, 6, 7), (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+            const float sc = sa * sw;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sum[q] = __builtin_fmaf(blk[q], sc, sum[q]);
+          } else if constexpr (W4) {
+            const W4Scale<FMT == Fmt::W4H> sc(gsc[W4 ? d : 0][f]);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const v4i wv = unpack8(static_cast<uint32_t>(wreg[d][f][0][t]), sc);
+              const v4i a = av[AV > 1 ? t : 0];
+              if constexpr (FMT == Fmt::W4)
+                acc[f][t & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wv), __builtin_bit_cast(v8bf, a), acc[f][t & 1], 0, 0, 0);
+              else
+                acc[f][t & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wv), __builtin_bit_cast(v8h, a), acc[f][t & 1], 0, 0, 0);
+            }
+          } else if constexpr (FMT == Fmt::BF16) {
+            sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wreg[d][f][0]), __builtin_bit_cast(v8bf, av[0]), sum, 0, 0, 0);
+          } else {
+            sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, wreg[d][f][0]), __builtin_bit_cast(v8h, av[0]), sum, 0, 0, 0);
+          }
+        }
+        if (i + D < klen) load_w(d, i + D);
+      }
+    }
+  }
+
+  // ---- the four parts of K meet; SiLU-mul ----
+  acc_t sum[2];
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    sum[f] = acc[f][0] + acc[f][1];
+    if (wave > 0) red[wave - 1][f][lane] = sum[f];
+  }
+  __syncthreads();
+  if (wave == 0 && li < rows) {
+    uint16_t g[4], u[4];
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+#pragma unroll
+      for (int part = 0; part < 3; ++part) sum[f] += red[part][f][lane];
+      const float wm[4] = {wmax[f].x, wmax[f].y, wmax[f].z, wmax[f].w};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        uint16_t& o = f == 0 ? g[q] : u[q];
+        if constexpr (FMT == Fmt::I8) o = f32_to_act((static_cast<float>(sum[f][q]) * (amax / 127.0f)) * (wm[q] / 127.0f), f16);
+        else o = f32_to_act(sum[f][q], f16);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) g[q] = f32_to_act(silu_hw(act_to_f32(g[q], f16)) * act_to_f32(u[q], f16), f16);
+    *reinterpret_cast<uint2*>(p.act + static_cast<size_t>(begin + li) * p.I + col + lg * 4) =
+        make_uint2(g[0] | (static_cast<uint32_t>(g[1]) << 16), g[2] | (static_cast<uint32_t>(g[3]) << 16));
+  }
+}
+
+template <Fmt FMT, int SLOTS, bool SIGMOID>
+int launch_few_gate_up(const FewGateUp& p, hipStream_t s) {
+  const int H = p.H;
+  const int row_bytes = H * (FMT == Fmt::I8 || FMT == Fmt::F8 ? 1 : 2) + (FMT == Fmt::F8 ? H / 32 : 0);
+  // LDS: routing's copy of the scores, then the rows in its place
+  const size_t bytes = std::max(static_cast<size_t>(p.route.M) * (row_bytes + 16), SIGMOID ? sizeof(float) * 4 * p.route.E : 0);
+  if (tracing_kernels())
+    note_kernel("few_gate_up_kernel<%s>: routing, quantisation, sort and gate_up of a pair's 16 channels", fmt_name(FMT));
+  hipLaunchKernelGGL((few_gate_up_kernel<FMT, SLOTS, SIGMOID>), dim3(p.I / 16, p.route.M * p.route.K + (p.w_tail ? 1 : 0) + 1), dim3(4 * kWave), bytes, s, p);
+  return check_launch("kmoe_moe_forward (routing + gate_up)");
+}
+
+template <Fmt FMT>
+int launch_few_gate_up(const FewGateUp& p, bool sigmoid, hipStream_t s) {
+  const int slots = ceil_div(p.route.E, kWave);
+  if (slots <= 2) return sigmoid ? launch_few_gate_up<FMT, 2, true>(p, s) : launch_few_gate_up<FMT, 2, false>(p, s);
+  if (slots <= 4) return sigmoid ? launch_few_gate_up<FMT, 4, true>(p, s) : launch_few_gate_up<FMT, 4, false>(p, s);
+  return sigmoid ? launch_few_gate_up<FMT, 8, true>(p, s) : launch_few_gate_up<FMT, 8, false>(p, s);
+}
+
 }  // namespace
 
 int few_down(const FewDown& p, int format, hipStream_t s) {
@@ -226,6 +520,15 @@ int few_down(const FewDown& p, int format, hipStream_t s) {
     case KMOE_FMT_FP8_BLOCK: return launch_few_down<Fmt::F8>(p, s);
     case KMOE_FMT_BF16: return p.f16 ? launch_few_down<Fmt::F16>(p, s) : launch_few_down<Fmt::BF16>(p, s);
     default: return p.f16 ? launch_few_down<Fmt::W4H>(p, s) : launch_few_down<Fmt::W4>(p, s);
+  }
+}
+
+int few_gate_up(const FewGateUp& p, int format, bool sigmoid, hipStream_t s) {
+  switch (format) {
+    case KMOE_FMT_INT8: return launch_few_gate_up<Fmt::I8>(p, sigmoid, s);
+    case KMOE_FMT_FP8_BLOCK: return launch_few_gate_up<Fmt::F8>(p, sigmoid, s);
+    case KMOE_FMT_BF16: return p.f16 ? launch_few_gate_up<Fmt::F16>(p, sigmoid, s) : launch_few_gate_up<Fmt::BF16>(p, sigmoid, s);
+    default: return p.f16 ? launch_few_gate_up<Fmt::W4H>(p, sigmoid, s) : launch_few_gate_up<Fmt::W4>(p, sigmoid, s);
   }
 }
 

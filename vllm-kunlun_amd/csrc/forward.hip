@@ -207,6 +207,10 @@ bool fold_shared(const kmoe_moe_args* a) {
 //   Kimi-K2 dims 4-bit 1 token 59.6 / 57.4, 2 93.3 / 92.8 (1), 4 160 / 161 (7).
 bool few_down_pays(const kmoe_moe_args* a, bool fold) {
   if (a->I > kFewMaxI || a->K + (fold ? 1 : 0) > kFewMaxWaves) return false;
+  // (what the GEMM launches refuse stays theirs to refuse)
+  for (const void* t : {static_cast<const void*>(a->w2), static_cast<const void*>(a->w2_max), static_cast<const void*>(a->w2_scale),
+                        static_cast<const void*>(a->ws2), static_cast<const void*>(a->ws2_max)})
+    if (reinterpret_cast<uintptr_t>(t) & 15) return false;
   const double pairs = static_cast<double>(a->M) * a->K;
   double hit = a->E;
   for (int m = 0; m < a->M; ++m) hit *= 1.0 - static_cast<double>(a->K) / a->E;
@@ -214,6 +218,28 @@ bool few_down_pays(const kmoe_moe_args* a, bool fold) {
   const double bytes = static_cast<double>(a->H) * a->I * (a->format == KMOE_FMT_BF16 ? 2.0 : (a->format == KMOE_FMT_W4A16 ? 0.5 : 1.0));
   return again * bytes <= (a->format == KMOE_FMT_FP8_BLOCK || a->format == KMOE_FMT_W4A16 ? 6e6 : 32e6);
 }
+
+// Whether such a layer also begins in one launch (few_gate_up): up to kFewRouted tokens, so that routing is a wave each,
+// whose rows leave room for five workgroups in a CU's LDS - fewer, and the launch no longer fills the chip at once (Kimi-K2
+// dims, 4-bit, 1 token 57.1 -> 52.6 us, 2 tokens, three workgroups, 92.7 -> 98.9). Layer, us, apart / in one launch: Qwen3 dims int8
+// 1 token 18.9 / 16.4, 4 37.0 / 32.2, bf16 1 22.0 / 20.4, 4-bit 1 18.4 / 15.5, 4 27.2 / 24.7; DeepSeek-V3 dims int8 1 87.7 /
+// 78.5, with the gate 96.6 / 87.6, fp8 1 88.7 / 84.
+bool few_gate_up_takes(const kmoe_moe_args* a) {
+  if (a->M > kFewRouted || a->M * a->K > kWave || a->E > 8 * kWave) return false;
+  const long long row = bf16_activations(a->format) ? 2ll * a->H : a->H + a->H / 32;
+  if (a->M * (row + 16) > 25 * 1024) return false;
+  for (const void* t : {static_cast<const void*>(a->x), static_cast<const void*>(a->w13), static_cast<const void*>(a->w13_max),
+                        static_cast<const void*>(a->w13_scale), static_cast<const void*>(a->ws13), static_cast<const void*>(a->ws13_max)})
+    if (reinterpret_cast<uintptr_t>(t) & 15) return false;
+  return true;
+}
+
+// What a layer whose gate_up launch routes its tokens itself hands to it.
+struct FewRouted {
+  RouteArgs route;
+  bool sigmoid;
+  const uint16_t* x;
+};
 
 // One expert-MLP pass (gate_up + SiLU-mul, requantise, down) over `rows` rows in
 // the layer's format. `x_rows` is what the first GEMM reads: quantised codes, or
@@ -254,6 +280,7 @@ struct MlpPass {
   const StreamScan* scan;
   const StreamSlots* slots;
   bool quant_in_gemm;  // the down launch quantises its rows itself: no launch between the two GEMMs
+  const FewRouted* first;  // a few tokens: the gate_up launch routes, quantises and sorts (scan: where it leaves the sort)
   bool few_down;       // a few tokens: one launch for quantisation, down projection and combine ends the layer
 };
 
@@ -382,6 +409,18 @@ int run_gemm(const MlpPass& m, bool first, kmoe_stream_t stream) {
   return grouped_gemm_bf16_checked(&g, stream, first ? m.scan : nullptr, first ? nullptr : m.slots);
 }
 
+// Group scales of packed 4-bit weights, as the decode kernels address them.
+template <class P>
+void set_group_scales(P* p, const uint16_t* scale, int k, int group_size, int layout) {
+  const bool frag16 = layout == KMOE_S_FRAG16;
+  p->w_scale = scale;
+  p->groups = k / group_size;
+  p->s_ch = frag16 ? 1 : p->groups;
+  p->s_g = frag16 ? 16 : 1;
+  p->gs32 = group_size / 32;
+  p->gs_shift = (p->gs32 & (p->gs32 - 1)) == 0 ? __builtin_ctz(p->gs32) : -1;
+}
+
 // The launch of a few tokens' down projection, combine included; gate_up has left its rows in m.act.
 int run_few_down(const MlpPass& m, const kmoe_moe_args* a, const int32_t* ids, const int32_t* moe_index, const float* topk_w, hipStream_t stream) {
   FewDown p = {};
@@ -403,15 +442,7 @@ int run_few_down(const MlpPass& m, const kmoe_moe_args* a, const int32_t* ids, c
     p.w_tail = static_cast<const int8_t*>(m.w2_tail);
     p.w_aux_tail = m.w2_aux_tail;
   }
-  if (m.format == KMOE_FMT_W4A16) {
-    const bool frag16 = m.scale_layout == KMOE_S_FRAG16;
-    p.w_scale = m.w2_scale;
-    p.groups = m.I / m.group_size;
-    p.s_ch = frag16 ? 1 : p.groups;
-    p.s_g = frag16 ? 16 : 1;
-    p.gs32 = m.group_size / 32;
-    p.gs_shift = (p.gs32 & (p.gs32 - 1)) == 0 ? __builtin_ctz(p.gs32) : -1;
-  }
+  if (m.format == KMOE_FMT_W4A16) set_group_scales(&p, m.w2_scale, m.I, m.group_size, m.scale_layout);
   p.down = m.out;
   p.out_scale = a->out_scale;
   p.shared_scale = a->shared_scale == 0.0f ? 1.0f : a->shared_scale;
@@ -420,13 +451,34 @@ int run_few_down(const MlpPass& m, const kmoe_moe_args* a, const int32_t* ids, c
   return few_down(p, m.format, stream);
 }
 
+// The launch that routes up to kFewRouted tokens and runs their gate_up projection.
+int run_few_gate_up(const MlpPass& m, hipStream_t stream) {
+  FewGateUp p = {};
+  p.route = m.first->route;
+  p.H = m.H;
+  p.I = m.I;
+  p.kbytes = m.format == KMOE_FMT_BF16 ? 2 * m.H : (m.format == KMOE_FMT_W4A16 ? m.H / 2 : m.H);
+  p.x = m.first->x;
+  p.w = static_cast<const int8_t*>(m.w13);
+  p.w_aux = m.w13_aux;
+  if (m.tail_rows > 0) {
+    p.w_tail = static_cast<const int8_t*>(m.w13_tail);
+    p.w_aux_tail = m.w13_aux_tail;
+  }
+  if (m.format == KMOE_FMT_W4A16) set_group_scales(&p, m.w13_scale, m.H, m.group_size, m.scale_layout);
+  p.sort = *m.scan;
+  p.act = m.act;
+  p.f16 = m.act_dtype == KMOE_DT_F16;
+  return few_gate_up(p, m.format, m.first->sigmoid, stream);
+}
+
 template <class Mark>
 int run_mlp(const MlpPass& m, kmoe_stream_t stream, Mark&& mark) {
   int rc;
   const char* whose = m.row_src || m.scan ? "routed experts" : "shared expert";
   mark(KMOE_STAGE_GEMM1, 0);
   if (tracing_kernels()) note_kernel("[gate_up, %s]", whose);
-  rc = run_gemm(m, true, stream);
+  rc = m.first ? run_few_gate_up(m, as_stream(stream)) : run_gemm(m, true, stream);
   if (rc) return rc;
   mark(KMOE_STAGE_GEMM1, 1);
   mark(KMOE_STAGE_QUANT2, 0);
@@ -621,19 +673,25 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
     if (rc) return rc;
   }
   // 1. routing; for the quantised formats together with step 3 (independent work, one launch)
-  const RouteArgs route{logits, a->bias, M, Eg, K, a->renormalize, a->n_group, a->topk_group, a->routed_scale, topk_w, topk_ids};
-  rc = route_and_quantise(route, a->scoring == KMOE_SCORE_SIGMOID, a->format, a->x, H, at(L.xq),
-                          static_cast<float*>(at(L.xmax)), stream_mode, f16, &quant_done, as_stream(stream));
+  const bool scan_in_gemm = routed_streams(a) && Eg == E && a->first_expert == 0 && P <= kStreamScanMaxPairs &&
+                            M <= kStreamScanMaxRows && scan_allowed();
+  // Fewer pairs than experts: a column of workgroups per pair instead of per expert.
+  const bool per_pair = scan_in_gemm && P < E && P <= kStreamSlotMaxPairs;
+  const bool fold = fold_shared(a);
+  const bool few_down = per_pair && (a->I_shared == 0 || fold) && few_down_pays(a, fold);
+  const bool few_routed = per_pair && (a->I_shared == 0 || fold) && few_gate_up_takes(a);
+  RouteArgs route{logits, a->bias, M, Eg, K, a->renormalize, a->n_group, a->topk_group, a->routed_scale, topk_w, topk_ids};
+  if (few_routed)
+    rc = check_route(&route, a->scoring == KMOE_SCORE_SIGMOID);  // (the gate_up launch does it, and steps 2 and 3)
+  else
+    rc = route_and_quantise(route, a->scoring == KMOE_SCORE_SIGMOID, a->format, a->x, H, at(L.xq),
+                            static_cast<float*>(at(L.xmax)), stream_mode, f16, &quant_done, as_stream(stream));
   if (rc) return rc;
   mark(KMOE_STAGE_ROUTING, 1);
   // 2. stable sort of the routed pairs by expert. On the weight-streaming path (a few rows per expert) the gate_up
   // launch does it in its prologue and writes the same four arrays: one launch and its round trips less
   // (Qwen3 decode: 4.8 us of 125). Not for an expert-parallel share (pairs of other ranks' experts get no row).
   mark(KMOE_STAGE_ALIGN, 0);
-  const bool scan_in_gemm = routed_streams(a) && Eg == E && a->first_expert == 0 && P <= kStreamScanMaxPairs &&
-                            M <= kStreamScanMaxRows && scan_allowed();
-  // Fewer pairs than experts: a column of workgroups per pair instead of per expert.
-  const bool per_pair = scan_in_gemm && P < E && P <= kStreamSlotMaxPairs;
   int2* slot_rows = per_pair ? static_cast<int2*>(at(L.align_ws)) : nullptr;
   const StreamScan scan{topk_ids, P, lod, static_cast<int32_t*>(at(L.expert_m)), moe_index, sorted_src, slot_rows};
   const StreamSlots slots{topk_ids, slot_rows, P};
@@ -648,6 +706,7 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   const void* x_rows = a->x;
   if (quant_done) {
     x_rows = at(L.xq);
+  } else if (few_routed) {
   } else if (a->format == KMOE_FMT_INT8) {
     rc = stream_mode ? kmoe_quant_i8_rows_chunked_dt(a->x, H, M, H, static_cast<int8_t*>(at(L.xq)),
                                                      static_cast<float*>(at(L.xmax)), a->act_dtype, stream)
@@ -710,7 +769,6 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   if (a->format == KMOE_FMT_FP8_BLOCK && a->w_layout == KMOE_W_TILED && (local_pairs(a) + E - 1) / E > 10 &&
       (tv == 5 || tv == 6 || tv == 8 || (tv >= 11 && tv <= 14) || (tv >= 17 && tv <= 19)))
     routed.variant = tv;
-  const bool fold = fold_shared(a);
   if (fold) {
     routed.w13_tail = a->ws13;
     routed.w2_tail = a->ws2;
@@ -718,7 +776,9 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
     routed.w2_aux_tail = a->ws2_max;
     routed.tail_rows = M;
   }
-  routed.few_down = per_pair && (a->I_shared == 0 || fold) && few_down_pays(a, fold);
+  const FewRouted first{route, a->scoring == KMOE_SCORE_SIGMOID, a->x};
+  routed.first = few_routed ? &first : nullptr;
+  routed.few_down = few_down;
   // 7. dense shared expert on all M rows: the grouped GEMM with a single expert whose lod is {0, M}. With a side
   // stream it is enqueued there BEFORE the routed pass (it reads x / its codes only) and joined after it.
   const uint16_t* shared_out = fold ? routed.out + static_cast<size_t>(P) * H : nullptr;
@@ -740,6 +800,7 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
     sh.scan = nullptr;
     sh.slots = nullptr;
     sh.quant_in_gemm = false;
+    sh.first = nullptr;
     sh.few_down = false;
     sh.src_div = 1;
     sh.w13 = a->ws13;

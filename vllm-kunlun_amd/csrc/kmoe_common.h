@@ -138,6 +138,26 @@ struct RouteArgs {
   float* topk_w;
   int32_t* topk_ids;
 };
+// Routing, first quantisation, sort and gate_up projection of a layer of up to kFewRouted tokens and 64 pairs in one launch
+// (few_tokens.hip); leaves topk_w / topk_ids, what the sort would leave, and act.
+struct FewGateUp {
+  RouteArgs route;
+  int32_t H, I, kbytes;
+  const uint16_t* x;  // [M, H]
+  const int8_t* w;    // [E, 2 I, H] tiled
+  const float* w_aux;
+  const int8_t* w_tail;
+  const float* w_aux_tail;
+  const uint16_t* w_scale;  // 4-bit: as in StreamParams
+  int32_t groups, s_ch, s_g, gs32, gs_shift;
+  StreamScan sort;  // what the sort would leave, slot_rows too (ids and n_pairs are not looked at)
+  uint16_t* act;  // [P (+ M), I]
+  int32_t f16;
+};
+constexpr int kFewRouted = 4;
+int few_gate_up(const FewGateUp& p, int format, bool sigmoid, hipStream_t stream);
+// The checks of the routing arguments (and n_group <= 1 made one group).
+int check_route(RouteArgs* r, bool sigmoid);
 // Routing of M tokens and, for KMOE_FMT_INT8 / _FP8_BLOCK where the kernel takes the row length, the quantisation of
 // x [M,H] in the same launch (*quantised says whether it was). M >= 1.
 int route_and_quantise(RouteArgs r, bool sigmoid, int format, const uint16_t* x, int H, void* xq, float* x_aux,

@@ -76,9 +76,8 @@ void launch_e(const RouteArgs& r, const QuantArgs& q, Quant kind, hipStream_t s)
 
 }  // namespace
 
-int route_and_quantise(RouteArgs r, bool sigmoid, int format, const uint16_t* x, int H, void* xq, float* x_aux,
-                       bool chunked, bool f16, bool* quantised, hipStream_t s) {
-  *quantised = false;
+int check_route(RouteArgs* route, bool sigmoid) {
+  RouteArgs& r = *route;
   KMOE_REQUIRE(r.E >= 1 && r.E <= kMaxSlots * kWave && r.K >= 1 && r.K <= r.E && r.K <= kWave, KMOE_ERR_SHAPE,
                "routing: E=%d K=%d", r.E, r.K);
   if (sigmoid) {
@@ -95,6 +94,13 @@ int route_and_quantise(RouteArgs r, bool sigmoid, int format, const uint16_t* x,
                    "routing: K=%d exceeds the %d experts of the kept groups", r.K, r.topk_group * (r.E / r.n_group));
     }
   }
+  return KMOE_OK;
+}
+
+int route_and_quantise(RouteArgs r, bool sigmoid, int format, const uint16_t* x, int H, void* xq, float* x_aux,
+                       bool chunked, bool f16, bool* quantised, hipStream_t s) {
+  *quantised = false;
+  if (int rc = check_route(&r, sigmoid)) return rc;
   Quant kind = Quant::None;
   if (format == KMOE_FMT_INT8 && H % 16 == 0 && H <= 256 * 8 * 4)  // wider rows: a launch of their own
     kind = H <= 64 * 8 * 4 ? Quant::I8Wave : Quant::I8Block;
