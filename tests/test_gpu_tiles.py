@@ -123,3 +123,49 @@ def test_packed_weights_on_rows_far_apart(variant, act, gather):
     got = y.float()
     per_row = (got - ref).norm(dim=1) / ref.norm(dim=1).clamp(min=1e-6)
     assert not got.isnan().any() and float(per_row.max()) <= 2e-2
+
+
+@pytest.mark.parametrize("variant", [0, 18, 19, 20])  # the height the sizes choose; 192, 128 and 160 rows
+@pytest.mark.parametrize("blocks", [3, 4, 5, 9])  # row scales travel four blocks at a time: too few, one group, a rest
+@pytest.mark.parametrize("act,dtype", [(0, torch.float16), (0, torch.bfloat16), (1, torch.bfloat16)])
+@pytest.mark.parametrize("tail", [0, 161])
+def test_block_fp8_wide_tiles(variant, blocks, act, dtype, tail):
+    """fp8 with 128-wide block scales: the wide tiles at the edges of their heights, rows gathered, with and without a
+    tail expert. The products are exact and summed in float32: what is left without SiLU is the rounding of the result,
+    half a unit of bfloat16's eight bits (2**-8). With it, a gate or up value whose float32 sums lie on both sides of a tie is rounded to
+    neighbours, a whole unit (2 * 2**-8) for each of the two; one large value can carry a row of 128 results."""
+    from vllm_kunlun_amd import _lib as L
+    gen = torch.Generator().manual_seed(100 * blocks + tail)
+    counts = ROWS + [159, 160, 161, 319, 321, 384, 385]
+    E, rows, n, k = len(counts), sum(counts), 384 - 128 * act, 128 * blocks
+    n_out = n // 2 if act else n
+    fp8 = torch.float8_e4m3fn
+    a = torch.randn(rows + tail, k, generator=gen).to(fp8).cuda()
+    a_scale = (torch.rand(rows + tail, blocks, generator=gen) + 0.5).cuda()
+    w = torch.randn(E + 1, n, k, generator=gen).to(fp8).cuda()
+    w_scale = (torch.rand(E + 1, n // 128, blocks, generator=gen) + 0.5).cuda()
+    tiled = torch.empty_like(w)
+    L.check(L.lib.kmoe_tile_weights_i8(w.data_ptr(), tiled.data_ptr(), E + 1, n, k, L.stream()))
+    src = torch.randperm(rows, generator=gen).cuda()
+    dsrc, lod = src.int(), torch.tensor([0] + counts).cumsum(0).int().cuda()
+    y = torch.full((rows + tail, n_out), float("nan"), dtype=dtype, device="cuda")
+    g = L.GemmFp8Args()
+    g.a, g.lda, g.a_scale, g.row_src, g.src_div = a.data_ptr(), k, a_scale.data_ptr(), dsrc.data_ptr(), 1
+    g.w, g.w_scale, g.w_layout, g.lod = tiled.data_ptr(), w_scale.data_ptr(), L.KMOE_W_TILED, lod.data_ptr()
+    g.E, g.n, g.k, g.rows = E, n, k, rows
+    g.y, g.ldy, g.act, g.variant, g.act_dtype = y.data_ptr(), n_out, act, variant, L.act_dtype(y, "test")
+    if tail:
+        g.w_tail, g.w_scale_tail = tiled[E].data_ptr(), w_scale[E].data_ptr()
+        g.tail_row0, g.tail_rows, g.tail_src0 = rows, tail, rows
+    L.check(L.lib.kmoe_grouped_gemm_fp8_block(g, L.stream()))
+    a_full = a.float() * a_scale.repeat_interleave(128, 1)
+    w_full = w.float() * w_scale.repeat_interleave(128, 1).repeat_interleave(128, 2)
+    parts = [a_full[src[lo:lo + c]] @ w_full[e].T for e, (c, lo) in enumerate(zip(counts, lod.tolist()))]
+    ref = torch.cat(parts + [a_full[rows:] @ w_full[E].T])
+    if act:
+        gate, up = (t.to(dtype).float() for t in ref.split(n_out, 1))
+        ref = torch.nn.functional.silu(gate) * up
+    got = y.float()
+    assert not got.isnan().any()
+    per_row = (got - ref).norm(dim=1) / ref.norm(dim=1).clamp(min=1e-6)
+    assert float(per_row.max()) <= (5 if act else 1) * 2 ** -8

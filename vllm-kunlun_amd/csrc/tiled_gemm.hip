@@ -4,13 +4,14 @@
 // Two workgroup shapes. Four waves on a 128-row x 256-channel tile (64-, 96-row forms for few rows per
 // expert), each wave owning 64 channels of all the rows (8 x 4 accumulator fragments = 128 registers), two
 // workgroups per CU: one workgroup's waits, barriers and VALU-heavy epilogue run under the other's MFMAs.
-// And, int8 with more than 72 rows per expert: EIGHT waves side by side along the channels (WN = 8) on a
-// 128-, 192- or 256-row x 256-channel tile, each wave owning 32 channels of all the rows, one workgroup
-// per CU, a deeper weight ring, and row fragments past an expert's last row skipped (see tiled_gemm_i8).
+// And, int8 with more than 72 rows per expert, fp8 with more than 76 or 44 (see tiled_gemm_fp8): EIGHT waves side by side
+// along the channels (WN = 8) on a 128-, 160-, 192- or 256-row x 256-channel tile, each wave owning 32 channels of all the
+// rows, one workgroup per CU, a deeper weight ring, and row fragments past an expert's last row skipped (see tiled_gemm_i8).
 //   activations: int8 / bf16: asynchronous copies global -> LDS (rows gathered through the
 //                sort), 128 bytes of K per row and chunk, three chunks ahead into a ring of
 //                four chunk buffers, swizzled so that fragment reads are conflict-free without
-//                padding; no register holds them. fp8: through registers into two padded
+//                padding; no register holds them; the wide tiles of fp8 likewise, a row's scales of four
+//                chunks at a time. fp8 in four waves: through registers into two padded
 //                buffers (pitch 160 B), one chunk ahead, with the row scales of the chunk.
 //                Every A fragment read from LDS feeds 4 MFMAs.
 //   weights:     straight from L2 into registers, 1 KB of consecutive bytes per
@@ -264,10 +265,11 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
   // F8: weight block scales of the tile [parity][wave][fragment][k block], and the row scales
   // of the chunk in each activation buffer
   __shared__ float wsc_lds[F8 ? 2 : 1][F8 ? kWN * NF * kMaxKBlocks : 4];
-  // (register path: every thread stores, rows repeat - no branch in the loop; asynchronous path: a ring like the
-  // chunks', each wave copying 64 row scales per chunk, waves past the tile's rows repeating earlier ones)
-  static_assert(!(F8 && ADMA) || kTM % kWave == 0, "row scales are copied 64 at a time");
-  __shared__ float asc_lds[F8 ? (ADMA ? kStagesA : 2) : 1][F8 ? (ADMA ? kTM : kThreads) : 4];
+  // (register path: every thread stores, rows repeat - no branch in the loop; asynchronous path: four chunks' scales of a
+  // row at a time, two groups of chunks in turn, each wave copying 64 rows; waves past the tile's rows copy one row's
+  // scales into the last 64 slots, which nobody reads)
+  constexpr int kScaleSlots = (kTM + kWave - 1) / kWave * kWave;
+  __shared__ __attribute__((aligned(16))) float asc_lds[F8 ? (ADMA ? 8 * kScaleSlots + 4 * kWave : 2 * kThreads) : 4];
   extern __shared__ int dyn_lds[];
   const int n_exp = p.E + (p.w_tail ? 1 : 0);
   int* row_lo = dyn_lds;               // [E + 1]: lod
@@ -477,9 +479,11 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
     if constexpr (!ADMA) {
 #pragma unroll
       for (int i = 0; i < kNA; ++i) *reinterpret_cast<v4i*>(&lds_a[buf][a_lds[i]]) = areg[i];
-      if constexpr (F8) asc_lds[buf][threadIdx.x] = asc_reg;
+      if constexpr (F8) asc_lds[buf * kThreads + threadIdx.x] = asc_reg;
     }
   };
+  // F8, ADMA: the first of the four chunks whose scales travel together (the last four of a row at its end)
+  auto scale_group = [&](int chunk) { return max(0, min(chunk & ~3, kblocks - 4)); };
   // ADMA: requests chunk `chunk` of the tile into ring buffer `stage` (4 copies per wave)
   auto dma_a = [&](int chunk, int stage) {
     if constexpr (ADMA) {
@@ -487,16 +491,20 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
 #pragma unroll
       for (int i = 0; i < kNA; ++i)
         buffer_load16_to_lds(a_rsrc, (lds_ptr_t)&lds_a[stage][(wave_id * kNA + i) * 1024], aoff[i], kc);
+      // The row scales travel the same way, with the first of four chunks (stage 0): lane l of wave w brings four scales of
+      // tile row 64 w + l. Every lane of such a copy is a cache line of its own: one per chunk and by every wave, whether the
+      // tile had rows for it or not, they were half of all the lines the loop asked for, and no removal of MFMAs, scaling or
+      // LDS reads made the launch faster (64 experts of [4096 x 7168], 94 rows each, 128-row tile: 391 us; copied by the
+      // waves with rows only 353; four chunks at a time as well 346).
       if constexpr (F8) {
-        // the chunk's row scales travel the same way: lane l of wave w brings the scale of tile row (64 w + l) % kTM
-        const uint32_t kb = static_cast<uint32_t>(min(chunk, last_chunk));
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(p.a_max), (lds_ptr_t)&asc_lds[stage][(wave_id * kWave) % kTM], 4,
-                                                 (static_cast<uint32_t>(my_srow) * static_cast<uint32_t>(kblocks) + kb) * 4u,
-                                                 0, 0, 0);
+        const int scale_slot = wave_id * kWave < kScaleSlots ? ((chunk >> 2) & 1) * 4 * kScaleSlots + 4 * wave_id * kWave : 8 * kScaleSlots;
+        if (stage == 0)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(p.a_max), (lds_ptr_t)&asc_lds[scale_slot], 16,
+                                                   (static_cast<uint32_t>(my_srow) * static_cast<uint32_t>(kblocks) + static_cast<uint32_t>(scale_group(chunk))) * 4u,
+                                                   0, 0, 0);
       }
     }
   };
-  constexpr int kND = kNA + ((F8 && ADMA) ? 1 : 0);  // copies per chunk and wave
   // one MFMA step: 8 A fragments from LDS, each against the 4 weight fragments of the slot
   auto mfma_row = [&](const v4i(&wcur)[kNF], const v4i& af, int mf, int t) {
     if constexpr (M32) {
@@ -743,7 +751,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       const uint32_t a_lo = fa[0] + (kFarStages ? buf * kStageBytes : 0);
       const uint32_t a_hi = fa[1] + (kFarStages ? buf * kStageBytes : 0);
       const uint32_t sc_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-          (lds_ptr_t)&asc_lds[buf][wave_m * 16 * kMF + li]));
+          (lds_ptr_t)&asc_lds[((chunk >> 2) & 1) * 4 * kScaleSlots + 4 * (wave_m * 16 * kMF + li) + chunk - scale_group(chunk)]));
       const uint32_t wsc_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
           (lds_ptr_t)&wsc_lds[parity][wave * kNF * kMaxKBlocks + chunk]));
       static_assert(kNF == 2, "the asynchronous fp8 path is written for two channel fragments a wave");
@@ -759,7 +767,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
         constexpr int n = decltype(n_tag)::value;
         if constexpr (n < kMF) {
           if constexpr (n + 1 < kMF) {
-            f8_request<kImm + (n + 1) * 16 * kChunk, (n + 1) * 64>(lo[(n + 1) & 1], hi[(n + 1) & 1], sar[(n + 1) & 1], a_lo, a_hi,
+            f8_request<kImm + (n + 1) * 16 * kChunk, (n + 1) * 256>(lo[(n + 1) & 1], hi[(n + 1) & 1], sar[(n + 1) & 1], a_lo, a_hi,
                                                                   sc_addr);
             f8_wait<3>(lo[n & 1], hi[n & 1], sar[n & 1], swc[0], swc[1]);
           } else {
@@ -816,7 +824,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       v8i av;
       av.lo = *reinterpret_cast<const v4i*>(&lds_a[buf][row * kPitchT + lg * 16]);
       av.hi = *reinterpret_cast<const v4i*>(&lds_a[buf][row * kPitchT + 64 + lg * 16]);
-      const float sa = asc_lds[buf][row];
+      const float sa = asc_lds[buf * kThreads + row];
 #pragma unroll
       for (int f = 0; f < kNF; ++f) {
         v8i wv;
@@ -965,7 +973,10 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
 #pragma unroll
     for (int i = 0; i < kNA; ++i)
       aoff[i] = static_cast<uint32_t>(src_row(t, t.row0 + a_row(i), rs[i])) * static_cast<uint32_t>(p.lda) + a_col;  // < 4 GiB: host-checked
-    if constexpr (F8) my_srow = src_row(t, t.row0 + scale_row, rs_scale);
+    if constexpr (F8) {
+      my_srow = src_row(t, t.row0 + scale_row, rs_scale);
+      if (ADMA && wave_id * kWave >= kScaleSlots) my_srow = __builtin_amdgcn_readfirstlane(my_srow);  // (see dma_a)
+    }
     load_a(0);
     dma_a(0, 0);
     dma_a(1, 1);
@@ -1119,12 +1130,12 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       pace_poll(std::integral_constant<int, h & 1>{});
       __builtin_amdgcn_sched_barrier(0);
       store_a(buf ^ 1);
-      // ADMA: the 12 loads above (and the two polls) may still be in flight, everything older has landed - among
+      // ADMA: the loads above (and the two polls) may still be in flight, everything older has landed - among
       // it this wave's part of chunks c + 1 and c + 2; the barrier publishes them
       // (a bare barrier: the fence of __syncthreads would drain every load in flight, since the
       // asynchronous copies count as stores to LDS)
       if constexpr (ADMA) {
-        vmem_wait<2 * kNF + kND + kPolls>();
+        vmem_wait<2 * kNF + kNA + (F8 && (buf + kStagesA - 1) % kStagesA == 0 ? 1 : 0) + kPolls>();
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       } else {
@@ -1633,6 +1644,35 @@ int tiled_gemm_fp8(const kmoe_gemm_fp8_args* a, hipStream_t s) {
   // its m-tiles the plain 128-row tiles are 2-4 % ahead of them at every batch: DeepSeek-V3 dims, layer at 2048 /
   // 4096 / 8192 / 12288 tokens 2.588 / 3.537 / 5.815 / 8.291 ms paced against 2.474 / 3.497 / 5.694 / 7.991.)
   const int avg_rows = ceil_div(live + (a->w_tail ? a->tail_rows : 0), a->E + (a->w_tail ? 1 : 0));
+  const long long weight_bytes = static_cast<long long>(a->E + (a->w_tail ? 1 : 0)) * a->n * a->k;
+  const int avg_routed = ceil_div(live, a->E);
+  // Wide tiles (eight waves side by side, 128, 160 or 192 rows, as for int8) on the ASYNCHRONOUS activation path: chunks
+  // and their row scales copied global -> LDS three chunks ahead, every LDS access in assembly, row fragments past a
+  // tile's rows not multiplied, an expert's rows split evenly over its tiles. The height: as few tiles per expert as 192
+  // rows allow, then the shortest that holds nearly every expert (average + 2.2 sqrt(average) rows) in that many - every row fragment of
+  // the tile is read from LDS, also those without rows. GEMM alone, us, 4-wave tiles (192-row wide tiles from 112 to 200 rows,
+  // before the scales came four chunks at a time) / 128- / 160- / 192-row wide tiles:
+  //   64 experts of [4096 x 7168], SiLU-mul: 80 rows per expert 389 / 344 / 365 / 381, 104 397 / 360 / 391 / 405, 110 466 / 404 / 366 /
+  //   384, 128 463 / 449 / 386 / 411, 144 498 / 559 / 485 / 427, 180 675 / 543 / 614 / 595, 256 826 / 696 / 666 / 698, 400 1138 / 956 / 941 / 947;
+  //   of [7168 x 2048]: 80 rows 207 / 198 / 204 / 227, 128 275 / 254 / 224 / 245, 180 363 / 317 / 341 / 302, 256 454 / 404 / 380 / 411;
+  //   128 experts of [1536 x 2048], SiLU-mul: 94 rows 100 / 93 / 100 / 106, 128 139 / 131 / 105 / 114, 512 364 / 320 / 325 / 300; of [2048 x
+  //   768] 94 rows 59 / 55 / 59 / 71, 128 81 / 78 / 66 / 78, 512 215 / 221 / 227 / 219.
+  // Few rows per expert on a long K take them too (64 experts of [4096 x 7168]: 52 rows 346 / 332, 72 354 / 344; 44 rows 326 / 330;
+  // [7168 x 2048], 64 rows 183 / 189: not). A row has at least the four scales that travel together: K from 512 on.
+  // 18 / 20 / 19 force the 192- / 160- / 128-row wide tile.
+  const bool wide_ok = a->k >= 512;
+  int wide = a->variant == 18 ? 12 : (a->variant == 20 ? 10 : (a->variant == 19 ? 8 : 0));
+  if (a->variant == 0 && (avg_rows > 76 || (avg_rows > 44 && a->k >= 4096 && weight_bytes > (1ll << 30)))) {
+    const float reach = avg_routed + 2.2f * sqrtf(static_cast<float>(avg_routed));
+    const float tiles = ceilf(reach / 192.0f);
+    wide = reach <= tiles * 128.0f ? 8 : (reach <= tiles * 160.0f ? 10 : 12);
+  }
+  // (the 192-row tile with a plain epilogue nearly fills the LDS: the copy of a thousand experts' row ranges does not fit)
+  if (wide == 12 && !swiglu && a->E > 896) wide = 10;
+  if (wide && wide_ok)
+    return wide == 8 ? launch_wide<K, 8>(p, a->rows, s, n_cu, what, swiglu, half)
+                     : (wide == 10 ? launch_wide<K, 10>(p, a->rows, s, n_cu, what, swiglu, half)
+                                   : launch_wide<K, 12>(p, a->rows, s, n_cu, what, swiglu, half));
   // 96-row tiles from 45 to 76 rows per expert: the padding rows of a 128-row tile cost this format its scaling work
   // on top of the MFMAs (gate_up GEMM alone, 64 rows per expert: Qwen3 shape 105 -> 85 us, DeepSeek-V3 shape 1515 ->
   // 1407 us; at 80 rows 107 -> 103 and 1541 -> 1508 us; at 90 rows the DeepSeek-V3 shape loses, 1578 -> 1812 us:
@@ -1644,19 +1684,6 @@ int tiled_gemm_fp8(const kmoe_gemm_fp8_args* a, hipStream_t s) {
     return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 6>(p, a->rows, s, n_cu, what)
                   : launch_tiled<K, false, 4, 4, 2, 1, false, 6>(p, a->rows, s, n_cu, what);
   }
-  const long long weight_bytes = static_cast<long long>(a->E + (a->w_tail ? 1 : 0)) * a->n * a->k;
-  const int avg_routed = ceil_div(live, a->E);
-  // Wide tiles (eight waves side by side, 192 or 128 rows, as for int8) on the ASYNCHRONOUS activation path: chunks
-  // and their row scales copied global -> LDS three chunks ahead, every LDS access in assembly, row fragments past a
-  // tile's rows not multiplied, an expert's rows split evenly over its tiles. This format gains less from them than
-  // int8 (its loop scales every chunk's partial sums, whatever the tile), and only where nearly every expert fills
-  // most of one 192-row tile: layer, tokens -> ms against the 4-wave tiles, DeepSeek-V3 dims 3072 / 4096 / 6144 /
-  // 8192 / 12288: 2.880 / 3.535 / 4.705 / 5.792 / 8.236 -> 2.881 / 3.326 / 4.653 / 6.001 / 7.989; Kimi-K2 dims 2048 /
-  // 4096 / 8192: 3.301 / 4.021 / 6.696 -> 3.501 / 4.360 / 6.322 (128-row wide: 3.330 / 4.050 / 6.693). So by default
-  // from 112 to 200 rows per expert with weights beyond 1 GiB; 18 / 19 force the 192- / 128-row wide tile.
-  if (a->variant == 18 || (a->variant == 0 && weight_bytes > (1ll << 30) && avg_routed >= 112 && avg_routed <= 200))
-    return launch_wide<K, 12>(p, a->rows, s, n_cu, what, swiglu, half);
-  if (a->variant == 19) return launch_wide<K, 8>(p, a->rows, s, n_cu, what, swiglu, half);
   // One 8-wave tile of 192 rows per expert on two rows of four waves (register path): variant 14, and the first
   // launch of the device-decided pair (variant 17); the wide tiles above took over where it had been the default.
   const bool by_rule = a->variant == 17 && avg_routed >= 124 && avg_routed <= 168;
