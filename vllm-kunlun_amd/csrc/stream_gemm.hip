@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
   __shared__ __attribute__((aligned(16))) int8_t qrows[QUANT ? 16 * kQuantStride : 16];
   __shared__ float qmax[16];
   const int lane = lane_id();
-  const int wave_id = W4 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = wave_id / KS;   // channel group of this wave
   const int wk = wave_id % KS;     // K part of this wave
   const int li = lane & 15;
@@ -146,14 +146,12 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
     return kb_begin + (s >= klen ? s - klen : s);
   };
 
-  // 4-bit weights: the loads of the K loop are raw buffer loads, a lane offset that stays and a scalar offset per step -
-  // no address arithmetic on the vector unit, which the unpacking keeps busy - and rows past the end lie past the
-  // descriptor's end: they read zero and fetch nothing (Kimi-K2 dimensions, 128 tokens: layer 1674 -> 1577 us, Qwen3
-  // 93 -> 90). The other formats leave the vector unit idle; there the same loads gain nothing (int8, bf16) or lose
-  // (fp8, DeepSeek-V3 at 128 tokens: 1800 -> 1854 us). A descriptor spans 4 GiB: the weights have one per fragment, the
-  // activations one in all, so launches whose rows may lie further apart (kRows32 false) read them through pointers.
+  // The weight loads of the K loop are raw buffer loads, a lane offset that stays and a scalar offset per step: no address
+  // arithmetic on the vector unit and 20 to 40 registers less than with pointers, and no select after a load, which
+  // would wait for it (with pointers the two kinds of load in load_w_step took twice the time of one). 4-bit weights: the
+  // activations too where their offsets fit 32 bits (kRows32), rows past the end lying past the descriptor's end: they
+  // read zero and fetch nothing (Kimi-K2 dimensions, 128 tokens: layer 1674 -> 1577 us, Qwen3 93 -> 90).
   __amdgpu_buffer_rsrc_t wr[NF];
-  const int8_t* wp[NF];
   bool wok[NF];
   int col[NF];
 #pragma unroll
@@ -164,10 +162,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
     col[f] = (SWIGLU && f >= NFH) ? n_half + c : c;
     const size_t frag = wok[f] ? col[f] / 16 : 0;
     const int frag_bytes = ksteps * (V * 1024);
-    if constexpr (W4)
-      wr[f] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w_base + frag * frag_bytes), 0, wok[f] ? frag_bytes : 0, 0x00020000);
-    else
-      wp[f] = w_base + frag * frag_bytes + lane * 16;
+    wr[f] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w_base + frag * frag_bytes), 0, wok[f] ? frag_bytes : 0, 0x00020000);
   }
 
   // The first weight steps are requested before anything else: their addresses depend on the block's coordinates
@@ -191,16 +186,22 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
     for (int f = 0; f < NF; ++f)
       sp[f] = p.w_scale + (static_cast<size_t>(e) * p.n + (wok[f] ? col[f] : 0)) * p.groups + li * p.s_ch;
   }
+  // The weights are read past the caches (see buffer_stream_load16), unless the workgroup will read them again: an expert's
+  // rows beyond TM take another pass. Qwen3 dims, int8, +2.0 on the logits of 8 experts, layer with ordinary loads / past the
+  // caches always / past them on an expert's last pass: 64 tokens 127 / 130 / 115 us, 140 tokens 182 / 203 / 163.
+  bool once = true;
   auto load_w_step = [&](int slot, int kb) {
+    auto load = [&](auto past) __attribute__((always_inline)) {
 #pragma unroll
-    for (int f = 0; f < NF; ++f)
+      for (int f = 0; f < NF; ++f)
 #pragma unroll
-      for (int v = 0; v < V; ++v)
-        if constexpr (W4)
-          wreg[slot][f][v] = buffer_load16(wr[f], lane * 16, static_cast<uint32_t>(kb) * (V * 1024) + v * 1024);
-        else
-          wreg[slot][f][v] = wok[f] ? *reinterpret_cast<const v4i*>(wp[f] + static_cast<size_t>(kb) * (V * 1024) + v * 1024)
-                                    : (v4i){0, 0, 0, 0};
+        for (int v = 0; v < V; ++v) {
+          const uint32_t at = static_cast<uint32_t>(kb) * (V * 1024) + v * 1024;
+          wreg[slot][f][v] = past ? buffer_stream_load16(wr[f], lane * 16, at) : buffer_load16(wr[f], lane * 16, at);
+        }
+    };
+    if (once) load(std::true_type{});
+    else load(std::false_type{});
     if constexpr (W4) {
       const int g32 = 4 * kb + lg;  // this lane's 32 values of the step
       const int g = p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / p.gs32;
@@ -333,6 +334,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
         if constexpr (FMT == Fmt::F8) asc[slot][mf] = asp[mf][kb];
       }
     };
+    once = __builtin_amdgcn_readfirstlane(row_end - row0) <= TM;
     auto load_step = [&](int slot, int kb) {
       load_w_step(slot, kb);
       load_a_step(slot, kb);
