@@ -21,6 +21,14 @@
 namespace kmoe {
 namespace {
 
+// Whether a launch reads its weights past the caches (see buffer_stream_load16): from 64 MB on. A layer called again at once with the
+// same few experts finds fewer bytes in the 256 MB memory-side cache. One to four tokens, layer, us, ordinary / past the caches: DeepSeek-V3
+// dims int8 (235 MB in gate_up) 78.3 / 72.0, fp8 83.5 / 74.6, Kimi-K2 dims 4-bit (117 MB) 52.5 / 49.1, Qwen3 dims int8, 4 tokens (101 MB)
+// 32.0 / 30.9; 1 token (25 MB) 16.3 / 17.9, bf16 (50 MB) 20.5 / 22.5.
+__device__ inline bool past_caches(size_t pairs, int channels, int row_bytes) {
+  return pairs * channels * row_bytes > (64u << 20);
+}
+
 constexpr bool few_wide_i8(Fmt f, int vecs) { return f == Fmt::I8 && vecs > 2; }
 
 // kVecs: vectors of 8 values a lane holds of its row (rows of up to 512 kVecs values)
@@ -52,12 +60,17 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
   const size_t frag_bytes = static_cast<size_t>(ksteps) * (V * 1024);
   const int8_t* w_base = (tail ? p.w_tail : p.w + static_cast<size_t>(e) * p.H * p.kbytes) + (col / 16) * frag_bytes;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w_base), 0, static_cast<int>(frag_bytes), 0x00020000);
+  const bool past = past_caches(static_cast<size_t>(p.M) * p.K, p.H, p.kbytes);
   v4i wreg[D][V];
   uint16_t gsc[W4 ? D : 1];
   const uint16_t* sp = W4 ? p.w_scale + (static_cast<size_t>(e) * p.H + col) * p.groups + li * p.s_ch : nullptr;
   auto load_w = [&](int slot, int s) {
 #pragma unroll
-    for (int v = 0; v < V; ++v) wreg[slot][v] = buffer_load16(wr, lane * 16, static_cast<uint32_t>(s) * (V * 1024) + v * 1024);
+    for (int v = 0; v < V; ++v) {
+      const uint32_t at = static_cast<uint32_t>(s) * (V * 1024) + v * 1024;
+      if (past) wreg[slot][v] = buffer_stream_load16(wr, lane * 16, at);
+      else wreg[slot][v] = buffer_load16(wr, lane * 16, at);
+    }
     if constexpr (W4) {
       const int g32 = 4 * s + lg;  // this lane's 32 values of the step
       gsc[slot] = sp[(p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / p.gs32) * p.s_g];
@@ -324,6 +337,7 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
     wr[f] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w_base + (c / 16) * frag_bytes), 0, static_cast<int>(frag_bytes), 0x00020000);
     sp[f] = W4 ? p.w_scale + (static_cast<size_t>(e) * (2 * p.I) + c) * p.groups + li * p.s_ch : nullptr;
   }
+  const bool past = past_caches(static_cast<size_t>(p.route.M) * p.route.K, 2 * p.I, p.kbytes);
   v4i wreg[D][2][V];
   uint16_t gsc[W4 ? D : 1][2];
   auto load_w = [&](int slot, int i) {
@@ -331,7 +345,11 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
 #pragma unroll
-      for (int v = 0; v < V; ++v) wreg[slot][f][v] = buffer_load16(wr[f], lane * 16, s * (V * 1024) + v * 1024);
+      for (int v = 0; v < V; ++v) {
+        const uint32_t at = s * (V * 1024) + v * 1024;
+        if (past) wreg[slot][f][v] = buffer_stream_load16(wr[f], lane * 16, at);
+        else wreg[slot][f][v] = buffer_load16(wr[f], lane * 16, at);
+      }
       if constexpr (W4) {
         const int g32 = 4 * s + lg;
         gsc[slot][f] = sp[f][(p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / p.gs32) * p.s_g];
