@@ -153,7 +153,10 @@ constexpr int w4_workgroups(int MF) { return MF <= 2 ? 4 : (MF == 4 ? 3 : 2); }
 // barrier, requests block kb + R - 1 of both and multiplies. No branch sits between a load and its use - the waits count
 // loads - so blocks past the end are requested as well, out of the descriptors' range: they fetch nothing.
 constexpr int w4_ring(int MF) { return MF == 6 ? 3 : 2; }
-template <int MF, bool SWIGLU, bool F16>
+// PAST: the weights are read past the caches (see buffer_stream_load16), where nearly every expert has one m-tile: always at 16 and 32
+// rows, at 64 rows up to 50 rows per expert. Layer, us, ordinary / past the caches: Qwen3 dims 128 tokens 84.0 / 79.8, Kimi-K2 dims
+// 64 tokens 1164 / 1125, 2048 2422 / 2392; with several tiles per expert their siblings miss: Qwen3 dims 2048 tokens 238 / 247.
+template <int MF, bool SWIGLU, bool F16, bool PAST>
 __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kernel(const W4Params p) {
   constexpr int NF = 4, R = w4_ring(MF);
   constexpr int kTileRows = 16 * MF;
@@ -234,7 +237,8 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
     const uint32_t s_at = lane_s + static_cast<uint32_t>((p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / (p.gs / 32)) * p.s_g) * 2u;
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
-      wbuf[slot][f] = buffer_load16(w_rsrc, lane16, live ? woff[f] + static_cast<uint32_t>(kb) * 1024u : kRange);
+      const uint32_t at = live ? woff[f] + static_cast<uint32_t>(kb) * 1024u : kRange;
+      wbuf[slot][f] = PAST ? buffer_stream_load16(w_rsrc, lane16, at) : buffer_load16(w_rsrc, lane16, at);
       sbuf[slot][f] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(s_rsrc, s_at, live ? soff[f] : kRange, 0));
     }
   };
@@ -335,7 +339,7 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
   }
 }
 
-template <int MF, bool SWIGLU>
+template <int MF, bool SWIGLU, bool PAST = (MF <= 2)>
 int launch_w4_tile(const W4Params& p, int rows, bool f16, hipStream_t s) {
   constexpr int kTileRows = 16 * MF;
   constexpr int NFH = SWIGLU ? 2 : 4;
@@ -348,9 +352,9 @@ int launch_w4_tile(const W4Params& p, int rows, bool f16, hipStream_t s) {
     note_kernel("w4_tile_kernel<%d-row tiles, %s, %s, %d per CU>", kTileRows, SWIGLU ? "SiLU-mul" : "plain",
                 f16 ? "f16" : "bf16", w4_workgroups(MF));
   if (f16)
-    hipLaunchKernelGGL((w4_tile_kernel<MF, SWIGLU, true>), grid, dim3(kWaves * kWave), 0, s, p);
+    hipLaunchKernelGGL((w4_tile_kernel<MF, SWIGLU, true, PAST>), grid, dim3(kWaves * kWave), 0, s, p);
   else
-    hipLaunchKernelGGL((w4_tile_kernel<MF, SWIGLU, false>), grid, dim3(kWaves * kWave), 0, s, p);
+    hipLaunchKernelGGL((w4_tile_kernel<MF, SWIGLU, false, PAST>), grid, dim3(kWaves * kWave), 0, s, p);
   return check_launch("kmoe_grouped_gemm_w4a16");
 }
 
@@ -460,7 +464,10 @@ int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t s
     case 4: return stream_gemm_w4(a, s, mf, scan, slots, stream_fits_32);
     case 16: return swiglu ? launch_w4_tile<1, true>(p, a->rows, f16, s) : launch_w4_tile<1, false>(p, a->rows, f16, s);
     case 32: return swiglu ? launch_w4_tile<2, true>(p, a->rows, f16, s) : launch_w4_tile<2, false>(p, a->rows, f16, s);
-    case 64: return swiglu ? launch_w4_tile<4, true>(p, a->rows, f16, s) : launch_w4_tile<4, false>(p, a->rows, f16, s);
+    case 64:
+      if (ceil_div(expected_rows(a->rows, a->rows_hint), a->E) <= 50)
+        return swiglu ? launch_w4_tile<4, true, true>(p, a->rows, f16, s) : launch_w4_tile<4, false, true>(p, a->rows, f16, s);
+      return swiglu ? launch_w4_tile<4, true>(p, a->rows, f16, s) : launch_w4_tile<4, false>(p, a->rows, f16, s);
     case 96: return swiglu ? launch_w4_tile<6, true>(p, a->rows, f16, s) : launch_w4_tile<6, false>(p, a->rows, f16, s);
     case 128: return swiglu ? launch_w4_tile<8, true>(p, a->rows, f16, s) : launch_w4_tile<8, false>(p, a->rows, f16, s);
     default:
