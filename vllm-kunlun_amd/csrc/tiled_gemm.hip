@@ -457,6 +457,11 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
   // Every load is unconditional (indices clamped to the last valid step / chunk, rows past a
   // tile's end read its first row, fragments past the last channel read fragment 0): the
   // results of those are never stored, and the loop body stays one basic block.
+  // The 64- and 96-row tiles run where nearly every expert has one m-tile: its weights are read once, past the caches (see
+  // buffer_stream_load16). GEMM alone, us, ordinary / past the caches: 64 experts of [4096 x 7168], 32 rows, int8 321 / 295, fp8 324 / 296;
+  // 128 experts of [1536 x 2048], 49 rows int8 77 / 72, 64 rows bf16 140 / 133. The taller tiles have siblings that read the
+  // same bytes from L2 (512 rows, int8 284 / 308; 256 rows, bf16 267 / 312).
+  constexpr bool kPast = NF == 4 && WM == 1 && MF <= 6 && !M32 && !PACE;
   auto load_w = [&](v4i(&dst)[kNF], int kb) {
     const uint32_t off = static_cast<uint32_t>(min(kb, last_step)) * 1024u;
     if constexpr (M32) {
@@ -464,7 +469,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       for (int f = 0; f < kNF; ++f) dst[f] = buffer_load16(w_rsrc, woff[f >> 1], off + (f & 1) * 512u);
     } else {
 #pragma unroll
-      for (int f = 0; f < kNF; ++f) dst[f] = buffer_load16(w_rsrc, woff[f], off);
+      for (int f = 0; f < kNF; ++f) dst[f] = kPast ? buffer_stream_load16(w_rsrc, woff[f], off) : buffer_load16(w_rsrc, woff[f], off);
     }
   };
   auto load_a = [&](int chunk) {
