@@ -108,7 +108,18 @@ __global__ __launch_bounds__(256) void silu_table_kernel(float* __restrict__ tab
 
 // ----------------------------------------------------------------- combine
 constexpr int kMaxTopK = 64;
+// PAST: the rows of the down projection, each read once, are read without a place in the caches: what they would push out of
+// the 256 MB memory-side cache is the rest of the same rows, just written there. From as many bytes on as it holds: 4096 tokens of 7168
+// values 132 -> 112 us, 3001 92 -> 80, 8192 of 2048 53 -> 51; 2048 of 7168 47 either way, 777 of 2048 10.2 -> 10.7.
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+template <bool PAST>
+__device__ inline uint4 load_row16(const uint16_t* p) {
+  if constexpr (!PAST) return *reinterpret_cast<const uint4*>(p);
+  const v4u v = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 
+template <bool PAST>
 __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict__ x, int64_t ld_x,
                                                      const int32_t* __restrict__ moe_index,
                                                      const float* __restrict__ topk_w,
@@ -136,7 +147,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
         r[i] = k0 + i < K ? rows[k0 + i] : -1;
-        p[i].v = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(max(r[i], 0)) * ld_x + c);
+        p[i].v = load_row16<PAST>(x + static_cast<size_t>(max(r[i], 0)) * ld_x + c);
       }
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
@@ -479,8 +490,9 @@ extern "C" int kmoe_combine_dt(const uint16_t* x, int64_t ld_x, const int32_t* m
                (long long)ld_addend);
   if (M == 0) return KMOE_OK;
   const int epilogue = (out_scale != 1.0f || addend) ? 1 : 0;
-  hipLaunchKernelGGL(combine_kernel, dim3(M, ceil_div(H, 256 * 8)), dim3(256), 0, as_stream(stream), x, ld_x, moe_index, topk_w,
-                     dequant_scale, K, H, out_scale, epilogue, addend, ld_addend, addend ? addend_scale : 1.0f, out, ld_out,
-                     act_dtype);
+  const bool past = static_cast<long long>(M) * K * H * 2 >= (256ll << 20);
+  hipLaunchKernelGGL((past ? combine_kernel<true> : combine_kernel<false>), dim3(M, ceil_div(H, 256 * 8)), dim3(256), 0, as_stream(stream), x, ld_x,
+                     moe_index, topk_w, dequant_scale, K, H, out_scale, epilogue, addend, ld_addend, addend ? addend_scale : 1.0f, out,
+                     ld_out, act_dtype);
   return check_launch("kmoe_combine");
 }
