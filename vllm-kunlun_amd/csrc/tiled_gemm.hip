@@ -459,9 +459,10 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
   // results of those are never stored, and the loop body stays one basic block.
   // The 64- and 96-row tiles run where nearly every expert has one m-tile: its weights are read once, past the caches (see
   // buffer_stream_load16). GEMM alone, us, ordinary / past the caches: 64 experts of [4096 x 7168], 32 rows, int8 321 / 295, fp8 324 / 296;
-  // 128 experts of [1536 x 2048], 49 rows int8 77 / 72, 64 rows bf16 140 / 133. The taller tiles have siblings that read the
-  // same bytes from L2 (512 rows, int8 284 / 308; 256 rows, bf16 267 / 312).
-  constexpr bool kPast = NF == 4 && WM == 1 && MF <= 6 && !M32 && !PACE;
+  // 128 experts of [1536 x 2048], 49 rows int8 77 / 72. Taller tiles have siblings that read the same bytes from L2 (512 rows,
+  // int8 284 / 308), and so have the hot experts of an uneven load, which weigh most with 16-bit weights: bf16 900 tokens 246 / 233, but
+  // 500 with +2.0 on the logits of 8 experts 236.4 / 237.0; those keep ordinary loads.
+  constexpr bool kPast = !BF && NF == 4 && WM == 1 && MF <= 6 && !M32 && !PACE;
   auto load_w = [&](v4i(&dst)[kNF], int kb) {
     const uint32_t off = static_cast<uint32_t>(min(kb, last_step)) * 1024u;
     if constexpr (M32) {
