@@ -7,7 +7,8 @@ import pytest
 import torch
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), ".."))
-from conftest import rel_l2  # noqa: E402
+from conftest import bits, from_bits, rel_l2  # noqa: E402
+from oracle import c_oracle as co  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -142,3 +143,54 @@ def test_rows_that_are_not_all_numbers(kind):
     assert ROUTED in named
     assert torch.equal(part.view(torch.int16)[[0, 2]], whole[:3].view(torch.int16)[[0, 2]])
     assert torch.equal(torch.isnan(part[1]), torch.isnan(whole[1])) and torch.equal(part[1].nan_to_num(), whole[1].nan_to_num())
+
+
+def _oracle(sl, M):
+    """The C oracle's output of a layer's first M tokens."""
+    s, f16 = sl.shape, sl.x.dtype == torch.float16
+    w13, a13, w2, a2, shared = sl.host_weights()
+    kw = dict(K=s.K, scoring=s.scoring, n_group=s.n_group, topk_group=s.topk_group, routed_scale=s.routed_scale, f16=f16,
+              bias=None if sl.bias is None else sl.bias.cpu().numpy())
+    x, logits = bits(sl.x[:M]), sl.logits[:M].float().cpu().numpy()
+    if s.quant == "int8":
+        shared = None if shared is None else tuple(t.numpy() for t in shared)
+        return co.forward_w8a8(x, logits, w13.numpy(), a13.numpy(), w2.numpy(), a2.numpy(), shared=shared, **kw)
+    if s.quant == "fp8":
+        w13, w2 = w13.view(torch.uint8), w2.view(torch.uint8)
+        shared = None if shared is None else tuple((t.view(torch.uint8) if t.dtype == torch.float8_e4m3fn else t).numpy() for t in shared)
+        return co.forward_fp8(x, logits, w13.numpy(), a13.numpy(), w2.numpy(), a2.numpy(), shared=shared, **kw)
+    if s.quant == "w4":
+        return co.forward_bf16(x, logits, co.dequant_w4_bf16(w13.numpy(), bits(a13), s.group_size, f16=f16),
+                               co.dequant_w4_bf16(w2.numpy(), bits(a2), s.group_size, f16=f16), **kw)
+    return co.forward_bf16(x, logits, bits(w13), bits(w2), **kw)
+
+
+@pytest.mark.parametrize("fmt,dims,dtype", [
+    ("int8", dict(M=6, H=2048, E=64, K=8, I=768), torch.bfloat16),     # 75 MB of down projections
+    ("int8", dict(M=9, H=1024, E=256, K=16, I=512), torch.float16),    # 75 MB, 144 pairs
+    ("int8", dict(M=3, H=4096, E=96, K=6, I=1024, I_shared=1024, n_group=1, topk_group=1), torch.bfloat16),  # ... a shared expert
+    ("fp8", dict(M=4, H=4096, E=96, K=4, I=1152), torch.bfloat16),
+    ("none", dict(M=6, H=2048, E=64, K=6, I=512), torch.bfloat16),
+    ("none", dict(M=6, H=2048, E=64, K=6, I=512), torch.float16),
+    ("w4", dict(M=3, H=4096, E=192, K=12, I=1024), torch.bfloat16)], ids=str)
+@pytest.mark.parametrize("common", [0, 1, 2])
+def test_down_projections_of_more_than_64_mb(fmt, dims, dtype, common):
+    """Launches of few tokens' down projection beyond 64 MB: experts of one token, of some and (`common` of them) of every
+    token, against the oracle. int8: its bits. Elsewhere the oracle's sums run in another order: 4e-3, as above."""
+    from vllm_kunlun_amd import synth
+    base = "dsv3-decode" if "I_shared" in dims else "qwen3-decode"
+    sl = synth.make_layer(synth.scaled(synth.SHAPES[base], quant=fmt, **dims), "cuda", seed=common, dtype=dtype)
+    M, E = dims["M"], dims["E"]
+    if common == 0:  # no expert twice (as far as they go)
+        for m in range(M):
+            sl.logits[m, [(m * dims["K"] + k) % E for k in range(dims["K"])]] += 9.0
+    sl.logits[:, :common] += 12.0
+    out, named = _named(lambda: sl.layer.quant_method.apply_monolithic(sl.layer, sl.x, sl.logits, **sl.apply_kwargs())
+                        if sl.shared is not None else sl.layer(sl.x, sl.logits))
+    assert FUSED in named, named
+    ref = _oracle(sl, M)
+    if fmt == "int8":
+        assert (bits(out) == ref).all()
+    else:
+        ref = torch.from_numpy(ref.view("int16")).view(dtype) if dtype == torch.float16 else from_bits(ref)
+        assert rel_l2(out.cpu(), ref) <= 4e-3

@@ -21,10 +21,12 @@
 namespace kmoe {
 namespace {
 
-// Whether a launch reads its weights past the caches (see buffer_stream_load16): from 64 MB on. A layer called again at once with the
-// same few experts finds fewer bytes in the 256 MB memory-side cache. One to four tokens, layer, us, ordinary / past the caches: DeepSeek-V3
-// dims int8 (235 MB in gate_up) 78.3 / 72.0, fp8 83.5 / 74.6, Kimi-K2 dims 4-bit (117 MB) 52.5 / 49.1, Qwen3 dims int8, 4 tokens (101 MB)
-// 32.0 / 30.9; 1 token (25 MB) 16.3 / 17.9, bf16 (50 MB) 20.5 / 22.5.
+// Whether a launch reads the weights that only one of its workgroups reads past the caches (see buffer_stream_load16): from 64 MB
+// of pairs on. A layer called again at once with the same few experts finds fewer bytes in the 256 MB memory-side cache; with other
+// layers' weights read in between they would gain from it too. Layer, us, ordinary / past the caches, called again at once; cold:
+// DeepSeek-V3 dims int8, 1 token (235 MB in gate_up) 78.3 / 72.0, fp8 83.5 / 74.6, Kimi-K2 dims 4-bit (117 MB) 52.5 / 49.1; Qwen3 dims
+// int8, 1 token (25 MB) 15.5 / 17.0; 19.5 / 18.5, 2 tokens (50 MB) 21.0 / 20.4; 24.0 / 22.5, bf16, 1 token (50 MB) 19.5 / 21.1; 24.4 / 23.3,
+// 4-bit, 1 token (13 MB) 14.8 / 15.6; 17.9 / 16.9.
 __device__ inline bool past_caches(size_t pairs, int channels, int row_bytes) {
   return pairs * channels * row_bytes > (64u << 20);
 }
@@ -60,7 +62,22 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
   const size_t frag_bytes = static_cast<size_t>(ksteps) * (V * 1024);
   const int8_t* w_base = (tail ? p.w_tail : p.w + static_cast<size_t>(e) * p.H * p.kbytes) + (col / 16) * frag_bytes;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w_base), 0, static_cast<int>(frag_bytes), 0x00020000);
-  const bool past = past_caches(static_cast<size_t>(p.M) * p.K, p.H, p.kbytes);
+  // What the workgroups of several tokens read - an expert that several chose, the shared expert - is left to the caches. Layer,
+  // us, past the caches all / as here, uniform routing cold; every token on the same eight experts, called again at once: Qwen3 dims int8 4
+  // tokens 33.5 / 33.4; 19.3 / 19.2, 6 44.7 / 43.6; 23.0 / 21.6, 8 54.0 / 53.0; 27.2 / 24.4, 10 62.2 / 61.6; 29.1 / 26.3, bf16 4 54.6 / 53.6; 25.6 /
+  // 22.5, 7 82.5 / 80.7; 34.5 / 27.0. (Uniform routing called again at once, 8 and 10 tokens: 52.4 / 52.8 and 60.4 / 61.5, with ordinary loads
+  // alone 51.7 and 59.5, but cold 54.5 and 62.8: part of what is left to the caches is there from the call before.)
+  bool past = past_caches(static_cast<size_t>(p.M) * p.K, p.H, p.kbytes);
+  if (past && p.M > 1) {
+    const int pairs = p.M * p.K;
+    int readers = tail ? p.M : 0;
+    if (!tail)
+      for (int j = lane; j - lane < pairs; j += 2 * kWave) {  // (two loads at once: 128 pairs are a memory round trip)
+        const int id[2] = {p.ids[min(j, pairs - 1)], p.ids[min(j + kWave, pairs - 1)]};
+        readers += __builtin_popcountll(__ballot(j < pairs && id[0] == e)) + __builtin_popcountll(__ballot(j + kWave < pairs && id[1] == e));
+      }
+    past = readers == 1;
+  }
   v4i wreg[D][V];
   uint16_t gsc[W4 ? D : 1];
   const uint16_t* sp = W4 ? p.w_scale + (static_cast<size_t>(e) * p.H + col) * p.groups + li * p.s_ch : nullptr;
