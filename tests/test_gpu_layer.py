@@ -153,6 +153,28 @@ def test_skewed_decode_batches_match_oracles(hot, boost):
         assert sl.layer.quant_method.last_layout.codes_chunked, "not on the weight-streaming path"
 
 
+@pytest.mark.parametrize("M", [15, 16, 17, 33])
+@pytest.mark.parametrize("quant", ["int8", "fp8"])
+@pytest.mark.parametrize("H,I", [(640, 128), (4096, 1152)])  # K split by one wave and by several
+def test_shared_expert_in_one_slice_and_in_several(quant, H, I, M):
+    """The shared expert's rows in the routed launches, 16 to a slice: one slice reads its weights past the caches, several share
+    them. int8: the oracle's bits. fp8: sums in another order than the oracle's move a 16-bit result by its rounding (2^-9 of
+    it, and the same again behind the second GEMM: 4e-3)."""
+    from vllm_kunlun_amd import synth
+    base = "dsv3-decode" if quant == "int8" else "dsv3-fp8-decode"
+    sl = synth.make_layer(synth.scaled(synth.SHAPES[base], M=M, H=H, E=32, K=4, I=I, I_shared=I, n_group=4, topk_group=2), "cuda", seed=M)
+    if quant == "int8":
+        _check_layer(sl)
+        return
+    out = sl.layer.quant_method.apply_monolithic(sl.layer, sl.x, sl.logits, **sl.apply_kwargs())
+    w13, a13, w2, a2, shared = sl.host_weights()
+    u8 = lambda t: (t.view(torch.uint8) if t.dtype == torch.float8_e4m3fn else t).numpy()  # noqa: E731
+    s = sl.shape
+    ref = co.forward_fp8(bits(sl.x), _host(sl.logits).numpy(), u8(w13), u8(a13), u8(w2), u8(a2), s.K, s.scoring, True, s.n_group,
+                         s.topk_group, s.routed_scale, _host(sl.bias).numpy(), tuple(u8(t) for t in shared))
+    assert rel_l2(out, from_bits(ref)) <= 4e-3
+
+
 def test_decode_launches_that_sort_and_quantise_keep_the_bits():
     """KMOE_SORT_IN_GEMM=0 / KMOE_QUANT_IN_GEMM=0 (read once per process, hence child processes) give the sort and
     the second quantisation launches of their own again: same output bits, same intermediates (int8 layers), same

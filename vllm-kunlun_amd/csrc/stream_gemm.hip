@@ -188,8 +188,11 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
   }
   // The weights are read past the caches (see buffer_stream_load16), unless the workgroup will read them again: an expert's
   // rows beyond TM take another pass. Qwen3 dims, int8, +2.0 on the logits of 8 experts, layer with ordinary loads / past the
-  // caches always / past them on an expert's last pass: 64 tokens 127 / 130 / 115 us, 140 tokens 182 / 203 / 163.
-  bool once = true;
+  // caches always / past them on an expert's last pass: 64 tokens 127 / 130 / 115 us, 140 tokens 182 / 203 / 163. Nor where another
+  // workgroup reads them: the slices of a tail expert. DeepSeek-V3 dims, layer with all slices past the caches / none: int8 23 tokens
+  // 838.7 / 831.7 us, 64 1462 / 1449, 128 1652 / 1630; fp8 23 843.9 / 835.2, 128 1663 / 1647, 250 1812 / 1781; 8 tokens (one slice) level.
+  const bool slices = tail && p.tail_rows > TM;
+  bool once = !slices;
   auto load_w_step = [&](int slot, int kb) {
     auto load = [&](auto past) __attribute__((always_inline)) {
 #pragma unroll
@@ -334,7 +337,7 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
         if constexpr (FMT == Fmt::F8) asc[slot][mf] = asp[mf][kb];
       }
     };
-    once = __builtin_amdgcn_readfirstlane(row_end - row0) <= TM;
+    once = !slices && __builtin_amdgcn_readfirstlane(row_end - row0) <= TM;
     auto load_step = [&](int slot, int kb) {
       load_w_step(slot, kb);
       load_a_step(slot, kb);
