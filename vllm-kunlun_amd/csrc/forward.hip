@@ -6,6 +6,7 @@
 #include <cstring>
 #include <mutex>
 
+#include "asked_once.h"
 #include "kmoe_common.h"
 
 namespace kmoe {
@@ -40,14 +41,13 @@ void note_kernel(const char* fmt, ...) {
 }
 
 int compute_units(int* n_cu) {
-  static int found = 0;
-  if (found == 0) {
-    int dev = 0, count = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || count < 1)
-      return fail(KMOE_ERR_LAUNCH, "cannot query the device");
-    found = count;
-  }
-  *n_cu = found;
+  static AskedOnce found;
+  const int count = found.get([] {
+    int dev = 0, n = 0;
+    return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess ? n : 0;
+  });
+  if (count < 1) return fail(KMOE_ERR_LAUNCH, "cannot query the device");
+  *n_cu = count;
   return KMOE_OK;
 }
 

@@ -1416,16 +1416,15 @@ int tiled_common(const TiledParams& p, int rows, int* n_cu_out, const char* what
   KMOE_REQUIRE(n_exp <= kMaxExperts, KMOE_ERR_SHAPE, "%s: E=%d > %d", what, p.E, kMaxExperts - 1);
   KMOE_REQUIRE(p.ldy % 8 == 0 && reinterpret_cast<uintptr_t>(p.y) % 16 == 0, KMOE_ERR_SHAPE,
                "%s: y must be 16-byte aligned with ldy %% 8 == 0 (ldy=%lld)", what, static_cast<long long>(p.ldy));
-  static int n_cu = 0;
-  if (n_cu == 0) {
-    if (int rc = compute_units(&n_cu)) return rc;
-    // KMOE_SPARE_CUS=n (read once): the persistent grids are cut for n fewer CUs, which stay free for a kernel that
-    // runs beside these launches on another stream (a collective; the clock probe). Multiples of 8 keep the XCDs even.
-    if (const char* spare = getenv("KMOE_SPARE_CUS")) {
-      const int n = atoi(spare);
-      if (n > 0 && n < n_cu) n_cu -= n;
-    }
-  }
+  int n_cu = 0;
+  if (int rc = compute_units(&n_cu)) return rc;
+  // KMOE_SPARE_CUS=n (read once): the persistent grids are cut for n fewer CUs, which stay free for a kernel that
+  // runs beside these launches on another stream (a collective; the clock probe). Multiples of 8 keep the XCDs even.
+  static const int spare = [] {
+    const char* v = getenv("KMOE_SPARE_CUS");
+    return v ? atoi(v) : 0;
+  }();
+  if (spare > 0 && spare < n_cu) n_cu -= spare;
   *n_cu_out = n_cu;
   return KMOE_OK;
 }
