@@ -233,3 +233,26 @@ def test_packed_launches_on_rows_beyond_4_gib_do_not_take_32_bit_offsets(L):
     g_tile.E, g_tile.n, g_tile.k, g_tile.rows, g_tile.lda, g_tile.ldy, g_tile.src_div = 4, 64, 128, 1 << 20, 4096, 64, 1
     g_tile.group_size, g_tile.variant, g_tile.w_layout = 32, 64, L.KMOE_W_TILED
     assert L.lib.kmoe_grouped_gemm_w4a16(g_tile, None) == -2 and b"32 bits" in L.lib.kmoe_last_error()
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="names the kernel a launch would take, on addresses that are not memory")
+def test_dense_products_beyond_32_bit_offsets_stay_on_the_streaming_kernel(L):
+    """kmoe_grouped_gemm_i8 with a tail matrix alone: the split-K kernel where its 32-bit offsets reach all activations (asked for
+    the compute units first, which fails without a GPU), else the streaming kernel (noted before its launch fails)."""
+    def call(a_rows, k):
+        g = L.GemmI8Args()
+        for f in ("a", "a_max", "w", "w_max", "lod", "y", "w_tail", "w_max_tail"):
+            setattr(g, f, 0x10000)
+        g.E, g.n, g.k, g.rows, g.ldy, g.a_rows, g.tail_rows = 1, 64, k, 0, 64, a_rows, 3
+        g.w_layout, g.a_layout = L.KMOE_W_TILED, L.KMOE_A_CHUNKED
+        L.lib.kmoe_trace_kernels(1)
+        rc = L.lib.kmoe_grouped_gemm_i8(g, None)
+        L.lib.kmoe_trace_kernels(0)
+        return rc, L.lib.kmoe_traced_kernels().decode(), L.lib.kmoe_last_error()
+
+    reach = 0xfff00000
+    rc, kernel, error = call(reach // 4096 - 1, 4096)
+    assert rc == -5 and kernel == "" and b"query the device" in error
+    for a_rows in (reach // 4096, 1 << 20, (1 << 20) + 1):
+        rc, kernel, error = call(a_rows, 4096)
+        assert rc == -5 and "stream_gemm_kernel<i8" in kernel, (a_rows, error)

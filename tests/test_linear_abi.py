@@ -44,3 +44,5 @@ def test_refusals(L):
                      ({"y": 4100}, -2), ({"act_dtype": 7}, -3)):
         assert call(**over) == rc, over
     assert call(rows=0, scratch_bytes=0) == 0
+    far = 0xfff00000 // 65536  # codes beyond 32-bit offsets: only through lod
+    assert call(rows=far, k=65536, ld_x=65536, scratch_bytes=1 << 40) == -2 and b"32-bit" in L.lib.kmoe_last_error()

@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kDenseWaves* kWave, WPS) void dense_i8_kernel(const
   for (int f = 0; f < NF; ++f)
     wr[f] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.w + static_cast<size_t>(min(frag0 + f, n_frags - 1)) * frag_bytes), 0,
                                               frag0 + f < n_frags ? frag_bytes : 0, 0x00020000);
-  const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.a), 0, QUANT ? 0 : p.a_rows * p.k, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.a), 0, QUANT ? 0 : static_cast<uint32_t>(p.a_rows) * static_cast<uint32_t>(p.k), 0x00020000);
   uint32_t aoff[MF];
 #pragma unroll
   for (int m = 0; m < MF; ++m) {
@@ -252,9 +252,9 @@ int launch_shape(const DenseParams& p, int shape, hipStream_t s) {
 // 5120] 96 rows 24.7 / 27.5, [24576 x 1536] 48 rows 11.7 / 12.0; [1536 x 7168] 512 rows, cost 8: 19.0 / 15.1)
 constexpr int kDenseCost = 15, kDenseMaxRows = 512;
 
+bool dense_gemm_i8_reaches(int a_rows, int k) { return static_cast<int64_t>(a_rows) * k < 0xfff00000ll; }
+
 int dense_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
-  KMOE_REQUIRE(static_cast<int64_t>(a->a_rows) * a->k < 0xfff00000ll, KMOE_ERR_SHAPE,
-               "grouped_gemm_i8 (dense): %d rows of %d codes need 32-bit offsets", a->a_rows, a->k);
   int n_cu = 0, shape = 0;
   if (int rc = compute_units(&n_cu)) return rc;
   DenseParams p = {};
@@ -348,6 +348,7 @@ extern "C" int kmoe_linear_i8(const kmoe_linear_i8_args* a, kmoe_stream_t stream
       return shape == 0 ? launch_dense<1, 1, 8, 4, true>(p, as_stream(stream)) : launch_dense<1, 2, 5, 4, true>(p, as_stream(stream));
     }
   }
+  KMOE_REQUIRE(dense_gemm_i8_reaches(a->rows, a->k), KMOE_ERR_SHAPE, "linear_i8: %d rows of %d codes need 32-bit offsets without lod", a->rows, a->k);
   if (int rc = kmoe_quant_i8_rows_chunked_dt(a->x, a->ld_x, a->rows, a->k, static_cast<int8_t*>(a->scratch), x_max, a->act_dtype, stream)) return rc;
   g.a_layout = KMOE_A_CHUNKED;
   g.a_rows = a->rows;

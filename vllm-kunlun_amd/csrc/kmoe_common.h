@@ -84,6 +84,7 @@ constexpr int kFewMaxI = 2048, kFewMaxWaves = 16;  // K, and one for the shared 
 int few_down(const FewDown& p, int format, hipStream_t stream);
 // Dense int8 GEMM of a few rows (a tail expert alone, tiled weights, chunk-major activations); arguments already validated.
 int dense_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream);
+bool dense_gemm_i8_reaches(int a_rows, int k);  // whether its 32-bit offsets reach these activations
 int stream_gemm_i8(const kmoe_gemm_i8_args* args, hipStream_t stream, const StreamScan* scan, const StreamQuant* quant,
                    const StreamSlots* slots);
 // The same kernel on fp8 block-scaled and on 16-bit weights (tiled; row-major activations).

@@ -565,8 +565,8 @@ int stream_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s, const StreamScan* 
     KMOE_REQUIRE(a->a_rows <= kStreamScanMaxRows, KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8 (stream): %d tokens", a->a_rows);
     return launch_rows16<Fmt::I8, true, true>(p, s);
   }
-  // a dense matrix: a tail expert alone
-  if (a->variant == 0 && a->rows == 0 && !swiglu) return dense_gemm_i8(a, s);
+  // a dense matrix: a tail expert alone (activations beyond that kernel's 32-bit offsets stay here)
+  if (a->variant == 0 && a->rows == 0 && !swiglu && dense_gemm_i8_reaches(a->a_rows, a->k)) return dense_gemm_i8(a, s);
   // m-fragments per pass from the rows an expert gets under uniform routing
   int mf = a->variant;
   if (mf == 0) {
