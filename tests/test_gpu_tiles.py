@@ -169,3 +169,32 @@ def test_block_fp8_wide_tiles(variant, blocks, act, dtype, tail):
     assert not got.isnan().any()
     per_row = (got - ref).norm(dim=1) / ref.norm(dim=1).clamp(min=1e-6)
     assert float(per_row.max()) <= (5 if act else 1) * 2 ** -8
+
+
+@pytest.mark.parametrize("variant,rows", [(19, 128), (20, 160), (18, 192)])
+@pytest.mark.parametrize("blocks", [3, 4])
+def test_block_fp8_wide_tiles_need_four_blocks(variant, rows, blocks):
+    """A forced wide tile runs from four blocks of K on; with fewer the launch is the four-wave tiles'. The bits are the same."""
+    from vllm_kunlun_amd import _lib as L
+    gen = torch.Generator().manual_seed(blocks)
+    counts = [200, 0, 17]
+    E, n, k, fp8 = len(counts), 256, 128 * blocks, torch.float8_e4m3fn
+    a = torch.randn(sum(counts), k, generator=gen).to(fp8).cuda()
+    a_scale = (torch.rand(sum(counts), blocks, generator=gen) + 0.5).cuda()
+    w = torch.randn(E, n, k, generator=gen).to(fp8).cuda()
+    w_scale = (torch.rand(E, n // 128, blocks, generator=gen) + 0.5).cuda()
+    lod = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    out = []
+    for v in (variant, 6):
+        y = torch.zeros(sum(counts), n, dtype=torch.bfloat16, device="cuda")
+        g = L.GemmFp8Args()
+        g.a, g.lda, g.a_scale, g.src_div, g.w, g.w_scale = a.data_ptr(), k, a_scale.data_ptr(), 1, w.data_ptr(), w_scale.data_ptr()
+        g.w_layout, g.lod, g.E, g.n, g.k, g.rows = L.KMOE_W_TILED, lod.data_ptr(), E, n, k, sum(counts)
+        g.y, g.ldy, g.variant, g.act_dtype = y.data_ptr(), n, v, L.act_dtype(y, "test")
+        L.lib.kmoe_trace_kernels(1)
+        L.check(L.lib.kmoe_grouped_gemm_fp8_block(g, L.stream()))
+        L.lib.kmoe_trace_kernels(0)
+        out.append((y, L.lib.kmoe_traced_kernels().decode()))
+    assert f"{rows if blocks >= 4 else 128}x256 tile, {8 if blocks >= 4 else 4} waves" in out[0][1], out[0][1]
+    assert "128x256 tile, 4 waves" in out[1][1], out[1][1]
+    assert torch.equal(out[0][0], out[1][0])
