@@ -138,12 +138,27 @@ def test_row_ranges_made_in_a_capture_are_the_graphs_own(monkeypatch):
     assert kept.tolist() == [0, 203] and scale_mm._row_range(cpu, 203) is kept
 
 
-def test_rows_the_streaming_kernel_takes_depend_on_the_channels():
-    """Narrow matrices stay on the weight-streaming kernel up to 256 rows, wide ones leave it as soon as its slices fill
-    the chip; every matrix has its first 16 rows there."""
-    from vllm_kunlun_amd.quantization.kernels.scale_mm import _DynamicCall
-    rows = [_DynamicCall._stream_max_rows(n) for n in (16, 576, 1536, 2560, 4096, 7168, 12288, 24576, 1 << 20)]
-    assert rows == [256, 256, 256, 256, 160, 64, 32, 16, 16]
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(16, 64), (576, 1024), (4096, 448), (12288, 192), (24576, 64)])
+def test_the_library_says_up_to_which_row_the_split_kernel_is_taken(n, k):
+    """Rows on both sides of kmoe_linear_i8_split_rows: the kernel whose waves split K, then the tile kernel (long rows of few
+    channels: up to its 512 rows; wide matrices: its first 16 at least), with the oracle's bits."""
+    from vllm_kunlun_amd import _lib as L
+    from vllm_kunlun_amd.quantization.kernels.scale_mm import KunlunScaledMMLinearKernel
+    layer, wq, w_max = _layer(n, k, "cuda", n + k)
+    kern = KunlunScaledMMLinearKernel()
+    kern.process_weights_after_loading(layer)
+    most = L.lib.kmoe_linear_i8_split_rows(n, k)
+    assert 16 <= most <= 512 and (most == 512) == (n <= 576) and (most < 64) == (n >= 24576), most
+    for rows in (most, most + 1):
+        x = (torch.randn(rows, k, generator=torch.Generator().manual_seed(rows)) * 1.5).bfloat16()
+        L.lib.kmoe_trace_kernels(1)
+        out = kern.apply_weights(layer, x.cuda())
+        L.lib.kmoe_trace_kernels(0)
+        assert ("dense_i8_kernel" in L.lib.kmoe_traced_kernels().decode()) == (rows == most)
+        xq, x_max = co.quant_i8_rows(bits(x))
+        ref, _ = co.grouped_gemm_i8(xq, x_max, wq.numpy()[None], w_max.numpy()[None], np.array([0, rows], np.int32))
+        assert np.array_equal(bits(out), ref)
 
 
 @pytest.mark.gpu

@@ -60,14 +60,6 @@ class _DynamicCall:
 
     __slots__ = ("args", "n", "k", "device", "scale", "at", "epoch", "split_max")
 
-    # Rows that go to the kernel whose waves split K: kmoe_linear_i8_split_rows knows from the matrix up to where it is
-    # ahead of the tile kernel; at least the rows below, which leave the tile kernel too few workgroups.
-    STREAM_MAX_GROUPS, STREAM_MAX_ROWS = 640, 256
-
-    @classmethod
-    def _stream_max_rows(cls, n: int) -> int:
-        return max(16, min(cls.STREAM_MAX_ROWS, 32 * (cls.STREAM_MAX_GROUPS // -(-n // 32))))
-
     def __init__(self, layer, names, w, w_max):
         L.require_device(w, w_max)
         L.require_contig(w, w_max)
@@ -77,9 +69,8 @@ class _DynamicCall:
         self.at = (w.data_ptr(), w_max.data_ptr())
         self.epoch = _plan._layout_epoch
         layout = weight_layout(w)
-        self.split_max = 0
-        if layout == L.KMOE_W_TILED:
-            self.split_max = max(self._stream_max_rows(self.n), L.lib.kmoe_linear_i8_split_rows(self.n, self.k))
+        # rows that go to the kernel whose waves split K; more, and row-major weights, to the tile kernel
+        self.split_max = L.lib.kmoe_linear_i8_split_rows(self.n, self.k) if layout == L.KMOE_W_TILED else 0
         g = L.LinearI8Args()
         g.w, g.w_max = self.at
         g.n, g.k, g.ld_x, g.ldy, g.w_layout = self.n, self.k, self.k, self.n, layout
