@@ -184,6 +184,22 @@ def _oracle(sl, M):
     return co.forward_bf16(x, logits, bits(w13), bits(w2), **kw)
 
 
+def _call(sl):
+    if sl.shared is None:
+        return sl.layer(sl.x, sl.logits)
+    return sl.layer.quant_method.apply_monolithic(sl.layer, sl.x, sl.logits, **sl.apply_kwargs())
+
+
+def _check(sl, out):
+    """int8: the oracle's bits. Elsewhere the oracle's sums run in another order, which moves a 16-bit result by its rounding
+    (2^-9 of it, and the same again behind the second GEMM): 4e-3."""
+    ref = _oracle(sl, sl.shape.M)
+    if sl.shape.quant == "int8":
+        assert (bits(out) == ref).all()
+    else:
+        assert rel_l2(out, from_bits(ref).view(out.dtype)) <= 4e-3
+
+
 @pytest.mark.parametrize("fmt,dims,dtype", [
     ("int8", dict(M=6, H=2048, E=64, K=8, I=768), torch.bfloat16),     # 75 MB of down projections
     ("int8", dict(M=9, H=1024, E=256, K=16, I=512), torch.float16),    # 75 MB, 144 pairs
@@ -195,7 +211,7 @@ def _oracle(sl, M):
 @pytest.mark.parametrize("common", [0, 1, 2])
 def test_down_projections_of_more_than_64_mb(fmt, dims, dtype, common):
     """Launches of few tokens' down projection beyond 64 MB: experts of one token, of some and (`common` of them) of every
-    token, against the oracle. int8: its bits. Elsewhere the oracle's sums run in another order: 4e-3, as above."""
+    token, against the oracle."""
     from vllm_kunlun_amd import synth
     base = "dsv3-decode" if "I_shared" in dims else "qwen3-decode"
     sl = synth.make_layer(synth.scaled(synth.SHAPES[base], quant=fmt, **dims), "cuda", seed=common, dtype=dtype)
@@ -204,12 +220,40 @@ def test_down_projections_of_more_than_64_mb(fmt, dims, dtype, common):
         for m in range(M):
             sl.logits[m, [(m * dims["K"] + k) % E for k in range(dims["K"])]] += 9.0
     sl.logits[:, :common] += 12.0
-    out, named = _named(lambda: sl.layer.quant_method.apply_monolithic(sl.layer, sl.x, sl.logits, **sl.apply_kwargs())
-                        if sl.shared is not None else sl.layer(sl.x, sl.logits))
+    out, named = _named(lambda: _call(sl))
     assert FUSED in named, named
-    ref = _oracle(sl, M)
-    if fmt == "int8":
-        assert (bits(out) == ref).all()
-    else:
-        ref = torch.from_numpy(ref.view("int16")).view(dtype) if dtype == torch.float16 else from_bits(ref)
-        assert rel_l2(out.cpu(), ref) <= 4e-3
+    _check(sl, out)
+
+
+@pytest.mark.parametrize("fmt,dims", [
+    ("int8", dict(M=4, H=4096, E=40, K=4, I=768)),                   # 101 MB of gate_up projections
+    ("int8", dict(M=3, H=4096, E=48, K=8, I=768, I_shared=768, n_group=4, topk_group=2)),   # ... sigmoid routing, a shared expert
+    ("fp8", dict(M=4, H=4096, E=40, K=4, I=640)),
+    ("fp8", dict(M=4, H=4096, E=40, K=4, I=640, I_shared=640, n_group=4, topk_group=2)),
+    ("none", dict(M=3, H=2048, E=40, K=8, I=768)),
+    ("w4", dict(M=2, H=4096, E=80, K=16, I=640))], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("common", [0, 2])
+def test_gate_up_projections_of_more_than_64_mb(fmt, dims, dtype, common):
+    """Layers whose first launch routes and streams more than 64 MB, so that it reads its weights past the caches, with experts of one
+    token and (`common` of them) of every token, against the oracle."""
+    from vllm_kunlun_amd import synth
+    base = ("dsv3-fp8-decode" if fmt == "fp8" else "dsv3-decode") if "I_shared" in dims else "qwen3-decode"
+    sl = synth.make_layer(synth.scaled(synth.SHAPES[base], quant=fmt, **dims), "cuda", seed=7 + common, dtype=dtype)
+    sl.logits[:, :common] += 12.0
+    out, named = _named(lambda: _call(sl))
+    assert ROUTED in named, named
+    _check(sl, out)
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8", "none", "w4"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,H,I", [(1, 8, 640, 384), (4, 6, 256, 1152), (7, 3, 1152, 128), (9, 8, 256, 1024)])
+def test_few_tokens_match_the_oracle(fmt, dtype, M, K, H, I):
+    """Batches on both sides of the launch that routes (4 tokens), experts shared and not."""
+    from vllm_kunlun_amd import synth
+    sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], M=M, H=H, E=96, K=K, I=I, quant=fmt), "cuda", seed=M, dtype=dtype)
+    sl.logits[:, :K // 3] += 9.0
+    out, named = _named(lambda: _call(sl))
+    assert FUSED in named and (ROUTED in named) == (M <= 4), named
+    _check(sl, out)

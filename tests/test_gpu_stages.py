@@ -453,6 +453,25 @@ def test_combine(L, M, K, H, epilogue):
     assert np.array_equal(bits(out), ref)
 
 
+@pytest.mark.parametrize("M", [2047, 2048])  # 256 MiB of rows, from which on they are read past the caches, and a token less
+@pytest.mark.parametrize("f16", [False, True])
+def test_combine_of_rows_the_caches_cannot_hold(L, M, f16):
+    """Strided rows, pairs without one (index -1), the caller's epilogue with both scales: the oracle's bits."""
+    K, H, ld = 8, 8192, 8192 + 8
+    dtype = torch.float16 if f16 else torch.bfloat16
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M * K, ld, generator=gen, device="cuda").to(dtype)
+    w = torch.rand(M, K, generator=gen, device="cuda")
+    index = torch.randperm(M * K, generator=gen, device="cuda").int()
+    index[::97] = -1
+    addend = torch.randn(M, H, generator=gen, device="cuda").to(dtype)
+    out = torch.empty(M, H, dtype=dtype, device="cuda")
+    L.check(L.lib.kmoe_combine_dt(L.ptr(x), ld, L.ptr(index), L.ptr(w), None, M, K, H, 0.5, L.ptr(addend), H, 0.75, L.ptr(out), H,
+                                  L.KMOE_DT_F16 if f16 else L.KMOE_DT_BF16, L.stream()))
+    ref = co.combine(bits(x[:, :H]), index.cpu().numpy(), w.cpu().numpy(), None, 0.5, bits(addend), 0.75, f16=f16)
+    assert np.array_equal(bits(out), ref)
+
+
 # ------------------------------------------- tiled weights / chunked activations
 def _tile_ref(w):
     """numpy restatement of the 1 KB block layout: [E][n/16][k/64][g(4)][c(16)][16]."""
