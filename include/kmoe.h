@@ -689,7 +689,11 @@ typedef struct kmoe_moe_args {
  * moe_index, sorted_src, expert_m and lod as the sort's launch would; the down launch of int8 layers quantises its rows
  * itself (rows up to 1024 values) and writes actq and actmax as the quantiser's launch would. Same bits, same workspace
  * contents, two launches fewer; KMOE_STAGE_ALIGN / KMOE_STAGE_QUANT2 then bracket nothing. The environment variables KMOE_SORT_IN_GEMM=0
- * and KMOE_QUANT_IN_GEMM=0 (read once per process) keep the launches apart: for measurements. */
+ * and KMOE_QUANT_IN_GEMM=0 (read once per process) keep the launches apart: for measurements.
+ * A few tokens with fewer pairs than experts may take two launches. One ends the layer: second quantisation, down projection and
+ * combine (actq, actmax and down are written as by launches of their own; KMOE_STAGE_QUANT2 and KMOE_STAGE_COMBINE bracket
+ * nothing). One begins it, up to four tokens: routing, first quantisation, sort and gate_up (xq and xmax are then not written;
+ * KMOE_STAGE_ROUTING brackets the gate's projection or nothing, KMOE_STAGE_ALIGN and KMOE_STAGE_QUANT1 nothing). int8: the bits of the separate launches. */
 
 #define KMOE_STAGE_ROUTING 0
 #define KMOE_STAGE_ALIGN 1

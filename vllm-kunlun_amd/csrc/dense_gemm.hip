@@ -9,6 +9,11 @@
 //   a squarer tile means fewer bytes: [100 x 7168] x [4096 x 7168] takes 256 workgroups (one per CU) of 64 x 32 that
 //   fetch 0.6 MB each, where slices of 32 rows with K split four ways fetched 0.9 MB per CU, 64 KB at a time.
 // Rows are split evenly over the row tiles and rows past a tile's end are out of the descriptor's range: no bytes.
+// The weights are read with ordinary loads: a Linear that is called again at once finds them in the 256 MB memory-side cache. With
+// other layers' weights read in between, loads past the caches (see buffer_stream_load16) would be ahead while one row tile holds
+// all rows. [4096 x 7168], SiLU-mul, [7168 x 2048], us, ordinary / past the caches, called again at once; cold: 1 row 14.8 / 14.7; 18.2 /
+// 17.0, 16 21.2 / 22.7; 25.5 / 23.9, 100 29.0 / 31.9; 35.6 / 34.3, 200 35.6 / 40.6; 41.6 / 43.0. Up to four rows, too, smaller matrices
+// lose: [1536 x 2048], SiLU-mul, [2048 x 768] 1 row 9.6 / 10.4; 11.2 / 10.9.
 // The eight partial sums meet in LDS once; wave w then finishes fragments w, w + 8, ... of the tile. int32 sums are exact,
 // so neither the split nor the order shows in a bit.
 #include "buffer_ops.h"

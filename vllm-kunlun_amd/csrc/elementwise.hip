@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void silu_table_kernel(float* __restrict__ tab
 constexpr int kMaxTopK = 64;
 // PAST: the rows of the down projection, each read once, are read without a place in the caches: what they would push out of
 // the 256 MB memory-side cache is the rest of the same rows, just written there. From as many bytes on as it holds: 4096 tokens of 7168
-// values 132 -> 112 us, 3001 92 -> 80, 8192 of 2048 53 -> 51; 2048 of 7168 47 either way, 777 of 2048 10.2 -> 10.7.
+// values 132 -> 114.5 us, 3001 91.5 -> 79, 8192 of 2048 54 -> 51.5; below, 2048 of 7168 46.5 -> 45.6, 777 of 2048 10.4 -> 10.5.
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 template <bool PAST>
 __device__ inline uint4 load_row16(const uint16_t* p) {

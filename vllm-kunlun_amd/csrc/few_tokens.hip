@@ -5,10 +5,10 @@
 // A batch of a few tokens is a chain of launches that each read a few MB: what it costs is launches and dependent memory
 // round trips. In the down projection every routed pair is one row, so a workgroup can own 16 output channels of one TOKEN:
 // a wave per routed expert (and one for the shared expert that rides along) streams that expert's 16 channels over all of K
-// for the pair's row, the rows of the result meet in LDS, and the workgroup adds them up as the combine would - no down
-// rows to write and read back, no launch for them, none for the quantisation in front: each wave quantises its own row
-// while its weights are on their way. An expert that several tokens share is read once per token (from the caches), which
-// is why this stops at a few of them.
+// for the pair's row, the rows of the result meet in LDS, and the workgroup adds them up as the combine would - no launch
+// that reads the down rows back, none for the quantisation in front: each wave quantises its own row while its weights are on
+// their way. (Down rows, codes and their scales are still written, for whoever inspects the workspace; nothing here waits for
+// them.) An expert that several tokens share is read once per token (from the caches), which is why this stops at a few of them.
 #include <algorithm>
 
 #include "buffer_ops.h"

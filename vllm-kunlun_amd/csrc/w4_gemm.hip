@@ -154,8 +154,8 @@ constexpr int w4_workgroups(int MF) { return MF <= 2 ? 4 : (MF == 4 ? 3 : 2); }
 // loads - so blocks past the end are requested as well, out of the descriptors' range: they fetch nothing.
 constexpr int w4_ring(int MF) { return MF == 6 ? 3 : 2; }
 // PAST: the weights are read past the caches (see buffer_stream_load16), where nearly every expert has one m-tile: always at 16 and 32
-// rows, at 64 rows up to 50 rows per expert. Layer, us, ordinary / past the caches: Qwen3 dims 128 tokens 84.0 / 79.8, Kimi-K2 dims
-// 64 tokens 1164 / 1125, 2048 2422 / 2392; with several tiles per expert their siblings miss: Qwen3 dims 2048 tokens 238 / 247.
+// rows, at 64 rows up to 50 rows per expert. Layer, us, ordinary / past the caches: Qwen3 dims 128 tokens 78.8 / 75.9, cold 84.0 / 79.8,
+// Kimi-K2 dims 64 tokens 1232 / 1191, 2048 2418 / 2390; with several tiles per expert their siblings miss: Qwen3 dims 2048 tokens 238 / 247.
 template <int MF, bool SWIGLU, bool F16, bool PAST>
 __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kernel(const W4Params p) {
   constexpr int NF = 4, R = w4_ring(MF);
