@@ -690,10 +690,12 @@ typedef struct kmoe_moe_args {
  * itself (rows up to 1024 values) and writes actq and actmax as the quantiser's launch would. Same bits, same workspace
  * contents, two launches fewer; KMOE_STAGE_ALIGN / KMOE_STAGE_QUANT2 then bracket nothing. The environment variables KMOE_SORT_IN_GEMM=0
  * and KMOE_QUANT_IN_GEMM=0 (read once per process) keep the launches apart: for measurements.
- * A few tokens with fewer pairs than experts may take two launches. One ends the layer: second quantisation, down projection and
- * combine (actq, actmax and down are written as by launches of their own; KMOE_STAGE_QUANT2 and KMOE_STAGE_COMBINE bracket
- * nothing). One begins it, up to four tokens: routing, first quantisation, sort and gate_up (xq and xmax are then not written;
- * KMOE_STAGE_ROUTING brackets the gate's projection or nothing, KMOE_STAGE_ALIGN and KMOE_STAGE_QUANT1 nothing). int8: the bits of the separate launches. */
+ * A few tokens with fewer pairs than experts may take two launches (either variable keeps those apart as well). One ends the
+ * layer: second quantisation, down projection and combine (actq, actmax and down are written as by launches of their own;
+ * KMOE_STAGE_QUANT2 and KMOE_STAGE_COMBINE bracket nothing). One begins it, up to four tokens: routing, first quantisation, sort and
+ * gate_up (xq and xmax are then not written; KMOE_STAGE_ROUTING brackets the gate's projection or nothing, KMOE_STAGE_ALIGN
+ * and KMOE_STAGE_QUANT1 nothing). int8: the bits of the separate launches; in the other formats a sum over K is added up in another
+ * order, so that a token's result may differ in its last bits from the same token's in a larger batch. */
 
 #define KMOE_STAGE_ROUTING 0
 #define KMOE_STAGE_ALIGN 1

@@ -257,3 +257,33 @@ def test_few_tokens_match_the_oracle(fmt, dtype, M, K, H, I):
     out, named = _named(lambda: _call(sl))
     assert FUSED in named and (ROUTED in named) == (M <= 4), named
     _check(sl, out)
+
+
+@pytest.mark.parametrize("variable", ["KMOE_QUANT_IN_GEMM", "KMOE_SORT_IN_GEMM"])
+def test_switches_keep_the_launches_apart(variable):
+    """Each of them set to 0 (read once per process, hence a child process) gives a few-token layer its launches back: the output
+    bits stay (int8), and the first quantisation's codes and maxima stand in the workspace."""
+    import subprocess
+    code = r"""
+import sys, zlib
+sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[2])
+import torch
+from vllm_kunlun_amd import _lib as L, synth
+sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], M=3, H=512, E=64, K=6, I=768), "cuda", seed=4)
+m = sl.layer.quant_method
+L.lib.kmoe_trace_kernels(1)
+out = sl.layer(sl.x, sl.logits)
+L.lib.kmoe_trace_kernels(0)
+named = L.lib.kmoe_traced_kernels().decode()
+lay, ws = m.last_layout, m.last_workspace
+x_max = ws[lay.xmax: lay.xmax + 12].view(torch.float32)
+print(zlib.crc32(out.view(torch.int16).cpu().numpy().tobytes()), int("few_" in named), int(torch.equal(x_max, sl.x.float().abs().amax(1))))
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = []
+    for flag in ("1", "0"):
+        run = subprocess.run([sys.executable, "-c", code, root, os.path.join(root, "vllm-kunlun_amd")], env=dict(os.environ, **{variable: flag}),
+                             capture_output=True, text=True, timeout=110)
+        assert run.returncode == 0, run.stderr[-2000:]
+        got.append(run.stdout.split())
+    assert got[0][0] == got[1][0] and got[0][1] == "1" and got[1][1:] == ["0", "1"], got

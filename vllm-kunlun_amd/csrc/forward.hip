@@ -140,7 +140,7 @@ bool scan_allowed() {
   return on;
 }
 
-// KMOE_QUANT_IN_GEMM=0 (read once) keeps the second quantisation a launch of its own there.
+// KMOE_QUANT_IN_GEMM=0 (read once) keeps both quantisations launches of their own there.
 bool quant_in_gemm_allowed() {
   static const bool on = [] {
     const char* v = getenv("KMOE_QUANT_IN_GEMM");
@@ -692,8 +692,9 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   // Fewer pairs than experts: a column of workgroups per pair instead of per expert.
   const bool per_pair = scan_in_gemm && P < E && P <= kStreamSlotMaxPairs;
   const bool fold = fold_shared(a);
-  const bool few_down = per_pair && (a->I_shared == 0 || fold) && few_down_pays(a, fold);
-  const bool few_routed = per_pair && (a->I_shared == 0 || fold) && few_gate_up_takes(a);
+  const bool few = per_pair && (a->I_shared == 0 || fold) && quant_in_gemm_allowed();
+  const bool few_down = few && few_down_pays(a, fold);
+  const bool few_routed = few && few_gate_up_takes(a);
   RouteArgs route{logits, a->bias, M, Eg, K, a->renormalize, a->n_group, a->topk_group, a->routed_scale, topk_w, topk_ids};
   if (few_routed)
     rc = check_route(&route, a->scoring == KMOE_SCORE_SIGMOID);  // (the gate_up launch does it, and steps 2 and 3)
