@@ -12,6 +12,7 @@
 #include <algorithm>
 
 #include "buffer_ops.h"
+#include "few_rows.h"
 #include "formats.h"
 #include "kmoe_common.h"
 #include "quant_body.h"
@@ -43,7 +44,7 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
   constexpr int AV = W4 ? 4 : V;              // 16-byte vectors of activations per lane and step ...
   constexpr int kAVStride = W4 ? 16 : 64, kALane = W4 ? 64 : 16, kAStep = W4 ? 256 : 64 * V;
   constexpr int D = FMT == Fmt::F8 ? 4 : (few_wide_i8(FMT, kVecs) ? 12 : 8);  // steps in flight (a multiple of the four chains)
-  extern __shared__ __attribute__((aligned(16))) int8_t rows_lds[];  // [wave][row bytes + 16]
+  extern __shared__ __attribute__((aligned(16))) int8_t rows_lds[];  // [wave][few_row_pitch]
   __shared__ float y_lds[kFewMaxWaves][16];
   __shared__ float w_lds[kFewMaxWaves];
   const int lane = lane_id();
@@ -112,8 +113,7 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
     val[i].v = make_uint4(0, 0, 0, 0);
     if (lane + i * kWave < nvec) val[i].v = src[lane + i * kWave];
   }
-  const int row_bytes = p.I * (QUANT ? 1 : 2) + (FMT == Fmt::F8 ? p.I / 32 : 0);  // (F8: and the scales of its groups)
-  int8_t* mine = rows_lds + wave * (row_bytes + 16);
+  int8_t* mine = rows_lds + wave * few_row_pitch(p.I, QUANT ? 1 : 2, FMT == Fmt::F8);
   [[maybe_unused]] float* scales = reinterpret_cast<float*>(mine + p.I);
   float amax = 1.0f;
   if constexpr (FMT == Fmt::I8) {
@@ -241,10 +241,10 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
 template <Fmt FMT, int kVecs>
 int launch_few_down(const FewDown& p, hipStream_t s) {
   const int waves = p.K + (p.w_tail ? 1 : 0);
-  const int row_bytes = p.I * (FMT == Fmt::I8 || FMT == Fmt::F8 ? 1 : 2) + (FMT == Fmt::F8 ? p.I / 32 : 0);
+  const size_t bytes = static_cast<size_t>(waves) * few_row_pitch(p.I, FMT == Fmt::I8 || FMT == Fmt::F8 ? 1 : 2, FMT == Fmt::F8);
   if (tracing_kernels())
     note_kernel("few_down_kernel<%s>, %d waves: quantisation, down projection and combine of a token's 16 channels", fmt_name(FMT), waves);
-  hipLaunchKernelGGL((few_down_kernel<FMT, kVecs>), dim3(p.H / 16, p.M), dim3(waves * kWave), static_cast<size_t>(waves) * (row_bytes + 16), s, p);
+  hipLaunchKernelGGL((few_down_kernel<FMT, kVecs>), dim3(p.H / 16, p.M), dim3(waves * kWave), bytes, s, p);
   return check_launch("kmoe_moe_forward (down + combine)");
 }
 
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
   constexpr int kAVStride = W4 ? 16 : 64, kALane = W4 ? 64 : 16, kAStep = W4 ? 256 : 64 * V;
   constexpr int D = FMT == Fmt::F8 || W4 ? 2 : (FMT == Fmt::I8 ? 4 : 8);
   constexpr int kStepValues = W4 ? 128 : (QUANT ? 64 * V : 32);
-  extern __shared__ __attribute__((aligned(16))) int8_t lds[];  // sigmoid routing: [4][E] floats; then [M][row bytes + 16]
+  extern __shared__ __attribute__((aligned(16))) int8_t lds[];  // sigmoid routing: [4][E] floats; then [M][few_row_pitch]
   __shared__ float tw_lds[kFewRouted * kFewMaxWaves];
   __shared__ int32_t id_lds[kFewRouted * kFewMaxWaves];
   __shared__ uint32_t max_lds[kFewRouted][4];
@@ -389,8 +389,7 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- the rows: this wave's part of K, quantised (the quantisers' arithmetic) or as it is, into LDS ----
-  const int row_bytes = p.H * (QUANT ? 1 : 2) + (FMT == Fmt::F8 ? p.H / 32 : 0);
-  const int pitch = row_bytes + 16;
+  const int pitch = few_row_pitch(p.H, QUANT ? 1 : 2, FMT == Fmt::F8);
   int8_t* rows_lds = lds;
   const int v0 = kb0 * (kStepValues / 8), nvec = klen * (kStepValues / 8);  // vectors of 8 values
   float amax = 1.0f;
@@ -529,10 +528,9 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
 
 template <Fmt FMT, int SLOTS, bool SIGMOID>
 int launch_few_gate_up(const FewGateUp& p, hipStream_t s) {
-  const int H = p.H;
-  const int row_bytes = H * (FMT == Fmt::I8 || FMT == Fmt::F8 ? 1 : 2) + (FMT == Fmt::F8 ? H / 32 : 0);
+  const int pitch = few_row_pitch(p.H, FMT == Fmt::I8 || FMT == Fmt::F8 ? 1 : 2, FMT == Fmt::F8);
   // LDS: routing's copy of the scores, then the rows in its place
-  const size_t bytes = std::max(static_cast<size_t>(p.route.M) * (row_bytes + 16), SIGMOID ? sizeof(float) * 4 * p.route.E : 0);
+  const size_t bytes = std::max(static_cast<size_t>(p.route.M) * pitch, SIGMOID ? sizeof(float) * 4 * p.route.E : 0);
   if (tracing_kernels())
     note_kernel("few_gate_up_kernel<%s>: routing, quantisation, sort and gate_up of a pair's 16 channels", fmt_name(FMT));
   hipLaunchKernelGGL((few_gate_up_kernel<FMT, SLOTS, SIGMOID>), dim3(p.I / 16, p.route.M * p.route.K + (p.w_tail ? 1 : 0) + 1), dim3(4 * kWave), bytes, s, p);

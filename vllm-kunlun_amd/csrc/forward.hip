@@ -7,6 +7,7 @@
 #include <mutex>
 
 #include "asked_once.h"
+#include "few_rows.h"
 #include "kmoe_common.h"
 
 namespace kmoe {
@@ -239,9 +240,9 @@ bool few_down_pays(const kmoe_moe_args* a, bool fold) {
 // 1 token 18.9 / 16.4, 4 37.0 / 32.2, bf16 1 22.0 / 20.4, 4-bit 1 18.4 / 15.5, 4 27.2 / 24.7; DeepSeek-V3 dims int8 1 87.7 /
 // 78.5, with the gate 96.6 / 87.6, fp8 1 88.7 / 84.
 bool few_gate_up_takes(const kmoe_moe_args* a) {
-  if (a->M > kFewRouted || a->M * a->K > kWave || a->E > 8 * kWave) return false;
-  const long long row = bf16_activations(a->format) ? 2ll * a->H : a->H + a->H / 32;
-  if (a->M * (row + 16) > 25 * 1024) return false;
+  constexpr int kRows = 25 * 1024;  // bytes
+  if (a->M > kFewRouted || a->M * a->K > kWave || a->E > 8 * kWave || a->H > kRows) return false;
+  if (a->M * few_row_pitch(a->H, bf16_activations(a->format) ? 2 : 1, a->format == KMOE_FMT_FP8_BLOCK) > kRows) return false;
   for (const void* t : {static_cast<const void*>(a->x), static_cast<const void*>(a->w13), static_cast<const void*>(a->w13_max),
                         static_cast<const void*>(a->w13_scale), static_cast<const void*>(a->ws13), static_cast<const void*>(a->ws13_max)})
     if (reinterpret_cast<uintptr_t>(t) & 15) return false;
