@@ -259,6 +259,19 @@ def test_few_tokens_match_the_oracle(fmt, dtype, M, K, H, I):
     _check(sl, out)
 
 
+@pytest.mark.parametrize("fmt,I_shared", [("int8", 0), ("int8", 2048), ("fp8", 0), ("fp8", 2048), ("none", 0), ("w4", 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_most_rows_of_the_greatest_length(fmt, I_shared, dtype):
+    """Sixteen waves with rows of 2048 values, the most LDS the launch asks for (16-bit rows: more than 64 KB), against the oracle."""
+    from vllm_kunlun_amd import synth
+    base, K = ("dsv3-fp8-decode" if fmt == "fp8" else "dsv3-decode", 15) if I_shared else ("qwen3-decode", 16)
+    over = dict(I_shared=I_shared, n_group=1, topk_group=1) if I_shared else {}
+    sl = synth.make_layer(synth.scaled(synth.SHAPES[base], M=1, H=256, E=32, K=K, I=2048, quant=fmt, **over), "cuda", seed=K, dtype=dtype)
+    out, named = _named(lambda: _call(sl))
+    assert FUSED in named and "16 waves" in named, named
+    _check(sl, out)
+
+
 @pytest.mark.parametrize("variable", ["KMOE_QUANT_IN_GEMM", "KMOE_SORT_IN_GEMM"])
 def test_switches_keep_the_launches_apart(variable):
     """Each of them set to 0 (read once per process, hence a child process) gives a few-token layer its launches back: the output

@@ -238,6 +238,8 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
   }
 }
 
+// (the most rows there may be - 16 of 2048 16-bit values, 64.25 KB - fit a CU's 160 KB twice, with what the kernel holds besides)
+static_assert(kFewMaxWaves * few_row_pitch(kFewMaxI, 2, false) + kFewMaxWaves * 17 * 4 <= 80 * 1024);
 template <Fmt FMT, int kVecs>
 int launch_few_down(const FewDown& p, hipStream_t s) {
   const int waves = p.K + (p.w_tail ? 1 : 0);
