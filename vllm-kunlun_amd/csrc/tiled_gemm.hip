@@ -217,8 +217,10 @@ struct Tile {
 // m-tiles (int8: a few percent of time, the re-reads were mostly served by the memory-side cache; fp8: 14 %).
 // F16: the outputs, and the rounding of gate and up before SiLU-mul, are IEEE half instead of bf16 (int8 and
 // fp8 operands); with KIND = BF16 the operands are half as well (v_mfma_f32_16x16x32_f16).
+// PAST: the weights are read past the caches (buffer_stream_load16).
 template <TKind KIND, bool SWIGLU, int NF, int R, int WGS, int WM, bool M32 = false, int MF = 8, bool OAI = false,
-          bool PACE = false, bool F16 = false, int WN = kWavesT>
+          bool PACE = false, bool F16 = false, int WN = kWavesT,
+          bool PAST = (KIND != TKind::BF16 && NF == 4 && WM == 1 && MF <= 6 && !M32 && !PACE)>
 __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const TiledParams p) {
   constexpr int kWN = WN;  // waves side by side along the channels
   static_assert(!F16 || KIND != TKind::BF16 || !OAI, "the interleaved activation is a bf16 epilogue");
@@ -457,12 +459,11 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
   // Every load is unconditional (indices clamped to the last valid step / chunk, rows past a
   // tile's end read its first row, fragments past the last channel read fragment 0): the
   // results of those are never stored, and the loop body stays one basic block.
-  // The 64- and 96-row tiles run where nearly every expert has one m-tile: its weights are read once, past the caches (see
-  // buffer_stream_load16). GEMM alone, us, ordinary / past the caches: 64 experts of [4096 x 7168], 32 rows, int8 321 / 295, fp8 324 / 296;
-  // 128 experts of [1536 x 2048], 49 rows int8 77 / 72. Taller tiles have siblings that read the same bytes from L2 (512 rows,
+  // PAST (the 64-row tile where nearly every expert has one m-tile, see launch_short, and the 96-row one): weights are read once, past the
+  // caches (see buffer_stream_load16). GEMM alone, us, ordinary / past the caches: 64 experts of [4096 x 7168], 32 rows, int8 321 / 295, fp8
+  // 324 / 296; 128 experts of [1536 x 2048], 49 rows int8 77 / 72. Taller tiles have siblings that read the same bytes from L2 (512 rows,
   // int8 284 / 308), and so have the hot experts of an uneven load, which weigh most with 16-bit weights: bf16 900 tokens 246 / 233, but
   // 500 with +2.0 on the logits of 8 experts 236.4 / 237.0; those keep ordinary loads.
-  constexpr bool kPast = !BF && NF == 4 && WM == 1 && MF <= 6 && !M32 && !PACE;
   auto load_w = [&](v4i(&dst)[kNF], int kb) {
     const uint32_t off = static_cast<uint32_t>(min(kb, last_step)) * 1024u;
     if constexpr (M32) {
@@ -470,7 +471,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       for (int f = 0; f < kNF; ++f) dst[f] = buffer_load16(w_rsrc, woff[f >> 1], off + (f & 1) * 512u);
     } else {
 #pragma unroll
-      for (int f = 0; f < kNF; ++f) dst[f] = kPast ? buffer_stream_load16(w_rsrc, woff[f], off) : buffer_load16(w_rsrc, woff[f], off);
+      for (int f = 0; f < kNF; ++f) dst[f] = PAST ? buffer_stream_load16(w_rsrc, woff[f], off) : buffer_load16(w_rsrc, woff[f], off);
     }
   };
   auto load_a = [&](int chunk) {
@@ -1379,7 +1380,8 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
 }
 
 template <TKind KIND, bool SWIGLU, int NF, int R, int WGS, int WM, bool M32 = false, int MF = 8, bool OAI = false,
-          bool PACE = false, bool F16 = false, int WN = kWavesT>
+          bool PACE = false, bool F16 = false, int WN = kWavesT,
+          bool PAST = (KIND != TKind::BF16 && NF == 4 && WM == 1 && MF <= 6 && !M32 && !PACE)>
 int launch_tiled(TiledParams p, int rows, hipStream_t s, int n_cu, const char* what) {
   constexpr int kTM = WM * 16 * MF;
   const int n_half = SWIGLU ? p.n / 2 : p.n;
@@ -1393,14 +1395,14 @@ int launch_tiled(TiledParams p, int rows, hipStream_t s, int n_cu, const char* w
   const int grid = min(min(ceil_div(p.max_items, 8) * 8, ceil_div(WGS * n_cu, 8) * 8), kBoardSlots);
   const size_t dyn = sizeof(int) * (static_cast<size_t>(p.E) + 1 + n_exp + 2);
   if (tracing_kernels())
-    note_kernel("tiled_gemm_kernel<%s%s, %s, %dx%d tile, %d waves, %d per CU%s%s%s>%s",
+    note_kernel("tiled_gemm_kernel<%s%s, %s, %dx%d tile, %d waves, %d per CU%s%s%s%s>%s",
                 KIND == TKind::I8 ? "int8" : (KIND == TKind::F8 ? "fp8" : (F16 ? "f16" : "bf16")),
                 (KIND != TKind::BF16 && F16) ? " -> f16" : "", SWIGLU ? "SiLU-mul" : (OAI ? "swigluoai" : "plain"), kTM,
                 WN * nfh * 16 * (SWIGLU ? 2 : 1), WM * WN, WGS, M32 ? ", 32x32 MFMA" : "",
-                PACE ? ", paced siblings" : "", R != 4 ? ", 8-slot weight ring" : "",
+                PACE ? ", paced siblings" : "", R != 4 ? ", 8-slot weight ring" : "", PAST ? ", weights past the caches" : "",
                 p.pick == 1 ? " [works if few experts overflow the tile, decided on the device]"
                             : (p.pick == 2 ? " [works otherwise]" : ""));
-  hipLaunchKernelGGL((tiled_gemm_kernel<KIND, SWIGLU, NF, R, WGS, WM, M32, MF, OAI, PACE, F16, WN>), dim3(grid),
+  hipLaunchKernelGGL((tiled_gemm_kernel<KIND, SWIGLU, NF, R, WGS, WM, M32, MF, OAI, PACE, F16, WN, PAST>), dim3(grid),
                      dim3(WM * WN * kWave), dyn, s, p);
   return check_launch(what);
 }
@@ -1467,6 +1469,29 @@ bool short_tiles(int variant, int rows, int n_experts, int n, bool swiglu, int n
   if (ceil_div(rows, n_experts) <= max_avg_rows) return true;
   const int n_blocks = ceil_div(swiglu ? n / 2 : n, kWavesT * (swiglu ? 2 : 4) * 16);
   return static_cast<long long>(rows / 128 + n_experts) * n_blocks < 2ll * n_cu;
+}
+
+// The 64-row tile: its weights past the caches where nearly every expert has one (44 rows on average; see load_w). A launch of few tiles
+// whose experts have more rows (short_tiles) has several per expert, which read the same weights; and one matrix alone that the 256 MB
+// memory-side cache holds is likely a Linear's, which finds it there on its next call. us, all past the caches / as here, called again
+// at once; cold: int8 Linear [4096 x 7168] 600 rows 49.5 / 41.5; 50.3 / 50.4, 1500 94.2 / 64.6; 95.9 / 65.9, 3500 191 / 127; 195 / 135,
+// [7168 x 2048] 1500 rows 45.8 / 37.4; 47.8 / 39.6; fp8 GEMM alone, [4096 x 7168] 128 rows 55.8 / 50.8; 60.6 / 60.4, 2048 107.5 / 80.5; 111 /
+// 94.9, 8 experts, 100 rows each 67.7 / 55.8; 74.1 / 63.8; 64 experts, 32 rows each (ordinary / past the caches) 319 / 306; 321 / 308.
+template <TKind K>
+int launch_short(TiledParams& p, int rows, int live, hipStream_t s, int n_cu, const char* what, bool swiglu, bool f16) {
+  constexpr bool kMayPass = K != TKind::BF16;
+  if (kMayPass && ceil_div(live, p.E) <= 44 && (p.E > 1 || static_cast<long long>(p.n) * p.k > (256ll << 20))) {
+    if (f16)
+      return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, true, kWavesT, kMayPass>(p, rows, s, n_cu, what)
+                    : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, true, kWavesT, kMayPass>(p, rows, s, n_cu, what);
+    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, false, kWavesT, kMayPass>(p, rows, s, n_cu, what)
+                  : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, false, kWavesT, kMayPass>(p, rows, s, n_cu, what);
+  }
+  if (f16)
+    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, true, kWavesT, false>(p, rows, s, n_cu, what)
+                  : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, true, kWavesT, false>(p, rows, s, n_cu, what);
+  return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, false, kWavesT, false>(p, rows, s, n_cu, what)
+                : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, false, kWavesT, false>(p, rows, s, n_cu, what);
 }
 
 }  // namespace
@@ -1592,9 +1617,7 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
     if (paced)
       return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 8, false, true, true>(p, a->rows, s, n_cu, what)
                     : launch_tiled<K, false, 4, 4, 2, 1, false, 8, false, true, true>(p, a->rows, s, n_cu, what);
-    if (shorter)
-      return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what)
-                    : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what);
+    if (shorter) return launch_short<K>(p, a->rows, live, s, n_cu, what, swiglu, true);
     return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 8, false, false, true>(p, a->rows, s, n_cu, what)
                   : launch_tiled<K, false, 4, 4, 2, 1, false, 8, false, false, true>(p, a->rows, s, n_cu, what);
   }
@@ -1613,9 +1636,7 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   if (paced)
     return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 8, false, true>(p, a->rows, s, n_cu, what)
                   : launch_tiled<K, false, 4, 4, 2, 1, false, 8, false, true>(p, a->rows, s, n_cu, what);
-  if (shorter)
-    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4>(p, a->rows, s, n_cu, what)
-                  : launch_tiled<K, false, 4, 4, 2, 1, false, 4>(p, a->rows, s, n_cu, what);
+  if (shorter) return launch_short<K>(p, a->rows, live, s, n_cu, what, swiglu, false);
   return swiglu ? launch_tiled<K, true, 4, 4, 2, 1>(p, a->rows, s, n_cu, what)
                 : launch_tiled<K, false, 4, 4, 2, 1>(p, a->rows, s, n_cu, what);
 }
@@ -1637,13 +1658,7 @@ int tiled_gemm_fp8(const kmoe_gemm_fp8_args* a, hipStream_t s) {
   // still bound by what one workgroup keeps in flight; not instantiated)
   const bool half = a->act_dtype == KMOE_DT_F16;  // half outputs: the same three shapes
   const int live = expected_rows(a->rows, a->rows_hint);
-  if (short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu)) {
-    if (half)
-      return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what)
-                    : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what);
-    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4>(p, a->rows, s, n_cu, what)
-                  : launch_tiled<K, false, 4, 4, 2, 1, false, 4>(p, a->rows, s, n_cu, what);
-  }
+  if (short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu)) return launch_short<K>(p, a->rows, live, s, n_cu, what, swiglu, half);
   // (Paced sibling m-tiles - variant 12 - had been the default where experts have several m-tiles, the weights are
   // far more than the memory-side cache holds and a tile walks a long K. With an expert's rows split evenly over
   // its m-tiles the plain 128-row tiles are 2-4 % ahead of them at every batch: DeepSeek-V3 dims, layer at 2048 /
@@ -1728,7 +1743,8 @@ int tiled_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s) {
   p.bias = a->bias;
   p.oai_alpha = a->act_alpha;
   p.oai_limit = a->act_limit;
-  const bool shorter = short_tiles(a->variant, expected_rows(a->rows, a->rows_hint), a->E, a->n, swiglu, n_cu, 40);  // measured: at 48 rows per expert the 128-row tiles are 4 % ahead
+  const int live = expected_rows(a->rows, a->rows_hint);
+  const bool shorter = short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu, 40);  // measured: at 48 rows per expert the 128-row tiles are 4 % ahead
   if (a->act == KMOE_ACT_SWIGLUOAI)
     return shorter ? launch_tiled<K, false, 4, 4, 2, 1, false, 4, true>(p, a->rows, s, n_cu, what)
                    : launch_tiled<K, false, 4, 4, 2, 1, false, 8, true>(p, a->rows, s, n_cu, what);
@@ -1739,16 +1755,10 @@ int tiled_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s) {
   // 265, 1536: 288 / 290 / 265.7 / 277 / 285, 2048: 340 / 308 / 316 / 296 / 304, 3072: 423 / 379 / 352 / 386 / 347, 4096:
   // 514 / 451 / 427 / 443 / 458, 8192: 891 / 772 / 733 / 727 / 745. (128-row tiles that multiplied every fragment: 1024
   // 251, 2048 319, 4096 440, 8192 747.)
-  const float avg = static_cast<float>(ceil_div(expected_rows(a->rows, a->rows_hint), a->E));
+  const float avg = static_cast<float>(ceil_div(live, a->E));
   const float reach = avg + 3.0f * sqrtf(avg);
   const bool half = a->act_dtype == KMOE_DT_F16;  // half operands and results (no bias, no interleaved activation: checked by the caller)
-  if (shorter) {
-    if (half)
-      return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what)
-                    : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what);
-    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4>(p, a->rows, s, n_cu, what)
-                  : launch_tiled<K, false, 4, 4, 2, 1, false, 4>(p, a->rows, s, n_cu, what);
-  }
+  if (shorter) return launch_short<K>(p, a->rows, live, s, n_cu, what, swiglu, half);
   if (a->variant == 13 || (a->variant == 0 && reach <= 96.0f)) {
     if (half)
       return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 6, false, false, true>(p, a->rows, s, n_cu, what)
