@@ -201,25 +201,27 @@ def test_block_fp8_wide_tiles_need_four_blocks(variant, rows, blocks):
 
 
 @pytest.mark.parametrize("fmt", ["int8", "fp8"])
-@pytest.mark.parametrize("counts,past", [([44, 44, 44], True), ([3, 0, 129], True), ([45, 44, 44], False), ([300, 1], False), ([40], False), ([200], False)],
-                         ids=str)
+@pytest.mark.parametrize("counts", [[64, 1, 65, 130] * 16, [3, 0, 129, 640, 64], [1, 63], [40], [200]],
+                         ids=lambda c: "-".join(map(str, c[:5])))
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("act", [False, True])
-def test_64_row_tiles_read_weights_past_the_caches_where_an_expert_has_one(fmt, counts, past, dtype, act):
-    """Several experts with up to 44 rows on average; more rows, or one matrix alone: ordinary loads. The bits are the 128-row tiles'."""
+@pytest.mark.parametrize("k", [384, 640, 1024])  # whole and partial periods of the loop
+def test_64_row_tiles_read_what_one_tile_reads_past_the_caches(fmt, counts, dtype, act, k):
+    """Experts with one tile and with several in a launch, one after the other on the same workgroup too; one matrix alone. The
+    bits are the 128-row tiles'."""
     from vllm_kunlun_amd import _lib as L
-    gen = torch.Generator().manual_seed(sum(counts))
-    E, n, k, rows = len(counts), 256, 640, sum(counts)
+    gen = torch.Generator(device="cuda").manual_seed(sum(counts))
+    E, n, rows = len(counts), 2048, sum(counts)
     lod = torch.tensor([0] + counts).cumsum(0).int().cuda()
     if fmt == "int8":
         g, call = L.GemmI8Args(), L.lib.kmoe_grouped_gemm_i8
-        a, w = (torch.randint(-127, 128, shape, generator=gen, dtype=torch.int8).cuda() for shape in ((rows, k), (E, n, k)))
-        scales = [(torch.rand(shape, generator=gen) + 0.5).cuda() for shape in ((rows,), (E, n))]
+        a, w = (torch.randint(-127, 128, shape, generator=gen, dtype=torch.int8, device="cuda") for shape in ((rows, k), (E, n, k)))
+        scales = [torch.rand(shape, generator=gen, device="cuda") + 0.5 for shape in ((rows,), (E, n))]
         g.a_max, g.w_max = (t.data_ptr() for t in scales)
     else:
         g, call = L.GemmFp8Args(), L.lib.kmoe_grouped_gemm_fp8_block
-        a, w = (torch.randn(shape, generator=gen).to(torch.float8_e4m3fn).cuda() for shape in ((rows, k), (E, n, k)))
-        scales = [(torch.rand(shape, generator=gen) + 0.5).cuda() for shape in ((rows, k // 128), (E, n // 128, k // 128))]
+        a, w = (torch.randn(shape, generator=gen, device="cuda").to(torch.float8_e4m3fn) for shape in ((rows, k), (E, n, k)))
+        scales = [torch.rand(shape, generator=gen, device="cuda") + 0.5 for shape in ((rows, k // 128), (E, n // 128, k // 128))]
         g.a_scale, g.w_scale = (t.data_ptr() for t in scales)
     g.a, g.lda, g.src_div, g.w, g.w_layout, g.lod = a.data_ptr(), k, 1, w.data_ptr(), L.KMOE_W_TILED, lod.data_ptr()
     g.E, g.n, g.k, g.rows, g.act = E, n, k, rows, L.KMOE_ACT_SWIGLU if act else L.KMOE_ACT_NONE
@@ -231,5 +233,5 @@ def test_64_row_tiles_read_weights_past_the_caches_where_an_expert_has_one(fmt, 
         L.check(call(g, L.stream()))
         L.lib.kmoe_trace_kernels(0)
         out.append((y, L.lib.kmoe_traced_kernels().decode()))
-    assert "64x256 tile" in out[0][1] and ("weights past the caches" in out[0][1]) == past, out[0][1]
+    assert "64x256 tile" in out[0][1] and ("weights past the caches" in out[0][1]) == (E > 1), out[0][1]
     assert "128x256 tile" in out[1][1] and torch.equal(out[0][0], out[1][0])

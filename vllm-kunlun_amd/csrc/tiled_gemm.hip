@@ -165,6 +165,7 @@ struct TiledParams {
   // of one m-tile next to each other (they read the same rows at the same time) - for experts whose weights stay in an
   // XCD's L2 anyway, where an expert with many m-tiles would otherwise fetch its rows once per channel block.
   int32_t m_major;
+  int32_t past;  // 64-row PAST kernels: whether any weights are read past the caches
 };
 
 // Progress board of the persistent workgroups: slot b (64 bytes apart) holds where workgroup b is,
@@ -184,7 +185,7 @@ static __device__ uint32_t g_board[kBoardSlots * kBoardStride];  // word 0 of a 
 
 struct Tile {
   int it;    // position in this workgroup's list
-  int sib;   // bit 0: the item before is an m-tile of the same (expert, channel block); bit 1: the item after
+  int sib;   // bit 0: the item before is an m-tile of the same (expert, channel block); bit 1: the item after; bit 2 (kPerTile): the expert has several
   int e;     // expert (E = the tail expert)
   int row0;  // first sorted row
   int nb;    // channel block
@@ -217,11 +218,12 @@ struct Tile {
 // m-tiles (int8: a few percent of time, the re-reads were mostly served by the memory-side cache; fp8: 14 %).
 // F16: the outputs, and the rounding of gate and up before SiLU-mul, are IEEE half instead of bf16 (int8 and
 // fp8 operands); with KIND = BF16 the operands are half as well (v_mfma_f32_16x16x32_f16).
-// PAST: the weights are read past the caches (buffer_stream_load16).
+// PAST: weights that one tile alone reads are read past the caches (see load_w).
 template <TKind KIND, bool SWIGLU, int NF, int R, int WGS, int WM, bool M32 = false, int MF = 8, bool OAI = false,
           bool PACE = false, bool F16 = false, int WN = kWavesT,
           bool PAST = (KIND != TKind::BF16 && NF == 4 && WM == 1 && MF <= 6 && !M32 && !PACE)>
 __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const TiledParams p) {
+  constexpr bool kPerTile = PAST && MF == 4;  // the choice of loads is a tile's (see load_w)
   constexpr int kWN = WN;  // waves side by side along the channels
   static_assert(!F16 || KIND != TKind::BF16 || !OAI, "the interleaved activation is a bf16 epilogue");
   static_assert(!OAI || (KIND == TKind::BF16 && !SWIGLU && !M32), "the interleaved activation is a bf16 epilogue");
@@ -378,6 +380,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
     end = min(rows_end(e), row0 + stride);
     // siblings run on the workgroups before / after this one in the XCD, at the same list position
     const int j = blockIdx.x >> 3;
+    if constexpr (kPerTile) sib = mt > 1 ? 4 : 0;
     if (m > 0 && j > 0) sib |= 1;
     if (m + 1 < mt && j + 1 < per_xcd && lid + 1 < seg_end) sib |= 2;
   };
@@ -459,19 +462,24 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
   // Every load is unconditional (indices clamped to the last valid step / chunk, rows past a
   // tile's end read its first row, fragments past the last channel read fragment 0): the
   // results of those are never stored, and the loop body stays one basic block.
-  // PAST (the 64-row tile where nearly every expert has one m-tile, see launch_short, and the 96-row one): weights are read once, past the
+  // PAST, the 64- and 96-row tiles of int8 and fp8, which run where nearly every expert has one m-tile: its weights are read once, past the
   // caches (see buffer_stream_load16). GEMM alone, us, ordinary / past the caches: 64 experts of [4096 x 7168], 32 rows, int8 321 / 295, fp8
-  // 324 / 296; 128 experts of [1536 x 2048], 49 rows int8 77 / 72. Taller tiles have siblings that read the same bytes from L2 (512 rows,
-  // int8 284 / 308), and so have the hot experts of an uneven load, which weigh most with 16-bit weights: bf16 900 tokens 246 / 233, but
-  // 500 with +2.0 on the logits of 8 experts 236.4 / 237.0; those keep ordinary loads.
-  auto load_w = [&](v4i(&dst)[kNF], int kb) {
+  // 324 / 296; 128 experts of [1536 x 2048], 49 rows int8 77 / 72. Tiles of the same expert read the same bytes from L2 (taller tiles, 512
+  // rows, int8 284 / 308): in 64-row tiles an expert with several - a hot one of an uneven load, a shared expert, a dense matrix - keeps ordinary
+  // loads (past: what kind this is of). Layer, us, ordinary / past the caches all / as here, even; +2.0 on the logits of 8 experts: DeepSeek-V3
+  // dims int8 900 tokens 2047 / 1952 / 1917; 2100 / 2139 / 2056, 1300 2142 / 2084 / 2074; 2206 / 2304 / 2174, fp8 900 2053 / 2020 / 1967; 2150 /
+  // 2220 / 2127, 1300 2158 / 2165 / 2169; 2258 / 2416 / 2252; Qwen3 dims int8 600 145.3 / 137.9 / 139.2; 156.0 / 156.5 / 148.2. The choice is
+  // between two loops: a branch at each load cost Qwen3 dims 2.7 % and had fp8 spill. The 96-row tile has no registers for two (800 tokens
+  // 144 -> 172) and reads everything past the caches: 800 tokens 153.2 / 144.3; 157.6 / 155.1, 1000 158.6 / 149.7; 169.6 / 169.5. 16-bit weights keep
+  // ordinary loads in both (900 tokens 246 / 233, but 500 with hot experts 236.4 / 237.0).
+  auto load_w = [&](v4i(&dst)[kNF], int kb, auto past) {
     const uint32_t off = static_cast<uint32_t>(min(kb, last_step)) * 1024u;
     if constexpr (M32) {
 #pragma unroll
       for (int f = 0; f < kNF; ++f) dst[f] = buffer_load16(w_rsrc, woff[f >> 1], off + (f & 1) * 512u);
     } else {
 #pragma unroll
-      for (int f = 0; f < kNF; ++f) dst[f] = PAST ? buffer_stream_load16(w_rsrc, woff[f], off) : buffer_load16(w_rsrc, woff[f], off);
+      for (int f = 0; f < kNF; ++f) dst[f] = past ? buffer_stream_load16(w_rsrc, woff[f], off) : buffer_load16(w_rsrc, woff[f], off);
     }
   };
   auto load_a = [&](int chunk) {
@@ -956,6 +964,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
   int rs_scale = fetch_src(cur, cur.row0 + scale_row);
   float wsc_reg[kMaxKBlocks / 16];     // F8: weight block scales k = c, c + 16, ... of fragment lane / 16
 
+  auto reads_past = [&](const Tile& t) { return p.past && !(t.sib & 4); };
   // Points the loaders at tile t and requests its first chunk, first three weight steps and scales.
   auto start_tile = [&](const Tile& t, int t_parity) {
     const int8_t* w_base = t.e >= p.E ? p.w_tail : p.w + static_cast<size_t>(t.e) * p.n * p.k;
@@ -1003,8 +1012,13 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
                                                  0);
     }
     __builtin_amdgcn_sched_barrier(0);  // the weight loads below stay younger than the copies above (see the wait at the loop top)
+    auto first_steps = [&](auto past) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < R - 1; ++i) load_w(wring[i], i);
+      for (int i = 0; i < R - 1; ++i) load_w(wring[i], i, past);
+    };
+    if constexpr (!kPerTile) first_steps(std::bool_constant<PAST>{});
+    else if (reads_past(t)) first_steps(std::true_type{});
+    else first_steps(std::false_type{});
     if constexpr (F8) {
       if (wave_m == 0 && (lane >> 4) < kNF) {  // thread (wave, f = lane / 16, c = lane % 16): block scales c, c + 16, ...
         bool ok;
@@ -1103,7 +1117,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
     // (the counters retire in issue order, so a wait lets the later loads stay in flight).
     // keep_j0: all ones, or zero for the half chunk at the end of an odd number of steps (the leftover
     // chunks below pass it; in the main loop it is a constant).
-    auto chunk_step = [&](int c0, auto h_tag, auto keep_j0) {
+    auto chunk_step = [&](int c0, auto h_tag, auto keep_j0, auto past) {
       constexpr int h = decltype(h_tag)::value;
       constexpr int buf = ADMA ? h % kStagesA : h & 1;
       using buf_t = std::integral_constant<int, buf>;
@@ -1113,21 +1127,21 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       pace(cur.it, c0 + h);
       __builtin_amdgcn_sched_barrier(0);
       load_a(c0 + h + 1);
-      load_w(wring[(2 * h + R - 1) % R], s0 + R - 1);
+      load_w(wring[(2 * h + R - 1) % R], s0 + R - 1, past);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (F8 && ADMA) {
         compute_f8_dma(wring[(2 * h) % R], wring[(2 * h + 1) % R], buf_t{}, c0 + h, parity);
         __builtin_amdgcn_sched_barrier(0);
-        load_w(wring[(2 * h) % R], s0 + R);
+        load_w(wring[(2 * h) % R], s0 + R, past);
         dma_a(c0 + h + kStagesA - 1, (buf + kStagesA - 1) % kStagesA);
       } else if constexpr (F8) {
         compute_f8(wring[(2 * h) % R], wring[(2 * h + 1) % R], buf, c0 + h, parity);
         __builtin_amdgcn_sched_barrier(0);
-        load_w(wring[(2 * h) % R], s0 + R);
+        load_w(wring[(2 * h) % R], s0 + R, past);
       } else {
         compute(wring[(2 * h) % R], buf_t{}, j0_t{}, keep_j0);
         __builtin_amdgcn_sched_barrier(0);
-        load_w(wring[(2 * h) % R], s0 + R);
+        load_w(wring[(2 * h) % R], s0 + R, past);
         // the buffer chunk c - 1 was read from is free since the last barrier: chunk c + 3 goes there
         dma_a(c0 + h + kStagesA - 1, (buf + kStagesA - 1) % kStagesA);
         __builtin_amdgcn_sched_barrier(0);
@@ -1153,26 +1167,51 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
     constexpr int kPeriod = ADMA ? kStagesA : R / 2;  // chunks after which ring slots and buffers repeat
     static_assert(kPeriod == 2 || kPeriod == 4, "unrolled by hand below");
     constexpr std::false_type kFull{};
-    int c = 0;
-    for (; c + kPeriod <= nfull; c += kPeriod) {
-      chunk_step(c, std::integral_constant<int, 0>{}, kFull);
-      chunk_step(c, std::integral_constant<int, 1>{}, kFull);
-      if constexpr (kPeriod == 4) {
-        chunk_step(c, std::integral_constant<int, 2>{}, kFull);
-        chunk_step(c, std::integral_constant<int, 3>{}, kFull);
-      }
-    }
-    // the chunks left over (fewer than a period, the half chunk last): same steps, loads past the end are clamped
+    // (fewer chunks than a period are left over, the half chunk last: same steps, loads past the end are clamped)
     auto keep = [&](int chunk) {
       if constexpr (ADMA) return (half_chunk && chunk == nfull) ? 0 : -1;
       else return kFull;
     };
-    if (c < nchunks) chunk_step(c, std::integral_constant<int, 0>{}, keep(c));
-    if constexpr (kPeriod == 4) {
-      if (c + 1 < nchunks) chunk_step(c, std::integral_constant<int, 1>{}, keep(c + 1));
-      if (c + 2 < nchunks) chunk_step(c, std::integral_constant<int, 2>{}, keep(c + 2));
-      if constexpr (ADMA) {
-        if (c + 3 < nchunks) chunk_step(c, std::integral_constant<int, 3>{}, keep(c + 3));
+    if constexpr (kPerTile) {
+      auto all_chunks = [&](auto past) __attribute__((always_inline)) {
+        int c = 0;
+        for (; c + kPeriod <= nfull; c += kPeriod) {
+          chunk_step(c, std::integral_constant<int, 0>{}, kFull, past);
+          chunk_step(c, std::integral_constant<int, 1>{}, kFull, past);
+          if constexpr (kPeriod == 4) {
+            chunk_step(c, std::integral_constant<int, 2>{}, kFull, past);
+            chunk_step(c, std::integral_constant<int, 3>{}, kFull, past);
+          }
+        }
+        if (c < nchunks) chunk_step(c, std::integral_constant<int, 0>{}, keep(c), past);
+        if constexpr (kPeriod == 4) {
+          if (c + 1 < nchunks) chunk_step(c, std::integral_constant<int, 1>{}, keep(c + 1), past);
+          if (c + 2 < nchunks) chunk_step(c, std::integral_constant<int, 2>{}, keep(c + 2), past);
+          if constexpr (ADMA) {
+            if (c + 3 < nchunks) chunk_step(c, std::integral_constant<int, 3>{}, keep(c + 3), past);
+          }
+        }
+      };
+      if (reads_past(cur)) all_chunks(std::true_type{});
+      else all_chunks(std::false_type{});
+    } else {  // (the same written out: called, it left the wide tiles with other registers and 0.5 to 1 % slower)
+      constexpr std::bool_constant<PAST> past{};
+      int c = 0;
+      for (; c + kPeriod <= nfull; c += kPeriod) {
+        chunk_step(c, std::integral_constant<int, 0>{}, kFull, past);
+        chunk_step(c, std::integral_constant<int, 1>{}, kFull, past);
+        if constexpr (kPeriod == 4) {
+          chunk_step(c, std::integral_constant<int, 2>{}, kFull, past);
+          chunk_step(c, std::integral_constant<int, 3>{}, kFull, past);
+        }
+      }
+      if (c < nchunks) chunk_step(c, std::integral_constant<int, 0>{}, keep(c), past);
+      if constexpr (kPeriod == 4) {
+        if (c + 1 < nchunks) chunk_step(c, std::integral_constant<int, 1>{}, keep(c + 1), past);
+        if (c + 2 < nchunks) chunk_step(c, std::integral_constant<int, 2>{}, keep(c + 2), past);
+        if constexpr (ADMA) {
+          if (c + 3 < nchunks) chunk_step(c, std::integral_constant<int, 3>{}, keep(c + 3), past);
+        }
       }
     }
 
@@ -1399,7 +1438,7 @@ int launch_tiled(TiledParams p, int rows, hipStream_t s, int n_cu, const char* w
                 KIND == TKind::I8 ? "int8" : (KIND == TKind::F8 ? "fp8" : (F16 ? "f16" : "bf16")),
                 (KIND != TKind::BF16 && F16) ? " -> f16" : "", SWIGLU ? "SiLU-mul" : (OAI ? "swigluoai" : "plain"), kTM,
                 WN * nfh * 16 * (SWIGLU ? 2 : 1), WM * WN, WGS, M32 ? ", 32x32 MFMA" : "",
-                PACE ? ", paced siblings" : "", R != 4 ? ", 8-slot weight ring" : "", PAST ? ", weights past the caches" : "",
+                PACE ? ", paced siblings" : "", R != 4 ? ", 8-slot weight ring" : "", PAST && (MF == 6 || p.past) ? ", lone tiles' weights past the caches" : "",
                 p.pick == 1 ? " [works if few experts overflow the tile, decided on the device]"
                             : (p.pick == 2 ? " [works otherwise]" : ""));
   hipLaunchKernelGGL((tiled_gemm_kernel<KIND, SWIGLU, NF, R, WGS, WM, M32, MF, OAI, PACE, F16, WN, PAST>), dim3(grid),
@@ -1471,27 +1510,18 @@ bool short_tiles(int variant, int rows, int n_experts, int n, bool swiglu, int n
   return static_cast<long long>(rows / 128 + n_experts) * n_blocks < 2ll * n_cu;
 }
 
-// The 64-row tile: its weights past the caches where nearly every expert has one (44 rows on average; see load_w). A launch of few tiles
-// whose experts have more rows (short_tiles) has several per expert, which read the same weights; and one matrix alone that the 256 MB
-// memory-side cache holds is likely a Linear's, which finds it there on its next call. us, all past the caches / as here, called again
-// at once; cold: int8 Linear [4096 x 7168] 600 rows 49.5 / 41.5; 50.3 / 50.4, 1500 94.2 / 64.6; 95.9 / 65.9, 3500 191 / 127; 195 / 135,
-// [7168 x 2048] 1500 rows 45.8 / 37.4; 47.8 / 39.6; fp8 GEMM alone, [4096 x 7168] 128 rows 55.8 / 50.8; 60.6 / 60.4, 2048 107.5 / 80.5; 111 /
-// 94.9, 8 experts, 100 rows each 67.7 / 55.8; 74.1 / 63.8; 64 experts, 32 rows each (ordinary / past the caches) 319 / 306; 321 / 308.
+// The 64-row tile. One matrix alone that the 256 MB memory-side cache holds is likely a Linear's, which finds it there on its next
+// call: ordinary loads also where a single tile reads it. us, all past the caches / as here and in load_w, called again at once;
+// cold: int8 Linear [4096 x 7168] 600 rows 49.5 / 41.5; 50.3 / 50.4, 1500 94.2 / 64.6; 95.9 / 65.9, 3500 191 / 127; 195 / 135; fp8 GEMM alone,
+// [4096 x 7168] 2048 rows 107.5 / 80.5; 111 / 94.9, 8 experts, 100 rows each 67.7 / 55.8; 74.1 / 63.8.
 template <TKind K>
-int launch_short(TiledParams& p, int rows, int live, hipStream_t s, int n_cu, const char* what, bool swiglu, bool f16) {
-  constexpr bool kMayPass = K != TKind::BF16;
-  if (kMayPass && ceil_div(live, p.E) <= 44 && (p.E > 1 || static_cast<long long>(p.n) * p.k > (256ll << 20))) {
-    if (f16)
-      return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, true, kWavesT, kMayPass>(p, rows, s, n_cu, what)
-                    : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, true, kWavesT, kMayPass>(p, rows, s, n_cu, what);
-    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, false, kWavesT, kMayPass>(p, rows, s, n_cu, what)
-                  : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, false, kWavesT, kMayPass>(p, rows, s, n_cu, what);
-  }
+int launch_short(TiledParams& p, int rows, hipStream_t s, int n_cu, const char* what, bool swiglu, bool f16) {
+  p.past = p.E > 1 || static_cast<long long>(p.n) * p.k > (256ll << 20);
   if (f16)
-    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, true, kWavesT, false>(p, rows, s, n_cu, what)
-                  : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, true, kWavesT, false>(p, rows, s, n_cu, what);
-  return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, false, kWavesT, false>(p, rows, s, n_cu, what)
-                : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, false, kWavesT, false>(p, rows, s, n_cu, what);
+    return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4, false, false, true>(p, rows, s, n_cu, what)
+                  : launch_tiled<K, false, 4, 4, 2, 1, false, 4, false, false, true>(p, rows, s, n_cu, what);
+  return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 4>(p, rows, s, n_cu, what)
+                : launch_tiled<K, false, 4, 4, 2, 1, false, 4>(p, rows, s, n_cu, what);
 }
 
 }  // namespace
@@ -1617,7 +1647,7 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
     if (paced)
       return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 8, false, true, true>(p, a->rows, s, n_cu, what)
                     : launch_tiled<K, false, 4, 4, 2, 1, false, 8, false, true, true>(p, a->rows, s, n_cu, what);
-    if (shorter) return launch_short<K>(p, a->rows, live, s, n_cu, what, swiglu, true);
+    if (shorter) return launch_short<K>(p, a->rows, s, n_cu, what, swiglu, true);
     return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 8, false, false, true>(p, a->rows, s, n_cu, what)
                   : launch_tiled<K, false, 4, 4, 2, 1, false, 8, false, false, true>(p, a->rows, s, n_cu, what);
   }
@@ -1636,7 +1666,7 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   if (paced)
     return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 8, false, true>(p, a->rows, s, n_cu, what)
                   : launch_tiled<K, false, 4, 4, 2, 1, false, 8, false, true>(p, a->rows, s, n_cu, what);
-  if (shorter) return launch_short<K>(p, a->rows, live, s, n_cu, what, swiglu, false);
+  if (shorter) return launch_short<K>(p, a->rows, s, n_cu, what, swiglu, false);
   return swiglu ? launch_tiled<K, true, 4, 4, 2, 1>(p, a->rows, s, n_cu, what)
                 : launch_tiled<K, false, 4, 4, 2, 1>(p, a->rows, s, n_cu, what);
 }
@@ -1658,7 +1688,7 @@ int tiled_gemm_fp8(const kmoe_gemm_fp8_args* a, hipStream_t s) {
   // still bound by what one workgroup keeps in flight; not instantiated)
   const bool half = a->act_dtype == KMOE_DT_F16;  // half outputs: the same three shapes
   const int live = expected_rows(a->rows, a->rows_hint);
-  if (short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu)) return launch_short<K>(p, a->rows, live, s, n_cu, what, swiglu, half);
+  if (short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu)) return launch_short<K>(p, a->rows, s, n_cu, what, swiglu, half);
   // (Paced sibling m-tiles - variant 12 - had been the default where experts have several m-tiles, the weights are
   // far more than the memory-side cache holds and a tile walks a long K. With an expert's rows split evenly over
   // its m-tiles the plain 128-row tiles are 2-4 % ahead of them at every batch: DeepSeek-V3 dims, layer at 2048 /
@@ -1758,7 +1788,7 @@ int tiled_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s) {
   const float avg = static_cast<float>(ceil_div(live, a->E));
   const float reach = avg + 3.0f * sqrtf(avg);
   const bool half = a->act_dtype == KMOE_DT_F16;  // half operands and results (no bias, no interleaved activation: checked by the caller)
-  if (shorter) return launch_short<K>(p, a->rows, live, s, n_cu, what, swiglu, half);
+  if (shorter) return launch_short<K>(p, a->rows, s, n_cu, what, swiglu, half);
   if (a->variant == 13 || (a->variant == 0 && reach <= 96.0f)) {
     if (half)
       return swiglu ? launch_tiled<K, true, 4, 4, 2, 1, false, 6, false, false, true>(p, a->rows, s, n_cu, what)
