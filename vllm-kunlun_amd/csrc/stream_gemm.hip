@@ -191,6 +191,9 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
   // caches always / past them on an expert's last pass: 64 tokens 127 / 130 / 115 us, 140 tokens 182 / 203 / 163. Nor where another
   // workgroup reads them: the slices of a tail expert. DeepSeek-V3 dims, layer with all slices past the caches / none: int8 23 tokens
   // 838.7 / 831.7 us, 64 1462 / 1449, 128 1652 / 1630; fp8 23 843.9 / 835.2, 128 1663 / 1647, 250 1812 / 1781; 8 tokens (one slice) level.
+  // (A single layer called again and again, of which the 256 MB memory-side cache holds what a batch hits, is faster with ordinary loads,
+  // among other layers it is not. Qwen3 dims, layer with ordinary loads / past the caches, called again at once; cold: 4-bit 8 tokens
+  // 41.9 / 43.7; 48.4 / 47.0, 16 55.6 / 61.2; 66.7 / 64.6, int8 8 49.1 / 50.9; 58.6 / 57.5.)
   const bool slices = tail && p.tail_rows > TM;
   bool once = !slices;
   auto load_w_step = [&](int slot, int kb) {

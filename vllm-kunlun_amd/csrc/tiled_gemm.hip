@@ -165,7 +165,7 @@ struct TiledParams {
   // of one m-tile next to each other (they read the same rows at the same time) - for experts whose weights stay in an
   // XCD's L2 anyway, where an expert with many m-tiles would otherwise fetch its rows once per channel block.
   int32_t m_major;
-  int32_t past;  // 64-row PAST kernels: whether any weights are read past the caches
+  int32_t past;  // 64-row tiles of int8 and fp8: whether any weights are read past the caches
 };
 
 // Progress board of the persistent workgroups: slot b (64 bytes apart) holds where workgroup b is,
@@ -193,6 +193,9 @@ struct Tile {
   bool valid;
 };
 
+// Tiles that run where nearly every expert has one, of formats that gain from reading its weights past the caches (see load_w).
+constexpr bool past_tile(TKind kind, int NF, int WM, int MF) { return kind != TKind::BF16 && NF == 4 && WM == 1 && MF <= 6; }
+
 // NF: 16-channel fragments per wave (4: 256-channel tiles, 2: 128-channel tiles);
 // R: weight ring slots (R - 1 MFMA steps of weights in flight per wave), 4 or 8;
 // WGS: workgroups per CU the register budget is cut for.
@@ -218,12 +221,11 @@ struct Tile {
 // m-tiles (int8: a few percent of time, the re-reads were mostly served by the memory-side cache; fp8: 14 %).
 // F16: the outputs, and the rounding of gate and up before SiLU-mul, are IEEE half instead of bf16 (int8 and
 // fp8 operands); with KIND = BF16 the operands are half as well (v_mfma_f32_16x16x32_f16).
-// PAST: weights that one tile alone reads are read past the caches (see load_w).
 template <TKind KIND, bool SWIGLU, int NF, int R, int WGS, int WM, bool M32 = false, int MF = 8, bool OAI = false,
-          bool PACE = false, bool F16 = false, int WN = kWavesT,
-          bool PAST = (KIND != TKind::BF16 && NF == 4 && WM == 1 && MF <= 6 && !M32 && !PACE)>
+          bool PACE = false, bool F16 = false, int WN = kWavesT>
 __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const TiledParams p) {
-  constexpr bool kPerTile = PAST && MF == 4;  // the choice of loads is a tile's (see load_w)
+  constexpr bool kPast = past_tile(KIND, NF, WM, MF) && !M32 && !PACE;  // weights that one tile alone reads: past the caches (see load_w)
+  constexpr bool kPerTile = kPast && MF == 4;
   constexpr int kWN = WN;  // waves side by side along the channels
   static_assert(!F16 || KIND != TKind::BF16 || !OAI, "the interleaved activation is a bf16 epilogue");
   static_assert(!OAI || (KIND == TKind::BF16 && !SWIGLU && !M32), "the interleaved activation is a bf16 epilogue");
@@ -462,7 +464,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
   // Every load is unconditional (indices clamped to the last valid step / chunk, rows past a
   // tile's end read its first row, fragments past the last channel read fragment 0): the
   // results of those are never stored, and the loop body stays one basic block.
-  // PAST, the 64- and 96-row tiles of int8 and fp8, which run where nearly every expert has one m-tile: its weights are read once, past the
+  // kPast, the 64- and 96-row tiles of int8 and fp8, which run where nearly every expert has one m-tile: its weights are read once, past the
   // caches (see buffer_stream_load16). GEMM alone, us, ordinary / past the caches: 64 experts of [4096 x 7168], 32 rows, int8 321 / 295, fp8
   // 324 / 296; 128 experts of [1536 x 2048], 49 rows int8 77 / 72. Tiles of the same expert read the same bytes from L2 (taller tiles, 512
   // rows, int8 284 / 308): in 64-row tiles an expert with several - a hot one of an uneven load, a shared expert, a dense matrix - keeps ordinary
@@ -1016,7 +1018,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
 #pragma unroll
       for (int i = 0; i < R - 1; ++i) load_w(wring[i], i, past);
     };
-    if constexpr (!kPerTile) first_steps(std::bool_constant<PAST>{});
+    if constexpr (!kPerTile) first_steps(std::bool_constant<kPast>{});
     else if (reads_past(t)) first_steps(std::true_type{});
     else first_steps(std::false_type{});
     if constexpr (F8) {
@@ -1195,7 +1197,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
       if (reads_past(cur)) all_chunks(std::true_type{});
       else all_chunks(std::false_type{});
     } else {  // (the same written out: called, it left the wide tiles with other registers and 0.5 to 1 % slower)
-      constexpr std::bool_constant<PAST> past{};
+      constexpr std::bool_constant<kPast> past{};
       int c = 0;
       for (; c + kPeriod <= nfull; c += kPeriod) {
         chunk_step(c, std::integral_constant<int, 0>{}, kFull, past);
@@ -1419,8 +1421,7 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
 }
 
 template <TKind KIND, bool SWIGLU, int NF, int R, int WGS, int WM, bool M32 = false, int MF = 8, bool OAI = false,
-          bool PACE = false, bool F16 = false, int WN = kWavesT,
-          bool PAST = (KIND != TKind::BF16 && NF == 4 && WM == 1 && MF <= 6 && !M32 && !PACE)>
+          bool PACE = false, bool F16 = false, int WN = kWavesT>
 int launch_tiled(TiledParams p, int rows, hipStream_t s, int n_cu, const char* what) {
   constexpr int kTM = WM * 16 * MF;
   const int n_half = SWIGLU ? p.n / 2 : p.n;
@@ -1438,10 +1439,10 @@ int launch_tiled(TiledParams p, int rows, hipStream_t s, int n_cu, const char* w
                 KIND == TKind::I8 ? "int8" : (KIND == TKind::F8 ? "fp8" : (F16 ? "f16" : "bf16")),
                 (KIND != TKind::BF16 && F16) ? " -> f16" : "", SWIGLU ? "SiLU-mul" : (OAI ? "swigluoai" : "plain"), kTM,
                 WN * nfh * 16 * (SWIGLU ? 2 : 1), WM * WN, WGS, M32 ? ", 32x32 MFMA" : "",
-                PACE ? ", paced siblings" : "", R != 4 ? ", 8-slot weight ring" : "", PAST && (MF == 6 || p.past) ? ", lone tiles' weights past the caches" : "",
+                PACE ? ", paced siblings" : "", R != 4 ? ", 8-slot weight ring" : "", past_tile(KIND, NF, WM, MF) && !M32 && !PACE && (MF == 6 || p.past) ? ", weights past the caches" : "",
                 p.pick == 1 ? " [works if few experts overflow the tile, decided on the device]"
                             : (p.pick == 2 ? " [works otherwise]" : ""));
-  hipLaunchKernelGGL((tiled_gemm_kernel<KIND, SWIGLU, NF, R, WGS, WM, M32, MF, OAI, PACE, F16, WN, PAST>), dim3(grid),
+  hipLaunchKernelGGL((tiled_gemm_kernel<KIND, SWIGLU, NF, R, WGS, WM, M32, MF, OAI, PACE, F16, WN>), dim3(grid),
                      dim3(WM * WN * kWave), dyn, s, p);
   return check_launch(what);
 }
