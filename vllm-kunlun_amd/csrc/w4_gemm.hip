@@ -156,6 +156,9 @@ constexpr int w4_ring(int MF) { return MF == 6 ? 3 : 2; }
 // PAST: the weights are read past the caches (see buffer_stream_load16), where nearly every expert has one m-tile: always at 16 and 32
 // rows, at 64 rows up to 50 rows per expert. Layer, us, ordinary / past the caches: Qwen3 dims 128 tokens 78.8 / 75.9, cold 84.0 / 79.8,
 // Kimi-K2 dims 64 tokens 1232 / 1191, 2048 2418 / 2390; with several tiles per expert their siblings miss: Qwen3 dims 2048 tokens 238 / 247.
+// (A hot expert's tiles do, too: Kimi-K2 dims, +2.0 on the logits of 8 experts, 1000 tokens 2120 / 2135, 2000 2639 / 2666, but 400 1799 / 1779. A
+// choice per tile between two loops, as the tile kernel of the other formats has, took 2627 at 2000, but more elsewhere: 400 even 1623 -> 1677,
+// Qwen3 dims, 400 with hot experts 111 -> 119.)
 template <int MF, bool SWIGLU, bool F16, bool PAST>
 __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kernel(const W4Params p) {
   constexpr int NF = 4, R = w4_ring(MF);
