@@ -323,7 +323,7 @@ int kmoe_grouped_gemm_i8(const kmoe_gemm_i8_args* args, kmoe_stream_t stream);
  * per token, then matmul): kmoe_quant_i8_rows_dt and the product above with one matrix, the same bits.
  *   y[r,c] = round( float(acc) * (x_max[r]/127) * (w_max[c]/127) ),  acc over the codes of x's rows.
  * lod == NULL: a kernel of tiles that split K over a workgroup's waves, ahead for up to kmoe_linear_i8_split_rows(n, k)
- * rows (tiled weights; up to 4 rows are quantised in its own launch); any number of rows with rows * k below
+ * rows (tiled weights; up to 4 rows, of a very wide matrix one, are quantised in its own launch); any number of rows with rows * k below
  * 0xfff00000 is computed. Else lod is the row range {0, rows} (device)
  * and the rows go to kmoe_grouped_gemm_i8 as one expert's.
  */

@@ -41,10 +41,10 @@ def test_dense_slices(rows, n, k):
     assert np.array_equal(bits(out), ref)
 
 
-# up to four rows are quantised by the GEMM's own launch, five are not; one channel fragment per workgroup and two, K up to
+# up to four rows are quantised by the GEMM's own launch, five are not, and of a matrix of more than two workgroups per CU only one; one channel fragment per workgroup and two, K up to
 # the most it takes and beyond, rows of zeros and of one tiny value
 @pytest.mark.parametrize("rows", [1, 2, 3, 4, 5])
-@pytest.mark.parametrize("n,k", [(16, 64), (4096, 576), (4112, 640), (80, 8192), (48, 8256)])
+@pytest.mark.parametrize("n,k", [(16, 64), (4096, 576), (4112, 640), (80, 8192), (48, 8256), (16384, 64), (16400, 64)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_rows_quantised_in_the_launch(rows, n, k, dtype):
     from vllm_kunlun_amd import _lib as L
@@ -58,7 +58,7 @@ def test_rows_quantised_in_the_launch(rows, n, k, dtype):
     out = kern.apply_weights(layer, x.cuda())
     named = L.lib.kmoe_traced_kernels().decode()
     L.lib.kmoe_trace_kernels(0)
-    assert ("quantises its rows itself" in named) == (rows <= 4 and k <= 8192), named
+    assert ("quantises its rows itself" in named) == (rows <= (4 if n <= 16384 else 1) and k <= 8192), named
     xq, x_max = co.quant_i8_rows(bits(x), f16=f16)
     ref, _ = co.grouped_gemm_i8(xq, x_max, codes.numpy()[None], w_max.numpy()[None], np.array([0, rows], np.int32), f16=f16)
     assert np.array_equal(bits(out), ref)

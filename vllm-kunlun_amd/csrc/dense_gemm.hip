@@ -43,7 +43,12 @@ struct DenseParams {
 };
 
 constexpr int kDenseWaves = 8;
-constexpr int kQuantCost = 12;  // (dense_cost) beyond, too many workgroups quantise the same rows
+// Whether the GEMM's launch quantises a few rows itself: every workgroup does, so a second row wants all of them on the chip at once, two
+// per CU, and one row a launch of a few rounds (kQuantCost). With the quantiser's launch / in the GEMM's, us, called again at once; cold:
+// [4096 x 7168] 1 row 11.9 / 8.5; 14.1 / 11.6, 4 rows 11.1 / 9.9; 14.4 / 16.3, [14336 x 4096] (448 workgroups) 1 13.8 / 11.5; 17.6 / 14.7, 4 13.8 /
+// 14.3; 17.7 / 17.7, [8192 x 8192] 4 16.2 / 17.2; 20.5 / 21.8; and beyond: [12288 x 5120] (768) 1 14.6 / 14.0; 18.8 / 17.9, 2 14.5 / 17.2; 18.8 / 20.9,
+// 4 14.8 / 22.4; 19.1 / 26.6, [10240 x 8192] (640) 4 18.4 / 25.0; 24.3 / 29.6, [24576 x 1536] (768) 1 11.6 / 9.6; 15.1 / 13.3, 4 12.0 / 14.8; 15.5 / 19.2.
+constexpr int kQuantCost = 12, kQuantPerCu = 2;
 constexpr int kQuantRows = 4, kQuantMaxK = 8192;  // QUANT: rows, and the values a lane holds of each (two vectors of 8)
 
 // D: MFMA steps in flight; WPS: waves per SIMD the registers are cut for (4: two workgroups on a CU).
@@ -337,7 +342,8 @@ extern "C" int kmoe_linear_i8(const kmoe_linear_i8_args* a, kmoe_stream_t stream
   if (a->rows <= kQuantRows && a->k <= kQuantMaxK && aligned(a->x, 16)) {
     int n_cu = 0, shape = 0;
     if (int rc = compute_units(&n_cu)) return rc;
-    if (dense_cost(a->n, a->rows, n_cu, &shape) <= kQuantCost) {
+    const int cost = dense_cost(a->n, a->rows, n_cu, &shape);
+    if (cost <= kQuantCost && (a->rows == 1 || ceil_div(a->n, 16 * kDenseShapes[shape].nf) <= kQuantPerCu * n_cu)) {
       DenseParams p = {};
       p.x = a->x;
       p.ld_x = a->ld_x;

@@ -10,7 +10,7 @@ few pieces of that base it relies on (the parameter names and what the base's
 
 Path taken by `apply_weights`: per-token absmax int8 quantisation and the int8 GEMM in one library call
 (`kmoe_linear_i8`) on the weights re-arranged at load time into the MFMA tiles - up to a number of rows that
-depends on the matrix (`_DynamicCall`) on a kernel whose waves split K, which quantises up to four rows itself, beyond as the
+depends on the matrix (`_DynamicCall`) on a kernel whose waves split K, which quantises up to four rows (of very wide matrices one) itself, beyond as the
 one-expert case of the tile kernel the fused MoE layer's prefill batches run on.
 """
 from __future__ import annotations
