@@ -1,0 +1,49 @@
+"""Routing where scores are equal: the way that ranks distinct keys gives up and the one that goes by expert id takes over,
+per token; against the oracle, for every slot count, the most experts per token and every group size the lanes hold."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from oracle import c_oracle as co  # noqa: E402
+
+
+def _logits(M, E, seed):
+    """Every other token's logits on a grid of eight values, so that the chosen ones repeat; the others' distinct."""
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((M, E)).astype(np.float32)
+    x[::2] = np.clip(np.round(x[::2] * 2) / 2, -1.5, 2)
+    return x
+
+
+def _run(call, M, K):
+    w = torch.empty(M, K, dtype=torch.float32, device="cuda")
+    ids = torch.empty(M, K, dtype=torch.int32, device="cuda")
+    call(w, ids)
+    return ids.cpu().numpy(), w.cpu().numpy().view(np.uint32)
+
+
+@pytest.mark.parametrize("E,K", [(2, 1), (17, 16), (63, 63), (64, 63), (64, 64), (100, 8), (128, 63), (130, 64), (512, 10), (1024, 63)])
+def test_softmax_routing_of_equal_scores(E, K):
+    from vllm_kunlun_amd import _lib as L
+    M = 13
+    logits = _logits(M, E, E + K)
+    w_ref, ids_ref = co.softmax_topk(logits, K, 1)
+    d = torch.from_numpy(logits).cuda()
+    ids, w = _run(lambda w, i: L.check(L.lib.kmoe_softmax_topk(L.ptr(d), M, E, K, 1, L.ptr(w), L.ptr(i), L.stream())), M, K)
+    assert np.array_equal(ids, ids_ref) and np.array_equal(w, w_ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("gsize", [2, 4, 8, 16, 32, 64, 12])
+@pytest.mark.parametrize("n_group", [2, 8, 15])
+def test_group_routing_of_equal_scores(gsize, n_group):
+    from vllm_kunlun_amd import _lib as L
+    M, E, tg = 9, gsize * n_group, (n_group + 1) // 2
+    K = min(8, tg * gsize)
+    logits = _logits(M, E, E)
+    w_ref, ids_ref = co.sigmoid_group_topk_norm(logits, None, K, n_group, tg, 2.5)
+    d = torch.from_numpy(logits).cuda()
+    ids, w = _run(lambda w, i: L.check(L.lib.kmoe_sigmoid_group_topk_norm(L.ptr(d), None, M, E, K, n_group, tg, 2.5, L.ptr(w), L.ptr(i),
+                                                                          L.stream())), M, K)
+    assert np.array_equal(ids, ids_ref) and np.array_equal(w, w_ref.view(np.uint32))

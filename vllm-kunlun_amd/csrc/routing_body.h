@@ -9,46 +9,120 @@ namespace kmoe {
 constexpr int kMaxSlots = 16;  // E <= 1024
 constexpr int kWavesPerBlock = 4;
 
-// Largest of a 32-bit value over the 64 lanes, in a scalar register: four DPP steps leave every 16-lane row with its
-// own maximum, four lane reads and three scalar maxima do the rest.
-__device__ inline uint32_t wave_max_u32(uint32_t v) {
-  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xf, 0xf, true)));   // quad_perm [1,0,3,2]
-  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xf, 0xf, true)));   // quad_perm [2,3,0,1]
-  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xf, 0xf, true)));  // row_half_mirror
-  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xf, 0xf, true)));  // row_mirror
-  const uint32_t a = __builtin_amdgcn_readlane(v, 0), b = __builtin_amdgcn_readlane(v, 16);
-  const uint32_t c = __builtin_amdgcn_readlane(v, 32), d = __builtin_amdgcn_readlane(v, 48);
-  return max(max(a, b), max(c, d));
+// Where scores are 16-bit values their patterns' 16 bits order them: bf16 in the upper half of the float's key; a half's own,
+// made to an ordered key as ordered_bits does it (-0 as +0, NaNs quiet as the conversion to float leaves them).
+__device__ inline uint32_t key_of_score(float score, int type, int id) {
+  if (type == 0) return ordered_bits(score);
+  uint32_t top;
+  if (type == 1) {
+    top = ordered_bits(score) >> 16;
+  } else {
+    const uint32_t h = __builtin_bit_cast(uint16_t, static_cast<_Float16>(score + 0.0f));
+    top = (h & 0x8000u) ? ~h & 0xffffu : h | 0x8000u;
+  }
+  return (top << 16) | (0xffffu - static_cast<uint32_t>(id));
+}
+template <int CTRL>
+__device__ inline float dpp_moved(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-// Picks the K best (score desc, expert id asc) entries of the row held as
-// score[s] (expert lane + 64*s); lane k < K returns the k-th winner in my_id.
-// A score is its order-preserving 32-bit pattern (0: not a candidate); the round's winner is the lowest slot and
-// lane that holds the maximum, found by ballots: a third of the instructions of a reduction on (score, id) pairs.
+// The largest of the wave's keys, in every lane.
 template <int SLOTS>
-__device__ inline void select_topk(const float (&score)[SLOTS], const bool (&eligible)[SLOTS], int K,
-                                   int lane, int& my_id) {
-  uint32_t key[SLOTS];
+__device__ inline uint32_t best_key(const uint32_t (&key)[SLOTS]) {
+  uint32_t best = 0;
 #pragma unroll
-  for (int s = 0; s < SLOTS; ++s) key[s] = eligible[s] ? ordered_bits(score[s]) : 0;
+  for (int s = 0; s < SLOTS; ++s) best = max(best, key[s]);
+  return group_max_u32<kWave>(best);
+}
+
+// The K best entries of the row held as key[s] (expert lane + 64 s; larger is better, 0: not a candidate) in K rounds
+// of the largest key: rank[s] < K is the place of a chosen entry. A round finds its winner by comparing keys, on the vector
+// unit alone - no ballot, whose way through the scalar unit was half of a round. False if equal keys (or too few
+// candidates) gave a round several winners: select_in_order then.
+template <int SLOTS>
+__device__ inline bool rank_topk(uint32_t (&key)[SLOTS], int K, int (&rank)[SLOTS]) {
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s) rank[s] = K;
+  for (int k = 0; k < K; ++k) {
+    const uint32_t best = best_key<SLOTS>(key);
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) {
+      const bool won = key[s] == best;
+      rank[s] = won ? k : rank[s];
+      key[s] = won ? 0 : key[s];
+    }
+  }
+  int chosen = 0;
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s) chosen += __builtin_popcountll(__ballot(rank[s] < K));
+  return chosen == K;
+}
+
+// The same with equal keys, lowest expert id first; lane k < K returns the k-th winner in my_id (-1: fewer candidates
+// than K, which the host refuses). A round's winner is the lowest slot and lane that holds the maximum, found by ballots.
+template <int SLOTS>
+__device__ inline void select_in_order(uint32_t (&key)[SLOTS], int K, int lane, int& my_id) {
   my_id = -1;
   for (int k = 0; k < K; ++k) {
-    uint32_t best = 0;
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s) best = max(best, key[s]);
-    best = wave_max_u32(best);
+    const uint32_t best = best_key<SLOTS>(key);
     int id = 0;
 #pragma unroll
     for (int s = SLOTS - 1; s >= 0; --s) {
       const uint64_t holds = __ballot(key[s] == best);
       if (holds != 0) id = kWave * s + __builtin_ctzll(holds);
     }
-    if (best == 0) id = -1;  // (fewer candidates than K: the host refuses such arguments)
+    if (best == 0) id = -1;
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s)
       if (id == lane + kWave * s) key[s] = 0;  // taken
     if (lane == k) my_id = id;
   }
+}
+
+// Picks the K best (score desc, expert id asc) entries of the row held as score[s] (expert lane + 64*s); lane k < K
+// returns the k-th winner in my_id and its value[] in got. An entry's key is its score's order-preserving 32-bit pattern;
+// where the scores are 16-bit values (`type` of LogitsView: 1 bf16, 2 half), which are often equal, the 16 bits that tell
+// them apart and the id, so that no two keys are the same. The winners send id and value to their lanes.
+template <int SLOTS>
+__device__ inline void select_topk(const float (&score)[SLOTS], const bool (&eligible)[SLOTS], const float (&value)[SLOTS], int type,
+                                   int K, int lane, int& my_id, float& got) {
+  uint32_t key[SLOTS], left[SLOTS];
+  int rank[SLOTS];
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s) key[s] = eligible[s] ? key_of_score(score[s], type, lane + kWave * s) : 0;
+  if (K < kWave) {
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) left[s] = key[s];
+    if (rank_topk<SLOTS>(left, K, rank)) {
+      int id = 0, bits = 0;  // (entries that were not chosen send zeros to the last lane, which has no winner)
+#pragma unroll
+      for (int s = 0; s < SLOTS; ++s) {
+        const bool chosen = rank[s] < K;
+        const int to = 4 * (chosen ? rank[s] : kWave - 1);
+        id |= __builtin_amdgcn_ds_permute(to, chosen ? lane + kWave * s : 0);
+        bits |= __builtin_amdgcn_ds_permute(to, chosen ? __builtin_bit_cast(int, value[s]) : 0);
+      }
+      my_id = id;
+      got = __builtin_bit_cast(float, bits);
+      return;
+    }
+  }
+  select_in_order<SLOTS>(key, K, lane, my_id);
+  const int want = my_id >= 0 ? my_id : 0;
+  got = 0.0f;
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s) {
+    const float t = __shfl(value[s], want & (kWave - 1), kWave);
+    if ((want >> 6) == s) got = t;
+  }
+}
+
+// p of lanes 0 ... K - 1 added in this order, in every lane.
+__device__ inline float sum_in_order(float p, int K) {
+  float sum = 0.0f;
+  for (int k = 0; k < K; ++k) sum = sum + __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), k));
+  return sum;
 }
 
 // The row's logits, expert lane + 64 s in v[s]; experts past the last read the last one. Every load is requested
@@ -115,26 +189,12 @@ __device__ inline void softmax_topk_body(const LogitsView& logits, int M, int E,
   }
   const float total = wave_sum_tree(part);
 
+  // lane k owns winner k and its exp
   int my_id;
-  select_topk<SLOTS>(v, ok, K, lane, my_id);
-
-  // Lane k owns winner k: fetch its exp from the owning lane/slot.
-  float p = 0.0f;
-  {
-    const int want = my_id >= 0 ? my_id : 0;
-    float got = 0.0f;
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s) {
-      const float t = __shfl(ex[s], want & (kWave - 1), kWave);
-      if ((want >> 6) == s) got = t;
-    }
-    if (lane < K) p = got / total;
-  }
-  if (renorm) {
-    float denom = 0.0f;
-    for (int k = 0; k < K; ++k) denom = denom + __shfl(p, k, kWave);  // k ascending
-    p = p / denom;
-  }
+  float got;
+  select_topk<SLOTS>(v, ok, ex, logits.type, K, lane, my_id, got);
+  float p = lane < K ? got / total : 0.0f;
+  if (renorm) p = p / sum_in_order(p, K);  // k ascending
   if (lane < K) {
     topk_w[static_cast<size_t>(m) * K + lane] = p;
     topk_ids[static_cast<size_t>(m) * K + lane] = my_id;
@@ -175,22 +235,42 @@ __device__ inline void sigmoid_group_topk_body(const LogitsView& logits, const f
     float gscore = -__builtin_inff();
     if ((gsize & (gsize - 1)) == 0 && gsize <= kWave) {
       // groups of 2 to 64 experts side by side in the lanes of a slot: a butterfly over the group keeps the two
-      // largest (for 32 experts five exchanges where one lane walking the LDS copy of its group is a chain of 32
-      // reads and compares: DeepSeek-V3 routing at 23 tokens 10.2 -> 6 us)
-      float top[SLOTS];
+      // largest, all slots side by side
+      float t1[SLOTS], t2[SLOTS];
 #pragma unroll
       for (int s = 0; s < SLOTS; ++s) {
-        float t1 = fmaxf(c[s], -__builtin_inff()), t2 = -__builtin_inff();  // (a NaN counts as no score)
-        for (int off = gsize >> 1; off > 0; off >>= 1) {
-          const float o1 = __shfl_xor(t1, off, kWave), o2 = __shfl_xor(t2, off, kWave);
-          t2 = fmaxf(fminf(t1, o1), fmaxf(t2, o2));
-          t1 = fmaxf(t1, o1);
-        }
-        top[s] = t1 + t2;
+        t1[s] = fmaxf(c[s], -__builtin_inff());  // (a NaN counts as no score)
+        t2[s] = -__builtin_inff();
       }
+      // (steps of 1, 2, 4 ... lanes: once groups of N agree, the mirrored half row and row serve as lane l ^ N)
+      auto merge = [&](auto other) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s) {
+          const float o1 = other(t1[s]), o2 = other(t2[s]);
+          t2[s] = fmaxf(fminf(t1[s], o1), fmaxf(t2[s], o2));
+          t1[s] = fmaxf(t1[s], o1);
+        }
+      };
+      merge([](float v) { return dpp_moved<0xB1>(v); });                    // quad_perm [1,0,3,2]
+      if (gsize >= 4) merge([](float v) { return dpp_moved<0x4E>(v); });    // quad_perm [2,3,0,1]
+      if (gsize >= 8) merge([](float v) { return dpp_moved<0x141>(v); });   // row_half_mirror
+      if (gsize >= 16) merge([](float v) { return dpp_moved<0x140>(v); });  // row_mirror
+      const bool odd_row = (lane & 16) != 0, upper = lane >= 32;
+      if (gsize >= 32)
+        merge([odd_row](float v) {
+          const uint32_t u = __builtin_bit_cast(uint32_t, v);
+          const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+          return __builtin_bit_cast(float, static_cast<uint32_t>(odd_row ? r[0] : r[1]));
+        });
+      if (gsize >= 64)
+        merge([upper](float v) {
+          const uint32_t u = __builtin_bit_cast(uint32_t, v);
+          const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+          return __builtin_bit_cast(float, static_cast<uint32_t>(upper ? r[0] : r[1]));
+        });
 #pragma unroll
       for (int s = 0; s < SLOTS; ++s) {
-        const float t = __shfl(top[s], (lane * gsize) & (kWave - 1), kWave);
+        const float t = __shfl(t1[s] + t2[s], (lane * gsize) & (kWave - 1), kWave);
         if (lane < n_group && (lane * gsize) / kWave == s) gscore = t;
       }
     } else {
@@ -214,37 +294,28 @@ __device__ inline void sigmoid_group_topk_body(const LogitsView& logits, const f
         gscore = t1 + t2;
       }
     }
-    uint64_t keep = 0;
-    uint32_t gkey = lane < n_group ? ordered_bits(gscore) : 0;
-    for (int t = 0; t < topk_group; ++t) {
-      const uint32_t best = wave_max_u32(gkey);
-      const int bi = __builtin_ctzll(__ballot(gkey == best));  // the lowest group among equals
-      if (bi == lane) gkey = 0;
-      keep |= static_cast<uint64_t>(1) << (bi & 63);
+    // kept: the groups that fewer than topk_group others precede (score desc, group asc)
+    const uint32_t gkey = lane < n_group ? ordered_bits(gscore) : 0;
+    int ahead = 0;
+    for (int g = 0; g < n_group; ++g) {
+      const uint32_t other = __builtin_amdgcn_readlane(gkey, g);
+      ahead += (other > gkey || (other == gkey && g < lane)) ? 1 : 0;
     }
+    const uint64_t keep = __ballot(lane < n_group && ahead < topk_group);
+    const int shift = (gsize & (gsize - 1)) == 0 ? __builtin_ctz(gsize) : -1;  // (a division takes some twenty instructions)
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) {
       const int e = lane + kWave * s;
-      if (ok[s]) ok[s] = (keep >> (e / gsize)) & 1u;
+      const int group = shift >= 0 ? e >> shift : e / gsize;
+      if (ok[s]) ok[s] = (keep >> group) & 1u;
     }
   }
 
   int my_id;
-  select_topk<SLOTS>(c, ok, K, lane, my_id);
-
-  float p = 0.0f;
-  {
-    const int want = my_id >= 0 ? my_id : 0;
-    float got = 0.0f;
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s) {
-      const float t = __shfl(sg[s], want & (kWave - 1), kWave);
-      if ((want >> 6) == s) got = t;
-    }
-    if (lane < K) p = got;
-  }
-  float denom = 0.0f;
-  for (int k = 0; k < K; ++k) denom = denom + __shfl(p, k, kWave);  // k ascending
+  float p;
+  select_topk<SLOTS>(c, ok, sg, 0, K, lane, my_id, p);
+  if (lane >= K) p = 0.0f;
+  float denom = sum_in_order(p, K);
   denom = denom + 1e-20f;
   p = (p / denom) * scale;
   if (lane < K) {
