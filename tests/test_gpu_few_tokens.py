@@ -300,3 +300,29 @@ print(zlib.crc32(out.view(torch.int16).cpu().numpy().tobytes()), int("few_" in n
         assert run.returncode == 0, run.stderr[-2000:]
         got.append(run.stdout.split())
     assert got[0][0] == got[1][0] and got[0][1] == "1" and got[1][1:] == ["0", "1"], got
+
+
+@pytest.mark.parametrize("fmt,H", [("int8", 128), ("int8", 7680), ("int8", 7808), ("int8", 8448), ("int8", 8576), ("fp8", 256), ("fp8", 8192),
+                                   ("none", 7680), ("none", 12672), ("w4", 256), ("w4", 7808)])
+@pytest.mark.parametrize("grouped", [False, True])
+@pytest.mark.parametrize("infinite", [False, True])
+def test_one_token_whose_row_the_other_waves_bring(fmt, H, grouped, infinite):
+    """One token: waves 1 to 3 bring its row to LDS, in one round of loads up to 7680 values, beside the routing's scores (sigmoid),
+    int8 up to 8448 values, whose copy in 16 bits shares the space; with an infinity in the row, which the usual way does not take."""
+    from vllm_kunlun_amd import synth
+    base = ("dsv3-fp8-decode" if fmt == "fp8" else "dsv3-decode") if grouped and fmt in ("int8", "fp8") else "qwen3-decode"
+    over = dict(I_shared=128, n_group=4, topk_group=2) if base != "qwen3-decode" else {}
+    sl = synth.make_layer(synth.scaled(synth.SHAPES[base], M=1, H=H, E=96, K=4, I=128, quant=fmt, **over), "cuda", seed=H)
+    if infinite:
+        sl.x[0, H - 3] = float("inf")
+    out, named = _named(lambda: _call(sl))
+    assert ROUTED in named, named
+    if infinite:  # as the launches apart make it
+        two = torch.cat([sl.x, sl.x[:0].new_zeros(40, H)])
+        logits = torch.cat([sl.logits, sl.logits.new_zeros(40, sl.logits.shape[1])])
+        sl.x, sl.logits = two, logits
+        whole = _call(sl)[:1]
+        assert torch.equal(torch.isnan(out), torch.isnan(whole))
+        assert rel_l2(out.nan_to_num(0, 0, 0), whole.nan_to_num(0, 0, 0)) <= 4e-3 or bool(torch.isnan(out).all())
+    else:
+        _check(sl, out)

@@ -260,9 +260,16 @@ int launch_few_down(const FewDown& p, hipStream_t s) {
 //
 // A workgroup serves 16 output channels of one routed PAIR's expert (columns of the grid: pairs, then the shared expert if
 // one rides along, then one that leaves the routing and the sort for whoever reads them). It routes every token itself, a
-// wave each, from the logits: a dozen cache lines and a microsecond against a launch of four before this one. The first
+// wave each, from the logits: a dozen cache lines and a microsecond against a launch of four before this one. (Which experts
+// only: their weights are the last column's business.) The first
 // pair that chose an expert serves all its rows; the other columns leave. The four waves split K; each quantises its own
 // part of the rows while its weights are on their way (int8: one exchange of the maxima), and the codes wait in LDS.
+// One token alone is routed by wave 0, and the others bring its row to LDS meanwhile - quantised, but for int8, whose scale
+// is known only when all three have their part: each wave then rounds its part of K from there. Layer, us, the row asked for
+// behind the weights / so, weights of the experts' routing left to the last column in both: Qwen3 dims int8 14.6 / 13.8, bf16 18.7 /
+// 18.4; with them, before: int8 14.8, bf16 18.8, DeepSeek-V3 dims int8 70.4 -> 69.6, Kimi-K2 dims 4-bit 48.7 -> 47.6.
+// (The same for up to four tokens, every wave its part of all rows before the routing: 4 tokens 30.2 -> 33.3, a row then is
+// looked at by every column and not by those that serve it.)
 template <Fmt FMT, int SLOTS, bool SIGMOID>
 __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up_kernel(const FewGateUp p) {
   using acc_t = typename std::conditional<FMT == Fmt::I8, v4i, v4f>::type;
@@ -288,15 +295,56 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
   const bool tail = p.w_tail != nullptr && column == P;
   const bool publish = column == P + (p.w_tail ? 1 : 0);
   if (publish && blockIdx.x != 0) return;
+  const int pitch = few_row_pitch(p.H, QUANT ? 1 : 2, FMT == Fmt::F8);
+  int8_t* const rows_lds = lds + (p.alone ? p.alone_at : 0);
+  auto store_codes = [&](const Pack8& val, const RowScale& s, int8_t* dst, int v) __attribute__((always_inline)) {  // vector v of a row
+    if constexpr (FMT == Fmt::I8) {
+      *reinterpret_cast<uint2*>(dst + v * 8) = quant8_i8_of(val, s, f16);
+    } else if constexpr (FMT == Fmt::F8) {
+      float sc;
+      *reinterpret_cast<uint2*>(dst + v * 8) = quant8_fp8(val, f16, sc);
+      if ((lane & 15) == 0) reinterpret_cast<float*>(dst + p.H)[v >> 4] = sc;
+    } else {
+      *reinterpret_cast<uint4*>(dst + v * 16) = val.v;
+    }
+  };
+
+  // ---- one token: waves 1 to 3 and its row ----
+  if (p.alone && wave > 0 && !publish) {
+    constexpr int kTakers = 3, kBatch = 5;  // (five vectors a lane: 7680 values in one round trip)
+    uint32_t mag = 0;
+    for (int v0 = (wave - 1) * kWave + lane; v0 - lane < p.H / 8; v0 += kBatch * kTakers * kWave) {
+      Pack8 val[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        val[i].v = make_uint4(0, 0, 0, 0);
+        if (v0 + i * kTakers * kWave < p.H / 8) val[i].v = reinterpret_cast<const uint4*>(p.x)[v0 + i * kTakers * kWave];
+      }
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int v = v0 + i * kTakers * kWave;
+        if constexpr (FMT == Fmt::I8) {
+          mag = max_magnitudes(mag, magnitudes8(val[i]));
+          if (v < p.H / 8) *reinterpret_cast<uint4*>(rows_lds + pitch + v * 16) = val[i].v;
+        } else {
+          if (v < p.H / 8) store_codes(val[i], RowScale{}, rows_lds, v);
+        }
+      }
+    }
+    if constexpr (FMT == Fmt::I8) {
+      mag = group_max_u32<kWave>(max_of_pair(mag));
+      if (lane == 0) max_lds[0][wave] = mag;
+    }
+  }
 
   // ---- which expert, which rows ----
   int e = 0, rows = 0, begin = 0;
   int my_pair = 0;  // lane l: the pair of row l % 16 of this column
   if (!tail) {
     if constexpr (SIGMOID)
-      sigmoid_group_topk_body<SLOTS>(r.logits, r.bias, r.M, r.E, r.K, r.n_group, r.topk_group, r.scale, tw_lds, id_lds, reinterpret_cast<float*>(lds), 0);
+      sigmoid_group_topk_body<SLOTS>(r.logits, r.bias, r.M, r.E, r.K, r.n_group, r.topk_group, r.scale, tw_lds, id_lds, reinterpret_cast<float*>(lds), 0, publish);
     else
-      softmax_topk_body<SLOTS>(r.logits, r.M, r.E, r.K, r.renorm, tw_lds, id_lds, 0);
+      softmax_topk_body<SLOTS>(r.logits, r.M, r.E, r.K, r.renorm, tw_lds, id_lds, 0, publish);
     __syncthreads();
     const int id = lane < P ? id_lds[lane] : 0x7fffffff;  // (P <= 64)
     if (publish) {
@@ -339,6 +387,7 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
   } else {
     rows = r.M;
     begin = P;
+    if (p.alone) __syncthreads();
   }
   const int my_token = tail ? min(li, rows - 1) : my_pair / r.K;  // of row li (rows past the last: any token)
 
@@ -391,15 +440,11 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- the rows: this wave's part of K, quantised (the quantisers' arithmetic) or as it is, into LDS ----
-  const int pitch = few_row_pitch(p.H, QUANT ? 1 : 2, FMT == Fmt::F8);
-  int8_t* rows_lds = lds;
   const int v0 = kb0 * (kStepValues / 8), nvec = klen * (kStepValues / 8);  // vectors of 8 values
   float amax = 1.0f;
-  for (int i = 0; i < rows; ++i) {
-    const int token = __builtin_amdgcn_readlane(my_token, i);
-    const uint4* src = reinterpret_cast<const uint4*>(p.x + static_cast<size_t>(token) * p.H) + v0;
-    int8_t* dst = rows_lds + i * pitch;
-    if constexpr (FMT == Fmt::I8) {
+  if constexpr (FMT == Fmt::I8) {
+    for (int i = 0; i < rows && !p.alone; ++i) {
+      const uint4* src = reinterpret_cast<const uint4*>(p.x + static_cast<size_t>(__builtin_amdgcn_readlane(my_token, i)) * p.H) + v0;
       uint32_t mag = 0;
       for (int v = lane; v < nvec; v += kWave) {
         Pack8 val;
@@ -408,41 +453,41 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
       }
       mag = group_max_u32<kWave>(max_of_pair(mag));
       if (lane == 0) max_lds[i][wave] = mag;
-    } else if constexpr (FMT == Fmt::F8) {
-      for (int v = lane; v < nvec; v += kWave) {
-        Pack8 val;
-        val.v = src[v];
-        float s;
-        *reinterpret_cast<uint2*>(dst + (v0 + v) * 8) = quant8_fp8(val, f16, s);
-        if ((lane & 15) == 0) reinterpret_cast<float*>(dst + p.H)[(v0 + v) >> 4] = s;
-      }
-    } else {
-      for (int v = lane; v < nvec; v += kWave) *reinterpret_cast<uint4*>(dst + (v0 + v) * 16) = src[v];
     }
+    if (!p.alone) __syncthreads();
   }
-  if constexpr (FMT == Fmt::I8) {
-    __syncthreads();
-    for (int i = 0; i < rows; ++i) {
-      const int token = __builtin_amdgcn_readlane(my_token, i);
-      const uint4* src = reinterpret_cast<const uint4*>(p.x + static_cast<size_t>(token) * p.H) + v0;
-      int8_t* dst = rows_lds + i * pitch;
-      RowScale s = row_scale_i8(max(max(max_lds[i][0], max_lds[i][1]), max(max_lds[i][2], max_lds[i][3])), f16);
+  for (int i = 0; i < rows; ++i) {
+    if (FMT != Fmt::I8 && p.alone) break;  // (done)
+    const int token = __builtin_amdgcn_readlane(my_token, i);
+    const uint4* src = reinterpret_cast<const uint4*>(p.x + static_cast<size_t>(token) * p.H);
+    int8_t* dst = rows_lds + i * pitch;
+    RowScale s = {};
+    if constexpr (FMT == Fmt::I8) {
+      s = row_scale_i8(max(max(p.alone ? 0u : max_lds[i][0], max_lds[i][1]), max(max_lds[i][2], max_lds[i][3])), f16);
       if (!s.numbers) {  // (the same for the whole workgroup) every wave goes over the whole row: rare
         float top = 0.0f;
         for (int v = lane; v < p.H / 8; v += kWave) {
           Pack8 val;
-          val.v = (src - v0)[v];
+          val.v = src[v];
           top = fmaxf(top, amax8(val, f16));
         }
         s.amax = __builtin_bit_cast(float, group_max_u32<kWave>(__builtin_bit_cast(uint32_t, top)));
         s.inv = s.amax > 0.0f ? 127.0f / s.amax : 0.0f;
       }
       if (li == i) amax = s.amax;
-      for (int v = lane; v < nvec; v += kWave) {
-        Pack8 val;
-        val.v = src[v];
-        *reinterpret_cast<uint2*>(dst + (v0 + v) * 8) = quant8_i8_of(val, s, f16);
+      if (p.alone) {
+        for (int v = lane; v < nvec; v += kWave) {
+          Pack8 val;
+          val.v = *reinterpret_cast<const uint4*>(rows_lds + pitch + (v0 + v) * 16);
+          store_codes(val, s, dst, v0 + v);
+        }
+        break;
       }
+    }
+    for (int v = lane; v < nvec; v += kWave) {
+      Pack8 val;
+      val.v = src[v0 + v];
+      store_codes(val, s, dst, v0 + v);
     }
   }
 
@@ -506,6 +551,16 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
     sum[f] = acc[f][0] + acc[f][1];
     if (wave > 0) red[wave - 1][f][lane] = sum[f];
   }
+  float sa = 1.0f;
+  if constexpr (FMT == Fmt::I8) {  // (the divisions of the scales while the other waves come in)
+    sa = amax / 127.0f;
+    asm("" : "+v"(sa));
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      wmax[f] = make_float4(wmax[f].x / 127.0f, wmax[f].y / 127.0f, wmax[f].z / 127.0f, wmax[f].w / 127.0f);
+      asm("" : "+v"(wmax[f].x), "+v"(wmax[f].y), "+v"(wmax[f].z), "+v"(wmax[f].w));
+    }
+  }
   __syncthreads();
   if (wave == 0 && li < rows) {
     uint16_t g[4], u[4];
@@ -517,7 +572,7 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         uint16_t& o = f == 0 ? g[q] : u[q];
-        if constexpr (FMT == Fmt::I8) o = f32_to_act((static_cast<float>(sum[f][q]) * (amax / 127.0f)) * (wm[q] / 127.0f), f16);
+        if constexpr (FMT == Fmt::I8) o = f32_to_act((static_cast<float>(sum[f][q]) * sa) * wm[q], f16);
         else o = f32_to_act(sum[f][q], f16);
       }
     }
@@ -529,10 +584,16 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
 }
 
 template <Fmt FMT, int SLOTS, bool SIGMOID>
-int launch_few_gate_up(const FewGateUp& p, hipStream_t s) {
+int launch_few_gate_up(FewGateUp p, hipStream_t s) {
   const int pitch = few_row_pitch(p.H, FMT == Fmt::I8 || FMT == Fmt::F8 ? 1 : 2, FMT == Fmt::F8);
-  // LDS: routing's copy of the scores, then the rows in its place
-  const size_t bytes = std::max(static_cast<size_t>(p.route.M) * pitch, SIGMOID ? sizeof(float) * 4 * p.route.E : 0);
+  // LDS: routing's copy of the scores, then the rows in its place; one token: beside that of the wave that routes it, with
+  // the row as it is behind its codes (int8), if that leaves the five workgroups of few_gate_up_takes their room
+  const size_t scores = SIGMOID ? sizeof(float) * p.route.E : 0;
+  size_t bytes = std::max(static_cast<size_t>(p.route.M) * pitch, 4 * scores);
+  const size_t alone = align_up(scores, 16) + pitch + (FMT == Fmt::I8 ? 2 * static_cast<size_t>(p.H) : 0);
+  p.alone = p.route.M == 1 && alone <= kFewRowBytes;
+  p.alone_at = static_cast<int32_t>(align_up(scores, 16));
+  if (p.alone) bytes = alone;
   if (tracing_kernels())
     note_kernel("few_gate_up_kernel<%s>: routing, quantisation, sort and gate_up of a pair's 16 channels", fmt_name(FMT));
   hipLaunchKernelGGL((few_gate_up_kernel<FMT, SLOTS, SIGMOID>), dim3(p.I / 16, p.route.M * p.route.K + (p.w_tail ? 1 : 0) + 1), dim3(4 * kWave), bytes, s, p);

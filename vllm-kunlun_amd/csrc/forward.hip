@@ -236,13 +236,11 @@ bool few_down_pays(const kmoe_moe_args* a, bool fold) {
 
 // Whether such a layer also begins in one launch (few_gate_up): up to kFewRouted tokens, so that routing is a wave each,
 // whose rows leave room for five workgroups in a CU's LDS - fewer, and the launch no longer fills the chip at once (Kimi-K2
-// dims, 4-bit, 1 token 57.1 -> 52.6 us, 2 tokens, three workgroups, 92.7 -> 98.9). Layer, us, apart / in one launch: Qwen3 dims int8
-// 1 token 18.9 / 16.4, 4 37.0 / 32.2, bf16 1 22.0 / 20.4, 4-bit 1 18.4 / 15.5, 4 27.2 / 24.7; DeepSeek-V3 dims int8 1 87.7 /
-// 78.5, with the gate 96.6 / 87.6, fp8 1 88.7 / 84.
+// dims, 4-bit, 1 token 57.1 -> 52.6 us, 2 tokens, three workgroups, 92.7 -> 98.9). Layer, us, apart / in one launch: Qwen3 dims int8 1 token 18.9 / 13.8, 4 36.3 / 29.4, bf16 1 22.0 / 18.4, 4-bit 1 18.4 / 14.9, 4 27.2 / 24.7; DeepSeek-V3 dims int8 1 87.7 /
+// 69.6, with the gate 96.6 / 78.4, fp8 1 88.7 / 68.8.
 bool few_gate_up_takes(const kmoe_moe_args* a) {
-  constexpr int kRows = 25 * 1024;  // bytes
-  if (a->M > kFewRouted || a->M * a->K > kWave || a->E > 8 * kWave || a->H > kRows) return false;
-  if (a->M * few_row_pitch(a->H, bf16_activations(a->format) ? 2 : 1, a->format == KMOE_FMT_FP8_BLOCK) > kRows) return false;
+  if (a->M > kFewRouted || a->M * a->K > kWave || a->E > 8 * kWave || a->H > kFewRowBytes) return false;
+  if (a->M * few_row_pitch(a->H, bf16_activations(a->format) ? 2 : 1, a->format == KMOE_FMT_FP8_BLOCK) > kFewRowBytes) return false;
   for (const void* t : {static_cast<const void*>(a->x), static_cast<const void*>(a->w13), static_cast<const void*>(a->w13_max),
                         static_cast<const void*>(a->w13_scale), static_cast<const void*>(a->ws13), static_cast<const void*>(a->ws13_max)})
     if (reinterpret_cast<uintptr_t>(t) & 15) return false;

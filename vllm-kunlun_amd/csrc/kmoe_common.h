@@ -154,8 +154,10 @@ struct FewGateUp {
   StreamScan sort;  // what the sort would leave, slot_rows too (ids and n_pairs are not looked at)
   uint16_t* act;  // [P (+ M), I]
   int32_t f16;
+  int32_t alone, alone_at;  // (the launcher's) one token whose row waves 1 to 3 bring to LDS, this far in
 };
 constexpr int kFewRouted = 4;
+constexpr int kFewRowBytes = 25 * 1024;  // of LDS for the rows of a launch: five workgroups on a CU
 int few_gate_up(const FewGateUp& p, int format, bool sigmoid, hipStream_t stream);
 // The checks of the routing arguments (and n_group <= 1 made one group).
 int check_route(RouteArgs* r, bool sigmoid);

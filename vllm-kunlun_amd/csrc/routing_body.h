@@ -158,10 +158,10 @@ __device__ inline void load_logits(const LogitsView& l, size_t row, int E, float
 }
 
 // One wave per token: workgroup `block` of kWavesPerBlock waves serves tokens
-// block * kWavesPerBlock + wave.
+// block * kWavesPerBlock + wave. weights: false leaves topk_w alone, for callers that ask only which experts a token goes to.
 template <int SLOTS>
 __device__ inline void softmax_topk_body(const LogitsView& logits, int M, int E, int K, int renorm,
-                                         float* __restrict__ topk_w, int32_t* __restrict__ topk_ids, int block) {
+                                         float* __restrict__ topk_w, int32_t* __restrict__ topk_ids, int block, bool weights = true) {
   const int lane = lane_id();
   const int m = block * kWavesPerBlock + (threadIdx.x >> 6);
   if (m >= M) return;
@@ -177,28 +177,29 @@ __device__ inline void softmax_topk_body(const LogitsView& logits, int M, int E,
     v[s] = ok[s] ? v[s] : -__builtin_inff();
     mx = fmaxf(mx, v[s]);
   }
-  mx = wave_max(mx);
-
   // exp and the row sum: per-lane running sum over slots, then the lane tree.
-  float ex[SLOTS];
-  float part = 0.0f;
+  float ex[SLOTS] = {};
+  float total = 1.0f;
+  if (weights) {
+    mx = wave_max(mx);
+    float part = 0.0f;
 #pragma unroll
-  for (int s = 0; s < SLOTS; ++s) {
-    ex[s] = ok[s] ? exp_fixed(v[s] - mx) : 0.0f;
-    part = part + ex[s];
+    for (int s = 0; s < SLOTS; ++s) {
+      ex[s] = ok[s] ? exp_fixed(v[s] - mx) : 0.0f;
+      part = part + ex[s];
+    }
+    total = wave_sum_tree(part);
   }
-  const float total = wave_sum_tree(part);
 
   // lane k owns winner k and its exp
   int my_id;
   float got;
   select_topk<SLOTS>(v, ok, ex, logits.type, K, lane, my_id, got);
+  if (lane < K) topk_ids[static_cast<size_t>(m) * K + lane] = my_id;
+  if (!weights) return;
   float p = lane < K ? got / total : 0.0f;
   if (renorm) p = p / sum_in_order(p, K);  // k ascending
-  if (lane < K) {
-    topk_w[static_cast<size_t>(m) * K + lane] = p;
-    topk_ids[static_cast<size_t>(m) * K + lane] = my_id;
-  }
+  if (lane < K) topk_w[static_cast<size_t>(m) * K + lane] = p;
 }
 
 // choice_lds: [kWavesPerBlock][E] floats of (dynamic) LDS.
@@ -206,7 +207,7 @@ template <int SLOTS>
 __device__ inline void sigmoid_group_topk_body(const LogitsView& logits, const float* __restrict__ bias, int M,
                                                int E, int K, int n_group, int topk_group, float scale,
                                                float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
-                                               float* choice_lds, int block) {
+                                               float* choice_lds, int block, bool weights = true) {
   const int lane = lane_id();
   const int wave = threadIdx.x >> 6;
   const int m = block * kWavesPerBlock + wave;
@@ -260,13 +261,15 @@ __device__ inline void sigmoid_group_topk_body(const LogitsView& logits, const f
         merge([odd_row](float v) {
           const uint32_t u = __builtin_bit_cast(uint32_t, v);
           const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-          return __builtin_bit_cast(float, static_cast<uint32_t>(odd_row ? r[0] : r[1]));
+          const uint32_t a = r[0], b = r[1];  // (chosen between as values: between elements it is an address, and the stack)
+          return __builtin_bit_cast(float, odd_row ? a : b);
         });
       if (gsize >= 64)
         merge([upper](float v) {
           const uint32_t u = __builtin_bit_cast(uint32_t, v);
           const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-          return __builtin_bit_cast(float, static_cast<uint32_t>(upper ? r[0] : r[1]));
+          const uint32_t a = r[0], b = r[1];  // (chosen between as values: between elements it is an address, and the stack)
+          return __builtin_bit_cast(float, upper ? a : b);
         });
 #pragma unroll
       for (int s = 0; s < SLOTS; ++s) {
@@ -314,15 +317,13 @@ __device__ inline void sigmoid_group_topk_body(const LogitsView& logits, const f
   int my_id;
   float p;
   select_topk<SLOTS>(c, ok, sg, 0, K, lane, my_id, p);
+  if (lane < K) topk_ids[static_cast<size_t>(m) * K + lane] = my_id;
+  if (!weights) return;
   if (lane >= K) p = 0.0f;
   float denom = sum_in_order(p, K);
   denom = denom + 1e-20f;
   p = (p / denom) * scale;
-  if (lane < K) {
-    topk_w[static_cast<size_t>(m) * K + lane] = p;
-    topk_ids[static_cast<size_t>(m) * K + lane] = my_id;
-  }
+  if (lane < K) topk_w[static_cast<size_t>(m) * K + lane] = p;
 }
-
 
 }  // namespace kmoe
