@@ -53,10 +53,37 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
   const int m = blockIdx.y, col = blockIdx.x * 16;
   const bool f16 = FMT == Fmt::F16 || FMT == Fmt::W4H || ((FMT == Fmt::I8 || FMT == Fmt::F8) && p.f16 != 0);
   const bool tail = wave >= p.K;
+  // A wave takes a pair; int8, one token's waves take the sorted rows 0 ... K - 1 instead, which they may ask for before they know
+  // whose they are (k: the pair's place among the token's). Layer, us: DeepSeek-V3 dims 69.5 -> 67.5, Qwen3 dims 13.7 -> 13.5. (fp8 has no
+  // registers for it, 68.8 -> 72.6; 16-bit and 4-bit weights have nothing to do between a row and its product, 18.7 -> 18.8.)
+  const bool row_first = FMT == Fmt::I8 && p.M == 1;
   const int pair = m * p.K + wave;
-  const int e = tail ? 0 : p.ids[pair];
-  const int row = tail ? p.M * p.K + m : p.moe_index[pair];
-  const float weight = tail ? 0.0f : p.topk_w[pair];
+  const int nvec = p.I / 8;
+  Pack8 val[kVecs];
+  auto load_row = [&](int row) __attribute__((always_inline)) {
+    const uint4* src = reinterpret_cast<const uint4*>(p.act + static_cast<size_t>(row) * p.I);
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+      val[i].v = make_uint4(0, 0, 0, 0);
+      if (lane + i * kWave < nvec) val[i].v = src[lane + i * kWave];
+    }
+  };
+  int k = wave, e, row;
+  float weight;
+  if (row_first) {
+    const int j = min(lane, p.K - 1);
+    const int id = p.ids[j], at = p.moe_index[j];
+    const float w = p.topk_w[j];
+    row = wave;  // (the shared expert's row follows those of the pairs)
+    load_row(row);
+    if (!tail) k = __builtin_ctzll(__ballot(at == wave));
+    e = tail ? 0 : __builtin_amdgcn_readlane(id, k);
+    weight = tail ? 0.0f : __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), k));
+  } else {
+    e = tail ? 0 : p.ids[pair];
+    row = tail ? p.M * p.K + m : p.moe_index[pair];
+    weight = tail ? 0.0f : p.topk_w[pair];
+  }
 
   // ---- weights: as many steps of the 16 channels as the ring holds ----
   const int ksteps = p.kbytes / (64 * V);
@@ -94,25 +121,18 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
       gsc[slot] = sp[(p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / p.gs32) * p.s_g];
     }
   };
+  float4 wmax = make_float4(0, 0, 0, 0);
+  if constexpr (FMT == Fmt::I8) wmax = *reinterpret_cast<const float4*>((tail ? p.w_aux_tail : p.w_aux + static_cast<size_t>(e) * p.H) + col + lg * 4);
 #pragma unroll
   for (int d = 0; d < D; ++d)
     if (d < ksteps) load_w(d, d);
-  float4 wmax = make_float4(0, 0, 0, 0);
   float wsc = 0.0f;  // F8: lane l holds the block scale of step l
-  if constexpr (FMT == Fmt::I8) wmax = *reinterpret_cast<const float4*>((tail ? p.w_aux_tail : p.w_aux + static_cast<size_t>(e) * p.H) + col + lg * 4);
   if constexpr (FMT == Fmt::F8)
     wsc = (tail ? p.w_aux_tail : p.w_aux + static_cast<size_t>(e) * (p.H / 128) * ksteps)[static_cast<size_t>(col / 128) * ksteps + min(lane, ksteps - 1)];
 
   __builtin_amdgcn_sched_barrier(0);
   // ---- the row: quantised (the arithmetic of the quantisers' launches, hence their bits) or as it is, into LDS ----
-  const uint4* src = reinterpret_cast<const uint4*>(p.act + static_cast<size_t>(row) * p.I);
-  const int nvec = p.I / 8;
-  Pack8 val[kVecs];
-#pragma unroll
-  for (int i = 0; i < kVecs; ++i) {
-    val[i].v = make_uint4(0, 0, 0, 0);
-    if (lane + i * kWave < nvec) val[i].v = src[lane + i * kWave];
-  }
+  if (!row_first) load_row(row);
   int8_t* mine = rows_lds + wave * few_row_pitch(p.I, QUANT ? 1 : 2, FMT == Fmt::F8);
   [[maybe_unused]] float* scales = reinterpret_cast<float*>(mine + p.I);
   float amax = 1.0f;
@@ -159,6 +179,12 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
 #pragma unroll
     for (int i = 0; i < kVecs; ++i)
       if (lane + i * kWave < nvec) *reinterpret_cast<uint4*>(mine + (lane + i * kWave) * 16) = val[i].v;
+  }
+
+  if constexpr (FMT == Fmt::I8) {  // (the scales' divisions while the weights come in)
+    amax = amax / 127.0f;
+    wmax = make_float4(wmax.x / 127.0f, wmax.y / 127.0f, wmax.z / 127.0f, wmax.w / 127.0f);
+    asm("" : "+v"(amax), "+v"(wmax.x), "+v"(wmax.y), "+v"(wmax.z), "+v"(wmax.w));
   }
 
   // ---- product: all 16 rows of the MFMA are this row (its bytes are broadcast from LDS); four chains of sums ----
@@ -212,13 +238,13 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
     const float wm[4] = {wmax.x, wmax.y, wmax.z, wmax.w};
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      if constexpr (FMT == Fmt::I8) y[q] = f32_to_act((static_cast<float>(total[q]) * (amax / 127.0f)) * (wm[q] / 127.0f), f16);
+      if constexpr (FMT == Fmt::I8) y[q] = f32_to_act((static_cast<float>(total[q]) * amax) * wm[q], f16);
       else y[q] = f32_to_act(total[q], f16);
-      y_lds[wave][lg * 4 + q] = act_to_f32(y[q], f16);
+      y_lds[k][lg * 4 + q] = act_to_f32(y[q], f16);
     }
     *reinterpret_cast<uint2*>(p.down + static_cast<size_t>(row) * p.H + col + lg * 4) =
         make_uint2(y[0] | (static_cast<uint32_t>(y[1]) << 16), y[2] | (static_cast<uint32_t>(y[3]) << 16));
-    if (lane == 0) w_lds[wave] = weight;
+    if (lane == 0) w_lds[k] = weight;
   }
   __syncthreads();
 
