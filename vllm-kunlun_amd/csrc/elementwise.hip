@@ -9,7 +9,7 @@ template <int TPR, int NV>
 __global__ __launch_bounds__(256) void quant_i8_rows_kernel(const uint16_t* __restrict__ x, int64_t ld_x, int R,
                                                            int C, int8_t* __restrict__ q, int64_t ld_q,
                                                            float* __restrict__ row_max, int chunked, int f16) {
-  quant_i8_rows_body<TPR, NV>(x, ld_x, R, C, q, ld_q, row_max, chunked, blockIdx.x, f16 != 0);
+  quant_i8_rows_body<TPR, NV>(x, ld_x, R, C, q, ld_q, row_max, chunked, blockIdx.x * (256 / TPR), f16 != 0);
 }
 
 // ---------------------------------------- static and asymmetric int8 (the other modes of scaled_int8_quant)
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void quant_i8_rows_azp_kernel(const uint16_t* 
 __global__ __launch_bounds__(256) void quant_fp8_group128_kernel(const uint16_t* __restrict__ x, int64_t ld_x,
                                                                 int R, int C, uint8_t* __restrict__ q,
                                                                 int64_t ld_q, float* __restrict__ scale, int f16) {
-  quant_fp8_group128_body(x, ld_x, R, C, q, ld_q, scale, blockIdx.x, f16 != 0);
+  quant_fp8_group128_body(x, ld_x, R, C, q, ld_q, scale, static_cast<long long>(blockIdx.x) * 16, f16 != 0);
 }
 
 // ------------------------------------------------------------ silu-and-mul

@@ -367,10 +367,13 @@ __global__ __launch_bounds__(4 * kWave, FMT == Fmt::F8 ? 4 : 5) void few_gate_up
   int e = 0, rows = 0, begin = 0;
   int my_pair = 0;  // lane l: the pair of row l % 16 of this column
   if (!tail) {
-    if constexpr (SIGMOID)
-      sigmoid_group_topk_body<SLOTS>(r.logits, r.bias, r.M, r.E, r.K, r.n_group, r.topk_group, r.scale, tw_lds, id_lds, reinterpret_cast<float*>(lds), 0, publish);
-    else
-      softmax_topk_body<SLOTS>(r.logits, r.M, r.E, r.K, r.renorm, tw_lds, id_lds, 0, publish);
+    if (wave < r.M) {
+      if constexpr (SIGMOID)
+        sigmoid_group_topk_body<SLOTS>(r.logits, r.bias, wave, r.E, r.K, r.n_group, r.topk_group, r.scale, tw_lds, id_lds,
+                                       reinterpret_cast<float*>(lds) + wave * r.E, publish);
+      else
+        softmax_topk_body<SLOTS>(r.logits, wave, r.E, r.K, r.renorm, tw_lds, id_lds, publish);
+    }
     __syncthreads();
     const int id = lane < P ? id_lds[lane] : 0x7fffffff;  // (P <= 64)
     if (publish) {

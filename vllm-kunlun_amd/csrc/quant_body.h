@@ -76,17 +76,14 @@ __device__ inline float amax8(const Pack8& v, bool f16) {
 }
 
 // TPR threads cooperate on one row (32: two rows per wave); each keeps NV vectors of 8 values in
-// registers, so the row is read from memory once.
-// Workgroup `block` (256 threads) serves rows block * (256 / TPR) ...
-template <int TPR, int NV>
+// registers, so the row is read from memory once. A workgroup of THREADS serves rows first_row ...
+template <int TPR, int NV, int THREADS = 256>
 __device__ inline void quant_i8_rows_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
                                           int8_t* __restrict__ q, int64_t ld_q, float* __restrict__ row_max,
-                                          int chunked, int block, bool f16 = false) {
-  constexpr int kRowsPerBlock = 256 / TPR;
-  __shared__ uint32_t red[256 / kWave];
-  const int sub = threadIdx.x / TPR;
+                                          int chunked, int first_row, bool f16 = false) {
+  __shared__ uint32_t red[THREADS / kWave];
   const int t = threadIdx.x % TPR;
-  const int r = block * kRowsPerBlock + sub;
+  const int r = first_row + threadIdx.x / TPR;
   const bool live = r < R;
   const int nvec = C / 8;
   Pack8 val[NV];
@@ -102,28 +99,33 @@ __device__ inline void quant_i8_rows_body(const uint16_t* __restrict__ x, int64_
 #pragma unroll
     for (int i = 0; i < NV; ++i) mag = max_magnitudes(mag, magnitudes8(val[i]));
   }
-  // max over the row's threads (one row per block: combine the waves)
+  // max over the row's threads (rows of several waves: all of the workgroup's meet at the barrier)
   auto row_max_of = [&](uint32_t m) {
     m = group_max_u32<(TPR < kWave ? TPR : kWave)>(m);
     if (TPR > kWave) {
       if (lane_id() == 0) red[threadIdx.x >> 6] = m;
       __syncthreads();
-      m = red[0];
+      const uint32_t* mine = red + threadIdx.x / TPR * (TPR / kWave);
+      m = mine[0];
 #pragma unroll
-      for (int w = 1; w < TPR / kWave; ++w) m = max(m, red[w]);
+      for (int w = 1; w < TPR / kWave; ++w) m = max(m, mine[w]);
     }
     return m;
   };
   RowScale s = row_scale_i8(row_max_of(max_of_pair(mag)), f16);
-  if (!s.numbers) {  // (the same for all of a row's threads)
+  // (the same for all of a row's threads; several rows with barriers go in together)
+  if (TPR > kWave && THREADS > TPR ? __syncthreads_or(!s.numbers) != 0 : !s.numbers) {
     float m = 0.0f;
     if (live) {
 #pragma unroll
       for (int i = 0; i < NV; ++i) m = fmaxf(m, amax8(val[i], f16));
     }
     if (TPR > kWave) __syncthreads();  // (every wave has read the maxima it is about to replace)
-    s.amax = __builtin_bit_cast(float, row_max_of(__builtin_bit_cast(uint32_t, m)));  // (no negative numbers: ordered as their bits)
-    s.inv = s.amax > 0.0f ? 127.0f / s.amax : 0.0f;
+    m = __builtin_bit_cast(float, row_max_of(__builtin_bit_cast(uint32_t, m)));  // (no negative numbers: ordered as their bits)
+    if (!s.numbers) {
+      s.amax = m;
+      s.inv = m > 0.0f ? 127.0f / m : 0.0f;
+    }
   }
   if (!live) return;
   // row-major: vector v of the row; chunk-major [C/64][R][64]: vector v is eighth v%8 of chunk v/8
@@ -196,10 +198,10 @@ __device__ inline uint2 quant8_fp8(const Pack8& val, bool f16, float& s) {
 
 __device__ inline void quant_fp8_group128_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
                                                uint8_t* __restrict__ q, int64_t ld_q, float* __restrict__ scale,
-                                               int block, bool f16) {
+                                               long long first_group, bool f16) {
   const int groups_per_row = C / 128;
   const long long total = static_cast<long long>(R) * groups_per_row;
-  const long long gid = static_cast<long long>(block) * 16 + (threadIdx.x >> 4);
+  const long long gid = first_group + (threadIdx.x >> 4);
   const int t = threadIdx.x & 15;
   if (gid >= total) return;  // (a group's 16 lanes leave together)
   const int r = static_cast<int>(gid / groups_per_row);

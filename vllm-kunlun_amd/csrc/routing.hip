@@ -9,7 +9,8 @@ template <int SLOTS>
 __global__ __launch_bounds__(kWavesPerBlock* kWave) void softmax_topk_kernel(
     const float* __restrict__ logits, int M, int E, int K, int renorm, float* __restrict__ topk_w,
     int32_t* __restrict__ topk_ids) {
-  softmax_topk_body<SLOTS>(LogitsView{logits, 1, 0, 0}, M, E, K, renorm, topk_w, topk_ids, blockIdx.x);
+  const int m = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
+  if (m < M) softmax_topk_body<SLOTS>(LogitsView{logits, 1, 0, 0}, m, E, K, renorm, topk_w, topk_ids);
 }
 
 template <int SLOTS>
@@ -18,8 +19,10 @@ __global__ __launch_bounds__(kWavesPerBlock* kWave) void sigmoid_group_topk_kern
     int n_group, int topk_group, float scale, float* __restrict__ topk_w,
     int32_t* __restrict__ topk_ids) {
   extern __shared__ float choice_lds[];  // [kWavesPerBlock][E]
-  sigmoid_group_topk_body<SLOTS>(LogitsView{logits, 1, 0, 0}, bias, M, E, K, n_group, topk_group, scale, topk_w, topk_ids, choice_lds,
-                                 blockIdx.x);
+  const int wave = threadIdx.x >> 6, m = blockIdx.x * kWavesPerBlock + wave;
+  if (m < M)
+    sigmoid_group_topk_body<SLOTS>(LogitsView{logits, 1, 0, 0}, bias, m, E, K, n_group, topk_group, scale, topk_w, topk_ids,
+                                   choice_lds + wave * E);
 }
 
 int check_common(const float* logits, int M, int E, int K, const float* w, const int32_t* ids) {

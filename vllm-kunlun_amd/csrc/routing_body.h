@@ -157,14 +157,12 @@ __device__ inline void load_logits(const LogitsView& l, size_t row, int E, float
   }
 }
 
-// One wave per token: workgroup `block` of kWavesPerBlock waves serves tokens
-// block * kWavesPerBlock + wave. weights: false leaves topk_w alone, for callers that ask only which experts a token goes to.
+// One wave routes token m; lane k < K returns the k-th expert. weights: false leaves topk_w alone, for callers that ask only
+// which experts a token goes to.
 template <int SLOTS>
-__device__ inline void softmax_topk_body(const LogitsView& logits, int M, int E, int K, int renorm,
-                                         float* __restrict__ topk_w, int32_t* __restrict__ topk_ids, int block, bool weights = true) {
+__device__ inline int softmax_topk_body(const LogitsView& logits, int m, int E, int K, int renorm,
+                                        float* __restrict__ topk_w, int32_t* __restrict__ topk_ids, bool weights = true) {
   const int lane = lane_id();
-  const int m = block * kWavesPerBlock + (threadIdx.x >> 6);
-  if (m >= M) return;
   const size_t row = static_cast<size_t>(m) * E;
 
   float v[SLOTS];
@@ -196,24 +194,21 @@ __device__ inline void softmax_topk_body(const LogitsView& logits, int M, int E,
   float got;
   select_topk<SLOTS>(v, ok, ex, logits.type, K, lane, my_id, got);
   if (lane < K) topk_ids[static_cast<size_t>(m) * K + lane] = my_id;
-  if (!weights) return;
+  if (!weights) return my_id;
   float p = lane < K ? got / total : 0.0f;
   if (renorm) p = p / sum_in_order(p, K);  // k ascending
   if (lane < K) topk_w[static_cast<size_t>(m) * K + lane] = p;
+  return my_id;
 }
 
-// choice_lds: [kWavesPerBlock][E] floats of (dynamic) LDS.
+// choice: E floats of the wave's own in LDS (groups that are no power of two, or longer than a wave).
 template <int SLOTS>
-__device__ inline void sigmoid_group_topk_body(const LogitsView& logits, const float* __restrict__ bias, int M,
-                                               int E, int K, int n_group, int topk_group, float scale,
-                                               float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
-                                               float* choice_lds, int block, bool weights = true) {
+__device__ inline int sigmoid_group_topk_body(const LogitsView& logits, const float* __restrict__ bias, int m,
+                                              int E, int K, int n_group, int topk_group, float scale,
+                                              float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
+                                              float* choice, bool weights = true) {
   const int lane = lane_id();
-  const int wave = threadIdx.x >> 6;
-  const int m = block * kWavesPerBlock + wave;
-  if (m >= M) return;  // whole wave leaves together; no block-level sync below
   const size_t row = static_cast<size_t>(m) * E;
-  float* choice = choice_lds + wave * E;
 
   float sg[SLOTS];  // un-biased sigmoid
   float c[SLOTS];   // score used for choosing
@@ -318,12 +313,13 @@ __device__ inline void sigmoid_group_topk_body(const LogitsView& logits, const f
   float p;
   select_topk<SLOTS>(c, ok, sg, 0, K, lane, my_id, p);
   if (lane < K) topk_ids[static_cast<size_t>(m) * K + lane] = my_id;
-  if (!weights) return;
+  if (!weights) return my_id;
   if (lane >= K) p = 0.0f;
   float denom = sum_in_order(p, K);
   denom = denom + 1e-20f;
   p = (p / denom) * scale;
   if (lane < K) topk_w[static_cast<size_t>(m) * K + lane] = p;
+  return my_id;
 }
 
 }  // namespace kmoe
