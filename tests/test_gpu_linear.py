@@ -81,6 +81,19 @@ def test_tiles_of_the_split_kernel(rows, n):
     assert np.array_equal(bits(out), ref)
 
 
+# k a multiple of 2048: every wave starts its part of K at a step of its own (the next k does not), on each tile and
+# where the launch quantises the rows
+@pytest.mark.parametrize("rows,n", [(3, 64), (16, 48), (24, 4112), (64, 4112), (100, 4080), (200, 4112)])
+@pytest.mark.parametrize("k", [2048, 2112, 6144])
+def test_k_steps_begun_apart(rows, n, k):
+    kern, layer, codes, w_max = _linear(n, k, n + k)
+    x = (torch.randn(rows, k, generator=torch.Generator().manual_seed(rows)) * 1.5).bfloat16()
+    out = kern.apply_weights(layer, x.cuda())
+    xq, x_max = co.quant_i8_rows(bits(x))
+    ref, _ = co.grouped_gemm_i8(xq, x_max, codes.numpy()[None], w_max.numpy()[None], np.array([0, rows], np.int32))
+    assert np.array_equal(bits(out), ref)
+
+
 # tiles of 32 x 128, 64 x 128 and beyond: rows and channels at their edges, an odd number of 64-byte steps, both types
 @pytest.mark.parametrize("rows,n", [(289, 4096), (384, 4112), (513, 4000), (449, 7168), (1100, 4096)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

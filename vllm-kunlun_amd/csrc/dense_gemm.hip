@@ -39,7 +39,7 @@ struct DenseParams {
   int64_t ldy;
   int32_t* acc_out;
   int32_t f16;
-  int32_t rotate;  // waves start their K range at a step of their own (fragments a multiple of 64 KB apart)
+  int32_t rotate;  // waves start their K range at a step of their own (rotates(k))
 };
 
 constexpr int kDenseWaves = 8;
@@ -219,6 +219,14 @@ int launch_dense(DenseParams p, hipStream_t s) {
   return check_launch("kmoe_grouped_gemm_i8 (dense)");
 }
 
+// Fragments (16 channels of k codes) begin a multiple of 32 KB apart where this holds, and waves in step ask the same
+// channels of memory: each starts its part of K at a step of its own (whole-number sums: same bits). GEMM alone, us, all
+// waves at the first step / rotated, weights cold: [7168 x 2048] 24 rows 5.8 / 5.5, 33 7.5 / 6.6, 100 8.4 / 8.1, 128 9.3 /
+// 8.7; [4096 x 2048] 200 9.4 / 8.6; [12288 x 2048] 64 11.9 / 10.9; [6144 x 6144] 80 16.6 / 16.1; 1 to 16 rows, k = 10240 and
+// weights in cache level. Other k gain a little or lose a little: [4096 x 2560] 33 rows 5.0 / 4.8, [4096 x 1024] 100 4.7 /
+// 4.8, [4096 x 7168] 100 11.2 / 11.4.
+bool rotates(int k) { return k % 2048 == 0; }
+
 // The tiles, and what a launch on one costs: rounds of workgroups over the CUs times the KB a workgroup fetches per K step
 // (MF + NF). The cheapest tile, the smaller of equals, is within 0.2 % of the fastest on average and 7 % at worst over
 // eight matrices ([4096 x 7168], [7168 x 2048], [8192 x 8192], [12288 x 5120], [24576 x 1536], [1536 x 7168], [2048 x 2048],
@@ -282,7 +290,7 @@ int dense_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   p.ldy = a->ldy;
   p.acc_out = a->acc_out;
   p.f16 = a->act_dtype == KMOE_DT_F16;
-  p.rotate = a->k % 4096 == 0;
+  p.rotate = rotates(a->k);
   dense_cost(a->n, a->tail_rows, n_cu, &shape);
   return launch_shape(p, shape, s);
 }
@@ -355,7 +363,7 @@ extern "C" int kmoe_linear_i8(const kmoe_linear_i8_args* a, kmoe_stream_t stream
       p.y = a->y;
       p.ldy = a->ldy;
       p.f16 = a->act_dtype == KMOE_DT_F16;
-      p.rotate = a->k % 4096 == 0;
+      p.rotate = rotates(a->k);
       return shape == 0 ? launch_dense<1, 1, 8, 4, true>(p, as_stream(stream)) : launch_dense<1, 2, 5, 4, true>(p, as_stream(stream));
     }
   }
