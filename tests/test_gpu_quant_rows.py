@@ -61,3 +61,24 @@ def test_rows_of_every_kind(R, C, dtype, chunked):
         got = q.view(R, C)
     assert np.array_equal(top.cpu().numpy().view(np.uint32), want_max.view(np.uint32))
     assert np.array_equal(got.cpu().numpy(), want)
+
+
+# the widths and numbers of rows at which the threads of a row, or their vectors, change; part of the last workgroup's rows
+# are there, and rows apart from each other leave what lies between alone
+@pytest.mark.parametrize("R,C", [(9, 256), (9, 320), (30, 512), (30, 576), (256, 1088), (257, 1088), (257, 1536), (257, 1600), (256, 2048),
+                                 (257, 2048), (5, 4096), (5, 4160), (5, 16384), (5, 16448), (3, 32768), (3, 32832)])
+@pytest.mark.parametrize("chunked", [False, True])
+def test_threads_and_vectors_of_a_row(R, C, chunked):
+    from vllm_kunlun_amd import _lib as L
+    x = _rows(R, C, torch.bfloat16)
+    want, want_max = co.quant_i8_rows(bits(x))
+    apart = torch.full((R, C + 64), float("inf"), dtype=torch.bfloat16, device="cuda")
+    apart[:, :C] = x.cuda()
+    q = torch.full((R * C + 64,), 99, dtype=torch.int8, device="cuda")
+    top = torch.empty(R, dtype=torch.float32, device="cuda")
+    args = (L.ptr(apart), C + 64, R, C, L.ptr(q)) + (() if chunked else (C,)) + (L.ptr(top), L.act_dtype(apart), L.stream())
+    L.check((L.lib.kmoe_quant_i8_rows_chunked_dt if chunked else L.lib.kmoe_quant_i8_rows_dt)(*args))
+    codes = q[:R * C]
+    got = codes.view(C // 64, R, 64).transpose(0, 1).reshape(R, C) if chunked else codes.view(R, C)
+    assert np.array_equal(top.cpu().numpy().view(np.uint32), want_max.view(np.uint32))
+    assert np.array_equal(got.cpu().numpy(), want) and bool((q[R * C:] == 99).all())

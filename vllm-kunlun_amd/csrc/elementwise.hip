@@ -5,11 +5,11 @@
 namespace kmoe {
 namespace {
 
-template <int TPR, int NV>
-__global__ __launch_bounds__(256) void quant_i8_rows_kernel(const uint16_t* __restrict__ x, int64_t ld_x, int R,
-                                                           int C, int8_t* __restrict__ q, int64_t ld_q,
-                                                           float* __restrict__ row_max, int chunked, int f16) {
-  quant_i8_rows_body<TPR, NV>(x, ld_x, R, C, q, ld_q, row_max, chunked, blockIdx.x * (256 / TPR), f16 != 0);
+template <int TPR, int NV, int THREADS = 256>
+__global__ __launch_bounds__(THREADS) void quant_i8_rows_kernel(const uint16_t* __restrict__ x, int64_t ld_x, int R,
+                                                               int C, int8_t* __restrict__ q, int64_t ld_q,
+                                                               float* __restrict__ row_max, int chunked, int f16, int from) {
+  quant_i8_rows_body<TPR, NV, THREADS>(x, ld_x, R, C, q, ld_q, row_max, chunked, from + blockIdx.x * (THREADS / TPR), f16 != 0);
 }
 
 // ---------------------------------------- static and asymmetric int8 (the other modes of scaled_int8_quant)
@@ -238,29 +238,41 @@ using namespace kmoe;
 namespace {
 int quant_i8_launch(const uint16_t* x, int64_t ld_x, int R, int C, int8_t* q, int64_t ld_q, float* row_max,
                     int chunked, int f16, hipStream_t s, const char* what) {
-  if (C <= 32 * 8 * 3 && R >= 2048) {
+  auto launch = [&](auto kernel, int threads, int rows_per_group) {
+    constexpr int kMost = 1 << 21;  // rows of a launch, whose threads are counted in 32 bits
+    for (int64_t from = 0; from < R; from += kMost)
+      hipLaunchKernelGGL(kernel, dim3(ceil_div(static_cast<int>(std::min<int64_t>(kMost, R - from)), rows_per_group)), dim3(threads), 0, s, x,
+                         ld_x, R, C, q, ld_q, row_max, chunked, f16, static_cast<int>(from));
+  };
+  // (figures: us behind a launch that writes the rows)
+  if (C <= 32 * 8) {
+    launch(quant_i8_rows_kernel<32, 1>, 256, 8);
+  } else if (C <= 32 * 8 * 3 && R >= 2048) {
     // short rows, many of them (the second quantisation of a prefill batch): half a wave per row keeps every lane
     // busy and two rows' loads in flight per wave (Qwen3 shape, 65536 rows of 768: 37 -> 31 us inside the layer)
-    hipLaunchKernelGGL((quant_i8_rows_kernel<32, 3>), dim3(ceil_div(R, 8)), dim3(256), 0, s, x, ld_x, R, C, q, ld_q,
-                       row_max, chunked, f16);
+    launch(quant_i8_rows_kernel<32, 3>, 256, 8);
+  } else if (C <= 64 * 8) {
+    launch(quant_i8_rows_kernel<64, 1>, 256, 4);
   } else if (C <= 64 * 8 * 2) {
-    hipLaunchKernelGGL((quant_i8_rows_kernel<64, 2>), dim3(ceil_div(R, 4)), dim3(256), 0, s, x, ld_x, R, C, q, ld_q,
-                       row_max, chunked, f16);
+    launch(quant_i8_rows_kernel<64, 2>, 256, 4);
+  } else if (C <= 256 * 8 && R <= 256) {
+    // a workgroup's worth of threads per row while there are no more rows than CUs; beyond, the waves' starts cost more
+    // than a wave's four vectors: [64, 2048] 2.0 us (a wave per row 2.4), [256, 2048] 2.4 (2.7), [1024, 2048] 4.6 (4.4)
+    launch(quant_i8_rows_kernel<256, 1>, 256, 1);
+  } else if (C <= 64 * 8 * 3) {
+    launch(quant_i8_rows_kernel<64, 3>, 256, 4);
   } else if (C <= 64 * 8 * 4) {
-    hipLaunchKernelGGL((quant_i8_rows_kernel<64, 4>), dim3(ceil_div(R, 4)), dim3(256), 0, s, x, ld_x, R, C, q, ld_q,
-                       row_max, chunked, f16);
-  } else if (C <= 256 * 8 * 4) {
-    hipLaunchKernelGGL((quant_i8_rows_kernel<256, 4>), dim3(R), dim3(256), 0, s, x, ld_x, R, C, q, ld_q, row_max,
-                       chunked, f16);
-  } else if (C <= 256 * 8 * 8) {
-    hipLaunchKernelGGL((quant_i8_rows_kernel<256, 8>), dim3(R), dim3(256), 0, s, x, ld_x, R, C, q, ld_q, row_max,
-                       chunked, f16);
-  } else if (C <= 256 * 8 * 16) {
-    hipLaunchKernelGGL((quant_i8_rows_kernel<256, 16>), dim3(R), dim3(256), 0, s, x, ld_x, R, C, q, ld_q, row_max,
-                       chunked, f16);
-  } else {  // up to 65536 values: 128 registers of row data per thread
-    hipLaunchKernelGGL((quant_i8_rows_kernel<256, 32>), dim3(R), dim3(256), 0, s, x, ld_x, R, C, q, ld_q, row_max,
-                       chunked, f16);
+    launch(quant_i8_rows_kernel<64, 4>, 256, 4);
+  } else if (C <= 256 * 8 * 2) {
+    launch(quant_i8_rows_kernel<256, 2>, 256, 1);
+  } else if (C <= 512 * 8 * 2) {
+    launch(quant_i8_rows_kernel<512, 2, 512>, 512, 1);  // ([64, 7168] 2.5 us, with 256 threads 2.8; [1024, 7168] 8.2 / 8.6)
+  } else if (C <= 512 * 8 * 4) {
+    launch(quant_i8_rows_kernel<512, 4, 512>, 512, 1);
+  } else if (C <= 1024 * 8 * 4) {
+    launch(quant_i8_rows_kernel<1024, 4, 1024>, 1024, 1);
+  } else {  // up to 65536 values
+    launch(quant_i8_rows_kernel<1024, 8, 1024>, 1024, 1);
   }
   return check_launch(what);
 }

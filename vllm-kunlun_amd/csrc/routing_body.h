@@ -251,20 +251,19 @@ __device__ inline int sigmoid_group_topk_body(const LogitsView& logits, const fl
       if (gsize >= 4) merge([](float v) { return dpp_moved<0x4E>(v); });    // quad_perm [2,3,0,1]
       if (gsize >= 8) merge([](float v) { return dpp_moved<0x141>(v); });   // row_half_mirror
       if (gsize >= 16) merge([](float v) { return dpp_moved<0x140>(v); });  // row_mirror
-      const bool odd_row = (lane & 16) != 0, upper = lane >= 32;
       if (gsize >= 32)
-        merge([odd_row](float v) {
+        merge([](float v) {
           const uint32_t u = __builtin_bit_cast(uint32_t, v);
           const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-          const uint32_t a = r[0], b = r[1];  // (chosen between as values: between elements it is an address, and the stack)
-          return __builtin_bit_cast(float, odd_row ? a : b);
+          const uint32_t a = r[0], b = r[1];  // (chosen between as values, and nothing captured: elements and captured flags went over the stack)
+          return __builtin_bit_cast(float, (lane_id() & 16) != 0 ? a : b);
         });
       if (gsize >= 64)
-        merge([upper](float v) {
+        merge([](float v) {
           const uint32_t u = __builtin_bit_cast(uint32_t, v);
           const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-          const uint32_t a = r[0], b = r[1];  // (chosen between as values: between elements it is an address, and the stack)
-          return __builtin_bit_cast(float, upper ? a : b);
+          const uint32_t a = r[0], b = r[1];
+          return __builtin_bit_cast(float, lane_id() >= 32 ? a : b);
         });
 #pragma unroll
       for (int s = 0; s < SLOTS; ++s) {
