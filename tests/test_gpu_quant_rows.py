@@ -82,3 +82,38 @@ def test_threads_and_vectors_of_a_row(R, C, chunked):
     got = codes.view(C // 64, R, 64).transpose(0, 1).reshape(R, C) if chunked else codes.view(R, C)
     assert np.array_equal(top.cpu().numpy().view(np.uint32), want_max.view(np.uint32))
     assert np.array_equal(got.cpu().numpy(), want) and bool((q[R * C:] == 99).all())
+
+
+# rows that the down projection's launch quantises itself (32 tokens: up to four rows a wave), their last vectors in one load
+# of a lane and in two: rows of zeros, NaNs, infinities and the smallest numbers among ordinary ones
+@pytest.mark.parametrize("I", [64, 576, 1024])
+def test_rows_quantised_by_the_down_launch(I):
+    from vllm_kunlun_amd import _lib as L
+    from vllm_kunlun_amd import _plan
+    from oracle import torch_moe as tm
+    M, E, K, H = 32, 8, 2, 256
+    g = torch.Generator().manual_seed(I)
+    x = (torch.randn(M, H, generator=g) * 1.5).bfloat16()
+    x[3], x[4, 7], x[5, 0], x[6], x[7] = 0, float("inf"), float("nan"), x[6] * 2.0 ** -126, x[7] * 1e38
+    logits = torch.randn(M, E, generator=g)
+    w, ids = co._route(logits.numpy(), K, "softmax", True, None, None, 1.0, None)
+    w13q, s13 = tm.quantize_weight_per_channel(torch.randn(E * 2 * I, H, generator=g) * 0.05)
+    w2q, s2 = tm.quantize_weight_per_channel(torch.randn(E * H, I, generator=g) * 0.05)
+    w13q, w2q = w13q.view(E, 2 * I, H), w2q.view(E, H, I)
+    w13_max, w2_max = (s13 * 127.0).view(E, 2 * I), (s2 * 127.0).view(E, H)
+    d13, d2 = w13q.clone().cuda(), w2q.clone().cuda()
+    assert _plan.tile_pair_(d13, d2)
+    out = torch.empty(M, H, dtype=torch.bfloat16, device="cuda")
+    plan = _plan.make_moe_plan(L.KMOE_FMT_INT8, x.cuda(), logits.cuda(), out, K, d13, d2, w13_max.cuda(), w2_max.cuda(),
+                               scoring_func="softmax", renormalize=True)
+    plan()
+    moe_index, src, _, lod = co.align(ids, E)
+    xq, x_max = co.quant_i8_rows(bits(x))
+    act, _ = co.grouped_gemm_i8(xq, x_max, w13q.numpy(), w13_max.numpy(), lod, act=1, row_src=src, src_div=K)
+    aq, a_max = co.quant_i8_rows(act)
+    down, _ = co.grouped_gemm_i8(aq, a_max, w2q.numpy(), w2_max.numpy(), lod)
+    ref = co.combine(down, moe_index, w)
+    got, nan = bits(out), np.isnan((ref.astype(np.uint32) << 16).view(np.float32))
+    assert nan.any() and not nan.all()
+    assert np.array_equal(np.isnan((got.astype(np.uint32) << 16).view(np.float32)), nan)
+    assert np.array_equal(got[~nan], ref[~nan])
