@@ -89,6 +89,13 @@ def test_stable_sort_by_expert(P, E, first):
     assert torch.equal(expert_m, counts) and torch.equal(lod, torch.cat([torch.zeros(1), counts.cumsum(0)]).long())
 
 
+# the one launch's batches of ids (two and eight a thread) and its end, none of the pairs here and all of them
+@pytest.mark.parametrize("P", [0, 2048, 2049, 4097, 16384, 16385, 32767, 32768, 32769])
+@pytest.mark.parametrize("E,first", [(40, 0), (384, 1000), (1000, 0)])
+def test_stable_sort_in_one_launch(P, E, first):
+    test_stable_sort_by_expert(P, E, first)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fp8_group_quantiser_on_every_mantissa(dtype):
     """Groups whose maximum has every mantissa, over the exponents where the quotients come from the reciprocal and those

@@ -13,15 +13,15 @@ from oracle import c_oracle as co  # noqa: E402
 
 
 @pytest.mark.parametrize("M,E,K,quant,H,scoring,n_group", [
-    (512, 128, 8, "int8", 256, "softmax", 1), (513, 128, 8, "int8", 256, "softmax", 1),        # 4096 pairs, and the first beyond
+    (1536, 128, 8, "int8", 256, "softmax", 1), (1537, 128, 8, "int8", 256, "softmax", 1),      # 12288 pairs, and the first beyond
     (2048, 128, 8, "none", 128, "softmax", 1), (2049, 128, 8, "int8", 128, "softmax", 1),      # one token a wave, two
     (4097, 100, 8, "int8", 128, "softmax", 1), (8192, 128, 8, "int8", 128, "softmax", 1),      # three, four
     (8193, 64, 4, "int8", 128, "softmax", 1),                                                  # five: a sort of its own
     (1025, 17, 17, "none", 128, "softmax", 1), (600, 128, 64, "none", 128, "softmax", 1),      # a chunk of 1024 pairs
-    (2047, 128, 8, "int8", 128, "sigmoid", 8), (999, 130, 8, "fp8", 256, "sigmoid", 5),        # up to 128 experts; more
-    (1000, 64, 8, "fp8", 128, "sigmoid", 1), (999, 120, 8, "fp8", 256, "sigmoid", 5),          # groups of 24: scores in LDS
-    (700, 96, 8, "int8", 2048, "softmax", 1), (700, 96, 8, "int8", 2064, "softmax", 1),        # rows of a wave, of four
-    (700, 96, 8, "int8", 8192, "softmax", 1), (3000, 128, 8, "w4", 128, "softmax", 1)])
+    (2047, 128, 8, "int8", 128, "sigmoid", 8), (1999, 130, 8, "fp8", 256, "sigmoid", 5),        # up to 128 experts; more
+    (1600, 64, 8, "fp8", 128, "sigmoid", 1), (1999, 120, 8, "fp8", 256, "sigmoid", 5),          # groups of 24: scores in LDS
+    (1600, 96, 8, "int8", 2048, "softmax", 1), (1600, 96, 8, "int8", 2064, "softmax", 1),        # rows of a wave, of four
+    (1600, 96, 8, "int8", 8192, "softmax", 1), (3000, 128, 8, "w4", 128, "softmax", 1)])
 @pytest.mark.parametrize("share", [False, True])
 def test_sort_of_a_routed_batch(M, E, K, quant, H, scoring, n_group, share):
     from vllm_kunlun_amd import _lib as L, _plan, synth

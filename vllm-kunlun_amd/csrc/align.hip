@@ -17,13 +17,14 @@ constexpr int kThreads = 1024;            // workgroup size of the multi-workgro
 constexpr int kWaves = kThreads / kWave;  // 16
 constexpr int kMaxE = 1024;
 // Launches by the number of pairs. One workgroup of 256 threads and cheap barriers up to 256 pairs and experts (3.3 us a
-// call in a row of calls; 4.1 by the next). One launch of P / 1024 workgroups that each count every pair: 4.2 us at 512
-// pairs, 5.3 at 4096, 5.7 at 6216, 7.5 at 16384, 10.6 at 32768 (one workgroup for all took 4.5 us at 512 and 9.1 at 4096,
-// launches for the histograms, their scan and the scatter 10.0 at 6216, 10.3 at 16384, 11.2 at 32768). Two launches beyond,
-// where reading all the ids in every workgroup costs more than the second launch: 9.3 us at 32768 pairs, 9.4 at 65536
-// (three: 13.2), 22 at 2^20 (76). With other kernels around, a second launch costs some 2 us more than in such a row.
+// call in a row of calls; 4.1 by the next). One launch of P / 1024 workgroups that each count every pair, us behind a launch
+// that writes the ids, 256 experts: 4.0 at 512 pairs, 4.9 at 4096, 5.1 at 8192, 6.1 at 16384, 7.0 at 24000, 7.9 at 32768 (one
+// workgroup for all took 4.5 at 512 and 9.1 at 4096). Two launches beyond, where reading all the ids in every workgroup costs
+// more than the second launch: 9.4 at 32768 pairs and some 2 more with other kernels around, 9.5 at 49152 and 65536 (one: 9.8,
+// 11.6), 22 at 2^20.
 constexpr int kSingleMaxP = 256, kSingleMaxE = 256;
-constexpr int kOneLaunchMaxP = 24576;
+constexpr int kOneLaunchMaxP = 32768;
+constexpr int kNoWorkspaceMaxP = 24576;   // pairs from which on callers have to bring a workspace
 constexpr int kMaxChunks = 128;           // workgroups of the two-launch path at most
 
 // two-launch path: pairs per thread
@@ -104,7 +105,10 @@ __global__ __launch_bounds__(kSingleMaxP) void align_single_kernel(
 // One launch for several workgroups (P <= kOneLaunchMaxP): workgroup b owns the kThreads pairs of chunk b, one per
 // thread, and counts ALL the pairs itself - those of earlier chunks apart from the rest - so that it knows where its
 // chunk begins in every expert without waiting for another workgroup. Bound by latencies: a launch, the round trip of
-// the ids (eight loads in flight per thread), the barriers and the scan.
+// the ids, the barriers and the scan. kBatch loads in flight per thread: past the end the last id is read again, as loads
+// under conditions of their own went out one after another (256 experts: 8192 pairs 7.2 -> 5.1 us, 24000 12.1 -> 7.0). Two
+// where that is all of them, eight beyond (2048 pairs: 4.1, with eight 4.7; 16384 6.1, with sixteen 6.2).
+template <int kBatch>
 __global__ __launch_bounds__(kThreads) void align_one_launch_kernel(
     const IdView ids, int P, int E, int32_t* __restrict__ moe_index, int32_t* __restrict__ sorted_src,
     int32_t* __restrict__ expert_m, int32_t* __restrict__ lod) {
@@ -116,23 +120,26 @@ __global__ __launch_bounds__(kThreads) void align_one_launch_kernel(
   int* wcnt = rest + E;      // [kWaves][E]
   const int t = threadIdx.x, wave = t >> 6;
   const int begin = blockIdx.x * kThreads;
-  const int key = load_key(ids, begin + t, P, E);
-  constexpr int kBatch = 8;
+  auto id_at = [&](int j) { return ids.ids[max(min(j, P - 1), 0)]; };
+  const int my_id = id_at(begin + t);
   int v[kBatch];
   auto load = [&](int j0) {
 #pragma unroll
-    for (int i = 0; i < kBatch; ++i) v[i] = load_key(ids, j0 + i * kThreads + t, P, E);
+    for (int i = 0; i < kBatch; ++i) v[i] = id_at(j0 + i * kThreads + t);
   };
   load(0);
   for (int i = t; i < (2 + kWaves) * E; i += kThreads) before[i] = 0;
   __syncthreads();
+  const int key = key_of(my_id, ids.first, begin + t < P, E);
   int rank, count;
   wave_match_rank(key, key_bits(E), rank, count);
   if (key >= 0 && rank == 0) wcnt[wave * E + key] = count;
   for (int j0 = 0; j0 < P; j0 += kBatch * kThreads) {
 #pragma unroll
-    for (int i = 0; i < kBatch; ++i)
-      if (v[i] >= 0) atomicAdd((j0 + i * kThreads < begin ? before : rest) + v[i], 1);  // (chunks are whole: uniform)
+    for (int i = 0; i < kBatch; ++i) {
+      const int e = key_of(v[i], ids.first, j0 + i * kThreads + t < P, E);
+      if (e >= 0) atomicAdd((j0 + i * kThreads < begin ? before : rest) + e, 1);  // (chunks are whole: uniform)
+    }
     load(j0 + kBatch * kThreads);
   }
   __syncthreads();
@@ -203,10 +210,13 @@ __global__ __launch_bounds__(kThreads) void align_scatter_kernel(const IdView id
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
         const int c = c0 + i * parts;
-        v[i] = c < n_chunks ? hist[static_cast<size_t>(c) * E + e] : 0;
+        v[i] = hist[static_cast<size_t>(min(c, n_chunks - 1)) * E + e];
       }
 #pragma unroll
-      for (int i = 0; i < kBatch; ++i) (c0 + i * parts < me ? lo : hi) += v[i];
+      for (int i = 0; i < kBatch; ++i) {
+        const int c = c0 + i * parts;
+        (c < me ? lo : hi) += c < n_chunks ? v[i] : 0;
+      }
     }
     if (lo) atomicAdd(&before[e], lo);
     if (hi) atomicAdd(&rest[e], hi);
@@ -249,7 +259,7 @@ __global__ void gather_rows_kernel(const uint16_t* __restrict__ src, int64_t ld_
 using namespace kmoe;
 
 extern "C" size_t kmoe_align_workspace_bytes(int P, int E) {
-  if (P <= kOneLaunchMaxP || E <= 0) return 256;  // unused, but never report zero
+  if (P <= kNoWorkspaceMaxP || E <= 0) return 256;  // unused, but never report zero
   return align_up(static_cast<size_t>(ceil_div(P, chunk_steps(P) * kThreads)) * E * sizeof(int32_t), 256);
 }
 
@@ -274,17 +284,20 @@ extern "C" int kmoe_align_local(const int32_t* ids_global, int P, int E, int fir
                        expert_m, lod);
     return check_launch("kmoe_align");
   }
+  const int steps = chunk_steps(P), n_chunks = ceil_div(P, steps * kThreads);
+  const size_t need = static_cast<size_t>(n_chunks) * E * sizeof(int32_t);
+  if (P > kNoWorkspaceMaxP) {
+    KMOE_REQUIRE(workspace, KMOE_ERR_WORKSPACE, "align: workspace is NULL (need %zu bytes)", need);
+    KMOE_REQUIRE(workspace_bytes >= need, KMOE_ERR_WORKSPACE, "align: workspace %zu < %zu bytes", workspace_bytes,
+                 need);
+  }
   if (P <= kOneLaunchMaxP) {
-    hipLaunchKernelGGL(align_one_launch_kernel, dim3(max(1, ceil_div(P, kThreads))), dim3(kThreads),
-                       sizeof(int) * (16 + (3 + static_cast<size_t>(kWaves)) * E), s, topk_ids, P, E, moe_index, sorted_src,
+    const IdView some{P > 0 ? ids_global : lod, first_expert};  // (of no pairs: memory to read, whatever it holds)
+    hipLaunchKernelGGL((P <= 2 * kThreads ? align_one_launch_kernel<2> : align_one_launch_kernel<8>), dim3(max(1, ceil_div(P, kThreads))),
+                       dim3(kThreads), sizeof(int) * (16 + (3 + static_cast<size_t>(kWaves)) * E), s, some, P, E, moe_index, sorted_src,
                        expert_m, lod);
     return check_launch("kmoe_align");
   }
-  const int steps = chunk_steps(P), n_chunks = ceil_div(P, steps * kThreads);
-  const size_t need = static_cast<size_t>(n_chunks) * E * sizeof(int32_t);
-  KMOE_REQUIRE(workspace, KMOE_ERR_WORKSPACE, "align: workspace is NULL (need %zu bytes)", need);
-  KMOE_REQUIRE(workspace_bytes >= need, KMOE_ERR_WORKSPACE, "align: workspace %zu < %zu bytes", workspace_bytes,
-               need);
   int32_t* hist = static_cast<int32_t*>(workspace);
   hipLaunchKernelGGL(align_hist_kernel, dim3(n_chunks), dim3(kThreads), sizeof(int) * E, s, topk_ids, P, E, steps, hist);
   hipLaunchKernelGGL(align_scatter_kernel, dim3(n_chunks), dim3(kThreads),

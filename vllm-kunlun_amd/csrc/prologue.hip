@@ -9,9 +9,9 @@
 // Larger batches over up to 128 experts: TWO launches of workgroups of 1024. In the first a routing workgroup serves a chunk of
 // 16, 32, 48 or 64 tokens, a wave each or several in turn, and leaves how many of its pairs went to each expert; in the second a
 // workgroup per chunk adds those counts up and writes its pairs' places. The rows are quantised beside them, in either launch.
-// Against the sort in one launch that counts all the pairs in every workgroup, or in two of its own beyond 24576 pairs, layer, us: Qwen3
-// dims int8 777 tokens 143.8 -> 142.3, 1500 180.8 -> 177.7, 2500 218.2 -> 214.0, 4096 311.9 -> 308.5, 8192 521.3 -> 517.5, bf16 2000 292.9 ->
-// 290.5; 300 tokens 128.3 / 128.8, so from 4096 pairs on. Routing is bound by issue: 256 chunks, on all CUs, cost the second launch what they
+// Against the sort in one launch that counts all the pairs in every workgroup, or in two of its own beyond 32768 pairs, layer, us: Qwen3
+// dims int8 1024 tokens 145.9 -> 146.8, 1500 175.0 both, 2048 194.4 -> 192.3, 4096 290.9 -> 289.3, 8192 521.3 -> 517.5, bf16 2048 286.5 ->
+// 287.2, so from 12288 pairs on. Routing is bound by issue: 256 chunks, on all CUs, cost the second launch what they
 // save the first (8192 tokens 523 to 527). More experts take longer to route: DeepSeek-V3 dims 1000 tokens 1944 / 1941, 4096 2569 / 2580,
 // Kimi-K2 dims 2048 2423 / 2424: those keep the launches above and a sort behind them.
 #include "quant_body.h"
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_quant_kernel(const SortArgs
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       const int c = c0 + i * parts;
-      v[i] = adds && c < s.chunks ? s.out.counts[static_cast<size_t>(c) * E + e] : 0;
+      v[i] = s.out.counts[static_cast<size_t>(min(c, s.chunks - 1)) * E + e];
     }
   };
   load(part);
@@ -142,7 +142,10 @@ __global__ __launch_bounds__(kSortThreads) void sort_quant_kernel(const SortArgs
   for (int c0 = part; adds && c0 < s.chunks; c0 += kBatch * parts) {
     if (c0 != part) load(c0);
 #pragma unroll
-    for (int i = 0; i < kBatch; ++i) (c0 + i * parts < me ? lo : hi) += v[i];
+    for (int i = 0; i < kBatch; ++i) {
+      const int c = c0 + i * parts;
+      (c < me ? lo : hi) += c < s.chunks ? v[i] : 0;
+    }
   }
   if (lo) atomicAdd(&before[e], lo);
   if (hi) atomicAdd(&rest[e], hi);
@@ -196,7 +199,7 @@ int score_floats(const RouteArgs& r, bool sigmoid) {
 
 // Whether a batch is sorted by the launches that route it: sizes that gain (above), a pair per thread, room for the counts.
 bool sorts_with_routing(const RouteArgs& r, const SortArgs& s) {
-  return s.P > 4096 && r.E <= kSortSlots * kWave && s.tokens <= 4 * kSortWaves && s.tokens * s.K <= kSortThreads &&
+  return s.P > 12288 && r.E <= kSortSlots * kWave && s.tokens <= 4 * kSortWaves && s.tokens * s.K <= kSortThreads &&
          static_cast<size_t>(s.chunks) * s.out.E * sizeof(int32_t) <= s.out.counts_bytes;
 }
 

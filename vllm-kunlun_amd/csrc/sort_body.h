@@ -29,10 +29,13 @@ struct IdView {
   __device__ int operator[](int j) const { return ids[j] - first; }
 };
 
+// The key of an id: its expert, or -1 (ids outside [0,E), pairs past the end: no sorted row).
+__device__ inline int key_of(int id, int first, bool live, int E) {
+  const int e = id - first;
+  return live && static_cast<unsigned>(e) < static_cast<unsigned>(E) ? e : -1;
+}
 __device__ inline int load_key(const IdView ids, int j, int end, int E) {
-  if (j >= end) return -1;
-  const int e = ids[j];
-  return static_cast<unsigned>(e) < static_cast<unsigned>(E) ? e : -1;  // ids outside [0,E): no sorted row
+  return j < end ? key_of(ids.ids[j], ids.first, true, E) : -1;
 }
 
 // Exclusive scan of cnt[0..E) by one workgroup (blockDim.x >= E): a shuffle scan
