@@ -166,3 +166,19 @@ def test_nan_logits_of_a_token_leave_the_others_alone(M):
     logits[0] = torch.full((1,), -1, dtype=torch.int32).view(torch.float32).cuda()
     got = sl.layer(sl.x, logits)
     assert torch.equal(got[1:], want[1:])
+
+
+# one group a lane and two, the last workgroup full and not, rows apart from each other
+@pytest.mark.parametrize("R,C", [(511, 16384), (512, 16384), (513, 16384), (21846, 384), (1, 128)])
+def test_fp8_groups_of_large_batches(R, C):
+    from vllm_kunlun_amd import _lib as L
+    x = torch.randn(R, C, generator=torch.Generator().manual_seed(R)).bfloat16()
+    q_ref, s_ref = co.quant_fp8_group128(bits(x))
+    apart = torch.full((R, C + 8), float("inf"), dtype=torch.bfloat16, device="cuda")
+    apart[:, :C] = x.cuda()
+    q = torch.full((R * C + 64,), 99, dtype=torch.uint8, device="cuda")
+    s = torch.full((R * C // 128 + 16,), -7.0, device="cuda")
+    L.check(L.lib.kmoe_quant_fp8_group128_dt(L.ptr(apart), C + 8, R, C, L.ptr(q), C, L.ptr(s), L.act_dtype(apart, "test"), L.stream()))
+    assert np.array_equal(q[:R * C].cpu().numpy().reshape(R, C), q_ref) and bool((q[R * C:] == 99).all())
+    got = s[:R * C // 128].cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), s_ref.reshape(-1).view(np.uint32)) and bool((s[R * C // 128:] == -7).all())

@@ -21,7 +21,8 @@ from oracle import c_oracle as co  # noqa: E402
     (2047, 128, 8, "int8", 128, "sigmoid", 8), (1999, 130, 8, "fp8", 256, "sigmoid", 5),        # up to 128 experts; more
     (1600, 64, 8, "fp8", 128, "sigmoid", 1), (1999, 120, 8, "fp8", 256, "sigmoid", 5),          # groups of 24: scores in LDS
     (1600, 96, 8, "int8", 2048, "softmax", 1), (1600, 96, 8, "int8", 2064, "softmax", 1),        # rows of a wave, of four
-    (1600, 96, 8, "int8", 8192, "softmax", 1), (3000, 128, 8, "w4", 128, "softmax", 1)])
+    (1600, 96, 8, "int8", 8192, "softmax", 1), (3000, 128, 8, "w4", 128, "softmax", 1),
+    (8193, 130, 8, "fp8", 1024, "sigmoid", 5)])                                                # two groups of 128 a lane
 @pytest.mark.parametrize("share", [False, True])
 def test_sort_of_a_routed_batch(M, E, K, quant, H, scoring, n_group, share):
     from vllm_kunlun_amd import _lib as L, _plan, synth

@@ -76,10 +76,11 @@ __global__ __launch_bounds__(256) void quant_i8_rows_azp_kernel(const uint16_t* 
   }
 }
 
+template <int NV>
 __global__ __launch_bounds__(256) void quant_fp8_group128_kernel(const uint16_t* __restrict__ x, int64_t ld_x,
                                                                 int R, int C, uint8_t* __restrict__ q,
                                                                 int64_t ld_q, float* __restrict__ scale, int f16) {
-  quant_fp8_group128_body(x, ld_x, R, C, q, ld_q, scale, static_cast<long long>(blockIdx.x) * 16, f16 != 0);
+  quant_fp8_group128_body<NV>(x, ld_x, R, C, q, ld_q, scale, blockIdx.x * (16u * NV), f16 != 0);
 }
 
 // ------------------------------------------------------------ silu-and-mul
@@ -337,8 +338,9 @@ extern "C" int kmoe_quant_fp8_group128_dt(const uint16_t* x, int64_t ld_x, int R
                (long long)ld_q);
   if (R == 0) return KMOE_OK;
   const long long groups = static_cast<long long>(R) * (C / 128);
-  hipLaunchKernelGGL(quant_fp8_group128_kernel, dim3(static_cast<unsigned>((groups + 15) / 16)), dim3(256), 0,
-                     as_stream(stream), x, ld_x, R, C, q, ld_q, scale, act_dtype == KMOE_DT_F16 ? 1 : 0);
+  const int nv = groups >= kFp8TwoGroups ? 2 : 1;
+  hipLaunchKernelGGL((nv == 2 ? quant_fp8_group128_kernel<2> : quant_fp8_group128_kernel<1>), dim3(static_cast<unsigned>((groups + 16 * nv - 1) / (16 * nv))),
+                     dim3(256), 0, as_stream(stream), x, ld_x, R, C, q, ld_q, scale, act_dtype == KMOE_DT_F16 ? 1 : 0);
   return check_launch("kmoe_quant_fp8_group128");
 }
 

@@ -32,7 +32,7 @@ struct QuantArgs {
   int f16;
 };
 
-enum class Quant { None, I8Wave, I8Block, Fp8 };  // I8Wave: rows of up to 2048 values, a wave each
+enum class Quant { None, I8Wave, I8Block, Fp8, Fp8Two };  // I8Wave: rows of up to 2048 values, a wave each; Fp8Two: two groups a lane (the launch that does not sort)
 
 template <int SLOTS, bool SIGMOID>
 __device__ inline int route_token(const RouteArgs& r, int m, float* choice) {
@@ -54,8 +54,9 @@ __global__ __launch_bounds__(256) void route_quant_kernel(const RouteArgs r, con
     quant_i8_rows_body<64, 4>(q.x, q.ld_x, q.R, q.C, static_cast<int8_t*>(q.q), q.ld_q, q.aux, q.chunked, quant_at * 4, q.f16 != 0);
   } else if (Q == Quant::I8Block) {
     quant_i8_rows_body<256, 4>(q.x, q.ld_x, q.R, q.C, static_cast<int8_t*>(q.q), q.ld_q, q.aux, q.chunked, quant_at, q.f16 != 0);
-  } else if (Q == Quant::Fp8) {
-    quant_fp8_group128_body(q.x, q.ld_x, q.R, q.C, static_cast<uint8_t*>(q.q), q.ld_q, q.aux, static_cast<long long>(quant_at) * 16, q.f16 != 0);
+  } else if (Q == Quant::Fp8 || Q == Quant::Fp8Two) {
+    constexpr int NV = Q == Quant::Fp8Two ? 2 : 1;
+    quant_fp8_group128_body<NV>(q.x, q.ld_x, q.R, q.C, static_cast<uint8_t*>(q.q), q.ld_q, q.aux, quant_at * (16u * NV), q.f16 != 0);
   }
 }
 
@@ -80,8 +81,7 @@ __device__ inline void quantise_part(const QuantArgs& q, int at) {
   else if constexpr (Q == Quant::I8Block)
     quant_i8_rows_body<256, 4, kSortThreads>(q.x, q.ld_x, q.R, q.C, static_cast<int8_t*>(q.q), q.ld_q, q.aux, q.chunked, at * sort_rows(Q), q.f16 != 0);
   else if constexpr (Q == Quant::Fp8)
-    quant_fp8_group128_body(q.x, q.ld_x, q.R, q.C, static_cast<uint8_t*>(q.q), q.ld_q, q.aux, static_cast<long long>(at) * (kSortThreads / 16),
-                            q.f16 != 0);
+    quant_fp8_group128_body<1, kSortThreads>(q.x, q.ld_x, q.R, q.C, static_cast<uint8_t*>(q.q), q.ld_q, q.aux, at * (kSortThreads / 16u), q.f16 != 0);
 }
 
 // Workgroup c < s.chunks: chunk c's tokens routed, and its counts per expert (of those this launch owns) in s.out.counts.
@@ -186,8 +186,11 @@ void launch_q(const RouteArgs& r, const QuantArgs& q, Quant kind, hipStream_t s)
     case Quant::I8Wave: return launch<SLOTS, SIGMOID, Quant::I8Wave>(r, q, ceil_div(q.R, 4), s);
     case Quant::I8Block: return launch<SLOTS, SIGMOID, Quant::I8Block>(r, q, q.R, s);
     case Quant::Fp8:
-      return launch<SLOTS, SIGMOID, Quant::Fp8>(
-          r, q, static_cast<int>((static_cast<long long>(q.R) * (q.C / 128) + 15) / 16), s);
+    case Quant::Fp8Two: {
+      const long long groups = static_cast<long long>(q.R) * (q.C / 128);
+      if (groups >= kFp8TwoGroups) return launch<SLOTS, SIGMOID, Quant::Fp8Two>(r, q, static_cast<int>((groups + 31) / 32), s);
+      return launch<SLOTS, SIGMOID, Quant::Fp8>(r, q, static_cast<int>((groups + 15) / 16), s);
+    }
   }
 }
 

@@ -191,21 +191,35 @@ __device__ inline uint2 quant8_fp8(const Pack8& val, bool f16, float& s) {
   return make_uint2(w[0], w[1]);
 }
 
-__device__ inline void quant_fp8_group128_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
-                                               uint8_t* __restrict__ q, int64_t ld_q, float* __restrict__ scale,
-                                               long long first_group, bool f16) {
-  const int groups_per_row = C / 128;
-  const long long total = static_cast<long long>(R) * groups_per_row;
-  const long long gid = first_group + (threadIdx.x >> 4);
+// A workgroup of THREADS serves the groups first_group ..., THREADS / 16 at a time and NV times, read together: one group of a
+// lane makes for waves so short that their starts (some three a nanosecond) are what a large batch waits for.
+// From kFp8TwoGroups groups on two a lane: behind a launch that writes the rows, us, one / two / three / four: [24008, 2048] 24.7 /
+// 23.6 / 23.4 / 24.4, [8192, 7168] 37.7 / 35.4 / 35.4 / 37.1, [2048, 2048] 6.7 / 6.8 / 6.7 / 6.9, [512, 768] 2.1 / 2.4 / 2.7 / 2.9; inside a
+// layer of 3001 tokens the second quantisation 38.9 -> 31.3, the first, beside the routing, 21.2 -> 19.5.
+constexpr long long kFp8TwoGroups = 1 << 16;
+template <int NV, int THREADS = 256>
+__device__ __forceinline__ void quant_fp8_group128_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
+                                                        uint8_t* __restrict__ q, int64_t ld_q, float* __restrict__ scale,
+                                                        uint32_t first_group, bool f16) {
+  const uint32_t groups_per_row = C / 128, total = static_cast<uint32_t>(R) * groups_per_row;
   const int t = threadIdx.x & 15;
-  if (gid >= total) return;  // (a group's 16 lanes leave together)
-  const int r = static_cast<int>(gid / groups_per_row);
-  const int g = static_cast<int>(gid - static_cast<long long>(r) * groups_per_row);
-  Pack8 val;
-  val.v = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(r) * ld_x + g * 128 + t * 8);
-  float s;
-  *reinterpret_cast<uint2*>(q + static_cast<size_t>(r) * ld_q + g * 128 + t * 8) = quant8_fp8(val, f16, s);
-  if (t == 0) scale[static_cast<size_t>(r) * groups_per_row + g] = s;
+  Pack8 val[NV];
+  uint32_t gid[NV], r[NV], g[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    gid[i] = first_group + i * (THREADS / 16) + (threadIdx.x >> 4);
+    const uint32_t at = min(gid[i], total - 1);
+    r[i] = at / groups_per_row;
+    g[i] = at - r[i] * groups_per_row;
+    val[i].v = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(r[i]) * ld_x + g[i] * 128 + t * 8);
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    if (gid[i] >= total) return;  // (a group's 16 lanes leave together)
+    float s;
+    *reinterpret_cast<uint2*>(q + static_cast<size_t>(r[i]) * ld_q + g[i] * 128 + t * 8) = quant8_fp8(val[i], f16, s);
+    if (t == 0) scale[static_cast<size_t>(r[i]) * groups_per_row + g[i]] = s;
+  }
 }
 
 }  // namespace kmoe
