@@ -60,12 +60,18 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
   const int pair = m * p.K + wave;
   const int nvec = p.I / 8;
   Pack8 val[kVecs];
+  // (layer, us, loads under conditions / together: Qwen3 dims int8 4 tokens 30.2 / 29.7, DeepSeek-V3 dims 1 token int8 66.8 / 66.5, fp8
+  // 71.7 / 70.6; 16-bit and 4-bit rows, more registers and fewer waves, lose: bf16 4 tokens 48.4 / 53.9, Kimi-K2 dims 47.5 / 51.4)
   auto load_row = [&](int row) __attribute__((always_inline)) {
     const uint4* src = reinterpret_cast<const uint4*>(p.act + static_cast<size_t>(row) * p.I);
 #pragma unroll
     for (int i = 0; i < kVecs; ++i) {
-      val[i].v = make_uint4(0, 0, 0, 0);
-      if (lane + i * kWave < nvec) val[i].v = src[lane + i * kWave];
+      if constexpr (QUANT) {  // lanes past the end read the last vector again: the loads go out together
+        val[i].v = src[min(lane + i * kWave, nvec - 1)];
+      } else {
+        val[i].v = make_uint4(0, 0, 0, 0);
+        if (lane + i * kWave < nvec) val[i].v = src[lane + i * kWave];
+      }
     }
   };
   int k = wave, e, row;
