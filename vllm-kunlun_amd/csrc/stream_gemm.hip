@@ -412,9 +412,11 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
               }
           }
           if (kb + D < klen) load_step(d, kb_of(kb + D));
-          // F8: a step's loads stay ahead of the next step's wait and scaling, where the compiler would sink them (DeepSeek-V3 dims,
-          // layer, 8 tokens 415 -> 413 us, 23 906.8 -> 902.9, 64 1454 -> 1446, 128 1668 -> 1656, 256 1792 -> 1774; other formats level)
-          if constexpr (FMT == Fmt::F8) __builtin_amdgcn_sched_barrier(0);
+          // F8, K split two ways (long streams, many columns): a step's loads stay ahead of the next step's wait and scaling, where the
+          // compiler would sink them (DeepSeek-V3 dims, layer, 8 tokens 393 -> 389 us, 23 898 -> 891, 64 1469 -> 1462, 128 1633 -> 1619, 256 1806 ->
+          // 1787; other formats level). Not where K is whole or split four ways: 64 experts of [2816 x 2048], top 6, layer, 32 tokens 93.5 -> 98.4
+          // us with it in the split launches, 100.3 in all; 100 of [1024 x 1024], top 8, 44.6 -> 48.3; 16 of [8192 x 4096], top 2, 138.1 -> 136.6.
+          if constexpr (FMT == Fmt::F8 && KS == 2) __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
