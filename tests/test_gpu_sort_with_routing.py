@@ -1,6 +1,7 @@
-"""Batches whose pairs are sorted by the launches that route and quantise them: what the sort leaves - row ranges, counts, places and their
-inverse - and the quantised rows, on both sides of the sizes where a wave routes one token, two and four, of the rule's ends, and for an
-expert-parallel share, against the stand-alone sort of the ids the routing left and the oracle's quantiser."""
+"""What a batch's launches before the first GEMM leave: experts and weights against the oracle's routing, the sort - row ranges, counts,
+places and their inverse - against a stable sort of those experts, and the quantised rows against the oracle's quantiser. On both sides of
+the sizes where the sort goes from one launch to two and the fp8 quantiser to two groups a lane, for an expert-parallel share, and for
+groups whose scores lie in LDS."""
 import numpy as np
 import pytest
 import torch
@@ -13,13 +14,13 @@ from oracle import c_oracle as co  # noqa: E402
 
 
 @pytest.mark.parametrize("M,E,K,quant,H,scoring,n_group", [
-    (1536, 128, 8, "int8", 256, "softmax", 1), (1537, 128, 8, "int8", 256, "softmax", 1),      # 12288 pairs, and the first beyond
-    (2048, 128, 8, "none", 128, "softmax", 1), (2049, 128, 8, "int8", 128, "softmax", 1),      # one token a wave, two
-    (4097, 100, 8, "int8", 128, "softmax", 1), (8192, 128, 8, "int8", 128, "softmax", 1),      # three, four
-    (8193, 64, 4, "int8", 128, "softmax", 1),                                                  # five: a sort of its own
-    (1025, 17, 17, "none", 128, "softmax", 1), (600, 128, 64, "none", 128, "softmax", 1),      # a chunk of 1024 pairs
-    (2047, 128, 8, "int8", 128, "sigmoid", 8), (1999, 130, 8, "fp8", 256, "sigmoid", 5),        # up to 128 experts; more
-    (1600, 64, 8, "fp8", 128, "sigmoid", 1), (1999, 120, 8, "fp8", 256, "sigmoid", 5),          # groups of 24: scores in LDS
+    (1536, 128, 8, "int8", 256, "softmax", 1), (1537, 128, 8, "int8", 256, "softmax", 1),
+    (2048, 128, 8, "none", 128, "softmax", 1), (2049, 128, 8, "int8", 128, "softmax", 1),
+    (4097, 100, 8, "int8", 128, "softmax", 1), (8192, 128, 8, "int8", 128, "softmax", 1),      # 32776 pairs: two launches
+    (8193, 64, 4, "int8", 128, "softmax", 1),                                                  # 32772
+    (1025, 17, 17, "none", 128, "softmax", 1), (600, 128, 64, "none", 128, "softmax", 1),      # every expert; the most a token may have
+    (2047, 128, 8, "int8", 128, "sigmoid", 8), (1999, 130, 8, "fp8", 256, "sigmoid", 5),        # groups of 16; of 26: scores in LDS
+    (1600, 64, 8, "fp8", 128, "sigmoid", 1), (1999, 120, 8, "fp8", 256, "sigmoid", 5),          # no groups; of 24
     (1600, 96, 8, "int8", 2048, "softmax", 1), (1600, 96, 8, "int8", 2064, "softmax", 1),        # rows of a wave, of four
     (1600, 96, 8, "int8", 8192, "softmax", 1), (3000, 128, 8, "w4", 128, "softmax", 1),
     (8193, 130, 8, "fp8", 1024, "sigmoid", 5)])                                                # two groups of 128 a lane
@@ -51,15 +52,18 @@ def test_sort_of_a_routed_batch(M, E, K, quant, H, scoring, n_group, share):
                                group_size=128 if quant == "w4" else None, first_expert=E // 2 if share else 0)
     plan()
     first = E // 2 if share else 0
-    ids = plan.view("topk_ids", P, torch.int32).clone()
-    want = [torch.full((n,), -7, dtype=torch.int32, device="cuda") for n in (P, P, E, E + 1)]
-    nbytes = L.lib.kmoe_align_workspace_bytes(P, E)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
-    L.check(L.lib.kmoe_align_local(L.ptr(ids), P, E, first, *(L.ptr(t) for t in want), L.ptr(ws), nbytes, L.stream()))
-    live = int(want[3][-1])
-    got = [plan.view(n, c, torch.int32) for n, c in (("moe_index", P), ("sorted_src", P), ("expert_m", E), ("lod", E + 1))]
-    assert torch.equal(got[0], want[0]) and torch.equal(got[1][:live], want[1][:live])
-    assert torch.equal(got[2], want[2]) and torch.equal(got[3], want[3])
+    w_ref, ids_ref = co._route(logits.cpu().numpy(), K, scoring, True, n_group, shape.topk_group, shape.routed_scale,
+                               sl.bias.cpu().numpy() if sl.bias is not None and not share else None)
+    assert np.array_equal(plan.view("topk_ids", P, torch.int32).cpu().numpy(), ids_ref.ravel())
+    assert np.array_equal(plan.view("topk_w", P, torch.float32).cpu().numpy().view(np.uint32), w_ref.ravel().view(np.uint32))
+    key = ids_ref.ravel() - first
+    here = np.flatnonzero((key >= 0) & (key < E))
+    src = here[np.argsort(key[here], kind="stable")]
+    place = np.full(P, -1, np.int32)
+    place[src] = np.arange(src.size)
+    counts = np.bincount(key[here], minlength=E)
+    for name, want in (("moe_index", place), ("sorted_src", src), ("expert_m", counts), ("lod", np.concatenate([[0], counts.cumsum()]))):
+        assert np.array_equal(plan.view(name, want.size, torch.int32).cpu().numpy(), want), name
     if quant in ("int8", "fp8") and not plan.layout.codes_chunked:
         ref = co.quant_i8_rows(bits(sl.x)) if quant == "int8" else co.quant_fp8_group128(bits(sl.x))
         codes = plan.view("xq", M * H, torch.uint8).cpu().numpy().reshape(M, H)

@@ -695,16 +695,11 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   const bool few_down = few && few_down_pays(a, fold);
   const bool few_routed = few && few_gate_up_takes(a);
   RouteArgs route{logits, a->bias, M, Eg, K, a->renormalize, a->n_group, a->topk_group, a->routed_scale, topk_w, topk_ids};
-  // (the counts of the sort that goes with the routing lie where the down projection's rows will)
-  const SortOut sort_out{moe_index, sorted_src, static_cast<int32_t*>(at(L.expert_m)), lod, E, a->first_expert,
-                         static_cast<int32_t*>(at(L.down)), static_cast<size_t>(P) * H * 2};
-  bool sorted = false;
   if (few_routed)
     rc = check_route(&route, a->scoring == KMOE_SCORE_SIGMOID);  // (the gate_up launch does it, and steps 2 and 3)
   else
     rc = route_and_quantise(route, a->scoring == KMOE_SCORE_SIGMOID, a->format, a->x, H, at(L.xq),
-                            static_cast<float*>(at(L.xmax)), stream_mode, f16, scan_in_gemm ? nullptr : &sort_out, &quant_done,
-                            &sorted, as_stream(stream));
+                            static_cast<float*>(at(L.xmax)), stream_mode, f16, &quant_done, as_stream(stream));
   if (rc) return rc;
   mark(KMOE_STAGE_ROUTING, 1);
   // 2. stable sort of the routed pairs by expert. On the weight-streaming path (a few rows per expert) the gate_up
@@ -714,7 +709,7 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   int2* slot_rows = per_pair ? static_cast<int2*>(at(L.align_ws)) : nullptr;
   const StreamScan scan{topk_ids, P, lod, static_cast<int32_t*>(at(L.expert_m)), moe_index, sorted_src, slot_rows};
   const StreamSlots slots{topk_ids, slot_rows, P};
-  if (!scan_in_gemm && !sorted) {
+  if (!scan_in_gemm) {
     rc = kmoe_align_local(topk_ids, P, E, a->first_expert, moe_index, sorted_src, static_cast<int32_t*>(at(L.expert_m)), lod,
                           at(L.align_ws), kmoe_align_workspace_bytes(P, E), stream);
     if (rc) return rc;

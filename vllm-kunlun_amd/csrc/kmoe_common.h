@@ -161,18 +161,10 @@ constexpr int kFewRowBytes = 25 * 1024;  // of LDS for the rows of a launch: fiv
 int few_gate_up(const FewGateUp& p, int format, bool sigmoid, hipStream_t stream);
 // The checks of the routing arguments (and n_group <= 1 made one group).
 int check_route(RouteArgs* r, bool sigmoid);
-// What the sort of the routed pairs leaves (kmoe_align_local) for E experts from `first` on, and room for counts of its own.
-struct SortOut {
-  int32_t *moe_index, *sorted_src, *expert_m, *lod;
-  int32_t E, first;
-  int32_t* counts;
-  size_t counts_bytes;
-};
 // Routing of M tokens and, for KMOE_FMT_INT8 / _FP8_BLOCK where the kernel takes the row length, the quantisation of
-// x [M,H] in the same launch (*quantised says whether it was); with `sort` the sort of the pairs too, in two launches, where
-// their number and the room for the counts allow (*sorted). M >= 1.
+// x [M,H] in the same launch (*quantised says whether it was). M >= 1.
 int route_and_quantise(RouteArgs r, bool sigmoid, int format, const uint16_t* x, int H, void* xq, float* x_aux,
-                       bool chunked, bool f16, const SortOut* sort, bool* quantised, bool* sorted, hipStream_t stream);
+                       bool chunked, bool f16, bool* quantised, hipStream_t stream);
 
 // Router GEMM pieces for the fused layer: the split (ks planes, mf*16 tokens per wave) chosen for
 // a shape, and the launch that leaves the partial planes [ks][M][E] (ks == 1: the logits).

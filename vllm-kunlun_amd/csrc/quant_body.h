@@ -76,14 +76,16 @@ __device__ inline float amax8(const Pack8& v, bool f16) {
 }
 
 // TPR threads cooperate on one row (32: two rows per wave); each keeps NV vectors of 8 values in
-// registers, so the row is read from memory once. A workgroup of THREADS serves rows first_row ... Few rows are bound by
+// registers, so the row is read from memory once. A workgroup of THREADS serves rows first_row ..., or the one row first_row
+// where that is a row's threads, more than a wave. Few rows are bound by
 // the trip to memory: lanes past the row's end read its last vector again (which changes no maximum), because loads under
 // conditions of their own went out one after another, each waiting for the one before. [64, 7168] 3.7 -> 2.8 us, [8, 2048]
 // 3.3 -> 2.3, [4096, 7168] 16.8 -> 15.1, [8192, 768] 8.7 -> 7.9 (behind a launch that writes the rows).
 template <int TPR, int NV, int THREADS = 256>
 __device__ __forceinline__ void quant_i8_rows_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
-                                          int8_t* __restrict__ q, int64_t ld_q, float* __restrict__ row_max,
-                                          int chunked, int first_row, bool f16 = false) {
+                                                   int8_t* __restrict__ q, int64_t ld_q, float* __restrict__ row_max,
+                                                   int chunked, int first_row, bool f16 = false) {
+  static_assert(TPR <= kWave || TPR == THREADS, "rows of several waves have a workgroup each");
   __shared__ uint32_t red[THREADS / kWave];
   const int t = threadIdx.x % TPR;
   const int r = first_row + threadIdx.x / TPR;
@@ -96,31 +98,26 @@ __device__ __forceinline__ void quant_i8_rows_body(const uint16_t* __restrict__ 
   uint32_t mag = 0;
 #pragma unroll
   for (int i = 0; i < NV; ++i) mag = max_magnitudes(mag, magnitudes8(val[i]));
-  // max over the row's threads (rows of several waves: all of the workgroup's meet at the barrier)
+  // max over the row's threads (one row per workgroup: combine the waves)
   auto row_max_of = [&](uint32_t m) {
     m = group_max_u32<(TPR < kWave ? TPR : kWave)>(m);
     if (TPR > kWave) {
       if (lane_id() == 0) red[threadIdx.x >> 6] = m;
       __syncthreads();
-      const uint32_t* mine = red + threadIdx.x / TPR * (TPR / kWave);
-      m = mine[0];
+      m = red[0];
 #pragma unroll
-      for (int w = 1; w < TPR / kWave; ++w) m = max(m, mine[w]);
+      for (int w = 1; w < TPR / kWave; ++w) m = max(m, red[w]);
     }
     return m;
   };
   RowScale s = row_scale_i8(row_max_of(max_of_pair(mag)), f16);
-  // (the same for all of a row's threads; several rows with barriers go in together)
-  if (TPR > kWave && THREADS > TPR ? __syncthreads_or(!s.numbers) != 0 : !s.numbers) {
+  if (!s.numbers) {  // (the same for all of a row's threads)
     float m = 0.0f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) m = fmaxf(m, amax8(val[i], f16));
     if (TPR > kWave) __syncthreads();  // (every wave has read the maxima it is about to replace)
-    m = __builtin_bit_cast(float, row_max_of(__builtin_bit_cast(uint32_t, m)));  // (no negative numbers: ordered as their bits)
-    if (!s.numbers) {
-      s.amax = m;
-      s.inv = m > 0.0f ? 127.0f / m : 0.0f;
-    }
+    s.amax = __builtin_bit_cast(float, row_max_of(__builtin_bit_cast(uint32_t, m)));  // (no negative numbers: ordered as their bits)
+    s.inv = s.amax > 0.0f ? 127.0f / s.amax : 0.0f;
   }
   if (!live) return;
   // row-major: vector v of the row; chunk-major [C/64][R][64]: vector v is eighth v%8 of chunk v/8
@@ -191,13 +188,13 @@ __device__ inline uint2 quant8_fp8(const Pack8& val, bool f16, float& s) {
   return make_uint2(w[0], w[1]);
 }
 
-// A workgroup of THREADS serves the groups first_group ..., THREADS / 16 at a time and NV times, read together: one group of a
+// A workgroup of 256 serves the groups first_group ..., 16 at a time and NV times, read together: one group of a
 // lane makes for waves so short that their starts (some three a nanosecond) are what a large batch waits for.
 // From kFp8TwoGroups groups on two a lane: behind a launch that writes the rows, us, one / two / three / four: [24008, 2048] 24.7 /
 // 23.6 / 23.4 / 24.4, [8192, 7168] 37.7 / 35.4 / 35.4 / 37.1, [2048, 2048] 6.7 / 6.8 / 6.7 / 6.9, [512, 768] 2.1 / 2.4 / 2.7 / 2.9; inside a
 // layer of 3001 tokens the second quantisation 38.9 -> 31.3, the first, beside the routing, 21.2 -> 19.5.
 constexpr long long kFp8TwoGroups = 1 << 16;
-template <int NV, int THREADS = 256>
+template <int NV>
 __device__ __forceinline__ void quant_fp8_group128_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
                                                         uint8_t* __restrict__ q, int64_t ld_q, float* __restrict__ scale,
                                                         uint32_t first_group, bool f16) {
@@ -207,7 +204,7 @@ __device__ __forceinline__ void quant_fp8_group128_body(const uint16_t* __restri
   uint32_t gid[NV], r[NV], g[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    gid[i] = first_group + i * (THREADS / 16) + (threadIdx.x >> 4);
+    gid[i] = first_group + i * 16 + (threadIdx.x >> 4);
     const uint32_t at = min(gid[i], total - 1);
     r[i] = at / groups_per_row;
     g[i] = at - r[i] * groups_per_row;

@@ -175,11 +175,11 @@ __device__ inline void load_logits(const LogitsView& l, size_t row, int E, float
   }
 }
 
-// One wave routes token m; lane k < K returns the k-th expert. weights: false leaves topk_w alone, for callers that ask only
+// One wave routes token m. weights: false leaves topk_w alone, for callers that ask only
 // which experts a token goes to.
 template <int SLOTS>
-__device__ inline int softmax_topk_body(const LogitsView& logits, int m, int E, int K, int renorm,
-                                        float* __restrict__ topk_w, int32_t* __restrict__ topk_ids, bool weights = true) {
+__device__ inline void softmax_topk_body(const LogitsView& logits, int m, int E, int K, int renorm,
+                                         float* __restrict__ topk_w, int32_t* __restrict__ topk_ids, bool weights = true) {
   const int lane = lane_id();
   const size_t row = static_cast<size_t>(m) * E;
 
@@ -212,19 +212,18 @@ __device__ inline int softmax_topk_body(const LogitsView& logits, int m, int E, 
   float got;
   select_topk<SLOTS>(v, ok, ex, logits.type, K, lane, my_id, got);
   if (lane < K) topk_ids[static_cast<size_t>(m) * K + lane] = my_id;
-  if (!weights) return my_id;
+  if (!weights) return;
   float p = lane < K ? got / total : 0.0f;
   if (renorm) p = p / sum_in_order(p, K);  // k ascending
   if (lane < K) topk_w[static_cast<size_t>(m) * K + lane] = p;
-  return my_id;
 }
 
 // choice: E floats of the wave's own in LDS (groups that are no power of two, or longer than a wave).
 template <int SLOTS>
-__device__ inline int sigmoid_group_topk_body(const LogitsView& logits, const float* __restrict__ bias, int m,
-                                              int E, int K, int n_group, int topk_group, float scale,
-                                              float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
-                                              float* choice, bool weights = true) {
+__device__ inline void sigmoid_group_topk_body(const LogitsView& logits, const float* __restrict__ bias, int m,
+                                               int E, int K, int n_group, int topk_group, float scale,
+                                               float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
+                                               float* choice, bool weights = true) {
   const int lane = lane_id();
   const size_t row = static_cast<size_t>(m) * E;
 
@@ -330,13 +329,12 @@ __device__ inline int sigmoid_group_topk_body(const LogitsView& logits, const fl
   float p;
   select_topk<SLOTS>(c, ok, sg, 0, K, lane, my_id, p);
   if (lane < K) topk_ids[static_cast<size_t>(m) * K + lane] = my_id;
-  if (!weights) return my_id;
+  if (!weights) return;
   if (lane >= K) p = 0.0f;
   float denom = sum_in_order(p, K);
   denom = denom + 1e-20f;
   p = (p / denom) * scale;
   if (lane < K) topk_w[static_cast<size_t>(m) * K + lane] = p;
-  return my_id;
 }
 
 }  // namespace kmoe
