@@ -96,6 +96,13 @@ def test_stable_sort_in_one_launch(P, E, first):
     test_stable_sort_by_expert(P, E, first)
 
 
+# the ends of the rule that goes by the number of experts
+@pytest.mark.parametrize("P", [24576, 24577, 32768, 32769])
+@pytest.mark.parametrize("E,first", [(1, 0), (63, 0), (64, 7)])
+def test_stable_sort_by_number_of_experts(P, E, first):
+    test_stable_sort_by_expert(P, E, first)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fp8_group_quantiser_on_every_mantissa(dtype):
     """Groups whose maximum has every mantissa, over the exponents where the quotients come from the reciprocal and those

@@ -20,10 +20,14 @@ constexpr int kMaxE = 1024;
 // that writes the ids, 256 experts: 4.0 at 512 pairs, 4.9 at 4096, 5.1 at 8192, 6.1 at 16384, 7.0 at 24000, 7.9 at 32768 (one
 // workgroup for all took 4.5 at 512 and 9.1 at 4096). Two launches beyond, where reading all the ids in every workgroup costs
 // more than the second launch: 9.4 at 32768 pairs and some 2 more with other kernels around, 9.5 at 49152 and 65536 (one: 9.8,
-// 11.6), 22 at 2^20.
+// 11.6), 22 at 2^20. Counting in every workgroup is what few experts, or few that most pairs go to, make slow (atomics on the
+// same counters): beyond kNoWorkspaceMaxP pairs one launch from 64 experts on. One / two there, us with the ids' launch, 28000
+// pairs: 8 experts 11.5 / 10.0, 16 10.2 / 10.4, 32 9.5 / 10.5, 64 9.6 / 11.0, 256 10.0 / 11.9, 1024 11.2 / 14.9; half of the pairs on a sixteenth
+// of the experts: 8 18.9 / 10.2, 32 13.6 / 10.4, 64 11.4 / 10.7, 128 10.4 / 11.3, 256 9.8 / 11.6.
 constexpr int kSingleMaxP = 256, kSingleMaxE = 256;
-constexpr int kOneLaunchMaxP = 32768;
-constexpr int kNoWorkspaceMaxP = 24576;   // pairs from which on callers have to bring a workspace
+// Pairs beyond which callers have to bring a workspace, by their number alone (one launch does not look at it).
+constexpr int kNoWorkspaceMaxP = 24576;
+inline bool takes_one_launch(int P, int E) { return P <= kNoWorkspaceMaxP || (P <= 32768 && E >= 64); }
 constexpr int kMaxChunks = 128;           // workgroups of the two-launch path at most
 
 // two-launch path: pairs per thread
@@ -162,7 +166,7 @@ __global__ __launch_bounds__(kSingleMaxP) void align_single_kernel(
   scatter_chunk(ids, 0, P, E, 1, base, wcnt, moe_index, sorted_src);
 }
 
-// One launch for several workgroups (P <= kOneLaunchMaxP): workgroup b owns the kThreads pairs of chunk b, one per
+// One launch for several workgroups (takes_one_launch): workgroup b owns the kThreads pairs of chunk b, one per
 // thread, and counts ALL the pairs itself - those of earlier chunks apart from the rest - so that it knows where its
 // chunk begins in every expert without waiting for another workgroup. Bound by latencies: a launch, the round trip of
 // the ids, the barriers and the scan. kBatch loads in flight per thread: past the end the last id is read again, as loads
@@ -351,7 +355,7 @@ extern "C" int kmoe_align_local(const int32_t* ids_global, int P, int E, int fir
     KMOE_REQUIRE(workspace_bytes >= need, KMOE_ERR_WORKSPACE, "align: workspace %zu < %zu bytes", workspace_bytes,
                  need);
   }
-  if (P <= kOneLaunchMaxP) {
+  if (takes_one_launch(P, E)) {
     const IdView some{P > 0 ? ids_global : lod, first_expert};  // (of no pairs: memory to read, whatever it holds)
     hipLaunchKernelGGL((P <= 2 * kThreads ? align_one_launch_kernel<2> : align_one_launch_kernel<8>), dim3(max(1, ceil_div(P, kThreads))),
                        dim3(kThreads), sizeof(int) * (16 + (3 + static_cast<size_t>(kWaves)) * E), s, some, P, E, moe_index, sorted_src,
