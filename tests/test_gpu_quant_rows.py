@@ -84,6 +84,20 @@ def test_threads_and_vectors_of_a_row(R, C, chunked):
     assert np.array_equal(got.cpu().numpy(), want) and bool((q[R * C:] == 99).all())
 
 
+# short rows, four of them a wave: parts of a wave's rows there, both sides of the widths and of the number of rows
+@pytest.mark.parametrize("R,C", [(1, 16), (15, 128), (17, 64), (2047, 192), (2048, 192), (2049, 256), (2051, 128), (2050, 144)])
+def test_short_rows(R, C):
+    from vllm_kunlun_amd import _lib as L
+    x = _rows(R, C, torch.bfloat16)
+    want, want_max = co.quant_i8_rows(bits(x))
+    dx = x.cuda()
+    q = torch.full((R * C + 64,), 99, dtype=torch.int8, device="cuda")
+    top = torch.full((R + 16,), -7.0, device="cuda")
+    L.check(L.lib.kmoe_quant_i8_rows_dt(L.ptr(dx), C, R, C, L.ptr(q), C, L.ptr(top), 0, L.stream()))
+    assert np.array_equal(top[:R].cpu().numpy().view(np.uint32), want_max.view(np.uint32)) and bool((top[R:] == -7).all())
+    assert np.array_equal(q[:R * C].view(R, C).cpu().numpy(), want) and bool((q[R * C:] == 99).all())
+
+
 # rows that the down projection's launch quantises itself (32 tokens: up to four rows a wave), their last vectors in one load
 # of a lane and in two: rows of zeros, NaNs, infinities and the smallest numbers among ordinary ones
 @pytest.mark.parametrize("I", [64, 576, 1024])

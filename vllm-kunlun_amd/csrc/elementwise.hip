@@ -246,7 +246,12 @@ int quant_i8_launch(const uint16_t* x, int64_t ld_x, int R, int C, int8_t* q, in
                          ld_x, R, C, q, ld_q, row_max, chunked, f16, static_cast<int>(from));
   };
   // (figures: us behind a launch that writes the rows)
-  if (C <= 32 * 8) {
+  if (C <= 16 * 8) {
+    // four rows a wave: many short rows are bound by the starts of waves ([65536, 128] 6.7 us, two rows a wave 10.4, a branch per load 9.3)
+    launch(quant_i8_rows_kernel<16, 1>, 256, 16);
+  } else if (C <= 32 * 8 && R >= 2048) {
+    launch(quant_i8_rows_kernel<16, 2>, 256, 16);  // ([65536, 256] 9.1 us, two rows a wave 11.4; [64, 256] 2.02 / 1.94)
+  } else if (C <= 32 * 8) {
     launch(quant_i8_rows_kernel<32, 1>, 256, 8);
   } else if (C <= 32 * 8 * 3 && R >= 2048) {
     // short rows, many of them (the second quantisation of a prefill batch): half a wave per row keeps every lane
@@ -257,8 +262,8 @@ int quant_i8_launch(const uint16_t* x, int64_t ld_x, int R, int C, int8_t* q, in
   } else if (C <= 64 * 8 * 2) {
     launch(quant_i8_rows_kernel<64, 2>, 256, 4);
   } else if (C <= 256 * 8 && R <= 256) {
-    // a workgroup's worth of threads per row while there are no more rows than CUs; beyond, the waves' starts cost more
-    // than a wave's four vectors: [64, 2048] 2.0 us (a wave per row 2.4), [256, 2048] 2.4 (2.7), [1024, 2048] 4.6 (4.4)
+    // a workgroup's worth of threads per row for few rows; beyond, the waves' starts cost more than a wave's four vectors:
+    // [64, 2048] 2.0 us (a wave per row 2.4), [256, 2048] 2.4 (2.7), [1024, 2048] 4.6 (4.4)
     launch(quant_i8_rows_kernel<256, 1>, 256, 1);
   } else if (C <= 64 * 8 * 3) {
     launch(quant_i8_rows_kernel<64, 3>, 256, 4);
