@@ -98,6 +98,21 @@ def test_short_rows(R, C):
     assert np.array_equal(q[:R * C].view(R, C).cpu().numpy(), want) and bool((q[R * C:] == 99).all())
 
 
+# rows of more bytes than the memory-side cache, whose vectors are asked for in turn, on both sides of its widths and size
+@pytest.mark.parametrize("R,C", [(43690, 3072), (42368, 3136), (32767, 4096), (32768, 4096), (32264, 4160), (29128, 4608), (28728, 4672)])
+def test_rows_beyond_the_memory_side_cache(R, C):
+    from vllm_kunlun_amd import _lib as L
+    few = 64
+    x = _rows(few, C, torch.bfloat16)
+    want, want_max = co.quant_i8_rows(bits(x))
+    dx = x.cuda().repeat(-(-R // few), 1)[:R].contiguous()
+    q = torch.empty(R, C, dtype=torch.int8, device="cuda")
+    top = torch.empty(R, dtype=torch.float32, device="cuda")
+    L.check(L.lib.kmoe_quant_i8_rows_dt(L.ptr(dx), C, R, C, L.ptr(q), C, L.ptr(top), 0, L.stream()))
+    dw, dm = torch.from_numpy(want).cuda(), torch.from_numpy(want_max.copy()).view(torch.int32).cuda()
+    assert torch.equal(q, dw.repeat(-(-R // few), 1)[:R]) and torch.equal(top.view(torch.int32), dm.repeat(-(-R // few))[:R])
+
+
 # rows that the down projection's launch quantises itself (32 tokens: up to four rows a wave), their last vectors in one load
 # of a lane and in two: rows of zeros, NaNs, infinities and the smallest numbers among ordinary ones
 @pytest.mark.parametrize("I", [64, 576, 1024])

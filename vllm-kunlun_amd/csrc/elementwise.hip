@@ -5,11 +5,11 @@
 namespace kmoe {
 namespace {
 
-template <int TPR, int NV, int THREADS = 256>
+template <int TPR, int NV, int THREADS = 256, bool IN_TURN = false>
 __global__ __launch_bounds__(THREADS) void quant_i8_rows_kernel(const uint16_t* __restrict__ x, int64_t ld_x, int R,
                                                                int C, int8_t* __restrict__ q, int64_t ld_q,
                                                                float* __restrict__ row_max, int chunked, int f16, int from) {
-  quant_i8_rows_body<TPR, NV, THREADS>(x, ld_x, R, C, q, ld_q, row_max, chunked, from + blockIdx.x * (THREADS / TPR), f16 != 0);
+  quant_i8_rows_body<TPR, NV, THREADS, IN_TURN>(x, ld_x, R, C, q, ld_q, row_max, chunked, from + blockIdx.x * (THREADS / TPR), f16 != 0);
 }
 
 // ---------------------------------------- static and asymmetric int8 (the other modes of scaled_int8_quant)
@@ -269,6 +269,12 @@ int quant_i8_launch(const uint16_t* x, int64_t ld_x, int R, int C, int8_t* q, in
     launch(quant_i8_rows_kernel<64, 3>, 256, 4);
   } else if (C <= 64 * 8 * 4) {
     launch(quant_i8_rows_kernel<64, 4>, 256, 4);
+  } else if (C > 3072 && C <= 4608 && static_cast<int64_t>(R) * C >= 1 << 27) {
+    // What the memory-side cache does not hold comes faster with fewer loads in flight. Together / in turn: [65536, 3072] 102.9
+    // / 102.3, [65536, 3584] 122.8 / 116.5, [65536, 4096] 138.0 / 132.4, [65536, 4160] 151.4 / 134.5, [65536, 4608] 161.0 / 150.2,
+    // [65536, 5120] 171.6 / 175.7, [65536, 2560] 85.5 / 93.5; [16384, 4096] 28.7 / 28.6
+    if (C <= 256 * 8 * 2) launch(quant_i8_rows_kernel<256, 2, 256, true>, 256, 1);
+    else launch(quant_i8_rows_kernel<256, 3, 256, true>, 256, 1);
   } else if (C <= 256 * 8 * 2) {
     launch(quant_i8_rows_kernel<256, 2>, 256, 1);
   } else if (C <= 512 * 8 * 2) {

@@ -81,7 +81,8 @@ __device__ inline float amax8(const Pack8& v, bool f16) {
 // the trip to memory: lanes past the row's end read its last vector again (which changes no maximum), because loads under
 // conditions of their own went out one after another, each waiting for the one before. [64, 7168] 3.7 -> 2.8 us, [8, 2048]
 // 3.3 -> 2.3, [4096, 7168] 16.8 -> 15.1, [8192, 768] 8.7 -> 7.9 (behind a launch that writes the rows).
-template <int TPR, int NV, int THREADS = 256>
+// IN_TURN: each vector of a lane is waited for before the next is asked for.
+template <int TPR, int NV, int THREADS = 256, bool IN_TURN = false>
 __device__ __forceinline__ void quant_i8_rows_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
                                                    int8_t* __restrict__ q, int64_t ld_q, float* __restrict__ row_max,
                                                    int chunked, int first_row, bool f16 = false) {
@@ -94,7 +95,10 @@ __device__ __forceinline__ void quant_i8_rows_body(const uint16_t* __restrict__ 
   Pack8 val[NV];
   const uint4* src = reinterpret_cast<const uint4*>(x + static_cast<size_t>(live ? r : R - 1) * ld_x);
 #pragma unroll
-  for (int i = 0; i < NV; ++i) val[i].v = src[min(t + i * TPR, nvec - 1)];
+  for (int i = 0; i < NV; ++i) {
+    val[i].v = src[min(t + i * TPR, nvec - 1)];
+    if (IN_TURN && i + 1 < NV) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  }
   uint32_t mag = 0;
 #pragma unroll
   for (int i = 0; i < NV; ++i) mag = max_magnitudes(mag, magnitudes8(val[i]));
