@@ -53,43 +53,13 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
   const int m = blockIdx.y, col = blockIdx.x * 16;
   const bool f16 = FMT == Fmt::F16 || FMT == Fmt::W4H || ((FMT == Fmt::I8 || FMT == Fmt::F8) && p.f16 != 0);
   const bool tail = wave >= p.K;
-  // A wave takes a pair; int8, one token's waves take the sorted rows 0 ... K - 1 instead, which they may ask for before they know
-  // whose they are (k: the pair's place among the token's). Layer, us: DeepSeek-V3 dims 69.5 -> 67.5, Qwen3 dims 13.7 -> 13.5. (fp8 has no
-  // registers for it, 68.8 -> 72.6; 16-bit and 4-bit weights have nothing to do between a row and its product, 18.7 -> 18.8.)
-  const bool row_first = FMT == Fmt::I8 && p.M == 1;
+  // (One token's waves could take the sorted rows 0 ... K - 1 and ask for them before they know whose they are. Layer, int8, so /
+  // that way, us: Qwen3 dims 13.25 / 13.68, 64 experts of [3072 x 2560] 19.85 / 20.0, DeepSeek-V3 dims 67.5 / 67.1: the weights are asked for
+  // later then, behind vector loads and a ballot where these three are scalar loads.)
   const int pair = m * p.K + wave;
-  const int nvec = p.I / 8;
-  Pack8 val[kVecs];
-  // (layer, us, loads under conditions / together: Qwen3 dims int8 4 tokens 30.2 / 29.7, DeepSeek-V3 dims 1 token int8 66.8 / 66.5, fp8
-  // 71.7 / 70.6; 16-bit and 4-bit rows, more registers and fewer waves, lose: bf16 4 tokens 48.4 / 53.9, Kimi-K2 dims 47.5 / 51.4)
-  auto load_row = [&](int row) __attribute__((always_inline)) {
-    const uint4* src = reinterpret_cast<const uint4*>(p.act + static_cast<size_t>(row) * p.I);
-#pragma unroll
-    for (int i = 0; i < kVecs; ++i) {
-      if constexpr (QUANT) {  // lanes past the end read the last vector again: the loads go out together
-        val[i].v = src[min(lane + i * kWave, nvec - 1)];
-      } else {
-        val[i].v = make_uint4(0, 0, 0, 0);
-        if (lane + i * kWave < nvec) val[i].v = src[lane + i * kWave];
-      }
-    }
-  };
-  int k = wave, e, row;
-  float weight;
-  if (row_first) {
-    const int j = min(lane, p.K - 1);
-    const int id = p.ids[j], at = p.moe_index[j];
-    const float w = p.topk_w[j];
-    row = wave;  // (the shared expert's row follows those of the pairs)
-    load_row(row);
-    if (!tail) k = __builtin_ctzll(__ballot(at == wave));
-    e = tail ? 0 : __builtin_amdgcn_readlane(id, k);
-    weight = tail ? 0.0f : __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), k));
-  } else {
-    e = tail ? 0 : p.ids[pair];
-    row = tail ? p.M * p.K + m : p.moe_index[pair];
-    weight = tail ? 0.0f : p.topk_w[pair];
-  }
+  const int e = tail ? 0 : p.ids[pair];
+  const int row = tail ? p.M * p.K + m : p.moe_index[pair];
+  const float weight = tail ? 0.0f : p.topk_w[pair];
 
   // ---- weights: as many steps of the 16 channels as the ring holds ----
   const int ksteps = p.kbytes / (64 * V);
@@ -138,7 +108,20 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
 
   __builtin_amdgcn_sched_barrier(0);
   // ---- the row: quantised (the arithmetic of the quantisers' launches, hence their bits) or as it is, into LDS ----
-  if (!row_first) load_row(row);
+  // (layer, us, loads under conditions / together: Qwen3 dims 3 tokens int8 24.75 / 24.5, fp8 25.8 / 25.5, DeepSeek-V3 dims fp8 1 token
+  // 72.6 / 71.4; 16-bit and 4-bit rows, more registers and fewer waves, lose: bf16 4 tokens 48.4 / 53.9, Kimi-K2 dims 1 token 47.5 / 51.4)
+  const uint4* src = reinterpret_cast<const uint4*>(p.act + static_cast<size_t>(row) * p.I);
+  const int nvec = p.I / 8;
+  Pack8 val[kVecs];
+#pragma unroll
+  for (int i = 0; i < kVecs; ++i) {
+    if constexpr (QUANT) {  // lanes past the end read the last vector again: the loads go out together
+      val[i].v = src[min(lane + i * kWave, nvec - 1)];
+    } else {
+      val[i].v = make_uint4(0, 0, 0, 0);
+      if (lane + i * kWave < nvec) val[i].v = src[lane + i * kWave];
+    }
+  }
   int8_t* mine = rows_lds + wave * few_row_pitch(p.I, QUANT ? 1 : 2, FMT == Fmt::F8);
   [[maybe_unused]] float* scales = reinterpret_cast<float*>(mine + p.I);
   float amax = 1.0f;
@@ -246,11 +229,11 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
     for (int q = 0; q < 4; ++q) {
       if constexpr (FMT == Fmt::I8) y[q] = f32_to_act((static_cast<float>(total[q]) * amax) * wm[q], f16);
       else y[q] = f32_to_act(total[q], f16);
-      y_lds[k][lg * 4 + q] = act_to_f32(y[q], f16);
+      y_lds[wave][lg * 4 + q] = act_to_f32(y[q], f16);
     }
     *reinterpret_cast<uint2*>(p.down + static_cast<size_t>(row) * p.H + col + lg * 4) =
         make_uint2(y[0] | (static_cast<uint32_t>(y[1]) << 16), y[2] | (static_cast<uint32_t>(y[3]) << 16));
-    if (lane == 0) w_lds[k] = weight;
+    if (lane == 0) w_lds[wave] = weight;
   }
   __syncthreads();
 
@@ -298,8 +281,8 @@ int launch_few_down(const FewDown& p, hipStream_t s) {
 // part of the rows while its weights are on their way (int8: one exchange of the maxima), and the codes wait in LDS.
 // One token alone is routed by wave 0, and the others bring its row to LDS meanwhile - quantised, but for int8, whose scale
 // is known only when all three have their part: each wave then rounds its part of K from there. Layer, us, the row asked for
-// behind the weights / so, weights of the experts' routing left to the last column in both: Qwen3 dims int8 14.6 / 13.8, bf16 18.7 /
-// 18.4; with them, before: int8 14.8, bf16 18.8, DeepSeek-V3 dims int8 70.4 -> 69.6, Kimi-K2 dims 4-bit 48.7 -> 47.6.
+// behind the weights / so: Qwen3 dims int8 14.75 / 13.7, fp8 15.1 / 14.7, bf16 19.0 / 18.8, 4-bit 13.7 / 13.5; DeepSeek-V3 dims int8 68.0 / 66.9,
+// fp8 71.0 / 72.1; Kimi-K2 dims 4-bit 49.5 / 48.5.
 // (The same for up to four tokens, every wave its part of all rows before the routing: 4 tokens 30.2 -> 33.3, a row then is
 // looked at by every column and not by those that serve it.)
 template <Fmt FMT, int SLOTS, bool SIGMOID>

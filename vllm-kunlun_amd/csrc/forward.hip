@@ -236,8 +236,9 @@ bool few_down_pays(const kmoe_moe_args* a, bool fold) {
 
 // Whether such a layer also begins in one launch (few_gate_up): up to kFewRouted tokens, so that routing is a wave each,
 // whose rows leave room for five workgroups in a CU's LDS - fewer, and the launch no longer fills the chip at once (Kimi-K2
-// dims, 4-bit, 1 token 57.1 -> 52.6 us, 2 tokens, three workgroups, 92.7 -> 98.9). Layer, us, apart / in one launch: Qwen3 dims int8 1 token 18.9 / 13.8, 4 36.3 / 29.4, bf16 1 22.0 / 18.4, 4-bit 1 18.4 / 14.9, 4 27.2 / 24.7; DeepSeek-V3 dims int8 1 87.7 /
-// 69.6, with the gate 96.6 / 78.4, fp8 1 88.7 / 68.8.
+// dims, 4-bit, 1 token 57.1 -> 52.6 us, 2 tokens, three workgroups, 92.7 -> 98.9). Layer, us, apart / in one launch: Qwen3 dims int8 1
+// token 16.8 / 13.3, 2 21.2 / 19.9, 4 32.6 / 29.6, bf16 1 20.3 / 18.8, 4 50.2 / 47.8, 4-bit 1 17.7 / 13.4, 4 26.0 / 24.7; DeepSeek-V3 dims int8 1 76.3 /
+// 67.2, 2 135.2 / 130.2, 3 174.3 / 177.8, with the gate 1 86.4 / 75.6, fp8 1 80.1 / 71.5, 3 172.5 / 174.1; Kimi-K2 dims 4-bit 1 52.6 / 48.5.
 bool few_gate_up_takes(const kmoe_moe_args* a) {
   if (a->M > kFewRouted || a->M * a->K > kWave || a->E > 8 * kWave || a->H > kFewRowBytes) return false;
   if (a->M * few_row_pitch(a->H, bf16_activations(a->format) ? 2 : 1, a->format == KMOE_FMT_FP8_BLOCK) > kFewRowBytes) return false;
