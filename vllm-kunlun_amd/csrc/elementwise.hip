@@ -245,7 +245,7 @@ int quant_i8_launch(const uint16_t* x, int64_t ld_x, int R, int C, int8_t* q, in
       hipLaunchKernelGGL(kernel, dim3(ceil_div(static_cast<int>(std::min<int64_t>(kMost, R - from)), rows_per_group)), dim3(threads), 0, s, x,
                          ld_x, R, C, q, ld_q, row_max, chunked, f16, static_cast<int>(from));
   };
-  // (figures: us behind a launch that writes the rows)
+  // (figures: us behind a launch that writes the rows; of short rows and rows beyond the memory-side cache, in a row of calls)
   if (C <= 16 * 8) {
     // four rows a wave: many short rows are bound by the starts of waves ([65536, 128] 6.7 us, two rows a wave 10.4, a branch per load 9.3)
     launch(quant_i8_rows_kernel<16, 1>, 256, 16);
