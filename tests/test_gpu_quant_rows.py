@@ -113,6 +113,27 @@ def test_rows_beyond_the_memory_side_cache(R, C):
     assert torch.equal(q, dw.repeat(-(-R // few), 1)[:R]) and torch.equal(top.view(torch.int32), dm.repeat(-(-R // few))[:R])
 
 
+def test_the_most_rows_there_can_be():
+    """Rows up to the last that 31 bits count: the last workgroup's rows past them are none."""
+    from vllm_kunlun_amd import _lib as L
+    R, C, end = 2 ** 31 - 2, 8, 40
+    if torch.cuda.mem_get_info()[0] < 80 << 30:
+        pytest.skip("60 GB of rows")
+    x = torch.zeros(R, C, dtype=torch.bfloat16, device="cuda")
+    tail = _rows(end, C, torch.bfloat16)
+    x[-end:] = tail.cuda()
+    q = torch.empty(R * C + 64, dtype=torch.int8, device="cuda")
+    q[R * C - end * C:] = 99
+    top = torch.full((R + 16,), -7.0, device="cuda")
+    L.check(L.lib.kmoe_quant_i8_rows_dt(L.ptr(x), C, R, C, L.ptr(q), C, L.ptr(top), 0, L.stream()))
+    want, want_max = co.quant_i8_rows(bits(tail))
+    assert np.array_equal(q[(R - end) * C:R * C].view(end, C).cpu().numpy(), want) and bool((q[R * C:] == 99).all())
+    assert np.array_equal(top[R - end:R].cpu().numpy().view(np.uint32), want_max.view(np.uint32)) and bool((top[R:] == -7).all())
+    assert not bool(q[:(R - end) * C].view(torch.int64).any()) and not bool(top[:R - end].any())
+    del x, q, top
+    torch.cuda.empty_cache()
+
+
 # rows that the down projection's launch quantises itself (32 tokens: up to four rows a wave), their last vectors in one load
 # of a lane and in two: rows of zeros, NaNs, infinities and the smallest numbers among ordinary ones
 @pytest.mark.parametrize("I", [64, 576, 1024])

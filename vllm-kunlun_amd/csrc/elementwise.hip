@@ -8,7 +8,7 @@ namespace {
 template <int TPR, int NV, int THREADS = 256, bool IN_TURN = false>
 __global__ __launch_bounds__(THREADS) void quant_i8_rows_kernel(const uint16_t* __restrict__ x, int64_t ld_x, int R,
                                                                int C, int8_t* __restrict__ q, int64_t ld_q,
-                                                               float* __restrict__ row_max, int chunked, int f16, int from) {
+                                                               float* __restrict__ row_max, int chunked, int f16, uint32_t from) {
   quant_i8_rows_body<TPR, NV, THREADS, IN_TURN>(x, ld_x, R, C, q, ld_q, row_max, chunked, from + blockIdx.x * (THREADS / TPR), f16 != 0);
 }
 
@@ -243,7 +243,7 @@ int quant_i8_launch(const uint16_t* x, int64_t ld_x, int R, int C, int8_t* q, in
     constexpr int kMost = 1 << 21;  // rows of a launch, whose threads are counted in 32 bits
     for (int64_t from = 0; from < R; from += kMost)
       hipLaunchKernelGGL(kernel, dim3(ceil_div(static_cast<int>(std::min<int64_t>(kMost, R - from)), rows_per_group)), dim3(threads), 0, s, x,
-                         ld_x, R, C, q, ld_q, row_max, chunked, f16, static_cast<int>(from));
+                         ld_x, R, C, q, ld_q, row_max, chunked, f16, static_cast<uint32_t>(from));
   };
   // (figures: us behind a launch that writes the rows; of short rows and rows beyond the memory-side cache, in a row of calls)
   if (C <= 16 * 8) {

@@ -85,15 +85,15 @@ __device__ inline float amax8(const Pack8& v, bool f16) {
 template <int TPR, int NV, int THREADS = 256, bool IN_TURN = false>
 __device__ __forceinline__ void quant_i8_rows_body(const uint16_t* __restrict__ x, int64_t ld_x, int R, int C,
                                                    int8_t* __restrict__ q, int64_t ld_q, float* __restrict__ row_max,
-                                                   int chunked, int first_row, bool f16 = false) {
+                                                   int chunked, uint32_t first_row, bool f16 = false) {
   static_assert(TPR <= kWave || TPR == THREADS, "rows of several waves have a workgroup each");
   __shared__ uint32_t red[THREADS / kWave];
   const int t = threadIdx.x % TPR;
-  const int r = first_row + threadIdx.x / TPR;
-  const bool live = r < R;
+  const uint32_t r = first_row + threadIdx.x / TPR;  // (a workgroup's last rows may lie beyond 2^31)
+  const bool live = r < static_cast<uint32_t>(R);
   const int nvec = C / 8;
   Pack8 val[NV];
-  const uint4* src = reinterpret_cast<const uint4*>(x + static_cast<size_t>(live ? r : R - 1) * ld_x);
+  const uint4* src = reinterpret_cast<const uint4*>(x + static_cast<size_t>(live ? r : static_cast<uint32_t>(R) - 1) * ld_x);
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     val[i].v = src[min(t + i * TPR, nvec - 1)];
