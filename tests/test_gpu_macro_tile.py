@@ -1,0 +1,84 @@
+"""The tiles with both operands in LDS (variant 23) against the 128-row tiles (variant 6), which add the same products in the same
+order: the same bits, at the edges of row fragments and tiles, of the channels, for every form of the operands' rows."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 15, 16, 17, 0, 191, 192, 193, 33, 384, 385, 0, 127, 128, 129, 800, 3100]  # up to 17 tiles of an expert
+
+
+def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, bound=0, seed=0):
+    """Outputs of the variants 6 and 23 for the same operands. pad: values between the rows of a and y; tail: rows of an expert
+    outside w (int8); bound: rows the caller allows for beyond the last expert's."""
+    from vllm_kunlun_amd import _lib as L
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    E, rows, n_out = len(counts), sum(counts), n // 2 if act else n
+    a_rows = (-(-rows // div) if gather else rows) + tail
+    src = torch.randperm(rows, generator=g, device="cuda").int()
+    lod = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    i8 = kind == "int8"
+    a = (torch.randint(-127, 128, (a_rows, k + pad), generator=g, device="cuda", dtype=torch.int8) if i8
+         else torch.randn(a_rows, k + pad, generator=g, device="cuda").to(dtype))
+    w = (torch.randint(-127, 128, (E + 1, n, k), generator=g, device="cuda", dtype=torch.int8) if i8
+         else torch.randn(E + 1, n, k, generator=g, device="cuda").mul_(0.05).to(dtype))
+    tiled = torch.empty_like(w)
+    L.check(L.lib.kmoe_tile_weights_i8(w.data_ptr(), tiled.data_ptr(), E + 1, n, k * w.element_size(), L.stream()))
+    a_max, w_max = (torch.rand(s, generator=g, device="cuda") * 0.1 + 0.01 for s in ((a_rows,), (E + 1, n)))
+    q = L.GemmI8Args() if i8 else L.GemmBf16Args()
+    if i8:
+        q.a_max, q.w_max = a_max.data_ptr(), w_max.data_ptr()
+        if tail:
+            q.w_tail, q.w_max_tail = tiled[E].data_ptr(), w_max[E].data_ptr()
+            q.tail_row0, q.tail_rows, q.tail_src0 = rows, tail, a_rows - tail
+    q.a, q.lda, q.w, q.w_layout, q.lod = a.data_ptr(), k + pad, tiled.data_ptr(), L.KMOE_W_TILED, lod.data_ptr()
+    q.row_src, q.src_div = (src.data_ptr(), div) if gather else (0, 1)
+    q.E, q.n, q.k, q.rows, q.act, q.ldy = E, n, k, rows + bound, act, n_out + pad
+    out = []
+    for variant in (6, 23):
+        y = torch.full((rows + tail, n_out + pad), float("nan"), dtype=dtype, device="cuda")
+        q.y, q.variant, q.act_dtype = y.data_ptr(), variant, L.act_dtype(y, "test")
+        L.check((L.lib.kmoe_grouped_gemm_i8 if i8 else L.lib.kmoe_grouped_gemm_bf16)(q, L.stream()))
+        out.append(y)
+    torch.cuda.synchronize()
+    return out, n_out
+
+
+def _same(out, n_out):
+    assert not out[1][:, :n_out].isnan().any() and torch.equal(out[0][:, :n_out], out[1][:, :n_out])
+    assert out[1][:, n_out:].isnan().all()  # nothing between the rows is written
+
+
+@pytest.mark.parametrize("kind", ["int8", "16 bit"])
+@pytest.mark.parametrize("n,k", [(64, 768), (320, 896), (256, 1024), (544, 2048)])  # bytes of K: 12, 14, 16, 32 steps
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tiles(kind, n, k, act, dtype):
+    _same(*_launch(kind, ROWS, n, k if kind == "int8" else k // 2, act, dtype, div=8))
+
+
+@pytest.mark.parametrize("kind", ["int8", "16 bit"])
+@pytest.mark.parametrize("form", [dict(gather=False), dict(div=1), dict(div=3), dict(div=6), dict(pad=64), dict(bound=500)], ids=str)
+@pytest.mark.parametrize("act", [0, 1])
+def test_forms(kind, form, act):
+    _same(*_launch(kind, ROWS, 288, 768, act, torch.bfloat16, **form))
+
+
+@pytest.mark.parametrize("tail", [1, 192, 700])
+@pytest.mark.parametrize("act", [0, 1])
+def test_tail_expert(tail, act):
+    _same(*_launch("int8", ROWS, 288, 768, act, torch.bfloat16, div=8, tail=tail))
+
+
+def test_more_items_than_are_resolved_at_once():
+    """Over 32 items per workgroup, and weights beyond the memory-side cache: those of experts with one tile are read past it."""
+    _same(*_launch("int8", [1, 192, 193, 0, 40] * 28, 16384, 768, 0, torch.bfloat16))
+
+
+@pytest.mark.parametrize("k,div,experts", [(640, 1, 3), (832, 1, 3), (768, 5, 3), (768, 1, 500)])
+def test_what_the_launch_does_not_take(k, div, experts):
+    """Too short a K, no whole chunks, a divisor whose quotients one multiplication does not give, too many experts for its LDS:
+    refused when asked for by name, and served by another kernel otherwise."""
+    from vllm_kunlun_amd import _lib as L
+    with pytest.raises(NotImplementedError):
+        _launch("int8", [5] * experts, 32, k, 0, torch.bfloat16, div=div)

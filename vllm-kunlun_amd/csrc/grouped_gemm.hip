@@ -490,7 +490,7 @@ int grouped_gemm_i8_checked(const kmoe_gemm_i8_args* a, kmoe_stream_t stream, co
   if (a->rows == 0 && !(a->w_tail && a->tail_rows > 0)) return KMOE_OK;
   // Tiled weights and more than a few rows per expert: the persistent tile kernel (variants 5-9, 11-16 force it)
   if (a->w_layout == KMOE_W_TILED && a->k >= 128 &&
-      ((a->variant >= 5 && a->variant <= 9) || (a->variant >= 11 && a->variant <= 22) ||
+      ((a->variant >= 5 && a->variant <= 9) || (a->variant >= 11 && a->variant <= 23) ||
        (a->variant == 0 && ceil_div(expected_rows(a->rows, a->rows_hint), a->E) > kTiledMinRows)))
     return tiled_gemm_i8(a, as_stream(stream));
   KMOE_REQUIRE(a->variant < 5, KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8: variants 5-12 need tiled weights and k >= 128");
@@ -538,7 +538,7 @@ int grouped_gemm_bf16_checked(const kmoe_gemm_bf16_args* a, kmoe_stream_t stream
     return stream_gemm_bf16(a, as_stream(stream), scan, slots);
   KMOE_REQUIRE(!scan && !slots, KMOE_ERR_UNSUPPORTED, "grouped_gemm_bf16: only the weight-streaming kernel sorts the pairs itself");
   // tiled weights and more rows: the persistent tile kernel (variants 5, 6, 11-13, 18 force it)
-  const bool forced = tile_variant(a->variant) || a->variant == 18;
+  const bool forced = tile_variant(a->variant) || a->variant == 18 || a->variant == 23;
   if (a->w_layout == KMOE_W_TILED && a->k >= 64 && a->ldy % 8 == 0 &&
       (forced || (a->variant == 0 && ceil_div(live, a->E) > kTiledMinRows)))
     return tiled_gemm_bf16(a, as_stream(stream));

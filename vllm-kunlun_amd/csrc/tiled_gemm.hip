@@ -38,6 +38,7 @@
 
 #include "buffer_ops.h"
 #include "kmoe_common.h"
+#include "macro_tile.h"
 
 namespace kmoe {
 namespace {
@@ -1477,6 +1478,48 @@ int tiled_common(const TiledParams& p, int rows, int* n_cu_out, const char* what
   return KMOE_OK;
 }
 
+// The launch as macro_tile.hip takes it; false where it does not.
+bool macro_params(const TiledParams& p, int live, MacroParams* out) {
+  uint32_t magic = 0;
+  if (p.row_src && p.src_div > 1) {  // entry / src_div = high half of entry * magic, for every entry where the excess is at most 2
+    magic = static_cast<uint32_t>(((1ull << 32) + p.src_div - 1) / p.src_div);
+    if (static_cast<uint64_t>(magic) * p.src_div - (1ull << 32) > 2) return false;
+  }
+  if (!macro_tile_takes(p.k, p.E, p.w_tail != nullptr) || p.acc_out || p.bias) return false;
+  const bool past = p.E > 1 && static_cast<long long>(p.E) * p.n * p.k > (256ll << 20);
+  const float mean = static_cast<float>(ceil_div(live, p.E));
+  *out = MacroParams{p.a, p.lda, p.a_max, p.row_src, magic, p.w, p.w_max, p.lod, p.E, p.n, p.k, p.y, p.ldy,
+                     p.w_tail, p.w_max_tail, p.tail_row0, p.tail_rows, p.tail_src0, 0, p.m_major,
+                     past && mean + 2.2f * sqrtf(mean) <= 192.0f, past};
+  return true;
+}
+
+// Where that launch is ahead of the tiles of this file. GEMM alone, us, those / that one, even load; +2.0 on the logits of 8 experts:
+//   int8, Qwen3 dims, gate_up, 49 rows per expert 70 / 72; 74 / 80, 75 83 / 76; 93 / 88, 156 106 / 92; 126 / 112, 256 152 / 136; 160 / 144, 512 243 / 219;
+//   264 / 239; down, 12 rows 37.0 / 36.5; 40.2 / 37.6, 49 46 / 41; 51.5 / 45, 188 92 / 69; 91 / 73, 512 187 / 135; 198 / 142
+//   int8, DeepSeek-V3 dims, gate_up, 12 rows 1136 / 1083; 1143 / 1111, 47 1285 / 1151; 1372 / 1220, 128 1424 / 1310; 1720 / 1582; down, 12 rows 619 /
+//   602; 623 / 602, 94 727 / 733; 845 / 809, 128 780 / 750; 902 / 882; Kimi-K2 dims, 85 rows 2021 / 1848; 2285 / 2051 and 1070 / 1087; 1217 / 1187
+//   int8, 32 experts of [2048 x 4096], gate_up, 150 rows 52 / 50; 70 / 75, of [4096 x 1024] 75 rows 30.7 / 32.4; 37 / 36; 16 of [4096 x 4096], 375 to
+//   1024 rows 0.97 to 1.05 times as fast; 8 of [4096 x 14336], 150 rows 153 / 107; 170 / 111 (their 192-row tiles are too few for the CUs)
+//   bf16, Qwen3 dims, gate_up, 49 rows 135 / 127; 139 / 147, 125 160 / 145; 186 / 171, 188 191 / 207; 215 / 210, 512 405 / 416; 395 / 426; down, 19 rows
+//   75.6 / 69.1; 80 / 73, 100 104 / 85; 112 / 96, 256 152 / 148; 164 / 152, 512 256 / 242; 259 / 255; 160 experts of [3072 x 2560], gate_up, 15 rows
+//   427 / 391; 438 / 384; 32 of [4096 x 1024], 75 rows 47 / 50; 51 / 58
+// So: wherever every CU gets four items of 192 rows; from two on where rows are many or, without SiLU-mul, 16-bit weights exceed the
+// memory-side cache. 16-bit gate_up launches are bound by their weights: only while one tile holds nearly every expert.
+bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_cu) {
+  const float mean = static_cast<float>(ceil_div(live, p.E));
+  const long long weights = static_cast<long long>(p.E) * p.n * p.k;
+  const long long items = static_cast<long long>(p.E) * ceil_div(static_cast<int>(mean), 192) * ceil_div(p.n, 256);
+  const bool many = items >= 4ll * n_cu, some = items >= 2ll * n_cu;
+  if (kind == TKind::BF16) {
+    if (!swiglu) return many || (some && weights > (256ll << 20));
+    return (many && mean + 2.2f * sqrtf(mean) <= 192.0f) || (some && mean > 80.0f && mean <= 150.0f);
+  }
+  if (many) return true;
+  if (swiglu) return some && mean > 72.0f;
+  return (some && mean > 88.0f && (p.k < 4096 || weights > (1ll << 30))) || (items < n_cu && mean > 128.0f);
+}
+
 // One 8-wave tile of 16 MF rows per workgroup with the eight waves side by side along the channels (32 channels
 // each, all rows): no two waves ask for the same weight bytes, and seven MFMA steps of them are on their way per
 // wave (8-slot ring of two fragments) - 112 KB of distinct weight bytes in flight per CU against 48 KB with two
@@ -1511,7 +1554,7 @@ int launch_tall(TiledParams& p, int rows, hipStream_t s, int n_cu, const char* w
 // Variant 6 (and 12) forces 128 rows, 11 forces 64, 13 forces 96.
 bool short_tiles(int variant, int rows, int n_experts, int n, bool swiglu, int n_cu, int max_avg_rows = 44) {
   if (variant == 11) return true;
-  if (variant == 6 || variant == 8 || (variant >= 12 && variant <= 22)) return false;
+  if (variant == 6 || variant == 8 || (variant >= 12 && variant <= 23)) return false;
   if (ceil_div(rows, n_experts) <= max_avg_rows) return true;
   const int n_blocks = ceil_div(swiglu ? n / 2 : n, kWavesT * (swiglu ? 2 : 4) * 16);
   return static_cast<long long>(rows / 128 + n_experts) * n_blocks < 2ll * n_cu;
@@ -1615,9 +1658,17 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
       return f16 ? launch_tiled<K, false, 2, 4, 3, 1, false, 4, false, false, true>(p, a->rows, s, n_cu, what)
                  : launch_tiled<K, false, 2, 4, 3, 1, false, 4>(p, a->rows, s, n_cu, what);
   }
+  MacroParams macro;
+  if (a->variant == 23) {
+    KMOE_REQUIRE(macro_params(p, live, &macro), KMOE_ERR_UNSUPPORTED, "%s: variant 23 needs k %% 128 == 0, k >= 768, at most some 410 experts, no acc_out and src_div 1 to 4, 6, 8 or another power of two", what);
+    return macro_tile(macro, 0, swiglu, a->act_dtype == KMOE_DT_F16, a->rows, s, n_cu, what);
+  }
   const float avg_routed = static_cast<float>(ceil_div(live, a->E));
   const float reach = avg_routed + 3.0f * sqrtf(avg_routed);
   const bool big = weight_bytes > (1ll << 30);
+  if (a->variant == 0 && macro_pays(K, p, live, swiglu, n_cu) && macro_params(p, live, &macro)) {
+    return macro_tile(macro, 0, swiglu, a->act_dtype == KMOE_DT_F16, a->rows, s, n_cu, what);
+  }
   int wide = 0;  // row fragments of the wide tile (8: 128 rows, 12: 192, 16: 256), 0: none
   bool pair = false;
   switch (a->variant) {
@@ -1795,6 +1846,15 @@ int tiled_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s) {
   const float avg = static_cast<float>(ceil_div(live, a->E));
   const float reach = avg + 3.0f * sqrtf(avg);
   const bool half = a->act_dtype == KMOE_DT_F16;  // half operands and results (no bias, no interleaved activation: checked by the caller)
+  if (a->variant == 23) {
+    MacroParams macro;
+    KMOE_REQUIRE(macro_params(p, live, &macro), KMOE_ERR_UNSUPPORTED, "%s: variant 23 needs k %% 64 == 0, k >= 384, at most some 410 experts, no bias and src_div 1 to 4, 6, 8 or another power of two", what);
+    return macro_tile(macro, 1, swiglu, half, a->rows, s, n_cu, what);
+  }
+  if (a->variant == 0 && macro_pays(K, p, live, swiglu, n_cu)) {
+    MacroParams macro;
+    if (macro_params(p, live, &macro)) return macro_tile(macro, 1, swiglu, half, a->rows, s, n_cu, what);
+  }
   if (shorter) return launch_short<K>(p, a->rows, s, n_cu, what, swiglu, half);
   if (a->variant == 13 || (a->variant == 0 && reach <= 96.0f)) {
     if (half)
