@@ -397,7 +397,8 @@ typedef struct kmoe_gemm_fp8_args {
   int64_t ldy;
   int32_t act;
   int32_t variant;        /* 0 = choose from the shape. Tuning and tests: 1-3 LDS-staged kernels; with tiled weights 5 =
-                             tile kernel (6, 11, 13, 12: as for int8), 19, 20, 18: wide tiles of 128, 160, 192 rows.
+                             tile kernel (6, 11, 13, 12: as for int8), 19, 20, 18: wide tiles of 128, 160, 192 rows,
+                             23: as for int8 (n % 256 == 0 with SiLU-mul).
                              Those copy a row's scales four at a time: with k < 512, which has fewer, 18-20 run the
                              four-wave tiles of 128 rows, and 18 without SiLU-mul and with more than 896
                              experts, whose row ranges do not fit its LDS, the 160-row wide tile (same bits) */

@@ -1,10 +1,12 @@
-"""The tiles with both operands in LDS (variant 23) against the 128-row tiles (variant 6), which add the same products in the same
-order: the same bits, at the edges of row fragments and tiles, of the channels, for every form of the operands' rows."""
+"""The tiles with both operands in LDS (variant 23) against the 128-row tiles (variant 6; fp8: the 128-row wide tiles, 19), which add
+the same products in the same order: the same bits, at the edges of row fragments and tiles, of the channels, for every form of the
+operands' rows."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
+FEW = [0, 1, 2, 0, 3] * 12  # with these an expert holds few rows on average: the lower tiles of fp8
 ROWS = [1, 15, 16, 17, 0, 191, 192, 193, 33, 384, 385, 0, 127, 128, 129, 800, 3100]  # up to 17 tiles of an expert
 
 
@@ -17,28 +19,36 @@ def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, b
     a_rows = (-(-rows // div) if gather else rows) + tail
     src = torch.randperm(rows, generator=g, device="cuda").int()
     lod = torch.tensor([0] + counts).cumsum(0).int().cuda()
-    i8 = kind == "int8"
-    a = (torch.randint(-127, 128, (a_rows, k + pad), generator=g, device="cuda", dtype=torch.int8) if i8
-         else torch.randn(a_rows, k + pad, generator=g, device="cuda").to(dtype))
-    w = (torch.randint(-127, 128, (E + 1, n, k), generator=g, device="cuda", dtype=torch.int8) if i8
-         else torch.randn(E + 1, n, k, generator=g, device="cuda").mul_(0.05).to(dtype))
+    i8, f8 = kind == "int8", kind == "fp8"
+    if f8:
+        a, w = (torch.randn(shape, generator=g, device="cuda").mul_(60).to(torch.float8_e4m3fn) for shape in ((a_rows, k + pad), (E + 1, n, k)))
+        a_max, w_max = (torch.rand(shape, generator=g, device="cuda") * 0.01 + 0.001 for shape in ((a_rows, k // 128), (E + 1, n // 128, k // 128)))
+    else:
+        a_max, w_max = (torch.rand(shape, generator=g, device="cuda") * 0.1 + 0.01 for shape in ((a_rows,), (E + 1, n)))
+    if not f8:
+        a = (torch.randint(-127, 128, (a_rows, k + pad), generator=g, device="cuda", dtype=torch.int8) if i8
+             else torch.randn(a_rows, k + pad, generator=g, device="cuda").to(dtype))
+        w = (torch.randint(-127, 128, (E + 1, n, k), generator=g, device="cuda", dtype=torch.int8) if i8
+             else torch.randn(E + 1, n, k, generator=g, device="cuda").mul_(0.05).to(dtype))
     tiled = torch.empty_like(w)
     L.check(L.lib.kmoe_tile_weights_i8(w.data_ptr(), tiled.data_ptr(), E + 1, n, k * w.element_size(), L.stream()))
-    a_max, w_max = (torch.rand(s, generator=g, device="cuda") * 0.1 + 0.01 for s in ((a_rows,), (E + 1, n)))
-    q = L.GemmI8Args() if i8 else L.GemmBf16Args()
-    if i8:
-        q.a_max, q.w_max = a_max.data_ptr(), w_max.data_ptr()
+    q = L.GemmI8Args() if i8 else (L.GemmFp8Args() if f8 else L.GemmBf16Args())
+    if i8 or f8:
+        for name, scales in (("a_max", a_max), ("w_max", w_max)) if i8 else (("a_scale", a_max), ("w_scale", w_max)):
+            setattr(q, name, scales.data_ptr())
         if tail:
-            q.w_tail, q.w_max_tail = tiled[E].data_ptr(), w_max[E].data_ptr()
+            q.w_tail = tiled[E].data_ptr()
+            setattr(q, "w_max_tail" if i8 else "w_scale_tail", w_max[E].data_ptr())
             q.tail_row0, q.tail_rows, q.tail_src0 = rows, tail, a_rows - tail
     q.a, q.lda, q.w, q.w_layout, q.lod = a.data_ptr(), k + pad, tiled.data_ptr(), L.KMOE_W_TILED, lod.data_ptr()
     q.row_src, q.src_div = (src.data_ptr(), div) if gather else (0, 1)
     q.E, q.n, q.k, q.rows, q.act, q.ldy = E, n, k, rows + bound, act, n_out + pad
     out = []
-    for variant in (6, 23):
+    for variant in (19 if f8 else 6, 23):
         y = torch.full((rows + tail, n_out + pad), float("nan"), dtype=dtype, device="cuda")
         q.y, q.variant, q.act_dtype = y.data_ptr(), variant, L.act_dtype(y, "test")
-        L.check((L.lib.kmoe_grouped_gemm_i8 if i8 else L.lib.kmoe_grouped_gemm_bf16)(q, L.stream()))
+        launch = L.lib.kmoe_grouped_gemm_i8 if i8 else (L.lib.kmoe_grouped_gemm_fp8_block if f8 else L.lib.kmoe_grouped_gemm_bf16)
+        L.check(launch(q, L.stream()))
         out.append(y)
     torch.cuda.synchronize()
     return out, n_out
@@ -57,17 +67,30 @@ def test_tiles(kind, n, k, act, dtype):
     _same(*_launch(kind, ROWS, n, k if kind == "int8" else k // 2, act, dtype, div=8))
 
 
-@pytest.mark.parametrize("kind", ["int8", "16 bit"])
+@pytest.mark.parametrize("n,k", [(256, 768), (768, 896), (512, 1024), (512, 1152), (256, 2048)])  # 6 to 9 and 16 blocks of K
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("few", [False, True])
+def test_tiles_fp8(n, k, act, dtype, few):
+    _same(*_launch("fp8", [r for r in ROWS if r < 800] + FEW if few else ROWS, n, k, act, dtype, div=8))
+
+
+def test_channels_that_end_inside_a_tile_fp8():
+    _same(*_launch("fp8", ROWS, 384, 896, 0, torch.bfloat16))
+
+
+@pytest.mark.parametrize("kind", ["int8", "16 bit", "fp8"])
 @pytest.mark.parametrize("form", [dict(gather=False), dict(div=1), dict(div=3), dict(div=6), dict(pad=64), dict(bound=500)], ids=str)
 @pytest.mark.parametrize("act", [0, 1])
 def test_forms(kind, form, act):
-    _same(*_launch(kind, ROWS, 288, 768, act, torch.bfloat16, **form))
+    _same(*_launch(kind, ROWS, 512 if kind == "fp8" else 288, 768, act, torch.bfloat16, **form))
 
 
+@pytest.mark.parametrize("kind", ["int8", "fp8"])
 @pytest.mark.parametrize("tail", [1, 192, 700])
 @pytest.mark.parametrize("act", [0, 1])
-def test_tail_expert(tail, act):
-    _same(*_launch("int8", ROWS, 288, 768, act, torch.bfloat16, div=8, tail=tail))
+def test_tail_expert(kind, tail, act):
+    _same(*_launch(kind, ROWS, 512 if kind == "fp8" else 288, 768, act, torch.bfloat16, div=8, tail=tail))
 
 
 def test_more_items_than_are_resolved_at_once():

@@ -587,7 +587,7 @@ int grouped_gemm_fp8_checked(const kmoe_gemm_fp8_args* a, kmoe_stream_t stream, 
     return stream_gemm_fp8(a, as_stream(stream), scan, slots);
   KMOE_REQUIRE(!scan && !slots, KMOE_ERR_UNSUPPORTED, "grouped_gemm_fp8_block: only the weight-streaming kernel sorts the pairs itself");
   // tiled weights and more rows: the persistent tile kernel (variants 5, 6, 11 force it)
-  const bool tall_variant = a->variant == 8 || a->variant == 14 || (a->variant >= 17 && a->variant <= 20);  // 8-wave tiles of 256 / 192 rows; 17: chosen on the device; 18, 20, 19: wide 192- / 160- / 128-row tiles
+  const bool tall_variant = a->variant == 8 || a->variant == 14 || (a->variant >= 17 && a->variant <= 20) || a->variant == 23;  // 8-wave tiles of 256 / 192 rows; 17: chosen on the device; 18, 20, 19: wide 192- / 160- / 128-row tiles
   if (a->w_layout == KMOE_W_TILED && a->k <= 8192 && a->ldy % 8 == 0 &&
       (tile_variant(a->variant) || tall_variant || (a->variant == 0 && ceil_div(live, a->E) > kTiledMinRows)))
     return tiled_gemm_fp8(a, as_stream(stream));

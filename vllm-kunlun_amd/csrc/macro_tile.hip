@@ -1,5 +1,5 @@
 // Grouped GEMM on tiles of up to 192 rows x 256 weight rows with BOTH operands staged in LDS; tiled weights, int8
-// (v_mfma_i32_16x16x64_i8) and 16-bit operands (v_mfma_f32_16x16x32_bf16 / _f16).
+// (v_mfma_i32_16x16x64_i8), 16-bit operands (v_mfma_f32_16x16x32_bf16 / _f16) and block-scaled fp8 (v_mfma_scale_f32_16x16x128_f8f6f4).
 //
 // One workgroup per CU, persistent: eight waves, two along the rows (every other fragment of 16 rows each) and four along the
 // channels (64 each), 6 x 4 accumulator fragments a wave. Activations and weights come global -> LDS by asynchronous copies, once
@@ -22,6 +22,9 @@
 // chunk of steps s + 5 and s + 6, then the weights of step s + 5; at an even one the weights alone. At the top of step s everything
 // older than what left after the weights of step s + 1 (at step s - 4) has landed; the barrier behind the wait publishes it, and says
 // that every wave holds its fragments of step s, whose buffers the copies issued behind it may overwrite.
+// fp8 runs chunk by chunk (see chunk_f8): registers for one set of fragments beside the partial sums, six weight buffers, and two
+// chunk buffers - or, where 128 rows hold nearly every expert, three and tiles of 128 rows (DeepSeek-V3 dims, gate_up, 94 rows 1338 ->
+// 1286 us). Its copies leave together behind the chunk's first LDS requests (one after each MFMA group: 1354, these 1276).
 // All LDS accesses of the pipeline are assembly statements: one that the compiler sees would wait for every copy in flight.
 #include <utility>
 
@@ -33,13 +36,13 @@ namespace kmoe {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kMWaves = 8, kMThreads = kMWaves * kWave;
 constexpr int kMWaveCols = 4;              // waves along the channels
 constexpr int kMFrags = 4;                 // channel fragments of a wave
 constexpr int kMWeightStep = 16 * 1024;    // bytes of weights per step: 16 fragments of 16 channels x 64 bytes of K
-constexpr int kMWeightSlots = 5, kMChunkBufs = 3;  // (the copies and waits below are written for these)
 constexpr int kMChunk = 128;               // bytes of K per activation row and chunk
 
 template <class F, int... I>
@@ -51,7 +54,7 @@ __device__ __forceinline__ void m_for(F&& f) {
   m_for_each(f, std::make_integer_sequence<int, N>{});
 }
 
-enum class MOp { I8, BF16, F16 };
+enum class MOp { I8, BF16, F16, F8 };
 
 // The four MFMAs of row fragment I, left out if the tile has no rows there (a branch the compiler does not see: the K loop
 // stays one basic block). FIRST: the sums begin here.
@@ -99,6 +102,11 @@ __device__ __forceinline__ void m_request_f32(float& v, uint32_t addr) {
 }
 __device__ __forceinline__ void m_landed(v4i (&w)[4]) {
   asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3])::"memory");
+}
+// at most N younger LDS operations in flight: these have landed
+template <int N>
+__device__ __forceinline__ void m_wait8(v4i& lo, v4i& hi) {
+  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(lo), "+v"(hi) : "n"(N) : "memory");
 }
 template <int MF>
 __device__ __forceinline__ void m_landed_a(v4i (&a)[MF]) {
@@ -175,23 +183,27 @@ struct MTile {
   bool valid;
 };
 
-// OP: operands; F16: the results are IEEE half; MF: row fragments of a wave (tiles of 32 MF rows).
+// OP: operands; F16: the results are IEEE half; MF: row fragments of a wave (tiles of 32 MF rows), 6; fp8 also 4.
 template <MOp OP, bool SWIGLU, bool F16, int MF>
 __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroParams p) {
-  constexpr bool I8 = OP == MOp::I8;
+  constexpr bool I8 = OP == MOp::I8, F8 = OP == MOp::F8;
+  constexpr int kWeightSlots = F8 ? 6 : 5, kChunkBufs = F8 && MF > 4 ? 2 : 3;  // (the copies and waits below are written for these)
   constexpr int kTM = 32 * MF;
   constexpr int NFH = SWIGLU ? kMFrags / 2 : kMFrags;  // output fragments of a wave
   constexpr int kNA = MF / 2;                          // copies per wave and activation chunk: 8 rows (1 KB) each
   constexpr int kABytes = kTM * kMChunk;
-  __shared__ __attribute__((aligned(1024))) int8_t ring_a[kMChunkBufs][kABytes];
-  __shared__ __attribute__((aligned(1024))) int8_t ring_w[kMWeightSlots][kMWeightStep];
+  __shared__ __attribute__((aligned(1024))) int8_t ring_a[kChunkBufs][kABytes];
+  __shared__ __attribute__((aligned(1024))) int8_t ring_w[kWeightSlots][kMWeightStep];
   // per tile parity: the tile's channel and row absmax values, divided by 127 in place at its start
   __shared__ __attribute__((aligned(16))) float sw_lds[I8 ? 2 : 1][I8 ? 256 : 4];
   __shared__ __attribute__((aligned(16))) float sa_lds[I8 ? 2 : 1][I8 ? kTM : 4];
+  // fp8: the row scales of four chunks, two groups of chunks in turn; per tile parity the scales of its two blocks of 128 channels
+  __shared__ __attribute__((aligned(16))) float asc_lds[F8 ? 2 : 1][F8 ? 4 * kTM : 4];
+  __shared__ __attribute__((aligned(16))) float wsc_lds[F8 ? 2 : 1][F8 ? 2 * kMacroBlocks : 4];
   __shared__ __attribute__((aligned(16))) int idx_lds[kTM];  // gather entries of the next tile's rows
   __shared__ int items[4][kMItems];
   extern __shared__ int m_dyn[];
-  static_assert(sizeof(ring_a) + sizeof(ring_w) + sizeof(sw_lds) + sizeof(sa_lds) + sizeof(idx_lds) + sizeof(items) + kMacroTables <= 160 * 1024, "LDS of a CU");
+  static_assert(sizeof(ring_a) + sizeof(ring_w) + sizeof(sw_lds) + sizeof(sa_lds) + sizeof(asc_lds) + sizeof(wsc_lds) + sizeof(idx_lds) + sizeof(items) + kMacroTables <= 160 * 1024, "LDS of a CU");
   const int n_exp = p.E + (p.w_tail ? 1 : 0);
   int* row_lo = m_dyn;              // [E + 1]: lod
   int* tile_lo = m_dyn + p.E + 1;   // [n_exp + 1]: first m-tile of each expert, then the total
@@ -389,6 +401,45 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
     __builtin_amdgcn_sched_barrier(0);
     dma_scales(cur, 0, fetched);
   }
+  // fp8: a row's scales of four chunks from block `base` on; the tile's weight scales
+  const int kblocks = p.k / 128;
+  uint32_t asc_off = 0;  // the scales of tile row 64 wave + lane (waves 0-2)
+  auto dma_row_scales = [&](int base, int group) __attribute__((always_inline)) {
+    if constexpr (F8) {
+      if (64 * wave < kTM)
+        buffer_load16_to_lds(make_rsrc(p.a_max), (lds_ptr_t)&asc_lds[group][256 * wave], asc_off, static_cast<uint32_t>(base) * 4u);
+    }
+  };
+  auto dma_tile_scales = [&](const MTile& t, int parity, int fetched) __attribute__((always_inline)) {
+    if constexpr (F8) {
+      asc_off = src_row(t, clamp_row(t, t.row0 + 64 * (wave & 3) + lane), fetched) * static_cast<uint32_t>(kblocks) * 4u;
+      const int b = wave - 4;  // waves 4 and 5: a block of 128 channels each
+      if (b == 0 || b == 1) {
+        const int row = SWIGLU ? t.nb + b * (n_half / 128) : min(2 * t.nb + b, p.n / 128 - 1);
+        const float* ws = t.e >= p.E ? p.w_max_tail : p.w_max + static_cast<size_t>(t.e) * (p.n / 128) * kblocks;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(ws), (lds_ptr_t)&wsc_lds[parity][b * kMacroBlocks], 4,
+                                                 static_cast<uint32_t>(row * kblocks + min(lane, kblocks - 1)) * 4u, 0, 0, 0);
+      }
+    }
+  };
+  if constexpr (F8) {
+    const int fetched = (p.row_src && cur.e < p.E) ? p.row_src[clamp_row(cur, cur.row0 + 64 * (wave & 3) + lane)] : 0;
+    __builtin_amdgcn_sched_barrier(0);
+    dma_tile_scales(cur, 0, fetched);
+    dma_row_scales(0, 0);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {  // in the order of the chunks -2 and -1
+#pragma unroll
+      for (int i = 0; i < kNA; ++i)
+        if (kChunkBufs == 3 || c == 1) dma_a(kChunkBufs == 3 ? c : 0, kChunkBufs == 3 ? c * kABytes : 0, i);
+#pragma unroll
+      for (int st = 2 * c; st < 2 * c + 2; ++st) {
+        dma_w(w_cur, st, st * kMWeightStep, 0);
+        dma_w(w_cur, st, st * kMWeightStep, 1);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  } else {
   // in the order of the steps -5 to -1
 #pragma unroll
   for (int st = 0; st < 5; ++st) {
@@ -407,6 +458,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   m_for<kMFrags>([&](auto f) __attribute__((always_inline)) { m_read<f * 1024>(wf[0][f], fw); });
   m_landed(wf[0]);
   m_landed_a(af[0]);
+  }
 
   uint32_t slot = 0;      // bytes: the weight slot of this step; the next one's follows it
   uint32_t buf = 0;       // bytes: the buffer of this step's chunk
@@ -415,7 +467,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   // ---- the results of the tile before: finished during step 0, stored during steps 0 to 5 ----
   constexpr int kPairs = NFH / 2;     // 64-byte pieces of a row a wave holds
   constexpr int kStores = MF * kPairs;
-  constexpr int kStoreSteps = 6;
+  constexpr int kStoreSteps = F8 ? (MF == 4 ? 2 : 3) : 6;  // (fp8: chunks)
   static_assert(kStores % kStoreSteps == 0, "the same number of stores in each of the first steps");
   constexpr int kPerStep = kStores / kStoreSteps;
   v4i done[MF][kPairs];
@@ -484,7 +536,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   // activation chunk to copy; w, w_step: the weights. One copy leaves after each of the first MFMA groups: all of them at once,
   // by eight waves, kept the last wave waiting for its turn while its MFMAs could run (232 -> 225 us at 256 rows). Steps 0 to 5
   // also store what step 0 finished.
-  auto step = [&](auto st_tag, int a_chunk, const Weights& w, int w_step, auto start) __attribute__((always_inline)) {
+  [[maybe_unused]] auto step = [&](auto st_tag, int a_chunk, const Weights& w, int w_step, auto start) __attribute__((always_inline)) {
     constexpr int st = decltype(st_tag)::value;  // 0-5: steps of a tile that store; beyond: its parity and whether stores may be in flight
     constexpr bool odd = st & 1, first = st == 0;
     constexpr int S = odd ? 1 : 0;
@@ -502,8 +554,8 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
     start();
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t w_to = slot, a_to = buf;
-    slot = slot + kMWeightStep == kMWeightSlots * kMWeightStep ? 0 : slot + kMWeightStep;
-    if constexpr (odd) buf = buf + kABytes == kMChunkBufs * kABytes ? 0 : buf + kABytes;
+    slot = slot + kMWeightStep == kWeightSlots * kMWeightStep ? 0 : slot + kMWeightStep;
+    if constexpr (odd) buf = buf + kABytes == kChunkBufs * kABytes ? 0 : buf + kABytes;
     const uint32_t a_at = fa[odd ? 0 : 1] + buf, w_at = fw + slot;
     m_for<MF>([&](auto i) __attribute__((always_inline)) {
       m_read<i * 32 * kMChunk>(af[S ^ 1][i], a_at);
@@ -534,7 +586,112 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   constexpr std::integral_constant<int, 10> even{};
   constexpr std::integral_constant<int, 11> odd{};
   auto nothing = [] {};
-  static_assert(kStoreSteps == 6, "steps written out below");
+  static_assert(F8 ? kStoreSteps <= 3 : kStoreSteps == 6, "steps written out below");
+
+  // fp8: one whole chunk. An MFMA covers its 128 bytes of K - the two 1 KB weight blocks are its two halves, and the activation
+  // fragment takes the same two - and one weight scale each: its partial sum is scaled and added in f32. The fragments of a chunk
+  // are read while it runs, so a buffer is free one chunk later than above: at its start chunk c copies the activations of
+  // c + kChunkBufs - 1 and the weights of c + 2. The scaling of fragment n - 1 follows the MFMAs of fragment n.
+  int group = 0;  // of asc_lds: that of this chunk
+  [[maybe_unused]] auto chunk_f8 = [&](auto st_tag, int c, int parity, int a_chunk, const Weights& w, int w_chunk, auto start) __attribute__((always_inline)) {
+    if constexpr (F8) {
+      constexpr int st = decltype(st_tag)::value;
+      constexpr bool first = st == 0;
+      __builtin_amdgcn_sched_barrier(0);
+      // younger than chunk c's operands: the weights of c + 1 and c - 1's stores; with three buffers, whose activations left before
+      // c's weights, the activations of c + 1 and c - 2's stores, too
+      constexpr int kStored = (st >= 1 && st - 1 < kStoreSteps ? 1 : 0) + (kChunkBufs == 3 && st >= 2 && st - 2 < kStoreSteps ? 1 : 0);
+      vmem_wait<4 + (kChunkBufs == 3 ? kNA : 0) + kStored * kPerStep>();
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      start();
+      __builtin_amdgcn_sched_barrier(0);
+      const uint32_t a_to = buf == 0 ? (kChunkBufs - 1) * kABytes : buf - kABytes;
+      const uint32_t w_to = slot >= 2 * kMWeightStep ? slot - 2 * kMWeightStep : slot + 4 * kMWeightStep;
+      const uint32_t a_lo = fa[0] + buf, a_hi = fa[1] + buf, w_at = fw + slot;
+      const int base = min(c & ~3, kblocks - 4);
+      const uint32_t sa_at = lds_addr(&asc_lds[0][0]) + static_cast<uint32_t>(group * 16 * kTM + (wm * 16 + li) * 16 + 4 * (c - base));
+      const uint32_t sw_at = lds_addr(&wsc_lds[parity][SWIGLU ? 0 : (wn >> 1) * kMacroBlocks]) + 4u * c;
+      float sw[2], sa_c[2], sc[2][2];
+      v4i lo[2], hi[2], wl[kMFrags], wh[kMFrags];
+      v4f blk[2][kMFrags];
+      auto request = [&](auto n_tag) __attribute__((always_inline)) {
+        constexpr int n = decltype(n_tag)::value;
+        m_read<n * 32 * kMChunk>(lo[n & 1], a_lo);
+        m_read<n * 32 * kMChunk>(hi[n & 1], a_hi);
+        m_request_f32<n * 512>(sa_c[n & 1], sa_at);
+      };
+      auto multiply = [&](int n, int f) __attribute__((always_inline)) {
+        v8i av, wv;
+        av.lo = lo[n & 1], av.hi = hi[n & 1];
+        wv.lo = wl[f], wv.hi = wh[f];
+        blk[n & 1][f] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wv, av, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+      };
+      auto add = [&](auto n_tag) __attribute__((always_inline)) {
+        constexpr int n = decltype(n_tag)::value;
+#pragma unroll
+        for (int f = 0; f < kMFrags; ++f) {
+          v4f sum = __builtin_bit_cast(v4f, acc[n][f]);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sum[q] = __builtin_fmaf(blk[n & 1][f][q], sc[n & 1][SWIGLU ? f / 2 : 0], first ? 0.0f : sum[q]);
+          acc[n][f] = __builtin_bit_cast(v4i, sum);
+        }
+      };
+      m_request_f32<0>(sw[0], sw_at);
+      if constexpr (SWIGLU) m_request_f32<4 * kMacroBlocks>(sw[1], sw_at);
+      request(std::integral_constant<int, 0>{});
+      m_for<kMFrags>([&](auto f) __attribute__((always_inline)) {
+        m_read<f * 1024>(wl[f], w_at);
+        m_read<kMWeightStep + f * 1024>(wh[f], w_at);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kNA; ++i) dma_a(a_chunk, a_to, i);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        dma_w(w, 2 * w_chunk + i, w_to + i * kMWeightStep, 0);
+        dma_w(w, 2 * w_chunk + i, w_to + i * kMWeightStep, 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      m_for<MF>([&](auto n) __attribute__((always_inline)) {
+        if constexpr (n == 0) {
+          m_wait8<6>(wl[0], wh[0]);
+          asm volatile("" : "+v"(lo[0]), "+v"(hi[0]), "+v"(sa_c[0]), "+v"(sw[0]));
+          if constexpr (SWIGLU) asm volatile("" : "+v"(sw[1]));
+          request(std::integral_constant<int, 1>{});
+          m_wait8<7>(wl[1], wh[1]);
+          m_wait8<5>(wl[2], wh[2]);
+          m_wait8<3>(wl[3], wh[3]);
+        } else {
+          if constexpr (n + 1 < MF) {
+            request(std::integral_constant<int, n + 1>{});
+            m_wait8<3>(lo[n & 1], hi[n & 1]);
+          } else {
+            m_wait8<0>(lo[n & 1], hi[n & 1]);
+          }
+          asm volatile("" : "+v"(sa_c[n & 1]));
+        }
+        if constexpr (first) {
+          if (n < live_done) finish(n);
+        }
+        if (n < live) {  // (wave-uniform)
+#pragma unroll
+          for (int f = 0; f < kMFrags; ++f) multiply(n, f);
+          sc[n & 1][0] = sa_c[n & 1] * sw[0];
+          if constexpr (SWIGLU) sc[n & 1][1] = sa_c[n & 1] * sw[1];
+        }
+        if constexpr (n > 0) {
+          if (n - 1 < live) add(std::integral_constant<int, n - 1>{});
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if (MF - 1 < live) add(std::integral_constant<int, MF - 1>{});
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (st < kStoreSteps) m_for<kPerStep>([&](auto n) __attribute__((always_inline)) { store(std::integral_constant<int, st * kPerStep + n>{}); });
+      buf = buf + kABytes == kChunkBufs * kABytes ? 0 : buf + kABytes;
+      slot = slot + 2 * kMWeightStep == kWeightSlots * kMWeightStep ? 0 : slot + 2 * kMWeightStep;
+    }
+  };
 
   for (int parity = 0;; parity ^= 1) {
     const MTile nxt = find_tile(cur.it + 1);
@@ -543,12 +700,45 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
       const int rows = cur.end - cur.row0;
       live = __builtin_amdgcn_readfirstlane(max(0, min(MF, (rows - 16 * wm + 31) >> 5)));
     }
-    step(s0, 0, w_cur, 5, [&]() __attribute__((always_inline)) {
+    auto fetch_next = [&]() __attribute__((always_inline)) {  // the gather entries of the next tile's rows
       if (p.row_src && 64 * wave < kTM && wave < 4) {
         const int rr = clamp_row(look, look.row0 + 64 * wave + lane);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(p.row_src), (lds_ptr_t)&idx_lds[64 * wave], 4,
                                                  static_cast<uint32_t>(look.e < p.E ? rr : 0) * 4u, 0, 0, 0);
       }
+    };
+    auto next_rows = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < kNA; ++i) a_off[i] = row_offset(look, i, m_read_i32(lds_addr(&idx_lds[dma_row + 8 * i])));
+      return m_read_i32(lds_addr(&idx_lds[min(64 * (wave & 3) + lane, kTM - 1)]));
+    };
+    const Weights w_nxt = weights_of(look);
+    if constexpr (F8) {
+      auto group_of = [&](int c) { return min(c, kblocks - 4); };
+      if (cur.it > 0) group ^= 1;  // (copied during the tile before)
+      constexpr int ahead = kChunkBufs - 1;
+      chunk_f8(s0, 0, parity, ahead, w_cur, 2, fetch_next);
+      chunk_f8(s1, 1, parity, 1 + ahead, w_cur, 3, nothing);
+      chunk_f8(s2, 2, parity, 2 + ahead, w_cur, 4, [&]() __attribute__((always_inline)) { dma_row_scales(group_of(4), group ^ 1); });
+      for (int c = 3; c < kblocks - 2; ++c) {
+        if ((c & 3) == 0) group ^= 1;
+        chunk_f8(even, c, parity, c + ahead, w_cur, c + 2, [&]() __attribute__((always_inline)) {
+          if ((c & 3) == 2 && c + 2 < kblocks) dma_row_scales(group_of(c + 2), group ^ 1);
+        });
+      }
+      // the last two: the copies go over to the next tile
+      if (((kblocks - 2) & 3) == 0) group ^= 1;
+      chunk_f8(even, kblocks - 2, parity, ahead == 2 ? 0 : kblocks - 1, w_nxt, 0, [&]() __attribute__((always_inline)) {
+        if constexpr (ahead == 2) dma_tile_scales(look, parity ^ 1, next_rows());
+      });
+      if (((kblocks - 1) & 3) == 0) group ^= 1;
+      chunk_f8(even, kblocks - 1, parity, ahead - 1, w_nxt, 1, [&]() __attribute__((always_inline)) {
+        if constexpr (ahead == 1) dma_tile_scales(look, parity ^ 1, next_rows());
+        dma_row_scales(0, group ^ 1);
+      });
+    } else {
+    step(s0, 0, w_cur, 5, [&]() __attribute__((always_inline)) {
+      fetch_next();
       scales_in_place(parity);
     });
     step(s1, 3, w_cur, 6, nothing);
@@ -561,17 +751,15 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
       step(odd, (ks >> 1) + 3, w_cur, ks + 6, nothing);
     }
     // the last six: the copies go over to the next tile
-    const Weights w_nxt = weights_of(look);
     step(even, 0, w_cur, ksteps - 1, [&]() __attribute__((always_inline)) {  // (the gather entries landed before the wait of an odd step before)
-#pragma unroll
-      for (int i = 0; i < kNA; ++i) a_off[i] = row_offset(look, i, m_read_i32(lds_addr(&idx_lds[dma_row + 8 * i])));
-      dma_scales(look, parity ^ 1, m_read_i32(lds_addr(&idx_lds[min(64 * (wave & 3) + lane, kTM - 1)])));
+      dma_scales(look, parity ^ 1, next_rows());
     });
     step(odd, 0, w_nxt, 0, nothing);
     step(even, 0, w_nxt, 1, nothing);
     step(odd, 1, w_nxt, 2, nothing);
     step(even, 0, w_nxt, 3, nothing);
     step(odd, 2, w_nxt, 4, nothing);
+    }
 
     // the MFMAs came from assembly statements, so the compiler knows of no wait for their results
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
@@ -601,8 +789,8 @@ int launch_macro(MacroParams p, int rows, hipStream_t s, int n_cu, const char* w
   const int grid = static_cast<int>(min((max_items + 7) / 8 * 8, static_cast<long long>(ceil_div(n_cu, 8) * 8)));
   const size_t dyn = sizeof(int) * (static_cast<size_t>(p.E) + 1 + n_exp + 1);
   if (tracing_kernels())
-    note_kernel("macro_tile_kernel<%s%s, %s, %dx256 tile, both operands through LDS>", OP == MOp::I8 ? "int8" : (OP == MOp::F16 ? "f16" : "bf16"),
-                (OP == MOp::I8 && F16) ? " -> f16" : "", SWIGLU ? "SiLU-mul" : "plain", 32 * MF);
+    note_kernel("macro_tile_kernel<%s%s, %s, %dx256 tile, both operands through LDS>", OP == MOp::I8 ? "int8" : (OP == MOp::F8 ? "fp8" : (OP == MOp::F16 ? "f16" : "bf16")),
+                ((OP == MOp::I8 || OP == MOp::F8) && F16) ? " -> f16" : "", SWIGLU ? "SiLU-mul" : "plain", 32 * MF);
   hipLaunchKernelGGL((macro_tile_kernel<OP, SWIGLU, F16, MF>), dim3(grid), dim3(kMThreads), dyn, s, p);
   return check_launch(what);
 }
@@ -610,6 +798,14 @@ int launch_macro(MacroParams p, int rows, hipStream_t s, int n_cu, const char* w
 }  // namespace
 
 int macro_tile(const MacroParams& p, int kind, bool swiglu, bool f16, int rows, hipStream_t s, int n_cu, const char* what) {
+  if (kind == 2) {
+    if (p.low) {
+      if (f16) return swiglu ? launch_macro<MOp::F8, true, true, 4>(p, rows, s, n_cu, what) : launch_macro<MOp::F8, false, true, 4>(p, rows, s, n_cu, what);
+      return swiglu ? launch_macro<MOp::F8, true, false, 4>(p, rows, s, n_cu, what) : launch_macro<MOp::F8, false, false, 4>(p, rows, s, n_cu, what);
+    }
+    if (f16) return swiglu ? launch_macro<MOp::F8, true, true, 6>(p, rows, s, n_cu, what) : launch_macro<MOp::F8, false, true, 6>(p, rows, s, n_cu, what);
+    return swiglu ? launch_macro<MOp::F8, true, false, 6>(p, rows, s, n_cu, what) : launch_macro<MOp::F8, false, false, 6>(p, rows, s, n_cu, what);
+  }
   if (kind == 0) {
     if (f16) return swiglu ? launch_macro<MOp::I8, true, true, 6>(p, rows, s, n_cu, what) : launch_macro<MOp::I8, false, true, 6>(p, rows, s, n_cu, what);
     return swiglu ? launch_macro<MOp::I8, true, false, 6>(p, rows, s, n_cu, what) : launch_macro<MOp::I8, false, false, 6>(p, rows, s, n_cu, what);

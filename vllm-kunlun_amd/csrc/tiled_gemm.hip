@@ -1490,7 +1490,7 @@ bool macro_params(const TiledParams& p, int live, MacroParams* out) {
   const float mean = static_cast<float>(ceil_div(live, p.E));
   *out = MacroParams{p.a, p.lda, p.a_max, p.row_src, magic, p.w, p.w_max, p.lod, p.E, p.n, p.k, p.y, p.ldy,
                      p.w_tail, p.w_max_tail, p.tail_row0, p.tail_rows, p.tail_src0, 0, p.m_major,
-                     past && mean + 2.2f * sqrtf(mean) <= 192.0f, past};
+                     mean + 2.2f * sqrtf(mean) <= 128.0f, past && mean + 2.2f * sqrtf(mean) <= 192.0f, past};
   return true;
 }
 
@@ -1504,8 +1504,12 @@ bool macro_params(const TiledParams& p, int live, MacroParams* out) {
 //   bf16, Qwen3 dims, gate_up, 49 rows 135 / 127; 139 / 147, 125 160 / 145; 186 / 171, 188 191 / 207; 215 / 210, 512 405 / 416; 395 / 426; down, 19 rows
 //   75.6 / 69.1; 80 / 73, 100 104 / 85; 112 / 96, 256 152 / 148; 164 / 152, 512 256 / 242; 259 / 255; 160 experts of [3072 x 2560], gate_up, 15 rows
 //   427 / 391; 438 / 384; 32 of [4096 x 1024], 75 rows 47 / 50; 51 / 58
+//   fp8, DeepSeek-V3 dims, gate_up, 12 rows 1147 / 1092; 1185 / 1148, 31 1206 / 1121; 1303 / 1190, 64 1306 / 1250; 1500 / 1390, 94 1350 / 1286; 1654 /
+//   1560, 128 1555 / 1487; 1882 / 1774; down, 31 rows 663 / 648; 700 / 675, 94 728 / 712; 866 / 849; 16 experts of [8192 x 4096], 75 rows 95 / 104;
+//   150 / 121, 150 132 / 118; 191 / 166; [2048 x 768], 125 rows 62 / 69; 72 / 83
 // So: wherever every CU gets four items of 192 rows; from two on where rows are many or, without SiLU-mul, 16-bit weights exceed the
-// memory-side cache. 16-bit gate_up launches are bound by their weights: only while one tile holds nearly every expert.
+// memory-side cache. 16-bit gate_up launches are bound by their weights: only while one tile holds nearly every expert. fp8, whose
+// fragments of a chunk are waited for at its start, where the weights exceed that cache, too.
 bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_cu) {
   const float mean = static_cast<float>(ceil_div(live, p.E));
   const long long weights = static_cast<long long>(p.E) * p.n * p.k;
@@ -1515,6 +1519,7 @@ bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_c
     if (!swiglu) return many || (some && weights > (256ll << 20));
     return (many && mean + 2.2f * sqrtf(mean) <= 192.0f) || (some && mean > 80.0f && mean <= 150.0f);
   }
+  if (kind == TKind::F8) return (many && weights > (256ll << 20)) || (some && swiglu && mean > 100.0f);
   if (many) return true;
   if (swiglu) return some && mean > 72.0f;
   return (some && mean > 88.0f && (p.k < 4096 || weights > (1ll << 30))) || (items < n_cu && mean > 128.0f);
@@ -1746,6 +1751,15 @@ int tiled_gemm_fp8(const kmoe_gemm_fp8_args* a, hipStream_t s) {
   // still bound by what one workgroup keeps in flight; not instantiated)
   const bool half = a->act_dtype == KMOE_DT_F16;  // half outputs: the same three shapes
   const int live = expected_rows(a->rows, a->rows_hint);
+  if (a->variant == 0 && macro_pays(K, p, live, swiglu, n_cu) && (!swiglu || a->n % 256 == 0)) {
+    MacroParams macro;
+    if (macro_params(p, live, &macro)) return macro_tile(macro, 2, swiglu, half, a->rows, s, n_cu, what);
+  }
+  if (a->variant == 23) {
+    MacroParams macro;
+    KMOE_REQUIRE((!swiglu || a->n % 256 == 0) && macro_params(p, live, &macro), KMOE_ERR_UNSUPPORTED, "%s: variant 23 needs k >= 768, at most some 410 experts, n %% 256 == 0 with SiLU-mul and src_div 1 to 4, 6, 8 or another power of two", what);
+    return macro_tile(macro, 2, swiglu, half, a->rows, s, n_cu, what);
+  }
   if (short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu)) return launch_short<K>(p, a->rows, s, n_cu, what, swiglu, half);
   // (Paced sibling m-tiles - variant 12 - had been the default where experts have several m-tiles, the weights are
   // far more than the memory-side cache holds and a tile walks a long K. With an expert's rows split evenly over
