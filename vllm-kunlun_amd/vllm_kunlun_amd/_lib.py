@@ -6,6 +6,7 @@ has not been built, importing this module raises.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 
 import torch
@@ -13,6 +14,7 @@ import torch
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 PROJECT_DIR = os.path.dirname(_PKG_DIR)
 LIB_PATH = os.path.join(PROJECT_DIR, "lib", "libkmoe.so")
+TORCH_CALLS_PATH = os.path.join(PROJECT_DIR, "lib", "kmoe_torch.so")
 
 KMOE_ACT_NONE = 0
 KMOE_ACT_SWIGLU = 1
@@ -174,7 +176,18 @@ def _load() -> C.CDLL:
     return lib
 
 
+def _load_torch_calls():
+    """The extension of calls whose host time matters (csrc/torch_calls.cpp), beside the library it calls."""
+    if not os.path.exists(TORCH_CALLS_PATH):
+        raise ImportError(f"{TORCH_CALLS_PATH} is missing: build it with `make -C {PROJECT_DIR}` (or __graft_entry__.build()).")
+    spec = importlib.util.spec_from_file_location("kmoe_torch", TORCH_CALLS_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
 lib = _load()
+torch_calls = _load_torch_calls()
 EXPORTS = (
     "kmoe_last_error", "kmoe_version", "kmoe_softmax_topk", "kmoe_sigmoid_group_topk_norm", "kmoe_block_statistic",
     "kmoe_align_workspace_bytes", "kmoe_align", "kmoe_gather_rows", "kmoe_quant_i8_rows", "kmoe_quant_i8_rows_chunked", "kmoe_tile_weights_i8", "kmoe_quant_fp8_group128", "kmoe_quant_fp8_group128_dt",

@@ -550,6 +550,10 @@ def silu_and_mul(out: torch.Tensor, x: torch.Tensor, axis: int = -1, turn: bool 
     L.check(L.lib.kmoe_silu_and_mul_dt(x.data_ptr(), two_i, R, d, out.data_ptr(), d, dt, L.raw_stream()))
 
 
+# On GPU tensors the native body is called (csrc/torch_calls.cpp), which leaves what is not ordinary to this one.
+L.torch_calls.install(L.check, silu_and_mul)
+
+
 @operator("_C::moe_post", mutates_args=("y",))
 def moe_post(x: torch.Tensor, moe_index: torch.Tensor, normed_scale: torch.Tensor, dequant_scale: torch.Tensor,
              y: torch.Tensor) -> None:
