@@ -10,8 +10,8 @@ FEW = [0, 1, 2, 0, 3] * 12  # with these an expert holds few rows on average: th
 ROWS = [1, 15, 16, 17, 0, 191, 192, 193, 33, 384, 385, 0, 127, 128, 129, 800, 3100]  # up to 17 tiles of an expert
 
 
-def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, bound=0, seed=0):
-    """Outputs of the variants 6 and 23 for the same operands. pad: values between the rows of a and y; tail: rows of an expert
+def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, bound=0, seed=0, variant=23):
+    """Outputs of the variants 6 and 23 (or another) for the same operands. pad: values between the rows of a and y; tail: rows of an expert
     outside w (int8); bound: rows the caller allows for beyond the last expert's."""
     from vllm_kunlun_amd import _lib as L
     g = torch.Generator(device="cuda").manual_seed(seed)
@@ -44,9 +44,9 @@ def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, b
     q.row_src, q.src_div = (src.data_ptr(), div) if gather else (0, 1)
     q.E, q.n, q.k, q.rows, q.act, q.ldy = E, n, k, rows + bound, act, n_out + pad
     out = []
-    for variant in (19 if f8 else 6, 23):
+    for v in (19 if f8 else 6, variant):
         y = torch.full((rows + tail, n_out + pad), float("nan"), dtype=dtype, device="cuda")
-        q.y, q.variant, q.act_dtype = y.data_ptr(), variant, L.act_dtype(y, "test")
+        q.y, q.variant, q.act_dtype = y.data_ptr(), v, L.act_dtype(y, "test")
         launch = L.lib.kmoe_grouped_gemm_i8 if i8 else (L.lib.kmoe_grouped_gemm_fp8_block if f8 else L.lib.kmoe_grouped_gemm_bf16)
         L.check(launch(q, L.stream()))
         out.append(y)
@@ -105,3 +105,16 @@ def test_what_the_launch_does_not_take(k, div, experts):
     from vllm_kunlun_amd import _lib as L
     with pytest.raises(NotImplementedError):
         _launch("int8", [5] * experts, 32, k, 0, torch.bfloat16, div=div)
+
+
+@pytest.mark.parametrize("n,k,rows", [(7168, 768, 700), (7168, 768, 1400), (7168, 640, 1400), (12288, 768, 3500), (7168, 4096, 1900), (4096, 4096, 4000), (65536, 128, 66)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_one_matrix_alone(n, k, rows, dtype):
+    """The tile taken by rounds: 64 rows, 192 (wide, wide, macro), 128, and a few rows of many channels."""
+    _same(*_launch("int8", [rows], n, k, 0, dtype, gather=False, variant=0))
+
+
+@pytest.mark.parametrize("n,k,rows,experts", [(7168, 768, 300, 4), (1536, 768, 150, 32), (1536, 768, 300, 16), (512, 4096, 150, 128), (512, 4096, 400, 128)])
+def test_less_than_a_round(n, k, rows, experts):
+    """Few tiles for the CUs, and a long K."""
+    _same(*_launch("int8", [rows] * experts, n, k, 0, torch.bfloat16, variant=0))

@@ -1486,43 +1486,63 @@ bool macro_params(const TiledParams& p, int live, MacroParams* out) {
     if (static_cast<uint64_t>(magic) * p.src_div - (1ull << 32) > 2) return false;
   }
   if (!macro_tile_takes(p.k, p.E, p.w_tail != nullptr) || p.acc_out || p.bias) return false;
-  const bool past = p.E > 1 && static_cast<long long>(p.E) * p.n * p.k > (256ll << 20);
+  const bool past = p.E > 1, big = static_cast<long long>(p.E) * p.n * p.k > (256ll << 20);
   const float mean = static_cast<float>(ceil_div(live, p.E));
   *out = MacroParams{p.a, p.lda, p.a_max, p.row_src, magic, p.w, p.w_max, p.lod, p.E, p.n, p.k, p.y, p.ldy,
                      p.w_tail, p.w_max_tail, p.tail_row0, p.tail_rows, p.tail_src0, 0, p.m_major,
-                     mean + 2.2f * sqrtf(mean) <= 128.0f, past && mean + 2.2f * sqrtf(mean) <= 192.0f, past};
+                     mean + 2.2f * sqrtf(mean) <= 128.0f, past && big && mean + 2.2f * sqrtf(mean) <= 192.0f, past};
   return true;
 }
 
-// Where that launch is ahead of the tiles of this file. GEMM alone, us, those / that one, even load; +2.0 on the logits of 8 experts:
-//   int8, Qwen3 dims, gate_up, 49 rows per expert 70 / 72; 74 / 80, 75 83 / 76; 93 / 88, 156 106 / 92; 126 / 112, 256 152 / 136; 160 / 144, 512 243 / 219;
-//   264 / 239; down, 12 rows 37.0 / 36.5; 40.2 / 37.6, 49 46 / 41; 51.5 / 45, 188 92 / 69; 91 / 73, 512 187 / 135; 198 / 142
-//   int8, DeepSeek-V3 dims, gate_up, 12 rows 1136 / 1083; 1143 / 1111, 47 1285 / 1151; 1372 / 1220, 128 1424 / 1310; 1720 / 1582; down, 12 rows 619 /
-//   602; 623 / 602, 94 727 / 733; 845 / 809, 128 780 / 750; 902 / 882; Kimi-K2 dims, 85 rows 2021 / 1848; 2285 / 2051 and 1070 / 1087; 1217 / 1187
-//   int8, 32 experts of [2048 x 4096], gate_up, 150 rows 52 / 50; 70 / 75, of [4096 x 1024] 75 rows 30.7 / 32.4; 37 / 36; 16 of [4096 x 4096], 375 to
-//   1024 rows 0.97 to 1.05 times as fast; 8 of [4096 x 14336], 150 rows 153 / 107; 170 / 111 (their 192-row tiles are too few for the CUs)
-//   bf16, Qwen3 dims, gate_up, 49 rows 135 / 127; 139 / 147, 125 160 / 145; 186 / 171, 188 191 / 207; 215 / 210, 512 405 / 416; 395 / 426; down, 19 rows
-//   75.6 / 69.1; 80 / 73, 100 104 / 85; 112 / 96, 256 152 / 148; 164 / 152, 512 256 / 242; 259 / 255; 160 experts of [3072 x 2560], gate_up, 15 rows
-//   427 / 391; 438 / 384; 32 of [4096 x 1024], 75 rows 47 / 50; 51 / 58
-//   fp8, DeepSeek-V3 dims, gate_up, 12 rows 1147 / 1092; 1185 / 1148, 31 1206 / 1121; 1303 / 1190, 64 1306 / 1250; 1500 / 1390, 94 1350 / 1286; 1654 /
-//   1560, 128 1555 / 1487; 1882 / 1774; down, 31 rows 663 / 648; 700 / 675, 94 728 / 712; 866 / 849; 16 experts of [8192 x 4096], 75 rows 95 / 104;
-//   150 / 121, 150 132 / 118; 191 / 166; [2048 x 768], 125 rows 62 / 69; 72 / 83
-// So: wherever every CU gets four items of 192 rows; from two on where rows are many or, without SiLU-mul, 16-bit weights exceed the
-// memory-side cache. 16-bit gate_up launches are bound by their weights: only while one tile holds nearly every expert. fp8, whose
-// fragments of a chunk are waited for at its start, where the weights exceed that cache, too.
+// Where that launch is ahead of the tiles of this file. The layer, us, those / that one, three layers' weights in turn (weights that the last
+// call left in the memory-side cache, which the next layer's never are, favour this launch by up to 8 % in down launches of few rows):
+//   Qwen3 dims, int8, 300 tokens (19 rows per expert) down 127.6 / 128.7, gate_up / 129.9, 1000 148.0 / 151.3, / 151.6, 1400 both 174 / 165, 2500 232 / 212,
+//   8192 519 / 475; +2.0 on the logits of 8 experts, 900 tokens 167 / 161, 1500 205 / 183
+//   Qwen3 dims, bf16, gate_up (down on it) 200 tokens 218 / 212, 500 222 / 215, 1200 244 / 236, 2500 316 / 307, 3500 372 / 404, 5000 462 / 461; down, 200 tokens
+//   222.6 / 218.5, 1200 255 / 244, 5000 471 / 462, 8000 694 / 680
+//   DeepSeek-V3 dims, int8, 300 tokens 1884 / 1880, 700 1943 / 1885, 1500 2170 / 2019, 4096 2526 / 2430; fp8, 300 1834 / 1833 (down on it too 1849), 500
+//   1891 / 1820, 1200 2080 / 1924, 2000 2230 / 2010, 3001 2378 / 2300, 4096 2831 / 2790
+// GEMM alone, weights cold, the same number of rows per expert:
+//   int8, gate_up, 64 experts of [4096 x 1024], 25 rows (uneven) 52.5 / 57.6, 32 of them 150 rows 38.5 / 34.1; bf16, 64 of them, 25 rows (uneven) 102 / 108,
+//   150 116 / 103
+//   int8, down, 32 experts of [7168 x 2048], 150 rows 119 / 106, 16 experts, 1000 256 / 244; of [4096 x 7168], 32 experts, 150 rows 196 / 173, 600 525 / 550;
+//   bf16, [7168 x 2048], 8 experts, 1000 rows 199 / 232, 32 experts, 300 304 / 297; [4096 x 7168], 16 experts, 300 rows 308 / 281, 600 504 / 526
+//   less than a round of items: int8, 32 experts of [1536 x 2048], 150 rows (192 items here, 576 of 64 rows) 30.7 / 26.6, 16 experts of 300 (192 and 480)
+//   22.7 / 26.9, 4 experts of [4096 x 7168], 300 (128 and 320) 51.7 / 58.7; 4 of [7168 x 2048], 375 on average, uneven (224) 31.1 / 42.6
+// So, by rounds of items of 192 rows over the CUs. gate_up: int8 from four rounds on, two where rows are many; 16-bit, bound by its weights, from two on
+// while one tile holds nearly every expert. down: four rounds and weights beyond the memory-side cache, or two and many rows (16-bit: one of the
+// two); over a long K only while an expert has few tiles. One round that leaves a quarter of the CUs free for an uneven load, where the 64-row
+// tiles, two per CU, need a second. fp8, whose fragments of a chunk are waited for at its start, only where the weights exceed that cache, too.
 bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_cu) {
   const float mean = static_cast<float>(ceil_div(live, p.E));
   const long long weights = static_cast<long long>(p.E) * p.n * p.k;
-  const long long items = static_cast<long long>(p.E) * ceil_div(static_cast<int>(mean), 192) * ceil_div(p.n, 256);
+  auto items_of = [&](int rows) { return static_cast<long long>(p.E) * ceil_div(static_cast<int>(mean), rows) * ceil_div(p.n, 256); };
+  const long long items = items_of(192);
   const bool many = items >= 4ll * n_cu, some = items >= 2ll * n_cu;
   if (kind == TKind::BF16) {
-    if (!swiglu) return many || (some && weights > (256ll << 20));
-    return (many && mean + 2.2f * sqrtf(mean) <= 192.0f) || (some && mean > 80.0f && mean <= 150.0f);
+    if (!swiglu) return (many || (some && weights > (256ll << 20))) && (mean <= 400.0f || p.k < 4096);
+    return some && (p.k >= 4096 || mean > 72.0f) && mean + 2.2f * sqrtf(mean) <= 192.0f;
   }
-  if (kind == TKind::F8) return (many && weights > (256ll << 20)) || (some && swiglu && mean > 100.0f);
-  if (many) return true;
-  if (swiglu) return some && mean > 72.0f;
-  return (some && mean > 88.0f && (p.k < 4096 || weights > (1ll << 30))) || (items < n_cu && mean > 128.0f);
+  if (kind == TKind::F8) return (many && weights > (256ll << 20) && (swiglu || p.k < 4096)) || (some && swiglu && mean > 100.0f);
+  if (swiglu) return (many && p.k >= 2048) || (some && mean > 72.0f);
+  if (p.k >= 4096) return some && mean > 88.0f && mean <= 320.0f;  // (never one matrix)
+  return (many && weights > (256ll << 20)) || (some && mean > 88.0f) || (p.E > 1 && mean > 128.0f && 4 * items <= 3ll * n_cu && items_of(64) > 2ll * n_cu);
+}
+
+// One int8 matrix alone (a Linear), whose rows are known exactly: the tile's rows by rounds of workgroups. A round of 64 x 256 tiles, two
+// per CU, takes 100, a last one of at most one per CU 65, of 128 x 256 tiles 180 and 110 (over a K of less than 4096 codes 200 and 120), of 192
+// x 256 ones, one per CU, 120. GEMM alone, us, 64 / 128 / 192 rows (wide tiles): [4096 x 7168] 1000 rows 37 / 57 / 57, 2000 60 / 63 / 59, 2500 83 /
+// 85 / 66, 4096 115 / 104 / 124; [7168 x 2048] 700 rows 19.9 / 24.6 / 22.9, 1400 30.1 / 34.7 / 26.1, 2000 38.8 / 37.5 / 44.2, 3000 56.9 / 55.4 / 48.6;
+// [12288 x 5120] 700 59.5 / 62.5 / 46.8, 1200 83 / 76 / 91; [4096 x 640] 2500 17.7 / 20.6 / 15.7, 3500 21.1 / 22.3 / 25.1.
+// The 192 rows as the macro tile from two rounds of a short K on, us, wide / macro: [24576 x 1536] 4096 rows 175 / 167, [7168 x 2048] 1400 26.1 / 27.8,
+// 6000 102 / 97; [8192 x 8192] 3000 161 / 168.
+int one_matrix_rows(int rows, int n, int k, int n_cu) {
+  auto cost = [&](int tile, int pair, int single) {
+    const long long items = static_cast<long long>(ceil_div(rows, tile)) * ceil_div(n, 256), rest = items % (2 * n_cu);
+    return items / (2 * n_cu) * pair + (rest == 0 ? 0 : rest <= n_cu ? single : pair);
+  };
+  const long long c64 = cost(64, 100, 65), c128 = k < 4096 ? cost(128, 200, 120) : cost(128, 180, 110), c192 = cost(192, 240, 120);
+  return c64 <= c128 && c64 <= c192 ? 64 : c128 < c192 ? 128 : 192;
 }
 
 // One 8-wave tile of 16 MF rows per workgroup with the eight waves side by side along the channels (32 channels
@@ -1596,7 +1616,9 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   const int live = expected_rows(a->rows, a->rows_hint);  // (chooses the tile shape; grids and bounds keep a->rows)
   const int n_exp = a->E + (a->w_tail ? 1 : 0);
   const int avg_rows = ceil_div(live + (a->w_tail ? a->tail_rows : 0), n_exp);
-  const bool shorter = short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu);
+  // (rows of the tile for one matrix alone, 0: the rules for experts)
+  const int one = a->variant == 0 && a->E == 1 && !swiglu && !a->w_tail ? one_matrix_rows(live, a->n, a->k, n_cu) : 0;
+  const bool shorter = one ? one == 64 : short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu);
   // 128-row 4-wave tiles whose sibling m-tiles are paced against each other (see g_board): variant 12, and the
   // second launch of the device-decided pair (variant 17). They were the default where experts have several m-tiles
   // and the launch's weights are far more than the 256 MB memory-side cache holds (a sibling that falls behind
@@ -1671,7 +1693,7 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   const float avg_routed = static_cast<float>(ceil_div(live, a->E));
   const float reach = avg_routed + 3.0f * sqrtf(avg_routed);
   const bool big = weight_bytes > (1ll << 30);
-  if (a->variant == 0 && macro_pays(K, p, live, swiglu, n_cu) && macro_params(p, live, &macro)) {
+  if (a->variant == 0 && (one == 0 || one == 192) && macro_pays(K, p, live, swiglu, n_cu) && macro_params(p, live, &macro)) {
     return macro_tile(macro, 0, swiglu, a->act_dtype == KMOE_DT_F16, a->rows, s, n_cu, what);
   }
   int wide = 0;  // row fragments of the wide tile (8: 128 rows, 12: 192, 16: 256), 0: none
@@ -1682,9 +1704,9 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
     case 8: case 16: case 22: wide = 16; break;
     default: break;
   }
-  if (a->variant == 0 && !shorter && (big || avg_rows > 72)) {
+  if (a->variant == 0 && !shorter && one != 128 && (big || one || avg_rows > 72)) {
     // (small weights keep the 96-row tiles up to 72 rows per expert: Qwen3 dims at 1024 tokens 0.164 against 0.169)
-    wide = reach <= 128.0f ? 8 : 12;
+    wide = reach <= 128.0f && !one ? 8 : 12;
   } else if (a->variant == 17) {
     wide = reach <= 128.0f ? 8 : (reach <= 192.0f ? 12 : 16);
     pair = true;
