@@ -1478,6 +1478,10 @@ int tiled_common(const TiledParams& p, int rows, int* n_cu_out, const char* what
   return KMOE_OK;
 }
 
+// fp8, where 128 rows hold nearly every expert: the lower macro tile, whose third chunk buffer is worth an expert in twelve with a second tile
+// (DeepSeek-V3 dims, 109 rows per expert 2749 -> 2691 us, 119 2822 -> 2832, 128 2908 -> 3086).
+bool macro_low(float mean) { return mean + 1.7f * sqrtf(mean) <= 128.0f; }
+
 // The launch as macro_tile.hip takes it; false where it does not.
 bool macro_params(const TiledParams& p, int live, MacroParams* out) {
   uint32_t magic = 0;
@@ -1490,7 +1494,7 @@ bool macro_params(const TiledParams& p, int live, MacroParams* out) {
   const float mean = static_cast<float>(ceil_div(live, p.E));
   *out = MacroParams{p.a, p.lda, p.a_max, p.row_src, magic, p.w, p.w_max, p.lod, p.E, p.n, p.k, p.y, p.ldy,
                      p.w_tail, p.w_max_tail, p.tail_row0, p.tail_rows, p.tail_src0, 0, p.m_major,
-                     mean + 2.2f * sqrtf(mean) <= 128.0f, past && big && mean + 2.2f * sqrtf(mean) <= 192.0f, past};
+                     macro_low(mean), past && big && mean + 2.2f * sqrtf(mean) <= 192.0f, past};
   return true;
 }
 
@@ -1512,7 +1516,10 @@ bool macro_params(const TiledParams& p, int live, MacroParams* out) {
 // So, by rounds of items of 192 rows over the CUs. gate_up: int8 from four rounds on, two where rows are many; 16-bit, bound by its weights, from two on
 // while one tile holds nearly every expert. down: four rounds and weights beyond the memory-side cache, or two and many rows (16-bit: one of the
 // two); over a long K only while an expert has few tiles. One round that leaves a quarter of the CUs free for an uneven load, where the 64-row
-// tiles, two per CU, need a second. fp8, whose fragments of a chunk are waited for at its start, only where the weights exceed that cache, too.
+// tiles, two per CU, need a second. fp8, whose fragments of a chunk are waited for at its start, only where the weights exceed that cache, too; and
+// of experts beyond an XCD's L2 only where one tile, two thirds full, holds most of them, or many do: layer, us, the other tiles / that one,
+// DeepSeek-V3 dims, 119 rows 2757 / 2813, 141 3149 / 2992, 163 3499 / 3361, 172 3820 / 3604, 219 4391 / 4732, 256 5040 / 5513, 384 7041 / 7225; Kimi-K2
+// dims, 125 4060 / 3850, 171 5159 / 4849. (Qwen3 dims, whose experts it holds: 128 rows 219 / 202, 256 335 / 326, 512 587 / 563.)
 bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_cu) {
   const float mean = static_cast<float>(ceil_div(live, p.E));
   const long long weights = static_cast<long long>(p.E) * p.n * p.k;
@@ -1523,7 +1530,12 @@ bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_c
     if (!swiglu) return (many || (some && weights > (256ll << 20))) && (mean <= 400.0f || p.k < 4096);
     return some && (p.k >= 4096 || mean > 72.0f) && mean + 2.2f * sqrtf(mean) <= 192.0f;
   }
-  if (kind == TKind::F8) return (many && weights > (256ll << 20) && (swiglu || p.k < 4096)) || (some && swiglu && mean > 100.0f);
+  if (kind == TKind::F8) {
+    if (static_cast<long long>(p.n) * p.k > (4ll << 20) && !macro_low(mean) && mean <= 800.0f &&
+        (mean < 124.0f || mean + 1.5f * sqrtf(mean) > 192.0f))
+      return false;
+    return (many && weights > (256ll << 20) && (swiglu || p.k < 4096)) || (some && swiglu && mean > 100.0f);
+  }
   if (swiglu) return (many && p.k >= 2048) || (some && mean > 72.0f);
   if (p.k >= 4096) return some && mean > 88.0f && mean <= 320.0f;  // (never one matrix)
   return (many && weights > (256ll << 20)) || (some && mean > 88.0f) || (p.E > 1 && mean > 128.0f && 4 * items <= 3ll * n_cu && items_of(64) > 2ll * n_cu);
