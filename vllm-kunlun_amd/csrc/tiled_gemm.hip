@@ -1504,6 +1504,8 @@ bool macro_params(const TiledParams& p, int live, MacroParams* out) {
 //   8192 519 / 475; +2.0 on the logits of 8 experts, 900 tokens 167 / 161, 1500 205 / 183
 //   Qwen3 dims, bf16, gate_up (down on it) 200 tokens 218 / 212, 500 222 / 215, 1200 244 / 236, 2500 316 / 307, 3500 372 / 404, 5000 462 / 461; down, 200 tokens
 //   222.6 / 218.5, 1200 255 / 244, 5000 471 / 462, 8000 694 / 680
+//   the same with +2.0 on the logits of 8 experts, gate_up (down on it), 280 tokens 232 / 221, 350 242 / 268, 450 235 / 243, 750 246 / 254, 1050 270 / 270; down,
+//   350 234 / 242, 450 235 / 235, 600 248 / 241, 900 262 / 252: where the launch is three or four rounds of items, an uneven load adds another
 //   DeepSeek-V3 dims, int8, 300 tokens 1884 / 1880, 700 1943 / 1885, 1500 2170 / 2019, 4096 2526 / 2430; fp8, 300 1834 / 1833 (down on it too 1849), 500
 //   1891 / 1820, 1200 2080 / 1924, 2000 2230 / 2010, 3001 2378 / 2300, 4096 2831 / 2790
 // GEMM alone, weights cold, the same number of rows per expert:
@@ -1514,7 +1516,7 @@ bool macro_params(const TiledParams& p, int live, MacroParams* out) {
 //   less than a round of items: int8, 32 experts of [1536 x 2048], 150 rows (192 items here, 576 of 64 rows) 30.7 / 26.6, 16 experts of 300 (192 and 480)
 //   22.7 / 26.9, 4 experts of [4096 x 7168], 300 (128 and 320) 51.7 / 58.7; 4 of [7168 x 2048], 375 on average, uneven (224) 31.1 / 42.6
 // So, by rounds of items of 192 rows over the CUs. gate_up: int8 from four rounds on, two where rows are many; 16-bit, bound by its weights, from two on
-// while one tile holds nearly every expert. down: four rounds and weights beyond the memory-side cache, or two and many rows (16-bit: one of the
+// while one tile holds nearly every expert, a hot one too (few rows) or many rows pay for a round more. down: four rounds and weights beyond the memory-side cache, or two and many rows (16-bit: one of the
 // two); over a long K only while an expert has few tiles. One round that leaves a quarter of the CUs free for an uneven load, where the 64-row
 // tiles, two per CU, need a second. fp8, whose fragments of a chunk are waited for at its start, only where the weights exceed that cache, too; and
 // of experts beyond an XCD's L2 only where one tile, two thirds full, holds most of them, or many do: layer, us, the other tiles / that one,
@@ -1527,6 +1529,7 @@ bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_c
   const long long items = items_of(192);
   const bool many = items >= 4ll * n_cu, some = items >= 2ll * n_cu;
   if (kind == TKind::BF16) {
+    if (items < 8ll * n_cu && mean > 18.0f && mean <= (swiglu ? 72.0f : 27.0f)) return false;
     if (!swiglu) return (many || (some && weights > (256ll << 20))) && (mean <= 400.0f || p.k < 4096);
     return some && (p.k >= 4096 || mean > 72.0f) && mean + 2.2f * sqrtf(mean) <= 192.0f;
   }
