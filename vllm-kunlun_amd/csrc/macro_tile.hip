@@ -134,12 +134,15 @@ __device__ __forceinline__ v4i m_rsrc(const void* base, uint32_t bytes) {
 }
 // 1 KB of weights global -> LDS, asynchronously: lane l's 16 bytes land at `to` + 16 l. Past the caches or not (buffer_ops.h) is a bit of the
 // instruction, so there are two of it and a branch that the compiler does not see (the step stays one basic block).
+// A vector-memory instruction may read a scalar register five wait states after a vector instruction wrote it - which reloads of
+// spilled ones do - and the compiler keeps that distance for its own instructions only: five stand in front of each load here.
 __device__ __forceinline__ void m_copy_weights(const int8_t* base, uint32_t lane_off, uint32_t at, uint32_t to, int past) {
   const v4i rsrc = m_rsrc(base, 0xffffffffu);
   uint32_t keep;  // (the compiler takes m0 for its own)
   asm volatile(
       "s_mov_b32 %[keep], m0\n\t"
       "s_mov_b32 m0, %[to]\n\t"
+      "s_nop 0\n\t"
       "s_cmp_eq_u32 %[past], 0\n\t"
       "s_cbranch_scc1 1f\n\t"
       "buffer_load_dwordx4 %[lo], %[r], %[at] offen nt lds\n\t"
@@ -154,9 +157,10 @@ __device__ __forceinline__ void m_copy_weights(const int8_t* base, uint32_t lane
 }
 
 // Sixteen bytes of results a lane, past the caches or not, likewise. (The wait states keep a vector instruction behind it from
-// overwriting the results before the store has read them.)
+// overwriting the results before the store has read them; those in front are the distance that m_copy_weights keeps.)
 __device__ __forceinline__ void m_store(const v4i& v, const v4i& rsrc, uint32_t at, int past) {
   asm volatile(
+      "s_nop 2\n\t"
       "s_cmp_eq_u32 %[past], 0\n\t"
       "s_cbranch_scc1 1f\n\t"
       "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen nt\n\t"

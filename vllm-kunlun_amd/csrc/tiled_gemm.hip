@@ -927,11 +927,13 @@ __global__ __launch_bounds__(WM * WN * kWave, WGS) void tiled_gemm_kernel(const 
   auto pace = [&](int it, int chunk) {
     if constexpr (!PACE) return;
     const uint32_t prog = (static_cast<uint32_t>(it + 1) << 16) | static_cast<uint32_t>(chunk);
-    // one lane stores (64 lanes writing one address through to memory cost a third of the kernel's time)
+    // one lane stores (64 lanes writing one address through to memory cost a third of the kernel's time); the wait states are
+    // those between a vector instruction that writes the address's registers and a store that reads them
     uint64_t saved_exec;
     asm volatile(
         "s_mov_b64 %[ex], exec\n\t"
         "s_mov_b64 exec, 1\n\t"
+        "s_nop 2\n\t"
         "global_store_dword %[zero], %[val], %[slot] \n\t"
         "s_mov_b64 exec, %[ex]\n\t"
         : [ex] "=&s"(saved_exec)
