@@ -312,6 +312,14 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   constexpr uint32_t kRange = 0xfffffff0u;  // an offset of kRange lies outside every descriptor here: nothing is read
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.a), 0, kRange, 0x00020000);
   const uint32_t lane16 = lane * 16u;
+  // What is computed from this is computed where it is used. fp8 without SiLU-mul, whose late results take twice the registers: addresses
+  // held through the tile loop were spilled, and each reload waited for all copies in flight (Qwen3 dims, down, 512 rows per expert
+  // 185 -> 167 us, DeepSeek-V3 dims, 170 931 -> 907, 512 2408 -> 2339). The other instances have the registers, and hold them.
+  constexpr bool kTight = F8 && !SWIGLU && MF == 6;
+  auto here = [](uint32_t v) __attribute__((always_inline)) -> uint32_t {
+    if constexpr (kTight) asm volatile("" : "+v"(v));
+    return v;
+  };
   // channel of fragment f of the waves in column c (0: past the last channel, never stored)
   auto col_of = [&](const MTile& t, int c, int f, bool& ok) -> int {
     const int fh = SWIGLU ? f % NFH : f;
@@ -341,8 +349,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   };
   uint32_t a_off[kNA];
   // copy i of this wave fills rows 8 (kNA wave + i) + lane / 8 of a chunk buffer
-  const int dma_row = wave * 8 * kNA + (lane >> 3);
-  const uint32_t a_col = static_cast<uint32_t>((lane & 7) ^ ((lane >> 3) & 7)) * 16u;
+  auto dma_row = [&]() __attribute__((always_inline)) { return wave * 8 * kNA + static_cast<int>(here(lane16) >> 7); };
   auto dma_a = [&](int chunk, uint32_t buf_at, int i) __attribute__((always_inline)) {
     buffer_load16_to_lds(a_rsrc, (lds_ptr_t)(&ring_a[0][0] + buf_at + (wave * kNA + i) * 1024), a_off[i],
                          static_cast<uint32_t>(chunk) * kMChunk);
@@ -392,13 +399,15 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
 
   // ---- first tile ----
   auto row_offset = [&](const MTile& t, int i, int fetched) -> uint32_t {  // rows past the tile's end are not read
-    const int r = t.row0 + dma_row + 8 * i;
+    const int r = t.row0 + dma_row() + 8 * i;
+    const uint32_t now = here(lane16);
+    const uint32_t a_col = (now ^ (now >> 3)) & 0x70u;  // vector c of row r at position c ^ r % 8
     return r < t.end ? src_row(t, r, fetched) * static_cast<uint32_t>(p.lda) + a_col : kRange;  // < 4 GiB: host-checked
   };
   Weights w_cur = weights_of(cur);
 #pragma unroll
   for (int i = 0; i < kNA; ++i)
-    a_off[i] = row_offset(cur, i, (p.row_src && cur.e < p.E) ? p.row_src[clamp_row(cur, cur.row0 + dma_row + 8 * i)] : 0);
+    a_off[i] = row_offset(cur, i, (p.row_src && cur.e < p.E) ? p.row_src[clamp_row(cur, cur.row0 + dma_row() + 8 * i)] : 0);
   {
     const int rr = clamp_row(cur, cur.row0 + 64 * (wave & 3) + lane);
     const int fetched = (p.row_src && cur.e < p.E) ? p.row_src[rr] : 0;
@@ -416,13 +425,13 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   };
   auto dma_tile_scales = [&](const MTile& t, int parity, int fetched) __attribute__((always_inline)) {
     if constexpr (F8) {
-      asc_off = src_row(t, clamp_row(t, t.row0 + 64 * (wave & 3) + lane), fetched) * static_cast<uint32_t>(kblocks) * 4u;
+      asc_off = src_row(t, clamp_row(t, t.row0 + 64 * (wave & 3) + static_cast<int>(here(lane16) >> 4)), fetched) * static_cast<uint32_t>(kblocks) * 4u;
       const int b = wave - 4;  // waves 4 and 5: a block of 128 channels each
       if (b == 0 || b == 1) {
         const int row = SWIGLU ? t.nb + b * (n_half / 128) : min(2 * t.nb + b, p.n / 128 - 1);
         const float* ws = t.e >= p.E ? p.w_max_tail : p.w_max + static_cast<size_t>(t.e) * (p.n / 128) * kblocks;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(ws), (lds_ptr_t)&wsc_lds[parity][b * kMacroBlocks], 4,
-                                                 static_cast<uint32_t>(row * kblocks + min(lane, kblocks - 1)) * 4u, 0, 0, 0);
+                                                 static_cast<uint32_t>(row * kblocks + min(static_cast<int>(here(lane16) >> 4), kblocks - 1)) * 4u, 0, 0, 0);
       }
     }
   };
@@ -612,9 +621,10 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
       __builtin_amdgcn_sched_barrier(0);
       const uint32_t a_to = buf == 0 ? (kChunkBufs - 1) * kABytes : buf - kABytes;
       const uint32_t w_to = slot >= 2 * kMWeightStep ? slot - 2 * kMWeightStep : slot + 4 * kMWeightStep;
-      const uint32_t a_lo = fa[0] + buf, a_hi = fa[1] + buf, w_at = fw + slot;
+      const uint32_t a_lo = fa[0] + buf, a_hi = kTight ? a_lo ^ 64u : fa[1] + buf;  // (bit 2 of the vector's position)
+      const uint32_t w_at = kTight ? lds_addr(&ring_w[0][0]) + wn * 4096u + slot + here(lane16) : fw + slot;
       const int base = min(c & ~3, kblocks - 4);
-      const uint32_t sa_at = lds_addr(&asc_lds[0][0]) + static_cast<uint32_t>(group * 16 * kTM + (wm * 16 + li) * 16 + 4 * (c - base));
+      const uint32_t sa_at = lds_addr(&asc_lds[0][0]) + static_cast<uint32_t>(group * 16 * kTM + (wm * 16 + static_cast<int>(here(lane16) >> 4 & 15)) * 16 + 4 * (c - base));
       const uint32_t sw_at = lds_addr(&wsc_lds[parity][SWIGLU ? 0 : (wn >> 1) * kMacroBlocks]) + 4u * c;
       float sw[2], sa_c[2], sc[2][2];
       v4i lo[2], hi[2], wl[kMFrags], wh[kMFrags];
@@ -706,15 +716,15 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
     }
     auto fetch_next = [&]() __attribute__((always_inline)) {  // the gather entries of the next tile's rows
       if (p.row_src && 64 * wave < kTM && wave < 4) {
-        const int rr = clamp_row(look, look.row0 + 64 * wave + lane);
+        const int rr = clamp_row(look, look.row0 + 64 * wave + static_cast<int>(here(lane16) >> 4));
         __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(p.row_src), (lds_ptr_t)&idx_lds[64 * wave], 4,
                                                  static_cast<uint32_t>(look.e < p.E ? rr : 0) * 4u, 0, 0, 0);
       }
     };
     auto next_rows = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < kNA; ++i) a_off[i] = row_offset(look, i, m_read_i32(lds_addr(&idx_lds[dma_row + 8 * i])));
-      return m_read_i32(lds_addr(&idx_lds[min(64 * (wave & 3) + lane, kTM - 1)]));
+      for (int i = 0; i < kNA; ++i) a_off[i] = row_offset(look, i, m_read_i32(lds_addr(&idx_lds[dma_row() + 8 * i])));
+      return m_read_i32(lds_addr(&idx_lds[min(64 * (wave & 3) + static_cast<int>(here(lane16) >> 4), kTM - 1)]));
     };
     const Weights w_nxt = weights_of(look);
     if constexpr (F8) {
