@@ -10,8 +10,8 @@ FEW = [0, 1, 2, 0, 3] * 12  # with these an expert holds few rows on average: th
 ROWS = [1, 15, 16, 17, 0, 191, 192, 193, 33, 384, 385, 0, 127, 128, 129, 800, 3100]  # up to 17 tiles of an expert
 
 
-def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, bound=0, seed=0, variant=23):
-    """Outputs of the variants 6 and 23 (or another) for the same operands. pad: values between the rows of a and y; tail: rows of an expert
+def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, bound=0, seed=0, variant=23, trace=False):
+    """Outputs of the variants 6 and 23 (or another) for the same operands; trace: and the latter's kernel. pad: values between the rows of a and y; tail: rows of an expert
     outside w (int8); bound: rows the caller allows for beyond the last expert's."""
     from vllm_kunlun_amd import _lib as L
     g = torch.Generator(device="cuda").manual_seed(seed)
@@ -48,10 +48,12 @@ def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, b
         y = torch.full((rows + tail, n_out + pad), float("nan"), dtype=dtype, device="cuda")
         q.y, q.variant, q.act_dtype = y.data_ptr(), v, L.act_dtype(y, "test")
         launch = L.lib.kmoe_grouped_gemm_i8 if i8 else (L.lib.kmoe_grouped_gemm_fp8_block if f8 else L.lib.kmoe_grouped_gemm_bf16)
+        L.lib.kmoe_trace_kernels(1)
         L.check(launch(q, L.stream()))
+        L.lib.kmoe_trace_kernels(0)
         out.append(y)
     torch.cuda.synchronize()
-    return out, n_out
+    return (out, n_out, L.lib.kmoe_traced_kernels().decode()) if trace else (out, n_out)
 
 
 def _same(out, n_out):
@@ -107,11 +109,19 @@ def test_what_the_launch_does_not_take(k, div, experts):
         _launch("int8", [5] * experts, 32, k, 0, torch.bfloat16, div=div)
 
 
-@pytest.mark.parametrize("n,k,rows", [(7168, 768, 700), (7168, 768, 1400), (7168, 640, 1400), (12288, 768, 3500), (7168, 4096, 1900), (4096, 4096, 4000), (65536, 128, 66)])
+@pytest.mark.parametrize("n,k,rows,tile", [
+    (7168, 768, 700, "64x256 tile, 4 waves"), (7168, 768, 1400, "192x256 tile, 8 waves"), (7168, 640, 1400, "192x256 tile, 8 waves"),
+    (12288, 768, 3500, "192x256 tile, both"), (7168, 4096, 1900, "128x256 tile, 4 waves"), (4096, 4096, 4000, "128x256 tile, 4 waves"),
+    # channel blocks for every CU: by the rows alone
+    (65536, 128, 64, "64x256 tile, 4 waves"), (65536, 128, 65, "96x256 tile, 4 waves"), (65536, 128, 96, "96x256 tile, 4 waves"),
+    (65536, 128, 97, "128x256 tile, 8 waves"), (65536, 128, 129, "192x256 tile, 8 waves"), (65536, 128, 193, "128x256 tile, 4 waves"),
+    (65536, 128, 257, "192x256 tile, 8 waves"), (65536, 4096, 300, "192x256 tile, 8 waves")])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_one_matrix_alone(n, k, rows, dtype):
-    """The tile taken by rounds: 64 rows, 192 (wide, wide, macro), 128, and a few rows of many channels."""
-    _same(*_launch("int8", [rows], n, k, 0, dtype, gather=False, variant=0))
+def test_one_matrix_alone(n, k, rows, tile, dtype):
+    """The tile for one matrix: by rounds of workgroups, by the rows where one row of tiles fills every CU, and the macro tile over short K."""
+    out, n_out, ran = _launch("int8", [rows], n, k, 0, dtype, gather=False, variant=0, trace=True)
+    _same(out, n_out)
+    assert tile in ran, ran
 
 
 @pytest.mark.parametrize("n,k,rows,experts", [(7168, 768, 300, 4), (1536, 768, 150, 32), (1536, 768, 300, 16), (512, 4096, 150, 128), (512, 4096, 400, 128)])

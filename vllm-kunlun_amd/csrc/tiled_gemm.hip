@@ -1542,7 +1542,7 @@ bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_c
     return (many && weights > (256ll << 20) && (swiglu || p.k < 4096)) || (some && swiglu && mean > 100.0f);
   }
   if (swiglu) return (many && p.k >= 2048) || (some && mean > 72.0f);
-  if (p.k >= 4096) return some && mean > 88.0f && mean <= 320.0f;  // (never one matrix)
+  if (p.k >= 4096) return p.E > 1 && some && mean > 88.0f && mean <= 320.0f;  // (never one matrix: [65536 x 4096] 300 rows 86.6 / 93.3)
   return (many && weights > (256ll << 20)) || (some && mean > 88.0f) || (p.E > 1 && mean > 128.0f && 4 * items <= 3ll * n_cu && items_of(64) > 2ll * n_cu);
 }
 
@@ -1551,15 +1551,30 @@ bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_c
 // x 256 ones, one per CU, 120. GEMM alone, us, 64 / 128 / 192 rows (wide tiles): [4096 x 7168] 1000 rows 37 / 57 / 57, 2000 60 / 63 / 59, 2500 83 /
 // 85 / 66, 4096 115 / 104 / 124; [7168 x 2048] 700 rows 19.9 / 24.6 / 22.9, 1400 30.1 / 34.7 / 26.1, 2000 38.8 / 37.5 / 44.2, 3000 56.9 / 55.4 / 48.6;
 // [12288 x 5120] 700 59.5 / 62.5 / 46.8, 1200 83 / 76 / 91; [4096 x 640] 2500 17.7 / 20.6 / 15.7, 3500 21.1 / 22.3 / 25.1.
-// The 192 rows as the macro tile from two rounds of a short K on, us, wide / macro: [24576 x 1536] 4096 rows 175 / 167, [7168 x 2048] 1400 26.1 / 27.8,
+// The 192 rows as the macro tile from three rounds of a short K on, us, wide / macro: [24576 x 1536] 4096 rows 175 / 167, [7168 x 2048] 1400 26.1 / 27.8,
 // 6000 102 / 97; [8192 x 8192] 3000 161 / 168.
-int one_matrix_rows(int rows, int n, int k, int n_cu) {
+// A matrix whose channel blocks alone occupy every CU (65536 channels and more) is bound by its weights, which each tile down the rows reads again: the
+// tile that holds the rows, wide beyond 96, and two of 128 four-wave rows ahead of two of 192 wide ones. us, 64 / 96 / 128 / 128 wide / 192 wide rows:
+// [131072 x 7168] 72 rows 208 / 154 / 184 / 172 / 173, 128 rows 214 / 263 / 194 / 182 / 185, 160 272 / - / 241 / 234 / 191, 230 318 / - / 255 / 251 / 274,
+// 300 383 / - / 328 / 327 / 295, 400 499 / - / 396 / 408 / 398; [129280 x 4096] 96 rows 112 / 93 / 108 / 102 / 103, 256 181 / - / 145 / 149 / 164,
+// 400 272 / - / 233 / 245 / 236; [152064 x 5120] 65 rows 183 / 148 / 178 / 162 / 166, 280 324 / - / 265 / 280 / 265.
+struct OneTile {
+  int rows;   // 0: the rules for experts
+  bool wide;  // eight waves side by side
+};
+OneTile one_matrix_tile(int rows, int n, int k, int n_cu) {
+  if (ceil_div(n, 256) >= n_cu) {
+    if (rows <= 64) return {64, false};
+    if (rows <= 96) return {96, false};
+    if (rows <= 128) return {128, true};
+    return rows > 192 && rows <= 256 ? OneTile{128, false} : OneTile{192, true};
+  }
   auto cost = [&](int tile, int pair, int single) {
     const long long items = static_cast<long long>(ceil_div(rows, tile)) * ceil_div(n, 256), rest = items % (2 * n_cu);
     return items / (2 * n_cu) * pair + (rest == 0 ? 0 : rest <= n_cu ? single : pair);
   };
   const long long c64 = cost(64, 100, 65), c128 = k < 4096 ? cost(128, 200, 120) : cost(128, 180, 110), c192 = cost(192, 240, 120);
-  return c64 <= c128 && c64 <= c192 ? 64 : c128 < c192 ? 128 : 192;
+  return c64 <= c128 && c64 <= c192 ? OneTile{64, false} : c128 < c192 ? OneTile{128, false} : OneTile{192, true};
 }
 
 // One 8-wave tile of 16 MF rows per workgroup with the eight waves side by side along the channels (32 channels
@@ -1633,9 +1648,8 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   const int live = expected_rows(a->rows, a->rows_hint);  // (chooses the tile shape; grids and bounds keep a->rows)
   const int n_exp = a->E + (a->w_tail ? 1 : 0);
   const int avg_rows = ceil_div(live + (a->w_tail ? a->tail_rows : 0), n_exp);
-  // (rows of the tile for one matrix alone, 0: the rules for experts)
-  const int one = a->variant == 0 && a->E == 1 && !swiglu && !a->w_tail ? one_matrix_rows(live, a->n, a->k, n_cu) : 0;
-  const bool shorter = one ? one == 64 : short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu);
+  const OneTile one = a->variant == 0 && a->E == 1 && !swiglu && !a->w_tail ? one_matrix_tile(live, a->n, a->k, n_cu) : OneTile{0, false};
+  const bool shorter = one.rows ? one.rows == 64 : short_tiles(a->variant, live, a->E, a->n, swiglu, n_cu);
   // 128-row 4-wave tiles whose sibling m-tiles are paced against each other (see g_board): variant 12, and the
   // second launch of the device-decided pair (variant 17). They were the default where experts have several m-tiles
   // and the launch's weights are far more than the 256 MB memory-side cache holds (a sibling that falls behind
@@ -1648,7 +1662,7 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   // quarter of the 128-row tile's MFMAs (all padding there) is saved (Qwen3 shape, layer: 768 tokens 0.169 ->
   // 0.158 ms, 1024 tokens 0.191 -> 0.165 ms; at 80 rows per expert too many experts need a second tile: -4 % on
   // the Qwen3 shape, +1 % on the DeepSeek-V3 one; DeepSeek-V3 shape at 64 rows per expert: -1.6 %).
-  const bool mid = a->variant == 13 || (a->variant == 0 && !shorter && avg_rows <= 72);
+  const bool mid = a->variant == 13 || (a->variant == 0 && !shorter && (avg_rows <= 72 || one.rows == 96));
   // Wide tiles: 128, 192 or 256 rows x 256 channels on EIGHT waves side by side along the channels (32 channels
   // each, all the tile's rows), one workgroup per CU. No two waves of a workgroup ask for the same weight bytes,
   // seven MFMA steps of them are on their way per wave (112 KB of distinct weight bytes in flight per CU, where two
@@ -1710,7 +1724,7 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
   const float avg_routed = static_cast<float>(ceil_div(live, a->E));
   const float reach = avg_routed + 3.0f * sqrtf(avg_routed);
   const bool big = weight_bytes > (1ll << 30);
-  if (a->variant == 0 && (one == 0 || one == 192) && macro_pays(K, p, live, swiglu, n_cu) && macro_params(p, live, &macro)) {
+  if (a->variant == 0 && (one.rows == 0 || one.rows == 192) && macro_pays(K, p, live, swiglu, n_cu) && macro_params(p, live, &macro)) {
     return macro_tile(macro, 0, swiglu, a->act_dtype == KMOE_DT_F16, a->rows, s, n_cu, what);
   }
   int wide = 0;  // row fragments of the wide tile (8: 128 rows, 12: 192, 16: 256), 0: none
@@ -1721,9 +1735,11 @@ int tiled_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s) {
     case 8: case 16: case 22: wide = 16; break;
     default: break;
   }
-  if (a->variant == 0 && !shorter && one != 128 && (big || one || avg_rows > 72)) {
+  if (one.rows) {
+    wide = one.wide ? one.rows / 16 : 0;
+  } else if (a->variant == 0 && !shorter && (big || avg_rows > 72)) {
     // (small weights keep the 96-row tiles up to 72 rows per expert: Qwen3 dims at 1024 tokens 0.164 against 0.169)
-    wide = reach <= 128.0f && !one ? 8 : 12;
+    wide = reach <= 128.0f ? 8 : 12;
   } else if (a->variant == 17) {
     wide = reach <= 128.0f ? 8 : (reach <= 192.0f ? 12 : 16);
     pair = true;
