@@ -128,3 +128,22 @@ def test_one_matrix_alone(n, k, rows, tile, dtype):
 def test_less_than_a_round(n, k, rows, experts):
     """Few tiles for the CUs, and a long K."""
     _same(*_launch("int8", [rows] * experts, n, k, 0, torch.bfloat16, variant=0))
+
+
+MACRO, LOW = "192x256 tile, both", "128x256 tile, both"
+
+
+def _runs(kind, E, n, k, act, rows, tile):
+    """The launch of E experts of `rows` rows each gives the 128-row tile's bits; `tile`: part of its kernel's name, or None for any but the macro tile."""
+    out, n_out, ran = _launch(kind, [rows] * E, n, k, act, torch.bfloat16, gather=False, variant=0, trace=True)
+    _same(out, n_out)
+    assert (tile in ran) if tile else ("both operands" not in ran), ran
+
+
+@pytest.mark.parametrize("E,n,k,act,rows,tile", [
+    (64, 1024, 1024, 1, 111, None), (64, 1024, 1024, 1, 384, None), (64, 1024, 1024, 1, 385, MACRO), (96, 2048, 1024, 1, 100, None), (96, 2048, 1024, 1, 111, MACRO),
+    (64, 2304, 2048, 1, 105, None), (64, 2304, 2048, 1, 123, None), (64, 2304, 2048, 1, 124, MACRO), (64, 2304, 2048, 1, 176, None), (32, 2304, 2048, 1, 900, None),
+    (96, 3072, 2048, 0, 105, LOW), (96, 3072, 2048, 0, 111, None), (96, 3072, 2048, 0, 300, None), (96, 3072, 2048, 0, 301, MACRO), (96, 2816, 768, 0, 100, None)])
+def test_choice_fp8(E, n, k, act, rows, tile):
+    """Experts an XCD's L2 holds and larger ones, in fewer rounds and more, one tile and several; a launch whose weights the memory-side cache holds."""
+    _runs("fp8", E, n, k, act, rows, tile)

@@ -1517,13 +1517,17 @@ bool macro_params(const TiledParams& p, int live, MacroParams* out) {
 //   bf16, [7168 x 2048], 8 experts, 1000 rows 199 / 232, 32 experts, 300 304 / 297; [4096 x 7168], 16 experts, 300 rows 308 / 281, 600 504 / 526
 //   less than a round of items: int8, 32 experts of [1536 x 2048], 150 rows (192 items here, 576 of 64 rows) 30.7 / 26.6, 16 experts of 300 (192 and 480)
 //   22.7 / 26.9, 4 experts of [4096 x 7168], 300 (128 and 320) 51.7 / 58.7; 4 of [7168 x 2048], 375 on average, uneven (224) 31.1 / 42.6
-// So, by rounds of items of 192 rows over the CUs. gate_up: int8 from four rounds on, two where rows are many; 16-bit, bound by its weights, from two on
-// while one tile holds nearly every expert, a hot one too (few rows) or many rows pay for a round more. down: four rounds and weights beyond the memory-side cache, or two and many rows (16-bit: one of the
-// two); over a long K only while an expert has few tiles. One round that leaves a quarter of the CUs free for an uneven load, where the 64-row
-// tiles, two per CU, need a second. fp8, whose fragments of a chunk are waited for at its start, only where the weights exceed that cache, too; and
-// of experts beyond an XCD's L2 only where one tile, two thirds full, holds most of them, or many do: layer, us, the other tiles / that one,
-// DeepSeek-V3 dims, 119 rows 2757 / 2813, 141 3149 / 2992, 163 3499 / 3361, 172 3820 / 3604, 219 4391 / 4732, 256 5040 / 5513, 384 7041 / 7225; Kimi-K2
-// dims, 125 4060 / 3850, 171 5159 / 4849. (Qwen3 dims, whose experts it holds: 128 rows 219 / 202, 256 335 / 326, 512 587 / 563.)
+// So, by rounds of items of 192 rows over the CUs. gate_up: int8 from four rounds on, two where rows are many; 16-bit, bound by its weights, from two
+// on while one tile holds nearly every expert, a hot one too (few rows) or many rows pay for a round more. down: four rounds and weights beyond the
+// memory-side cache, or two and many rows (16-bit: one of the two); over a long K only while an expert has few tiles. One round that leaves a quarter
+// of the CUs free for an uneven load, where the 64-row tiles, two per CU, need a second. fp8, whose fragments of a chunk are waited for at its start,
+// only where the weights exceed that cache, too; and of experts beyond an XCD's L2 only where one tile, two thirds full, holds most of them, and in
+// down launches where they have two or more: GEMM alone, us, the other tiles / that one, DeepSeek-V3 dims, gate_up, 150 rows 1773 / 1638, 170 2063 /
+// 1738, 200 2190 / 2298, 256 2610 / 2934, 384 3759 / 3572 (uneven 3746 / 3806), 512 4594 / 4691, 1024 9191 / 9667; down, 150 rows 927 / 851, 170 1131
+// / 923, 200 1174 / 1243, 256 1421 / 1454, 300 1669 / 1553, 384 2030 / 1883, 512 2535 / 2399, 1024 4886 / 4750; Kimi-K2 dims, gate_up, 1024 14206 /
+// 15078, down, 512 3808 / 3603. Smaller experts from three rounds on: Qwen3 dims, gate_up, 110 rows (the lower tile) 92 / 95, 128 100 / 90, 200 131 /
+// 152 (uneven 162 / 117), 256 165 / 160, 800 441 / 397; 64 experts of [1024 x 4096], 200 rows (two rounds) 79 / 111 (uneven 83 / 96), 256 96 / 102,
+// 384 131 / 158, 800 (five) 258 / 257.
 bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_cu) {
   const float mean = static_cast<float>(ceil_div(live, p.E));
   const long long weights = static_cast<long long>(p.E) * p.n * p.k;
@@ -1536,10 +1540,9 @@ bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_c
     return some && (p.k >= 4096 || mean > 72.0f) && mean + 2.2f * sqrtf(mean) <= 192.0f;
   }
   if (kind == TKind::F8) {
-    if (static_cast<long long>(p.n) * p.k > (4ll << 20) && !macro_low(mean) && mean <= 800.0f &&
-        (mean < 124.0f || mean + 1.5f * sqrtf(mean) > 192.0f))
-      return false;
-    return (many && weights > (256ll << 20) && (swiglu || p.k < 4096)) || (some && swiglu && mean > 100.0f);
+    const bool beyond_l2 = static_cast<long long>(p.n) * p.k > (4ll << 20), low = macro_low(mean);
+    if (beyond_l2 && !low && (swiglu || mean <= 300.0f) && (mean < 124.0f || mean + 1.5f * sqrtf(mean) > 192.0f)) return false;
+    return (many && weights > (256ll << 20) && (swiglu || p.k < 4096)) || (swiglu && !low && items >= (beyond_l2 ? 2ll : 3ll) * n_cu);
   }
   if (swiglu) return (many && p.k >= 2048) || (some && mean > 72.0f);
   if (p.k >= 4096) return p.E > 1 && some && mean > 88.0f && mean <= 320.0f;  // (never one matrix: [65536 x 4096] 300 rows 86.6 / 93.3)
