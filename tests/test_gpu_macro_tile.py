@@ -147,3 +147,14 @@ def _runs(kind, E, n, k, act, rows, tile):
 def test_choice_fp8(E, n, k, act, rows, tile):
     """Experts an XCD's L2 holds and larger ones, in fewer rounds and more, one tile and several; a launch whose weights the memory-side cache holds."""
     _runs("fp8", E, n, k, act, rows, tile)
+
+
+@pytest.mark.parametrize("E,n,k,act,rows,tile", [
+    (80, 2304, 1024, 0, 18, MACRO), (80, 2304, 1024, 0, 19, None), (80, 2304, 1024, 0, 27, None), (80, 2304, 1024, 0, 28, MACRO),
+    (80, 2304, 1024, 0, 172, MACRO), (80, 2304, 1024, 0, 173, None), (80, 2304, 1024, 0, 280, None), (80, 2304, 1024, 0, 281, MACRO),
+    (128, 2048, 768, 0, 200, MACRO), (64, 2304, 2048, 0, 400, MACRO), (64, 2304, 2048, 0, 401, None), (1, 65536, 2048, 0, 200, None),
+    (1, 131072, 1152, 0, 160, None), (1, 131072, 1152, 0, 161, MACRO),
+    (64, 4096, 1024, 1, 72, None), (64, 4096, 1024, 1, 73, MACRO), (64, 4096, 1024, 1, 163, MACRO), (64, 4096, 1024, 1, 170, None)])
+def test_choice_16_bit(E, n, k, act, rows, tile):
+    """Few rows, one tile, the beginning of a second, a long K, one matrix; gate_up."""
+    _runs("16 bit", E, n, k, act, rows, tile)
