@@ -158,3 +158,12 @@ def test_choice_fp8(E, n, k, act, rows, tile):
 def test_choice_16_bit(E, n, k, act, rows, tile):
     """Few rows, one tile, the beginning of a second, a long K, one matrix; gate_up."""
     _runs("16 bit", E, n, k, act, rows, tile)
+
+
+@pytest.mark.parametrize("E,n,k,act,rows,tile", [
+    (96, 3072, 2048, 1, 60, MACRO), (96, 2560, 2048, 1, 72, None), (96, 2560, 2048, 1, 73, MACRO), (64, 1024, 1024, 1, 193, None), (64, 1024, 1024, 1, 384, None),
+    (64, 2048, 1024, 1, 193, MACRO), (64, 1024, 1024, 1, 385, MACRO), (128, 1024, 4096, 0, 88, None), (128, 1024, 4096, 0, 89, MACRO),
+    (128, 1024, 4096, 0, 176, MACRO), (128, 1024, 4096, 0, 177, None), (16, 2048, 768, 0, 600, None), (16, 2048, 768, 0, 961, MACRO), (96, 2048, 768, 0, 88, None), (96, 2048, 768, 0, 89, MACRO)])
+def test_choice_int8(E, n, k, act, rows, tile):
+    """Four rounds and two, the second tile in few rounds, a long K, down launches in few rounds and more."""
+    _runs("int8", E, n, k, act, rows, tile)

@@ -1517,21 +1517,23 @@ bool macro_params(const TiledParams& p, int live, MacroParams* out) {
 //   bf16, [7168 x 2048], 8 experts, 1000 rows 199 / 232, 32 experts, 300 304 / 297; [4096 x 7168], 16 experts, 300 rows 308 / 281, 600 504 / 526
 //   less than a round of items: int8, 32 experts of [1536 x 2048], 150 rows (192 items here, 576 of 64 rows) 30.7 / 26.6, 16 experts of 300 (192 and 480)
 //   22.7 / 26.9, 4 experts of [4096 x 7168], 300 (128 and 320) 51.7 / 58.7; 4 of [7168 x 2048], 375 on average, uneven (224) 31.1 / 42.6
-// So, by rounds of items of 192 rows over the CUs. gate_up: int8 from four rounds on, two where rows are many; 16-bit, bound by its weights, from two
-// on while one tile holds nearly every expert, a hot one too (few rows) or many rows pay for a round more. down: four rounds and weights beyond the
-// memory-side cache, or two and many rows (16-bit: one of the two, and not where experts beyond an XCD's L2 begin a second tile: GEMM alone, us, the
-// other tiles / that one, DeepSeek-V3 dims, 160 rows 1671 / 1509, 185 1723 / 1724, 200 1771 / 1943, 240 2014 / 2139 (uneven 2065 / 2145), 300 2566 /
-// 2332; 32 of these experts, 176 rows 211 / 229, 200 213 / 273 (uneven 245 / 259), 256 265 / 288, 300 308 / 304; [65536 x 4096] alone, 185 132 / 114,
-// 200 133 / 149, 256 139 / 160, 300 178 / 168; Qwen3 dims, which it holds, 200 129 / 129, uneven 145 / 120; nor one matrix of up to 160 rows, [131072
-// x 2048] 64 rows 96 / 104, 150 105 / 115, 170 123 / 117); over a long K only while an expert has few tiles. One round that leaves a quarter of the
-// CUs free for an uneven load, where the 64-row tiles, two per CU, need a second. fp8, whose fragments of a chunk are waited for at its start, only
-// where the weights exceed that cache, too; and of experts beyond an XCD's L2 only where one tile, two thirds full, holds most of them, and in down
-// launches where they have two or more: GEMM alone, us, the other tiles / that one, DeepSeek-V3 dims, gate_up, 150 rows 1773 / 1638, 170 2063 / 1738,
-// 200 2190 / 2298, 256 2610 / 2934, 384 3759 / 3572 (uneven 3746 / 3806), 512 4594 / 4691, 1024 9191 / 9667; down, 150 rows 927 / 851, 170 1131 /
-// 923, 200 1174 / 1243, 256 1421 / 1454, 300 1669 / 1553, 384 2030 / 1883, 512 2535 / 2399, 1024 4886 / 4750; Kimi-K2 dims, gate_up, 1024 14206 /
-// 15078, down, 512 3808 / 3603. Smaller experts from three rounds on: Qwen3 dims, gate_up, 110 rows (the lower tile) 92 / 95, 128 100 / 90, 200 131 /
-// 152 (uneven 162 / 117), 256 165 / 160, 800 441 / 397; 64 experts of [1024 x 4096], 200 rows (two rounds) 79 / 111 (uneven 83 / 96), 256 96 / 102,
-// 384 131 / 158, 800 (five) 258 / 257.
+// So, by rounds of items of 192 rows over the CUs. gate_up: int8 from four rounds on, two where rows are many (of 193 to 384 rows three, the second
+// tiles being half empty: 64 experts of [1024 x 4096], 200 rows 82 / 85, 300 94 / 95, uneven 96 / 98); 16-bit, bound by its weights, from two on
+// while one tile holds nearly every expert, a hot one too (few rows) or many rows pay for a round more. down: four rounds and weights beyond the
+// memory-side cache, or three and many rows (two: 16 experts of [2048 x 768], 600 rows 30 / 32, 1400 rows, four, 56 / 53; 16-bit: one of the two, and
+// not where experts beyond an XCD's L2 begin a second tile: GEMM alone, us, the other tiles / that one, DeepSeek-V3 dims, 160 rows 1671 / 1509, 185
+// 1723 / 1724, 200 1771 / 1943, 240 2014 / 2139 (uneven 2065 / 2145), 300 2566 / 2332; 32 of these experts, 176 rows 211 / 229, 200 213 / 273 (uneven
+// 245 / 259), 256 265 / 288, 300 308 / 304; [65536 x 4096] alone, 185 132 / 114, 200 133 / 149, 256 139 / 160, 300 178 / 168; Qwen3 dims, which it
+// holds, 200 129 / 129, uneven 145 / 120; nor one matrix of up to 160 rows, [131072 x 2048] 64 rows 96 / 104, 150 105 / 115, 170 123 / 117); over a
+// long K only while an expert has one tile (128 experts of [2048 x 4096], 160 rows 235 / 218, 185 274 / 291, 200 293 / 312, 300 357 / 369). One round
+// that leaves a quarter of the CUs free for an uneven load, where the 64-row tiles, two per CU, need a second. fp8, whose fragments of a chunk are
+// waited for at its start, only where the weights exceed that cache, too; and of experts beyond an XCD's L2 only where one tile, two thirds full,
+// holds most of them, and in down launches where they have two or more: GEMM alone, us, the other tiles / that one, DeepSeek-V3 dims, gate_up, 150
+// rows 1773 / 1638, 170 2063 / 1738, 200 2190 / 2298, 256 2610 / 2934, 384 3759 / 3572 (uneven 3746 / 3806), 512 4594 / 4691, 1024 9191 / 9667; down,
+// 150 rows 927 / 851, 170 1131 / 923, 200 1174 / 1243, 256 1421 / 1454, 300 1669 / 1553, 384 2030 / 1883, 512 2535 / 2399, 1024 4886 / 4750; Kimi-K2
+// dims, gate_up, 1024 14206 / 15078, down, 512 3808 / 3603. Smaller experts from three rounds on: Qwen3 dims, gate_up, 110 rows (the lower tile) 92 /
+// 95, 128 100 / 90, 200 131 / 152 (uneven 162 / 117), 256 165 / 160, 800 441 / 397; 64 experts of [1024 x 4096], 200 rows (two rounds) 79 / 111
+// (uneven 83 / 96), 256 96 / 102, 384 131 / 158, 800 (five) 258 / 257.
 bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_cu) {
   const float mean = static_cast<float>(ceil_div(live, p.E));
   const long long weights = static_cast<long long>(p.E) * p.n * p.k;
@@ -1549,9 +1551,10 @@ bool macro_pays(TKind kind, const TiledParams& p, int live, bool swiglu, int n_c
     if (beyond_l2 && !low && (swiglu || mean <= 300.0f) && (mean < 124.0f || mean + 1.5f * sqrtf(mean) > 192.0f)) return false;
     return (many && weights > (256ll << 20) && (swiglu || p.k < 4096)) || (swiglu && !low && items >= (beyond_l2 ? 2ll : 3ll) * n_cu);
   }
-  if (swiglu) return (many && p.k >= 2048) || (some && mean > 72.0f);
-  if (p.k >= 4096) return p.E > 1 && some && mean > 88.0f && mean <= 320.0f;  // (never one matrix: [65536 x 4096] 300 rows 86.6 / 93.3)
-  return (many && weights > (256ll << 20)) || (some && mean > 88.0f) || (p.E > 1 && mean > 128.0f && 4 * items <= 3ll * n_cu && items_of(64) > 2ll * n_cu);
+  const bool three = items >= 3ll * n_cu;
+  if (swiglu) return (many && p.k >= 2048) || (some && mean > 72.0f && (three || mean <= 192.0f || mean > 384.0f));
+  if (p.k >= 4096) return p.E > 1 && some && mean > 88.0f && mean <= 176.0f;  // (never one matrix: [65536 x 4096] 300 rows 86.6 / 93.3)
+  return (many && weights > (256ll << 20)) || (three && mean > 88.0f) || (p.E > 1 && mean > 128.0f && 4 * items <= 3ll * n_cu && items_of(64) > 2ll * n_cu);
 }
 
 // One int8 matrix alone (a Linear), whose rows are known exactly: the tile's rows by rounds of workgroups. A round of 64 x 256 tiles, two
