@@ -659,9 +659,9 @@ typedef struct kmoe_moe_args {
   float shared_scale;    /* caller epilogue for half activations (models/deepseek_v2.py:286-292: the routed sum stays
                             unscaled and the shared expert's output is multiplied by 1/routed_scaling_factor):
                             out = dt( dt(routed * out_scale) + dt(shared * shared_scale) ); 0 means 1 */
-  int32_t tile_variant;  /* INT8 and FP8_BLOCK, tuning: 0, or the `variant` (int8: 5-22; fp8: 5, 6, 8, 11-14, 17-20) handed to
+  int32_t tile_variant;  /* INT8 and FP8_BLOCK, tuning: 0, or the `variant` (int8: 5-23; fp8: 5, 6, 8, 11-14, 17-20, 23) handed to
                             the two routed GEMMs when the batch runs on the tile kernel (more than 10 rows per
-                            expert); ignored otherwise */
+                            expert; 23 also only where H, I, E and K are what it takes); ignored otherwise */
   int32_t w_scale_layout; /* W4A16: KMOE_S_* of w13_scale and w2_scale                                  */
   /* An expert-parallel share (ops/_kunlun_ops.py:640-696: each rank holds num_local_experts of the experts and
      computes what the pairs routed to them contribute; the sum over ranks is the caller's all-reduce). The routing

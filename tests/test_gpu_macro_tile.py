@@ -167,3 +167,28 @@ def test_choice_16_bit(E, n, k, act, rows, tile):
 def test_choice_int8(E, n, k, act, rows, tile):
     """Four rounds and two, the second tile in few rounds, a long K, down launches in few rounds and more."""
     _runs("int8", E, n, k, act, rows, tile)
+
+
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+@pytest.mark.parametrize("I,K,E,takes", [(768, 4, 16, True), (768, 6, 16, True), (640, 4, 16, False), (768, 5, 16, False), (768, 4, 416, False)])
+def test_layer_asked_for_the_tile(fmt, I, K, E, takes):
+    """tile_variant = 23 reaches both routed GEMMs where their shapes are what the tile takes, and is ignored otherwise."""
+    from vllm_kunlun_amd import _lib as L
+    from vllm_kunlun_amd import synth
+    from vllm_kunlun_amd._plan import make_moe_plan
+    shape = synth.scaled(synth.SHAPES["qwen3-decode"], M=300 * E // 16, H=1024, E=E, K=K, I=I)
+    sl = (synth.make_w8a8_layer if fmt == "int8" else synth.make_fp8_layer)(shape, "cuda", seed=5)
+    lay, outs = sl.layer, []
+    for variant in (6 if fmt == "int8" else 19, 23):
+        out = torch.empty_like(sl.x)
+        plan = make_moe_plan(L.KMOE_FMT_INT8 if fmt == "int8" else L.KMOE_FMT_FP8_BLOCK, sl.x, sl.logits, out, shape.K, lay.w13_weight, lay.w2_weight,
+                             lay.w13_weight_scale, lay.w2_weight_scale, shape.scoring, True, shape.n_group, shape.topk_group, 1.0, sl.bias, None, 1.0,
+                             tile_variant=variant)
+        L.lib.kmoe_trace_kernels(1)
+        plan()
+        L.lib.kmoe_trace_kernels(0)
+        outs.append(out)
+    torch.cuda.synchronize()
+    ran = L.lib.kmoe_traced_kernels().decode()
+    assert ran.count("both operands") == (2 if takes else 0), ran
+    assert torch.equal(*outs)

@@ -9,6 +9,7 @@
 #include "asked_once.h"
 #include "few_rows.h"
 #include "kmoe_common.h"
+#include "macro_tile.h"
 
 namespace kmoe {
 
@@ -777,12 +778,14 @@ int moe_forward_impl(const kmoe_moe_args* a, void* workspace, size_t workspace_b
   // and its gap less); wider rows would not fit the workgroup's LDS copy next to three resident workgroups per CU.
   routed.quant_in_gemm = stream_mode && I <= kStreamQuantMaxK && quant_in_gemm_allowed();
   routed.x_count = M;
+  uint32_t magic;
+  const bool macro = a->tile_variant == 23 && macro_tile_takes(H, E, fold) && macro_tile_takes(I, E, fold) && macro_tile_divides(K, &magic);
   if (a->format == KMOE_FMT_INT8 && !stream_mode && a->w_layout == KMOE_W_TILED && a->tile_variant >= 5 &&
-      a->tile_variant <= 22 && (local_pairs(a) + E - 1) / E > 10 && H >= 128 && I >= 128)
+      (a->tile_variant <= 22 || macro) && (local_pairs(a) + E - 1) / E > 10 && H >= 128 && I >= 128)
     routed.variant = a->tile_variant;
   const int tv = a->tile_variant;
   if (a->format == KMOE_FMT_FP8_BLOCK && a->w_layout == KMOE_W_TILED && (local_pairs(a) + E - 1) / E > 10 &&
-      (tv == 5 || tv == 6 || tv == 8 || (tv >= 11 && tv <= 14) || (tv >= 17 && tv <= 20)))
+      (tv == 5 || tv == 6 || tv == 8 || (tv >= 11 && tv <= 14) || (tv >= 17 && tv <= 20) || macro))
     routed.variant = tv;
   if (fold) {
     routed.w13_tail = a->ws13;

@@ -31,6 +31,11 @@ constexpr int kMacroTables = 3296, kMacroBlocks = 64;
 inline bool macro_tile_takes(int kbytes, int E, bool tail) {
   return kbytes % 128 == 0 && kbytes >= 768 && 4 * (2 * E + 2 + (tail ? 1 : 0)) <= kMacroTables;
 }
+// Gather entries it divides by one multiplication: entry / div = high half of entry * magic, for every entry where the excess is at most 2.
+inline bool macro_tile_divides(int div, uint32_t* magic) {
+  *magic = div > 1 ? static_cast<uint32_t>(((1ull << 32) + div - 1) / div) : 0;
+  return div <= 1 || static_cast<uint64_t>(*magic) * div - (1ull << 32) <= 2;
+}
 // kind 0: int8, 1: 16-bit, 2: fp8 block-scaled (a_max: [a_rows, k/128] scales, w_max: [E, n/128, k/128]; K of up to kMacroBlocks blocks;
 // with SiLU-mul gate and up in whole blocks: n % 256 == 0). Arguments already checked as for the tile kernel.
 int macro_tile(const MacroParams& p, int kind, bool swiglu, bool f16, int rows, hipStream_t s, int n_cu, const char* what);

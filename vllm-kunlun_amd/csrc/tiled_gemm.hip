@@ -1487,10 +1487,7 @@ bool macro_low(float mean) { return mean + 1.7f * sqrtf(mean) <= 128.0f; }
 // The launch as macro_tile.hip takes it; false where it does not.
 bool macro_params(const TiledParams& p, int live, MacroParams* out) {
   uint32_t magic = 0;
-  if (p.row_src && p.src_div > 1) {  // entry / src_div = high half of entry * magic, for every entry where the excess is at most 2
-    magic = static_cast<uint32_t>(((1ull << 32) + p.src_div - 1) / p.src_div);
-    if (static_cast<uint64_t>(magic) * p.src_div - (1ull << 32) > 2) return false;
-  }
+  if (p.row_src && !macro_tile_divides(p.src_div, &magic)) return false;
   if (!macro_tile_takes(p.k, p.E, p.w_tail != nullptr) || p.acc_out || p.bias) return false;
   const bool past = p.E > 1, big = static_cast<long long>(p.E) * p.n * p.k > (256ll << 20);
   const float mean = static_cast<float>(ceil_div(live, p.E));
