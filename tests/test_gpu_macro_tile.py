@@ -10,9 +10,9 @@ FEW = [0, 1, 2, 0, 3] * 12  # with these an expert holds few rows on average: th
 ROWS = [1, 15, 16, 17, 0, 191, 192, 193, 33, 384, 385, 0, 127, 128, 129, 800, 3100]  # up to 17 tiles of an expert
 
 
-def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, bound=0, seed=0, variant=23, trace=False):
+def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, bound=0, seed=0, variant=23, trace=False, strange=False):
     """Outputs of the variants 6 and 23 (or another) for the same operands; trace: and the latter's kernel. pad: values between the rows of a and y; tail: rows of an expert
-    outside w (int8); bound: rows the caller allows for beyond the last expert's."""
+    outside w (int8); bound: rows the caller allows for beyond the last expert's; strange: infinities and NaN in some rows of a."""
     from vllm_kunlun_amd import _lib as L
     g = torch.Generator(device="cuda").manual_seed(seed)
     E, rows, n_out = len(counts), sum(counts), n // 2 if act else n
@@ -30,6 +30,11 @@ def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, b
              else torch.randn(a_rows, k + pad, generator=g, device="cuda").to(dtype))
         w = (torch.randint(-127, 128, (E + 1, n, k), generator=g, device="cuda", dtype=torch.int8) if i8
              else torch.randn(E + 1, n, k, generator=g, device="cuda").mul_(0.05).to(dtype))
+    if strange and f8:
+        a[5:200:40].view(torch.int8)[:, 3] = 0x7f  # NaN
+        a_max[7:200:40, 1] = float("inf")
+    elif strange:
+        a[5:200:40, 3], a[7:200:40, 700] = float("nan"), float("inf")
     tiled = torch.empty_like(w)
     L.check(L.lib.kmoe_tile_weights_i8(w.data_ptr(), tiled.data_ptr(), E + 1, n, k * w.element_size(), L.stream()))
     q = L.GemmI8Args() if i8 else (L.GemmFp8Args() if f8 else L.GemmBf16Args())
@@ -100,13 +105,63 @@ def test_more_items_than_are_resolved_at_once():
     _same(*_launch("int8", [1, 192, 193, 0, 40] * 28, 16384, 768, 0, torch.bfloat16))
 
 
-@pytest.mark.parametrize("k,div,experts", [(640, 1, 3), (832, 1, 3), (768, 5, 3), (768, 1, 500)])
-def test_what_the_launch_does_not_take(k, div, experts):
+@pytest.mark.parametrize("kind,k,div,experts", [("int8", 640, 1, 3), ("int8", 832, 1, 3), ("int8", 768, 5, 3), ("int8", 768, 1, 500), ("16 bit", 352, 1, 3), ("16 bit", 416, 1, 3),
+                                                ("16 bit", 384, 5, 3), ("16 bit", 384, 1, 500), ("fp8", 640, 1, 3), ("fp8", 768, 5, 3), ("fp8", 768, 1, 500)])
+def test_what_the_launch_does_not_take(kind, k, div, experts):
     """Too short a K, no whole chunks, a divisor whose quotients one multiplication does not give, too many experts for its LDS:
-    refused when asked for by name, and served by another kernel otherwise."""
+    refused when asked for by name."""
+    with pytest.raises(NotImplementedError, match="variant 23 needs"):
+        _launch(kind, [5] * experts, 128, k, 0, torch.bfloat16, div=div)
+
+
+@pytest.mark.parametrize("kind,E,n,k,act,rows,div,tile", [
+    ("int8", 96, 2560, 2048, 1, 100, 6, True), ("int8", 96, 2560, 2048, 1, 100, 5, False), ("int8", 96, 2560, 1984, 1, 100, 1, False),
+    ("int8", 411, 1024, 2048, 1, 20, 1, True), ("int8", 412, 1024, 2048, 1, 20, 1, False),
+    ("16 bit", 96, 3072, 1024, 0, 100, 6, True), ("16 bit", 96, 3072, 1024, 0, 100, 5, False), ("16 bit", 96, 3072, 1056, 0, 100, 1, False), ("16 bit", 412, 1024, 512, 0, 15, 1, False),
+    ("fp8", 96, 3072, 2048, 1, 150, 6, True), ("fp8", 96, 3072, 2048, 1, 150, 5, False), ("fp8", 412, 1024, 2048, 1, 20, 1, False)])
+def test_served_by_another_kernel(kind, E, n, k, act, rows, div, tile):
+    """Launches that the choice would give to the tile and whose form it does not take, beside their neighbours that it does."""
+    out, n_out, ran = _launch(kind, [rows] * E, n, k, act, torch.bfloat16, div=div, variant=0, trace=True)
+    _same(out, n_out)
+    assert ("both operands" in ran) == tile, ran
+
+
+def test_accumulators_are_served_by_another_kernel():
+    """int32 accumulators (asymmetric activations) of a matrix whose plain product takes the tile."""
     from vllm_kunlun_amd import _lib as L
-    with pytest.raises(NotImplementedError):
-        _launch("int8", [5] * experts, 32, k, 0, torch.bfloat16, div=div)
+    from vllm_kunlun_amd.ops import _custom_ops  # noqa: F401
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.randint(-127, 128, (3500, 768), generator=g, device="cuda", dtype=torch.int8)
+    w = torch.randint(-127, 128, (12288, 768), generator=g, device="cuda", dtype=torch.int8)
+    one = torch.ones(1, 1, device="cuda")
+    from vllm_kunlun_amd._plan import tile_int8_weights_
+    want = a.float() @ w.float().t()  # (sums below 2^24: exact)
+    tile_int8_weights_(w)
+    L.lib.kmoe_trace_kernels(1)
+    got = torch.ops._C.cutlass_scaled_mm_azp(a, w.t(), one, one, torch.bfloat16, torch.zeros(1, 12288, dtype=torch.int32, device="cuda"))
+    L.lib.kmoe_trace_kernels(0)
+    ran = L.lib.kmoe_traced_kernels().decode()
+    assert "tiled_gemm_kernel" in ran and "both operands" not in ran, ran
+    assert torch.equal(got, want.bfloat16())
+
+
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("few", [False, True])
+def test_longest_k_fp8(act, few):
+    """64 blocks of K: the most whose weight scales its LDS holds."""
+    _same(*_launch("fp8", [r for r in ROWS if r < 400] + FEW if few else ROWS, 256, 8192, act, torch.bfloat16, div=8))
+
+
+@pytest.mark.parametrize("kind", ["16 bit", "fp8"])
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_infinities_and_nan_stay_in_their_rows(kind, act, dtype):
+    """Operand rows of infinities and of NaN (fp8: its NaN; its scales infinite): those rows as the other kernel has them, all others
+    their own values, and results beyond the largest half or bfloat16."""
+    out, n_out = _launch(kind, ROWS, 512, 768, act, dtype, strange=True)
+    a, b = (o[:, :n_out].float() for o in out)
+    assert a.isnan().any() and a.isinf().any() and a.isfinite().any(dim=1).any()
+    assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())
 
 
 @pytest.mark.parametrize("n,k,rows,tile", [
