@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes as C
 import importlib.util
 import os
+import warnings
 
 import torch
 
@@ -177,12 +178,16 @@ def _load() -> C.CDLL:
 
 
 def _load_torch_calls():
-    """The extension of calls whose host time matters (csrc/torch_calls.cpp), beside the library it calls."""
-    if not os.path.exists(TORCH_CALLS_PATH):
-        raise ImportError(f"{TORCH_CALLS_PATH} is missing: build it with `make -C {PROJECT_DIR}` (or __graft_entry__.build()).")
-    spec = importlib.util.spec_from_file_location("kmoe_torch", TORCH_CALLS_PATH)
-    module = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(module)
+    """The extension of calls whose host time matters (csrc/torch_calls.cpp), beside the library it calls. None where it was not
+    built, or for another torch: the same calls then run in Python, on the same kernels."""
+    try:
+        spec = importlib.util.spec_from_file_location("kmoe_torch", TORCH_CALLS_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except (ImportError, OSError) as problem:
+        warnings.warn(f"{TORCH_CALLS_PATH} cannot be loaded ({problem}): small Linears cost more host time. Build it with "
+                      f"`make -C {PROJECT_DIR}`.", RuntimeWarning)
+        return None
     return module
 
 

@@ -551,7 +551,8 @@ def silu_and_mul(out: torch.Tensor, x: torch.Tensor, axis: int = -1, turn: bool 
 
 
 # On GPU tensors the native body is called (csrc/torch_calls.cpp), which leaves what is not ordinary to this one.
-L.torch_calls.install(L.check, silu_and_mul)
+if L.torch_calls is not None:
+    L.torch_calls.install(L.check, silu_and_mul)
 
 
 @operator("_C::moe_post", mutates_args=("y",))

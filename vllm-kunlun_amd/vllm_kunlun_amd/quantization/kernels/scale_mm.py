@@ -76,7 +76,7 @@ class _DynamicCall:
         g.n, g.k, g.ld_x, g.ldy, g.w_layout = self.n, self.k, self.k, self.n, layout
         self.args = g
         self.native = (L.torch_calls.Linear(*self.at, self.n, self.k, layout, self.device.index, self.split_max)
-                       if self.device.type == "cuda" else None)
+                       if self.device.type == "cuda" and L.torch_calls is not None else None)
 
     @staticmethod
     def _value(layer, name):
