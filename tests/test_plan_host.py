@@ -120,3 +120,14 @@ def test_layers_that_hit_outlive_calls_that_always_miss(monkeypatch):
     for step in range(4):
         _plan._keep_call(("other", step), _kept_call(w))
     assert _plan._kept_call("layer") is None
+
+
+def test_workspace_keeps_no_stand_in():
+    """A call under a fake-tensor mode fails, as it always did, and leaves nothing behind for the real calls after it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from vllm_kunlun_amd._plan import _Workspace
+    pool, device = _Workspace(), torch.device("cpu")
+    with FakeTensorMode():
+        pool.get(64, device, 1)
+    real = pool.get(64, device, 1)
+    assert type(real) is torch.Tensor and pool.get(32, device, 1) is real

@@ -43,6 +43,8 @@ class _Workspace:
         if buf is None or buf.numel() < nbytes:
             # allocated with the launching stream current, so the allocator ties the block to that stream
             buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+            if type(buf) is not torch.Tensor:  # (a tracing mode's stand-in: real calls would find it)
+                return buf
             self._buf[key] = buf
         self._buf.move_to_end(key)
         while len(self._buf) > self.MAX_STREAMS:
