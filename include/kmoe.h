@@ -359,7 +359,8 @@ typedef struct kmoe_gemm_bf16_args {
   uint16_t* y;            /* bf16 [rows, n] or [rows, n/2] with SwiGLU                */
   int64_t ldy;
   int32_t act;
-  int32_t variant;
+  int32_t variant;        /* 0 = choose from the shape. Tuning and tests: 1-3 LDS-staged kernels; with tiled weights 5, 6, 11, 13,
+                             12, 18 as for int8, 23: as for int8 with k % 64 == 0, k >= 384, no bias and no SWIGLUOAI */
   int32_t w_layout;       /* KMOE_W_ROWMAJOR, or KMOE_W_TILED: the BYTES of w ([E, n, 2k])
                              re-arranged by kmoe_tile_weights_i8(E, n, 2k); needs k % 32 == 0 */
   /* the expert-bias branch of KunlunOps.fused_moe (ops/_kunlun_ops.py:433-468): */

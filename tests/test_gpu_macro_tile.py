@@ -10,9 +10,10 @@ FEW = [0, 1, 2, 0, 3] * 12  # with these an expert holds few rows on average: th
 ROWS = [1, 15, 16, 17, 0, 191, 192, 193, 33, 384, 385, 0, 127, 128, 129, 800, 3100]  # up to 17 tiles of an expert
 
 
-def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, bound=0, seed=0, variant=23, trace=False, strange=False):
+def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, bound=0, seed=0, variant=23, trace=False, strange=False, reference=False):
     """Outputs of the variants 6 and 23 (or another) for the same operands; trace: and the latter's kernel. pad: values between the rows of a and y; tail: rows of an expert
-    outside w (int8); bound: rows the caller allows for beyond the last expert's; strange: infinities and NaN in some rows of a."""
+    outside w (int8); bound: rows the caller allows for beyond the last expert's; strange: infinities and NaN in some rows of a;
+    reference: the second is the float32 product of the dequantised operands instead."""
     from vllm_kunlun_amd import _lib as L
     g = torch.Generator(device="cuda").manual_seed(seed)
     E, rows, n_out = len(counts), sum(counts), n // 2 if act else n
@@ -58,6 +59,20 @@ def _launch(kind, counts, n, k, act, dtype, div=1, gather=True, pad=0, tail=0, b
         L.lib.kmoe_trace_kernels(0)
         out.append(y)
     torch.cuda.synchronize()
+    if reference:
+        rows_of_a = (src.long() // div if gather else torch.arange(rows, device="cuda"))
+        x = a[:, :k].float()
+        x = x * (a_max.repeat_interleave(128, 1) if f8 else (a_max / 127)[:, None]) if i8 or f8 else x
+        for e in range(E):
+            if counts[e]:
+                we = w[e].float()
+                we = we * (w_max[e].repeat_interleave(128, 0).repeat_interleave(128, 1) if f8 else (w_max[e] / 127)[:, None]) if i8 or f8 else we
+                at = slice(int(lod[e]), int(lod[e + 1]))
+                v = x[rows_of_a[at]] @ we.t()
+                if act:
+                    gate, up = (t.to(dtype).float() for t in v.split(n_out, 1))
+                    v = torch.nn.functional.silu(gate) * up
+                out[0][at, :n_out] = v.to(dtype)
     return (out, n_out, L.lib.kmoe_traced_kernels().decode()) if trace else (out, n_out)
 
 
@@ -72,6 +87,19 @@ def _same(out, n_out):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_tiles(kind, n, k, act, dtype):
     _same(*_launch(kind, ROWS, n, k if kind == "int8" else k // 2, act, dtype, div=8))
+
+
+@pytest.mark.parametrize("kind", ["int8", "16 bit", "fp8"])
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_against_float32(kind, act, dtype):
+    """The bounds that the other tiles are held to against the product of the same values in float32: two roundings of 2^-9 relative
+    (gate and up before SiLU-mul, and the result)."""
+    out, n_out = _launch(kind, ROWS, 512, 768, act, dtype, div=8, reference=True)
+    ref, got = (o[:, :n_out].float() for o in out)
+    assert not got.isnan().any()
+    per_row = (got - ref).norm(dim=1) / ref.norm(dim=1).clamp(min=1e-6)
+    assert float((got - ref).norm() / ref.norm()) <= 4e-3 and float(per_row.max()) <= 2e-2
 
 
 @pytest.mark.parametrize("n,k", [(256, 768), (768, 896), (512, 1024), (512, 1152), (256, 2048)])  # 6 to 9 and 16 blocks of K

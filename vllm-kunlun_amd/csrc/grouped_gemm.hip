@@ -488,12 +488,12 @@ int grouped_gemm_i8_checked(const kmoe_gemm_i8_args* a, kmoe_stream_t stream, co
   KMOE_REQUIRE(a->a_layout == KMOE_A_ROWMAJOR, KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8: a_layout=%d unknown",
                a->a_layout);
   if (a->rows == 0 && !(a->w_tail && a->tail_rows > 0)) return KMOE_OK;
-  // Tiled weights and more than a few rows per expert: the persistent tile kernel (variants 5-9, 11-16 force it)
+  // Tiled weights and more than a few rows per expert: the persistent tile kernels (variants 5-9, 11-23 force one)
   if (a->w_layout == KMOE_W_TILED && a->k >= 128 &&
       ((a->variant >= 5 && a->variant <= 9) || (a->variant >= 11 && a->variant <= 23) ||
        (a->variant == 0 && ceil_div(expected_rows(a->rows, a->rows_hint), a->E) > kTiledMinRows)))
     return tiled_gemm_i8(a, as_stream(stream));
-  KMOE_REQUIRE(a->variant < 5, KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8: variants 5-12 need tiled weights and k >= 128");
+  KMOE_REQUIRE(a->variant < 5, KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8: variants 5-9 and 11-23 need tiled weights and k >= 128");
   GemmParams p{a->a,   a->lda, a->a_max, a->row_src, a->src_div, a->w,   a->w_max,
                a->lod, a->E,   a->n,     a->k,       a->y,       a->ldy, a->acc_out, a->w_layout == KMOE_W_TILED,
                a->w_tail, a->w_max_tail, a->tail_row0, a->w_tail ? a->tail_rows : 0, a->tail_src0, nullptr, 0, 0.f, 0.f,
@@ -537,12 +537,12 @@ int grouped_gemm_bf16_checked(const kmoe_gemm_bf16_args* a, kmoe_stream_t stream
   if (a->w_layout == KMOE_W_TILED && a->variant == 0 && !a->bias && !oai && streams_bf16(live, a->E, a->k))
     return stream_gemm_bf16(a, as_stream(stream), scan, slots);
   KMOE_REQUIRE(!scan && !slots, KMOE_ERR_UNSUPPORTED, "grouped_gemm_bf16: only the weight-streaming kernel sorts the pairs itself");
-  // tiled weights and more rows: the persistent tile kernel (variants 5, 6, 11-13, 18 force it)
+  // tiled weights and more rows: the persistent tile kernels (variants 5, 6, 11-13, 18, 23 force one)
   const bool forced = tile_variant(a->variant) || a->variant == 18 || a->variant == 23;
   if (a->w_layout == KMOE_W_TILED && a->k >= 64 && a->ldy % 8 == 0 &&
       (forced || (a->variant == 0 && ceil_div(live, a->E) > kTiledMinRows)))
     return tiled_gemm_bf16(a, as_stream(stream));
-  KMOE_REQUIRE(!forced, KMOE_ERR_UNSUPPORTED, "grouped_gemm_bf16: variants 5, 6, 11-13 and 18 need tiled weights, k >= 64 and ldy %% 8 == 0");
+  KMOE_REQUIRE(!forced, KMOE_ERR_UNSUPPORTED, "grouped_gemm_bf16: variants 5, 6, 11-13, 18 and 23 need tiled weights, k >= 64 and ldy %% 8 == 0");
   GemmParams p{reinterpret_cast<const int8_t*>(a->a), a->lda * 2, nullptr, a->row_src, a->src_div,
                reinterpret_cast<const int8_t*>(a->w), nullptr,    a->lod,  a->E,       a->n,
                a->k * 2,                              a->y,       a->ldy,  nullptr, a->w_layout == KMOE_W_TILED,
@@ -586,13 +586,13 @@ int grouped_gemm_fp8_checked(const kmoe_gemm_fp8_args* a, kmoe_stream_t stream, 
   if (a->w_layout == KMOE_W_TILED && a->variant == 0 && streams_fp8(live, a->E, a->k))
     return stream_gemm_fp8(a, as_stream(stream), scan, slots);
   KMOE_REQUIRE(!scan && !slots, KMOE_ERR_UNSUPPORTED, "grouped_gemm_fp8_block: only the weight-streaming kernel sorts the pairs itself");
-  // tiled weights and more rows: the persistent tile kernel (variants 5, 6, 11 force it)
+  // tiled weights and more rows: the persistent tile kernels (variants 5, 6, 8, 11-14, 17-20, 23 force one)
   const bool tall_variant = a->variant == 8 || a->variant == 14 || (a->variant >= 17 && a->variant <= 20) || a->variant == 23;  // 8-wave tiles of 256 / 192 rows; 17: chosen on the device; 18, 20, 19: wide 192- / 160- / 128-row tiles
   if (a->w_layout == KMOE_W_TILED && a->k <= 8192 && a->ldy % 8 == 0 &&
       (tile_variant(a->variant) || tall_variant || (a->variant == 0 && ceil_div(live, a->E) > kTiledMinRows)))
     return tiled_gemm_fp8(a, as_stream(stream));
   KMOE_REQUIRE(!tile_variant(a->variant) && !tall_variant, KMOE_ERR_UNSUPPORTED,
-               "grouped_gemm_fp8_block: variants 5, 6, 8, 11-14 need tiled weights, k <= 8192");
+               "grouped_gemm_fp8_block: variants 5, 6, 8, 11-14, 17-20 and 23 need tiled weights, k <= 8192");
   GemmParams p{reinterpret_cast<const int8_t*>(a->a), a->lda, a->a_scale, a->row_src, a->src_div,
                reinterpret_cast<const int8_t*>(a->w), a->w_scale, a->lod,  a->E,       a->n,
                a->k,                                  a->y,       a->ldy,  nullptr, a->w_layout == KMOE_W_TILED,
