@@ -320,6 +320,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
     if constexpr (kTight) asm volatile("" : "+v"(v));
     return v;
   };
+  auto lane_here = [&]() __attribute__((always_inline)) -> int { return kTight ? static_cast<int>(here(lane16) >> 4) : lane; };
   // channel of fragment f of the waves in column c (0: past the last channel, never stored)
   auto col_of = [&](const MTile& t, int c, int f, bool& ok) -> int {
     const int fh = SWIGLU ? f % NFH : f;
@@ -349,7 +350,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   };
   uint32_t a_off[kNA];
   // copy i of this wave fills rows 8 (kNA wave + i) + lane / 8 of a chunk buffer
-  auto dma_row = [&]() __attribute__((always_inline)) { return wave * 8 * kNA + static_cast<int>(here(lane16) >> 7); };
+  auto dma_row = [&]() __attribute__((always_inline)) { return wave * 8 * kNA + (lane_here() >> 3); };
   auto dma_a = [&](int chunk, uint32_t buf_at, int i) __attribute__((always_inline)) {
     buffer_load16_to_lds(a_rsrc, (lds_ptr_t)(&ring_a[0][0] + buf_at + (wave * kNA + i) * 1024), a_off[i],
                          static_cast<uint32_t>(chunk) * kMChunk);
@@ -400,8 +401,8 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   // ---- first tile ----
   auto row_offset = [&](const MTile& t, int i, int fetched) -> uint32_t {  // rows past the tile's end are not read
     const int r = t.row0 + dma_row() + 8 * i;
-    const uint32_t now = here(lane16);
-    const uint32_t a_col = (now ^ (now >> 3)) & 0x70u;  // vector c of row r at position c ^ r % 8
+    const int l = lane_here();
+    const uint32_t a_col = static_cast<uint32_t>((l & 7) ^ ((l >> 3) & 7)) * 16u;  // vector c of row r at position c ^ r % 8
     return r < t.end ? src_row(t, r, fetched) * static_cast<uint32_t>(p.lda) + a_col : kRange;  // < 4 GiB: host-checked
   };
   Weights w_cur = weights_of(cur);
@@ -425,13 +426,13 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   };
   auto dma_tile_scales = [&](const MTile& t, int parity, int fetched) __attribute__((always_inline)) {
     if constexpr (F8) {
-      asc_off = src_row(t, clamp_row(t, t.row0 + 64 * (wave & 3) + static_cast<int>(here(lane16) >> 4)), fetched) * static_cast<uint32_t>(kblocks) * 4u;
+      asc_off = src_row(t, clamp_row(t, t.row0 + 64 * (wave & 3) + lane_here()), fetched) * static_cast<uint32_t>(kblocks) * 4u;
       const int b = wave - 4;  // waves 4 and 5: a block of 128 channels each
       if (b == 0 || b == 1) {
         const int row = SWIGLU ? t.nb + b * (n_half / 128) : min(2 * t.nb + b, p.n / 128 - 1);
         const float* ws = t.e >= p.E ? p.w_max_tail : p.w_max + static_cast<size_t>(t.e) * (p.n / 128) * kblocks;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(ws), (lds_ptr_t)&wsc_lds[parity][b * kMacroBlocks], 4,
-                                                 static_cast<uint32_t>(row * kblocks + min(static_cast<int>(here(lane16) >> 4), kblocks - 1)) * 4u, 0, 0, 0);
+                                                 static_cast<uint32_t>(row * kblocks + min(lane_here(), kblocks - 1)) * 4u, 0, 0, 0);
       }
     }
   };
@@ -624,7 +625,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
       const uint32_t a_lo = fa[0] + buf, a_hi = kTight ? a_lo ^ 64u : fa[1] + buf;  // (bit 2 of the vector's position)
       const uint32_t w_at = kTight ? lds_addr(&ring_w[0][0]) + wn * 4096u + slot + here(lane16) : fw + slot;
       const int base = min(c & ~3, kblocks - 4);
-      const uint32_t sa_at = lds_addr(&asc_lds[0][0]) + static_cast<uint32_t>(group * 16 * kTM + (wm * 16 + static_cast<int>(here(lane16) >> 4 & 15)) * 16 + 4 * (c - base));
+      const uint32_t sa_at = lds_addr(&asc_lds[0][0]) + static_cast<uint32_t>(group * 16 * kTM + (wm * 16 + (lane_here() & 15)) * 16 + 4 * (c - base));
       const uint32_t sw_at = lds_addr(&wsc_lds[parity][SWIGLU ? 0 : (wn >> 1) * kMacroBlocks]) + 4u * c;
       float sw[2], sa_c[2], sc[2][2];
       v4i lo[2], hi[2], wl[kMFrags], wh[kMFrags];
@@ -716,7 +717,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
     }
     auto fetch_next = [&]() __attribute__((always_inline)) {  // the gather entries of the next tile's rows
       if (p.row_src && 64 * wave < kTM && wave < 4) {
-        const int rr = clamp_row(look, look.row0 + 64 * wave + static_cast<int>(here(lane16) >> 4));
+        const int rr = clamp_row(look, look.row0 + 64 * wave + lane_here());
         __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(p.row_src), (lds_ptr_t)&idx_lds[64 * wave], 4,
                                                  static_cast<uint32_t>(look.e < p.E ? rr : 0) * 4u, 0, 0, 0);
       }
@@ -724,7 +725,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
     auto next_rows = [&]() __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < kNA; ++i) a_off[i] = row_offset(look, i, m_read_i32(lds_addr(&idx_lds[dma_row() + 8 * i])));
-      return m_read_i32(lds_addr(&idx_lds[min(64 * (wave & 3) + static_cast<int>(here(lane16) >> 4), kTM - 1)]));
+      return m_read_i32(lds_addr(&idx_lds[min(64 * (wave & 3) + lane_here(), kTM - 1)]));
     };
     const Weights w_nxt = weights_of(look);
     if constexpr (F8) {
