@@ -90,6 +90,39 @@ def _dequantised(packed, scale, dtype):
     return (codes * scale.float().repeat_interleave(32, 1)).to(dtype).float()
 
 
+@pytest.mark.parametrize("variant", [16, 32, 64, 96, 128])
+@pytest.mark.parametrize("blocks,group", [(1, 32), (1, 128), (2, 256), (3, 64), (5, 32), (8, 1024), (9, 128), (9, 384)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_packed_tiles_take_scales_by_chunks(variant, blocks, group, dtype):
+    """Re-arranged group scales (which the tile kernel copies several blocks at a time: less than a chunk, chunks and a rest, groups of
+    part of a block to several chunks) give the bits of row-major ones, and so do scales that begin between 16-byte boundaries."""
+    from vllm_kunlun_amd import _lib as L
+    gen = torch.Generator().manual_seed(blocks + group)
+    counts = [variant + 1, 0, 1, 17]
+    E, rows, n, k = len(counts), sum(counts), 160, 128 * blocks
+    groups = k // group
+    a = torch.randn(rows, k, generator=gen).to(dtype).cuda()
+    packed = torch.randint(0, 256, (E, n, k // 2), generator=gen, dtype=torch.uint8).cuda()
+    scale = (torch.rand(E, n, groups, generator=gen) * 0.02 + 0.002).to(dtype).cuda()
+    tiled, chunks = torch.empty_like(packed), torch.empty_like(scale)
+    L.check(L.lib.kmoe_tile_weights_i8(packed.data_ptr(), tiled.data_ptr(), E, n, k // 2, L.stream()))
+    L.check(L.lib.kmoe_tile_scales_w4(scale.data_ptr(), chunks.data_ptr(), E, n, groups, L.stream()))
+    shifted = torch.empty(scale.numel() + 8, dtype=dtype, device="cuda")[4:-4].copy_(chunks.flatten())
+    lod = torch.tensor([0] + counts).cumsum(0).int().cuda()
+    for act in (0, 1):
+        out = []
+        for s, layout in ((scale, L.KMOE_S_ROWMAJOR), (chunks, L.KMOE_S_FRAG16), (shifted, L.KMOE_S_FRAG16)):
+            y = torch.full((rows, n // 2 if act else n), float("nan"), dtype=dtype, device="cuda")
+            g = L.GemmW4Args()
+            g.a, g.lda, g.src_div, g.scale_layout = a.data_ptr(), k, 1, layout
+            g.w, g.w_scale, g.group_size, g.lod = tiled.data_ptr(), s.data_ptr(), group, lod.data_ptr()
+            g.E, g.n, g.k, g.rows, g.w_layout = E, n, k, rows, L.KMOE_W_TILED
+            g.y, g.ldy, g.act, g.variant, g.act_dtype = y.data_ptr(), y.shape[1], act, variant, L.act_dtype(a, "test")
+            L.check(L.lib.kmoe_grouped_gemm_w4a16(g, L.stream()))
+            out.append(y)
+        assert not out[0].isnan().any() and torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
 @pytest.mark.parametrize("variant", [0, 1, 2, 4])
 @pytest.mark.parametrize("act,gather", [(0, False), (1, False), (1, True)])
 def test_packed_weights_on_rows_far_apart(variant, act, gather):

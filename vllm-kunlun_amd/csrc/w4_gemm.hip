@@ -59,7 +59,7 @@ constexpr int kWaves = 4;
 // the row fragments of the tile, one MFMA each; the kernel is bound by issuing both, at a quarter of the 16-bit weights'
 // bytes. One workgroup: one tile of sorted rows of one expert x 4 waves x 4 fragments of 16 channels. Activations are
 // copied global -> LDS asynchronously in 128-value blocks of K (256 bytes per row); every wave reads its A fragments
-// from there. Weights and their scales go global -> registers, one or two blocks ahead; they never pass through LDS.
+// from there. Weights go global -> registers, one or two blocks ahead; they never pass through LDS.
 
 // Work item `item` = (m-tile, channel block) when every expert's rows are cut into tiles of kTileRows and the
 // items are numbered m-tile by m-tile: expert, first row and channel block (false: no such item). The hardware
@@ -159,9 +159,18 @@ constexpr int w4_ring(int MF) { return MF == 6 ? 3 : 2; }
 // (A hot expert's tiles do, too: Kimi-K2 dims, +2.0 on the logits of 8 experts, 1000 tokens 2120 / 2135, 2000 2639 / 2666, but 400 1799 / 1779. A
 // choice per tile between two loops, as the tile kernel of the other formats has, took 2627 at 2000, but more elsewhere: 400 even 1623 -> 1677,
 // Qwen3 dims, 400 with hot experts 111 -> 119.)
-template <int MF, bool SWIGLU, bool F16, bool PAST>
+// CHUNKED: the scales come CB blocks at a time, by asynchronous copies into LDS of the wave's own, one chunk ahead, and from there to
+// registers one block ahead (a group of 32: 512 consecutive bytes of each fragment). Asked for block by block and lane by lane they were a third
+// of the load instructions for a ninth of the bytes, in pieces of 128: with nothing but its loads the gate_up launch of Kimi-K2 dims, 2048 tokens, took
+// 1275 us with them and 1160 without. For layouts KMOE_S_FRAG16 with groups of a power of two; others keep those loads. With rows past a tile's
+// end no longer fetched and a step unpacked right before its MFMAs (ten registers less, the other waves' MFMAs run beside it), layer, us,
+// before / after: Kimi-K2 dims 64 tokens 1167 / 1124, 150 1517 / 1466, 400 1662 / 1608, 800 1807 / 1768, 2048 2416 / 2374; Qwen3 dims 64 75.4 / 74.1,
+// 240 88.3 / 85.5, 400 101.0 / 98.5, 1000 145.7 / 145.4, 4096 403 / 400.
+constexpr int w4_chunk(int MF) { return MF >= 6 ? 2 : 4; }
+template <int MF, bool SWIGLU, bool F16, bool PAST, bool CHUNKED>
 __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kernel(const W4Params p) {
-  constexpr int NF = 4, R = w4_ring(MF);
+  constexpr int NF = 4, R = w4_ring(MF), CB = w4_chunk(MF);
+  constexpr int kScaleBytes = NF * CB * 128;  // a chunk of groups of 32; fewer bytes of larger groups
   constexpr int kTileRows = 16 * MF;
   constexpr int NFH = SWIGLU ? NF / 2 : NF;
   constexpr int NA = kTileRows / 4 / kWaves;  // asynchronous copies per wave and block: 4 rows (1 KB) each
@@ -175,6 +184,7 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
   // four clocks more per read).
   auto swizzle = [](int r) { return r ^ ((r & 4) << 1); };
   __shared__ __attribute__((aligned(1024))) int8_t lds_a[R][kBufBytes];
+  __shared__ __attribute__((aligned(1024))) int8_t lds_s[CHUNKED ? kWaves : 1][2][CHUNKED ? kScaleBytes : 16];
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15;
@@ -194,8 +204,8 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a), 0, kRange, 0x00020000);
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(p.w + static_cast<size_t>(e) * p.n * (p.k / 2)), 0, kRange, 0x00020000);
-  const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(p.scale + static_cast<size_t>(e) * p.n * groups), 0, kRange, 0x00020000);
+  const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.scale + static_cast<size_t>(e) * p.n * groups), 0,
+                                                                          CHUNKED ? static_cast<uint32_t>(p.n * groups) * 2u : kRange, 0x00020000);
 
   uint32_t woff[NF], soff[NF];  // scalar: the fragment's first block; vector: the lane's channel in the fragment's scales
   bool wok[NF];
@@ -216,9 +226,10 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
   for (int i = 0; i < NA; ++i) {
     const int tr = kWaveRows * wave + 4 * i + lg;
     const int r = row0 + tr;
-    const int rr = r < row_end ? r : row0;  // rows past the end read the tile's first row: never stored
+    const int rr = r < row_end ? r : row0;
     const int src = p.row_src ? p.row_src[rr] / p.src_div : rr;
-    aoff[i] = static_cast<uint32_t>(src) * static_cast<uint32_t>(p.lda * 2) + ((li ^ swizzle(tr & 15)) << 4);  // < 4 GiB: host-checked
+    // < 4 GiB: host-checked; rows past the end are not read (and never stored)
+    aoff[i] = r < row_end ? static_cast<uint32_t>(src) * static_cast<uint32_t>(p.lda * 2) + ((li ^ swizzle(tr & 15)) << 4) : kRange;
   }
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)&lds_a[0][0]));
   // fragment reads of MFMA step t: row li (+ 16 per fragment: same row % 16), vector 4 lg + t
@@ -231,18 +242,49 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
 #pragma unroll
     for (int f = 0; f < NF; ++f) acc[mf][f] = (v4f){0.f, 0.f, 0.f, 0.f};
   v4i wbuf[R][NF];
-  uint16_t sbuf[R][NF];
+  int sbuf[CHUNKED ? 1 : R][NF];  // (the upper halves are not looked at)
   const uint32_t lane16 = lane * 16u;
   const uint32_t lane_s = li * p.s_ch * 2u;
+  // chunked scales: a fragment's groups of a chunk are s_frag consecutive bytes; copy j of a chunk takes bytes 1024 j + 16 lane of the
+  // wave's fragments, one behind the other
+  constexpr int NS = CHUNKED ? kScaleBytes / 1024 : 1;
+  const int s_frag = 32 * max(1, (4 * CB) >> max(p.gs_shift, 0));
+  uint32_t s_off[NS];
+  const uint32_t s_lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)&lds_s[CHUNKED ? wave : 0][0][0]));
+  if constexpr (CHUNKED) {
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+      const int at = j * 1024 + lane * 16, f = at / s_frag;
+      uint32_t off = kRange;
+#pragma unroll
+      for (int g = 0; g < NF; ++g) off = f == g ? soff[g] + static_cast<uint32_t>(at & (s_frag - 1)) : off;
+      s_off[j] = off;
+    }
+  }
+  auto first_group = [&](int kb) __attribute__((always_inline)) { return (4 * (kb & ~(CB - 1))) >> p.gs_shift; };  // of the chunk of block kb
+  auto dma_s = [&](int kb) __attribute__((always_inline)) {  // the chunk that begins with block kb
+    const uint32_t at = kb < kblocks ? static_cast<uint32_t>(first_group(kb)) * 32u : kRange;
+#pragma unroll
+    for (int j = 0; j < NS; ++j) buffer_load16_to_lds(s_rsrc, (lds_ptr_t)&lds_s[CHUNKED ? wave : 0][kb / CB & 1][j * 1024], s_off[j], at);
+  };
+  // the scales of block kb, which the caller has seen land in LDS; usable behind the wait for a younger LDS read
+  auto request_s = [&](int kb) __attribute__((always_inline)) {
+    const uint32_t at = s_lds + static_cast<uint32_t>((kb / CB & 1) * kScaleBytes + (((4 * kb + lg) >> p.gs_shift) - first_group(kb)) * 32 + li * 2);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) asm volatile("ds_read_u16 %0, %1" : "=v"(sbuf[0][f]) : "v"(at + static_cast<uint32_t>(f * s_frag)) : "memory");
+  };
   auto load_w = [&](int slot, int kb) __attribute__((always_inline)) {
     const bool live = kb < kblocks;
-    const int g32 = 4 * kb + lg;  // this lane's 32 values of the block
-    const uint32_t s_at = lane_s + static_cast<uint32_t>((p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / (p.gs / 32)) * p.s_g) * 2u;
+    uint32_t s_at = 0;
+    if constexpr (!CHUNKED) {
+      const int g32 = 4 * kb + lg;  // this lane's 32 values of the block
+      s_at = lane_s + static_cast<uint32_t>((p.gs_shift >= 0 ? g32 >> p.gs_shift : g32 / (p.gs / 32)) * p.s_g) * 2u;
+    }
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       const uint32_t at = live ? woff[f] + static_cast<uint32_t>(kb) * 1024u : kRange;
       wbuf[slot][f] = PAST ? buffer_stream_load16(w_rsrc, lane16, at) : buffer_load16(w_rsrc, lane16, at);
-      sbuf[slot][f] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(s_rsrc, s_at, live ? soff[f] : kRange, 0));
+      if constexpr (!CHUNKED) sbuf[slot][f] = __builtin_amdgcn_raw_buffer_load_b16(s_rsrc, s_at, live ? soff[f] : kRange, 0);
     }
   };
   auto dma_a = [&](int buf, int kb) __attribute__((always_inline)) {
@@ -252,12 +294,18 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
       buffer_load16_to_lds(a_rsrc, (lds_ptr_t)&lds_a[buf][(kWaveRows * wave + 4 * i) * 256], aoff[i], at);
   };
   // One block: word t of a lane's 16 packed bytes is its operand of MFMA step t; the activation lane (lg, row)
-  // supplies values 32 lg + 8 t + [0, 8) of the block, i.e. vector 4 lg + t of the row's 16. The words of step t + 1
-  // are unpacked between the row fragments of step t: the matrix and the vector unit both have work from one wave.
-  auto compute = [&](auto slot_tag) __attribute__((always_inline)) {
-    constexpr int slot = decltype(slot_tag)::value;
-    const W4Scale<F16> sc[NF] = {W4Scale<F16>(sbuf[slot][0]), W4Scale<F16>(sbuf[slot][1]), W4Scale<F16>(sbuf[slot][2]),
-                                 W4Scale<F16>(sbuf[slot][3])};
+  // supplies values 32 lg + 8 t + [0, 8) of the block, i.e. vector 4 lg + t of the row's 16.
+  auto compute = [&](int kb, auto slot_tag) __attribute__((always_inline)) {
+    constexpr int slot = decltype(slot_tag)::value, ss = CHUNKED ? 0 : slot;
+    if constexpr (CHUNKED) {  // (asked for a block ago; the reads behind them have landed)
+#pragma unroll
+      for (int f = 0; f < NF; ++f) asm volatile("" : "+v"(sbuf[0][f])::"memory");
+    }
+    const W4Scale<F16> sc[NF] = {W4Scale<F16>(sbuf[ss][0]), W4Scale<F16>(sbuf[ss][1]), W4Scale<F16>(sbuf[ss][2]), W4Scale<F16>(sbuf[ss][3])};
+    if constexpr (CHUNKED) {
+      __builtin_amdgcn_sched_barrier(0);
+      request_s(kb + 1);
+    }
     // Row fragments are read two ahead, across the steps: fragment i = t MF + mf of the block's 4 MF.
     v4i af[3];
     auto request = [&](auto i_tag) __attribute__((always_inline)) {
@@ -269,9 +317,7 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
     };
     request(std::integral_constant<int, 0>{});
     request(std::integral_constant<int, 1>{});
-    v4i wv[2][NF];
-#pragma unroll
-    for (int f = 0; f < NF; ++f) wv[0][f] = unpack8(static_cast<uint32_t>(wbuf[slot][f][0]), sc[f]);
+    v4i wv[NF];
     __builtin_amdgcn_sched_barrier(0);
     static_for<4 * MF>([&](auto i_tag) __attribute__((always_inline)) {
       constexpr int i = decltype(i_tag)::value;
@@ -284,29 +330,37 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
       } else {
         lds_wait<0>(af[i % 3]);
       }
-      mfma4_if_live<F16, mf>(acc[mf], wv[t & 1], af[i % 3], live_frags);
-      if constexpr (t < 3) {
+      if constexpr (mf == 0) {
 #pragma unroll
-        for (int f = 0; f < NF; ++f)
-          if (f * MF / NF == mf) wv[(t + 1) & 1][f] = unpack8(static_cast<uint32_t>(wbuf[slot][f][t + 1]), sc[f]);
+        for (int f = 0; f < NF; ++f) wv[f] = unpack8(static_cast<uint32_t>(wbuf[slot][f][t]), sc[f]);
       }
+      mfma4_if_live<F16, mf>(acc[mf], wv, af[i % 3], live_frags);
       __builtin_amdgcn_sched_barrier(0);  // (all the unpacking of a block at once would not fit the registers)
     });
   };
   auto stage = [&](int kb, auto u_tag) __attribute__((always_inline)) {
     constexpr int u = decltype(u_tag)::value;
-    vmem_wait<(R - 2) * (NA + 2 * NF)>();  // the loads of a wave younger than those the stage needs
+    vmem_wait<(R - 2) * (NA + (CHUNKED ? 1 : 2) * NF)>();  // the loads of a wave younger than those the stage needs
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (CHUNKED) {
+      if ((kb & (CB - 1)) == 0) dma_s(kb + CB);
+    }
     dma_a((u + R - 1) % R, kb + R - 1);
     load_w((u + R - 1) % R, kb + R - 1);
     __builtin_amdgcn_sched_barrier(0);
-    compute(u_tag);
+    compute(kb, u_tag);
   };
+  if constexpr (CHUNKED) dma_s(0);
 #pragma unroll
   for (int i = 0; i < R - 1; ++i) {
     dma_a(i, i);
     load_w(i, i);
+  }
+  if constexpr (CHUNKED) {  // (the first stage waits for the loads behind these anyway)
+    vmem_wait<0>();
+    request_s(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
   // (no exit inside the body: as one basic block it fits the registers)
   int kb = 0;
@@ -354,10 +408,11 @@ int launch_w4_tile(const W4Params& p, int rows, bool f16, hipStream_t s) {
   if (tracing_kernels())
     note_kernel("w4_tile_kernel<%d-row tiles, %s, %s, %d per CU>", kTileRows, SWIGLU ? "SiLU-mul" : "plain",
                 f16 ? "f16" : "bf16", w4_workgroups(MF));
-  if (f16)
-    hipLaunchKernelGGL((w4_tile_kernel<MF, SWIGLU, true, PAST>), grid, dim3(kWaves * kWave), 0, s, p);
-  else
-    hipLaunchKernelGGL((w4_tile_kernel<MF, SWIGLU, false, PAST>), grid, dim3(kWaves * kWave), 0, s, p);
+  const bool chunked = p.gs_shift >= 0 && p.s_g == 16 && reinterpret_cast<uintptr_t>(p.scale) % 16 == 0 &&
+                       static_cast<int64_t>(p.n) * (p.k / p.gs) < (1ll << 30);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kWaves * kWave), 0, s, p); };
+  if (f16) chunked ? launch(w4_tile_kernel<MF, SWIGLU, true, PAST, true>) : launch(w4_tile_kernel<MF, SWIGLU, true, PAST, false>);
+  else chunked ? launch(w4_tile_kernel<MF, SWIGLU, false, PAST, true>) : launch(w4_tile_kernel<MF, SWIGLU, false, PAST, false>);
   return check_launch("kmoe_grouped_gemm_w4a16");
 }
 
