@@ -128,6 +128,14 @@ def test_tail_expert(kind, tail, act):
     _same(*_launch(kind, ROWS, 512 if kind == "fp8" else 288, 768, act, torch.bfloat16, div=8, tail=tail))
 
 
+@pytest.mark.parametrize("kind", ["int8", "fp8"])
+@pytest.mark.parametrize("counts", [[], [1], [193], [5] * 40], ids=len)  # routed items: none, fewer than XCDs, of two tiles, a share each
+@pytest.mark.parametrize("tail", [7, 1600, 3100])
+def test_tail_expert_is_shared_out(kind, counts, tail):
+    counts = counts or [0]
+    _same(*_launch(kind, counts, 1024, 768, 0, torch.bfloat16, tail=tail))
+
+
 def test_more_items_than_are_resolved_at_once():
     """Over 32 items per workgroup, and weights beyond the memory-side cache: those of experts with one tile are read past it."""
     _same(*_launch("int8", [1, 192, 193, 0, 40] * 28, 16384, 768, 0, torch.bfloat16))
