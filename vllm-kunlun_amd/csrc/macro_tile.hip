@@ -158,20 +158,29 @@ __device__ __forceinline__ void m_copy_weights(const int8_t* base, uint32_t lane
 
 // Sixteen bytes of results a lane, past the caches or not, likewise. (The wait states keep a vector instruction behind it from
 // overwriting the results before the store has read them; those in front are the distance that m_copy_weights keeps.)
+// "Past" is non-temporal for the gate_up launch's rows (SHORT), and for the down launch's, several times as many, written through
+// the L2 as they come (sc1): DeepSeek-V3 dims, layer, us, non-temporal / written through: int8, 700 tokens 1884 / 1863, 2048 2093 / 2080, 4096
+// 2478 / 2465; fp8, 1200 1937 / 1914, 3001 2380 / 2376 (down launch 732 -> 710 at 2048, combine 63 -> 51; the gate_up launch's rows written through:
+// 1262 -> 1301).
+template <bool SHORT>
 __device__ __forceinline__ void m_store(const v4i& v, const v4i& rsrc, uint32_t at, int past) {
-  asm volatile(
-      "s_nop 2\n\t"
-      "s_cmp_eq_u32 %[past], 0\n\t"
-      "s_cbranch_scc1 1f\n\t"
-      "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen nt\n\t"
-      "s_branch 2f\n"
-      "1:\n\t"
-      "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen\n"
-      "2:\n\t"
-      "s_nop 1"
-      :
-      : [v] "v"(v), [at] "v"(at), [r] "s"(rsrc), [past] "s"(past)
-      : "scc", "memory");
+#define KMOE_M_STORE(HOW)                                                       \
+  asm volatile(                                                                 \
+      "s_nop 2\n\t"                                                             \
+      "s_cmp_eq_u32 %[past], 0\n\t"                                             \
+      "s_cbranch_scc1 1f\n\t"                                                   \
+      "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen " HOW "\n\t"             \
+      "s_branch 2f\n"                                                           \
+      "1:\n\t"                                                                  \
+      "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen\n"                       \
+      "2:\n\t"                                                                  \
+      "s_nop 1"                                                                 \
+      :                                                                         \
+      : [v] "v"(v), [at] "v"(at), [r] "s"(rsrc), [past] "s"(past)               \
+      : "scc", "memory")
+  if constexpr (SHORT) KMOE_M_STORE("nt");
+  else KMOE_M_STORE("sc1");
+#undef KMOE_M_STORE
 }
 // Rows of each of an expert's mt tiles: split evenly in whole fragments (an expert with more tiles than a tile has fragments
 // keeps full ones: the rounding could leave the last one without rows).
@@ -551,7 +560,7 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
     constexpr int n = decltype(n_tag)::value;
     constexpr int i = n / kPairs, h = n % kPairs;
     const uint32_t at = y_col + 32 * h < n_half ? y_off + static_cast<uint32_t>(i * 32) * ld_bytes + 64u * h : kRange;
-    m_store(done[i][h], y_rsrc, at, p.y_past);
+    m_store<SWIGLU>(done[i][h], y_rsrc, at, p.y_past);
   };
 
   // One step: its fragments are in registers (set S), the next step's are read into the other set. a_chunk (odd steps): the
