@@ -164,23 +164,34 @@ __device__ __forceinline__ void m_copy_weights(const int8_t* base, uint32_t lane
 // 1262 -> 1301).
 template <bool SHORT>
 __device__ __forceinline__ void m_store(const v4i& v, const v4i& rsrc, uint32_t at, int past) {
-#define KMOE_M_STORE(HOW)                                                       \
-  asm volatile(                                                                 \
-      "s_nop 2\n\t"                                                             \
-      "s_cmp_eq_u32 %[past], 0\n\t"                                             \
-      "s_cbranch_scc1 1f\n\t"                                                   \
-      "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen " HOW "\n\t"             \
-      "s_branch 2f\n"                                                           \
-      "1:\n\t"                                                                  \
-      "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen\n"                       \
-      "2:\n\t"                                                                  \
-      "s_nop 1"                                                                 \
-      :                                                                         \
-      : [v] "v"(v), [at] "v"(at), [r] "s"(rsrc), [past] "s"(past)               \
-      : "scc", "memory")
-  if constexpr (SHORT) KMOE_M_STORE("nt");
-  else KMOE_M_STORE("sc1");
-#undef KMOE_M_STORE
+  if constexpr (SHORT)
+    asm volatile(
+        "s_nop 2\n\t"
+        "s_cmp_eq_u32 %[past], 0\n\t"
+        "s_cbranch_scc1 1f\n\t"
+        "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen nt\n\t"
+        "s_branch 2f\n"
+        "1:\n\t"
+        "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen\n"
+        "2:\n\t"
+        "s_nop 1"
+        :
+        : [v] "v"(v), [at] "v"(at), [r] "s"(rsrc), [past] "s"(past)
+        : "scc", "memory");
+  else
+    asm volatile(
+        "s_nop 2\n\t"
+        "s_cmp_eq_u32 %[past], 0\n\t"
+        "s_cbranch_scc1 1f\n\t"
+        "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen sc1\n\t"
+        "s_branch 2f\n"
+        "1:\n\t"
+        "buffer_store_dwordx4 %[v], %[at], %[r], 0 offen\n"
+        "2:\n\t"
+        "s_nop 1"
+        :
+        : [v] "v"(v), [at] "v"(at), [r] "s"(rsrc), [past] "s"(past)
+        : "scc", "memory");
 }
 // Rows of each of an expert's mt tiles: split evenly in whole fragments (an expert with more tiles than a tile has fragments
 // keeps full ones: the rounding could leave the last one without rows).
