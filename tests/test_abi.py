@@ -236,6 +236,28 @@ def test_packed_launches_on_rows_beyond_4_gib_do_not_take_32_bit_offsets(L):
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="names the kernel a launch would take, on addresses that are not memory")
+@pytest.mark.parametrize("k,most", [(4096, 768), (4224, 96)])
+def test_few_rows_per_expert_decide_the_packed_gate_up_kernel(L, k, most):
+    """A packed gate_up launch on 384 experts: the streaming kernel up to two rows per expert, and with rows longer than 4096
+    values up to a row for every fourth; tiles beyond, also where all but that many rows are other ranks'."""
+    def kernel(rows, hint=0):
+        g = L.GemmW4Args()
+        for f in ("a", "w", "w_scale", "lod", "y"):
+            setattr(g, f, 0x10000)
+        g.E, g.n, g.k, g.rows, g.lda, g.ldy, g.src_div, g.rows_hint = 384, 4096, k, rows, k, 2048, 1, hint
+        g.group_size, g.act, g.w_layout = 32, 1, L.KMOE_W_TILED
+        L.lib.kmoe_trace_kernels(1)
+        assert L.lib.kmoe_grouped_gemm_w4a16(g, None) == -5
+        L.lib.kmoe_trace_kernels(0)
+        return L.lib.kmoe_traced_kernels().decode()
+
+    for rows, hint in ((1, 0), (most, 0), (8 * most, most)):
+        assert "stream_gemm_kernel" in kernel(rows, hint)
+    for rows, hint in ((most + 1, 0), (8 * most, 0), (8 * most, most + 1)):
+        assert "w4_tile_kernel" in kernel(rows, hint)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="names the kernel a launch would take, on addresses that are not memory")
 def test_dense_products_beyond_32_bit_offsets_stay_on_the_streaming_kernel(L):
     """kmoe_grouped_gemm_i8 with a tail matrix alone: the split-K kernel where its 32-bit offsets reach all activations (asked for
     the compute units first, which fails without a GPU), else the streaming kernel (noted before its launch fails)."""

@@ -429,11 +429,16 @@ __global__ __launch_bounds__(256) void tile_scales_kernel(const uint16_t* __rest
 
 }  // namespace
 
-// Layer, us, 16-row passes of the streaming kernel (which sorts the pairs on the way) against 16-row tiles (whose launch
-// needs the sort's): Qwen3 dims 16 tokens (1 row per expert) 62.9 / 64.6, 64 (4) 79.1 / 78.4, 96 (6) 83.5 / 79.7, 128 88.0 /
-// 79.7; Kimi-K2 dims 8 tokens 287 / 291, 32 (1) 832 / 813, 64 (2) 1236 / 1188, 128 (3) 1599 / 1537 - with a long K the sort's launch is nothing.
+// Layer, us, 16-row passes of the streaming kernel (which sorts the pairs on the way) against 16-row tiles (whose launch needs
+// the sort's, and which read a scale once per chunk of the contraction, not per block). Qwen3 dims: 12 tokens 53.7 / 54.4, 20
+// (2 rows per expert) 61.0 / 65.0, 32 (2) 69.9 / 70.5, 40 (3) 76.0 / 71.7, 48 (3) 73.4 / 72.7, 64 (4) 72.8 / 72.3; with eight experts
+// chosen far more often, where the streaming kernel reads an expert's weights again for every 16 rows, 16 tokens 48.9 / 50.8, 24 57.1 /
+// 55.5, 32 63.6 / 62.9, 64 86.1 / 75.1. With a long K the sort's launch is little and the scales are more: Kimi-K2 dims, 5 tokens
+// 187 / 198, 8 (64 rows on 384 experts) 277 / 273, 10 334 / 353, 12 389 / 387, 16 500 / 482, 24 682 / 636, 32 837 / 778, 45 992 / 934,
+// and 45 with eight such experts 779 / 724.
 bool w4_gate_up_streams(int rows, int rows_hint, int E, int k) {
-  return ceil_div(expected_rows(rows, rows_hint), E) <= (k > 4096 ? 1 : 4);
+  const int expected = expected_rows(rows, rows_hint);
+  return k > 4096 ? expected <= E / 4 : ceil_div(expected, E) <= 2;
 }
 
 }  // namespace kmoe
