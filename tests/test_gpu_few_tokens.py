@@ -259,6 +259,27 @@ def test_few_tokens_match_the_oracle(fmt, dtype, M, K, H, I):
     _check(sl, out)
 
 
+@pytest.mark.parametrize("dims,shape", [
+    (dict(M=5, E=48, K=4, H=3072, I=2176), "4 channel fragments"),   # 20 columns, whose down launch splits 17 steps
+    (dict(M=5, E=40, K=6, H=3072, I=384), "2 channel fragments"),    # few workgroups
+    (dict(M=9, E=96, K=8, H=3200, I=640), "4 channel fragments"),    # 25 steps; a column per pair
+    (dict(M=20, E=64, K=4, H=3072, I=512), "4 channel fragments"),   # ... per expert
+    (dict(M=6, E=96, K=4, H=2944, I=640), None)], ids=str)            # shorter rows
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_packed_launches_on_long_rows_match_the_oracle(dims, shape, dtype):
+    """4-bit layers of a few tokens whose gate_up launch splits its long rows over four waves, with as many channels a wave as leave
+    enough workgroups."""
+    from vllm_kunlun_amd import synth
+    sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], quant="w4", **dims), "cuda", seed=dims["M"], dtype=dtype)
+    out, named = _named(lambda: _call(sl))
+    gate_up = [k for k in named.replace(">", ">\n").splitlines() if "SiLU-mul" in k]
+    assert len(gate_up) == 1 and "sorts the pairs itself" in gate_up[0], named
+    assert ("K split 4" in gate_up[0]) == (shape is not None) and (shape is None or shape in gate_up[0]), named
+    if dims["I"] > 2048:
+        assert "plain" in named and named.count("K split 4") == 2, named
+    _check(sl, out)
+
+
 @pytest.mark.parametrize("fmt,I_shared", [("int8", 0), ("int8", 2048), ("fp8", 0), ("fp8", 2048), ("none", 0), ("w4", 0)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_most_rows_of_the_greatest_length(fmt, I_shared, dtype):
