@@ -280,6 +280,20 @@ def test_packed_launches_on_long_rows_match_the_oracle(dims, shape, dtype):
     _check(sl, out)
 
 
+@pytest.mark.parametrize("fmt,dims,launches", [
+    ("int8", dict(M=7, E=256, K=4, H=1600, I=512), ["SiLU-mul, 4 steps in flight, K split 4"]),   # 25 steps
+    ("fp8", dict(M=7, E=256, K=4, H=3200, I=512), ["SiLU-mul, 2 steps in flight, K split 4"]),    # 25 steps
+    ("none", dict(M=9, E=64, K=6, H=4096, I=832), ["SiLU-mul, 4 steps in flight, K split 4", "plain, 4 steps in flight, K split 4"])], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_columns_of_pairs_of_large_layers_match_the_oracle(fmt, dims, launches, dtype):
+    """Large layers of a few tokens, whose column-per-pair launches split K over four waves."""
+    from vllm_kunlun_amd import synth
+    sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], quant=fmt, **dims), "cuda", seed=dims["M"], dtype=dtype)
+    out, named = _named(lambda: _call(sl))
+    assert all(k in named for k in launches) and "a column per pair" in named, named
+    _check(sl, out)
+
+
 @pytest.mark.parametrize("fmt,I_shared", [("int8", 0), ("int8", 2048), ("fp8", 0), ("fp8", 2048), ("none", 0), ("w4", 0)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_most_rows_of_the_greatest_length(fmt, I_shared, dtype):
