@@ -510,8 +510,13 @@ int launch_stream(const StreamParams& p, hipStream_t s) {
 // experts of [3072 x 5120], top 6, int8 5 tokens 74 / 71, bf16 24 456 / 440; 64 of [4096 x 4096], top 8, bf16 7 215 / 203. Down launch, bf16: 64
 // experts of [4096 x 2048] 24 columns 65 / 59, 56 107 / 101, 160 of [5120 x 1536] 36 85 / 85, 72 145 / 152, 144 218 / 261; int8: DeepSeek-V3 dims 24 columns 60
 // / 58.5, 64 of [6144 x 3072] 28 72 / 76, 64 of [4096 x 2048] 32 41.7 / 43.3, DeepSeek-V3 dims 128 236 / 255.
+// From four rows per expert on every workgroup of a large gate_up launch reads rows enough for them to count, and waves of four fragments halve the
+// workgroups that read them, K split four ways where it is long (int8 beyond 4096 codes, fp8 from 6144 on). Layer, us, two fragments / four: DeepSeek-V3 dims int8
+// 110 tokens 1597 / 1596, 128 1668 / 1624, 250 1802 / 1753, 320 1897 / 1821, 250 with +2.0 on the logits of 8 experts 1903 / 1868, fp8 140 1696 / 1682, 250 1821 /
+// 1774; 64 experts of [6144 x 6144], top 4, int8 80 560 / 552; 128 of [3072 x 4096], top 8, int8 150 405 / 386, but fp8 80 374 / 398, bf16 70 748 / 764. Fewer rows: int8
+// 70 tokens 1429 / 1432, 33 1100 / 1101. K split two ways there: 250 tokens 1802 / 1745, and 64 of [4096 x 4096], int8 70 274 / 265 (four ways 270).
 template <Fmt FMT, bool SWIGLU, bool SCAN>
-int launch_rows16(const StreamParams& p, hipStream_t s) {
+int launch_rows16(const StreamParams& p, int rows, hipStream_t s) {
   constexpr int V = FMT == Fmt::F8 ? 2 : 1;
   const int ksteps = p.kbytes / 64;
   const int n_half = SWIGLU ? p.n / 2 : p.n;
@@ -521,6 +526,12 @@ int launch_rows16(const StreamParams& p, hipStream_t s) {
   if (ksteps >= 24 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, 2, 4, SCAN>(p, s);
   if (ksteps >= 24 && p.slots.n > 0 && (SWIGLU || (k16 && p.slots.n < 64)))
     return launch_stream<FMT, 1, 2, SWIGLU, 4 / V, 4, SCAN>(p, s);
+  if constexpr (SWIGLU && FMT == Fmt::I8) {
+    if (ksteps >= 24 && ksteps <= 64 && rows >= 4ll * p.E) return launch_stream<FMT, 1, 4, SWIGLU, 4, 2, SCAN>(p, s);
+  }
+  if constexpr (SWIGLU && (FMT == Fmt::I8 || FMT == Fmt::F8)) {
+    if (ksteps > (FMT == Fmt::I8 ? 64 : 96) && rows >= 4ll * p.E) return launch_stream<FMT, 1, 4, SWIGLU, 4 / V, 4, SCAN>(p, s);
+  }
   if (ksteps >= 24) return launch_stream<FMT, 1, 2, SWIGLU, 4 / V, 2, SCAN>(p, s);
   return launch_stream<FMT, 1, 2, SWIGLU, 4 / V, 1, SCAN>(p, s);
 }
@@ -585,7 +596,7 @@ int stream_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s, const StreamScan* 
   if (scan) {
     if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
     KMOE_REQUIRE(a->a_rows <= kStreamScanMaxRows, KMOE_ERR_UNSUPPORTED, "grouped_gemm_i8 (stream): %d tokens", a->a_rows);
-    return launch_rows16<Fmt::I8, true, true>(p, s);
+    return launch_rows16<Fmt::I8, true, true>(p, live, s);
   }
   // a dense matrix: a tail expert alone (activations beyond that kernel's 32-bit offsets stay here)
   if (a->variant == 0 && a->rows == 0 && !swiglu && dense_gemm_i8_reaches(a->a_rows, a->k)) return dense_gemm_i8(a, s);
@@ -599,8 +610,8 @@ int stream_gemm_i8(const kmoe_gemm_i8_args* a, hipStream_t s, const StreamScan* 
   }
   switch (mf) {
     case 1:
-      return swiglu ? launch_rows16<Fmt::I8, true, false>(p, s)
-                    : launch_rows16<Fmt::I8, false, false>(p, s);
+      return swiglu ? launch_rows16<Fmt::I8, true, false>(p, live, s)
+                    : launch_rows16<Fmt::I8, false, false>(p, live, s);
     case 2:
       return swiglu ? launch_stream<Fmt::I8, 2, 2, true, 4>(p, s) : launch_stream<Fmt::I8, 2, 2, false, 4>(p, s);
     case 4:
@@ -619,27 +630,29 @@ int stream_gemm_fp8(const kmoe_gemm_fp8_args* a, hipStream_t s, const StreamScan
                        a->tail_src0, a->act_dtype == KMOE_DT_F16, 0, scan ? *scan : StreamScan{}, StreamQuant{},
                        nullptr, 0, 0, 0, 0, 0, slots_of(scan, slots)};
   const bool swiglu = a->act == KMOE_ACT_SWIGLU;
+  const int live = expected_rows(a->rows, a->rows_hint);
   if (scan) {
     if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
-    return launch_rows16<Fmt::F8, true, true>(p, s);
+    return launch_rows16<Fmt::F8, true, true>(p, live, s);
   }
-  return swiglu ? launch_rows16<Fmt::F8, true, false>(p, s) : launch_rows16<Fmt::F8, false, false>(p, s);
+  return swiglu ? launch_rows16<Fmt::F8, true, false>(p, live, s) : launch_rows16<Fmt::F8, false, false>(p, live, s);
 }
 
 int stream_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s, const StreamScan* scan, const StreamSlots* slots) {
   const bool half = a->act_dtype == KMOE_DT_F16;
   const StreamSlots columns = slots_of(scan, slots);
+  const int live = expected_rows(a->rows, a->rows_hint);
   const StreamParams p{reinterpret_cast<const int8_t*>(a->a), a->lda * 2, 64, 0, nullptr, a->row_src, a->src_div,
                        reinterpret_cast<const int8_t*>(a->w), nullptr, a->lod, a->E, a->n, a->k * 2, a->y, a->ldy, nullptr,
                        nullptr, nullptr, 0, 0, 0, half, 0, scan ? *scan : StreamScan{}, StreamQuant{},
-                       nullptr, 0, 0, 0, 0, 0, columns, columns.n == 0 && expected_rows(a->rows, a->rows_hint) < 3ll * a->E};
+                       nullptr, 0, 0, 0, 0, 0, columns, columns.n == 0 && live < 3ll * a->E};
   const bool swiglu = a->act == KMOE_ACT_SWIGLU;
   if (scan) {
     if (int rc = check_scan(scan, swiglu, a->variant, a->row_src, a->rows)) return rc;
-    return half ? launch_rows16<Fmt::F16, true, true>(p, s) : launch_rows16<Fmt::BF16, true, true>(p, s);
+    return half ? launch_rows16<Fmt::F16, true, true>(p, live, s) : launch_rows16<Fmt::BF16, true, true>(p, live, s);
   }
-  if (half) return swiglu ? launch_rows16<Fmt::F16, true, false>(p, s) : launch_rows16<Fmt::F16, false, false>(p, s);
-  return swiglu ? launch_rows16<Fmt::BF16, true, false>(p, s) : launch_rows16<Fmt::BF16, false, false>(p, s);
+  if (half) return swiglu ? launch_rows16<Fmt::F16, true, false>(p, live, s) : launch_rows16<Fmt::F16, false, false>(p, live, s);
+  return swiglu ? launch_rows16<Fmt::BF16, true, false>(p, live, s) : launch_rows16<Fmt::BF16, false, false>(p, live, s);
 }
 
 // 16-row launches split K two ways and keep one step (128 values) of loads in flight per wave: fewer registers and more
