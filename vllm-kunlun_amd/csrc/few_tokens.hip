@@ -43,7 +43,10 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
   constexpr int V = FMT == Fmt::F8 ? 2 : 1;   // 1 KB blocks of weights per step
   constexpr int AV = W4 ? 4 : V;              // 16-byte vectors of activations per lane and step ...
   constexpr int kAVStride = W4 ? 16 : 64, kALane = W4 ? 64 : 16, kAStep = W4 ? 256 : 64 * V;
-  constexpr int D = FMT == Fmt::F8 ? 4 : (few_wide_i8(FMT, kVecs) ? 12 : 8);  // steps in flight (a multiple of the four chains)
+  // steps in flight (a multiple of the four chains; 4-bit, whose chains are a step's own: three, which hide the unpacking, are fewer registers than
+  // eight and less code to bring in. Layer, us, eight / four / three / two: Qwen3 dims 2 tokens 17.8 / 17.4 / 17.2 / 17.2, 6 36.7 / 35.6 / 35.4 / 35.2,
+  // Kimi-K2 dims 1 46.9 / 45.0 / 45.0 / 45.3, 160 experts of [5120 x 1536] 2 42.8 / 40.4 / 40.0 / 40.0, 64 of [4096 x 2048] 1 29.6 / 29.7 / 30.0 / 30.8)
+  constexpr int D = W4 ? 3 : FMT == Fmt::F8 ? 4 : (few_wide_i8(FMT, kVecs) ? 12 : 8);
   extern __shared__ __attribute__((aligned(16))) int8_t rows_lds[];  // [wave][few_row_pitch]
   __shared__ float y_lds[kFewMaxWaves][16];
   __shared__ float w_lds[kFewMaxWaves];
