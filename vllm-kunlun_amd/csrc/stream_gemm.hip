@@ -505,8 +505,8 @@ int launch_stream(const StreamParams& p, hipStream_t s) {
 // 16-bit gate_up launches keep four steps in flight, whose weights are twice the bytes and nothing to work on (layer, us, two steps / four: Qwen3 dims bf16
 // 5 tokens 65.6 / 64.2, 12 119.0 / 117.6, 20 with +2.0 on the logits of 8 experts 111.4 / 108.6, 110 196.6 / 194.1; int8 12 73.3 / 74.6), but not on the
 // longest rows (16 experts of [8192 x 8192], top 2, 3 tokens 193 / 199, 12 441 / 442).
-// A layer too large for the first rule, with a column per pair: K split four ways at full depth in the gate_up launch, and in a down launch of
-// 16-bit weights on fewer than 64 columns. gate_up launch, us, two ways / four: DeepSeek-V3 dims int8 6 tokens 210 / 207, 8 265 / 262, fp8 4 155 / 150; 160
+// A layer too large for the first rule, with a column per pair: K split four ways at full depth in the gate_up launch (fp8: on fewer than 128 columns;
+// DeepSeek-V3 dims, layer, 23 tokens 854.5 / 858.3), and in a down launch of 16-bit weights on fewer than 64 columns. gate_up launch, us, two ways / four: DeepSeek-V3 dims int8 6 tokens 210 / 207, 8 265 / 262, fp8 4 155 / 150; 160
 // experts of [3072 x 5120], top 6, int8 5 tokens 74 / 71, bf16 24 456 / 440; 64 of [4096 x 4096], top 8, bf16 7 215 / 203. Down launch, bf16: 64
 // experts of [4096 x 2048] 24 columns 65 / 59, 56 107 / 101, 160 of [5120 x 1536] 36 85 / 85, 72 145 / 152, 144 218 / 261; int8: DeepSeek-V3 dims 24 columns 60
 // / 58.5, 64 of [6144 x 3072] 28 72 / 76, 64 of [4096 x 2048] 32 41.7 / 43.3, DeepSeek-V3 dims 128 236 / 255.
@@ -524,7 +524,7 @@ int launch_rows16(const StreamParams& p, int rows, hipStream_t s) {
   constexpr bool k16 = FMT == Fmt::BF16 || FMT == Fmt::F16;
   if (k16 && SWIGLU && ksteps >= 24 && ksteps < 256 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, k16 ? 4 : 2, 4, SCAN>(p, s);
   if (ksteps >= 24 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, 2, 4, SCAN>(p, s);
-  if (ksteps >= 24 && p.slots.n > 0 && (SWIGLU || (k16 && p.slots.n < 64)))
+  if (ksteps >= 24 && p.slots.n > 0 && (SWIGLU ? FMT != Fmt::F8 || p.slots.n < 128 : k16 && p.slots.n < 64))
     return launch_stream<FMT, 1, 2, SWIGLU, 4 / V, 4, SCAN>(p, s);
   if constexpr (SWIGLU && FMT == Fmt::I8) {
     if (ksteps >= 24 && ksteps <= 64 && rows >= 4ll * p.E) return launch_stream<FMT, 1, 4, SWIGLU, 4, 2, SCAN>(p, s);
