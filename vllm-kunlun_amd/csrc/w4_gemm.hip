@@ -262,8 +262,10 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
     }
   }
   auto first_group = [&](int kb) __attribute__((always_inline)) { return (4 * (kb & ~(CB - 1))) >> p.gs_shift; };  // of the chunk of block kb
-  auto dma_s = [&](int kb) __attribute__((always_inline)) {  // the chunk that begins with block kb
-    const uint32_t at = kb < kblocks ? static_cast<uint32_t>(first_group(kb)) * 32u : kRange;
+  // the chunk that begins with block kb, which has to exist: the descriptor ends with the expert's scales, and a scalar offset beyond its
+  // end would wrap in the range check (limit minus offset); what a last chunk has beyond it is not fetched
+  auto dma_s = [&](int kb) __attribute__((always_inline)) {
+    const uint32_t at = static_cast<uint32_t>(first_group(kb)) * 32u;
 #pragma unroll
     for (int j = 0; j < NS; ++j) buffer_load16_to_lds(s_rsrc, (lds_ptr_t)&lds_s[CHUNKED ? wave : 0][kb / CB & 1][j * 1024], s_off[j], at);
   };
@@ -344,7 +346,7 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (CHUNKED) {
-      if ((kb & (CB - 1)) == 0) dma_s(kb + CB);
+      if ((kb & (CB - 1)) == 0 && kb + CB < kblocks) dma_s(kb + CB);  // (the waits do not count on these copies)
     }
     dma_a((u + R - 1) % R, kb + R - 1);
     load_w((u + R - 1) % R, kb + R - 1);
