@@ -269,11 +269,16 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
 #pragma unroll
     for (int j = 0; j < NS; ++j) buffer_load16_to_lds(s_rsrc, (lds_ptr_t)&lds_s[CHUNKED ? wave : 0][kb / CB & 1][j * 1024], s_off[j], at);
   };
-  // the scales of block kb, which the caller has seen land in LDS; usable behind the wait for a younger LDS read
+  // the scales of block kb, which the caller has seen land in LDS; usable behind the wait for a younger LDS read and hold_s(), which keeps their
+  // registers theirs until then, also where nothing uses the values (the last block asks for the next one's, too)
   auto request_s = [&](int kb) __attribute__((always_inline)) {
     const uint32_t at = s_lds + static_cast<uint32_t>((kb / CB & 1) * kScaleBytes + (((4 * kb + lg) >> p.gs_shift) - first_group(kb)) * 32 + li * 2);
 #pragma unroll
     for (int f = 0; f < NF; ++f) asm volatile("ds_read_u16 %0, %1" : "=v"(sbuf[0][f]) : "v"(at + static_cast<uint32_t>(f * s_frag)) : "memory");
+  };
+  auto hold_s = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) asm volatile("" : "+v"(sbuf[0][f])::"memory");
   };
   auto load_w = [&](int slot, int kb) __attribute__((always_inline)) {
     const bool live = kb < kblocks;
@@ -299,10 +304,6 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
   // supplies values 32 lg + 8 t + [0, 8) of the block, i.e. vector 4 lg + t of the row's 16.
   auto compute = [&](int kb, auto slot_tag) __attribute__((always_inline)) {
     constexpr int slot = decltype(slot_tag)::value, ss = CHUNKED ? 0 : slot;
-    if constexpr (CHUNKED) {  // (asked for a block ago; the reads behind them have landed)
-#pragma unroll
-      for (int f = 0; f < NF; ++f) asm volatile("" : "+v"(sbuf[0][f])::"memory");
-    }
     const W4Scale<F16> sc[NF] = {W4Scale<F16>(sbuf[ss][0]), W4Scale<F16>(sbuf[ss][1]), W4Scale<F16>(sbuf[ss][2]), W4Scale<F16>(sbuf[ss][3])};
     if constexpr (CHUNKED) {
       __builtin_amdgcn_sched_barrier(0);
@@ -339,6 +340,7 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
       mfma4_if_live<F16, mf>(acc[mf], wv, af[i % 3], live_frags);
       __builtin_amdgcn_sched_barrier(0);  // (all the unpacking of a block at once would not fit the registers)
     });
+    if constexpr (CHUNKED) hold_s();
   };
   auto stage = [&](int kb, auto u_tag) __attribute__((always_inline)) {
     constexpr int u = decltype(u_tag)::value;
@@ -363,6 +365,7 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
     vmem_wait<0>();
     request_s(0);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    hold_s();
   }
   // (no exit inside the body: as one basic block it fits the registers)
   int kb = 0;
