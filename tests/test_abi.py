@@ -258,6 +258,31 @@ def test_few_rows_per_expert_decide_the_packed_gate_up_kernel(L, k, most):
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="names the kernel a launch would take, on addresses that are not memory")
+@pytest.mark.parametrize("E,n,k,top,most", [
+    (384, 4096, 7168, 8, 16), (160, 3072, 5120, 6, 16),  # long rows: tokens that one pass holds, and at most a row per expert
+    (64, 6144, 6144, 4, 16), (64, 4096, 7168, 8, 8),
+    (128, 1536, 2048, 8, 48), (64, 5120, 3584, 6, 42),   # shorter: three passes, and at most four rows
+    (32, 4096, 8192, 4, 8), (32, 2048, 2048, 4, 32)])    # few workgroups
+def test_tokens_that_share_experts_decide_the_packed_gate_up_kernel(L, E, n, k, top, most):
+    """A packed gate_up launch for a number of tokens, which the rows' sources say: where no expert can need more than a pass or a few, or tiles
+    would leave the GPU idle, the streaming kernel, which splits the contraction, up to a row per expert (rows of at most 4096 values: four)."""
+    def kernel(tokens):
+        g = L.GemmW4Args()
+        for f in ("a", "w", "w_scale", "lod", "y", "row_src"):
+            setattr(g, f, 0x10000)
+        g.E, g.n, g.k, g.rows, g.lda, g.ldy, g.src_div = E, n, k, tokens * top, k, n // 2, top
+        g.group_size, g.act, g.w_layout = 32, 1, L.KMOE_W_TILED
+        L.lib.kmoe_trace_kernels(1)
+        assert L.lib.kmoe_grouped_gemm_w4a16(g, None) == -5
+        L.lib.kmoe_trace_kernels(0)
+        return L.lib.kmoe_traced_kernels().decode()
+
+    for tokens in (1, 2, 5, 8, 13, most):
+        assert ("stream_gemm_kernel" if tokens <= most else "w4_tile_kernel") in kernel(tokens)
+    assert "w4_tile_kernel" in kernel(most + 1)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="names the kernel a launch would take, on addresses that are not memory")
 def test_dense_products_beyond_32_bit_offsets_stay_on_the_streaming_kernel(L):
     """kmoe_grouped_gemm_i8 with a tail matrix alone: the split-K kernel where its 32-bit offsets reach all activations (asked for
     the compute units first, which fails without a GPU), else the streaming kernel (noted before its launch fails)."""

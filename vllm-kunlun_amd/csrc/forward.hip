@@ -169,13 +169,9 @@ bool routed_streams(const kmoe_moe_args* a) {
     case KMOE_FMT_BF16:
       return streams_bf16(static_cast<int>(rows), a->E, a->H) && streams_bf16(static_cast<int>(rows), a->E, a->I) &&
              !a->w13_bias && !a->w2_bias && a->activation != KMOE_ACT_SWIGLUOAI;
-    default: {
-      // (up to kFewRouted tokens on fewer pairs than experts: the launches that take a layer of a few tokens as a whole)
-      const int pairs = a->M * a->K;
-      return ((a->M <= kFewRouted && pairs <= a->E) ||
-              w4_gate_up_streams(pairs, a->E_global > a->E ? static_cast<int>(rows) : 0, a->E, a->H)) &&
+    default:
+      return w4_gate_up_streams(a->M * a->K, a->E_global > a->E ? static_cast<int>(rows) : 0, a->M, a->E, 2 * a->I, a->H) &&
              w4_rows_fit_32(a->M, a->H, a->H) && w4_rows_fit_32(static_cast<long long>(a->M) * a->K, a->I, a->I);
-    }
   }
 }
 

@@ -111,7 +111,7 @@ int grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* args, kmoe_stream_t stre
 // offsets reach every source row.
 int stream_gemm_w4(const kmoe_gemm_w4_args* args, hipStream_t stream, int passes, const StreamScan* scan,
                    const StreamSlots* slots, bool rows_fit_32);
-bool w4_gate_up_streams(int rows, int rows_hint, int E, int k);
+bool w4_gate_up_streams(int rows, int rows_hint, long long tokens, int E, int n, int k);
 // Whether a 32-bit byte offset reaches every value of `rows` 16-bit activation rows (and a row's worth beyond, what the
 // kernels' K steps add to the offset of a row).
 inline bool w4_rows_fit_32(long long rows, int64_t lda, int k) {

@@ -434,16 +434,24 @@ __global__ __launch_bounds__(256) void tile_scales_kernel(const uint16_t* __rest
 
 }  // namespace
 
-// Layer, us, 16-row passes of the streaming kernel (which sorts the pairs on the way) against 16-row tiles (whose launch needs
-// the sort's, and which read a scale once per chunk of the contraction, not per block). Qwen3 dims: 12 tokens 53.7 / 54.4, 20
-// (2 rows per expert) 61.0 / 65.0, 32 (2) 69.9 / 70.5, 40 (3) 76.0 / 71.7, 48 (3) 73.4 / 72.7, 64 (4) 72.8 / 72.3; with eight experts
-// chosen far more often, where the streaming kernel reads an expert's weights again for every 16 rows, 16 tokens 48.9 / 50.8, 24 57.1 /
-// 55.5, 32 63.6 / 62.9, 64 86.1 / 75.1. With a long K the sort's launch is little and the scales are more: Kimi-K2 dims, 5 tokens
-// 187 / 198, 8 (64 rows on 384 experts) 277 / 273, 10 334 / 353, 12 389 / 387, 16 500 / 482, 24 682 / 636, 32 837 / 778, 45 992 / 934,
-// and 45 with eight such experts 779 / 724.
-bool w4_gate_up_streams(int rows, int rows_hint, int E, int k) {
+// Layer, time on 16-row tiles (whose launch needs the sort's, and which read a scale once per chunk of the contraction) over time on 16-row passes of
+// the streaming kernel (which sorts the pairs on the way and splits the contraction over its waves): even load / +2.0 on the logits of eight
+// experts / every token on the same experts.
+// Rows beyond 4096 values. Up to 16 tokens no expert needs a second pass, and tiles lack workgroups where tokens share experts: 160 experts of
+// [5120 x 1536], top 6, 8 tokens 1.09 / 1.08 / 1.58, 64 of [6144 x 3072], top 4, 10 1.03 / 1.10 / 1.59, 32 of [8192 x 2048], top 4, 6 1.19 / 1.14 /
+// 1.92, Kimi-K2 dims 10 1.06 / 1.02 / 1.36, 16 0.97 / 1.03 / 1.08. From 17 on: Kimi-K2 dims 20 0.95 / 0.97 / 0.86, 32 0.96 / 0.92 / 0.68, 160 of [5120 x
+// 1536] 24 0.98 / 0.88 / 1.00, 160 of [6144 x 2560], top 8, 20 0.96 / 0.97 / 0.77.
+// Shorter rows, where the sort's launch counts: only from 49 tokens on, when an expert that most of them choose takes four passes. Qwen3 dims 20
+// 1.08 / 1.01 / 0.84, 40 1.01 / 0.97 / 0.69, 49 to 64 1.00 / 0.90 to 0.82 / 0.64 to 0.53; 128 of [3072 x 1024], top 8, 36 1.03 / 0.99 / -, 56 0.99 / 0.92 /
+// 0.61; 64 of [3584 x 2560], top 6, 40 1.05 / 0.97 / 0.75.
+// Few workgroups, even load: 32 of [2048 x 1024], top 4, (256) 20 to 32 tokens 1.09, 16 of [8192 x 4096], top 2, (512) 8 1.18, 12 1.08, 32 of [7168 x
+// 2048], top 8, 5 tokens (350) 1.10, 8 (450) 1.04.
+bool w4_gate_up_streams(int rows, int rows_hint, long long tokens, int E, int n, int k) {
   const int expected = expected_rows(rows, rows_hint);
-  return k > 4096 ? expected <= E / 4 : ceil_div(expected, E) <= 2;
+  const int avg = ceil_div(expected, E);
+  const bool fills = static_cast<long long>(min(expected, E)) * ceil_div(n / 2, kWaves * 32) > 512;  // two workgroups a CU
+  if (k > 4096) return avg <= 1 && !(tokens > 16 && expected > E / 4 && fills);
+  return avg <= 4 && !(tokens > 48 && avg > 2 && fills);
 }
 
 }  // namespace kmoe
@@ -514,7 +522,8 @@ int kmoe::grouped_gemm_w4a16_checked(const kmoe_gemm_w4_args* a, kmoe_stream_t s
     // 176, 1800 (113) 225 / 251 / 224, 2048 (128) 252 / 263 / 262, 2300 (144) 275 / 270 / 290, 2560 (160) 291 / 285 / 305,
     // 3072 (192) 333 / 335 / 324, 8192 (512) 776 / 756 / 716.
     const int avg = ceil_div(expected_rows(a->rows, a->rows_hint), a->E);
-    if (scan || slots || (swiglu && w4_gate_up_streams(a->rows, a->rows_hint, a->E, a->k))) mf = 1;
+    const long long tokens = a_rows >= 0 ? a_rows : ceil_div(a->rows, a->src_div);
+    if (scan || slots || (swiglu && w4_gate_up_streams(a->rows, a->rows_hint, tokens, a->E, a->n, a->k))) mf = 1;
     else if (!tile_ok) mf = avg <= 13 ? 1 : (avg <= 20 ? 2 : 4);
     else if (avg <= 22) mf = avg <= 8 ? 16 : 32;
     else if (avg <= 112) mf = avg <= 50 ? 64 : (avg <= 76 ? 96 : 128);
