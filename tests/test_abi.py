@@ -283,6 +283,23 @@ def test_tokens_that_share_experts_decide_the_packed_gate_up_kernel(L, E, n, k, 
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="names the kernel a launch would take, on addresses that are not memory")
+@pytest.mark.parametrize("E,n,k,split", [(128, 2048, 3072, 4), (129, 2048, 3072, 2), (128, 8192, 3072, 2), (64, 8192, 3584, 4), (64, 8192, 4992, 4),
+                                         (64, 16384, 3584, 2), (64, 16384, 4992, 2), (64, 16384, 5120, 4), (8, 8192, 2944, 2)])
+def test_many_workgroups_of_short_work_split_packed_rows_two_ways(L, E, n, k, split):
+    """A packed gate_up launch on the streaming kernel: rows from 3072 values on split four ways, shorter than 3584 and 5120 values only while
+    that makes no more than 4096 and 8192 workgroups."""
+    g = L.GemmW4Args()
+    for f in ("a", "w", "w_scale", "lod", "y"):
+        setattr(g, f, 0x10000)
+    g.E, g.n, g.k, g.rows, g.lda, g.ldy, g.src_div = E, n, k, 4, k, n // 2, 1
+    g.group_size, g.act, g.w_layout = 32, 1, L.KMOE_W_TILED
+    L.lib.kmoe_trace_kernels(1)
+    assert L.lib.kmoe_grouped_gemm_w4a16(g, None) == -5
+    L.lib.kmoe_trace_kernels(0)
+    assert f"K split {split}" in L.lib.kmoe_traced_kernels().decode()
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="names the kernel a launch would take, on addresses that are not memory")
 def test_dense_products_beyond_32_bit_offsets_stay_on_the_streaming_kernel(L):
     """kmoe_grouped_gemm_i8 with a tail matrix alone: the split-K kernel where its 32-bit offsets reach all activations (asked for
     the compute units first, which fails without a GPU), else the streaming kernel (noted before its launch fails)."""

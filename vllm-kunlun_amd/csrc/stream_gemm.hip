@@ -658,20 +658,33 @@ int stream_gemm_bf16(const kmoe_gemm_bf16_args* a, hipStream_t s, const StreamSc
 // 16-row launches split K two ways and keep one step (128 values) of loads in flight per wave: fewer registers and more
 // waves hide the unpacking and the loads of each other better than a deeper queue does (Qwen3, 64 tokens, layer, steps
 // in flight x split: 1x1 81.7 us, 2x1 81.9, 3x1 83.3, 1x2 78.8, 2x2 81.5; Kimi-K2 dimensions, 128 tokens: 1584 / 1577 /
-// 1606 / 1568 / 1598). A gate_up launch of long rows splits K four ways, and so that there are no more workgroups than before, each of which
-// finds its rows first, its waves take twice the channels - where that would leave fewer than four for a CU, the same channels. Layer, us, two
-// ways / four with twice the channels / four: Kimi-K2 dims 2 tokens 86.5 / 82.0 / 83.7, 4 150.7 / 144.4 / 148.4, 7 247.7 / 238.9 / -, 12 390.7 / 374.5 /
-// 389.4; 160 experts of [3072 x 5120], top 6, 3 tokens 60.4 / 57.6 / 55.8, 6 96.8 / 91.0 / 90.2; 128 of [3072 x 4096] 6 94.4 / 92.0 / 92.1, 32 209.8 / 205.7 /
-// -; 128 of [2048 x 3072] 10 77.8 / 75.9 / -, 20 103.1 / 102.4 / -; four ways, shorter rows: Qwen3 dims 5 33.2 / 33.1 / 32.7, 7 41.9 / 44.2 / 43.1, 24 66.0 / 68.4 /
-// 68.4. Up to 32 columns of a launch with a column per pair do not fill the chip: gate_up launches keep two steps there (one
-// token 22.5 -> 21.1 and 62 -> 59 us), down launches split K four ways (the down launch of Kimi-K2 dims, 2 tokens 31.6 -> 28.6 us, 4 54.4 -> 51.7, 6 - 48
-// columns - 70.5 -> 74.2; 64 experts of [6144 x 3072], 8 columns 21.6 -> 22.3, 16 35.3 -> 31.9). A caller's variant, and rows beyond the reach of the split launches' 32-bit
-// offsets, keep one wave per K range: the tile kernel's order of sums, and rows anywhere in memory.
+// 1606 / 1568 / 1598).
+//
+// A gate_up launch of long rows splits K four ways (kW4LongSteps), and so that there are no more workgroups than before, each of which finds its
+// rows first, its waves take twice the channels - where that would leave fewer than four for a CU, the same channels. Layers as [hidden x
+// intermediate], time over the time with two ways, even load / +2.0 on the logits of eight experts / every token on the same experts:
+//   Kimi-K2 dims 2 tokens 0.97 / 0.97 / 0.99, 5 0.95 / 0.95 / 0.95, 12 0.97 / 0.96 / 1.00; 160 of [5120 x 1536], top 6, 3 0.96 / 0.91 / 0.93, 6 0.97 /
+//   0.95 / 0.94; 128 of [4096 x 1536], top 8, 5 0.95 / 0.99 / 0.96, 24 1.00 / 0.97 / 0.89; 64 of [4096 x 2048], top 8, 5 0.97 / 1.03 / 1.00, 24 1.01 / 0.95 /
+//   0.82; 32 of [4096 x 4096], top 4, 8 1.01 / 1.03 / 0.99, 24 1.01 / 0.95 / 0.90; 256 of [3072 x 512], top 8, 5 0.89 / 0.89 / 0.81.
+// Columns of pairs whose expert an earlier column serves ask for their first weights in vain, and twice the channels are twice of them: with many
+// workgroups of short work (below 40 and below 28 steps) two ways stay. Four ways there: 128 of [3072 x 4096], top 8, 8 tokens (64 columns of 128
+// workgroups) 1.03 / 1.02 / 1.10, 16 (a column per expert) 1.05 / 1.06 / 1.01, 160 of [3072 x 5120], top 6, 10 (60 of 160) 1.02 / 1.02 / 1.09, but 5 (30 of 160)
+// 0.99 / 0.98 / 0.98; 128 of [4096 x 6144], top 6, 12 (72 of 192) 1.00 / 1.02 / 1.07, but 5 (30 of 192) 0.97 / 0.98 / 0.97; 64 of [3584 x 8192], top 8, 6 (48 of 256)
+// 1.02 / 1.03 / 1.10, but 4 (32 of 256) 0.99 / 0.98 / 0.98. Rows of 2048 values lose 0 to 6 % (Qwen3 dims 7 tokens 41.9 -> 43.1 us, 24 66.0 -> 68.4).
+//
+// Up to 32 columns of a launch with a column per pair do not fill the chip: gate_up launches keep two steps in flight there (one token 22.5 -> 21.1 and
+// 62 -> 59 us), down launches split K four ways (layer: Kimi-K2 dims 2 tokens 0.98 of the time, 3 0.98, 64 of [6144 x 3072], top 4, 3 0.96 / 0.98 / 0.94, but
+// 48 columns of Kimi-K2 dims: launch 70.5 -> 74.2 us).
+//
+// A caller's variant, and rows beyond the reach of the split launches' 32-bit offsets, keep one wave per K range: the tile kernel's order of sums, and
+// rows anywhere in memory.
 constexpr int kW4LongSteps = 24;  // of 128 values
 template <Fmt FMT>
 int stream_w4_shape(const StreamParams& p, bool swiglu, bool scan, int passes, bool split, hipStream_t s) {
-  if (passes == 1 && split && swiglu && p.kbytes / 64 >= kW4LongSteps) {
-    if (static_cast<long long>(ceil_div(p.n / 2, 32)) * (p.slots.n > 0 ? p.slots.n : p.E) < 1024)
+  const int steps = p.kbytes / 64;
+  const long long four_ways = static_cast<long long>(ceil_div(p.n / 2, 32)) * (p.slots.n > 0 ? p.slots.n : p.E);  // workgroups then
+  if (passes == 1 && split && swiglu && steps >= kW4LongSteps && (steps >= 40 || four_ways <= (steps >= 28 ? 8192 : 4096))) {
+    if (four_ways < 1024)
       return scan ? launch_stream<FMT, 1, 2, true, 1, 4, true>(p, s) : launch_stream<FMT, 1, 2, true, 1, 4>(p, s);
     return scan ? launch_stream<FMT, 1, 4, true, 1, 4, true>(p, s) : launch_stream<FMT, 1, 4, true, 1, 4>(p, s);
   }
