@@ -46,6 +46,18 @@ def test_rows_of_every_length(fmt, I, dtype):
         assert rel_l2(part, whole[:M]) <= 4e-3
 
 
+@pytest.mark.parametrize("M,K,H,I,steps", [(1, 2, 4096, 2048, 8), (4, 2, 4096, 2048, 8), (1, 4, 2048, 512, 8), (2, 4, 2048, 896, 3), (3, 3, 512, 1152, 8),
+                                           (1, 8, 4096, 1920, 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_packed_steps_in_flight(M, K, H, I, steps, dtype):
+    """4-bit weights: deep rings where the launch has no more waves than a row values."""
+    from vllm_kunlun_amd import synth
+    sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], M=M, E=40, K=K, H=H, I=I, quant="w4"), "cuda", seed=I, dtype=dtype)
+    out, named = _named(lambda: _call(sl))
+    assert f"{steps} steps in flight>" in named[named.index("few_down_kernel"):], named
+    _check(sl, out)
+
+
 @pytest.mark.parametrize("fmt", ["int8", "fp8"])
 @pytest.mark.parametrize("K,fused", [(1, True), (15, True), (16, False)])
 @pytest.mark.parametrize("scales", [(1.0, 1.0), (0.5, 0.75)])

@@ -34,8 +34,16 @@ __device__ inline bool past_caches(size_t pairs, int channels, int row_bytes) {
 
 constexpr bool few_wide_i8(Fmt f, int vecs) { return f == Fmt::I8 && vecs > 2; }
 
+// Steps of weights in flight (a multiple of the four chains; 4-bit, whose chains are a step's own: three, which hide the unpacking, are fewer
+// registers than eight and less code to bring in, but eight - DEEP - where the launch has fewer waves than a row values, long rows and too few waves to
+// keep the memory busy with three. Layer, time with three over time with eight, even load: Qwen3 dims 2 tokens 0.97, 6 0.96, Kimi-K2 dims 1 0.94, 160
+// experts of [5120 x 1536] (hidden x intermediate), top 6, 1 0.97, 256 of [3072 x 512], top 8, 3 0.95, but 32 of [4096 x 2048], top 2, 1 to 4 tokens 1.05 / 1.02 /
+// 1.01 / 1.01, 32 of [2048 x 1024], top 4, 1 and 2 1.03 / 1.02, 3 0.99, 64 of [4096 x 2048], top 8, 1 1.015, 2 0.97)
+constexpr int few_down_steps(Fmt f, int vecs, bool deep) {
+  return f == Fmt::W4 || f == Fmt::W4H ? (deep ? 8 : 3) : (f == Fmt::F8 ? 4 : (few_wide_i8(f, vecs) ? 12 : 8));
+}
 // kVecs: vectors of 8 values a lane holds of its row (rows of up to 512 kVecs values)
-template <Fmt FMT, int kVecs>
+template <Fmt FMT, int kVecs, bool DEEP>
 __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 5) void few_down_kernel(const FewDown p) {
   using acc_t = typename std::conditional<FMT == Fmt::I8, v4i, v4f>::type;
   constexpr bool W4 = FMT == Fmt::W4 || FMT == Fmt::W4H;
@@ -43,10 +51,7 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
   constexpr int V = FMT == Fmt::F8 ? 2 : 1;   // 1 KB blocks of weights per step
   constexpr int AV = W4 ? 4 : V;              // 16-byte vectors of activations per lane and step ...
   constexpr int kAVStride = W4 ? 16 : 64, kALane = W4 ? 64 : 16, kAStep = W4 ? 256 : 64 * V;
-  // steps in flight (a multiple of the four chains; 4-bit, whose chains are a step's own: three, which hide the unpacking, are fewer registers than
-  // eight and less code to bring in. Layer, us, eight / four / three / two: Qwen3 dims 2 tokens 17.8 / 17.4 / 17.2 / 17.2, 6 36.7 / 35.6 / 35.4 / 35.2,
-  // Kimi-K2 dims 1 46.9 / 45.0 / 45.0 / 45.3, 160 experts of [5120 x 1536] 2 42.8 / 40.4 / 40.0 / 40.0, 64 of [4096 x 2048] 1 29.6 / 29.7 / 30.0 / 30.8)
-  constexpr int D = W4 ? 3 : FMT == Fmt::F8 ? 4 : (few_wide_i8(FMT, kVecs) ? 12 : 8);
+  constexpr int D = few_down_steps(FMT, kVecs, DEEP);
   extern __shared__ __attribute__((aligned(16))) int8_t rows_lds[];  // [wave][few_row_pitch]
   __shared__ float y_lds[kFewMaxWaves][16];
   __shared__ float w_lds[kFewMaxWaves];
@@ -258,18 +263,23 @@ __global__ __launch_bounds__(kFewMaxWaves* kWave, few_wide_i8(FMT, kVecs) ? 4 : 
 
 // (the most rows there may be - 16 of 2048 16-bit values, 64.25 KB - fit a CU's 160 KB twice, with what the kernel holds besides)
 static_assert(kFewMaxWaves * few_row_pitch(kFewMaxI, 2, false) + kFewMaxWaves * 17 * 4 <= 80 * 1024);
-template <Fmt FMT, int kVecs>
+template <Fmt FMT, int kVecs, bool DEEP = false>
 int launch_few_down(const FewDown& p, hipStream_t s) {
   const int waves = p.K + (p.w_tail ? 1 : 0);
   const size_t bytes = static_cast<size_t>(waves) * few_row_pitch(p.I, FMT == Fmt::I8 || FMT == Fmt::F8 ? 1 : 2, FMT == Fmt::F8);
   if (tracing_kernels())
-    note_kernel("few_down_kernel<%s>, %d waves: quantisation, down projection and combine of a token's 16 channels", fmt_name(FMT), waves);
-  hipLaunchKernelGGL((few_down_kernel<FMT, kVecs>), dim3(p.H / 16, p.M), dim3(waves * kWave), bytes, s, p);
+    note_kernel("few_down_kernel<%s, %d steps in flight>, %d waves: quantisation, down projection and combine of a token's 16 channels", fmt_name(FMT),
+                few_down_steps(FMT, kVecs, DEEP), waves);
+  hipLaunchKernelGGL((few_down_kernel<FMT, kVecs, DEEP>), dim3(p.H / 16, p.M), dim3(waves * kWave), bytes, s, p);
   return check_launch("kmoe_moe_forward (down + combine)");
 }
 
 template <Fmt FMT>
 int launch_few_down(const FewDown& p, hipStream_t s) {
+  if constexpr (FMT == Fmt::W4 || FMT == Fmt::W4H) {
+    if (static_cast<long long>(p.H / 16) * p.M * p.K <= p.I)
+      return p.I <= 1024 ? launch_few_down<FMT, 2, true>(p, s) : launch_few_down<FMT, 4, true>(p, s);
+  }
   return p.I <= 1024 ? launch_few_down<FMT, 2>(p, s) : launch_few_down<FMT, 4>(p, s);
 }
 
