@@ -58,6 +58,16 @@ def test_packed_steps_in_flight(M, K, H, I, steps, dtype):
     _check(sl, out)
 
 
+@pytest.mark.parametrize("M,fused", [(6, True), (7, False), (8, False)])
+def test_packed_layers_whose_tokens_may_share_experts_end_apart(M, fused):
+    """Qwen3 dims, 4-bit: one launch at the end up to six tokens; with more, samples of one prompt would read shared weights too often."""
+    from vllm_kunlun_amd import synth
+    sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], M=M, quant="w4"), "cuda", seed=M)
+    out, named = _named(lambda: _call(sl))
+    assert (FUSED in named) == fused, named
+    _check(sl, out)
+
+
 @pytest.mark.parametrize("fmt", ["int8", "fp8"])
 @pytest.mark.parametrize("K,fused", [(1, True), (15, True), (16, False)])
 @pytest.mark.parametrize("scales", [(1.0, 1.0), (0.5, 0.75)])

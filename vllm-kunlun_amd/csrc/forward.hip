@@ -205,14 +205,15 @@ bool fold_shared(const kmoe_moe_args* a) {
 // Two bounds, both on what is read again. Under uniform routing, at about 6 MB a microsecond; layer, launches apart / in one, us, and
 // those MB:
 //   Qwen3 dims int8 1 token 23.7 / 18.9 (0), 4 42.5 / 36.6 (4), 8 60.4 / 56.6 (20), 10 64.9 / 62.2 (30), 12 74.4 / 74.0 (43);
-//   bf16 1 token 26.3 / 22.3, 8 89.9 / 88.3 (39), 12 116 / 118 (85); 4-bit 1 token 21.4 / 18.6, 6 39.4 / 35.4 (6), 8 44.0 / 40.5 (10), 10 48.8 / 45.6 (15);
+//   bf16 1 token 26.3 / 22.3, 8 89.9 / 88.3 (39), 12 116 / 118 (85); 4-bit 1 token 21.4 / 18.6, 6 39.4 / 35.4 (6);
 //   DeepSeek-V3 dims int8 1 token 95.3 / 87.5, 3 193.7 / 198.3 (40); fp8 1 token 95.3 / 88.6, 2 149 / 153 (18);
-//   Kimi-K2 dims 4-bit 1 token 59.6 / 57.4, 3 116.9 / 116.0 (2); 32 experts of [2048 x 1024], top 4, 4-bit 7 31.4 / 29.0 (9).
+//   Kimi-K2 dims 4-bit 1 token 59.6 / 57.4, 3 116.9 / 116.0 (2).
 // And with every token on the same experts (samples of one prompt), where the launch must not lose more than it gains under uniform
 // routing. There one token's weights come from the L2 of the XCD that read them for the token before (column blocks keep their XCD)
 // while an eighth of them fits its 4 MB, and from the memory-side cache beyond. Layer, us, apart / in one, uniform; same experts, and the MB:
 //   Qwen3 dims int8 10 tokens 65.4 / 61.5; 27.2 / 26.2 (113), bf16 7 84.6 / 81.8; 26.9 / 27.0 (151), 4-bit 6 40.6 / 37.0; 20.7 / 22.0 (31),
-//   8 44.0 / 40.5; 24.6 / 26.6 (44), 128 experts of [4096 x 1536], 4-bit 3 59.4 / 56.7; 30.8 / 33.7 (50), 160 of [5120 x 1536], top 6, 3 58.1 / 57.0; 35.9 / 40.6 (47);
+//   8 44.0 / 40.5; 24.6 / 26.6 (44; left apart, as 7 are: samples of one prompt would pay 8 %), 128 experts of [4096 x 1536], 4-bit 3 59.4 / 56.7; 30.8 / 33.7 (50),
+//   160 of [5120 x 1536], top 6, 3 58.1 / 57.0; 35.9 / 40.6 (47);
 //   128 experts of [3072 x 4096], int8 2 tokens 60.5 / 53.8; 40.8 / 36.0 (50), 3 82.3 / 76.8; 42.4 / 45.9 (101), bf16 2 102.6 / 99.4; 57.5 / 61.9
 //   (101), 4-bit 2 45.5 / 43.3; 29.9 / 31.0 (25), 3 62.8 / 60.9; 32.4 / 36.6 (50), fp8, 4 experts per token, 4 57.3 / 54.1; 29.3 / 28.2 (75);
 //   DeepSeek-V3 dims int8 2 tokens 125.4 / 125.1; 87.4 / 104.3 (132); Kimi-K2 dims 4-bit 2 82.7 / 82.0; 56.7 / 62.7 (59).
@@ -230,7 +231,7 @@ bool few_down_pays(const kmoe_moe_args* a, bool fold) {
   const double token = (a->K + (fold ? 1 : 0)) * bytes;
   const double same = (a->M - 1) * token;
   switch (a->format) {
-    case KMOE_FMT_W4A16: return again * bytes <= 10e6 && same <= 45e6;
+    case KMOE_FMT_W4A16: return again * bytes <= 6e6 && same <= 42e6;
     case KMOE_FMT_FP8_BLOCK: return again * bytes <= 6e6 && same <= 80e6;
     default: return again * bytes <= 32e6 && same <= (token <= 8 * (4u << 20) ? 160e6 : 110e6);
   }
