@@ -303,16 +303,22 @@ def test_packed_launches_on_long_rows_match_the_oracle(dims, shape, dtype):
 
 
 @pytest.mark.parametrize("fmt,dims,launches", [
-    ("int8", dict(M=7, E=256, K=4, H=1600, I=512), ["SiLU-mul, 4 steps in flight, K split 4"]),   # 25 steps
-    ("fp8", dict(M=7, E=256, K=4, H=3200, I=512), ["SiLU-mul, 2 steps in flight, K split 4"]),    # 25 steps
-    ("none", dict(M=9, E=64, K=6, H=4096, I=832), ["SiLU-mul, 4 steps in flight, K split 4", "plain, 4 steps in flight, K split 4"])], ids=str)
+    ("int8", dict(M=7, E=256, K=4, H=1600, I=512), ["SiLU-mul, 4 steps in flight, K split 2"]),   # 25 steps
+    ("fp8", dict(M=7, E=256, K=4, H=3200, I=512), ["SiLU-mul, 2 steps in flight, K split 2"]),    # 25 steps
+    ("none", dict(M=9, E=64, K=7, H=4096, I=2048), ["SiLU-mul, 4 steps in flight, K split 4", "plain, 4 steps in flight, K split 4"]),
+    ("none", dict(M=9, E=96, K=7, H=3040, I=2016), ["SiLU-mul, 4 steps in flight, K split 2", "plain, 4 steps in flight, K split 2"]),
+    ("none", dict(M=16, E=96, K=4, H=3072, I=2048), ["SiLU-mul, 4 steps in flight, K split 2", "plain, 4 steps in flight, K split 2"]),
+    ("none", dict(M=9, E=64, K=4, H=1024, I=512), ["SiLU-mul, 2 steps in flight, K split 4"]),
+    ("none", dict(M=16, E=48, K=4, H=2048, I=512), ["SiLU-mul, 4 steps in flight, K split 4"]),   # a column per expert
+    ("none", dict(M=16, E=48, K=4, H=2016, I=512), ["SiLU-mul, 2 steps in flight, K split 4"])], ids=str)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_columns_of_pairs_of_large_layers_match_the_oracle(fmt, dims, launches, dtype):
-    """Large layers of a few tokens, whose column-per-pair launches split K over four waves."""
+    """Layers of a few tokens, whose column-per-pair launches split K over four waves where they are large, have 16-bit weights, long rows and
+    few columns; steps in flight of smaller ones."""
     from vllm_kunlun_amd import synth
     sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], quant=fmt, **dims), "cuda", seed=dims["M"], dtype=dtype)
     out, named = _named(lambda: _call(sl))
-    assert all(k in named for k in launches) and "a column per pair" in named, named
+    assert all(k in named for k in launches) and ("a column per pair" in named) == (dims["M"] * dims["K"] < dims["E"]), named
     _check(sl, out)
 
 

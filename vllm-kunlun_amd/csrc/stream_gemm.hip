@@ -502,14 +502,20 @@ int launch_stream(const StreamParams& p, hipStream_t s) {
 // the tail (measured: +6..12% at k = 2048). Batches of a few tokens take the same shapes: with a column of workgroups per
 // pair (Qwen3, one token: layer 53 -> 24 us, its launches no longer mostly workgroups of experts without rows) keeping
 // a wave's whole K range in flight (8 steps) gains nothing at one token and loses 10 to 25 % from four tokens on.
-// 16-bit gate_up launches keep four steps in flight, whose weights are twice the bytes and nothing to work on (layer, us, two steps / four: Qwen3 dims bf16
-// 5 tokens 65.6 / 64.2, 12 119.0 / 117.6, 20 with +2.0 on the logits of 8 experts 111.4 / 108.6, 110 196.6 / 194.1; int8 12 73.3 / 74.6), but not on the
-// longest rows (16 experts of [8192 x 8192], top 2, 3 tokens 193 / 199, 12 441 / 442).
-// A layer too large for the first rule, with a column per pair: K split four ways at full depth in the gate_up launch (fp8: on fewer than 128 columns;
-// DeepSeek-V3 dims, layer, 23 tokens 854.5 / 858.3), and in a down launch of 16-bit weights on fewer than 64 columns. gate_up launch, us, two ways / four: DeepSeek-V3 dims int8 6 tokens 210 / 207, 8 265 / 262, fp8 4 155 / 150; 160
-// experts of [3072 x 5120], top 6, int8 5 tokens 74 / 71, bf16 24 456 / 440; 64 of [4096 x 4096], top 8, bf16 7 215 / 203. Down launch, bf16: 64
-// experts of [4096 x 2048] 24 columns 65 / 59, 56 107 / 101, 160 of [5120 x 1536] 36 85 / 85, 72 145 / 152, 144 218 / 261; int8: DeepSeek-V3 dims 24 columns 60
-// / 58.5, 64 of [6144 x 3072] 28 72 / 76, 64 of [4096 x 2048] 32 41.7 / 43.3, DeepSeek-V3 dims 128 236 / 255.
+// Figures below are the layer's time over its time without the branch, even load / +2.0 on the logits of eight experts / every token on the same
+// experts (samples of one prompt), layers as [hidden x intermediate].
+// (1) 16-bit gate_up launches with a column per expert keep four steps in flight, whose weights are twice the bytes and nothing to work on: Qwen3 dims
+// 16 tokens 0.99 / 0.98 / 0.99, 64 0.99 / 0.97 / 0.95, 160 0.99 / 0.95 / 0.92, 32 of [7168 x 2048], top 8, 8 0.99 / 0.98 / 0.91, of [2048 x 1024], top 4, 24
+// 0.98 / 0.92 / 1.03. Not with a column per
+// pair (Qwen3 dims 8 tokens 1.00 / 0.99 / 1.03; 128 of [1024 x 768], top 8, 8 1.02 / 1.08 / 1.16), nor on rows whose first steps are asked for before the
+// workgroup knows its rows (w_first; 64 of [1024 x 512], top 8, 24 0.99 / 0.99 / 1.10), nor on rows of 4096 and 8192 values and beyond (16 of [4096 x
+// 4096], top 2, 32 1.03 / 0.99 / 1.02, of [8192 x 8192] 1.03).
+// (2) 16-bit columns of fewer than 64 pairs in a layer too large for the first rule, long rows: K split four ways at full depth. 160 of [5120 x 1536],
+// top 6, 3 tokens 0.95 / 0.94 / 0.95, 10 0.98 / 0.96 / 0.91, 64 of [4096 x 2048], top 8, 5 0.96 / 0.93 / 0.94, 64 of [6144 x 3072], top 4, 8 0.97 / 0.97 / 0.89,
+// 128 of [3072 x 4096], top 8, 4 0.98 / 0.99 / 0.97, 6 0.98 / 0.98 / 1.03. More columns read shared weights too often ([3072 x 4096], 12 tokens 0.99 / 0.99 /
+// 1.16), and so do shorter rows (128 of [2048 x 3072], top 8, gate_up so too, 6 0.99 / 0.97 / 1.06; [5120 x 1536], down launch so too, 8 0.99 / 1.02 / 1.28). int8
+// and fp8 gain 0 to 2 % and lose up to 24 where tokens share experts: DeepSeek-V3 dims int8 5 tokens 0.99 / 0.99 / 0.97, 16 1.00 / 1.00 / 1.05, 128 of
+// [4096 x 4096], top 4, 8 1.00 / 0.98 / 1.12, 16 1.00 / 0.99 / 1.24, fp8 16 1.00 / 1.00 / 1.18.
 // From four rows per expert on every workgroup of a large gate_up launch reads rows enough for them to count, and waves of four fragments halve the
 // workgroups that read them, K split four ways where it is long (int8 beyond 4096 codes, fp8 from 6144 on). Layer, us, two fragments / four: DeepSeek-V3 dims int8
 // 110 tokens 1597 / 1596, 128 1668 / 1624, 250 1802 / 1753, 320 1897 / 1821, 250 with +2.0 on the logits of 8 experts 1903 / 1868, fp8 140 1696 / 1682, 250 1821 /
@@ -522,10 +528,13 @@ int launch_rows16(const StreamParams& p, int rows, hipStream_t s) {
   const int n_half = SWIGLU ? p.n / 2 : p.n;
   const int blocks = p.E * ceil_div(n_half, kWaves * (SWIGLU ? 1 : 2) * 16);
   constexpr bool k16 = FMT == Fmt::BF16 || FMT == Fmt::F16;
-  if (k16 && SWIGLU && ksteps >= 24 && ksteps < 256 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, k16 ? 4 : 2, 4, SCAN>(p, s);
+  if constexpr (k16 && SWIGLU) {  // (1)
+    if (p.slots.n == 0 && ksteps >= 64 && ksteps < 256 && ksteps != 128 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, 4, 4, SCAN>(p, s);
+  }
   if (ksteps >= 24 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, 2, 4, SCAN>(p, s);
-  if (ksteps >= 24 && p.slots.n > 0 && (SWIGLU ? FMT != Fmt::F8 || p.slots.n < 128 : k16 && p.slots.n < 64))
-    return launch_stream<FMT, 1, 2, SWIGLU, 4 / V, 4, SCAN>(p, s);
+  if constexpr (k16 && SWIGLU == SCAN) {  // (2): a gate_up launch with columns of pairs sorts them, a down launch never does
+    if (p.slots.n > 0 && p.slots.n < 64 && ksteps >= (SWIGLU ? 96 : 64)) return launch_stream<FMT, 1, 2, SWIGLU, 4, 4, SCAN>(p, s);
+  }
   if constexpr (SWIGLU && FMT == Fmt::I8) {
     if (ksteps >= 24 && ksteps <= 64 && rows >= 4ll * p.E) return launch_stream<FMT, 1, 4, SWIGLU, 4, 2, SCAN>(p, s);
   }
