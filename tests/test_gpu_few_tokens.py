@@ -322,16 +322,18 @@ def test_columns_of_pairs_of_large_layers_match_the_oracle(fmt, dims, launches, 
     _check(sl, out)
 
 
-@pytest.mark.parametrize("fmt,H,dtype,split", [("int8", 1600, torch.bfloat16, 2), ("int8", 4160, torch.float16, 4), ("fp8", 6272, torch.bfloat16, 4)])
-def test_four_rows_per_expert_of_large_layers_match_the_oracle(fmt, H, dtype, split):
-    """gate_up launches of large layers from four rows per expert on, whose waves take four channel fragments; some experts have more
-    rows than a pass, some none."""
+@pytest.mark.parametrize("fmt,H,M,dtype,fragments", [
+    ("int8", 4160, 32, torch.float16, 4), ("int8", 4160, 31, torch.bfloat16, 2), ("int8", 4096, 32, torch.bfloat16, 2),
+    ("fp8", 6272, 32, torch.bfloat16, 4), ("fp8", 6144, 32, torch.float16, 2), ("fp8", 8064, 32, torch.bfloat16, 4), ("fp8", 8192, 32, torch.bfloat16, 2)])
+def test_four_rows_per_expert_of_large_layers_match_the_oracle(fmt, H, M, dtype, fragments):
+    """gate_up launches of large layers with long rows from four rows per expert on, whose waves take four channel fragments; some experts have
+    more rows than a pass, some none."""
     from vllm_kunlun_amd import synth
-    sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], quant=fmt, M=32, E=32, K=4, H=H, I=4096), "cuda", seed=H, dtype=dtype)
+    sl = synth.make_layer(synth.scaled(synth.SHAPES["qwen3-decode"], quant=fmt, M=M, E=32, K=4, H=H, I=4096), "cuda", seed=H, dtype=dtype)
     sl.logits[:20, :2] += 9.0
     sl.logits[:, 30:] -= 9.0
     out, named = _named(lambda: _call(sl))
-    assert f"4 channel fragments per wave, SiLU-mul, {2 if fmt == 'fp8' else 4} steps in flight, K split {split}" in named, named
+    assert f"{fragments} channel fragments per wave, SiLU-mul, {2 if fmt == 'fp8' else 4} steps in flight, K split {fragments}" in named, named
     _check(sl, out)
 
 

@@ -413,9 +413,9 @@ __global__ __launch_bounds__(kWaves* kWave, QUANT ? 4 : 1) void stream_gemm_kern
           }
           if (kb + D < klen) load_step(d, kb_of(kb + D));
           // F8, K split two ways (long streams, many columns): a step's loads stay ahead of the next step's wait and scaling, where the
-          // compiler would sink them (DeepSeek-V3 dims, layer, 8 tokens 393 -> 389 us, 23 898 -> 891, 64 1469 -> 1462, 128 1633 -> 1619, 256 1806 ->
-          // 1787; other formats level). Not where K is whole or split four ways: 64 experts of [2816 x 2048], top 6, layer, 32 tokens 93.5 -> 98.4
-          // us with it in the split launches, 100.3 in all; 100 of [1024 x 1024], top 8, 44.6 -> 48.3; 16 of [8192 x 4096], top 2, 138.1 -> 136.6.
+          // compiler would sink them (DeepSeek-V3 dims, layer, 8 tokens 393 -> 389 us, 23 898 -> 891, 64 1469 -> 1462; other formats level). Not where K
+          // is whole or split four ways: 64 experts of [2816 x 2048], top 6, layer, 32 tokens 93.5 -> 98.4 us with it in the split launches, 100.3 in
+          // all; 100 of [1024 x 1024], top 8, 44.6 -> 48.3; 16 of [8192 x 4096], top 2, 138.1 -> 136.6; level with four channel fragments a wave.
           if constexpr (FMT == Fmt::F8 && KS == 2) __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -516,11 +516,14 @@ int launch_stream(const StreamParams& p, hipStream_t s) {
 // 1.16), and so do shorter rows (128 of [2048 x 3072], top 8, gate_up so too, 6 0.99 / 0.97 / 1.06; [5120 x 1536], down launch so too, 8 0.99 / 1.02 / 1.28). int8
 // and fp8 gain 0 to 2 % and lose up to 24 where tokens share experts: DeepSeek-V3 dims int8 5 tokens 0.99 / 0.99 / 0.97, 16 1.00 / 1.00 / 1.05, 128 of
 // [4096 x 4096], top 4, 8 1.00 / 0.98 / 1.12, 16 1.00 / 0.99 / 1.24, fp8 16 1.00 / 1.00 / 1.18.
-// From four rows per expert on every workgroup of a large gate_up launch reads rows enough for them to count, and waves of four fragments halve the
-// workgroups that read them, K split four ways where it is long (int8 beyond 4096 codes, fp8 from 6144 on). Layer, us, two fragments / four: DeepSeek-V3 dims int8
-// 110 tokens 1597 / 1596, 128 1668 / 1624, 250 1802 / 1753, 320 1897 / 1821, 250 with +2.0 on the logits of 8 experts 1903 / 1868, fp8 140 1696 / 1682, 250 1821 /
-// 1774; 64 experts of [6144 x 6144], top 4, int8 80 560 / 552; 128 of [3072 x 4096], top 8, int8 150 405 / 386, but fp8 80 374 / 398, bf16 70 748 / 764. Fewer rows: int8
-// 70 tokens 1429 / 1432, 33 1100 / 1101. K split two ways there: 250 tokens 1802 / 1745, and 64 of [4096 x 4096], int8 70 274 / 265 (four ways 270).
+// (3) From four rows per expert on every workgroup of a large gate_up launch reads rows enough for them to count: waves of four channel fragments, K
+// split four ways, halve the workgroups that read them, where rows are long (int8 beyond 4096 codes, fp8 beyond 6144 and below 8192). Even load / hot
+// experts: DeepSeek-V3 dims int8 128 tokens (4 rows) 1.00 / 1.00, 160 0.99 / 1.00, 250 0.97 / 0.98, 320 0.96 / 0.97, fp8 128 1.00 / 0.99, 250 0.98 / 0.98;
+// 160 of [5120 x 1536], top 6, int8 112 1.00 / 0.95, 250 0.98 / 0.95; 128 of [7168 x 2048], top 8, int8 64 1.00 / 0.98, 160 0.97 / 0.96, fp8 96 1.00 / 0.96;
+// 128 of [5120 x 5120], top 6, int8 160 0.99 / 1.01. Split two ways an expert's further passes weigh more: DeepSeek-V3 dims int8 250 0.97 / 1.01, 128 of
+// [7168 x 2048] 96 0.99 / 1.02. Shorter rows, two ways: 64 of [4096 x 2048], top 8, int8 56 1.00 / 1.02, 128 of [3072 x 4096], top 8, 112 1.00 / 1.02, 256 of
+// [2048 x 2048], top 8, 144 1.01 / 1.04, 128 of [4096 x 4096], top 4, 200 0.98 / 1.02. fp8 rows of 8192 values: 16 of [8192 x 8192], top 2, 40 1.08 / 1.09, 64 of [8192 x
+// 3072], top 4, 80 1.06 / 1.01. (The fp8 fence, below, changes nothing here: 0.998 to 1.002.)
 template <Fmt FMT, bool SWIGLU, bool SCAN>
 int launch_rows16(const StreamParams& p, int rows, hipStream_t s) {
   constexpr int V = FMT == Fmt::F8 ? 2 : 1;
@@ -535,11 +538,8 @@ int launch_rows16(const StreamParams& p, int rows, hipStream_t s) {
   if constexpr (k16 && SWIGLU == SCAN) {  // (2): a gate_up launch with columns of pairs sorts them, a down launch never does
     if (p.slots.n > 0 && p.slots.n < 64 && ksteps >= (SWIGLU ? 96 : 64)) return launch_stream<FMT, 1, 2, SWIGLU, 4, 4, SCAN>(p, s);
   }
-  if constexpr (SWIGLU && FMT == Fmt::I8) {
-    if (ksteps >= 24 && ksteps <= 64 && rows >= 4ll * p.E) return launch_stream<FMT, 1, 4, SWIGLU, 4, 2, SCAN>(p, s);
-  }
-  if constexpr (SWIGLU && (FMT == Fmt::I8 || FMT == Fmt::F8)) {
-    if (ksteps > (FMT == Fmt::I8 ? 64 : 96) && rows >= 4ll * p.E) return launch_stream<FMT, 1, 4, SWIGLU, 4 / V, 4, SCAN>(p, s);
+  if constexpr (SWIGLU && (FMT == Fmt::I8 || FMT == Fmt::F8)) {  // (3)
+    if ((FMT == Fmt::I8 ? ksteps > 64 : ksteps > 96 && ksteps < 128) && rows >= 4ll * p.E) return launch_stream<FMT, 1, 4, SWIGLU, 4 / V, 4, SCAN>(p, s);
   }
   if (ksteps >= 24) return launch_stream<FMT, 1, 2, SWIGLU, 4 / V, 2, SCAN>(p, s);
   return launch_stream<FMT, 1, 2, SWIGLU, 4 / V, 1, SCAN>(p, s);
