@@ -129,9 +129,9 @@ def test_tail_expert(kind, tail, act):
 
 
 @pytest.mark.parametrize("kind", ["int8", "fp8"])
-@pytest.mark.parametrize("counts", [[], [1], [193], [5] * 40], ids=len)  # routed items: none, fewer than XCDs, of two tiles, a share each
+@pytest.mark.parametrize("counts", [[], [1], [193], [5] * 40], ids=len)  # routed items: none, fewer than XCDs, of two tiles, some each
 @pytest.mark.parametrize("tail", [7, 1600, 3100])
-def test_tail_expert_is_shared_out(kind, counts, tail):
+def test_tail_expert_beside_few_items(kind, counts, tail):
     counts = counts or [0]
     _same(*_launch(kind, counts, 1024, 768, 0, torch.bfloat16, tail=tail))
 

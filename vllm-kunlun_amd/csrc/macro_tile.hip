@@ -262,25 +262,20 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
   }
   __syncthreads();
   // ---- the workgroup's items, as in tiled_gemm.hip: the list of (m-tile, channel block) pairs, expert by expert, in eight
-  // segments, one per XCD, which the workgroups of the XCD walk side by side; an expert's rows split evenly over its m-tiles. A tail
-  // expert's items are an eighth each XCD's, too, which XCD x takes up when x eighths of its others are done: they have the rows
-  // of all tokens and keep the matrix unit busy on weights that the caches hold, while the other XCDs' items wait for memory. At the end of
-  // the list they were all one XCD's, whose share of the weights the others had to bring. DeepSeek-V3 dims, layer, us, at the end / first on every
-  // XCD / in turn with the others / so: int8 2048 tokens 2080 / 2086 / 2099 / 2053, 4096 2473 / 2496 / 2492 / 2444, 1000 1933 / 1950 / 1961 / 1930;
-  // fp8 3001 2402 / 2423 / 2394 / 2390, 1200 1975 / 2008 / 1990 / 1965. ----
+  // segments, one per XCD, which the workgroups of the XCD walk side by side; an expert's rows split evenly over its m-tiles. (A tail
+  // expert's items, which the list ends with, shared out over the XCDs: DeepSeek-V3 dims, layer, even load / +2.0 on the logits of eight experts, time
+  // over this order's, int8 2048 tokens 0.99 / 0.99, 4096 1.00 / 1.02, 5000 1.00 / 1.02, but 256 experts of [4096 x 1024], top 8, 2048 1.01 / 1.03, 128 of
+  // [5120 x 1536], top 8, 2048 1.00 / 1.03, 64 of [4096 x 1408], top 6, 2048 1.00 / 1.07.) ----
+  const int n_items = tile_lo[n_exp] * p.n_blocks;
+  const int seg = (n_items + 7) >> 3;
   const int xcd = blockIdx.x & 7;
-  const int n_routed = tile_lo[p.E] * p.n_blocks, n_tail = tile_lo[n_exp] * p.n_blocks - n_routed;
-  const int seg = (n_routed + 7) >> 3, seg_tail = (n_tail + 7) >> 3;
-  const int first = min(xcd * seg, n_routed), mine = min(seg, n_routed - first);
-  const int first_tail = min(xcd * seg_tail, n_tail), mine_tail = min(seg_tail, n_tail - first_tail);
-  const int before = (mine * xcd) >> 3;  // routed items before the tail's
+  const int seg_end = min((xcd + 1) * seg, n_items);
   const int per_xcd = gridDim.x >> 3;  // gridDim.x is a multiple of 8
   auto resolve_items = [&](int it0) {
     if (wave == 0 && lane < kMItems) {
-      const int at = (blockIdx.x >> 3) + (it0 + lane) * per_xcd;
-      const int lid = at < before ? first + at : at < before + mine_tail ? n_routed + first_tail + at - before : first + at - mine_tail;
+      const int lid = xcd * seg + (blockIdx.x >> 3) + (it0 + lane) * per_xcd;
       int e = -1, row0 = 0, nb = 0, end = 0, past = 0;
-      if (at < mine + mine_tail) {
+      if (lid < seg_end) {
         const int m_tile = lid / p.n_blocks;
         int lo = 0, hi = n_exp - 1;  // the last e with tile_lo[e] <= m_tile
         while (lo < hi) {
@@ -289,8 +284,8 @@ __global__ __launch_bounds__(kMThreads, 1) void macro_tile_kernel(const MacroPar
           else hi = mid - 1;
         }
         e = lo;
-        const int tile0 = tile_lo[e], mt = tile_lo[e + 1] - tile0;
-        const int u = lid - tile0 * p.n_blocks;
+        const int first = tile_lo[e], mt = tile_lo[e + 1] - first;
+        const int u = lid - first * p.n_blocks;
         int m;
         if (p.m_major) {
           m = u / p.n_blocks;
