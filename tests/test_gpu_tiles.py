@@ -110,7 +110,7 @@ def test_packed_tiles_take_scales_by_chunks(variant, blocks, group, dtype):
     shifted = torch.empty(scale.numel() + 8, dtype=dtype, device="cuda")[4:-4].copy_(chunks.flatten())
     lod = torch.tensor([0] + counts).cumsum(0).int().cuda()
     for act in (0, 1):
-        out = []
+        out, by_chunks = [], []
         for s, layout in ((scale, L.KMOE_S_ROWMAJOR), (chunks, L.KMOE_S_FRAG16), (shifted, L.KMOE_S_FRAG16)):
             y = torch.full((rows, n // 2 if act else n), float("nan"), dtype=dtype, device="cuda")
             g = L.GemmW4Args()
@@ -118,8 +118,12 @@ def test_packed_tiles_take_scales_by_chunks(variant, blocks, group, dtype):
             g.w, g.w_scale, g.group_size, g.lod = tiled.data_ptr(), s.data_ptr(), group, lod.data_ptr()
             g.E, g.n, g.k, g.rows, g.w_layout = E, n, k, rows, L.KMOE_W_TILED
             g.y, g.ldy, g.act, g.variant, g.act_dtype = y.data_ptr(), y.shape[1], act, variant, L.act_dtype(a, "test")
+            L.lib.kmoe_trace_kernels(1)
             L.check(L.lib.kmoe_grouped_gemm_w4a16(g, L.stream()))
+            by_chunks.append("scales by chunks" in L.lib.kmoe_traced_kernels().decode())
+            L.lib.kmoe_trace_kernels(0)
             out.append(y)
+        assert by_chunks == [False, group != 384, False]
         assert not out[0].isnan().any() and torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
 
 

@@ -410,11 +410,11 @@ int launch_w4_tile(const W4Params& p, int rows, bool f16, hipStream_t s) {
   const int n_blocks = ceil_div(n_half, kWaves * NFH * 16);
   const int items = (rows / kTileRows + min(p.E, rows)) * n_blocks;
   const dim3 grid(ceil_div(items, 8) * 8);
-  if (tracing_kernels())
-    note_kernel("w4_tile_kernel<%d-row tiles, %s, %s, %d per CU>", kTileRows, SWIGLU ? "SiLU-mul" : "plain",
-                f16 ? "f16" : "bf16", w4_workgroups(MF));
   const bool chunked = p.gs_shift >= 0 && p.s_g == 16 && reinterpret_cast<uintptr_t>(p.scale) % 16 == 0 &&
                        static_cast<int64_t>(p.n) * (p.k / p.gs) < (1ll << 30);
+  if (tracing_kernels())
+    note_kernel("w4_tile_kernel<%d-row tiles, %s, %s, %d per CU, scales by %s>", kTileRows, SWIGLU ? "SiLU-mul" : "plain",
+                f16 ? "f16" : "bf16", w4_workgroups(MF), chunked ? "chunks" : "lanes");
   auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kWaves * kWave), 0, s, p); };
   if (f16) chunked ? launch(w4_tile_kernel<MF, SWIGLU, true, PAST, true>) : launch(w4_tile_kernel<MF, SWIGLU, true, PAST, false>);
   else chunked ? launch(w4_tile_kernel<MF, SWIGLU, false, PAST, true>) : launch(w4_tile_kernel<MF, SWIGLU, false, PAST, false>);
