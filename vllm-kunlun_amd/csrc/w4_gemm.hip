@@ -150,8 +150,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 // The tall tiles' accumulators leave room for two.
 constexpr int w4_workgroups(int MF) { return MF <= 2 ? 4 : (MF == 4 ? 3 : 2); }
 // R: blocks of weights (registers) and of activations (LDS) in the rings. A stage waits for its own block, passes a
-// barrier, requests block kb + R - 1 of both and multiplies. No branch sits between a load and its use - the waits count
-// loads - so blocks past the end are requested as well, out of the descriptors' range: they fetch nothing.
+// barrier, requests block kb + R - 1 of both and multiplies. The waits count the loads of weights and activations, so blocks past the end
+// are requested as well, out of the descriptors' range: they fetch nothing. The scales' chunks are copied under a uniform branch; no wait counts
+// on them, and one that still counts them waits for more than it has to, never for less.
 constexpr int w4_ring(int MF) { return MF == 6 ? 3 : 2; }
 // PAST: the weights are read past the caches (see buffer_stream_load16), where nearly every expert has one m-tile: always at 16 and 32
 // rows, at 64 rows up to 50 rows per expert. Layer, us, ordinary / past the caches: Qwen3 dims 128 tokens 78.8 / 75.9, cold 84.0 / 79.8,
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(kWaves* kWave, w4_workgroups(MF)) void w4_tile_kern
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     hold_s();
   }
-  // (no exit inside the body: as one basic block it fits the registers)
+  // (no exit inside the body: with one the accumulators do not fit the registers)
   int kb = 0;
   for (; kb + R <= kblocks; kb += R)
     static_for<R>([&](auto u) __attribute__((always_inline)) { stage(kb + decltype(u)::value, u); });
@@ -434,7 +435,7 @@ __global__ __launch_bounds__(256) void tile_scales_kernel(const uint16_t* __rest
 
 }  // namespace
 
-// Layer, time on 16-row tiles (whose launch needs the sort's, and which read a scale once per chunk of the contraction) over time on 16-row passes of
+// Layers as [hidden x intermediate], time on 16-row tiles (whose launch needs the sort's, and which read a scale once per chunk of the contraction) over time on 16-row passes of
 // the streaming kernel (which sorts the pairs on the way and splits the contraction over its waves): even load / +2.0 on the logits of eight
 // experts / every token on the same experts.
 // Rows beyond 4096 values. Up to 16 tokens no expert needs a second pass, and tiles lack workgroups where tokens share experts: 160 experts of
