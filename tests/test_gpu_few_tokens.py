@@ -309,7 +309,8 @@ def test_packed_launches_on_long_rows_match_the_oracle(dims, shape, dtype):
     ("none", dict(M=16, E=96, K=4, H=3072, I=2048), ["SiLU-mul, 4 steps in flight, K split 2", "plain, 4 steps in flight, K split 2"]),
     ("none", dict(M=9, E=64, K=4, H=1024, I=512), ["SiLU-mul, 2 steps in flight, K split 4"]),
     ("none", dict(M=16, E=48, K=4, H=2048, I=512), ["SiLU-mul, 4 steps in flight, K split 4"]),   # a column per expert
-    ("none", dict(M=16, E=48, K=4, H=2016, I=512), ["SiLU-mul, 2 steps in flight, K split 4"])], ids=str)
+    ("none", dict(M=16, E=48, K=4, H=2016, I=512), ["SiLU-mul, 2 steps in flight, K split 4"]),
+    ("none", dict(M=16, E=31, K=4, H=2048, I=512), ["SiLU-mul, 2 steps in flight, K split 4"])], ids=str)   # fewer workgroups than CUs
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_columns_of_pairs_of_large_layers_match_the_oracle(fmt, dims, launches, dtype):
     """Layers of a few tokens, whose column-per-pair launches split K over four waves where they are large, have 16-bit weights, long rows and

@@ -509,7 +509,8 @@ int launch_stream(const StreamParams& p, hipStream_t s) {
 // 0.98 / 0.92 / 1.03. Not with a column per
 // pair (Qwen3 dims 8 tokens 1.00 / 0.99 / 1.03; 128 of [1024 x 768], top 8, 8 1.02 / 1.08 / 1.16), nor on rows whose first steps are asked for before the
 // workgroup knows its rows (w_first; 64 of [1024 x 512], top 8, 24 0.99 / 0.99 / 1.10), nor on rows of 4096 and 8192 values and beyond (16 of [4096 x
-// 4096], top 2, 32 1.03 / 0.99 / 1.02, of [8192 x 8192] 1.03).
+// 4096], top 2, 32 1.03 / 0.99 / 1.02, of [8192 x 8192] 1.03), nor in launches of fewer workgroups than CUs (a rank's 16 of the 128 experts of Qwen3 dims, 32
+// 1.04 / 1.01 / 1.00).
 // (2) 16-bit columns of fewer than 64 pairs in a layer too large for the first rule, long rows: K split four ways at full depth. 160 of [5120 x 1536],
 // top 6, 3 tokens 0.95 / 0.94 / 0.95, 10 0.98 / 0.96 / 0.91, 64 of [4096 x 2048], top 8, 5 0.96 / 0.93 / 0.94, 64 of [6144 x 3072], top 4, 8 0.97 / 0.97 / 0.89,
 // 128 of [3072 x 4096], top 8, 4 0.98 / 0.99 / 0.97, 6 0.98 / 0.98 / 1.03. More columns read shared weights too often ([3072 x 4096], 12 tokens 0.99 / 0.99 /
@@ -532,7 +533,7 @@ int launch_rows16(const StreamParams& p, int rows, hipStream_t s) {
   const int blocks = p.E * ceil_div(n_half, kWaves * (SWIGLU ? 1 : 2) * 16);
   constexpr bool k16 = FMT == Fmt::BF16 || FMT == Fmt::F16;
   if constexpr (k16 && SWIGLU) {  // (1)
-    if (p.slots.n == 0 && ksteps >= 64 && ksteps < 256 && ksteps != 128 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, 4, 4, SCAN>(p, s);
+    if (p.slots.n == 0 && ksteps >= 64 && ksteps < 256 && ksteps != 128 && blocks >= 256 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, 4, 4, SCAN>(p, s);
   }
   if (ksteps >= 24 && blocks < 2048) return launch_stream<FMT, 1, 2, SWIGLU, 2, 4, SCAN>(p, s);
   if constexpr (k16 && SWIGLU == SCAN) {  // (2): a gate_up launch with columns of pairs sorts them, a down launch never does
